@@ -20,13 +20,90 @@ __device__ __forceinline__ unsigned int hash2(unsigned int a, unsigned int b) {
   return h;
 }
 
-// logits bf16 [S, V]; one block (256 threads) per row.
-template <bool GUMBEL>
-__global__ __launch_bounds__(256) void argmax_kernel(
+// One row of bf16 logits walked by a block of NT threads. The row starts at
+// any 2-byte boundary (odd vocabularies): `head` elements up to the first
+// 16-byte boundary, nvec vectors of 8, and a tail; head and tail (7 at most
+// each) are one extra element of the first 16 threads.
+template <int NT>
+struct Bf16Row {
+  const short* row;
+  const short8_t* rv;
+  int head, nvec, ex;  // ex: index of the extra element, -1 for none
+
+  __device__ __forceinline__ Bf16Row(const short* p, int V) {
+    row = p;
+    const int tid = threadIdx.x;
+    head = min(V, (int)(((16 - ((uintptr_t)p & 15)) & 15) >> 1));
+    nvec = (V - head) >> 3;
+    rv = reinterpret_cast<const short8_t*>(p + head);
+    const int tail0 = head + nvec * 8;
+    ex = tid < head ? tid : (tid >= 8 && tail0 + tid - 8 < V) ? tail0 + tid - 8 : -1;
+  }
+  // f(eight elements, index of the first) with four loads in flight, then
+  // one(element, index) for this thread's extra element
+  template <typename F, typename G>
+  __device__ __forceinline__ void each8(F f, G one) const {
+    int i = threadIdx.x;
+    for (; i + 3 * NT < nvec; i += 4 * NT) {
+      short8_t v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = rv[i + u * NT];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) f(v[u], head + (i + u * NT) * 8);
+    }
+    for (; i < nvec; i += NT) f(rv[i], head + i * 8);
+    if (ex >= 0) one(row[ex], ex);
+  }
+  template <typename F>
+  __device__ __forceinline__ void each(F f) const {
+    each8(
+        [&](const short8_t& v, int i0) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) f(v[j], i0 + j);
+        },
+        f);
+  }
+};
+
+// the block's largest value and its index (ties: the lower index) to out
+template <int NT>
+__device__ __forceinline__ void block_argmax(float best, int best_idx, long* out) {
+  __shared__ float s_val[NT / 64];
+  __shared__ int s_idx[NT / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  auto merge = [&](float ov, int oi) {
+    if (ov > best || (ov == best && oi < best_idx)) {
+      best = ov;
+      best_idx = oi;
+    }
+  };
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+    merge(__shfl_xor(best, off, 64), __shfl_xor(best_idx, off, 64));
+  if (lane == 0) {
+    s_val[wave] = best;
+    s_idx[wave] = best_idx;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < NT / 64; ++w) merge(s_val[w], s_idx[w]);
+    *out = best_idx;
+  }
+}
+
+__device__ __forceinline__ float gumbel_noise(unsigned int seed, int idx) {
+  const unsigned int h = hash2(seed, (unsigned int)idx);
+  // u in (0,1): (h + 1) / 2^32
+  const float u = ((float)h + 1.0f) * 2.3283064e-10f;
+  return __logf(-__logf(u));
+}
+
+// logits bf16 [S, V]; one block of NT threads per row.
+template <bool GUMBEL, int NT>
+__global__ __launch_bounds__(NT) void argmax_kernel(
     long* __restrict__ out,            // [S]
     const short* __restrict__ logits,  // [S, V] bf16
     const float* __restrict__ temperatures,  // [S] (GUMBEL)
-    const int* __restrict__ top_k,           // [S] (GUMBEL; -1 = off)
     const long* __restrict__ seeds,          // [S] (GUMBEL)
     const int V) {
   const int s = blockIdx.x;
@@ -39,7 +116,7 @@ __global__ __launch_bounds__(256) void argmax_kernel(
   // vectorized short8 loads over the vocab row
   const int nvec = V >> 3;
   const short8_t* rv = reinterpret_cast<const short8_t*>(row);
-  for (int i = threadIdx.x; i < nvec; i += blockDim.x) {
+  for (int i = threadIdx.x; i < nvec; i += NT) {
     short8_t v = rv[i];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -47,10 +124,7 @@ __global__ __launch_bounds__(256) void argmax_kernel(
       float val = bf16_bits_to_float(v[j]);
       if constexpr (GUMBEL) {
         val *= inv_t;
-        const unsigned int h = hash2(seed, (unsigned int)idx);
-        // u in (0,1): (h + 1) / 2^32
-        const float u = ((float)h + 1.0f) * 2.3283064e-10f;
-        val += -__logf(-__logf(u));
+        val -= gumbel_noise(seed, idx);
       }
       if (val > best) {
         best = val;
@@ -59,46 +133,18 @@ __global__ __launch_bounds__(256) void argmax_kernel(
     }
   }
   // tail (V not divisible by 8)
-  for (int idx = nvec * 8 + threadIdx.x; idx < V; idx += blockDim.x) {
+  for (int idx = nvec * 8 + threadIdx.x; idx < V; idx += NT) {
     float val = bf16_bits_to_float(row[idx]);
     if constexpr (GUMBEL) {
       val *= inv_t;
-      const unsigned int h = hash2(seed, (unsigned int)idx);
-      const float u = ((float)h + 1.0f) * 2.3283064e-10f;
-      val += -__logf(-__logf(u));
+      val -= gumbel_noise(seed, idx);
     }
     if (val > best) {
       best = val;
       best_idx = idx;
     }
   }
-  // block argmax reduce: pack (value, idx); ties -> lower idx wins
-  __shared__ float s_val[4];
-  __shared__ int s_idx[4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    float ov = __shfl_xor(best, off, 64);
-    int oi = __shfl_xor(best_idx, off, 64);
-    if (ov > best || (ov == best && oi < best_idx)) {
-      best = ov;
-      best_idx = oi;
-    }
-  }
-  if (lane == 0) {
-    s_val[wave] = best;
-    s_idx[wave] = best_idx;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 4; ++w) {
-      if (s_val[w] > best || (s_val[w] == best && s_idx[w] < best_idx)) {
-        best = s_val[w];
-        best_idx = s_idx[w];
-      }
-    }
-    out[s] = best_idx;
-  }
+  block_argmax<NT>(best, best_idx, out + s);
 }
 
 // fp32 logits [S, V]: argmax of every bit, ties to the lower index; one block
@@ -165,23 +211,82 @@ __global__ __launch_bounds__(AM_NT) void argmax_f32_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Fused top-k/top-p + Gumbel-max sampler.
+// Fused top-k/top-p + Gumbel-max sampler, one block of 1024 threads per row.
 //
 // bf16 logits have 16-bit patterns that order monotonically once sign-flipped
-// (key = bits<0 ? ~bits : bits|0x8000), so a 256-bin histogram over the high
-// byte plus a second one over the boundary bin's low byte finds the EXACT
-// k-th-largest value and the exact top-p mass threshold — no sort. The final
-// pass Gumbel-argmaxes over {key >= threshold}, which samples the truncated
-// softmax exactly. One 256-thread block per row; 4 passes over the vocab.
-// (Replaces the torch sort path the reference's vLLM sampler falls back to.)
+// (key = bits<0 ? ~bits : bits|0x8000). The limits of top-k and top-p are
+// found as keys from histograms, without a sort, and the last pass
+// Gumbel-argmaxes over {key >= threshold}, which samples the truncated softmax
+// exactly.
+//
+// All elements of one key have one probability, so counts per key are enough
+// for the mass too: pass 2 counts the WIN keys below the row's largest (64 KB
+// of LDS) and sums the whole row's mass in registers; a scan over the bins
+// from the top then gives both limits exactly. WIN keys are 128 octaves below
+// a positive maximum (all positive logits down to 2^-120 of it). Where a limit
+// lies below the window (nearly flat rows, k of the order of the row) two
+// coarser histograms find it: the keys' upper 12 bits, then the lower 4 inside
+// the bin that the limit falls into.
+//
+// What bounds it: one pass of LDS atomics, an exponential per element and the
+// three passes over the row, which come from the L2 and the memory-side cache.
+// A histogram over the keys' upper byte puts a model's logits into half a
+// dozen bins and serialises a wave's 64 adds, for count and mass each. Rows of
+// N(0, 2.5) logits, top-k and top-p mixed, that form -> this one: 256 x 128256
+// 704 -> 78 us, 256 x 32000 141 -> 34 us, 1 x 128256 465 -> 44 us; limits
+// below the window (k of the order of the row) 702 -> 156 us. Holding the row
+// in registers over the passes is not faster (80 us).
 // ---------------------------------------------------------------------------
+constexpr int RT = 1024;
+constexpr int WIN = 16384;
+constexpr int KBINS = 4096;
+
 __device__ __forceinline__ unsigned int bf16_sort_key(short bits) {
   const unsigned short u = (unsigned short)bits;
   return (u & 0x8000u) ? (unsigned int)(unsigned short)~u
                        : (unsigned int)(u | 0x8000u);
 }
+__device__ __forceinline__ float key_value(unsigned int key) {
+  return bf16_bits_to_float((short)((key & 0x8000u) ? (key & 0x7fffu) : ~key));
+}
 
-__global__ __launch_bounds__(256) void topk_topp_sample_kernel(
+// Of bins 0, 1, ... with value(bin) each, PER per thread in order: the first
+// bin at which the running sum reaches `target` goes to *bin and the sum
+// before it to *above (neither is written if the total stays below). All
+// threads of the block call it; the results can be read on return.
+template <int PER, typename T, typename F>
+__device__ __forceinline__ void find_bin(F value, T target, T* wave_sum, int* bin,
+                                         T* above) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  T v[PER], own = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    v[j] = value(tid * PER + j);
+    own += v[j];
+  }
+  T incl = own;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const T o = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += o;
+  }
+  if (lane == 63) wave_sum[wave] = incl;
+  __syncthreads();
+  T c = incl - own;
+  for (int w = 0; w < wave; ++w) c += wave_sum[w];
+  // a thread's end is the next one's start in exact sums only: in floating
+  // point the first thread at or past the target is taken by the smaller bin
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    if (c < target && c + v[j] >= target) {
+      if (atomicMin(bin, tid * PER + j) > tid * PER + j) *above = c;
+    }
+    c += v[j];
+  }
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
     long* __restrict__ out,            // [S]
     const short* __restrict__ logits,  // [S, V] bf16
     const float* __restrict__ temperatures,
@@ -189,148 +294,224 @@ __global__ __launch_bounds__(256) void topk_topp_sample_kernel(
     const int* __restrict__ top_k,    // [S] (<=0 disables)
     const long* __restrict__ seeds,   // [S]
     const int V) {
+  typedef unsigned long long u64;
   const int s = blockIdx.x;
-  const short* row = logits + (long)s * V;
   const float inv_t = 1.f / fmaxf(temperatures[s], 1e-5f);
   const float p = top_p[s];
   const int k = top_k[s];
   const unsigned int seed = (unsigned int)(seeds[s] & 0xFFFFFFFF);
   const bool use_k = (k > 0) && (k < V);
-  const bool use_p = p < 1.0f;
+  bool use_p = p < 1.0f;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
+  constexpr int NWV = RT / 64;
+  constexpr int NONE = 0x7fffffff;
 
-  __shared__ int h_cnt[256];
-  __shared__ float h_mass[256];
-  __shared__ float s_red[4];
-  __shared__ int s_redi[4];
-  __shared__ float sh_m;
-  __shared__ int sh_bk, sh_bp, sh_need_k;
-  __shared__ float sh_need_p;
-  __shared__ unsigned int sh_thresh;
+  __shared__ union {
+    unsigned int win[WIN];
+    struct {
+      unsigned int cnt[KBINS];
+      u64 mass[KBINS];
+    } h;
+  } lds;
+  __shared__ unsigned int f_cnt[16];
+  __shared__ u64 f_mass[16];
+  __shared__ unsigned int s_key[NWV];
+  __shared__ unsigned int s_bad[NWV];
+  __shared__ double w_mass[NWV];
+  __shared__ unsigned int w_cnt[NWV];
+  __shared__ u64 w_fix[NWV];
+  __shared__ int sh_bin[4];
+  __shared__ unsigned int sh_above_k;
+  __shared__ double sh_above_p;
+  __shared__ u64 sh_above_f;
 
-  // ---- pass A: row max (exp stability) ----
-  float lmax = -1e38f;
-  for (int i = tid; i < V; i += 256)
-    lmax = fmaxf(lmax, bf16_bits_to_float(row[i]));
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-    lmax = fmaxf(lmax, __shfl_xor(lmax, off, 64));
-  if (lane == 0) s_red[wave] = lmax;
-  __syncthreads();
-  if (tid == 0) {
-    float m = s_red[0];
-    for (int w = 1; w < 4; ++w) m = fmaxf(m, s_red[w]);
-    sh_m = m;
-  }
-  h_cnt[tid] = 0;
-  h_mass[tid] = 0.f;
-  __syncthreads();
-  const float m = sh_m;
-
-  // ---- pass B: high-byte histogram of (count, exp-mass) ----
-  for (int i = tid; i < V; i += 256) {
-    const short b = row[i];
-    const unsigned int key = bf16_sort_key(b);
-    const float e = __expf((bf16_bits_to_float(b) - m) * inv_t);
-    atomicAdd(&h_cnt[key >> 8], 1);
-    atomicAdd(&h_mass[key >> 8], e);
-  }
-  __syncthreads();
-  if (tid == 0) {
-    float Z = 0.f;
-    for (int b = 0; b < 256; ++b) Z += h_mass[b];
-    int bk = 0, need_k = 0x7FFFFFFF;
-    if (use_k) {
-      int c = 0;
-      for (int b = 255; b >= 0; --b) {
-        if (c + h_cnt[b] >= k) { bk = b; need_k = k - c; break; }
-        c += h_cnt[b];
-      }
-    }
-    int bp = 0;
-    float need_p = 1e38f;
-    if (use_p) {
-      const float target = p * Z;
-      float c = 0.f;
-      for (int b = 255; b >= 0; --b) {
-        if (c + h_mass[b] >= target) { bp = b; need_p = target - c; break; }
-        c += h_mass[b];
-      }
-    }
-    sh_bk = bk; sh_bp = bp; sh_need_k = need_k; sh_need_p = need_p;
-  }
-  __syncthreads();
-  const int bk = sh_bk, bp = sh_bp;
-  h_cnt[tid] = 0;
-  h_mass[tid] = 0.f;
-  __syncthreads();
-
-  // ---- pass C: low-byte histograms inside the two boundary bins ----
+  const Bf16Row<RT> row(logits + (long)s * V, V);
+  unsigned int thr = 0;
   if (use_k || use_p) {
-    for (int i = tid; i < V; i += 256) {
-      const short b = row[i];
-      const unsigned int key = bf16_sort_key(b);
-      const int hi = key >> 8;
-      if (use_k && hi == bk) atomicAdd(&h_cnt[key & 255], 1);
-      if (use_p && hi == bp)
-        atomicAdd(&h_mass[key & 255],
-                  __expf((bf16_bits_to_float(b) - m) * inv_t));
+    // ---- largest number (exp stability), and whether a mass can be formed ----
+    unsigned int mk = 0;
+    unsigned int bad = 0;  // a NaN or +inf: no mass, as its sum would be NaN
+    row.each([&](short b, int) {
+      const unsigned int mag = (unsigned short)b & 0x7fffu;
+      if (mag > 0x7f80u || (unsigned short)b == 0x7f80u) bad = 1;
+      else mk = max(mk, bf16_sort_key(b));
+    });
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      mk = max(mk, (unsigned int)__shfl_xor((int)mk, off, 64));
+    bad = __ballot(bad != 0) != 0;
+    if (lane == 0) {
+      s_key[wave] = mk;
+      s_bad[wave] = bad;
     }
-  }
-  __syncthreads();
-  if (tid == 0) {
-    unsigned int tk = 0, tp = 0;
-    if (use_k) {
-      int c = 0, lo = 0;
-      for (int l = 255; l >= 0; --l) {
-        if (c + h_cnt[l] >= sh_need_k) { lo = l; break; }
-        c += h_cnt[l];
-      }
-      tk = ((unsigned int)bk << 8) | lo;
+    for (int i = tid; i < WIN; i += RT) lds.win[i] = 0;
+    if (tid < 16) {
+      f_cnt[tid] = 0;
+      f_mass[tid] = 0;
     }
-    if (use_p) {
-      float c = 0.f;
-      int lo = 0;
-      for (int l = 255; l >= 0; --l) {
-        if (c + h_mass[l] >= sh_need_p) { lo = l; break; }
-        c += h_mass[l];
-      }
-      tp = ((unsigned int)bp << 8) | lo;
+    if (tid < 4) sh_bin[tid] = NONE;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) {
+      mk = max(mk, s_key[w]);
+      bad |= s_bad[w];
     }
-    sh_thresh = tk > tp ? tk : tp;
-  }
-  __syncthreads();
-  const unsigned int thr = sh_thresh;
+    // all of them -inf: no mass either
+    if (bad || mk <= 0x7fu) use_p = false;
+    // with NaNs and infinities above it the largest number is not the
+    // largest key, and the counts start at the top
+    const unsigned int top = bad ? 0xffffu : mk;
+    const float m = key_value(mk);
+    auto weight = [&](float x) { return __expf((x - m) * inv_t); };
 
-  // ---- pass D: Gumbel-argmax over the surviving set ----
+    // ---- counts per key in the window, mass of the row ----
+    float z = 0.f;
+    row.each([&](short b, int) {
+      const unsigned int at = top - bf16_sort_key(b);
+      if (at < WIN) atomicAdd(&lds.win[at], 1u);
+      if (use_p) z += weight(bf16_bits_to_float(b));
+    });
+    double zz = z;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) zz += __shfl_xor(zz, off, 64);
+    if (lane == 0) w_mass[wave] = zz;
+    __syncthreads();
+    zz = 0;
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) zz += w_mass[w];
+    __syncthreads();  // w_mass is written again below
+    const double want_p = (double)p * zz;
+    if (use_k)
+      find_bin<WIN / RT, unsigned int>([&](int i) { return lds.win[i]; },
+                                       (unsigned int)k, w_cnt, &sh_bin[0],
+                                       &sh_above_k);
+    if (use_p)
+      find_bin<WIN / RT, double>(
+          [&](int i) {
+            const unsigned int n = lds.win[i];
+            return n ? n * (double)weight(key_value(top - i)) : 0.0;
+          },
+          want_p, w_mass, &sh_bin[1], &sh_above_p);
+    bool far_k = use_k, far_p = use_p && want_p > 0;
+    if (use_k && sh_bin[0] != NONE) {
+      thr = top - sh_bin[0];
+      far_k = false;
+    }
+    if (far_p && sh_bin[1] != NONE) {
+      thr = max(thr, top - sh_bin[1]);
+      far_p = false;
+    }
+    // the larger threshold wins, so a limit below the window matters only if
+    // the other one is not inside it
+    if ((far_k || far_p) && thr == 0) {
+      constexpr float ONE = 1099511627776.0f;  // mass in 2^-40 of the largest term
+      auto fixed = [&](short b) {
+        return (u64)(fminf(weight(bf16_bits_to_float(b)), 1.f) * ONE + 0.5f);
+      };
+      __syncthreads();
+      for (int i = tid; i < KBINS; i += RT) {
+        lds.h.cnt[i] = 0;
+        lds.h.mass[i] = 0;
+      }
+      if (tid < 4) sh_bin[tid] = NONE;
+      __syncthreads();
+      u64 zf = 0;
+      row.each([&](short b, int) {
+        const int hi = KBINS - 1 - (bf16_sort_key(b) >> 4);
+        if (far_k) atomicAdd(&lds.h.cnt[hi], 1u);
+        if (far_p) {
+          const u64 f = fixed(b);
+          zf += f;
+          atomicAdd(&lds.h.mass[hi], f);
+        }
+      });
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) zf += __shfl_xor(zf, off, 64);
+      if (lane == 0) w_fix[wave] = zf;
+      __syncthreads();
+      zf = 0;
+#pragma unroll
+      for (int w = 0; w < NWV; ++w) zf += w_fix[w];
+      __syncthreads();
+      const u64 want_f = max((u64)1, (u64)((double)p * (double)zf));
+      if (far_k)
+        find_bin<KBINS / RT, unsigned int>([&](int i) { return lds.h.cnt[i]; },
+                                           (unsigned int)k, w_cnt, &sh_bin[0],
+                                           &sh_above_k);
+      if (far_p)
+        find_bin<KBINS / RT, u64>([&](int i) { return lds.h.mass[i]; }, want_f,
+                                  w_fix, &sh_bin[1], &sh_above_f);
+      const int bk = sh_bin[0], bp = sh_bin[1];
+      // lower bits inside the two boundary bins
+      row.each([&](short b, int) {
+        const unsigned int key = bf16_sort_key(b);
+        const int hi = KBINS - 1 - (key >> 4);
+        if (hi == bk) atomicAdd(&f_cnt[15 - (key & 15)], 1u);
+        if (hi == bp) atomicAdd(&f_mass[15 - (key & 15)], fixed(b));
+      });
+      __syncthreads();
+      if (bk != NONE) {
+        const unsigned int want = (unsigned int)k - sh_above_k;
+        find_bin<1, unsigned int>([&](int i) { return i < 16 ? f_cnt[i] : 0u; }, want,
+                                  w_cnt, &sh_bin[2], &sh_above_k);
+        thr = ((KBINS - 1 - bk) << 4) | (15 - sh_bin[2]);
+      }
+      if (bp != NONE) {
+        const u64 want = want_f - sh_above_f;
+        find_bin<1, u64>([&](int i) { return i < 16 ? f_mass[i] : (u64)0; }, want,
+                         w_fix, &sh_bin[3], &sh_above_f);
+        thr = max(thr, (unsigned int)((KBINS - 1 - bp) << 4) | (15 - sh_bin[3]));
+      }
+    }
+  }
+
+  // ---- Gumbel-argmax over the surviving set: the lanes of a wave go through
+  // their own survivors, so a sparse set costs few rounds of hash and logs ----
   float best = -1e38f;
   int best_idx = 0;
-  for (int i = tid; i < V; i += 256) {
-    const short b = row[i];
-    if (bf16_sort_key(b) < thr) continue;
-    const unsigned int h = hash2(seed, (unsigned int)i);
-    const float u = ((float)h + 1.0f) * 2.3283064e-10f;
-    const float val = bf16_bits_to_float(b) * inv_t - __logf(-__logf(u));
-    if (val > best) { best = val; best_idx = i; }
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    float ov = __shfl_xor(best, off, 64);
-    int oi = __shfl_xor(best_idx, off, 64);
-    if (ov > best || (ov == best && oi < best_idx)) { best = ov; best_idx = oi; }
-  }
-  if (lane == 0) { s_red[wave] = best; s_redi[wave] = best_idx; }
-  __syncthreads();
-  if (tid == 0) {
-    for (int w = 1; w < 4; ++w) {
-      if (s_red[w] > best || (s_red[w] == best && s_redi[w] < best_idx)) {
-        best = s_red[w];
-        best_idx = s_redi[w];
-      }
+  auto take = [&](short b, int i) {
+    const float val = bf16_bits_to_float(b) * inv_t - gumbel_noise(seed, i);
+    if (val > best || (val == best && i < best_idx)) {
+      best = val;
+      best_idx = i;
     }
-    out[s] = best_idx;
-  }
+  };
+  row.each8(
+      [&](const short8_t& v, int i0) {
+        unsigned int in = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) in |= (bf16_sort_key(v[j]) >= thr ? 1u : 0u) << j;
+        while (in) {
+          const int j = __builtin_ctz(in);
+          in &= in - 1;
+          short b = v[0];
+#pragma unroll
+          for (int q = 1; q < 8; ++q) b = j == q ? v[q] : b;
+          take(b, i0 + j);
+        }
+      },
+      [&](short b, int i) {
+        if (bf16_sort_key(b) >= thr) take(b, i);
+      });
+  block_argmax<RT>(best, best_idx, out + s);
+}
+
+// 1024 threads for rows past 64k elements (256 rows of 128256, greedy 24.7 ->
+// 12.3 us, with noise 36.5 -> 30.8); shorter rows are over before a block that
+// size has merged its waves (256 x 32000, greedy: 5.9 us with 256 threads, 7.0
+// with 1024)
+template <bool GUMBEL>
+void launch_argmax(void* out, const void* logits, const void* temperatures,
+                   const void* seeds, int num_seqs, int vocab, hipStream_t stream) {
+  if (vocab > 65536)
+    hipLaunchKernelGGL((argmax_kernel<GUMBEL, 1024>), dim3(num_seqs), dim3(1024), 0,
+                       stream, (long*)out, (const short*)logits,
+                       (const float*)temperatures, (const long*)seeds, vocab);
+  else
+    hipLaunchKernelGGL((argmax_kernel<GUMBEL, 256>), dim3(num_seqs), dim3(256), 0,
+                       stream, (long*)out, (const short*)logits,
+                       (const float*)temperatures, (const long*)seeds, vocab);
 }
 
 }  // namespace
@@ -347,9 +528,7 @@ hipError_t ks_greedy_sample(void* out, const void* logits, int num_seqs,
     HIP_CHECK_KERNEL();
     return hipSuccess;
   }
-  hipLaunchKernelGGL((argmax_kernel<false>), dim3(num_seqs), dim3(256), 0,
-                     stream, (long*)out, (const short*)logits, nullptr,
-                     nullptr, nullptr, vocab);
+  launch_argmax<false>(out, logits, nullptr, nullptr, num_seqs, vocab, stream);
   HIP_CHECK_KERNEL();
   return hipSuccess;
 }
@@ -359,10 +538,8 @@ hipError_t ks_gumbel_sample(void* out, const void* logits,
                             const void* seeds, int num_seqs, int vocab,
                             hipStream_t stream) {
   if (num_seqs == 0) return hipSuccess;
-  hipLaunchKernelGGL((argmax_kernel<true>), dim3(num_seqs), dim3(256), 0,
-                     stream, (long*)out, (const short*)logits,
-                     (const float*)temperatures, (const int*)top_k,
-                     (const long*)seeds, vocab);
+  // sampling from the whole row: top_k is not read
+  launch_argmax<true>(out, logits, temperatures, seeds, num_seqs, vocab, stream);
   HIP_CHECK_KERNEL();
   return hipSuccess;
 }
@@ -372,7 +549,7 @@ hipError_t ks_topk_topp_sample(void* out, const void* logits,
                                const void* top_k, const void* seeds,
                                int num_seqs, int vocab, hipStream_t stream) {
   if (num_seqs == 0) return hipSuccess;
-  hipLaunchKernelGGL(topk_topp_sample_kernel, dim3(num_seqs), dim3(256), 0,
+  hipLaunchKernelGGL(topk_topp_sample_kernel, dim3(num_seqs), dim3(RT), 0,
                      stream, (long*)out, (const short*)logits,
                      (const float*)temperatures, (const float*)top_p,
                      (const int*)top_k, (const long*)seeds, vocab);

@@ -432,6 +432,68 @@ class TestSampling:
         assert (out1 == out2).all()
 
 
+    @pytest.mark.parametrize("mode", ["model", "flat", "masked", "far_k"])
+    @pytest.mark.parametrize("vocab", [7, 1031, 32000, 65537, 128257])
+    def test_topk_topp_against_fp64(self, dev, vocab, mode):
+        """Thresholds from the 16384-key window (model-like rows), from below
+        it (flat rows, k near the vocabulary) and rows that start at any
+        2-byte boundary: token for token what top-k/top-p and the Gumbel noise
+        of the kernel's hash give in float64."""
+        import kserve_amd_C
+
+        n = 12
+        g = torch.Generator().manual_seed(vocab)
+        logits = (torch.randn(n, vocab, generator=g) * 2.5)
+        top_p = torch.tensor([1.0, 0.9, 0.95, 0.5] * 3)
+        top_k = torch.tensor([0, 50, 1, 0, 5, 0] * 2, dtype=torch.int32)
+        if mode == "flat":
+            logits = logits * 0.01 - 3.0
+            top_p[::2] = 0.999
+        if mode == "masked":
+            logits[:, vocab // 2 + 1:] = float("-inf")
+        if mode == "far_k":
+            top_k[:] = vocab - 1 - vocab // 7
+            top_p[::2], top_p[1::2] = 1.0, 0.99999
+        logits = logits.to(torch.bfloat16)
+        temps = torch.rand(n, generator=g) * 0.6 + 0.6
+        seeds = torch.randint(0, 1 << 31, (n,), generator=g)
+        out = torch.empty(n, dtype=torch.int64, device=dev)
+        kserve_amd_C.topk_topp_sample(
+            out, logits.to(dev), temps.to(dev), top_p.to(dev), top_k.to(dev),
+            seeds.to(dev),
+        )
+        # the kernel's counter hash, in 32-bit arithmetic
+        M = 0xFFFFFFFF
+        idx = torch.arange(vocab, dtype=torch.int64)
+        h = ((seeds[:, None] * 0x9E3779B1) & M) + ((idx * 0x85EBCA77) & M)
+        h = (h + 0x165667B1) & M
+        h = h ^ (h >> 15)
+        h = (h * 0x2C1B3C6D) & M
+        h = h ^ (h >> 12)
+        h = (h * 0x297A2D39) & M
+        h = h ^ (h >> 15)
+        u = (h.float() + 1.0) * 2.3283064e-10
+        x = logits.double() / temps[:, None].double()
+        score = x - torch.log(-torch.log(u.double()))
+        for r in range(n):
+            probs = torch.softmax(x[r], 0)
+            vals, order = x[r].sort(descending=True)
+            least = float("-inf")
+            if 0 < top_k[r] < vocab:
+                least = max(least, float(vals[top_k[r] - 1]))
+            if top_p[r] < 1:
+                c = probs[order].cumsum(0)
+                at = int((c < float(top_p[r])).sum())
+                least = max(least, float(vals[min(at, vocab - 1)]))
+            s = score[r].masked_fill(x[r] < least, float("-inf"))
+            got = int(out[r])
+            # the kernel's noise carries the error of two fast fp32 logarithms
+            # (2e-6 relative of values up to 20): only scores closer than
+            # that may change places
+            assert x[r][got] >= least, (r, got)
+            assert s[got] >= s.max() - 1e-4, (r, got, int(s.argmax()))
+
+
 class TestSkinnyGemm:
     @pytest.mark.parametrize(
         "N,K,M",
