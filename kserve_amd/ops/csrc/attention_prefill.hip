@@ -1,706 +1,403 @@
-// Flash-style causal prefill attention (varlen, GQA) on MFMA.
+// Flash-style prefill attention (bf16, GQA, varlen) on MFMA: rows of the
+// current batch (flash_prefill_varlen) or pages of the KV cache
+// (context_prefill_varlen: chunked prefill, prefix reuse, draft verification).
 //
-// CDNA4 design (guide §5/§B): per workgroup 4 waves x 16 q-rows = 64 q rows
-// of one (seq, head); K/V staged in LDS in 32-token tiles; QK^T and PV on
-// v_mfma_f32_16x16x32_bf16; online softmax on the C-fragment rows; LDS
-// XOR-swizzled (G4) to kill the D=128 row-major bank conflict; V stored
-// transposed at stage time so the PV B-operand reads are contiguous.
+// The tiles are transposed: S^T = K Q^T puts one query per lane column of
+// v_mfma_f32_32x32x16_bf16, so the running maximum, sum and rescale factor are
+// per-lane scalars, and the 16 score registers of a lane are already the B
+// operand of O^T += V^T P^T: the contraction runs over keys in the
+// accumulator's own order (lane half h, element j -> key 4h + j, then
+// 8 + 4h + j of a 16-key chunk), and V is read from its row-major LDS tile in
+// that order by the transposing LDS loads (ds_read_b64_tr_b16). The weights
+// never leave registers.
+//
+// A block is 4 waves of 32 queries and shares double-buffered tiles of 64 keys
+// that the LDS-direct loads fill while the other buffer is computed on; the
+// XOR swizzles below are on the source side of those loads. With several query
+// heads per KV head the waves take up to four heads of one group over the same
+// queries (equal causal ranges, and a K/V tile is fetched once for the group);
+// otherwise consecutive queries of one head.
+//
+// What bounds it: per 64 keys and 32 queries a wave issues 32 MFMAs (1024
+// cycles of its matrix core), reads 32 KB of LDS operands (a quarter of the
+// LDS bandwidth for the same time, times four waves) and has 32 exponentials
+// and about 130 further vector instructions per lane; two waves per SIMD
+// overlap the three. Measured (32 query and 8 KV heads of 128, causal; the
+// 16x16x32 kernel with one head per block, V transposed by 2-byte LDS stores and
+// a barrier on each side of the staging, before this one): 1 x 8191 tokens
+// 2497 -> 652 us (220 -> 843 TFLOP/s), 8 x 2048 1280 -> 387 us, 32 x 512
+// 413 -> 149 us; 2 x 1000 queries over 13000 paged keys 2441 -> 509 us (E4M3
+// pages 2596 -> 625); 64 x 128, 12 heads of 64, bidirectional 28 -> 13 us.
 //
 // Replaces the vLLM flash prefill the reference delegates to
-// (SURVEY.md §2.7 row 1). Numerics oracle: ops/torch_ref.flash_prefill_varlen.
+// (SURVEY.md §2.7 row 1). Numerics oracles: ops/torch_ref.flash_prefill_varlen
+// and context_attention_varlen.
 #include "common.h"
 #include "mfma_layouts.h"
 
-#define NEG_INF (-1e30f)
-
 namespace {
 
-constexpr int KT = 32;        // kv tokens per tile
-constexpr int QW = 16;        // q rows per wave
-constexpr int NWAVES = 4;     // waves per workgroup (64 q rows)
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
 
-// swizzled LDS index helpers (short units)
+constexpr int KT = 64;      // keys per tile
+constexpr int NWAVES = 4;
+constexpr int QW = 32;      // queries per wave
+constexpr float MASKED = -3e38f;
+constexpr float NO_MAX = -1e30f;  // above MASKED: an all-masked tile adds 0
+
+// where K and V rows come from
+enum Src {
+  ROWS_DMA,   // flat rows, 16-byte aligned: loaded straight into LDS
+  ROWS_REG,   // flat rows at any alignment: through registers
+  PAGES_DMA,  // bf16 pages of 16 tokens
+  PAGES_REG,  // bf16 pages at any alignment
+  PAGES_FP8,  // E4M3 pages, widened to bf16 on the way
+};
+
+// 16-byte chunk that chunk c of row r sits at. K fragments: 16 consecutive
+// rows at one chunk must hit different banks; V fragments: 4 consecutive rows
+// of 32 bytes each (a pair of chunks stays a pair).
 template <int D>
-__device__ __forceinline__ int k_idx(int row, int col) {
-  // [32][D] shorts; XOR 8-short chunks with row&7 (D=64: modulo row width)
-  constexpr int MASK = (D / 8) - 1;
-  const int chunk = (col >> 3) ^ ((row & 7) & MASK);
-  return row * D + (chunk << 3) + (col & 7);
+__device__ __forceinline__ int k_swz(int r) {
+  return D == 128 ? (r & 15) : ((r >> 1) & 7);
 }
-__device__ __forceinline__ int v_idx(int d, int tok) {
-  // transposed [128 dims][32 tokens] shorts; XOR 8-short chunks with d&3
-  return d * KT + (tok ^ ((d & 3) << 3));
+template <int D>
+__device__ __forceinline__ int v_swz(int r) {
+  return D == 128 ? (r & 7) << 1 : ((r >> 1) & 3) << 1;
 }
 
-template <int D, bool CAUSAL, bool WIN = false>  // D == 128
-__global__ __launch_bounds__(256) void flash_prefill_kernel(
-    short* __restrict__ out,      // [T, Hq, D] bf16
-    const short* __restrict__ q,  // [T, Hq, D]
-    const short* __restrict__ k,  // [T, Hkv, D]
-    const short* __restrict__ v,  // [T, Hkv, D]
-    const int* __restrict__ cu_seqlens,  // [S+1]
-    const int Hq, const int Hkv, const float scale, const long sq,
-    const long sk, const long sv, const int window) {
-  const int head = blockIdx.x;
-  const int tile = blockIdx.y;
+__device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// larger of a lane's value and its partner's in the other half of the wave
+__device__ __forceinline__ float half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float half_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// eight E4M3 bytes as bf16 (exact)
+__device__ __forceinline__ short8_t widen_fp8(uint2 x) {
+  short8_t o;
+  const unsigned int w[2] = {x.x, x.y};
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const float2_t lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[d], false);
+    const float2_t hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[d], true);
+    o[d * 4 + 0] = float_to_bf16_bits(lo[0]);
+    o[d * 4 + 1] = float_to_bf16_bits(lo[1]);
+    o[d * 4 + 2] = float_to_bf16_bits(hi[0]);
+    o[d * 4 + 3] = float_to_bf16_bits(hi[1]);
+  }
+  return o;
+}
+
+struct PrefillArgs {
+  short* out;         // [T, Hq, D]
+  const short* q;     // [T, Hq, D], row stride sq
+  const void* k;      // [T, Hkv, D] rows (stride sk) or pages [NB, Hkv, 16, D]
+  const void* v;
+  const int* cu_q;          // [S+1]
+  const int* ctx_lens;      // [S] keys of a sequence (pages)
+  const int* block_tables;  // [S, max_nb] (pages)
+  int Hq, Hkv, max_nb;
+  int hpb;  // query heads per block: 1, 2 or 4, divides the group
+  float scale;
+  long sq, sk, sv;
+  int window;
+};
+
+template <int D, int SRC, bool CAUSAL, bool WIN>
+__global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
+    const PrefillArgs p) {
+  constexpr bool PAGED = SRC >= PAGES_DMA;
+  constexpr bool DMA = SRC == ROWS_DMA || SRC == PAGES_DMA;
+  constexpr int CPR = D / 8;          // 16-byte chunks per row
+  constexpr int RPI = 64 / CPR;       // rows per wave-wide 16-byte load
+  constexpr int NI = 16 / RPI;        // such loads per wave and tile (K or V)
+  constexpr int TILE = KT * D;
+  constexpr int KC = D / 16;          // contraction chunks of Q K^T
+  constexpr int DB = D / 32;          // 32-column blocks of the output
+
   const int seq = blockIdx.z;
-  const int q_start = cu_seqlens[seq];
-  const int len = cu_seqlens[seq + 1] - q_start;
-  const int tile_base = tile * (NWAVES * QW);
-  if (tile_base >= len) return;
-  const int group = Hq / Hkv;
-  const int kv_head = head / group;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-
-  __shared__ short k_tile[KT * D];        // 8 KB swizzled
-  __shared__ short v_t[D * KT];           // 8 KB transposed+swizzled
-  __shared__ short p_lds[NWAVES][QW * KT];  // 4 KB
-
-  const int wq0 = tile_base + wave * QW;  // first q row of this wave
-  const bool active = wq0 < len;
-
-  // ---- load Q fragments (A operand), rows clamped to len-1 ----
-  bf16x8_t a_q[D / 32];
-  {
-    const int qrow = min(wq0 + MFMA_RC_OF(lane), len - 1);
-    const short* qp = q + (long)(q_start + qrow) * sq + (long)head * D;
-#pragma unroll
-    for (int c = 0; c < D / 32; ++c) {
-      const int off = c * 32 + ((lane >> 4) << 3);
-      a_q[c] = *reinterpret_cast<const bf16x8_t*>(qp + off);
-    }
-  }
-
-  float m[4], l[4];
-  f32x4_t o_acc[D / 16];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) { m[r] = NEG_INF; l[r] = 0.f; }
-#pragma unroll
-  for (int c = 0; c < D / 16; ++c) o_acc[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  // causal bound: last token needed by this workgroup (bidirectional: all)
-  const int kv_limit = CAUSAL ? min(len, tile_base + NWAVES * QW) : len;
-  const int ntiles = (kv_limit + KT - 1) / KT;
-
-  for (int kt = 0; kt < ntiles; ++kt) {
-    const int t0 = kt * KT;
-    __syncthreads();
-    // ---- stage K tile (swizzled) and V tile (transposed) ----
-    for (int i = threadIdx.x; i < KT * (D / 8); i += 256) {
-      const int r = i / (D / 8);          // token within tile
-      const int c8 = (i % (D / 8)) * 8;   // first dim of this short8
-      const int tok = t0 + r;
-      short8_t val;
-      if (tok < len) {
-        val = *reinterpret_cast<const short8_t*>(
-            k + (long)(q_start + tok) * sk + (long)kv_head * D + c8);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) val[j] = 0;
-      }
-      *reinterpret_cast<short8_t*>(&k_tile[k_idx<D>(r, c8)]) = val;
-      short8_t vv;
-      if (tok < len) {
-        vv = *reinterpret_cast<const short8_t*>(
-            v + (long)(q_start + tok) * sv + (long)kv_head * D + c8);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vv[j] = 0;
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v_t[v_idx(c8 + j, r)] = vv[j];
-    }
-    __syncthreads();
-    if (!active) continue;
-    // causal skip: this wave's rows are all below the tile's first token
-    if (CAUSAL && t0 > wq0 + QW - 1) continue;
-
-    // ---- QK^T: S[16 q][32 t] as 2 sub-tiles of 16 tokens ----
-    f32x4_t s_frag[2] = {f32x4_t{0, 0, 0, 0}, f32x4_t{0, 0, 0, 0}};
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      const int tok_row = n * 16 + MFMA_RC_OF(lane);
-#pragma unroll
-      for (int c = 0; c < D / 32; ++c) {
-        const int col = c * 32 + ((lane >> 4) << 3);
-        bf16x8_t bk =
-            *reinterpret_cast<bf16x8_t*>(&k_tile[k_idx<D>(tok_row, col)]);
-        s_frag[n] = mfma16x16x32(a_q[c], bk, s_frag[n]);
-      }
-    }
-    // ---- mask + online softmax ----
-    float p[2][4];
-    float rescale[4];
-#pragma unroll
-    for (int reg = 0; reg < 4; ++reg) {
-      const int qrow = wq0 + MFMA_C_ROW(lane, reg);
-      float sv[2];
-#pragma unroll
-      for (int n = 0; n < 2; ++n) {
-        const int tok = t0 + n * 16 + MFMA_C_COL(lane);
-        const bool valid =
-            (!CAUSAL || tok <= qrow) && (qrow < len) && (tok < len) &&
-            (!WIN || tok > qrow - window);
-        sv[n] = valid ? s_frag[n][reg] * scale : NEG_INF;
-      }
-      float rowmax = group_reduce_max<16>(fmaxf(sv[0], sv[1]));
-      const float m_new = fmaxf(m[reg], rowmax);
-      rescale[reg] = (m[reg] > NEG_INF && m_new > NEG_INF)
-                         ? __expf(m[reg] - m_new)
-                         : 0.f;
-#pragma unroll
-      for (int n = 0; n < 2; ++n)
-        p[n][reg] = (sv[n] > NEG_INF) ? __expf(sv[n] - m_new) : 0.f;
-      const float rowsum = group_reduce_sum<16>(p[0][reg] + p[1][reg]);
-      l[reg] = l[reg] * rescale[reg] + rowsum;
-      m[reg] = m_new;
-    }
-#pragma unroll
-    for (int c = 0; c < D / 16; ++c) {
-#pragma unroll
-      for (int reg = 0; reg < 4; ++reg) o_acc[c][reg] *= rescale[reg];
-    }
-    // ---- P -> LDS (C layout -> A layout relayout) ----
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-#pragma unroll
-      for (int reg = 0; reg < 4; ++reg) {
-        const int prow = MFMA_C_ROW(lane, reg);
-        const int pcol = n * 16 + MFMA_C_COL(lane);
-        p_lds[wave][prow * KT + pcol] = float_to_bf16_bits(p[n][reg]);
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)");
-    __builtin_amdgcn_sched_barrier(0);  // keep reads after the waitcnt (G#18)
-    // ---- PV: O[16 q][D] += P[16 q][32 t] @ V[32 t][D] ----
-    bf16x8_t pa = *reinterpret_cast<bf16x8_t*>(
-        &p_lds[wave][MFMA_RC_OF(lane) * KT + ((lane >> 4) << 3)]);
-#pragma unroll
-    for (int c = 0; c < D / 16; ++c) {
-      const int d = c * 16 + MFMA_RC_OF(lane);
-      bf16x8_t bv =
-          *reinterpret_cast<bf16x8_t*>(&v_t[v_idx(d, (lane >> 4) << 3)]);
-      o_acc[c] = mfma16x16x32(pa, bv, o_acc[c]);
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)");
-    __builtin_amdgcn_sched_barrier(0);  // p_lds overwritten next iter
-  }
-
-  if (!active) return;
-  // ---- epilogue: normalize and store ----
-  float inv_l[4];
-#pragma unroll
-  for (int reg = 0; reg < 4; ++reg)
-    inv_l[reg] = (l[reg] > 0.f) ? 1.f / l[reg] : 0.f;
-#pragma unroll
-  for (int c = 0; c < D / 16; ++c) {
-#pragma unroll
-    for (int reg = 0; reg < 4; ++reg) {
-      const int qrow = wq0 + MFMA_C_ROW(lane, reg);
-      if (qrow < len) {
-        out[((long)(q_start + qrow) * Hq + head) * D + c * 16 +
-            MFMA_C_COL(lane)] = float_to_bf16_bits(o_acc[c][reg] * inv_l[reg]);
-      }
-    }
-  }
-}
-
-}  // namespace
-
-// ---------------------------------------------------------------------------
-// v2: 32 q-rows per wave (128/wg) x 64-token KV tiles — 4x the MFMA work per
-// barrier of v1 (guide ladder: bigger tiles amortize staging + softmax).
-// D=128 only; v1 stays for D=64 and as the KS_PREFILL_V1 ablation.
-// ---------------------------------------------------------------------------
-namespace {
-
-constexpr int KT2 = 64;   // kv tokens per tile
-constexpr int QW2 = 32;   // q rows per wave
-constexpr int PSTR = 72;  // p_lds row stride (64 + 8 shorts: 2-way banks)
-
-template <int D, bool CAUSAL, bool AS = false, bool WIN = false>
-__global__ __launch_bounds__(256) void flash_prefill_v2_kernel(
-    short* __restrict__ out, const short* __restrict__ q,
-    const short* __restrict__ k, const short* __restrict__ v,
-    const int* __restrict__ cu_seqlens, const int Hq, const int Hkv,
-    const float scale, const long sq, const long sk, const long sv,
-    const int window) {
-  const int head = blockIdx.x;
-  const int tile = blockIdx.y;
-  const int seq = blockIdx.z;
-  const int q_start = cu_seqlens[seq];
-  const int len = cu_seqlens[seq + 1] - q_start;
-  const int tile_base = tile * (NWAVES * QW2);
-  if (tile_base >= len) return;
-  const int group = Hq / Hkv;
-  const int kv_head = head / group;
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-
-  __shared__ short k_tile[KT2 * D];            // 16 KB swizzled
-  __shared__ short v_t[D * KT2];               // 16 KB transposed+swizzled
-  __shared__ short p_lds[NWAVES][QW2 * PSTR];  // 18 KB
-
-  const int wq0 = tile_base + wave * QW2;
-  const bool active = wq0 < len;
-
-  // Q fragments: 2 row-tiles x 4 k-chunks (A operand)
-  bf16x8_t a_q[2][D / 32];
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int qrow = min(wq0 + rt * 16 + MFMA_RC_OF(lane), len - 1);
-    const short* qp = q + (long)(q_start + qrow) * sq + (long)head * D;
-#pragma unroll
-    for (int c = 0; c < D / 32; ++c) {
-      a_q[rt][c] = *reinterpret_cast<const bf16x8_t*>(
-          qp + c * 32 + ((lane >> 4) << 3));
-    }
-  }
-
-  float m[2][4], l[2][4];
-  f32x4_t o_acc[2][D / 16];
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      m[rt][r] = NEG_INF;
-      l[rt][r] = 0.f;
-    }
-#pragma unroll
-    for (int c = 0; c < D / 16; ++c)
-      o_acc[rt][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-
-  const int kv_limit = CAUSAL ? min(len, tile_base + NWAVES * QW2) : len;
-  const int ntiles = (kv_limit + KT2 - 1) / KT2;
-
-  // T14 async-stage split (guide: +17% attn): the NEXT tile's K/V global
-  // loads are ISSUED into registers during this tile's compute; the
-  // ds_writes land after the barrier, so HBM latency hides under the
-  // MFMA phase instead of serializing the staging loop.
-  constexpr int CHUNKS = AS ? (KT2 * (D / 8) + 255) / 256 : 1;
-  short8_t kreg[CHUNKS], vreg[CHUNKS];
-  auto issue_tile = [&](int tt0) {
-#pragma unroll
-    for (int n = 0; n < CHUNKS; ++n) {
-      const int i = threadIdx.x + n * 256;
-      const int r = i / (D / 8);
-      const int c8 = (i % (D / 8)) * 8;
-      const int tok = tt0 + r;
-      if (tok < len) {
-        kreg[n] = *reinterpret_cast<const short8_t*>(
-            k + (long)(q_start + tok) * sk + (long)kv_head * D + c8);
-        vreg[n] = *reinterpret_cast<const short8_t*>(
-            v + (long)(q_start + tok) * sv + (long)kv_head * D + c8);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          kreg[n][j] = 0;
-          vreg[n][j] = 0;
-        }
-      }
-    }
-  };
-  auto commit_tile = [&]() {
-#pragma unroll
-    for (int n = 0; n < CHUNKS; ++n) {
-      const int i = threadIdx.x + n * 256;
-      const int r = i / (D / 8);
-      const int c8 = (i % (D / 8)) * 8;
-      *reinterpret_cast<short8_t*>(&k_tile[k_idx<D>(r, c8)]) = kreg[n];
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        v_t[(c8 + j) * KT2 + (r ^ (((c8 + j) & 3) << 3))] = vreg[n][j];
-    }
-  };
-  if constexpr (AS) issue_tile(0);
-
-  for (int kt = 0; kt < ntiles; ++kt) {
-    const int t0 = kt * KT2;
-    __syncthreads();
-    if constexpr (AS) {
-      commit_tile();
-      __syncthreads();
-      if (kt + 1 < ntiles) issue_tile(t0 + KT2);
-    } else {
-      for (int i = threadIdx.x; i < KT2 * (D / 8); i += 256) {
-        const int r = i / (D / 8);
-        const int c8 = (i % (D / 8)) * 8;
-        const int tok = t0 + r;
-        short8_t val, vv;
-        if (tok < len) {
-          val = *reinterpret_cast<const short8_t*>(
-              k + (long)(q_start + tok) * sk + (long)kv_head * D + c8);
-          vv = *reinterpret_cast<const short8_t*>(
-              v + (long)(q_start + tok) * sv + (long)kv_head * D + c8);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            val[j] = 0;
-            vv[j] = 0;
-          }
-        }
-        *reinterpret_cast<short8_t*>(&k_tile[k_idx<D>(r, c8)]) = val;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v_t[(c8 + j) * KT2 + (r ^ (((c8 + j) & 3) << 3))] = vv[j];
-      }
-      __syncthreads();
-    }
-    if (!active) continue;
-    if (CAUSAL && t0 > wq0 + QW2 - 1) continue;
-
-    // ---- per row-tile: QK^T over 4 token sub-tiles, online softmax ----
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      const int rbase = wq0 + rt * 16;
-      if (CAUSAL && t0 > rbase + 15) continue;  // fully-masked row-tile
-      f32x4_t s_frag[KT2 / 16];
-#pragma unroll
-      for (int n = 0; n < KT2 / 16; ++n) {
-        s_frag[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        const int tok_row = n * 16 + MFMA_RC_OF(lane);
-#pragma unroll
-        for (int c = 0; c < D / 32; ++c) {
-          const int col = c * 32 + ((lane >> 4) << 3);
-          bf16x8_t bk =
-              *reinterpret_cast<bf16x8_t*>(&k_tile[k_idx<D>(tok_row, col)]);
-          s_frag[n] = mfma16x16x32(a_q[rt][c], bk, s_frag[n]);
-        }
-      }
-      float p[KT2 / 16][4];
-      float rescale[4];
-#pragma unroll
-      for (int reg = 0; reg < 4; ++reg) {
-        const int qrow = rbase + MFMA_C_ROW(lane, reg);
-        float rowmax = NEG_INF;
-        float sv_[KT2 / 16];
-#pragma unroll
-        for (int n = 0; n < KT2 / 16; ++n) {
-          const int tok = t0 + n * 16 + MFMA_C_COL(lane);
-          const bool valid =
-              (!CAUSAL || tok <= qrow) && (qrow < len) && (tok < len) &&
-              (!WIN || tok > qrow - window);
-          sv_[n] = valid ? s_frag[n][reg] * scale : NEG_INF;
-          rowmax = fmaxf(rowmax, sv_[n]);
-        }
-        rowmax = group_reduce_max<16>(rowmax);
-        const float m_new = fmaxf(m[rt][reg], rowmax);
-        rescale[reg] = (m[rt][reg] > NEG_INF && m_new > NEG_INF)
-                           ? __expf(m[rt][reg] - m_new)
-                           : 0.f;
-        float psum = 0.f;
-#pragma unroll
-        for (int n = 0; n < KT2 / 16; ++n) {
-          p[n][reg] = (sv_[n] > NEG_INF) ? __expf(sv_[n] - m_new) : 0.f;
-          psum += p[n][reg];
-        }
-        psum = group_reduce_sum<16>(psum);
-        l[rt][reg] = l[rt][reg] * rescale[reg] + psum;
-        m[rt][reg] = m_new;
-      }
-#pragma unroll
-      for (int c = 0; c < D / 16; ++c) {
-#pragma unroll
-        for (int reg = 0; reg < 4; ++reg) o_acc[rt][c][reg] *= rescale[reg];
-      }
-#pragma unroll
-      for (int n = 0; n < KT2 / 16; ++n) {
-#pragma unroll
-        for (int reg = 0; reg < 4; ++reg) {
-          p_lds[wave][(rt * 16 + MFMA_C_ROW(lane, reg)) * PSTR + n * 16 +
-                      MFMA_C_COL(lane)] = float_to_bf16_bits(p[n][reg]);
-        }
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)");
-    __builtin_amdgcn_sched_barrier(0);
-    // ---- PV: O[32 q][D] += P[32 q][64 t] @ V[64 t][D] ----
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      if (CAUSAL && t0 > wq0 + rt * 16 + 15) continue;
-#pragma unroll
-      for (int kk = 0; kk < KT2 / 32; ++kk) {
-        bf16x8_t pa = *reinterpret_cast<bf16x8_t*>(
-            &p_lds[wave][(rt * 16 + MFMA_RC_OF(lane)) * PSTR + kk * 32 +
-                         ((lane >> 4) << 3)]);
-#pragma unroll
-        for (int c = 0; c < D / 16; ++c) {
-          const int d = c * 16 + MFMA_RC_OF(lane);
-          const int tok0 = kk * 32 + ((lane >> 4) << 3);
-          bf16x8_t bv = *reinterpret_cast<bf16x8_t*>(
-              &v_t[d * KT2 + (tok0 ^ ((d & 3) << 3))]);
-          o_acc[rt][c] = mfma16x16x32(pa, bv, o_acc[rt][c]);
-        }
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)");
-    __builtin_amdgcn_sched_barrier(0);
-  }
-
-  if (!active) return;
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    float inv_l[4];
-#pragma unroll
-    for (int reg = 0; reg < 4; ++reg)
-      inv_l[reg] = (l[rt][reg] > 0.f) ? 1.f / l[rt][reg] : 0.f;
-#pragma unroll
-    for (int c = 0; c < D / 16; ++c) {
-#pragma unroll
-      for (int reg = 0; reg < 4; ++reg) {
-        const int qrow = wq0 + rt * 16 + MFMA_C_ROW(lane, reg);
-        if (qrow < len) {
-          out[((long)(q_start + qrow) * Hq + head) * D + c * 16 +
-              MFMA_C_COL(lane)] =
-              float_to_bf16_bits(o_acc[rt][c][reg] * inv_l[reg]);
-        }
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Paged-context prefill (chunked prefill): the chunk's q rows attend causally
-// to the WHOLE context — previous chunks' KV plus this chunk's — read from
-// the paged cache (the chunk's KV was written by reshape_and_cache first).
-// Same MFMA/LDS structure as v2; staging gathers 64-token tiles as 4
-// contiguous 16xD pages via the block table. Reference parity: the chunked
-// prefill path of the vLLM backend the reference delegates to.
-// Numerics oracle: ops/torch_ref.context_attention_varlen.
-// ---------------------------------------------------------------------------
-// CT: cache element type — short (bf16) or unsigned char (fp8 E4M3,
-// converted to bf16 during LDS staging; MFMA math stays bf16)
-template <int D, typename CT = short, bool WIN = false>  // D == 128
-__global__ __launch_bounds__(256) void context_prefill_kernel(
-    short* __restrict__ out,        // [Tq, Hq, D] bf16
-    const short* __restrict__ q,    // [Tq, Hq, D] (row stride sq)
-    const CT* __restrict__ k_cache,  // [NB, Hkv, 16, D]
-    const CT* __restrict__ v_cache,
-    const int* __restrict__ block_tables,  // [S, max_nb]
-    const int* __restrict__ ctx_lens,      // [S] total context incl. chunk
-    const int* __restrict__ cu_seqlens_q,  // [S+1]
-    const int Hq, const int Hkv, const int max_nb, const float scale,
-    const long sq, const int window) {
-  const int head = blockIdx.x;
-  const int tile = blockIdx.y;
-  const int seq = blockIdx.z;
-  const int q_start = cu_seqlens_q[seq];
-  const int q_len = cu_seqlens_q[seq + 1] - q_start;
-  const int ctx = ctx_lens[seq];
-  const int start_pos = ctx - q_len;  // absolute position of chunk row 0
-  const int tile_base = tile * (NWAVES * QW2);
+  const int q_start = p.cu_q[seq];
+  const int q_len = p.cu_q[seq + 1] - q_start;
+  const int qpb = NWAVES * QW / p.hpb;  // queries per block
+  // the last tiles have the most keys: they start first
+  const int tile_base = (gridDim.y - 1 - blockIdx.y) * qpb;
   if (tile_base >= q_len) return;
-  const int group = Hq / Hkv;
-  const int kv_head = head / group;
+  const int len = PAGED ? p.ctx_lens[seq] : q_len;  // keys
+  const int start_pos = len - q_len;                // position of query 0
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int* bt = block_tables + (long)seq * max_nb;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int head = blockIdx.x * p.hpb + wave % p.hpb;
+  const int kvh = blockIdx.x * p.hpb / (p.Hq / p.Hkv);
+  const int q0 = tile_base + wave / p.hpb * QW;  // the wave's first query
+  const int half = lane >> 5;
 
-  __shared__ short k_tile[KT2 * D];
-  __shared__ short v_t[D * KT2];
-  __shared__ short p_lds[NWAVES][QW2 * PSTR];
+  __shared__ __attribute__((aligned(16))) short lds[2][2][TILE];  // [buffer][K, V]
 
-  const int wq0 = tile_base + wave * QW2;
-  const bool active = wq0 < q_len;
-
-  bf16x8_t a_q[2][D / 32];
+  // ---- queries: B operands, 8 consecutive columns per lane ----
+  bf16x8_t qf[KC];
+  {
+    const int qrow = min(q0 + (lane & 31), q_len - 1);
+    const short* qp = p.q + (long)(q_start + qrow) * p.sq + (long)head * D + half * 8;
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    const int qrow = min(wq0 + rt * 16 + MFMA_RC_OF(lane), q_len - 1);
-    const short* qp = q + (long)(q_start + qrow) * sq + (long)head * D;
-#pragma unroll
-    for (int c = 0; c < D / 32; ++c) {
-      a_q[rt][c] = *reinterpret_cast<const bf16x8_t*>(
-          qp + c * 32 + ((lane >> 4) << 3));
-    }
+    for (int c = 0; c < KC; ++c)
+      qf[c] = *reinterpret_cast<const bf16x8_t*>(qp + c * 16);
   }
 
-  float m[2][4], l[2][4];
-  f32x4_t o_acc[2][D / 16];
-#pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      m[rt][r] = NEG_INF;
-      l[rt][r] = 0.f;
+  // ---- key range ----
+  const int last_q = min(tile_base + qpb, q_len) - 1;
+  const int hi = CAUSAL ? min(len, start_pos + last_q + 1) : len;
+  const int lo = WIN ? max(0, start_pos + tile_base - p.window + 1) : 0;
+  const int t_lo = lo / KT;
+  const int t_hi = (hi + KT - 1) / KT;
+  const int pos_lo = start_pos + q0;
+  const int pos_hi = start_pos + min(q0 + QW, q_len) - 1;
+  const int my_pos = start_pos + q0 + (lane & 31);
+
+  // ---- staging: wave w brings rows 16 w .. 16 w + 15 of a tile (one page);
+  // rows past the keys repeat the last one (their weights are 0, their values
+  // finite) ----
+  const int* bt = PAGED ? p.block_tables + (long)seq * p.max_nb : nullptr;
+  const int lrow = lane / CPR, lchunk = lane % CPR;
+  auto group_of = [&](int t) { return min(t * KT + wave * 16, len - 1); };
+  auto page_of = [&](int t) { return PAGED ? bt[group_of(t) >> 4] : 0; };
+  // address of this lane's chunk (c, already unswizzled) of row r of tile t
+  auto src = [&](const void* base, long stride, int t, int page, int r, int c) {
+    const int g0 = PAGED ? group_of(t) & ~15 : group_of(t);
+    const int row = min(r, len - 1 - g0);
+    if constexpr (PAGED) {
+      constexpr int ES = SRC == PAGES_FP8 ? 1 : 2;
+      return reinterpret_cast<const char*>(base) +
+             ((long)page * p.Hkv + kvh) * (16 * D * ES) + (row * D + c * 8) * ES;
+    } else {
+      return reinterpret_cast<const char*>(base) +
+             ((long)(q_start + g0) * stride + (long)kvh * D) * 2 +
+             (long)row * stride * 2 + c * 16;
     }
+  };
+  uint2 raw8[SRC == PAGES_FP8 ? 2 * NI : 1];
+  short8_t raw16[!DMA && SRC != PAGES_FP8 ? 2 * NI : 1];
+  // DMA: fills buffer `buf`; otherwise the rows wait in registers for commit()
+  auto stage = [&](int t, int page, int buf) {
 #pragma unroll
-    for (int c = 0; c < D / 16; ++c)
-      o_acc[rt][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-
-  // causal bound in ABSOLUTE positions: last key this workgroup's rows see
-  const int kv_limit =
-      min(ctx, start_pos + tile_base + NWAVES * QW2);
-  const int ntiles = (kv_limit + KT2 - 1) / KT2;
-
-  for (int kt = 0; kt < ntiles; ++kt) {
-    const int t0 = kt * KT2;
-    __syncthreads();
-    // stage 64 context tokens = 4 pages of 16, gathered via the block table
-    for (int i = threadIdx.x; i < KT2 * (D / 8); i += 256) {
-      const int r = i / (D / 8);
-      const int c8 = (i % (D / 8)) * 8;
-      const int tok = t0 + r;
-      short8_t val, vv;
-      if (tok < ctx) {
-        const long base =
-            (((long)bt[tok >> 4] * Hkv + kv_head) * 16 + (tok & 15)) * D + c8;
-        if constexpr (sizeof(CT) == 2) {
-          val = *reinterpret_cast<const short8_t*>(k_cache + base);
-          vv = *reinterpret_cast<const short8_t*>(v_cache + base);
-        } else {
-          // fp8: 8 bytes -> 8 bf16 via two packed converts per dword
-          const unsigned int k2[2] = {
-              reinterpret_cast<const unsigned int*>(k_cache + base)[0],
-              reinterpret_cast<const unsigned int*>(k_cache + base)[1]};
-          const unsigned int v2[2] = {
-              reinterpret_cast<const unsigned int*>(v_cache + base)[0],
-              reinterpret_cast<const unsigned int*>(v_cache + base)[1]};
-#pragma unroll
-          for (int d = 0; d < 2; ++d) {
-            const float2_t klo =
-                __builtin_amdgcn_cvt_pk_f32_fp8((int)k2[d], false);
-            const float2_t khi =
-                __builtin_amdgcn_cvt_pk_f32_fp8((int)k2[d], true);
-            const float2_t vlo =
-                __builtin_amdgcn_cvt_pk_f32_fp8((int)v2[d], false);
-            const float2_t vhi =
-                __builtin_amdgcn_cvt_pk_f32_fp8((int)v2[d], true);
-            val[d * 4 + 0] = float_to_bf16_bits(klo[0]);
-            val[d * 4 + 1] = float_to_bf16_bits(klo[1]);
-            val[d * 4 + 2] = float_to_bf16_bits(khi[0]);
-            val[d * 4 + 3] = float_to_bf16_bits(khi[1]);
-            vv[d * 4 + 0] = float_to_bf16_bits(vlo[0]);
-            vv[d * 4 + 1] = float_to_bf16_bits(vlo[1]);
-            vv[d * 4 + 2] = float_to_bf16_bits(vhi[0]);
-            vv[d * 4 + 3] = float_to_bf16_bits(vhi[1]);
-          }
-        }
+    for (int i = 0; i < NI; ++i) {
+      const int r = i * RPI + lrow;
+      const char* ks = src(p.k, p.sk, t, page, r, lchunk ^ k_swz<D>(r));
+      const char* vs = src(p.v, p.sv, t, page, r, lchunk ^ v_swz<D>(r));
+      if constexpr (DMA) {
+        const int at = (wave * 16 + i * RPI) * D;
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const unsigned int*>(ks),
+            reinterpret_cast<unsigned int*>(&lds[buf][0][at]), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const unsigned int*>(vs),
+            reinterpret_cast<unsigned int*>(&lds[buf][1][at]), 16, 0, 0);
+      } else if constexpr (SRC == PAGES_FP8) {
+        raw8[2 * i] = *reinterpret_cast<const uint2*>(ks);
+        raw8[2 * i + 1] = *reinterpret_cast<const uint2*>(vs);
       } else {
+        raw16[2 * i] = *reinterpret_cast<const short8_t*>(ks);
+        raw16[2 * i + 1] = *reinterpret_cast<const short8_t*>(vs);
+      }
+    }
+  };
+  auto commit = [&](int buf) {
+    if constexpr (!DMA) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          val[j] = 0;
-          vv[j] = 0;
+      for (int i = 0; i < NI; ++i) {
+        const int at = (wave * 16 + i * RPI) * D + lane * 8;
+#pragma unroll
+        for (int kv = 0; kv < 2; ++kv) {
+          short8_t x;
+          if constexpr (SRC == PAGES_FP8) x = widen_fp8(raw8[2 * i + kv]);
+          else x = raw16[2 * i + kv];
+          *reinterpret_cast<short8_t*>(&lds[buf][kv][at]) = x;
         }
       }
-      *reinterpret_cast<short8_t*>(&k_tile[k_idx<D>(r, c8)]) = val;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        v_t[(c8 + j) * KT2 + (r ^ (((c8 + j) & 3) << 3))] = vv[j];
     }
+  };
+
+  // ---- operand addresses inside a tile (elements) ----
+  const int krow = lane & 31;
+  int kaddr[KC];
+#pragma unroll
+  for (int c = 0; c < KC; ++c)
+    kaddr[c] = krow * D + ((2 * c + half) ^ k_swz<D>(krow)) * 8;
+  // transposing load: lane i of 16 brings key i/4, columns 4 (i%4) .. + 3 of a
+  // 4 x 16 block and receives column i of its four keys
+  const int ti = lane & 15;
+  const int vrow = half * 4 + (ti >> 2);
+  int vaddr[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+    vaddr[b] = vrow * D +
+               (((4 * b + ((lane >> 4) & 1) * 2 + ((ti & 3) >> 1)) ^ v_swz<D>(vrow)) * 8) +
+               (ti & 1) * 4;
+
+  float c2 = p.scale * 1.44269504088896340736f;
+  const bool flip = c2 < 0.f;
+  c2 = fabsf(c2);
+  float m = NO_MAX, l = 0.f;
+  f32x16_t o[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[b][r] = 0.f;
+
+  if (t_lo < t_hi) stage(t_lo, page_of(t_lo), 0);
+  int page = t_lo + 1 < t_hi ? page_of(t_lo + 1) : 0;
+  commit(0);
+
+  for (int t = t_lo; t < t_hi; ++t) {
+    const int buf = (t - t_lo) & 1;
     __syncthreads();
-    if (!active) continue;
-    // wave-level causal skip: first key of tile past this wave's last q pos
-    if (t0 > start_pos + wq0 + QW2 - 1) continue;
-
-#pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      const int rbase = wq0 + rt * 16;
-      if (t0 > start_pos + rbase + 15) continue;
-      f32x4_t s_frag[KT2 / 16];
-#pragma unroll
-      for (int n = 0; n < KT2 / 16; ++n) {
-        s_frag[n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        const int tok_row = n * 16 + MFMA_RC_OF(lane);
-#pragma unroll
-        for (int c = 0; c < D / 32; ++c) {
-          const int col = c * 32 + ((lane >> 4) << 3);
-          bf16x8_t bk =
-              *reinterpret_cast<bf16x8_t*>(&k_tile[k_idx<D>(tok_row, col)]);
-          s_frag[n] = mfma16x16x32(a_q[rt][c], bk, s_frag[n]);
-        }
-      }
-      float p[KT2 / 16][4];
-      float rescale[4];
-#pragma unroll
-      for (int reg = 0; reg < 4; ++reg) {
-        const int qrow = rbase + MFMA_C_ROW(lane, reg);
-        const int qpos = start_pos + qrow;
-        float rowmax = NEG_INF;
-        float sv_[KT2 / 16];
-#pragma unroll
-        for (int n = 0; n < KT2 / 16; ++n) {
-          const int tok = t0 + n * 16 + MFMA_C_COL(lane);
-          const bool valid = (tok <= qpos) && (qrow < q_len) && (tok < ctx) &&
-                             (!WIN || tok > qpos - window);
-          sv_[n] = valid ? s_frag[n][reg] * scale : NEG_INF;
-          rowmax = fmaxf(rowmax, sv_[n]);
-        }
-        rowmax = group_reduce_max<16>(rowmax);
-        const float m_new = fmaxf(m[rt][reg], rowmax);
-        rescale[reg] = (m[rt][reg] > NEG_INF && m_new > NEG_INF)
-                           ? __expf(m[rt][reg] - m_new)
-                           : 0.f;
-        float psum = 0.f;
-#pragma unroll
-        for (int n = 0; n < KT2 / 16; ++n) {
-          p[n][reg] = (sv_[n] > NEG_INF) ? __expf(sv_[n] - m_new) : 0.f;
-          psum += p[n][reg];
-        }
-        psum = group_reduce_sum<16>(psum);
-        l[rt][reg] = l[rt][reg] * rescale[reg] + psum;
-        m[rt][reg] = m_new;
-      }
-#pragma unroll
-      for (int c = 0; c < D / 16; ++c) {
-#pragma unroll
-        for (int reg = 0; reg < 4; ++reg) o_acc[rt][c][reg] *= rescale[reg];
-      }
-#pragma unroll
-      for (int n = 0; n < KT2 / 16; ++n) {
-#pragma unroll
-        for (int reg = 0; reg < 4; ++reg) {
-          p_lds[wave][(rt * 16 + MFMA_C_ROW(lane, reg)) * PSTR + n * 16 +
-                      MFMA_C_COL(lane)] = float_to_bf16_bits(p[n][reg]);
-        }
-      }
+    if (t + 1 < t_hi) {
+      stage(t + 1, page, buf ^ 1);
+      if (PAGED && t + 2 < t_hi) page = page_of(t + 2);
     }
-    asm volatile("s_waitcnt lgkmcnt(0)");
-    __builtin_amdgcn_sched_barrier(0);
+    const int t0 = t * KT;
+    const bool mine = q0 < q_len && (!CAUSAL || t0 <= pos_hi) &&
+                      (!WIN || t0 + KT - 1 > pos_lo - p.window);
+    if (mine) {
+      const short* kt = lds[buf][0];
+      const short* vt = lds[buf][1];
+      f32x16_t s[2];
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      if (t0 > start_pos + wq0 + rt * 16 + 15) continue;
+      for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
-      for (int kk = 0; kk < KT2 / 32; ++kk) {
-        bf16x8_t pa = *reinterpret_cast<bf16x8_t*>(
-            &p_lds[wave][(rt * 16 + MFMA_RC_OF(lane)) * PSTR + kk * 32 +
-                         ((lane >> 4) << 3)]);
+        for (int r = 0; r < 16; ++r) s[kb][r] = 0.f;
 #pragma unroll
-        for (int c = 0; c < D / 16; ++c) {
-          const int d = c * 16 + MFMA_RC_OF(lane);
-          const int tok0 = kk * 32 + ((lane >> 4) << 3);
-          bf16x8_t bv = *reinterpret_cast<bf16x8_t*>(
-              &v_t[d * KT2 + (tok0 ^ ((d & 3) << 3))]);
-          o_acc[rt][c] = mfma16x16x32(pa, bv, o_acc[rt][c]);
+        for (int c = 0; c < KC; ++c) {
+          const bf16x8_t a =
+              *reinterpret_cast<const bf16x8_t*>(kt + kb * 32 * D + kaddr[c]);
+          s[kb] = mfma32(a, qf[c], s[kb]);
         }
       }
+      if (flip) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) s[kb] = -s[kb];
+      }
+      // register r of block kb: key 32 kb + (r & 3) + 8 (r / 4) + 4 half
+      if (t0 + KT > len || (CAUSAL && t0 + KT - 1 > pos_lo) ||
+          (WIN && t0 <= pos_hi - p.window)) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = t0 + 32 * kb + (r & 3) + 8 * (r >> 2) + 4 * half;
+            const bool ok = key < len && (!CAUSAL || key <= my_pos) &&
+                            (!WIN || key > my_pos - p.window);
+            s[kb][r] = ok ? s[kb][r] : MASKED;
+          }
+      }
+      float mx = s[0][0];
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
+      mx = half_max(mx);
+      if (__any(mx > m)) {
+        const float mn = fmaxf(m, mx);
+        const float f = __builtin_amdgcn_exp2f((m - mn) * c2);
+        m = mn;
+        l *= f;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[b][r] *= f;
+      }
+      const float mc = m * c2;
+      bf16x8_t pf[KT / 16];
+      float sum = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float w = __builtin_amdgcn_exp2f(s[kb][r] * c2 - mc);
+          sum += w;
+          pf[kb * 2 + (r >> 3)][r & 7] = (__bf16)w;
+        }
+      l += sum;
+#pragma unroll
+      for (int kc = 0; kc < KT / 16; ++kc)
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+          typedef __attribute__((address_space(3))) s16x4_t lds4_t;
+          const short* a0 = vt + kc * 16 * D + vaddr[b];
+          const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)a0);
+          const s16x4_t v1 =
+              __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)(a0 + 8 * D));
+          union {
+            s16x4_t h[2];
+            bf16x8_t v;
+          } a;
+          a.h[0] = v0;
+          a.h[1] = v1;
+          o[b] = mfma32(a.v, pf[kc], o[b]);
+        }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)");
-    __builtin_amdgcn_sched_barrier(0);
+    if (t + 1 < t_hi) commit(buf ^ 1);
   }
 
-  if (!active) return;
+  if (q0 >= q_len) return;
+  const int qrow = q0 + (lane & 31);
+  l = half_sum(l);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (qrow < q_len) {
+    short* op = p.out + ((long)(q_start + qrow) * p.Hq + head) * D + half * 4;
 #pragma unroll
-  for (int rt = 0; rt < 2; ++rt) {
-    float inv_l[4];
+    for (int b = 0; b < DB; ++b)
 #pragma unroll
-    for (int reg = 0; reg < 4; ++reg)
-      inv_l[reg] = (l[rt][reg] > 0.f) ? 1.f / l[rt][reg] : 0.f;
+      for (int g = 0; g < 4; ++g) {
+        short4_t w;
 #pragma unroll
-    for (int c = 0; c < D / 16; ++c) {
-#pragma unroll
-      for (int reg = 0; reg < 4; ++reg) {
-        const int qrow = wq0 + rt * 16 + MFMA_C_ROW(lane, reg);
-        if (qrow < q_len) {
-          out[((long)(q_start + qrow) * Hq + head) * D + c * 16 +
-              MFMA_C_COL(lane)] =
-              float_to_bf16_bits(o_acc[rt][c][reg] * inv_l[reg]);
-        }
+        for (int r = 0; r < 4; ++r) w[r] = float_to_bf16_bits(o[b][g * 4 + r] * inv);
+        *reinterpret_cast<short4_t*>(op + b * 32 + g * 8) = w;
       }
-    }
   }
+}
+
+template <int D, int SRC>
+hipError_t launch(PrefillArgs p, int num_seqs, int max_q_len, bool causal,
+                  hipStream_t stream) {
+  const int group = p.Hq / p.Hkv;
+  p.hpb = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+  const int qpb = NWAVES * QW / p.hpb;
+  const int tiles = (max_q_len + qpb - 1) / qpb;
+  if (tiles == 0 || num_seqs == 0) return hipSuccess;
+  const dim3 grid(p.Hq / p.hpb, tiles, num_seqs);
+#define GO(CC, WW)                                                             \
+  hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, CC, WW>), grid,         \
+                     dim3(256), 0, stream, p)
+  const bool win = p.window > 0;
+  if constexpr (SRC >= PAGES_DMA) {
+    if (win) GO(true, true);
+    else GO(true, false);
+  } else if (causal) {
+    if (win) GO(true, true);
+    else GO(true, false);
+  } else {
+    if (win) GO(false, true);
+    else GO(false, false);
+  }
+#undef GO
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
+}
+
+bool aligned16(const void* a, const void* b) {
+  return (((uintptr_t)a | (uintptr_t)b) & 15) == 0;
 }
 
 }  // namespace
@@ -712,27 +409,14 @@ extern "C" hipError_t ks_context_prefill_varlen(
     float scale, long sq, int fp8_cache, int window, hipStream_t stream) {
   if (head_dim != 128) return hipErrorInvalidValue;
   if (Hq % Hkv != 0) return hipErrorInvalidValue;
-  const int max_tiles = (max_q_len + NWAVES * QW2 - 1) / (NWAVES * QW2);
-  if (max_tiles == 0 || num_seqs == 0) return hipSuccess;
-  dim3 grid(Hq, max_tiles, num_seqs);
-#define LAUNCH_CTX(CT, WW)                                                  \
-  hipLaunchKernelGGL((context_prefill_kernel<128, CT, WW>), grid,           \
-                     dim3(256), 0, stream, (short*)out, (const short*)q,    \
-                     (const CT*)k_cache, (const CT*)v_cache,                \
-                     (const int*)block_tables, (const int*)ctx_lens,        \
-                     (const int*)cu_seqlens_q, Hq, Hkv, max_nb, scale, sq,  \
-                     window)
-  const bool winc = window > 0;
-  if (fp8_cache) {
-    if (winc) LAUNCH_CTX(unsigned char, true);
-    else LAUNCH_CTX(unsigned char, false);
-  } else {
-    if (winc) LAUNCH_CTX(short, true);
-    else LAUNCH_CTX(short, false);
-  }
-#undef LAUNCH_CTX
-  HIP_CHECK_KERNEL();
-  return hipSuccess;
+  PrefillArgs p{(short*)out, (const short*)q, k_cache, v_cache,
+                (const int*)cu_seqlens_q, (const int*)ctx_lens,
+                (const int*)block_tables, Hq, Hkv, max_nb, 1, scale, sq, 0, 0,
+                window};
+  if (fp8_cache) return launch<128, PAGES_FP8>(p, num_seqs, max_q_len, true, stream);
+  if (aligned16(k_cache, v_cache))
+    return launch<128, PAGES_DMA>(p, num_seqs, max_q_len, true, stream);
+  return launch<128, PAGES_REG>(p, num_seqs, max_q_len, true, stream);
 }
 
 extern "C" hipError_t ks_flash_prefill_varlen(
@@ -742,60 +426,14 @@ extern "C" hipError_t ks_flash_prefill_varlen(
     int window, hipStream_t stream) {
   if (head_dim != 128 && head_dim != 64) return hipErrorInvalidValue;
   if (Hq % Hkv != 0) return hipErrorInvalidValue;
-  const int max_tiles = (max_seqlen + NWAVES * QW - 1) / (NWAVES * QW);
-  if (max_tiles == 0 || num_seqs == 0) return hipSuccess;
-  dim3 grid(Hq, max_tiles, num_seqs);
-  // v2 (32 q-rows/wave, 64-token tiles) for D=128; KS_PREFILL_V1=1 reverts
-  static const bool use_v1 = [] {
-    const char* e = getenv("KS_PREFILL_V1");
-    return e != nullptr && e[0] == '1';
-  }();
-  if (head_dim == 128 && !use_v1) {
-    const int max_tiles2 = (max_seqlen + NWAVES * QW2 - 1) / (NWAVES * QW2);
-    dim3 grid2(Hq, max_tiles2, num_seqs);
-    static const bool use_as = [] {  // T14 A/B: KS_PREFILL_AS=1
-      const char* e = getenv("KS_PREFILL_AS");
-      return e != nullptr && e[0] == '1';
-    }();
-#define LAUNCH_FP2(CC, AA, WW)                                              \
-  hipLaunchKernelGGL((flash_prefill_v2_kernel<128, CC, AA, WW>), grid2,     \
-                     dim3(256), 0, stream, (short*)out, (const short*)q,    \
-                     (const short*)k, (const short*)v,                      \
-                     (const int*)cu_seqlens, Hq, Hkv, scale, sq, sk, sv,    \
-                     window)
-    const bool win = window > 0;
-    if (causal && use_as) {
-      if (win) LAUNCH_FP2(true, true, true);
-      else LAUNCH_FP2(true, true, false);
-    } else if (causal) {
-      if (win) LAUNCH_FP2(true, false, true);
-      else LAUNCH_FP2(true, false, false);
-    } else if (use_as) {
-      if (win) LAUNCH_FP2(false, true, true);
-      else LAUNCH_FP2(false, true, false);
-    } else {
-      if (win) LAUNCH_FP2(false, false, true);
-      else LAUNCH_FP2(false, false, false);
-    }
-#undef LAUNCH_FP2
-    HIP_CHECK_KERNEL();
-    return hipSuccess;
-  }
-#define LAUNCH_FP(DD, CC, WW)                                               \
-  hipLaunchKernelGGL((flash_prefill_kernel<DD, CC, WW>), grid, dim3(256),   \
-                     0, stream, (short*)out, (const short*)q,               \
-                     (const short*)k, (const short*)v,                      \
-                     (const int*)cu_seqlens, Hq, Hkv, scale, sq, sk, sv,    \
-                     window)
-  const bool win1 = window > 0;
+  PrefillArgs p{(short*)out, (const short*)q, k, v, (const int*)cu_seqlens,
+                nullptr, nullptr, Hq, Hkv, 0, 1, scale, sq, sk, sv, window};
+  // LDS-direct loads move 16 aligned bytes per lane
+  const bool dma = aligned16(k, v) && sk % 8 == 0 && sv % 8 == 0;
   if (head_dim == 128) {
-    if (causal) { if (win1) LAUNCH_FP(128, true, true); else LAUNCH_FP(128, true, false); }
-    else { if (win1) LAUNCH_FP(128, false, true); else LAUNCH_FP(128, false, false); }
-  } else {
-    if (causal) { if (win1) LAUNCH_FP(64, true, true); else LAUNCH_FP(64, true, false); }
-    else { if (win1) LAUNCH_FP(64, false, true); else LAUNCH_FP(64, false, false); }
+    if (dma) return launch<128, ROWS_DMA>(p, num_seqs, max_seqlen, causal, stream);
+    return launch<128, ROWS_REG>(p, num_seqs, max_seqlen, causal, stream);
   }
-#undef LAUNCH_FP
-  HIP_CHECK_KERNEL();
-  return hipSuccess;
+  if (dma) return launch<64, ROWS_DMA>(p, num_seqs, max_seqlen, causal, stream);
+  return launch<64, ROWS_REG>(p, num_seqs, max_seqlen, causal, stream);
 }

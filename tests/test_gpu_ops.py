@@ -305,6 +305,80 @@ class TestPrefillAttention:
         )
         bf16_close(got, ref, atol=3e-2, rtol=3e-2)
 
+    @pytest.mark.parametrize("causal,window", [(True, 0), (False, 0), (True, 40)])
+    @pytest.mark.parametrize(
+        "lens,H,Hkv,D,pad",
+        [
+            ([1, 31, 32, 33], 4, 1, 128, 0),      # four heads of a group per block
+            ([127, 2, 129], 6, 3, 128, 0),        # two heads per block
+            ([64, 65, 128, 300], 3, 1, 64, 0),    # one head per block
+            ([63, 200], 8, 1, 64, 0),
+            ([77, 130], 4, 2, 128, 1),            # rows at odd 2-byte offsets
+            ([77, 130], 2, 2, 64, 4),
+        ],
+    )
+    def test_prefill_tile_edges(self, dev, lens, H, Hkv, D, pad, causal, window):
+        """Query and key counts around the 32/64/128-row tiles, each number of
+        heads per block, and rows that LDS-direct loads cannot take."""
+        import kserve_amd_C
+
+        torch.manual_seed(sum(lens) + H)
+        T = sum(lens)
+        cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+        rows = torch.randn(T, (H + 2 * Hkv) * D + pad, dtype=torch.bfloat16, device=dev)
+        rows = rows[:, pad:]
+        q, k, v = (
+            x.unflatten(1, (-1, D))
+            for x in rows.split([H * D, Hkv * D, Hkv * D], dim=1)
+        )
+        out = torch.empty(T, H, D, dtype=torch.bfloat16, device=dev)
+        scale = D ** -0.5
+        kserve_amd_C.flash_prefill_varlen(
+            out, q, k, v, cu.to(dev), max(lens), scale, causal, window
+        )
+        ref = torch_ref.flash_prefill_varlen(
+            q.float().cpu(), k.float().cpu(), v.float().cpu(), cu, scale,
+            causal=causal, window=window,
+        )
+        # weights and output are each rounded to bf16: 2^-9 relative twice
+        err = (out.float().cpu() - ref).norm() / ref.norm()
+        assert err < 2 * 2 ** -9, float(err)
+
+    @pytest.mark.parametrize("fp8", [False, True])
+    @pytest.mark.parametrize("window", [0, 50])
+    @pytest.mark.parametrize("H,Hkv", [(4, 1), (6, 3), (2, 2), (8, 1)])
+    def test_context_prefill_tile_edges(self, dev, H, Hkv, window, fp8):
+        """Chunks of 1 to 129 queries over contexts that end anywhere in a page
+        and in a 64-key tile, one of them without any earlier key."""
+        from kserve_amd import ops
+
+        D = 128
+        qlens, ctx = [1, 5, 32, 129, 17], [1, 48, 64, 333, 1001]
+        torch.manual_seed(H)
+        nb = [-(-c // 16) for c in ctx]
+        kc = torch.randn(sum(nb) + 2, Hkv, 16, D, device=dev).to(torch.bfloat16)
+        vc = torch.randn(sum(nb) + 2, Hkv, 16, D, device=dev).to(torch.bfloat16)
+        if fp8:
+            kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+        order, at = torch.randperm(sum(nb) + 2), 0
+        bt = torch.zeros(len(ctx), max(nb), dtype=torch.int32)
+        for i, n in enumerate(nb):
+            bt[i, :n] = order[at : at + n]
+            at += n
+        cu = torch.tensor([0] + list(torch.tensor(qlens).cumsum(0)), dtype=torch.int32)
+        ctx_t = torch.tensor(ctx, dtype=torch.int32)
+        q = torch.randn(sum(qlens), H, D, dtype=torch.bfloat16, device=dev)
+        got = ops.context_attention_varlen(
+            q, kc, vc, bt.to(dev), cu.to(dev), ctx_t.to(dev), max(qlens),
+            D ** -0.5, window=window,
+        )
+        ref = torch_ref.context_attention_varlen(
+            q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt, cu, ctx_t,
+            D ** -0.5, window=window,
+        )
+        err = (got.float().cpu() - ref).norm() / ref.norm()
+        assert err < 2 * 2 ** -9, float(err)
+
 
 class TestSampling:
     def test_greedy(self, dev):
