@@ -471,7 +471,9 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
   float best = -1e38f;
   int best_idx = 0;
   auto take = [&](short b, int i) {
-    const float val = bf16_bits_to_float(b) * inv_t - gumbel_noise(seed, i);
+    // top-k of one is the greedy choice, ties included: no noise
+    float val = bf16_bits_to_float(b) * inv_t;
+    if (k != 1) val -= gumbel_noise(seed, i);
     if (val > best || (val == best && i < best_idx)) {
       best = val;
       best_idx = i;

@@ -559,13 +559,29 @@ class TestSampling:
                 c = probs[order].cumsum(0)
                 at = int((c < float(top_p[r])).sum())
                 least = max(least, float(vals[min(at, vocab - 1)]))
-            s = score[r].masked_fill(x[r] < least, float("-inf"))
+            # top-k of one draws nothing
+            s = x[r] if top_k[r] == 1 else score[r]
+            s = s.masked_fill(x[r] < least, float("-inf"))
             got = int(out[r])
             # the kernel's noise carries the error of two fast fp32 logarithms
             # (2e-6 relative of values up to 20): only scores closer than
             # that may change places
             assert x[r][got] >= least, (r, got)
             assert s[got] >= s.max() - 1e-4, (r, got, int(s.argmax()))
+
+    @pytest.mark.parametrize("vocab", [5, 32000, 70001])
+    def test_topk1_ties_are_greedy(self, dev, vocab):
+        """Equal largest logits: top_k 1 takes the one that greedy takes."""
+        from kserve_amd import ops
+
+        g = torch.Generator().manual_seed(vocab)
+        logits = torch.randn(8, vocab, generator=g).clamp(max=0.5).to(torch.bfloat16)
+        seeds = torch.arange(8, device=dev)
+        ones = torch.ones(8, device=dev)
+        k = torch.ones(8, dtype=torch.int32, device=dev)
+        logits = logits.to(dev)
+        got = ops.random_sample(logits, ones * 0.7, ones, k, seeds=seeds)
+        assert torch.equal(got, ops.greedy_sample(logits))
 
 
 class TestSkinnyGemm:
