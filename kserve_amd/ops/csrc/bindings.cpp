@@ -17,8 +17,9 @@ hipError_t ks_reshape_and_cache(const void*, const void*, void*, void*,
 hipError_t ks_paged_attention_decode(void*, const void*, const void*,
                                      const void*, const void*, const void*,
                                      float, int, int, int, int, int, int,
-                                     long, int, void*, void*, int,
+                                     long, int, void*, void*, int, int,
                                      hipStream_t);
+int ks_paged_decode_splits(int, int, int);
 hipError_t ks_flash_prefill_varlen(void*, const void*, const void*,
                                    const void*, const void*, int, int, int,
                                    int, int, float, long, long, long, int,
@@ -28,11 +29,6 @@ hipError_t ks_context_prefill_varlen(void*, const void*, const void*,
                                      const void*, int, int, int, int, int,
                                      int, float, long, int, int,
                                      hipStream_t);
-hipError_t ks_paged_attention_decode_fp8(void*, const void*, const void*,
-                                         const void*, const void*,
-                                         const void*, float, int, int, int,
-                                         int, int, int, long, int, void*,
-                                         void*, int, hipStream_t);
 hipError_t ks_reshape_and_cache_fp8(const void*, const void*, void*, void*,
                                     const void*, int, int, int, int, long,
                                     long, hipStream_t);
@@ -165,35 +161,7 @@ void paged_attention_decode(at::Tensor& out, at::Tensor& q,
   int Hkv = k_cache.size(1);
   int block_size = k_cache.size(2);
   int max_blocks = block_tables.size(1);
-  // split-context heuristic, measured A/B 2026-09-12 (gpurun_out/
-  // attn_split_*.log): splitting HURTS at S>=256 (3.69->3.43 TB/s, the
-  // fp32 partials + reduce outweigh extra waves) and for the group=8
-  // HPW=2 shapes (2.05->1.81), but the 512-workgroup group<=4 regime
-  // gains (S=64: 3.75->3.96 at 4 splits) and tiny batches need deep
-  // splits (S=8: 0.71 unsplit vs 1.6-1.7 at 8-16). Rule: group<=4 AND
-  // base<=512 -> clamp(2048/base, 2, 8); otherwise split only below
-  // 512 workgroups (the original rule).
-  int n_splits = 1;
-  long base_wgs = (long)S * Hkv;
-  const int grp = H / Hkv;
-  static const int split_override = [] {
-    const char* e = getenv("KS_ATTN_SPLIT");
-    return e ? atoi(e) : 0;  // 0 = heuristic
-  }();
-  if (split_override > 0) {
-    n_splits = split_override;
-  } else if (grp <= 4 && base_wgs <= 512) {
-    n_splits = (int)(2048 / base_wgs);
-    if (n_splits < 2) n_splits = 2;
-    if (n_splits > 8) n_splits = 8;
-  } else if (base_wgs < 512) {
-    n_splits = (int)((512 + base_wgs - 1) / base_wgs);
-    if (n_splits > 16) n_splits = 16;
-  }
-  if (n_splits > 1) {
-    int max_split_blocks = (max_blocks + n_splits - 1) / n_splits;
-    if (max_split_blocks < 1) n_splits = 1;
-  }
+  const int n_splits = ks_paged_decode_splits(S, Hkv, max_blocks);
   at::Tensor part_out, part_ml;
   void *po = nullptr, *pml = nullptr;
   if (n_splits > 1) {
@@ -203,24 +171,15 @@ void paged_attention_decode(at::Tensor& out, at::Tensor& q,
     po = part_out.data_ptr();
     pml = part_ml.data_ptr();
   }
-  if (fp8) {
+  if (fp8)
     TORCH_CHECK(H / Hkv <= 4 && D == 128,
                 "fp8 KV decode supports D=128 and GQA group <= 4");
-    check_hip(ks_paged_attention_decode_fp8(
-                  out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
-                  v_cache.data_ptr(), block_tables.data_ptr(),
-                  context_lens.data_ptr(), (float)scale, S, H, Hkv, D,
-                  max_blocks, block_size, (long)q.stride(0), n_splits, po,
-                  pml, (int)window, current_stream()),
-              "paged_attention_decode_fp8");
-    return;
-  }
   check_hip(ks_paged_attention_decode(
                 out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
                 v_cache.data_ptr(), block_tables.data_ptr(),
                 context_lens.data_ptr(), (float)scale, S, H, Hkv, D,
                 max_blocks, block_size, (long)q.stride(0), n_splits, po, pml,
-                (int)window, current_stream()),
+                (int)window, fp8 ? 1 : 0, current_stream()),
             "paged_attention_decode");
 }
 

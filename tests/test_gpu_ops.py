@@ -153,6 +153,61 @@ class TestDecodeAttention:
         )
         bf16_close(got, ref)
 
+    @pytest.mark.parametrize(
+        "H,Hkv,D,window,off,fp8",
+        [
+            (4, 1, 128, 0, 0, False), (5, 1, 128, 0, 0, False),  # one product
+            (6, 1, 128, 0, 0, False), (8, 1, 64, 0, 0, False),   # two products
+            (3, 3, 64, 0, 0, False), (14, 2, 128, 0, 0, False),
+            (8, 2, 128, 50, 0, False), (8, 2, 64, 33, 0, False),
+            (8, 2, 128, 0, 3, False), (4, 4, 64, 0, 1, False),   # odd page address
+            (4, 1, 128, 0, 0, True), (6, 2, 128, 50, 0, True), (2, 2, 128, 0, 0, True),
+        ],
+    )
+    @pytest.mark.parametrize("copies", [1, 64])
+    def test_paged_decode_edges(self, dev, H, Hkv, D, window, off, fp8, copies):
+        """Contexts that end anywhere in a page and a page pair, split over
+        blocks (12 sequences) and not (768), with NaN in every cached row that
+        no sequence owns."""
+        from kserve_amd import ops
+
+        ctx = [1, 15, 16, 17, 31, 32, 33, 64, 65, 200, 1000, 3001]
+        torch.manual_seed(H + D)
+        nb = [-(-c // 16) for c in ctx]
+        NB = sum(nb) + 2
+
+        def pages():
+            x = torch.randn(NB * Hkv * 16 * D + off, device=dev).to(torch.bfloat16)
+            return x[off:].view(NB, Hkv, 16, D)
+
+        kc, vc = pages(), pages()
+        order, at = torch.randperm(NB), 0
+        bt = torch.zeros(len(ctx), max(nb), dtype=torch.int32)
+        for i, n in enumerate(nb):
+            bt[i, :n] = order[at : at + n]
+            at += n
+            if ctx[i] % 16:
+                for c in (kc, vc):
+                    c[bt[i, n - 1], :, ctx[i] % 16 :] = float("nan")
+        if fp8:
+            kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+        ctx_t = torch.tensor(ctx, dtype=torch.int32)
+        q = (torch.randn(len(ctx), H, D, device=dev) * 1.5).to(torch.bfloat16)
+        got = ops.paged_attention_decode(
+            q.repeat(copies, 1, 1), kc, vc, bt.repeat(copies, 1).to(dev),
+            ctx_t.repeat(copies).to(dev), D ** -0.5, window=window,
+        )
+        ref = torch_ref.paged_attention_decode(
+            q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt, ctx_t,
+            D ** -0.5, window=window,
+        )
+        for part in got.float().cpu().split(len(ctx)):
+            # fp32 weights and sums: what is left is the bf16 output, half a
+            # unit in the last place (2^-9) at most per element
+            err = (part - ref).abs()
+            assert (err <= 2 ** -8 * ref.abs() + 1e-5).all(), float(err.max())
+            assert err.norm() < 2 ** -9 * ref.norm()
+
 
 class TestPrefillAttention:
     @pytest.mark.parametrize(
