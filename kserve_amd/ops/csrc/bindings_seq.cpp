@@ -22,7 +22,7 @@ hipError_t ks_causal_conv_silu(void*, const void*, long, const void*,
                                int, int, hipStream_t);
 hipError_t ks_ssd_scan(void*, const void*, const void*, long, int, const void*,
                        const void*, const void*, void*, const void*,
-                       const void*, const void*, int, int, int, int, int,
+                       const void*, const void*, int, int, int, int, int, int,
                        hipStream_t);
 hipError_t ks_qk_norm_temp_cache(void*, const void*, const void*, const void*,
                                  long, const void*, const void*, const void*,
@@ -340,8 +340,8 @@ void ssd_scan(at::Tensor& y, at::Tensor& xbc, at::Tensor& dt_raw,
                         dt_bias.data_ptr(), a_log.data_ptr(),
                         d_skip.data_ptr(), state.data_ptr(),
                         positions.data_ptr(), cu_seqlens.data_ptr(),
-                        slots.data_ptr(), num_seqs, heads, (int)groups, P, N,
-                        current_stream()),
+                        slots.data_ptr(), tokens, num_seqs, heads, (int)groups,
+                        P, N, current_stream()),
             "ssd_scan");
 }
 

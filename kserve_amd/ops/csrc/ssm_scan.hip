@@ -330,6 +330,279 @@ ssd_scan_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// The scan in chunks of 64 tokens on the fp32 matrix cores
+// (v_mfma_f32_16x16x4_f32), for portions that are long enough to fill chunks.
+// With c_t the running sum of A dt inside the chunk and S the state at its
+// start:
+//     y_t = exp(c_t) S^T C_t + sum_{s <= t} (C_t . B_s) exp(c_t - c_s) dt_s x_s
+//           + D x_t
+//     S  <- exp(c_end) S + sum_s exp(c_end - c_s) dt_s B_s x_s^T
+// A block takes 64 columns (p) of one head of one sequence; each of its 8 waves
+// owns 16 columns and half of the states, S^T in accumulator layout (row
+// n = 16 nb + 4 g + r in register r of lane group g), which is already the B
+// operand of C S for the contraction order "lane group g, product r -> state
+// 4 g + r"; C is then read from LDS four states at a time. The waves share the
+// 64 x 64 products C B^T (the 10 16 x 16 tiles on and below the diagonal); the
+// two halves of a column block add their sums over states through LDS, each
+// finishing half of the token tiles. The next chunk's rows are on their way in
+// registers meanwhile.
+//
+// Bound by the products of one chunk after the other: 212 per wave of 32
+// cycles each, two waves per SIMD (5.6 us of the 10 us that a chunk takes).
+// Token by token a chunk took 64 times the latency of one step (LDS reads,
+// update, lane tree), whatever the arithmetic. 64 heads of 64 columns, 128
+// states: 4 x 2000 tokens 1855 -> 320 us, 8 x 2000 1962 -> 627 us, 1 x 2000
+// 1793 -> 299 us, 1 x 40 43 -> 13 us; one wave per column block with all states
+// (4 waves) took 391 us for 4 x 2000. Error against 64 bits, mean over portions
+// of 50 to 400 tokens: y 8.0e-8 both, state 8.3e-8 -> 7.9e-8.
+// ---------------------------------------------------------------------------
+constexpr int CQ = 64;  // tokens per chunk
+constexpr int CT = 512;
+typedef float f32x4s __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4s mfma4(float a, float b, f32x4s c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+template <int NB>  // blocks of 16 states: N <= 16 NB
+__global__ void __launch_bounds__(CT) ssd_chunk_kernel(
+    float* __restrict__ y, const float* __restrict__ xbc,
+    const float* __restrict__ dt_raw_f32, const short* __restrict__ dt_raw_bf16,
+    long dt_stride, const float* __restrict__ dt_bias,
+    const float* __restrict__ a_log, const float* __restrict__ d_skip,
+    float* __restrict__ state, const long* __restrict__ positions,
+    const int* __restrict__ cu_seqlens, const int* __restrict__ slots,
+    int heads, int groups, int P, int N) {
+  constexpr int NP = NB * 16;
+  constexpr int RS = NP + 4;  // B and C rows: 4 rows apart fall 16 banks apart
+  constexpr int XS = 64 + 4;
+  constexpr int NH = NB / 2;  // of them, a wave's own
+  constexpr int NV = CQ * NP / 4 / CT;  // float4 per thread of a B or C tile
+  constexpr int XV = CQ * 64 / 4 / CT;
+  __shared__ __attribute__((aligned(16))) float Bs[CQ * RS];
+  __shared__ __attribute__((aligned(16))) float Cs[CQ * RS];
+  __shared__ __attribute__((aligned(16))) float Xs[CQ * XS];
+  __shared__ __attribute__((aligned(16))) float Ms[CQ * XS];
+  __shared__ __attribute__((aligned(16))) f32x4s part[CT / 64][2][64];
+  __shared__ __attribute__((aligned(16))) float dts[CQ], grow[CQ], left[CQ];
+  // running sums in 64 bits: their differences are exponents, and a sum over a
+  // chunk may be far larger than the difference of two neighbours
+  __shared__ double cum[CQ];
+
+  const int s = blockIdx.z, h = blockIdx.y;
+  const int first = cu_seqlens[s];
+  const int len = cu_seqlens[s + 1] - first;
+  if (len <= 0) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int p0 = blockIdx.x * 64;
+  const int pw = wave & 3, nh = wave >> 2;
+  const int p = p0 + pw * 16 + col;
+  const int grp = h / (heads / groups);
+  const int inner = heads * P;
+  const int channels = inner + 2 * groups * N;
+  const float A = -expf(a_log[h]);
+  const float bias = dt_bias[h];
+  const float Dh = d_skip[h];
+  const bool fresh = positions[first] == 0;
+  float* sp = state + ((slots[s] * (long)heads + h) * P + p) * N;
+
+  f32x4s S[NH];
+#pragma unroll
+  for (int b = 0; b < NH; ++b) {
+    const int n = (nh * NH + b) * 16 + g * 4;
+    S[b] = (!fresh && p < P && n < N) ? *reinterpret_cast<const f32x4s*>(sp + n)
+                                      : f32x4s{0.f, 0.f, 0.f, 0.f};
+  }
+
+  f32x4s rB[NV], rC[NV], rX[XV];
+  float rdt = 0.f;
+  auto fetch = [&](int t0) {
+    const f32x4s zero = f32x4s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int e = threadIdx.x + i * CT;
+      const int tk = e / (NP / 4), n = e % (NP / 4) * 4;
+      const bool ok = t0 + tk < len && n < N;
+      const float* row = xbc + (long)(first + t0 + tk) * channels + inner + grp * N + n;
+      rB[i] = ok ? *reinterpret_cast<const f32x4s*>(row) : zero;
+      rC[i] = ok ? *reinterpret_cast<const f32x4s*>(row + groups * N) : zero;
+    }
+#pragma unroll
+    for (int i = 0; i < XV; ++i) {
+      const int e = threadIdx.x + i * CT;
+      const int tk = e / 16, c = e % 16 * 4;
+      const bool ok = t0 + tk < len && p0 + c < P;
+      rX[i] = ok ? *reinterpret_cast<const f32x4s*>(
+                       xbc + (long)(first + t0 + tk) * channels + h * P + p0 + c)
+                 : zero;
+    }
+    if (wave == 0) {
+      const long i = (long)(first + min(t0 + lane, len - 1)) * dt_stride + h;
+      rdt = (dt_raw_f32 ? dt_raw_f32[i] : bf16_bits_to_float(dt_raw_bf16[i])) + bias;
+    }
+  };
+  auto commit = [&](int cnt) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int e = threadIdx.x + i * CT;
+      const int at = e / (NP / 4) * RS + e % (NP / 4) * 4;
+      *reinterpret_cast<f32x4s*>(Bs + at) = rB[i];
+      *reinterpret_cast<f32x4s*>(Cs + at) = rC[i];
+    }
+#pragma unroll
+    for (int i = 0; i < XV; ++i) {
+      const int e = threadIdx.x + i * CT;
+      *reinterpret_cast<f32x4s*>(Xs + e / 16 * XS + e % 16 * 4) = rX[i];
+    }
+    if (wave == 0) {
+      // softplus without a clamp; log1p(exp(v)) is v itself past v ~ 30.
+      // Rows past the portion: dt 0, so they change nothing
+      const float dt = lane < cnt ? (rdt > 30.f ? rdt : log1pf(expf(rdt))) : 0.f;
+      double c = (double)A * dt;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_up(c, off, 64);
+        if (lane >= off) c += o;
+      }
+      const double end = __shfl(c, 63, 64);
+      cum[lane] = c;
+      dts[lane] = dt;
+      grow[lane] = expf((float)c);
+      left[lane] = dt * expf((float)(end - c));
+    }
+  };
+
+  fetch(0);
+  for (int t0 = 0; t0 < len; t0 += CQ) {
+    const int cnt = min(CQ, len - t0);
+    __syncthreads();  // the previous chunk's tiles are consumed
+    commit(cnt);
+    __syncthreads();
+    if (t0 + CQ < len) fetch(t0 + CQ);
+
+    // ---- C B^T on and below the diagonal, with decays and step sizes ----
+    for (int i = wave; i < 10; i += CT / 64) {
+      const int tb = i < 1 ? 0 : i < 3 ? 1 : i < 6 ? 2 : 3;
+      const int sb = i - tb * (tb + 1) / 2;
+      // eight chains: fewer roundings in a row than one sum over the states
+      f32x4s acc[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) acc[r] = f32x4s{0.f, 0.f, 0.f, 0.f};
+      const float* ca = Cs + (tb * 16 + col) * RS + g * 4;
+      const float* ba = Bs + (sb * 16 + col) * RS + g * 4;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const f32x4s c4 = *reinterpret_cast<const f32x4s*>(ca + b * 16);
+        const f32x4s b4 = *reinterpret_cast<const f32x4s*>(ba + b * 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          f32x4s& to = acc[r + (b & 1) * 4];
+          to = mfma4(c4[r], b4[r], to);
+        }
+      }
+      const f32x4s cb = ((acc[0] + acc[1]) + (acc[2] + acc[3])) +
+                        ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+      const int sk = sb * 16 + col;
+      const double cs = cum[sk];
+      const float ds = dts[sk];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int tk = tb * 16 + g * 4 + r;
+        Ms[tk * XS + sk] = sk <= tk ? cb[r] * expf((float)(cum[tk] - cs)) * ds : 0.f;
+      }
+    }
+
+    // ---- what the state at the chunk's start contributes ----
+    f32x4s Y[4], Y2[4];
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) Y[tb] = Y2[tb] = f32x4s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int b = 0; b < NH; ++b) {
+      f32x4s c4[4];
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb)
+        c4[tb] = *reinterpret_cast<const f32x4s*>(Cs + (tb * 16 + col) * RS +
+                                                  (nh * NH + b) * 16 + g * 4);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int tb = 0; tb < 4; ++tb) {
+          f32x4s& to = r & 1 ? Y2[tb] : Y[tb];
+          to = mfma4(c4[tb][r], S[b][r], to);
+        }
+    }
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) Y[tb] += Y2[tb];
+    // token tiles 0 and 3 are finished by the first half, 1 and 2 by the other
+    part[wave][0][lane] = nh ? Y[0] : Y[1];
+    part[wave][1][lane] = nh ? Y[3] : Y[2];
+
+    // ---- the state moves on ----
+    f32x4s X[4];  // token 16 tb + 4 g + r, this lane's column
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        X[tb][r] = Xs[(tb * 16 + g * 4 + r) * XS + pw * 16 + col];
+    const float keep = grow[CQ - 1];
+#pragma unroll
+    for (int b = 0; b < NH; ++b) S[b] *= keep;
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+      const f32x4s xw =
+          X[tb] * *reinterpret_cast<const f32x4s*>(left + tb * 16 + g * 4);
+      const float* brow = Bs + (tb * 16 + g * 4) * RS + nh * NH * 16 + col;
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int b = 0; b < NH; ++b)
+          S[b] = mfma4(brow[r * RS + b * 16], xw[r], S[b]);
+    }
+
+    __syncthreads();  // Ms and the partial sums are complete
+    // ---- what the chunk's own tokens contribute ----
+    auto finish = [&](auto tile, f32x4s own, int k) {
+      constexpr int tb = decltype(tile)::value;
+      f32x4s acc[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = f32x4s{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int sb = 0; sb <= tb; ++sb) {
+        const f32x4s m4 = *reinterpret_cast<const f32x4s*>(
+            Ms + (tb * 16 + col) * XS + sb * 16 + g * 4);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = mfma4(m4[r], X[sb][r], acc[r]);
+      }
+      f32x4s z = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      const f32x4s e4 = *reinterpret_cast<const f32x4s*>(grow + tb * 16 + g * 4);
+      z += (own + part[wave ^ 4][k][lane]) * e4;
+      if (p < P) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int tk = tb * 16 + g * 4 + r;
+          if (tk < cnt)
+            y[(long)(first + t0 + tk) * inner + h * P + p] = z[r] + Dh * X[tb][r];
+        }
+      }
+    };
+    if (nh == 0) {
+      finish(std::integral_constant<int, 0>{}, Y[0], 0);
+      finish(std::integral_constant<int, 3>{}, Y[3], 1);
+    } else {
+      finish(std::integral_constant<int, 1>{}, Y[1], 0);
+      finish(std::integral_constant<int, 2>{}, Y[2], 1);
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < NH; ++b) {
+    const int n = (nh * NH + b) * 16 + g * 4;
+    if (p < P && n < N) *reinterpret_cast<f32x4s*>(sp + n) = S[b];
+  }
+}
+
 }  // namespace
 
 extern "C" hipError_t ks_causal_conv_silu(
@@ -412,11 +685,37 @@ extern "C" hipError_t ks_ssd_scan(void* y, const void* xbc, const void* dt_raw,
                                   const void* d_skip, void* state,
                                   const void* positions,
                                   const void* cu_seqlens, const void* slots,
-                                  int num_seqs, int heads, int groups, int P,
-                                  int N, hipStream_t stream) {
+                                  int tokens, int num_seqs, int heads,
+                                  int groups, int P, int N,
+                                  hipStream_t stream) {
   if (num_seqs == 0) return hipSuccess;
   if (groups <= 0 || heads % groups != 0 || N < 1 || N > 256)
     return hipErrorInvalidValue;
+  // Chunks of 64 tokens pay off from 32 tokens per sequence on, and from 16
+  // where blocks are few enough to be in flight at once (us, token by token ->
+  // chunks, 64 heads: 64 x 16 tokens 108 -> 193, 64 x 32 197 -> 188, 16 x 24
+  // 47 -> 48; 8 x 16 25 -> 24, 8 x 8 18 -> 24; 1 x 24 29 -> 13)
+  const long chunk_blocks = (long)cdiv(P, 64) * heads * num_seqs;
+  if (tokens >= (chunk_blocks <= 512 ? 16L : 32L) * num_seqs && N % 4 == 0 &&
+      N <= 128 && P % 4 == 0 &&
+      (((uintptr_t)xbc | (uintptr_t)state) & 15) == 0) {
+    const dim3 cgrid(cdiv(P, 64), heads, num_seqs);
+#define SSD_CHUNK(nb)                                                         \
+  hipLaunchKernelGGL((ssd_chunk_kernel<nb>), cgrid, dim3(CT), 0, stream,      \
+                     (float*)y, (const float*)xbc,                            \
+                     dt_is_f32 ? (const float*)dt_raw : nullptr,              \
+                     dt_is_f32 ? nullptr : (const short*)dt_raw, dt_stride,   \
+                     (const float*)dt_bias, (const float*)a_log,              \
+                     (const float*)d_skip, (float*)state,                     \
+                     (const long*)positions, (const int*)cu_seqlens,          \
+                     (const int*)slots, heads, groups, P, N)
+    if (N <= 32) SSD_CHUNK(2);
+    else if (N <= 64) SSD_CHUNK(4);
+    else SSD_CHUNK(8);
+#undef SSD_CHUNK
+    HIP_CHECK_KERNEL();
+    return hipSuccess;
+  }
   // columns per lane: a block covers up to 64 columns of one head; wide
   // state rows (R = 16) keep two columns so the state stays in registers
   const int R = cdiv(N, 16);

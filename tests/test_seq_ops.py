@@ -235,6 +235,52 @@ class TestScan:
             at += n
         close(torch.cat(outs), want, be, f32_tol=5e-5, bf16_tol=5e-5)
 
+    @pytest.mark.parametrize(
+        "H,G,P,N", [(2, 1, 64, 128), (4, 2, 24, 16), (2, 2, 72, 100), (3, 1, 8, 36)]
+    )
+    def test_long_portions(self, be, H, G, P, N):
+        """Portions around the 64-token chunks, in one call: fresh and
+        continued sequences, one of a single token, states handed on."""
+        inner = H * P
+        lens = ((63, 1, 130, 64), (65, 40, 2, 66))
+        starts = (0, 0, 0, 0)
+        dt_bias = rnd(H, seed=42) - 1.0
+        a_log = rnd(H, seed=43, scale=0.5)
+        d_skip = rnd(H, seed=44)
+        total = [a + b for a, b in zip(*lens)]
+        xs = [rnd(n, inner + 2 * G * N, seed=50 + i, scale=0.7) for i, n in enumerate(total)]
+        dts = [rnd(n, H, seed=60 + i, dtype=be[1]) for i, n in enumerate(total)]
+        want = []
+        for x, d in zip(xs, dts):
+            n = x.shape[0]
+            want.append(
+                O.ssd(
+                    x[:, :inner].double().reshape(n, H, P),
+                    x[:, inner : inner + G * N].double().reshape(n, G, N),
+                    x[:, inner + G * N :].double().reshape(n, G, N),
+                    O.softplus(d.double() + dt_bias.double()), a_log.double(),
+                    d_skip.double(), G,
+                ).reshape(n, inner)
+            )
+        state = torch.full((6, H, P, N), 5.0, device=be[0])
+        slots = [3, 1, 5, 2]
+        got = [[], [], [], []]
+        at = list(starts)
+        for step in lens:
+            cu, _, pos = layout(list(step), at)
+            x = torch.cat([xs[i][a : a + n] for i, (a, n) in enumerate(zip(at, step))])
+            d = torch.cat([dts[i][a : a + n] for i, (a, n) in enumerate(zip(at, step))])
+            y = ops.ssd_scan(
+                f32(x, be), act(d, be), f32(dt_bias, be), f32(a_log, be),
+                f32(d_skip, be), state, i64(pos, be), i32(cu, be), i32(slots, be), G,
+            )
+            for i in range(4):
+                got[i].append(y[cu[i] : cu[i + 1]])
+                at[i] += step[i]
+        for g, w in zip(got, want):
+            # fp32 sums of at most 130 + 128 terms against the largest output
+            close(torch.cat(g), w, be, f32_tol=5e-6, bf16_tol=5e-6)
+
     def test_large_step_sizes_are_not_clamped(self, be):
         """softplus of a large argument is the argument itself."""
         H, P, N, T = 1, 4, 8, 3
