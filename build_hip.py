@@ -59,7 +59,8 @@ MODULES = {
     },
 }
 
-HEADERS = ["common.h", "mfma_layouts.h", "dtype_io.h", "cache_chunk.h"]
+HEADERS = ["common.h", "mfma_layouts.h", "dtype_io.h", "cache_chunk.h",
+           "mfma_attention.h"]
 # hipcc makes packed-fp32 instructions on its own from plain float code; keep
 # them off for every kernel of this package
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

@@ -36,6 +36,10 @@ hipError_t ks_ctx_attention_f32(void*, const void*, const void*, const void*,
                                 const void*, int, long, void*, int, int, float,
                                 int, int, hipStream_t);
 int ks_ctx_attention_decode_splits(int, int, int, int, int, int);
+int ks_ctx_attention_mfma(const void*, const void*, const void*, const void*, int,
+                          int, int, int, int, int, int, const void*, long, int,
+                          float, int);
+int ks_ctx_attention_mfma_splits(int, int, int);
 hipError_t ks_qk_headnorm_rope_cache(void*, const void*, const void*,
                                      const void*, long, const void*,
                                      const void*, const void*, const void*,
@@ -461,9 +465,15 @@ void ctx_attention_f32(at::Tensor& out, at::Tensor& q, at::Tensor& k_cache,
   int nsplit = 1;
   at::Tensor ws;
   if (max_q_len == 1 && maps * D <= 256) {
-    nsplit = ks_ctx_attention_decode_splits(num_seqs, (int)heads, G,
-                                            (int)window, (int)keep_first,
-                                            fp != nullptr);
+    const bool mfma = ks_ctx_attention_mfma(
+        out.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), 1,
+        (int)heads, G, D, DV, bs, f32, fp, (long)vrs, (int)maps, (float)softcap,
+        (int)keep_first);
+    nsplit = mfma ? ks_ctx_attention_mfma_splits(num_seqs, G,
+                                                 (int)block_tables.size(1))
+                  : ks_ctx_attention_decode_splits(num_seqs, (int)heads, G,
+                                                   (int)window, (int)keep_first,
+                                                   fp != nullptr);
     if (nsplit > 1)
       ws = at::empty({(int64_t)num_seqs * heads * nsplit * (DV + 2)},
                      q.options().dtype(at::kFloat));

@@ -1,0 +1,924 @@
+// Paged and flat softmax attention on the bf16 matrix cores: the kernels behind
+// attention_prefill.hip and attention_decode.hip (bf16 queries) and the bf16
+// pages of attention_f32.hip (fp32 queries and softmax weights).
+//
+// PARTS is how many bf16 parts an fp32 operand enters with: three hold its 24
+// bits exactly (high, middle, low: 8 bits each), so the products with bf16 keys
+// and values are exact and everything is summed in fp32.
+#pragma once
+
+#include "common.h"
+#include "mfma_layouts.h"
+
+namespace {
+namespace mfma_attn {
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+
+constexpr float LOG2E = 1.44269504088896340736f;
+constexpr float MASKED = -3e38f;
+constexpr float NO_MAX = -1e30f;  // above MASKED: an all-masked tile adds 0
+constexpr int PAGE = 16;
+
+// where K and V rows come from
+enum Src {
+  ROWS_DMA,   // flat rows, 16-byte aligned: loaded straight into LDS
+  ROWS_REG,   // flat rows at any alignment: through registers
+  PAGES_DMA,  // bf16 pages of 16 tokens
+  PAGES_REG,  // bf16 pages at any alignment
+  PAGES_FP8,  // E4M3 pages, widened to bf16 on the way
+};
+
+// 16-byte chunk that chunk c of row r of a tile sits at. K fragments: 16
+// consecutive rows at one chunk must hit different banks; V fragments: 4
+// consecutive rows of 32 bytes each (a pair of chunks stays a pair).
+template <int D>
+__device__ __forceinline__ int k_swz(int r) {
+  return D == 128 ? (r & 15) : ((r >> 1) & 7);
+}
+template <int D>
+__device__ __forceinline__ int v_swz(int r) {
+  return D == 128 ? (r & 7) << 1 : ((r >> 1) & 3) << 1;
+}
+
+__device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// x as the sum of three bf16 numbers, exactly
+struct Split3 {
+  __bf16 hi, mid, lo;
+  __device__ __forceinline__ explicit Split3(float x) {
+    hi = (__bf16)x;
+    const float r1 = x - (float)hi;
+    mid = (__bf16)r1;
+    lo = (__bf16)(r1 - (float)mid);
+  }
+};
+
+// what the fp32 form adds to plain attention
+struct Extra {
+  const short* gate;  // [T, H] bf16 (row stride gate_stride): output * sigmoid
+  long gate_stride;
+  const float* sink;  // [H]: one more term exp(sink) in the denominator
+  int chunk;          // a query sees its own block of that many positions
+  int out_f32;        // fp32 output (else bf16)
+};
+
+// first position that a query at `pos` sees
+__device__ __forceinline__ int low_of(int pos, int window, int chunk) {
+  return chunk > 0 ? pos / chunk * chunk : window > 0 ? max(pos - window + 1, 0) : 0;
+}
+
+__device__ __forceinline__ float sigmoid_gate(const Extra& x, long tok, int head) {
+  return x.gate ? 1.f / (1.f + expf(-bf16_bits_to_float(x.gate[tok * x.gate_stride + head])))
+                : 1.f;
+}
+
+__device__ __forceinline__ void store4(void* out, long at, f32x4_t v, int f32) {
+  if (f32) {
+    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(out) + at) = v;
+  } else {
+    short4_t w;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[r] = float_to_bf16_bits(v[r]);
+    *reinterpret_cast<short4_t*>(reinterpret_cast<short*>(out) + at) = w;
+  }
+}
+
+// larger of a lane's value and its partner's in the other half of the wave
+__device__ __forceinline__ float half_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float half_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// eight E4M3 bytes as bf16 (exact)
+__device__ __forceinline__ short8_t widen_fp8(uint2 x) {
+  short8_t o;
+  const unsigned int w[2] = {x.x, x.y};
+#pragma unroll
+  for (int d = 0; d < 2; ++d) {
+    const float2_t lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[d], false);
+    const float2_t hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)w[d], true);
+    o[d * 4 + 0] = float_to_bf16_bits(lo[0]);
+    o[d * 4 + 1] = float_to_bf16_bits(lo[1]);
+    o[d * 4 + 2] = float_to_bf16_bits(hi[0]);
+    o[d * 4 + 3] = float_to_bf16_bits(hi[1]);
+  }
+  return o;
+}
+
+constexpr int KT = 64;      // keys per tile
+constexpr int NWAVES = 4;
+constexpr int QW = 32;      // queries per wave
+
+struct PrefillArgs {
+  void* out;          // [T, Hq, D]
+  const void* q;      // [T, Hq, D] bf16 (PARTS 1) or fp32, row stride sq
+  const void* k;      // [T, Hkv, D] rows (stride sk) or pages [NB, Hkv, 16, D]
+  const void* v;      // likewise, page rows sv apart
+  const int* cu_q;          // [S+1]
+  const int* ctx_lens;      // [S] keys of a sequence (pages)
+  const int* block_tables;  // [S, max_nb] (pages, row stride max_nb)
+  int Hq, Hkv, max_nb;
+  int hpb;  // query heads per block: 1, 2 or 4, divides the group
+  float scale;
+  long sq, sk, sv;
+  int window;
+  Extra x;
+};
+
+template <int D, int SRC, bool CAUSAL, bool WIN, int PARTS = 1>
+__global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
+    const PrefillArgs p) {
+  // key blocks of 32 that go through softmax together: with three parts the
+  // operands of one fill the registers
+  constexpr int NKB = PARTS == 1 ? 2 : 1;
+  constexpr bool PAGED = SRC >= PAGES_DMA;
+  constexpr bool DMA = SRC == ROWS_DMA || SRC == PAGES_DMA;
+  constexpr int CPR = D / 8;          // 16-byte chunks per row
+  constexpr int RPI = 64 / CPR;       // rows per wave-wide 16-byte load
+  constexpr int NI = 16 / RPI;        // such loads per wave and tile (K or V)
+  constexpr int TILE = KT * D;
+  constexpr int KC = D / 16;          // contraction chunks of Q K^T
+  constexpr int DB = D / 32;          // 32-column blocks of the output
+
+  const int seq = blockIdx.z;
+  const int q_start = p.cu_q[seq];
+  const int q_len = p.cu_q[seq + 1] - q_start;
+  const int qpb = NWAVES * QW / p.hpb;  // queries per block
+  // the last tiles have the most keys: they start first
+  const int tile_base = (gridDim.y - 1 - blockIdx.y) * qpb;
+  if (tile_base >= q_len) return;
+  const int len = PAGED ? p.ctx_lens[seq] : q_len;  // keys
+  const int start_pos = len - q_len;                // position of query 0
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int head = blockIdx.x * p.hpb + wave % p.hpb;
+  const int kvh = blockIdx.x * p.hpb / (p.Hq / p.Hkv);
+  const int q0 = tile_base + wave / p.hpb * QW;  // the wave's first query
+  const int half = lane >> 5;
+
+  __shared__ __attribute__((aligned(16))) short lds[2][2][TILE];  // [buffer][K, V]
+
+  // ---- queries: B operands, 8 consecutive columns per lane ----
+  bf16x8_t qf[PARTS][KC];
+  {
+    const int qrow = min(q0 + (lane & 31), q_len - 1);
+    const long at = (long)(q_start + qrow) * p.sq + (long)head * D + half * 8;
+    if constexpr (PARTS == 1) {
+      const short* qp = reinterpret_cast<const short*>(p.q) + at;
+#pragma unroll
+      for (int c = 0; c < KC; ++c)
+        qf[0][c] = *reinterpret_cast<const bf16x8_t*>(qp + c * 16);
+    } else {
+      const float* qp = reinterpret_cast<const float*>(p.q) + at;
+#pragma unroll
+      for (int c = 0; c < KC; ++c)
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+          const f32x4_t x = *reinterpret_cast<const f32x4_t*>(qp + c * 16 + j);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const Split3 w(x[e]);
+            qf[0][c][j + e] = w.hi;
+            qf[1][c][j + e] = w.mid;
+            qf[2][c][j + e] = w.lo;
+          }
+        }
+    }
+  }
+
+  // ---- key range ----
+  const int last_q = min(tile_base + qpb, q_len) - 1;
+  const int hi = CAUSAL ? min(len, start_pos + last_q + 1) : len;
+  auto low = [&](int pos) { return low_of(pos, p.window, p.x.chunk); };
+  const int lo = WIN ? max(0, low(start_pos + tile_base)) : 0;
+  const int t_lo = lo / KT;
+  const int t_hi = (hi + KT - 1) / KT;
+  const int pos_lo = start_pos + q0;
+  const int pos_hi = start_pos + min(q0 + QW, q_len) - 1;
+  const int my_pos = start_pos + q0 + (lane & 31);
+  // first visible key of the wave's first and last query and of this lane's
+  const int low_lo = WIN ? low(pos_lo) : 0, low_hi = WIN ? low(pos_hi) : 0;
+  const int my_low = WIN ? low(my_pos) : 0;
+
+  // ---- staging: wave w brings rows 16 w .. 16 w + 15 of a tile (one page);
+  // rows past the keys repeat the last one (their weights are 0, their values
+  // finite) ----
+  const int* bt = PAGED ? p.block_tables + (long)seq * p.max_nb : nullptr;
+  const int lrow = lane / CPR, lchunk = lane % CPR;
+  auto group_of = [&](int t) { return min(t * KT + wave * 16, len - 1); };
+  auto page_of = [&](int t) { return PAGED ? bt[group_of(t) >> 4] : 0; };
+  // address of this lane's chunk (c, already unswizzled) of row r of tile t
+  auto src = [&](const void* base, long stride, int t, int page, int r, int c) {
+    const int g0 = PAGED ? group_of(t) & ~15 : group_of(t);
+    const int row = min(r, len - 1 - g0);
+    if constexpr (PAGED) {
+      constexpr int ES = SRC == PAGES_FP8 ? 1 : 2;
+      const long st = PARTS == 1 ? D : stride;  // bf16 queries: whole rows
+      return reinterpret_cast<const char*>(base) +
+             ((long)page * p.Hkv + kvh) * PAGE * st * ES +
+             (row * (int)st + c * 8) * ES;
+    } else {
+      return reinterpret_cast<const char*>(base) +
+             ((long)(q_start + g0) * stride + (long)kvh * D) * 2 +
+             (long)row * stride * 2 + c * 16;
+    }
+  };
+  uint2 raw8[SRC == PAGES_FP8 ? 2 * NI : 1];
+  short8_t raw16[!DMA && SRC != PAGES_FP8 ? 2 * NI : 1];
+  // DMA: fills buffer `buf`; otherwise the rows wait in registers for commit()
+  auto stage = [&](int t, int page, int buf) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int r = i * RPI + lrow;
+      const char* ks = src(p.k, p.sk, t, page, r, lchunk ^ k_swz<D>(r));
+      const char* vs = src(p.v, p.sv, t, page, r, lchunk ^ v_swz<D>(r));
+      if constexpr (DMA) {
+        const int at = (wave * 16 + i * RPI) * D;
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const unsigned int*>(ks),
+            reinterpret_cast<unsigned int*>(&lds[buf][0][at]), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const unsigned int*>(vs),
+            reinterpret_cast<unsigned int*>(&lds[buf][1][at]), 16, 0, 0);
+      } else if constexpr (SRC == PAGES_FP8) {
+        raw8[2 * i] = *reinterpret_cast<const uint2*>(ks);
+        raw8[2 * i + 1] = *reinterpret_cast<const uint2*>(vs);
+      } else {
+        raw16[2 * i] = *reinterpret_cast<const short8_t*>(ks);
+        raw16[2 * i + 1] = *reinterpret_cast<const short8_t*>(vs);
+      }
+    }
+  };
+  auto commit = [&](int buf) {
+    if constexpr (!DMA) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int at = (wave * 16 + i * RPI) * D + lane * 8;
+#pragma unroll
+        for (int kv = 0; kv < 2; ++kv) {
+          short8_t x;
+          if constexpr (SRC == PAGES_FP8) x = widen_fp8(raw8[2 * i + kv]);
+          else x = raw16[2 * i + kv];
+          *reinterpret_cast<short8_t*>(&lds[buf][kv][at]) = x;
+        }
+      }
+    }
+  };
+
+  // ---- operand addresses inside a tile (elements) ----
+  const int krow = lane & 31;
+  int kaddr[KC];
+#pragma unroll
+  for (int c = 0; c < KC; ++c)
+    kaddr[c] = krow * D + ((2 * c + half) ^ k_swz<D>(krow)) * 8;
+  // transposing load: lane i of 16 brings key i/4, columns 4 (i%4) .. + 3 of a
+  // 4 x 16 block and receives column i of its four keys
+  const int ti = lane & 15;
+  const int vrow = half * 4 + (ti >> 2);
+  int vaddr[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+    vaddr[b] = vrow * D +
+               (((4 * b + ((lane >> 4) & 1) * 2 + ((ti & 3) >> 1)) ^ v_swz<D>(vrow)) * 8) +
+               (ti & 1) * 4;
+
+  float c2 = p.scale * 1.44269504088896340736f;
+  const bool flip = c2 < 0.f;
+  c2 = fabsf(c2);
+  float m = NO_MAX, l = 0.f;
+  f32x16_t o[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[b][r] = 0.f;
+
+  if (t_lo < t_hi) stage(t_lo, page_of(t_lo), 0);
+  int page = t_lo + 1 < t_hi ? page_of(t_lo + 1) : 0;
+  commit(0);
+
+  for (int t = t_lo; t < t_hi; ++t) {
+    const int buf = (t - t_lo) & 1;
+    __syncthreads();
+    if (t + 1 < t_hi) {
+      stage(t + 1, page, buf ^ 1);
+      if (PAGED && t + 2 < t_hi) page = page_of(t + 2);
+    }
+    const int t0 = t * KT;
+    const bool mine = q0 < q_len && (!CAUSAL || t0 <= pos_hi) &&
+                      (!WIN || t0 + KT - 1 >= low_lo);
+    if (mine) {
+      const short* kt = lds[buf][0];
+      const short* vt = lds[buf][1];
+#pragma unroll
+      for (int kg = 0; kg < 2; kg += NKB) {
+      f32x16_t s[NKB];
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb) {
+        f32x16_t rest;  // the products with the query's lower parts
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[kb][r] = rest[r] = 0.f;
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+          const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(
+              kt + (kg + kb) * 32 * D + kaddr[c]);
+          if constexpr (PARTS == 3) {
+            rest = mfma32(a, qf[PARTS - 1][c], rest);
+            rest = mfma32(a, qf[PARTS - 2][c], rest);
+          }
+          s[kb] = mfma32(a, qf[0][c], s[kb]);
+        }
+        if constexpr (PARTS == 3) s[kb] += rest;
+      }
+      if (flip) {
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) s[kb] = -s[kb];
+      }
+      // register r of block kb: key 32 kb + (r & 3) + 8 (r / 4) + 4 half
+      if (t0 + KT > len || (CAUSAL && t0 + KT - 1 > pos_lo) ||
+          (WIN && t0 < low_hi)) {
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = t0 + 32 * (kg + kb) + (r & 3) + 8 * (r >> 2) + 4 * half;
+            const bool ok = key < len && (!CAUSAL || key <= my_pos) &&
+                            (!WIN || key >= my_low);
+            s[kb][r] = ok ? s[kb][r] : MASKED;
+          }
+      }
+      float mx = s[0][0];
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
+      mx = half_max(mx);
+      if (__any(mx > m)) {
+        const float mn = fmaxf(m, mx);
+        const float f = __builtin_amdgcn_exp2f((m - mn) * c2);
+        m = mn;
+        l *= f;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[b][r] *= f;
+      }
+      const float mc = m * c2;
+      bf16x8_t pf[PARTS][NKB * 2];
+      float sum = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float w = __builtin_amdgcn_exp2f(s[kb][r] * c2 - mc);
+          sum += w;
+          if constexpr (PARTS == 1) {
+            pf[0][kb * 2 + (r >> 3)][r & 7] = (__bf16)w;
+          } else {
+            const Split3 w3(w);
+            pf[0][kb * 2 + (r >> 3)][r & 7] = w3.hi;
+            pf[1][kb * 2 + (r >> 3)][r & 7] = w3.mid;
+            pf[2][kb * 2 + (r >> 3)][r & 7] = w3.lo;
+          }
+        }
+      l += sum;
+#pragma unroll
+      for (int kc = 0; kc < NKB * 2; ++kc)
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+          typedef __attribute__((address_space(3))) s16x4_t lds4_t;
+          const short* a0 = vt + (kg * 2 + kc) * 16 * D + vaddr[b];
+          const s16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)a0);
+          const s16x4_t v1 =
+              __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)(a0 + 8 * D));
+          union {
+            s16x4_t h[2];
+            bf16x8_t v;
+          } a;
+          a.h[0] = v0;
+          a.h[1] = v1;
+#pragma unroll
+          for (int part = PARTS - 1; part >= 0; --part)
+            o[b] = mfma32(a.v, pf[part][kc], o[b]);
+        }
+      }
+    }
+    if (t + 1 < t_hi) commit(buf ^ 1);
+  }
+
+  if (q0 >= q_len) return;
+  const int qrow = q0 + (lane & 31);
+  l = half_sum(l);
+  if (qrow >= q_len) return;
+  const long tok = q_start + qrow;
+  float inv;
+  if constexpr (PARTS == 1) {
+    inv = l > 0.f ? 1.f / l : 0.f;
+  } else {
+    if (p.x.sink) {
+      // exp(sink) joins the denominator; the larger of the two maxima scales
+      const float sl = p.x.sink[head] * LOG2E, ml = m * c2, top = fmaxf(ml, sl);
+      const float f = exp2f(ml - top);
+      l = l * f + exp2f(sl - top);
+      inv = f / l;
+    } else {
+      inv = 1.f / l;
+    }
+    inv *= sigmoid_gate(p.x, tok, head);
+  }
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4_t w;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) w[r] = o[b][g * 4 + r] * inv;
+      store4(p.out, (tok * p.Hq + head) * D + half * 4 + b * 32 + g * 8, w,
+             PARTS == 1 ? 0 : p.x.out_f32);
+    }
+}
+
+// over the four lanes that share a column (lane & 15)
+__device__ __forceinline__ float column_max(float x) {
+  const unsigned int u = __float_as_uint(x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned int v = __float_as_uint(
+      fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1])));
+  const auto b = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float column_sum(float x) {
+  x += __shfl_xor(x, 16, 64);
+  return x + __shfl_xor(x, 32, 64);
+}
+
+// the pages of a sequence that are read, in pairs, and how they are split
+struct Range {
+  int first, last;  // page numbers
+  int pairs;
+  int splits;       // of the launched ones, those with work
+  int per;          // pairs per split
+};
+__device__ __forceinline__ Range page_range(int ctx, int window, int chunk,
+                                            int n_splits, int waves) {
+  Range r;
+  const int lo = ctx > 0 ? low_of(ctx - 1, window, chunk) : 0;
+  r.first = lo / PAGE;
+  r.last = (ctx - 1) / PAGE;
+  r.pairs = ctx > 0 ? (r.last - r.first) / 2 + 1 : 0;
+  // a pair per wave at least
+  r.splits = max(1, min(n_splits, (r.pairs + waves - 1) / waves));
+  r.per = (r.pairs + r.splits - 1) / r.splits;
+  return r;
+}
+
+struct DecodeArgs {
+  void* out;                // [S, H, D]
+  const void* q;            // [S, H, D] bf16 (PARTS 1) or fp32, row stride sq
+  const void* k_cache;      // [NB, Hkv, 16, D], rows sk elements apart
+  const void* v_cache;      // likewise, sv
+  const int* block_tables;  // [S, max_blocks]
+  const int* ctx_lens;      // [S]
+  float scale;
+  int H, Hkv, group, max_blocks;
+  long sq;
+  int n_splits;
+  float* part_out;  // [S, H, n_splits, D]
+  float* part_ml;   // [S, H, n_splits, 2]
+  int window;
+  long sk, sv;
+  const int* cu_q;  // [S+1] first token of a sequence (null: sequence s's is s)
+  Extra x;
+};
+
+// query token of sequence s, -1 if it has none in this batch
+__device__ __forceinline__ int token_of(const DecodeArgs& p, int s) {
+  if (!p.cu_q) return s;
+  return p.cu_q[s + 1] > p.cu_q[s] ? p.cu_q[s] : -1;
+}
+
+// what a (token, head)'s weighted values are multiplied by: their largest
+// exponent m (log2) and the sum of the weights relative to it
+template <int PARTS>
+__device__ __forceinline__ float final_factor(const DecodeArgs& p, long tok, int head,
+                                              float m, float sum) {
+  if constexpr (PARTS == 1) {
+    return sum > 0.f ? 1.f / sum : 0.f;
+  } else {
+    float f = 1.f;
+    if (p.x.sink) {
+      const float sl = p.x.sink[head] * LOG2E, top = fmaxf(m, sl);
+      f = exp2f(m - top);
+      sum = sum * f + exp2f(sl - top);
+    }
+    return f / sum * sigmoid_gate(p.x, tok, head);
+  }
+}
+
+template <int D, int NW, int SRC, bool WIDE, int PARTS = 1>  // WIDE: groups of 6 to 8
+__global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
+    const DecodeArgs p) {
+  constexpr int KC = D / 32;           // contraction chunks of K Q^T
+  constexpr int DB = D / 16;           // 16-column blocks of the output
+  constexpr int ROWS = 2 * PAGE;       // rows of a stage (a pair of pages)
+  constexpr int STAGE = 2 * ROWS * D;  // K rows, then V rows
+  constexpr int RING = SRC == PAGES_DMA ? 2 : 1;
+  // elements per lane and load, loads per stage and tensor
+  constexpr int EPL = SRC == PAGES_FP8 ? 16 : 8;
+  constexpr int LPR = D / EPL;  // lanes per row
+  constexpr int RPI = 64 / LPR;
+  constexpr int NI = ROWS / RPI;
+
+  const int kvh = blockIdx.x, s = blockIdx.y, split = blockIdx.z;
+  const int ctx = p.ctx_lens[s];
+  const Range rg = page_range(ctx, p.window, p.x.chunk, p.n_splits, NW);
+  const int tok = token_of(p, s);
+  if (split >= rg.splits || tok < 0) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int G = p.group;
+  const int part = col / G;  // of the weights: high, middle, low
+  const bool used = part < (WIDE ? 2 : 3);
+
+  __shared__ __attribute__((aligned(16))) short lds[NW][RING][STAGE];
+  static_assert(RING * STAGE * 2 >= 8 * (D + 4) * 4 + 64, "merge area");
+
+  bf16x8_t qf[PARTS][KC];
+  {
+    const long at = (long)tok * p.sq + (long)(kvh * G + col % G) * D + g * 8;
+    if constexpr (PARTS == 1) {
+      const short* qp = reinterpret_cast<const short*>(p.q) + at;
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        short8_t x = *reinterpret_cast<const short8_t*>(qp + c * 32);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = used ? x[j] : 0;
+        qf[0][c] = __builtin_bit_cast(bf16x8_t, x);
+      }
+    } else {
+      const float* qp = reinterpret_cast<const float*>(p.q) + at;
+#pragma unroll
+      for (int c = 0; c < KC; ++c)
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+          const f32x4_t x = *reinterpret_cast<const f32x4_t*>(qp + c * 32 + j);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const Split3 w(used ? x[e] : 0.f);
+            qf[0][c][j + e] = w.hi;
+            qf[1][c][j + e] = w.mid;
+            qf[2][c][j + e] = w.lo;
+          }
+        }
+    }
+  }
+
+  const int* bt = p.block_tables + (long)s * p.max_blocks;
+  const int lrow = lane / LPR, lchunk = lane % LPR;
+  struct Pages {
+    int a, b;
+  };
+  // page ids of pair n (past the end: the last page again, as its rows are)
+  auto pages_of = [&](int n) {
+    const int a = min(rg.first + 2 * n, rg.last), b = min(a + 1, rg.last);
+    return Pages{bt[a], bt[b]};
+  };
+  // where this lane's bytes of load i come from; rows past the context repeat
+  // its last one (their weights are 0, their values finite)
+  auto src = [&](const void* cache, long stride, int n, Pages pg, int i, int chunk) {
+    constexpr int ES = SRC == PAGES_FP8 ? 1 : 2;
+    const bool second = i >= NI / 2;
+    const int number = min(rg.first + 2 * n + (second ? 1 : 0), rg.last);
+    const int row = min((i % (NI / 2)) * RPI + lrow, ctx - 1 - number * PAGE);
+    const long st = PARTS == 1 ? D : stride;  // bf16 queries: whole rows
+    return reinterpret_cast<const char*>(cache) +
+           ((long)(second ? pg.b : pg.a) * p.Hkv + kvh) * PAGE * st * ES +
+           (row * (int)st + chunk * EPL) * ES;
+  };
+  auto load_dma = [&](int n, Pages pg, int slot) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int r = i * RPI + lrow;
+      short* dst = &lds[wave][slot][i * RPI * D];
+      __builtin_amdgcn_global_load_lds(
+          reinterpret_cast<const unsigned int*>(
+              src(p.k_cache, p.sk, n, pg, i, lchunk ^ k_swz<D>(r))),
+          reinterpret_cast<unsigned int*>(dst), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(
+          reinterpret_cast<const unsigned int*>(
+              src(p.v_cache, p.sv, n, pg, i, lchunk ^ v_swz<D>(r))),
+          reinterpret_cast<unsigned int*>(dst + ROWS * D), 16, 0, 0);
+    }
+  };
+  uint4 raw[SRC == PAGES_DMA ? 1 : 2 * NI];
+  auto load_reg = [&](int n, Pages pg) {
+    if constexpr (SRC != PAGES_DMA) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        raw[2 * i] = *reinterpret_cast<const uint4*>(src(p.k_cache, p.sk, n, pg, i, lchunk));
+        raw[2 * i + 1] =
+            *reinterpret_cast<const uint4*>(src(p.v_cache, p.sv, n, pg, i, lchunk));
+      }
+    }
+  };
+  auto commit = [&]() {
+    if constexpr (SRC != PAGES_DMA) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int r = i * RPI + lrow;
+#pragma unroll
+        for (int kv = 0; kv < 2; ++kv) {
+          short* row = &lds[wave][0][kv * ROWS * D + r * D];
+          const int sw = kv ? v_swz<D>(r) : k_swz<D>(r);
+          const uint4 x = raw[2 * i + kv];
+          if constexpr (SRC == PAGES_REG) {
+            *reinterpret_cast<uint4*>(row + (lchunk ^ sw) * 8) = x;
+          } else {
+            const unsigned int w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              uint4 o;
+              o.x = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h], 1.0f, false));
+              o.y = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h], 1.0f, true));
+              o.z = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h + 1], 1.0f, false));
+              o.w = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h + 1], 1.0f, true));
+              *reinterpret_cast<uint4*>(row + ((2 * lchunk + h) ^ sw) * 8) = o;
+            }
+          }
+        }
+      }
+    }
+  };
+
+  // operand addresses inside a stage (elements)
+  int kaddr[KC];
+#pragma unroll
+  for (int c = 0; c < KC; ++c)
+    kaddr[c] = col * D + ((4 * c + g) ^ k_swz<D>(col)) * 8;
+  // transposing load: lane i of 16 brings key i/4, columns 4 (i%4) .. + 3 and
+  // receives column i of its four keys
+  const int vrow = g * 4 + (col >> 2);
+  int vaddr[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b)
+    vaddr[b] = ROWS * D + vrow * D +
+               ((2 * b + ((col & 3) >> 1)) ^ v_swz<D>(vrow)) * 8 + (col & 1) * 4;
+
+  float c2 = p.scale * 1.44269504088896340736f;
+  const bool flip = c2 < 0.f;
+  c2 = fabsf(c2);
+  const int key_lo = low_of(ctx - 1, p.window, p.x.chunk);  // first visible key
+  float m = NO_MAX, l = 0.f;
+  f32x4_t o[DB];
+#pragma unroll
+  for (int b = 0; b < DB; ++b) o[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  auto compute = [&](int n, const short* st) {
+    f32x4_t sc[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      sc[h] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      f32x4_t rest = sc[h];  // the products with the query's lower parts
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const bf16x8_t a =
+            *reinterpret_cast<const bf16x8_t*>(st + h * PAGE * D + kaddr[c]);
+        if constexpr (PARTS == 3) {
+          rest = mfma16x16x32(a, qf[PARTS - 1][c], rest);
+          rest = mfma16x16x32(a, qf[PARTS - 2][c], rest);
+        }
+        sc[h] = mfma16x16x32(a, qf[0][c], sc[h]);
+      }
+      if constexpr (PARTS == 3) sc[h] += rest;
+    }
+    if (flip) {
+      sc[0] = -sc[0];
+      sc[1] = -sc[1];
+    }
+    const int key0 = (rg.first + 2 * n) * PAGE;
+    if (key0 + ROWS > ctx || key0 < key_lo) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = key0 + h * PAGE + g * 4 + r;
+          sc[h][r] = key < ctx && key >= key_lo ? sc[h][r] : MASKED;
+        }
+    }
+    float mx = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
+                     fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
+    mx = column_max(mx);
+    if (__any(mx > m)) {
+      const float mn = fmaxf(m, mx);
+      const float f = __builtin_amdgcn_exp2f((m - mn) * c2);
+      m = mn;
+      l *= f;
+#pragma unroll
+      for (int b = 0; b < DB; ++b) o[b] *= f;
+    }
+    const float mc = m * c2;
+    bf16x8_t pf, pl;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float w = __builtin_amdgcn_exp2f(sc[h][r] * c2 - mc);
+        l += w;
+        const Split3 w3(w);
+        if constexpr (WIDE) {
+          pf[h * 4 + r] = part == 0 ? w3.hi : w3.mid;
+          pl[h * 4 + r] = part == 0 ? w3.lo : (__bf16)0.f;
+        } else {
+          pf[h * 4 + r] = part == 0 ? w3.hi : part == 1 ? w3.mid : w3.lo;
+        }
+      }
+#pragma unroll
+    for (int b = 0; b < DB; ++b) {
+      typedef __attribute__((address_space(3))) s16x4_t lds4_t;
+      const short* a0 = st + vaddr[b];
+      union {
+        s16x4_t h[2];
+        bf16x8_t v;
+      } a;
+      a.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)a0);
+      a.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)(a0 + PAGE * D));
+      o[b] = mfma16x16x32(a.v, pf, o[b]);
+      if constexpr (WIDE) o[b] = mfma16x16x32(a.v, pl, o[b]);
+    }
+  };
+
+  const int n_lo = split * rg.per + wave;
+  const int n_hi = min((split + 1) * rg.per, rg.pairs);
+  if constexpr (SRC == PAGES_DMA) {
+    // s_waitcnt immediates (vmcnt in bits 3:0 and 15:14; no wait on the rest)
+    constexpr int NL = 2 * NI;  // loads of one stage
+    constexpr int WAIT_STAGE = (0xF << 8) | (0x7 << 4) | (NL & 0xF) | ((NL >> 4) << 14);
+    constexpr int WAIT_ALL = (0xF << 8) | (0x7 << 4);
+    if (n_lo < n_hi) load_dma(n_lo, pages_of(n_lo), 0);
+    if (n_lo + NW < n_hi) load_dma(n_lo + NW, pages_of(n_lo + NW), 1);
+    int slot = 0;
+    for (int n = n_lo; n < n_hi; n += NW, slot ^= 1) {
+      const int next = n + 2 * NW;
+      Pages pg{0, 0};
+      if (next < n_hi) pg = pages_of(next);
+      if (n + NW < n_hi) __builtin_amdgcn_s_waitcnt(WAIT_STAGE);
+      else __builtin_amdgcn_s_waitcnt(WAIT_ALL);
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+      compute(n, lds[wave][slot]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (next < n_hi) load_dma(next, pg, slot);
+    }
+  } else {
+    if (n_lo < n_hi) load_reg(n_lo, pages_of(n_lo));
+    for (int n = n_lo; n < n_hi; n += NW) {
+      commit();
+      if (n + NW < n_hi) load_reg(n + NW, pages_of(n + NW));
+      compute(n, lds[wave][0]);
+    }
+  }
+
+  // ---- merge: the parts of the weights, then the waves ----
+  l = column_sum(l);
+  float* mo = reinterpret_cast<float*>(lds[wave]);  // [8][D + 4], then m and l
+  float* mm = mo + 8 * (D + 4);
+#pragma unroll
+  for (int b = 0; b < DB; ++b) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float x = o[b][r] + __shfl(o[b][r], lane + G, 64);
+      if constexpr (!WIDE) x += __shfl(o[b][r], lane + 2 * G, 64);
+      o[b][r] = x;
+    }
+    if (col < G)
+      *reinterpret_cast<f32x4_t*>(mo + col * (D + 4) + b * 16 + g * 4) = o[b];
+  }
+  if (lane < G) {
+    mm[lane] = m;
+    mm[8 + lane] = l;
+  }
+  __syncthreads();
+  constexpr int WF = RING * STAGE / 2;  // floats between the waves' areas
+  const float* all = reinterpret_cast<const float*>(lds);
+  for (int i = threadIdx.x; i < G * (D / 4); i += NW * 64) {
+    const int h = i / (D / 4), d = i % (D / 4) * 4;
+    float top = NO_MAX;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) top = fmaxf(top, all[w * WF + 8 * (D + 4) + h]);
+    float sum = 0.f;
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float* a = all + w * WF;
+      const float f = __builtin_amdgcn_exp2f((a[8 * (D + 4) + h] - top) * c2);
+      sum += f * a[8 * (D + 4) + 8 + h];
+      acc += f * *reinterpret_cast<const f32x4_t*>(a + h * (D + 4) + d);
+    }
+    const int head = kvh * G + h;
+    if (rg.splits == 1) {
+      const float f = final_factor<PARTS>(p, tok, head, top * c2, sum);
+      store4(p.out, ((long)tok * p.H + head) * D + d, acc * f,
+             PARTS == 1 ? 0 : p.x.out_f32);
+    } else {
+      const long at = ((long)s * p.H + head) * p.n_splits + split;
+      *reinterpret_cast<f32x4_t*>(p.part_out + at * D + d) = acc;
+      if (d == 0) {
+        p.part_ml[at * 2] = top * c2;
+        p.part_ml[at * 2 + 1] = sum;
+      }
+    }
+  }
+}
+
+// Combine split-context partials: one wave per (seq, head); a lane owns D/64
+// columns across all splits. Sequences that one split covers are done.
+template <int D, int NW, int PARTS = 1>
+__global__ __launch_bounds__(256) void paged_attention_reduce_kernel(
+    const DecodeArgs p, long total) {
+  constexpr int ACC = D / 64;
+  const long sh = blockIdx.x * 4L + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (sh >= total) return;
+  const int s = sh / p.H;
+  const Range rg = page_range(p.ctx_lens[s], p.window, p.x.chunk, p.n_splits, NW);
+  const int tok = token_of(p, s);
+  if (rg.splits == 1 || tok < 0) return;
+  const float* ml = p.part_ml + sh * p.n_splits * 2;
+  float m = NO_MAX * 1e6f;
+  for (int sp = lane; sp < rg.splits; sp += 64) m = fmaxf(m, ml[sp * 2]);
+  m = wave_reduce_max(m);
+  float l = 0.f, acc[ACC];
+#pragma unroll
+  for (int a = 0; a < ACC; ++a) acc[a] = 0.f;
+#pragma unroll 4
+  for (int sp = 0; sp < rg.splits; ++sp) {
+    const float w = __builtin_amdgcn_exp2f(ml[sp * 2] - m);
+    l += w * ml[sp * 2 + 1];
+    const float* po = p.part_out + (sh * p.n_splits + sp) * D + lane * ACC;
+#pragma unroll
+    for (int a = 0; a < ACC; ++a) acc[a] += w * po[a];
+  }
+  const float f = final_factor<PARTS>(p, tok, sh % p.H, m, l);
+  const long at = ((long)tok * p.H + sh % p.H) * D + lane * ACC;
+#pragma unroll
+  for (int a = 0; a < ACC; ++a) {
+    if (PARTS == 3 && p.x.out_f32) reinterpret_cast<float*>(p.out)[at + a] = acc[a] * f;
+    else reinterpret_cast<short*>(p.out)[at + a] = float_to_bf16_bits(acc[a] * f);
+  }
+}
+
+// Two waves per block: 64 KB of LDS, two blocks per compute unit, so one
+// block's first loads run under the other's last ones. (256 sequences of 819 to
+// 3277 tokens: 389 us with 2 waves, 390 with 4, 431 with 1; 64 of 400 to 1600:
+// 48.4 / 50.0 / 66.4.)
+constexpr int WAVES = 2;
+
+template <int D, int SRC, int PARTS = 1>
+hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) {
+  const dim3 grid(p.Hkv, num_seqs, p.n_splits);
+  if (3 * p.group <= 16)
+    hipLaunchKernelGGL((paged_attention_kernel<D, WAVES, SRC, false, PARTS>), grid,
+                       dim3(WAVES * 64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((paged_attention_kernel<D, WAVES, SRC, true, PARTS>), grid,
+                       dim3(WAVES * 64), 0, stream, p);
+  HIP_CHECK_KERNEL();
+  if (p.n_splits > 1) {
+    const long sh = (long)num_seqs * p.H;
+    hipLaunchKernelGGL((paged_attention_reduce_kernel<D, WAVES, PARTS>),
+                       dim3((unsigned)((sh + 3) / 4)), dim3(256), 0, stream, p, sh);
+    HIP_CHECK_KERNEL();
+  }
+  return hipSuccess;
+}
+
+// Context splits for a launch over num_seqs x num_kv_heads: none from 512
+// blocks on, which fill the chip (64 sequences, 8 KV heads: 48.4 us unsplit,
+// 51.4 with 2 splits, 50.4 with 4; 96 of 3000, E4M3: 128 / 140 / 129), about
+// 640 blocks below that (24 sequences of 900: 30.4 us with 3 splits, 27.4 with
+// 4, 29.8 with 6; 8 of 600: 9.3 with 8, 11.9 with 16), and at most 32 (one of
+// 7000: 12.0 us with 32, 12.8 with 64, 14.7 with 16). A sequence uses as many
+// of them as it has page pairs for every wave.
+inline int decode_splits(int num_seqs, int num_kv_heads, int max_blocks) {
+  const long base = (long)num_seqs * num_kv_heads;
+  if (base <= 0 || base >= 512) return 1;
+  long n = (640 + base - 1) / base;
+  const long most = ((long)max_blocks + 2 * WAVES - 1) / (2 * WAVES);
+  if (n > most) n = most;
+  if (n > 32) n = 32;
+  return n < 1 ? 1 : (int)n;
+}
+
+}  // namespace mfma_attn
+}  // namespace

@@ -396,3 +396,90 @@ class TestAttention:
         close(out[0, :DV], want, be)
         close(out[0, DV:], want, be)
         assert (want - v.to(be[1])[3].double()).abs().max() < 1e-3
+
+
+def attention_64(q, kc, vc, bt, qlens, ctx, scale, H, gate, sink, window, chunk):
+    """Paged causal attention in float64, sequence by sequence."""
+    _, G, bs, D = kc.shape
+    out = []
+    at = 0
+    for i, (n, c) in enumerate(zip(qlens, ctx)):
+        pages = bt[i, : -(-c // bs)].long()
+        k = kc[pages].double().transpose(1, 2).reshape(-1, G, D)[:c]
+        v = vc[pages].double().transpose(1, 2).reshape(-1, G, vc.shape[3])[:c]
+        pos = torch.arange(n) + c - n
+        j = torch.arange(c)
+        vis = j[None] <= pos[:, None]
+        if window:
+            vis &= j[None] > pos[:, None] - window
+        if chunk:
+            vis &= j[None] >= (pos // chunk * chunk)[:, None]
+        for h in range(H):
+            s = q[at : at + n, h * D : (h + 1) * D].double() @ k[:, h * G // H].t() * scale
+            s = s.masked_fill(~vis, float("-inf"))
+            if sink is not None:
+                s = torch.cat([s, sink[h].double().expand(n, 1)], 1)
+            y = torch.softmax(s, -1)[:, :c] @ v[:, h * G // H]
+            if gate is not None:
+                y = y * torch.sigmoid(gate[at : at + n, h : h + 1].double())
+            out.append(y)
+        at += n
+    rows, at = [], 0
+    for i, n in enumerate(qlens):
+        rows.append(torch.cat(out[at : at + H], 1))
+        at += H
+    return torch.cat(rows)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "window,chunk,gated,sunk", [(0, 0, False, False), (40, 0, True, True), (0, 32, False, True)]
+)
+@pytest.mark.parametrize(
+    "H,G,D,off",
+    [
+        (4, 1, 128, 0), (6, 3, 64, 0), (3, 3, 128, 0), (8, 1, 64, 0), (16, 1, 128, 0),
+        (4, 1, 128, 1),  # odd page addresses: the fp32 products
+    ],
+)
+@pytest.mark.parametrize("decode", [False, True])
+def test_attention_parts(decode, H, G, D, off, window, chunk, gated, sunk):
+    """bf16 pages of 16: the fp32 operands in three bf16 parts lose nothing.
+    Portions around the 32/64/128-row tiles and contexts that end anywhere in
+    a page; NaN in the rows that no sequence owns."""
+    ctx = [1, 17, 64, 200, 2000, 333] if decode else [1, 33, 200, 130, 333]
+    qlens = [1] * 6 if decode else [1, 33, 64, 130, 5]
+    g = torch.Generator().manual_seed(H + D)
+    nb = [-(-c // 16) for c in ctx]
+    NB = sum(nb) + 2
+    pages = []
+    for _ in range(2):
+        flat = torch.randn(NB * G * 16 * D + off, generator=g).to(torch.bfloat16)
+        pages.append(flat)
+    order = torch.randperm(NB, generator=g)
+    bt = torch.zeros(len(ctx), max(nb) + 2, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(nb):
+        bt[i, :n] = order[at : at + n]
+        at += n
+    kc, vc = (x[off:].view(NB, G, 16, D) for x in pages)
+    T = sum(qlens)
+    q = torch.randn(T, H * D, generator=g) * 1.3
+    gate = torch.randn(T, H + 5, generator=g).to(torch.bfloat16)[:, 3 : 3 + H] if gated else None
+    sink = torch.randn(H, generator=g) if sunk else None
+    want = attention_64(q, kc, vc, bt, qlens, ctx, D ** -0.5, H, gate, sink, window, chunk)
+    for i, c in enumerate(ctx):
+        if c % 16:
+            for x in (kc, vc):
+                x[bt[i, nb[i] - 1].long(), :, c % 16 :] = float("nan")
+    dev_pages = [x.cuda()[off:].view(NB, G, 16, D) for x in pages]
+    cu = torch.tensor([0] + list(torch.tensor(qlens).cumsum(0)), dtype=torch.int32)
+    got = ops.ctx_attention_f32(
+        q.cuda(), dev_pages[0], dev_pages[1], bt.cuda(), cu.cuda(),
+        torch.tensor(ctx, dtype=torch.int32).cuda(), D ** -0.5, max(qlens), H,
+        gate=gate.cuda() if gated else None, sink=sink.cuda() if sunk else None,
+        window=window, chunk=chunk,
+    ).double().cpu()
+    # fp32 sums over up to 2000 keys: a few units in the last place (6e-8)
+    err = (got - want).norm() / want.norm()
+    assert err < 1e-6, float(err)
