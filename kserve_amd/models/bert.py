@@ -137,19 +137,24 @@ class BertModel(nn.Module):
         cu_seqlens: torch.Tensor,     # [num_seqs + 1] int32
         token_type_ids: Optional[torch.Tensor] = None,
     ) -> torch.Tensor:
-        device = input_ids.device
-        # per-sequence positions
         lens = cu_seqlens[1:] - cu_seqlens[:-1]
-        positions = torch.cat(
-            [torch.arange(int(n), device=device) for n in lens]
+        # one transfer for what the host needs to know, behind the embedding
+        stats = torch.stack([lens.max(), lens.min(), lens.sum()])
+        hidden = ops.embed_layer_norm(
+            self.word_embeddings, self.position_embeddings,
+            self.token_type_embeddings, input_ids, cu_seqlens, token_type_ids,
+            self.emb_ln_w, self.emb_ln_b, self.config.layer_norm_eps,
         )
-        emb = self.word_embeddings[input_ids] + self.position_embeddings[positions]
-        if token_type_ids is None:
-            emb = emb + self.token_type_embeddings[0]
-        else:
-            emb = emb + self.token_type_embeddings[token_type_ids]
-        hidden = ops.layer_norm(emb, self.emb_ln_w, self.emb_ln_b, self.config.layer_norm_eps)
-        max_seqlen = int(lens.max())
+        max_seqlen, shortest, tokens = stats.tolist()
+        if shortest < 0 or tokens != input_ids.shape[0]:
+            raise ValueError(
+                f"cu_seqlens covers {tokens} tokens of {input_ids.shape[0]}"
+            )
+        if max_seqlen > self.position_embeddings.shape[0]:
+            raise IndexError(
+                f"sequence of {max_seqlen} tokens: the model has "
+                f"{self.position_embeddings.shape[0]} positions"
+            )
         for layer in self.layers:
             hidden = layer(hidden, cu_seqlens, max_seqlen)
         return hidden
@@ -238,8 +243,7 @@ class BertForMaskedLM(nn.Module):
         hidden = self.bert(input_ids, cu_seqlens, token_type_ids)
         t = ops.gelu(ops.linear(hidden, self.transform_w, self.transform_b))
         t = ops.layer_norm(t, self.transform_ln_w, self.transform_ln_b, self.eps)
-        logits = ops.linear(t, self.bert.word_embeddings) + self.decoder_bias
-        return logits
+        return ops.linear(t, self.bert.word_embeddings, self.decoder_bias)
 
     @torch.no_grad()
     def load_hf_state_dict(self, sd: Dict[str, torch.Tensor]):

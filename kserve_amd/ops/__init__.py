@@ -267,6 +267,27 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     return F.linear(x, weight, bias)
 
 
+def embed_layer_norm(
+    word, pos_table, type_table, ids, cu_seqlens, types, weight, bias, eps: float
+):
+    """LayerNorm of word[id] + pos_table[place in its sequence] +
+    type_table[type] (``types`` None: type 0) for flat varlen tokens. On the
+    GPU an index outside its table gives a row of NaN."""
+    if word.is_cuda and word.shape[1] <= 2048:  # the kernel's row in registers
+        out = torch.empty(
+            (ids.numel(), word.shape[1]), dtype=word.dtype, device=word.device
+        )
+        _native("embed_layer_norm").embed_layer_norm(
+            out, word, pos_table, type_table, ids.to(torch.int64).contiguous(),
+            None if types is None else types.to(torch.int64).contiguous(),
+            cu_seqlens.to(torch.int32).contiguous(), weight, bias, eps,
+        )
+        return out
+    return torch_ref.embed_layer_norm(
+        word, pos_table, type_table, ids, cu_seqlens, types, weight, bias, eps
+    )
+
+
 def layer_norm(x, weight, bias, eps: float):
     if x.is_cuda:
         out = torch.empty_like(x)

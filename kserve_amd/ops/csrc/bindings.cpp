@@ -32,6 +32,10 @@ hipError_t ks_context_prefill_varlen(void*, const void*, const void*,
 hipError_t ks_reshape_and_cache_fp8(const void*, const void*, void*, void*,
                                     const void*, int, int, int, int, long,
                                     long, hipStream_t);
+hipError_t ks_embed_layer_norm(void*, const void*, const void*, const void*,
+                               const void*, const void*, const void*,
+                               const void*, const void*, float, int, int, int,
+                               int, int, int, hipStream_t);
 hipError_t ks_layer_norm(void*, const void*, const void*, const void*, float,
                          int, int, hipStream_t);
 hipError_t ks_fused_add_layer_norm(void*, const void*, const void*,
@@ -235,6 +239,43 @@ void context_prefill_varlen(at::Tensor& out, at::Tensor& q,
             "context_prefill_varlen");
 }
 
+void embed_layer_norm(at::Tensor& out, at::Tensor& word, at::Tensor& pos_table,
+                      at::Tensor& type_table, at::Tensor& ids,
+                      const c10::optional<at::Tensor>& types,
+                      at::Tensor& cu_seqlens, at::Tensor& weight,
+                      at::Tensor& bias, double eps) {
+  CHECK_BF16_CONTIG(out);
+  CHECK_BF16_CONTIG(word);
+  CHECK_BF16_CONTIG(pos_table);
+  CHECK_BF16_CONTIG(type_table);
+  CHECK_BF16_CONTIG(weight);
+  CHECK_BF16_CONTIG(bias);
+  const int64_t hidden = word.size(1), tokens = ids.numel();
+  TORCH_CHECK(ids.is_cuda() && ids.scalar_type() == at::kLong &&
+                  ids.is_contiguous(),
+              "ids int64");
+  TORCH_CHECK(cu_seqlens.is_cuda() && cu_seqlens.scalar_type() == at::kInt &&
+                  cu_seqlens.is_contiguous() && cu_seqlens.numel() >= 2,
+              "cu_seqlens int32 [seqs + 1]");
+  if (types.has_value())
+    TORCH_CHECK(types->is_cuda() && types->scalar_type() == at::kLong &&
+                    types->is_contiguous() && types->numel() == tokens,
+                "token types int64 [tokens]");
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == tokens && out.size(1) == hidden &&
+                  pos_table.size(1) == hidden && type_table.size(1) == hidden &&
+                  weight.numel() == hidden && bias.numel() == hidden,
+              "embed_layer_norm: shape mismatch");
+  check_hip(ks_embed_layer_norm(
+                out.data_ptr(), word.data_ptr(), pos_table.data_ptr(),
+                type_table.data_ptr(), ids.data_ptr(),
+                types.has_value() ? types->data_ptr() : nullptr,
+                cu_seqlens.data_ptr(), weight.data_ptr(), bias.data_ptr(),
+                (float)eps, (int)tokens, (int)cu_seqlens.numel() - 1, (int)hidden,
+                (int)word.size(0), (int)pos_table.size(0),
+                (int)type_table.size(0), current_stream()),
+            "embed_layer_norm");
+}
+
 void layer_norm(at::Tensor& out, at::Tensor& input, at::Tensor& weight,
                 at::Tensor& bias, double eps) {
   CHECK_BF16_CONTIG(out);
@@ -337,6 +378,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("causal") = true, pybind11::arg("window") = 0);
   m.def("context_prefill_varlen", &context_prefill_varlen,
         "MFMA prefill attention against the paged KV cache (chunked prefill)");
+  m.def("embed_layer_norm", &embed_layer_norm,
+        "word + position + type embedding rows and their LayerNorm (bf16)");
   m.def("layer_norm", &layer_norm, "LayerNorm (bf16)");
   m.def("fused_add_layer_norm", &fused_add_layer_norm,
         "residual-add + LayerNorm");

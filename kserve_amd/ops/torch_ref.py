@@ -290,6 +290,16 @@ def random_sample(
     return sorted_idx.gather(-1, choice.unsqueeze(-1)).squeeze(-1)
 
 
+def embed_layer_norm(
+    word, pos_table, type_table, ids, cu_seqlens, types, weight, bias, eps
+):
+    lens = cu_seqlens[1:] - cu_seqlens[:-1]
+    positions = torch.cat([torch.arange(int(n), device=ids.device) for n in lens])
+    emb = word[ids] + pos_table[positions]
+    emb = emb + (type_table[0] if types is None else type_table[types])
+    return layer_norm(emb, weight, bias, eps)
+
+
 def layer_norm(
     x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: float
 ) -> torch.Tensor:

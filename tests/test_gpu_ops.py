@@ -788,3 +788,55 @@ class TestSlidingWindowKernels:
             cl, scale, window=W,
         )
         bf16_close(got, ref)
+
+
+class TestEmbedLayerNorm:
+    @pytest.mark.parametrize("hidden", [64, 768, 1032, 2048])
+    @pytest.mark.parametrize("typed", [False, True])
+    def test_against_fp32(self, dev, hidden, typed):
+        """Row widths below, at and above a wave's vectors, empty and full
+        sequences, negative ids."""
+        from kserve_amd import ops
+
+        g = torch.Generator().manual_seed(hidden)
+
+        def table(n):
+            return torch.randn(n, hidden, generator=g).to(torch.bfloat16)
+
+        word, pos, ty = table(50), table(40), table(2)
+        w, b = table(1)[0], table(1)[0]
+        cu = torch.tensor([0, 0, 1, 41, 41, 58], dtype=torch.int32)
+        ids = torch.randint(-50, 50, (58,), generator=g)
+        types = torch.randint(0, 2, (58,), generator=g) if typed else None
+        got = ops.embed_layer_norm(
+            *(t.to(dev) for t in (word, pos, ty, ids, cu)),
+            None if types is None else types.to(dev), w.to(dev), b.to(dev), 1e-12,
+        )
+        ref = torch_ref.embed_layer_norm(
+            word.double(), pos.double(), ty.double(), ids, cu, types, w, b, 1e-12
+        )
+        bf16_close(got, ref, atol=1e-2, rtol=2 ** -8)
+
+    def test_indexes_outside_the_tables(self, dev):
+        from kserve_amd import ops
+
+        word = torch.randn(10, 64, device=dev).to(torch.bfloat16)
+        pos = torch.randn(3, 64, device=dev).to(torch.bfloat16)
+        ids = torch.tensor([1, 10, -11, 2, 3], device=dev)
+        cu = torch.tensor([0, 1, 2, 5], dtype=torch.int32, device=dev)
+        got = ops.embed_layer_norm(
+            word, pos[:2].contiguous(), pos, ids, cu, None, word[0], word[1], 1e-12
+        )
+        assert got.isnan().all(1).tolist() == [False, True, True, False, True]
+
+    def test_too_long_sequence_is_refused(self, dev):
+        from kserve_amd.models.bert import BertConfig, BertModel
+
+        model = BertModel(BertConfig.tiny(), dtype=torch.bfloat16, device="cuda")
+        ids = torch.zeros(129, dtype=torch.int64, device=dev)
+        cu = torch.tensor([0, 129], dtype=torch.int32, device=dev)
+        with pytest.raises(IndexError):
+            model(ids, cu)
+        with pytest.raises(ValueError):
+            model(ids[:100], cu)
+
