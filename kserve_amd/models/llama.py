@@ -145,13 +145,15 @@ class LlamaMLP(nn.Module):
         )
 
     def forward(self, x: torch.Tensor, meta=None) -> torch.Tensor:
-        gate_up = self.gate_up_proj(x)
         lora = meta.lora if meta is not None else None
-        if lora is not None:
+        if lora is None:
+            act = self.gate_up_proj(x, activate=True)
+        else:
+            gate_up = self.gate_up_proj(x)
             half = gate_up.shape[-1] // 2
             lora.apply(self.layer_idx, "gate_proj", x, gate_up, 0)
             lora.apply(self.layer_idx, "up_proj", x, gate_up, half)
-        act = ops.silu_and_mul(gate_up)
+            act = ops.silu_and_mul(gate_up)
         d_delta = (
             lora.delta_for(self.layer_idx, "down_proj", act)
             if lora is not None

@@ -238,33 +238,101 @@ def random_sample(
     )
 
 
-def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """GEMM dispatch: custom MFMA skinny-GEMM for decode-sized batches
-    (weight-streaming regime where hipBLASLt underperforms ~4x on gfx950 —
-    see tools/gemm_bench.py), hipBLASLt via F.linear otherwise."""
-    import torch.nn.functional as F
-
-    # measured crossover (tools/gemm_bench.py on MI355X): the custom kernel
-    # beats hipBLASLt only for small token batches on qkv/o-sized shapes;
-    # hipBLASLt keeps the wide-M / large-K / large-N shapes.
-    if (
+def _skinny_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """What the few-row kernels read directly: plain bf16 matrices on one GPU
+    with 16-byte aligned rows, outside autograd and its transforms."""
+    return (
         _C is not None
         and x.is_cuda
-        and bias is None
         and x.dim() == 2
-        and 0 < x.shape[0] <= 64
-        and weight.shape[0] % 64 == 0
-        and weight.shape[0] <= 8192
-        and weight.shape[1] % 64 == 0
-        and weight.shape[1] <= 8192
+        and weight.dim() == 2
+        and x.dtype == torch.bfloat16
+        and weight.dtype == torch.bfloat16
+        and x.device == weight.device
+        and 0 < x.shape[0] <= 256
+        and x.shape[1] == weight.shape[1]
+        and x.shape[1] > 0
+        and x.shape[1] % 64 == 0
         and x.stride(1) == 1
+        and x.stride(0) % 8 == 0
+        and weight.is_contiguous()
+        and type(x) in (torch.Tensor, torch.nn.Parameter)
+        and type(weight) in (torch.Tensor, torch.nn.Parameter)
+        and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+        and not torch._C._functorch.is_functorch_wrapped_tensor(weight)
+        and torch.autograd.forward_ad._current_level < 0
+        and not (
+            torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
+        )
+        and x.data_ptr() % 16 == 0
+        and weight.data_ptr() % 16 == 0
+    )
+
+
+def _skinny_rows(n: int, k: int, m: int) -> bool:
+    """Whether the few-row kernel beats the library at [n, k] x [m, k]^T
+    (MI355X, us, kernel / library, reduction of the K splits included).
+
+    Up to 48 rows it streams weights faster wherever there are enough of them
+    to outlast a launch: k 4096, m 32000 at 1 row 48 / 60, at 24 rows 50 / 60;
+    k 14336, m 4096 at 24 rows 27 / 32; but 512 x 512 4.6 / 4.2. Up to 64 rows
+    the widest ones are even (m 16384 38 / 35). Above, it gains where the
+    library does not split K over the chip: k 14336, m 4096 at 128 rows
+    36 / 76, k 4096, m 6144 22 / 26; and loses on small weights (2048 x 2048
+    15 / 11) and wide ones (m 16384 44 / 38). Past 192 rows the lighter of the
+    former turn (4096 x 4096 27 / 23 at 256 rows; m 6144 33 / 40)."""
+    weights = k * m
+    if m % 4 or weights < 1 << 20:
+        return False
+    if n <= 48 or (n <= 64 and m <= 8192):
+        return True
+    return 4096 <= m <= 10240 and weights >= (16 if n <= 192 else 24) << 20
+
+
+def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
+    """The same for the gate|up product with silu(gate) * up on its sums,
+    against the library's product and the activation kernel (k 4096, m 14336:
+    1 row 43 / 66, 48 rows 49 / 69, 96 rows 58 / 60, 192 rows 73 / 72). A
+    block takes 32 or, above 64 rows, 64 features and K is not split, so m
+    has to fill the chip (k 4096, m 3584 24 / 21 at 64 rows); above 16384
+    features the library is level (k 8192, m 28672 at 1 row 182 / 180)."""
+    if m % 4 or m > 16384:
+        return False
+    return (n <= 64 and m >= 4608) or (n <= 112 and m >= 12288)
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x @ weight^T (+ bias): a kernel of our own for the few rows of a decode
+    batch where it is the faster one, the library otherwise."""
+    if (
+        bias is None
+        and _skinny_operands(x, weight)
+        and _skinny_rows(x.shape[0], x.shape[1], weight.shape[0])
     ):
         out = torch.empty(
             (x.shape[0], weight.shape[0]), dtype=x.dtype, device=x.device
         )
         _C.skinny_gemm(out, x, weight)
         return out
-    return F.linear(x, weight, bias)
+    return torch.nn.functional.linear(x, weight, bias)
+
+
+def linear_silu_and_mul(
+    x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None
+) -> torch.Tensor:
+    """silu(gate) * up for [gate | up] = x @ weight^T (+ bias)."""
+    if (
+        bias is None
+        and _skinny_operands(x, weight)
+        and weight.shape[0] % 2 == 0
+        and _skinny_glu_rows(x.shape[0], x.shape[1], weight.shape[0] // 2)
+    ):
+        out = torch.empty(
+            (x.shape[0], weight.shape[0] // 2), dtype=x.dtype, device=x.device
+        )
+        _C.skinny_glu(out, x, weight)
+        return out
+    return silu_and_mul(linear(x, weight, bias))
 
 
 def embed_layer_norm(

@@ -43,8 +43,9 @@ hipError_t ks_fused_add_layer_norm(void*, const void*, const void*,
                                    hipStream_t);
 hipError_t ks_gelu(void*, const void*, long, hipStream_t);
 hipError_t ks_mfma_probe(void*, const void*, const void*, hipStream_t);
+int ks_skinny_splits(int, int, int, int);
 hipError_t ks_skinny_gemm(void*, void*, const void*, const void*, int, int,
-                          int, long, hipStream_t);
+                          int, long, int, int, hipStream_t);
 hipError_t ks_gemm8(void*, const void*, const void*, int, int, int, int,
                     hipStream_t);
 }
@@ -311,33 +312,40 @@ void gelu(at::Tensor& out, at::Tensor& input) {
             "gelu");
 }
 
-void skinny_gemm(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
-  // out [N, M] bf16 = x [N, K] @ w [M, K]^T  (decode shapes, N <= 256)
+static void skinny_product(at::Tensor& out, at::Tensor& x, at::Tensor& w,
+                           bool glu) {
   CHECK_BF16_CONTIG(out);
   CHECK_BF16_CONTIG(w);
-  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && x.is_cuda() &&
-                  x.stride(1) == 1,
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && x.is_cuda() && x.dim() == 2 &&
+                  w.dim() == 2 && out.dim() == 2 && x.stride(1) == 1,
               "x must be bf16 row-dense");
-  int N = x.size(0);
-  int K = x.size(1);
-  int M = w.size(0);
-  TORCH_CHECK(w.size(1) == K, "shape mismatch");
-  at::Tensor ws;
-  void* wsp = nullptr;
-  // mirror the kernel's K-split decision to size the partials workspace
-  int nsplit = 1;
-  int feat_wgs = M / 64;
-  while (feat_wgs * nsplit < 768 && nsplit < 8 && (K / (nsplit * 2)) >= 64)
-    nsplit *= 2;
-  if (nsplit > 1) {
-    // bf16 partials (each a full-precision-accumulated K/nsplit dot)
-    ws = at::empty({(long)nsplit * N * M},
-                   at::TensorOptions().dtype(at::kBFloat16).device(x.device()));
-    wsp = ws.data_ptr();
-  }
-  check_hip(ks_skinny_gemm(out.data_ptr(), wsp, x.data_ptr(), w.data_ptr(),
-                           M, K, N, (long)x.stride(0), current_stream()),
+  const long N = x.size(0), K = x.size(1), M = w.size(0) / (glu ? 2 : 1);
+  TORCH_CHECK(w.size(1) == K && w.size(0) == M * (glu ? 2 : 1) &&
+                  out.size(0) == N && out.size(1) == M,
+              "shape mismatch");
+  TORCH_CHECK(x.device() == w.device() && x.device() == out.device(),
+              "operands on different devices");
+  TORCH_CHECK(N >= 1 && N <= 256 && M < (1L << 30) && K < (1L << 30),
+              "size out of range");
+  const c10::DeviceGuard guard(x.device());
+  const int splits = ks_skinny_splits(M, K, N, glu);
+  at::Tensor part;  // fp32 sums of the K splits
+  if (splits > 1)
+    part = at::empty({splits * N * M}, x.options().dtype(at::kFloat));
+  check_hip(ks_skinny_gemm(out.data_ptr(), splits > 1 ? part.data_ptr() : nullptr,
+                           x.data_ptr(), w.data_ptr(), (int)M, (int)K, (int)N,
+                           (long)x.stride(0), splits, glu, current_stream()),
             "skinny_gemm");
+}
+
+void skinny_gemm(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
+  // out [N, M] = x [N, K] @ w [M, K]^T, bf16, N <= 256
+  skinny_product(out, x, w, false);
+}
+
+void skinny_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
+  // out [N, M] = silu(x @ w[:M]^T) * (x @ w[M:]^T), bf16, N <= 256
+  skinny_product(out, x, w, true);
 }
 
 void gemm8(at::Tensor& d, at::Tensor& a, at::Tensor& w, int64_t swizzle) {
@@ -386,6 +394,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gelu", &gelu, "erf GELU");
   def_sampling(m);
   m.def("skinny_gemm", &skinny_gemm, "decode GEMM (N<=256, MFMA streaming)");
+  m.def("skinny_glu", &skinny_glu, "gate|up GEMM (N<=256) with silu(gate) * up");
   m.def("gemm8", &gemm8,
         "EXPERIMENTAL 8-phase 256x256 MFMA GEMM");
   m.def("mfma_probe", &mfma_probe, "MFMA layout probe (tests)");

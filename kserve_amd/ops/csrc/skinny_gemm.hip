@@ -1,223 +1,272 @@
-// Skinny GEMM for decode-path projections: C[N][M] = X[N][K] @ W[M][K]^T,
-// N <= 256 tokens (weight-streaming regime where hipBLASLt reaches only
-// ~1-4 TB/s on gfx950; measured in tools/gemm_bench.py).
+// Products of few rows with a weight matrix: out[N][M] = x[N][K] w[M][K]^T for
+// N <= 256 tokens (decode batches, short prompts), where reading the weights
+// is what bounds them.
 //
-// m97-shaped CDNA4 structure (guide §5): both operands staged through LDS
-// via global_load_lds (16 B/lane) with PRE-SWIZZLED global sources so the
-// linear LDS destination equals the XOR-swizzled layout that makes the
-// ds_read_b128 fragment reads bank-conflict-free (rule #21: linear dest +
-// inverse-swizzled source + swizzled read share one involution). Two
-// barriers per K-step; cross-workgroup overlap hides HBM latency (m97
-// finding: implicit wave-level overlap ~ explicit pipelining).
+// A block takes 64 F features (16 F per wave) and all tokens over a range of
+// K, in steps of 64: each step's weight and token rows come by LDS-direct
+// loads into one slot of a ring, so up to S - 1 steps are in flight behind the
+// one that is multiplied, with one barrier per step. K is split over blocks
+// until the chip is full; the splits leave fp32 partial sums that a second
+// kernel adds in order (no atomics). With GLU the block's rows are as many
+// gate as up features and silu(gate) * up leaves it directly.
 //
-// The X tile is shared by all 4 waves (each wave owns 16 output features,
-// all token tiles). K-split fills the chip for small-M projections; the
-// splits write disjoint f32 partials reduced by a second kernel (no atomic
-// RMW contention).
+// Measured (us with the reduction, weights not in cache; the library's in
+// parentheses): K 4096, M 14336 GLU at 1 row 43 = 5.4 TB/s (66 with the
+// activation kernel), at 24 rows 46; K 4096, M 32000 at 1 row 48 (60); K
+// 14336, M 4096 at 1 / 24 / 96 / 256 rows 26 / 27 / 32 / 53 (27 / 32 / 63 / 62).
+// Up to 48 rows the loads bound it (non-temporal ones took 5 to 10 % off; no
+// gain above); above, LDS reads and the matrix cores of the few blocks that
+// fit, so wide M goes back to the library. The kernel before kept a barrier
+// per step behind one load in flight and rounded the splits to bf16.
+//
+// C = W X^T on v_mfma_f32_16x16x32_bf16: a lane ends with four consecutive
+// features of one token. LDS rows are 128 bytes; the 16-byte chunk c of row r
+// sits at c ^ ((r >> 1) & 7), so 16 rows at one chunk hit different banks; the
+// swizzle is on the source side of the loads.
 #include "common.h"
 #include "mfma_layouts.h"
 
 namespace {
 
-constexpr int BK = 64;           // K per stage step
-constexpr int FEAT_PER_WAVE = 16;
-constexpr int NWAVES = 4;        // 64 features per workgroup
+constexpr int BK = 64;  // K per step
+constexpr int NWAVES = 4;
+constexpr int NT_AUX = 2;  // cache policy of a non-temporal load
 
-// chunk = 8 bf16 = 16 B. Row-chunk swizzle: kc_lds = kc_src ^ (row & 7).
-__device__ __forceinline__ int lds_row_idx(int row, int kc) {
-  return (row * (BK / 8) + (kc ^ (row & 7))) * 8;  // shorts
-}
+enum Epilogue { BF16_OUT, PARTIAL, GLU };
 
-template <int NT, bool SPLIT>
-__global__ __launch_bounds__(256) void skinny_gemm_kernel(
-    short* __restrict__ out,      // [N][M] bf16 (!SPLIT)
-    short* __restrict__ out_ws,   // [nsplit][N][M] bf16 partials (SPLIT)
-    const short* __restrict__ x,  // [N][K] row stride xs
-    const short* __restrict__ w,  // [M][K]
-    const int M, const int K, const int N, const long xs,
-    const int k_per_split) {
-  const int wave = threadIdx.x >> 6;
+struct GemmArgs {
+  void* out;       // [N][M] bf16; PARTIAL: [splits][N][M] fp32
+  const short* x;  // [N][K], row stride xs
+  const short* w;  // [M][K]; GLU: [2 M][K], gate rows first
+  int M, K, N;
+  long xs;
+};
+
+// s_waitcnt with vmcnt <= n (bits 3:0 and 15:14), lgkmcnt 0, expcnt free
+constexpr int wait_imm(int n) { return (0x7 << 4) | (n & 0xF) | ((n >> 4) << 14); }
+
+template <int NT, int F, int S, int EPI>
+__global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
+  constexpr int BN = NT * 16, BM = NWAVES * F * 16;
+  constexpr int STAGE = (BN + BM) * BK;        // elements
+  constexpr int LOADS = (BN + BM) / 8;         // 1 KB loads of a step
+  constexpr int NI = (LOADS + NWAVES - 1) / NWAVES;
+  constexpr int REM = LOADS % NWAVES;          // waves < REM (or all) issue NI
+  static_assert(S >= 2 && S * STAGE * 2 <= 160 * 1024, "ring");
+  __shared__ __attribute__((aligned(16))) short ring[S * STAGE];
+
   const int lane = threadIdx.x & 63;
-  const int f_base = blockIdx.x * (NWAVES * FEAT_PER_WAVE);
-  const int k_lo = blockIdx.y * k_per_split;
-  const int k_hi = min(K, k_lo + k_per_split);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int steps = p.K / BK;
+  const int lo = (int)((long)steps * blockIdx.y / gridDim.y);
+  const int n = (int)((long)steps * (blockIdx.y + 1) / gridDim.y) - lo;
 
-  // LDS: double-buffered {X tile [NT*16][BK] | W tile [64][BK]}, swizzled,
-  // + one 1 KB scratch slot for stage-count padding
-  constexpr int X_CHUNKS = NT * 16 * (BK / 8);  // 16B chunks
-  constexpr int W_CHUNKS = 64 * (BK / 8);
-  constexpr int TOTAL_CHUNKS = X_CHUNKS + W_CHUNKS;
-  constexpr int NINSTR = TOTAL_CHUNKS / 64;          // wg-wide 1 KB instrs
-  constexpr int NI = (NINSTR + NWAVES - 1) / NWAVES;  // per-wave, padded
-  constexpr int TILE_SHORTS = (NT * 16 + 64) * BK;
-  __shared__ short tile[2][TILE_SHORTS];
-  __shared__ short scratch[512];  // dump target for padding instrs
-
-  f32x4_t acc[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const int m_local = lane & 15;
-  const int kgrp = lane >> 4;
-
-  // stage buf with the BK-slice at k-offset k0; every wave issues exactly
-  // NI instructions so the counted s_waitcnt below is uniform (T4)
-  auto stage = [&](int buf, int k0) {
-#pragma unroll
-    for (int ii = 0; ii < NI; ++ii) {
-      const int i = wave + ii * NWAVES;
-      const int g = i * 64 + lane;
-      const short* src;
-      short* dst;
-      if (i < NINSTR) {
-        dst = &tile[buf][i * 64 * 8];
-        if (g < X_CHUNKS) {
-          int row = g >> 3;  // token row
-          const int kc_src = (g & 7) ^ (row & 7);
-          if (row >= N) row = N - 1;  // clamp padded token rows
-          src = x + (long)row * xs + (kc_src << 3) + k0;
-        } else {
-          const int gw = g - X_CHUNKS;
-          const int m = gw >> 3;
-          const int kc_src = (gw & 7) ^ (m & 7);
-          src = w + (long)(f_base + m) * K + (kc_src << 3) + k0;
-        }
-      } else {  // padding instr keeps per-wave vmcnt uniform
-        dst = scratch;
-        src = x;
-      }
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const unsigned int*>(src),
-          reinterpret_cast<unsigned int*>(dst), 16, 0, 0);
+  // first feature of the block's W rows (GLU: of gate and up rows)
+  const int f0 = blockIdx.x * (EPI == GLU ? BM / 2 : BM);
+  auto w_row = [&](int r) {  // row of w for row r of the tile, clamped
+    if constexpr (EPI == GLU) {
+      const int f = min(f0 + (r < BM / 2 ? r : r - BM / 2), p.M - 1);
+      return r < BM / 2 ? f : p.M + f;
+    } else {
+      return min(f0 + r, p.M - 1);
     }
   };
+  // per load: where this lane's 16 bytes of step 0 come from
+  const bool full = REM == 0 || wave < REM;
+  const char* src[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = (wave + i * NWAVES) * 8 + (lane >> 3);  // row of the stage
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const short* row = r < BN ? p.x + (long)min(r, p.N - 1) * p.xs
+                              : p.w + (long)w_row(r - BN) * p.K;
+    src[i] = reinterpret_cast<const char*>(row + (long)lo * BK + c * 8);
+  }
+  int issue_slot = 0;
+  auto issue = [&]() {  // the next step's loads
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if (i < NI - 1 || full) {
+        const auto* from = reinterpret_cast<const unsigned int*>(src[i]);
+        auto* to = reinterpret_cast<unsigned int*>(
+            &ring[issue_slot * STAGE + (wave + i * NWAVES) * 8 * BK]);
+        if (wave + i * NWAVES < BN / 8)  // token rows: every block reads them
+          __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+        else
+          __builtin_amdgcn_global_load_lds(from, to, 16, 0, NT <= 3 ? NT_AUX : 0);
+        src[i] += BK * 2;
+      }
+    }
+    issue_slot = issue_slot + 1 == S ? 0 : issue_slot + 1;
+  };
 
-  // s_waitcnt imm waiting vmcnt==NI, ignore lgkm/exp (gfx9 encoding:
-  // vmcnt[3:0]|vmcnt[5:4]<<14, expcnt[6:4], lgkmcnt[11:8])
-  constexpr int WAIT_NI =
-      (0xF << 8) | (0x7 << 4) | (NI & 0xF) | (((NI >> 4) & 0x3) << 14);
-  constexpr int WAIT_0 = (0xF << 8) | (0x7 << 4);
+  f32x4_t acc[F][NT];
+#pragma unroll
+  for (int f = 0; f < F; ++f)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[f][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  // prologue: stage first slice into buf 0
-  int cur = 0;
-  stage(0, k_lo);
-  for (int k0 = k_lo; k0 < k_hi; k0 += BK) {
-    const int k_next = k0 + BK;
-    if (k_next < k_hi) {
-      stage(cur ^ 1, k_next);
-      __builtin_amdgcn_s_waitcnt(WAIT_NI);  // buf[cur] landed; next in flight
+  const int sw = ((col >> 1) & 7);
+  const int xat = col * BK, wat = (BN + wave * F * 16 + col) * BK;
+  for (int j = 0; j < S - 1 && j < n; ++j) issue();
+  int slot = 0;
+  for (int j = 0; j < n; ++j) {
+    // step j has landed (this wave's part; the barrier covers the others'),
+    // and every LDS read of step j - 1 is done
+    if (n - 1 - j >= S - 2) {
+      if (full) __builtin_amdgcn_s_waitcnt(wait_imm(NI * (S - 2)));
+      else __builtin_amdgcn_s_waitcnt(wait_imm((NI - 1) * (S - 2)));
     } else {
-      __builtin_amdgcn_s_waitcnt(WAIT_0);
+      __builtin_amdgcn_s_waitcnt(wait_imm(0));
     }
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();  // raw: no vmcnt drain (counted pipeline)
-    // ---- fragments + MFMA from buf[cur] ----
-    const int wf = NT * 16 + wave * FEAT_PER_WAVE;  // W row base in tile
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (j + S - 1 < n) issue();
+    const short* st = &ring[slot * STAGE];
+    slot = slot + 1 == S ? 0 : slot + 1;
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
-      const int kc = kk * 4 + kgrp;
-      bf16x8_t b = *reinterpret_cast<bf16x8_t*>(
-          &tile[cur][lds_row_idx(wf + m_local, kc)]);
+      const int c = ((kk * 4 + g) ^ sw) * 8;
+      bf16x8_t a[F];
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        a[f] = *reinterpret_cast<const bf16x8_t*>(st + wat + f * 16 * BK + c);
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        bf16x8_t a = *reinterpret_cast<bf16x8_t*>(
-            &tile[cur][lds_row_idx(t * 16 + m_local, kc)]);
-        acc[t] = mfma16x16x32(a, b, acc[t]);
+        const bf16x8_t b =
+            *reinterpret_cast<const bf16x8_t*>(st + xat + t * 16 * BK + c);
+#pragma unroll
+        for (int f = 0; f < F; ++f) acc[f][t] = mfma16x16x32(a[f], b, acc[f][t]);
       }
     }
-    __builtin_amdgcn_s_barrier();  // readers done before buf[cur] is reused
-    cur ^= 1;
   }
 
-  // ---- epilogue: C row = token, col = feature ----
-  const int feat = f_base + wave * FEAT_PER_WAVE + MFMA_C_COL(lane);
+  if constexpr (EPI == GLU) {
+    // up waves hand their sums to the gate waves through LDS
+    __syncthreads();
+    f32x4_t* up = reinterpret_cast<f32x4_t*>(ring);  // [2][F][NT][64]
+    if (wave >= 2) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
+      for (int f = 0; f < F; ++f)
 #pragma unroll
-    for (int reg = 0; reg < 4; ++reg) {
-      const int tokn = t * 16 + MFMA_C_ROW(lane, reg);
-      if (tokn < N) {
-        if constexpr (SPLIT) {
-          // bf16 partials: each is a full K/nsplit-length dot in f32 first,
-          // so the rounding is one bf16 quantization per partial
-          out_ws[((long)blockIdx.y * N + tokn) * M + feat] =
-              float_to_bf16_bits(acc[t][reg]);
-        } else {
-          out[(long)tokn * M + feat] = float_to_bf16_bits(acc[t][reg]);
+        for (int t = 0; t < NT; ++t)
+          up[(((wave - 2) * F + f) * NT + t) * 64 + lane] = acc[f][t];
+    }
+    __syncthreads();
+    if (wave >= 2) return;
+#pragma unroll
+    for (int f = 0; f < F; ++f)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const f32x4_t u = up[((wave * F + f) * NT + t) * 64 + lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float x = acc[f][t][r];
+          acc[f][t][r] = x / (1.f + __expf(-x)) * u[r];
         }
       }
+  }
+#pragma unroll
+  for (int f = 0; f < F; ++f) {
+    const int feat = f0 + (wave * F + f) * 16 + g * 4;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int tok = t * 16 + col;
+      if (tok >= p.N || feat >= p.M) continue;
+      if constexpr (EPI == PARTIAL) {
+        float* o = reinterpret_cast<float*>(p.out) +
+                   ((long)blockIdx.y * p.N + tok) * p.M + feat;
+        *reinterpret_cast<f32x4_t*>(o) = acc[f][t];
+      } else {
+        short4_t o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = float_to_bf16_bits(acc[f][t][r]);
+        *reinterpret_cast<short4_t*>(reinterpret_cast<short*>(p.out) +
+                                     (long)tok * p.M + feat) = o;
+      }
     }
   }
 }
 
-// sum bf16 partials (f32 accumulate) and store bf16
-__global__ void reduce_ws_kernel(short* __restrict__ out,
-                                 const short* __restrict__ ws, const long nm,
-                                 const int nsplit) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < nm;
-       i += (long)gridDim.x * blockDim.x) {
-    float acc = 0.f;
-    for (int s = 0; s < nsplit; ++s)
-      acc += bf16_bits_to_float(ws[s * nm + i]);
-    out[i] = float_to_bf16_bits(acc);
-  }
+// partial sums of the splits, added in order, as bf16; four per thread
+__global__ __launch_bounds__(256) void reduce_splits_kernel(
+    short* __restrict__ out, const float* __restrict__ part, const long nm,
+    const int splits) {
+  const long i = (blockIdx.x * 256L + threadIdx.x) * 4;
+  if (i >= nm) return;
+  f32x4_t a = *reinterpret_cast<const f32x4_t*>(part + i);
+  for (int s = 1; s < splits; ++s)
+    a += *reinterpret_cast<const f32x4_t*>(part + s * nm + i);
+  short4_t o;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = float_to_bf16_bits(a[r]);
+  *reinterpret_cast<short4_t*>(out + i) = o;
 }
 
-template <int NT>
-void launch_nt(short* out, short* ws, const short* x, const short* w, int M,
-               int K, int N, long xs, int nsplit, int k_per_split,
-               hipStream_t stream) {
-  dim3 grid(M / (NWAVES * FEAT_PER_WAVE), nsplit);
-  if (nsplit > 1) {
-    hipLaunchKernelGGL((skinny_gemm_kernel<NT, true>), grid, dim3(256), 0,
-                       stream, out, ws, x, w, M, K, N, xs, k_per_split);
-  } else {
-    hipLaunchKernelGGL((skinny_gemm_kernel<NT, false>), grid, dim3(256), 0,
-                       stream, out, ws, x, w, M, K, N, xs, k_per_split);
-  }
-}
+// token tiles, feature groups per wave and ring slots: two blocks per compute
+// unit up to 64 tokens, one with twice the features above
+#define FOR_TILE(N, GO)                 \
+  if ((N) <= 16) GO(1, 1, 8)            \
+  else if ((N) <= 32) GO(2, 1, 6)       \
+  else if ((N) <= 48) GO(3, 1, 5)       \
+  else if ((N) <= 64) GO(4, 1, 5)       \
+  else if ((N) <= 96) GO(6, 2, 5)       \
+  else if ((N) <= 128) GO(8, 2, 5)      \
+  else if ((N) <= 192) GO(12, 2, 4)     \
+  else GO(16, 2, 3)
+
+int feature_tile(int N) { return N <= 64 ? 64 : 128; }
 
 }  // namespace
 
-extern "C" hipError_t ks_skinny_gemm(void* out, void* workspace,
-                                     const void* x, const void* w, int M,
-                                     int K, int N, long x_row_stride,
-                                     hipStream_t stream) {
-  if (M % 64 != 0 || K % BK != 0 || N > 256) return hipErrorInvalidValue;
-  const int feat_wgs = M / 64;
-  // fill the chip (G11): aim for >= 768 workgroups via K-splits
-  int nsplit = 1;
-  while (feat_wgs * nsplit < 768 && nsplit < 8 && (K / (nsplit * 2)) >= BK)
-    nsplit *= 2;
-  if (nsplit > 1 && workspace == nullptr) return hipErrorInvalidValue;
-  int k_per_split = ((K / nsplit + BK - 1) / BK) * BK;
-  const int NT = (N + 15) / 16;
-  short* ws = (short*)workspace;
-  const short* xs = (const short*)x;
-  const short* wp = (const short*)w;
-#define CASE(nt)                                                            \
-  launch_nt<nt>((short*)out, ws, xs, wp, M, K, N, x_row_stride, nsplit,     \
-                k_per_split, stream)
-  switch (NT) {
-    case 1: CASE(1); break;
-    case 2: CASE(2); break;
-    case 3: CASE(3); break;
-    case 4: CASE(4); break;
-    case 5: CASE(5); break;
-    case 6: CASE(6); break;
-    case 7: CASE(8); break;
-    case 8: CASE(8); break;
-    default:
-      if (NT <= 12) CASE(12);
-      else CASE(16);
-      break;
+// K splits for [N][K] x [M][K]: until every slot for a block is taken, with
+// four steps per split at least
+extern "C" int ks_skinny_splits(int M, int K, int N, int glu) {
+  const int bm = feature_tile(N);
+  const long tiles = glu ? (M + bm / 2 - 1) / (bm / 2) : (M + bm - 1) / bm;
+  if (glu) return 1;
+  const long want = N <= 64 ? 512 : 256;
+  long s = want / (tiles > 0 ? tiles : 1);
+  const long most = K / BK / 4;
+  if (s > most) s = most;
+  if (s > 16) s = 16;
+  return s < 1 ? 1 : (int)s;
+}
+
+extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
+                                     const void* w, int M, int K, int N, long xs,
+                                     int splits, int glu, hipStream_t stream) {
+  if (N < 1 || N > 256 || M < 1 || M % 4 != 0 || K < BK || K % BK != 0 || splits < 1 ||
+      splits > K / BK || (splits > 1 && (!partial || glu)) || xs % 8 != 0 ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
+    return hipErrorInvalidValue;
+  const GemmArgs p{splits > 1 ? partial : out, (const short*)x, (const short*)w, M,
+                   K, N, xs};
+  const int bm = feature_tile(N) / (glu ? 2 : 1);
+  const dim3 grid((M + bm - 1) / bm, splits);
+#define GO(nt, f, s)                                                           \
+  {                                                                            \
+    if (glu)                                                                   \
+      hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, GLU>), grid, dim3(256), \
+                         0, stream, p);                                        \
+    else if (splits > 1)                                                       \
+      hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, PARTIAL>), grid,        \
+                         dim3(256), 0, stream, p);                             \
+    else                                                                       \
+      hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, BF16_OUT>), grid,       \
+                         dim3(256), 0, stream, p);                             \
   }
-#undef CASE
+  FOR_TILE(N, GO)
+#undef GO
   HIP_CHECK_KERNEL();
-  if (nsplit > 1) {
+  if (splits > 1) {
     const long nm = (long)N * M;
-    hipLaunchKernelGGL(reduce_ws_kernel, dim3(2048), dim3(256), 0, stream,
-                       (short*)out, ws, nm, nsplit);
+    hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)((nm / 4 + 255) / 256)),
+                       dim3(256), 0, stream, (short*)out, (const float*)partial, nm,
+                       splits);
     HIP_CHECK_KERNEL();
   }
   return hipSuccess;

@@ -259,7 +259,10 @@ class MergedColumnParallelLinear(nn.Module):
             else None
         )
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, activate: bool = False) -> torch.Tensor:
+        """[gate | up], or with ``activate`` silu(gate) * up."""
+        if activate:
+            return ops.linear_silu_and_mul(x, self.weight, self.bias)
         return ops.linear(x, self.weight, self.bias)
 
     def load_shards(self, gate_weight: torch.Tensor, up_weight: torch.Tensor):

@@ -678,6 +678,80 @@ class TestSkinnyGemm:
         torch.testing.assert_close(out.float(), ref, atol=0.05, rtol=0.05)
 
 
+class TestSkinnyGemmEdges:
+    """Edges of the token and feature tiles, of the K steps and their splits,
+    against fp64. Bound: an fp32 sum of K products is off by K 2^-24 of the
+    products' magnitudes at most, then one rounding to bf16 (2^-8 covers it
+    and silu's few ulp)."""
+
+    @pytest.mark.parametrize("N", [1, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 128,
+                                   129, 192, 193, 256])
+    @pytest.mark.parametrize("K,M", [(64, 36), (320, 132), (1088, 4096 + 68)])
+    @pytest.mark.parametrize("glu", [False, True])
+    def test_against_fp64(self, dev, N, K, M, glu):
+        import kserve_amd_C
+
+        torch.manual_seed(N + K)
+        x = torch.randn(N, K + 8, device=dev, dtype=torch.bfloat16)[:, :K]
+        w = torch.randn((2 if glu else 1) * M, K, device=dev).mul_(K ** -0.5)
+        w = w.to(torch.bfloat16)
+        out = torch.full((N, M), float("nan"), device=dev, dtype=torch.bfloat16)
+        (kserve_amd_C.skinny_glu if glu else kserve_amd_C.skinny_gemm)(out, x, w)
+        ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        off = mag * (K * 2.0 ** -24)
+        if glu:
+            g, u = ref[:, :M], ref[:, M:]
+            og, ou = off[:, :M], off[:, M:]
+            sg = torch.nn.functional.silu(g)
+            ref, off = sg * u, 1.1 * og * (u.abs() + ou) + sg.abs() * ou
+        assert ((out.double() - ref).abs() <= off + ref.abs() * 2.0 ** -8).all()
+
+    def test_dispatch_takes_every_form(self, dev):
+        from kserve_amd import ops
+
+        F = torch.nn.functional
+        torch.manual_seed(0)
+        w = torch.randn(4608 * 2, 256, device=dev, dtype=torch.bfloat16) / 16
+        wide = torch.randn(70, 520, device=dev, dtype=torch.bfloat16)
+        forms = [
+            (wide[:5, :256], w), (wide[:5, 1:257], w),        # rows, shifted rows
+            (wide[:5, 8:264], w), (wide[:48, :512:2], w),     # strided columns
+            (wide[:1, :256].expand(9, 256), w),               # one row repeated
+            (wide[:7, :256].t().contiguous().t(), w),         # column-major
+            (wide[:40, :248], w[:, :248]),                    # K not of 64
+            (wide[:3, :256], w[1:4609]), (wide[:3, :256], w[:4610]),
+            (wide[:6, :256].reshape(3, 2, 256), w),
+            (wide[0, :256], w), (wide[:0, :256], w),          # a vector, no rows
+            (wide[:5, :256].float(), w.float()),
+        ]
+        for x, m in forms:
+            for got, want in ((ops.linear(x, m), F.linear(x, m)),
+                              (ops.linear(x, m, m[:, 0]), F.linear(x, m, m[:, 0]))):
+                assert got.shape == want.shape and got.dtype == want.dtype
+                torch.testing.assert_close(got, want, rtol=2.0 ** -7, atol=1e-2)
+        x = wide[:5, :256].clone().requires_grad_()
+        ops.linear(x, w).float().sum().backward()             # autograd stays
+        assert x.grad is not None and x.grad.abs().sum() > 0
+        rows = torch.func.vmap(lambda r: ops.linear(r[None], w)[0])(wide[:5, :256])
+        torch.testing.assert_close(rows, F.linear(wide[:5, :256], w), rtol=2.0 ** -7, atol=1e-2)
+        _, t = torch.func.jvp(lambda v: ops.linear(v, w), (wide[:5, :256],), (wide[5:10, :256],))
+        torch.testing.assert_close(t, F.linear(wide[5:10, :256], w), rtol=2.0 ** -7, atol=1e-2)
+        with pytest.raises(RuntimeError):
+            ops.linear(wide[:5, :512], w)
+
+    @pytest.mark.parametrize("N", [3, 64, 100])
+    def test_glu_route(self, dev, N):
+        from kserve_amd import ops
+
+        torch.manual_seed(N)
+        x = torch.randn(N, 128, device=dev, dtype=torch.bfloat16)
+        w = torch.randn(2 * 12288, 128, device=dev, dtype=torch.bfloat16) / 11
+        want = ops.silu_and_mul(torch.nn.functional.linear(x, w))
+        got = ops.linear_silu_and_mul(x, w)
+        # the unfused form rounds gate and up to bf16 first
+        torch.testing.assert_close(got, want, rtol=2.0 ** -6, atol=2e-2)
+
+
 class TestGemm8Experimental:
     """8-phase MFMA GEMM (experimental; not in the serving path).
     GPU-validated across the full SW x SCHED matrix — runs by
