@@ -87,21 +87,24 @@ class LlamaAttention(nn.Module):
         cos_sin_cache: torch.Tensor,
         kv_cache: Tuple[torch.Tensor, torch.Tensor],
         meta: AttentionMetadata,
-    ) -> torch.Tensor:
+        add_norm=None,  # see RowParallelLinear.forward
+    ):
         T = hidden.shape[0]
-        q, k, v = self.qkv_proj(hidden)
-        if meta.lora is not None:
+        k_cache, v_cache = kv_cache
+        rotate = (positions, cos_sin_cache, k_cache, v_cache, meta.slot_mapping)
+        # q, k, v: strided views into the fused qkv output; kernels take row
+        # strides
+        if meta.lora is None:
+            q, k, v = self.qkv_proj(hidden, rotate)
+        else:
+            q, k, v = self.qkv_proj(hidden)
             meta.lora.apply(self.layer_idx, "q_proj", hidden, q)
             meta.lora.apply(self.layer_idx, "k_proj", hidden, k)
             meta.lora.apply(self.layer_idx, "v_proj", hidden, v)
-        # strided views into the fused qkv output; kernels take row strides
-        q = q.view(T, self.num_heads_local, self.head_dim)
-        k = k.view(T, self.num_kv_heads_local, self.head_dim)
-        v = v.view(T, self.num_kv_heads_local, self.head_dim)
-        q, k = ops.rotary_embedding(positions, q, k, cos_sin_cache)
-        k_cache, v_cache = kv_cache
-        if k_cache.numel() > 0:
-            ops.reshape_and_cache(k, v, k_cache, v_cache, meta.slot_mapping)
+            q = q.view(T, self.num_heads_local, self.head_dim)
+            k = k.view(T, self.num_kv_heads_local, self.head_dim)
+            v = v.view(T, self.num_kv_heads_local, self.head_dim)
+            q, k = ops.rope_and_cache(positions, q, k, v, *rotate[1:])
         if meta.is_prefill:
             if meta.context_lens is not None:
                 # chunked prefill: attend to the whole paged context (past
@@ -127,7 +130,7 @@ class LlamaAttention(nn.Module):
             if meta.lora is not None
             else None
         )
-        return self.o_proj(o_in, o_delta)
+        return self.o_proj(o_in, o_delta, add_norm)
 
 
 class LlamaMLP(nn.Module):
@@ -144,7 +147,7 @@ class LlamaMLP(nn.Module):
             config.intermediate_size, config.hidden_size, bias=False, dtype=dtype
         )
 
-    def forward(self, x: torch.Tensor, meta=None) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, meta=None, add_norm=None):
         lora = meta.lora if meta is not None else None
         if lora is None:
             act = self.gate_up_proj(x, activate=True)
@@ -159,7 +162,7 @@ class LlamaMLP(nn.Module):
             if lora is not None
             else None
         )
-        return self.down_proj(act, d_delta)
+        return self.down_proj(act, d_delta, add_norm)
 
 
 class MixtralMoE(nn.Module):
@@ -331,20 +334,33 @@ class LlamaDecoderLayer(nn.Module):
         )
         self.eps = config.rms_norm_eps
 
-    def forward(self, hidden, residual, positions, cos_sin_cache, kv_cache, meta):
-        if residual is None:
+    def forward(
+        self, hidden, residual, positions, cos_sin_cache, kv_cache, meta,
+        normed: bool = False, next_norm=None,
+    ):
+        """``normed``: hidden is the input norm of the residual already.
+        ``next_norm`` (a norm's weight): the result is that norm of the new
+        residual in place of what is still to be added to it."""
+        if normed:
+            pass
+        elif residual is None:
             residual = hidden
             hidden = ops.rms_norm(hidden, self.input_layernorm, self.eps)
         else:
             hidden, residual = ops.fused_add_rms_norm(
                 hidden, residual, self.input_layernorm, self.eps
             )
-        hidden = self.self_attn(hidden, positions, cos_sin_cache, kv_cache, meta)
-        hidden, residual = ops.fused_add_rms_norm(
-            hidden, residual, self.post_attention_layernorm, self.eps
+        hidden, residual = self.self_attn(
+            hidden, positions, cos_sin_cache, kv_cache, meta,
+            add_norm=(residual, self.post_attention_layernorm, self.eps),
         )
-        hidden = self.mlp(hidden, meta)
-        return hidden, residual
+        if next_norm is None:
+            return self.mlp(hidden, meta), residual
+        if isinstance(self.mlp, LlamaMLP):
+            return self.mlp(hidden, meta, add_norm=(residual, next_norm, self.eps))
+        return ops.fused_add_rms_norm(
+            self.mlp(hidden, meta), residual, next_norm, self.eps
+        )
 
 
 class LlamaForCausalLM(nn.Module):
@@ -447,15 +463,20 @@ class LlamaForCausalLM(nn.Module):
             H = self.config.hidden_size
             hidden = comm.pp_recv((T, H), self.dtype, input_ids.device)
             residual = comm.pp_recv((T, H), self.dtype, input_ids.device)
+        # each layer leaves the norm that follows it; the last one of a stage
+        # leaves its sum to the next
+        norms = [layer.input_layernorm for layer in self.layers[1:]] + [self.norm]
         for i, layer in enumerate(self.layers):
             hidden, residual = layer(
-                hidden, residual, positions, self.cos_sin_cache, kv_caches[i], meta
+                hidden, residual, positions, self.cos_sin_cache, kv_caches[i], meta,
+                normed=i > 0, next_norm=norms[i],
             )
         if not self.is_last_stage:
             comm.pp_send(hidden)
             comm.pp_send(residual)
             return hidden
-        hidden, _ = ops.fused_add_rms_norm(hidden, residual, self.norm, self.eps)
+        if not len(self.layers):  # a last stage with no layers of its own
+            hidden, _ = ops.fused_add_rms_norm(hidden, residual, self.norm, self.eps)
         return hidden
 
     def compute_logits(self, hidden: torch.Tensor):

@@ -335,6 +335,125 @@ def linear_silu_and_mul(
     return silu_and_mul(linear(x, weight, bias))
 
 
+def linear_add_rms_norm(
+    x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor,
+    norm_weight: torch.Tensor, eps: float,
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """residual + x @ weight^T and its RMS norm: (norm, residual); the residual
+    in place on the GPU. Few rows: the norm's kernel adds the GEMM's splits."""
+    m = weight.shape[0]
+    if (
+        _skinny_operands(x, weight)
+        and _skinny_rows(x.shape[0], x.shape[1], m)
+        and m <= 16384
+        and residual.shape == (x.shape[0], m)
+        and norm_weight.shape == (m,)
+        and residual.dtype == norm_weight.dtype == torch.bfloat16
+        and residual.device == norm_weight.device == x.device
+        and residual.is_contiguous()
+        and norm_weight.is_contiguous()
+        and residual.data_ptr() % 16 == 0
+        and norm_weight.data_ptr() % 16 == 0
+    ):
+        out = torch.empty_like(residual)
+        _C.skinny_add_rms_norm(out, residual, x, weight, norm_weight, eps)
+        return out, residual
+    return fused_add_rms_norm(linear(x, weight), residual, norm_weight, eps)
+
+
+def _rope_cache_direct(positions, q, k, v, cos_sin, k_cache, v_cache, slots) -> bool:
+    """Forms that the one-pass kernel takes; the others go through
+    rotary_embedding and reshape_and_cache one after the other."""
+    D = q.shape[2]
+    return (
+        D % 16 == 0
+        and D <= 1024
+        and k.shape[0] == q.shape[0]
+        and k.shape == v.shape
+        and k.shape[2] == D
+        and positions.numel() == q.shape[0]
+        and positions.is_contiguous()
+        and cos_sin.is_contiguous()
+        and cos_sin.shape[-1] == D
+        and all(t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (q, k, v))
+        and cos_sin.data_ptr() % 16 == 0
+        and (
+            k_cache.numel() == 0
+            or (
+                k_cache.dim() == 4
+                and k_cache.shape == v_cache.shape
+                and k_cache.dtype == v_cache.dtype
+                and k_cache.shape[1] == k.shape[1]
+                and k_cache.shape[3] == D
+                and slots.is_contiguous()
+                and slots.numel() >= q.shape[0]
+                and k_cache.data_ptr() % 16 == 0
+                and v_cache.data_ptr() % 16 == 0
+            )
+        )
+    )
+
+
+def rope_and_cache(
+    positions: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
+    cos_sin_cache: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+    slot_mapping: torch.Tensor,
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """Rotates q and k (in place on the GPU) and scatters k and v into their
+    pages (an empty k_cache: no scatter); returns q and k."""
+    if q.is_cuda and _rope_cache_direct(
+        positions, q, k, v, cos_sin_cache, k_cache, v_cache, slot_mapping
+    ):
+        _native("rope_and_cache").rope_and_cache(
+            positions, q, k, v, cos_sin_cache, k_cache, v_cache,
+            slot_mapping if k_cache.numel() > 0 else k_cache,  # not read
+        )
+        return q, k
+    q, k = rotary_embedding(positions, q, k, cos_sin_cache)
+    if k_cache.numel() > 0:
+        reshape_and_cache(k, v, k_cache, v_cache, slot_mapping)
+    return q, k
+
+
+def linear_rope_and_cache(
+    x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
+    heads: int, kv_heads: int, positions: torch.Tensor,
+    cos_sin_cache: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+    slot_mapping: torch.Tensor,
+) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """q, k, v [T, heads, D] = x @ weight^T (+ bias) with ``rope_and_cache``
+    applied. Few rows: its kernel adds the GEMM's splits."""
+    T, D = x.shape[0], weight.shape[0] // (heads + 2 * kv_heads)
+
+    def parts(qkv):
+        q, k, v = qkv.split([heads * D, kv_heads * D, kv_heads * D], dim=-1)
+        return (
+            q.view(T, heads, D), k.view(T, kv_heads, D), v.view(T, kv_heads, D)
+        )
+
+    if (
+        bias is None
+        and _skinny_operands(x, weight)
+        and _skinny_rows(T, x.shape[1], weight.shape[0])
+    ):
+        q, k, v = parts(
+            torch.empty((T, weight.shape[0]), dtype=x.dtype, device=x.device)
+        )
+        if _rope_cache_direct(
+            positions, q, k, v, cos_sin_cache, k_cache, v_cache, slot_mapping
+        ):
+            _C.skinny_rope_cache(
+                q, k, v, x, weight, positions, cos_sin_cache, k_cache, v_cache,
+                slot_mapping if k_cache.numel() > 0 else k_cache,  # not read
+            )
+            return q, k, v
+    q, k, v = parts(linear(x, weight, bias))
+    q, k = rope_and_cache(
+        positions, q, k, v, cos_sin_cache, k_cache, v_cache, slot_mapping
+    )
+    return q, k, v
+
+
 def embed_layer_norm(
     word, pos_table, type_table, ids, cu_seqlens, types, weight, bias, eps: float
 ):

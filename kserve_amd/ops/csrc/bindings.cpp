@@ -43,6 +43,11 @@ hipError_t ks_fused_add_layer_norm(void*, const void*, const void*,
                                    hipStream_t);
 hipError_t ks_gelu(void*, const void*, long, hipStream_t);
 hipError_t ks_mfma_probe(void*, const void*, const void*, hipStream_t);
+hipError_t ks_rope_cache(void*, void*, void*, const void*, int, const void*,
+                         const void*, void*, void*, const void*, int, int, int,
+                         int, int, int, long, long, long, hipStream_t);
+hipError_t ks_add_splits_rms_norm(void*, void*, const void*, const void*, float,
+                                  int, int, int, hipStream_t);
 int ks_skinny_splits(int, int, int, int);
 hipError_t ks_skinny_gemm(void*, void*, const void*, const void*, int, int,
                           int, long, int, int, hipStream_t);
@@ -312,29 +317,50 @@ void gelu(at::Tensor& out, at::Tensor& input) {
             "gelu");
 }
 
+struct SkinnyShape {
+  int M, K, N;
+  long stride;
+};
+
+static SkinnyShape skinny_shape(const at::Tensor& x, const at::Tensor& w, int halves) {
+  CHECK_BF16_CONTIG(w);
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && x.is_cuda() && x.dim() == 2 &&
+                  w.dim() == 2 && x.stride(1) == 1,
+              "x must be bf16 row-dense");
+  const long N = x.size(0), K = x.size(1), M = w.size(0) / halves;
+  TORCH_CHECK(w.size(1) == K && w.size(0) == M * halves, "shape mismatch");
+  TORCH_CHECK(x.device() == w.device(), "operands on different devices");
+  TORCH_CHECK(N >= 1 && N <= 256 && M < (1L << 30) && K < (1L << 30),
+              "size out of range");
+  return {(int)M, (int)K, (int)N, (long)x.stride(0)};
+}
+
+// fp32 sums of the K splits of x @ w^T, [splits][N][M]
+static at::Tensor skinny_sums(const at::Tensor& x, const at::Tensor& w) {
+  const SkinnyShape z = skinny_shape(x, w, 1);
+  const int splits = ks_skinny_splits(z.M, z.K, z.N, 0);
+  at::Tensor part = at::empty({splits, z.N, z.M}, x.options().dtype(at::kFloat));
+  check_hip(ks_skinny_gemm(nullptr, part.data_ptr(), x.data_ptr(), w.data_ptr(), z.M,
+                           z.K, z.N, z.stride, splits, 0, current_stream()),
+            "skinny_gemm");
+  return part;
+}
+
 static void skinny_product(at::Tensor& out, at::Tensor& x, at::Tensor& w,
                            bool glu) {
   CHECK_BF16_CONTIG(out);
-  CHECK_BF16_CONTIG(w);
-  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && x.is_cuda() && x.dim() == 2 &&
-                  w.dim() == 2 && out.dim() == 2 && x.stride(1) == 1,
-              "x must be bf16 row-dense");
-  const long N = x.size(0), K = x.size(1), M = w.size(0) / (glu ? 2 : 1);
-  TORCH_CHECK(w.size(1) == K && w.size(0) == M * (glu ? 2 : 1) &&
-                  out.size(0) == N && out.size(1) == M,
-              "shape mismatch");
-  TORCH_CHECK(x.device() == w.device() && x.device() == out.device(),
-              "operands on different devices");
-  TORCH_CHECK(N >= 1 && N <= 256 && M < (1L << 30) && K < (1L << 30),
-              "size out of range");
+  const SkinnyShape z = skinny_shape(x, w, glu ? 2 : 1);
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == z.N && out.size(1) == z.M &&
+                  out.device() == x.device(),
+              "output shape mismatch");
   const c10::DeviceGuard guard(x.device());
-  const int splits = ks_skinny_splits(M, K, N, glu);
+  const int splits = ks_skinny_splits(z.M, z.K, z.N, glu);
   at::Tensor part;  // fp32 sums of the K splits
   if (splits > 1)
-    part = at::empty({splits * N * M}, x.options().dtype(at::kFloat));
+    part = at::empty({(long)splits * z.N * z.M}, x.options().dtype(at::kFloat));
   check_hip(ks_skinny_gemm(out.data_ptr(), splits > 1 ? part.data_ptr() : nullptr,
-                           x.data_ptr(), w.data_ptr(), (int)M, (int)K, (int)N,
-                           (long)x.stride(0), splits, glu, current_stream()),
+                           x.data_ptr(), w.data_ptr(), z.M, z.K, z.N, z.stride,
+                           splits, glu, current_stream()),
             "skinny_gemm");
 }
 
@@ -346,6 +372,91 @@ void skinny_gemm(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
 void skinny_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
   // out [N, M] = silu(x @ w[:M]^T) * (x @ w[M:]^T), bf16, N <= 256
   skinny_product(out, x, w, true);
+}
+
+void skinny_add_rms_norm(at::Tensor& out, at::Tensor& residual, at::Tensor& x,
+                         at::Tensor& w, at::Tensor& norm_weight, double eps) {
+  // residual += x @ w^T; out = RMS norm of residual
+  CHECK_BF16_CONTIG(out);
+  CHECK_BF16_CONTIG(residual);
+  CHECK_BF16_CONTIG(norm_weight);
+  const long N = x.size(0), M = w.size(0);
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == N && out.size(1) == M &&
+                  residual.sizes() == out.sizes() && norm_weight.numel() == M,
+              "shape mismatch");
+  TORCH_CHECK(x.device() == out.device() && x.device() == residual.device() &&
+                  x.device() == norm_weight.device(),
+              "operands on different devices");
+  const c10::DeviceGuard guard(x.device());
+  const at::Tensor part = skinny_sums(x, w);
+  check_hip(ks_add_splits_rms_norm(out.data_ptr(), residual.data_ptr(),
+                                   part.data_ptr(), norm_weight.data_ptr(),
+                                   (float)eps, (int)N, (int)M, (int)part.size(0),
+                                   current_stream()),
+            "skinny_add_rms_norm");
+}
+
+// rotation and scatter, in place or (part) out of the sums of a projection
+static void rope_cache_run(at::Tensor& q, at::Tensor& k, at::Tensor& v,
+                           const at::Tensor* part, at::Tensor& positions,
+                           at::Tensor& cos_sin, at::Tensor& k_cache,
+                           at::Tensor& v_cache, at::Tensor& slot_mapping) {
+  CHECK_BF16_ROWS(q);
+  CHECK_BF16_ROWS(k);
+  CHECK_BF16_ROWS(v);
+  TORCH_CHECK(positions.scalar_type() == at::kLong, "positions must be int64");
+  TORCH_CHECK(cos_sin.scalar_type() == at::kFloat && cos_sin.is_contiguous(),
+              "cos_sin_cache must be fp32");
+  const int T = q.size(0), Hq = q.size(1), Hk = k.size(1), D = q.size(2);
+  TORCH_CHECK(k.size(0) == T && v.sizes() == k.sizes() && k.size(2) == D &&
+                  positions.numel() == T && positions.is_contiguous() &&
+                  cos_sin.size(-1) == D,
+              "rope_and_cache: shape mismatch");
+  const bool cached = k_cache.numel() > 0;
+  bool fp8 = false;
+  int block = 1;
+  if (cached) {
+    CHECK_KV_CACHE(k_cache);
+    CHECK_KV_CACHE(v_cache);
+    TORCH_CHECK(slot_mapping.scalar_type() == at::kInt && slot_mapping.is_contiguous() &&
+                    slot_mapping.numel() >= T,
+                "slot_mapping int32");
+    TORCH_CHECK(k_cache.dim() == 4 && k_cache.size(1) == Hk && k_cache.size(3) == D &&
+                    v_cache.sizes() == k_cache.sizes() &&
+                    v_cache.scalar_type() == k_cache.scalar_type(),
+                "rope_and_cache: page shape mismatch");
+    fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn;
+    block = k_cache.size(2);
+  }
+  check_hip(ks_rope_cache(q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                          part ? part->data_ptr() : nullptr,
+                          part ? (int)part->size(0) : 0, positions.data_ptr(),
+                          cos_sin.data_ptr(), cached ? k_cache.data_ptr() : nullptr,
+                          cached ? v_cache.data_ptr() : nullptr,
+                          cached ? slot_mapping.data_ptr() : nullptr, T, Hq, Hk, D,
+                          block, fp8, (long)q.stride(0), (long)k.stride(0),
+                          (long)v.stride(0), current_stream()),
+            "rope_and_cache");
+}
+
+void rope_and_cache(at::Tensor& positions, at::Tensor& q, at::Tensor& k,
+                    at::Tensor& v, at::Tensor& cos_sin, at::Tensor& k_cache,
+                    at::Tensor& v_cache, at::Tensor& slot_mapping) {
+  rope_cache_run(q, k, v, nullptr, positions, cos_sin, k_cache, v_cache,
+                 slot_mapping);
+}
+
+void skinny_rope_cache(at::Tensor& q, at::Tensor& k, at::Tensor& v, at::Tensor& x,
+                       at::Tensor& w, at::Tensor& positions, at::Tensor& cos_sin,
+                       at::Tensor& k_cache, at::Tensor& v_cache,
+                       at::Tensor& slot_mapping) {
+  // q, k and v (written whole) are the parts of x @ w^T, rotated
+  TORCH_CHECK(x.size(0) == q.size(0) &&
+                  w.size(0) == (q.size(1) + k.size(1) + v.size(1)) * q.size(2),
+              "shape mismatch");
+  const at::Tensor part = skinny_sums(x, w);
+  rope_cache_run(q, k, v, &part, positions, cos_sin, k_cache, v_cache,
+                 slot_mapping);
 }
 
 void gemm8(at::Tensor& d, at::Tensor& a, at::Tensor& w, int64_t swizzle) {
@@ -394,6 +505,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gelu", &gelu, "erf GELU");
   def_sampling(m);
   m.def("skinny_gemm", &skinny_gemm, "decode GEMM (N<=256, MFMA streaming)");
+  m.def("skinny_add_rms_norm", &skinny_add_rms_norm,
+        "few-row GEMM into a residual and its RMS norm");
+  m.def("rope_and_cache", &rope_and_cache,
+        "rotary embedding and K/V scatter in one pass");
+  m.def("skinny_rope_cache", &skinny_rope_cache,
+        "few-row qkv GEMM, rotary embedding and K/V scatter");
   m.def("skinny_glu", &skinny_glu, "gate|up GEMM (N<=256) with silu(gate) * up");
   m.def("gemm8", &gemm8,
         "EXPERIMENTAL 8-phase 256x256 MFMA GEMM");

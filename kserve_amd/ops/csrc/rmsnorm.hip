@@ -78,9 +78,85 @@ __global__ void rms_norm_kernel(
   }
 }
 
+// residual += sum of the K splits of a projection (fp32, in order), and the
+// row's norm, for few rows: a block per row with the row in registers, so the
+// splits are read once and the launch that added them is gone. Launch-bound:
+// 4.6 us where the two kernels took 4.7 + 4.7 (1 to 77 rows of 4096, 8 splits).
+template <int V>
+__global__ __launch_bounds__(1024) void add_splits_rms_norm_kernel(
+    short* __restrict__ out, short* __restrict__ residual,
+    const float* __restrict__ part, const short* __restrict__ weight,
+    const float eps, const int rows, const int hidden, const int splits) {
+  __shared__ float s_part[16];
+  const long row = blockIdx.x, nm = (long)rows * hidden;
+  const int step = blockDim.x * 4, at = threadIdx.x * 4;
+  float4_t a[V];
+  float ssq = 0.f;
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const int i = at + v * step;
+    a[v] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (i >= hidden) continue;
+    const float* src = part + row * hidden + i;
+    const short4_t r = *reinterpret_cast<const short4_t*>(residual + row * hidden + i);
+#pragma unroll 8
+    for (int s = 0; s < splits; ++s)
+      a[v] += *reinterpret_cast<const float4_t*>(src + s * nm);
+    short4_t o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      a[v][j] += bf16_bits_to_float(r[j]);
+      o[j] = float_to_bf16_bits(a[v][j]);
+      ssq += a[v][j] * a[v][j];
+    }
+    *reinterpret_cast<short4_t*>(residual + row * hidden + i) = o;
+  }
+  ssq = wave_reduce_sum(ssq);
+  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = ssq;
+  __syncthreads();
+  float total = 0.f;
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) total += s_part[w];
+  const float scale = rsqrtf(total / hidden + eps);
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const int i = at + v * step;
+    if (i >= hidden) continue;
+    const short4_t w = *reinterpret_cast<const short4_t*>(weight + i);
+    short4_t o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      o[j] = float_to_bf16_bits(a[v][j] * scale * bf16_bits_to_float(w[j]));
+    *reinterpret_cast<short4_t*>(out + row * hidden + i) = o;
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+// residual <- residual + sum of splits, out <- its RMS norm
+hipError_t ks_add_splits_rms_norm(void* out, void* residual, const void* part,
+                                  const void* weight, float eps, int rows,
+                                  int hidden, int splits, hipStream_t stream) {
+  if (rows < 1 || hidden < 4 || hidden % 4 != 0 || hidden > 16384 || splits < 1 ||
+      (((uintptr_t)out | (uintptr_t)residual | (uintptr_t)weight) & 7) != 0 ||
+      ((uintptr_t)part & 15) != 0)
+    return hipErrorInvalidValue;
+  const int vecs = hidden / 4;
+  const int threads = vecs >= 1024 ? 1024 : (vecs + 63) / 64 * 64;
+  const int v = (vecs + threads - 1) / threads;
+#define GO(V)                                                                   \
+  hipLaunchKernelGGL((add_splits_rms_norm_kernel<V>), dim3(rows), dim3(threads), \
+                     0, stream, (short*)out, (short*)residual,                  \
+                     (const float*)part, (const short*)weight, eps, rows,       \
+                     hidden, splits)
+  if (v == 1) GO(1);
+  else if (v == 2) GO(2);
+  else GO(4);
+#undef GO
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
+}
 
 hipError_t ks_rms_norm(void* out, const void* input, const void* weight,
                        float eps, int rows, int hidden, hipStream_t stream) {

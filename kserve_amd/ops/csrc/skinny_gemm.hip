@@ -236,14 +236,16 @@ extern "C" int ks_skinny_splits(int M, int K, int N, int glu) {
   return s < 1 ? 1 : (int)s;
 }
 
+// `out` null: the sums of the splits stay in `partial` for the caller's kernel.
 extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
                                      const void* w, int M, int K, int N, long xs,
                                      int splits, int glu, hipStream_t stream) {
   if (N < 1 || N > 256 || M < 1 || M % 4 != 0 || K < BK || K % BK != 0 || splits < 1 ||
-      splits > K / BK || (splits > 1 && (!partial || glu)) || xs % 8 != 0 ||
-      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
+      splits > K / BK || ((splits > 1 || !out) && (!partial || glu)) || xs % 8 != 0 ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)partial) & 15) != 0)
     return hipErrorInvalidValue;
-  const GemmArgs p{splits > 1 ? partial : out, (const short*)x, (const short*)w, M,
+  const bool sums = splits > 1 || !out;
+  const GemmArgs p{sums ? partial : out, (const short*)x, (const short*)w, M,
                    K, N, xs};
   const int bm = feature_tile(N) / (glu ? 2 : 1);
   const dim3 grid((M + bm - 1) / bm, splits);
@@ -252,7 +254,7 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
     if (glu)                                                                   \
       hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, GLU>), grid, dim3(256), \
                          0, stream, p);                                        \
-    else if (splits > 1)                                                       \
+    else if (sums)                                                             \
       hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, PARTIAL>), grid,        \
                          dim3(256), 0, stream, p);                             \
     else                                                                       \
@@ -262,7 +264,7 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
   FOR_TILE(N, GO)
 #undef GO
   HIP_CHECK_KERNEL();
-  if (splits > 1) {
+  if (sums && out) {
     const long nm = (long)N * M;
     hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)((nm / 4 + 255) / 256)),
                        dim3(256), 0, stream, (short*)out, (const float*)partial, nm,

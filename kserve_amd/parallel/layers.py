@@ -108,7 +108,15 @@ class QKVParallelLinear(nn.Module):
             else None
         )
 
-    def forward(self, x: torch.Tensor):
+    def forward(self, x: torch.Tensor, rotate=None):
+        """q, k, v as [T, heads * D]; with ``rotate`` (positions, cos_sin_cache,
+        k_cache, v_cache, slot_mapping) rotated, written to their pages and
+        shaped [T, heads, D]."""
+        if rotate is not None:
+            return ops.linear_rope_and_cache(
+                x, self.weight, self.bias, self.heads_local, self.kv_heads_local,
+                *rotate,
+            )
         qkv = ops.linear(x, self.weight, self.bias)
         return qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
 
@@ -183,7 +191,19 @@ class RowParallelLinear(nn.Module):
         self.overlap_chunks = max(1, overlap_chunks)
 
     def forward(
-        self, x: torch.Tensor, delta: Optional[torch.Tensor] = None
+        self, x: torch.Tensor, delta: Optional[torch.Tensor] = None, add_norm=None
+    ):
+        """x @ weight^T (+ delta) summed over the ranks. With ``add_norm``
+        (residual, norm weight, eps): the RMS norm of that plus the residual,
+        and the new residual."""
+        if add_norm is not None:
+            if self.tp_size == 1 and delta is None and self.bias is None:
+                return ops.linear_add_rms_norm(x, self.weight, *add_norm)
+            return ops.fused_add_rms_norm(self._product(x, delta), *add_norm)
+        return self._product(x, delta)
+
+    def _product(
+        self, x: torch.Tensor, delta: Optional[torch.Tensor]
     ) -> torch.Tensor:
         use_overlap = (
             self.reduce_output

@@ -752,6 +752,117 @@ class TestSkinnyGemmEdges:
         torch.testing.assert_close(got, want, rtol=2.0 ** -6, atol=2e-2)
 
 
+class TestFusedProjections:
+    """The kernels that take a few-row GEMM's K splits, and the one-pass
+    rotation and scatter, against fp64 and against the separate ops."""
+
+    @staticmethod
+    def _pages(dev, T, Hk, D, fp8, block=16):
+        dt = torch.float8_e4m3fn if fp8 else torch.bfloat16
+        k = torch.zeros(T // block + 3, Hk, block, D, device=dev, dtype=torch.bfloat16).to(dt)
+        slots = torch.randperm((T // block + 3) * block, device=dev)[:T].to(torch.int32)
+        if T > 2:
+            slots[1] = -1  # a padded row
+        return k, k.clone(), slots
+
+    @pytest.mark.parametrize("T", [1, 3, 4, 17, 200, 5000])
+    @pytest.mark.parametrize("Hq,Hk,D", [(32, 8, 128), (3, 1, 64), (5, 5, 80), (2, 1, 256), (9, 3, 16)])
+    @pytest.mark.parametrize("fp8", [False, True])
+    def test_rope_and_cache(self, dev, T, Hq, Hk, D, fp8):
+        from kserve_amd import ops
+
+        torch.manual_seed(T + D)
+        qkv = torch.randn(T, (Hq + 2 * Hk) * D + 8, device=dev, dtype=torch.bfloat16)
+        def parts(t):
+            q, k, v = t[:, : (Hq + 2 * Hk) * D].split([Hq * D, Hk * D, Hk * D], -1)
+            return q.view(T, Hq, D), k.view(T, Hk, D), v.view(T, Hk, D)
+        pos = torch.randint(0, 512, (T,), device=dev)
+        ang = torch.rand(512, D // 2, device=dev) * 6.3
+        cs = torch.cat([ang.cos(), ang.sin()], -1).contiguous()
+        a, b = qkv.clone(), qkv.clone()
+        kc, vc, slots = self._pages(dev, T, Hk, D, fp8)
+        kc2, vc2 = kc.clone(), vc.clone()
+        q, k, v = parts(a)
+        ops.rope_and_cache(pos, q, k, v, cs, kc, vc, slots)
+        q2, k2, v2 = parts(b)
+        ops.rotary_embedding(pos, q2, k2, cs)
+        # one rounding of the same fp32 expression, its products fused or not
+        c, s = cs[pos].double().chunk(2, -1)
+        for got, src in ((q, parts(qkv)[0]), (k, parts(qkv)[1])):
+            x1, x2 = src.double().chunk(2, -1)
+            c_, s_ = c[:, None], s[:, None]
+            want = torch.cat([x1 * c_ - x2 * s_, x2 * c_ + x1 * s_], -1)
+            mag = torch.cat([(x1 * c_).abs() + (x2 * s_).abs(), (x2 * c_).abs() + (x1 * s_).abs()], -1)
+            assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + mag * 2.0 ** -22).all()
+        assert torch.equal(v, v2) and torch.equal(a[:, -8:], qkv[:, -8:])
+        ops.reshape_and_cache(k, v, kc2, vc2, slots)
+        assert torch.equal(kc.view(torch.uint8), kc2.view(torch.uint8))
+        assert torch.equal(vc.view(torch.uint8), vc2.view(torch.uint8))
+        # without pages, and the forms that go through the separate ops
+        a2 = qkv.clone()
+        e = torch.empty(0, device=dev, dtype=torch.bfloat16)
+        q3, k3, _ = parts(a2)
+        ops.rope_and_cache(pos, q3, k3, parts(a2)[2], cs, e, e, None)
+        assert torch.equal(a2, a)
+
+    @pytest.mark.parametrize("T", [1, 5, 48, 65, 100, 192])
+    @pytest.mark.parametrize("Hq,Hk,D,K", [(32, 8, 128, 4096), (30, 5, 80, 1024), (14, 2, 64, 1280)])
+    def test_linear_rope_and_cache(self, dev, T, Hq, Hk, D, K):
+        from kserve_amd import ops
+
+        torch.manual_seed(T)
+        M = (Hq + 2 * Hk) * D
+        x = torch.randn(T, K, device=dev, dtype=torch.bfloat16)
+        w = (torch.randn(M, K, device=dev) * K ** -0.5).to(torch.bfloat16)
+        pos = torch.randint(0, 512, (T,), device=dev)
+        ang = torch.rand(512, D // 2, device=dev) * 6.3
+        cs = torch.cat([ang.cos(), ang.sin()], -1).contiguous()
+        kc, vc, slots = self._pages(dev, T, Hk, D, False)
+        kc2, vc2 = kc.clone(), vc.clone()
+        q, k, v = ops.linear_rope_and_cache(x, w, None, Hq, Hk, pos, cs, kc, vc, slots)
+        full = x.double() @ w.double().t()
+        off = (x.double().abs() @ w.double().abs().t()) * (K * 2.0 ** -24)
+        c, s = cs[pos].double().chunk(2, -1)
+        at = 0
+        for got, n, turn in ((q, Hq, True), (k, Hk, True), (v, Hk, False)):
+            y = full[:, at : at + n * D].view(T, n, D)
+            o = off[:, at : at + n * D].view(T, n, D)
+            at += n * D
+            if turn:
+                x1, x2 = y.chunk(2, -1)
+                e1, e2 = o.chunk(2, -1)
+                c_, s_ = c[:, None], s[:, None]
+                y = torch.cat([x1 * c_ - x2 * s_, x2 * c_ + x1 * s_], -1)
+                o = torch.cat([e1 + e2, e1 + e2], -1)
+            # a row may also come through bf16 before its rotation (2^-8 more)
+            assert ((got.double() - y).abs() <= o + 2.0 ** -8 * y.abs() + 2.0 ** -8 * full.abs().max()).all()
+        ops.reshape_and_cache(k, v, kc2, vc2, slots)
+        assert torch.equal(kc, kc2) and torch.equal(vc, vc2)
+
+    @pytest.mark.parametrize("N", [1, 7, 48, 100, 200])
+    @pytest.mark.parametrize("K,M", [(4096, 4096), (1024, 1284), (14336, 4100), (64, 16384)])
+    def test_linear_add_rms_norm(self, dev, N, K, M):
+        from kserve_amd import ops
+
+        torch.manual_seed(N + M)
+        x = torch.randn(N, K, device=dev, dtype=torch.bfloat16)
+        w = (torch.randn(M, K, device=dev) * K ** -0.5).to(torch.bfloat16)
+        r = torch.randn(N, M, device=dev, dtype=torch.bfloat16)
+        g = torch.rand(M, device=dev).to(torch.bfloat16)
+        if M % 8 and not ops._skinny_rows(N, K, M):
+            pytest.skip("the separate norm takes rows of eight")
+        y = x.double() @ w.double().t()
+        want = r.double() + y
+        out, res = ops.linear_add_rms_norm(x, w, r, g, 1e-5)
+        assert res is r
+        # the sum through bf16 on the general route, then one more rounding
+        off = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+        lim = off + 2.0 ** -8 * (want.abs() + y.abs())
+        assert ((res.double() - want).abs() <= lim).all()
+        norm = want * (want.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * g.double()
+        torch.testing.assert_close(out.double(), norm, rtol=2.0 ** -6, atol=2.0 ** -6)
+
+
 class TestGemm8Experimental:
     """8-phase MFMA GEMM (experimental; not in the serving path).
     GPU-validated across the full SW x SCHED matrix — runs by
