@@ -273,20 +273,20 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     """Whether the few-row kernel beats the library at [n, k] x [m, k]^T
     (MI355X, us, kernel / library, reduction of the K splits included).
 
-    Up to 48 rows it streams weights faster wherever there are enough of them
-    to outlast a launch: k 4096, m 32000 at 1 row 48 / 60, at 24 rows 50 / 60;
-    k 14336, m 4096 at 24 rows 27 / 32; but 512 x 512 4.6 / 4.2. Up to 64 rows
-    the widest ones are even (m 16384 38 / 35). Above, it gains where the
-    library does not split K over the chip: k 14336, m 4096 at 128 rows
-    36 / 76, k 4096, m 6144 22 / 26; and loses on small weights (2048 x 2048
-    15 / 11) and wide ones (m 16384 44 / 38). Past 192 rows the lighter of the
-    former turn (4096 x 4096 27 / 23 at 256 rows; m 6144 33 / 40)."""
-    weights = k * m
-    if m % 4 or weights < 1 << 20:
+    Up to 48 rows it streams weights faster (k 4096, m 32000 at 1 row 48 / 60,
+    at 24 rows 50 / 60; k 14336, m 4096 at 24 rows 27 / 32; level on small
+    ones, 512 x 512 4.6 / 4.2), up to 64 rows but for the widest (m 16384
+    38 / 35). So far a row's sums do not depend on the rows beside it, and
+    small weights stay here for that. Above, it gains where the library does
+    not split K over the chip: k 14336, m 4096 at 128 rows 36 / 76, k 4096,
+    m 6144 22 / 26; and loses on small weights (2048 x 2048 15 / 11) and wide
+    ones (m 16384 44 / 38). Past 192 rows the lighter of the former turn
+    (4096 x 4096 27 / 23 at 256 rows; m 6144 33 / 40)."""
+    if m % 4:
         return False
     if n <= 48 or (n <= 64 and m <= 8192):
         return True
-    return 4096 <= m <= 10240 and weights >= (16 if n <= 192 else 24) << 20
+    return 4096 <= m <= 10240 and k * m >= (16 if n <= 192 else 24) << 20
 
 
 def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
