@@ -35,6 +35,7 @@ MODULES = {
             "attention_decode.hip",
             "attention_prefill.hip",
             "sampling.hip",
+            "decode_step.hip",
             "skinny_gemm.hip",
             "gemm8.hip",
             "mfma_probe.hip",
@@ -53,6 +54,7 @@ MODULES = {
             "moe_route.hip",
             "activation.hip",
             "sampling.hip",
+            "decode_step.hip",
         ],
         "bindings": "bindings_seq.cpp",
         "fast_math": False,

@@ -14,6 +14,7 @@ from typing import Dict, List, Optional, Tuple
 
 import torch
 
+from kserve_amd import ops
 from kserve_amd.engine.block_manager import BlockManager
 from kserve_amd.engine.config import EngineConfig
 from kserve_amd.engine.request import Request
@@ -58,8 +59,9 @@ class ModelRunner:
         # the count on the host between windows)
         self._rng_step = 0
         # pinned staging + per-request numpy block-table cache
-        self._pin: Optional[Dict[str, torch.Tensor]] = None
+        self._pin: Optional[torch.Tensor] = None
         self._pin_np = None
+        self._pin_stride = 0
         # recorded after a step's async copies out of the pinned buffers; the
         # next fill waits on it, so a caller that never reads the step's
         # result back cannot overwrite inputs still in flight
@@ -362,28 +364,28 @@ class ModelRunner:
         return input_ids, pos, meta, sel
 
     def _ensure_decode_buffers(self, n: int, max_blocks: int):
-        """Pinned host staging buffers + numpy views (fast CPU fill, one
-        async H2D per tensor per step)."""
-        import numpy as np
-
-        need = self._pin is None or self._pin["input_ids"].shape[0] < n or self._pin[
-            "block_tables"
-        ].shape[1] < max_blocks
-        if need:
-            cap = max(n, self.config.scheduler.max_num_seqs)
-            mb = max(max_blocks, self.max_blocks_per_seq)
-            pin = self.is_cuda
-            self._pin = {
-                "input_ids": torch.empty(cap, dtype=torch.int64, pin_memory=pin),
-                "positions": torch.empty(cap, dtype=torch.int64, pin_memory=pin),
-                "slot_mapping": torch.empty(cap, dtype=torch.int32, pin_memory=pin),
-                "context_lens": torch.empty(cap, dtype=torch.int32, pin_memory=pin),
-                "state_slots": torch.zeros(cap, dtype=torch.int32, pin_memory=pin),
-                "block_tables": torch.zeros(
-                    (cap, mb), dtype=torch.int32, pin_memory=pin
-                ),
-            }
-            self._pin_np = {k: v.numpy() for k, v in self._pin.items()}
+        """Pinned staging rows for a decode batch (one async H2D per step) as
+        (pin, views): the rows' fields as numpy arrays, their page tables just
+        wide enough for this batch."""
+        rows = max(n, self.config.scheduler.max_num_seqs)
+        stride = ops.DECODE_ROW_HEAD + max_blocks + max_blocks % 2
+        if self._pin is None or self._pin.numel() < rows * stride:
+            widest = max(max_blocks, self.max_blocks_per_seq) + 1
+            self._pin = torch.zeros(
+                rows * (ops.DECODE_ROW_HEAD + widest), dtype=torch.int32,
+                pin_memory=self.is_cuda,
+            )
+        i32 = self._pin[: rows * stride].view(rows, stride).numpy()
+        i64 = i32.view("int64")
+        self._pin_np = {
+            "input_ids": i64[:, 0],
+            "positions": i64[:, 1],
+            "context_lens": i32[:, 4],
+            "state_slots": i32[:, 5],
+            "slot_mapping": i32[:, 6],
+            "block_tables": i32[:, ops.DECODE_ROW_HEAD :],
+        }
+        self._pin_stride = stride
         return self._pin, self._pin_np
 
     def _fill_pinned(self, batch: ScheduledBatch, block_manager: BlockManager):
@@ -408,11 +410,16 @@ class ModelRunner:
         ctx = pnp["context_lens"]
         btab = pnp["block_tables"]
         ss = pnp.get("state_slots")
+        btab[:n] = 0  # past a table's end: the scratch page
         for i, req in enumerate(batch.requests):
             pos = req.num_computed_tokens
             if ss is not None:
                 ss[i] = req.state_slot
-            ii[i] = req.all_token_ids[pos]
+            prompt = req.prompt_token_ids
+            ii[i] = (
+                prompt[pos] if pos < len(prompt)
+                else req.output_token_ids[pos - len(prompt)]
+            )
             pp[i] = pos
             t = tables[i]
             sm[i] = t[pos // bs] * bs + pos % bs
@@ -445,23 +452,33 @@ class ModelRunner:
         self, batch: ScheduledBatch, block_manager: BlockManager
     ):
         n, nb = self._fill_pinned(batch, block_manager)
-        pin = self._pin
         dev = self.device
+
+        def vector(dtype):
+            return torch.empty(n, dtype=dtype, device=dev)
+
+        input_ids, pos = vector(torch.int64), vector(torch.int64)
+        state_slots = vector(torch.int32)
         meta = AttentionMetadata(
             is_prefill=False,
-            slot_mapping=pin["slot_mapping"][:n].to(dev, non_blocking=True),
-            block_tables=pin["block_tables"][:n, :nb].to(dev, non_blocking=True)
-            .contiguous(),
-            context_lens=pin["context_lens"][:n].to(dev, non_blocking=True),
+            slot_mapping=vector(torch.int32),
+            block_tables=torch.empty((n, nb), dtype=torch.int32, device=dev),
+            context_lens=vector(torch.int32),
+        )
+        ops.unpack_decode_rows(
+            self._staged_rows(n), nb, input_ids, pos, meta.context_lens,
+            state_slots, meta.slot_mapping, meta.block_tables,
         )
         if self._layout is not None:
-            self._decode_layout_meta(
-                meta, n, pin["state_slots"][:n].to(dev, non_blocking=True)
-            )
-        input_ids = pin["input_ids"][:n].to(dev, non_blocking=True)
-        pos = pin["positions"][:n].to(dev, non_blocking=True)
-        self._mark_staging()
+            self._decode_layout_meta(meta, n, state_slots)
         return input_ids, pos, meta
+
+    def _staged_rows(self, rows: int) -> torch.Tensor:
+        """The first pinned rows on the device, in one copy."""
+        rows_pin = self._pin[: rows * self._pin_stride]
+        staged = rows_pin.to(self.device, non_blocking=True)
+        self._mark_staging()
+        return staged.view(rows, self._pin_stride)
 
     def _decode_layout_meta(self, meta, n: int, state_slots) -> None:
         """Decode is the flat-batch layout with one token per sequence."""
@@ -602,6 +619,7 @@ class ModelRunner:
             ),
             "context_lens": torch.ones(max_bs, dtype=torch.int32, device=dev),
             "state_slots": torch.zeros(max_bs, dtype=torch.int32, device=dev),
+            "slots": torch.zeros(max_bs, dtype=torch.int32, device=dev),
             # per-request sampling params (sampled-window variants)
             "temps": torch.ones(max_bs, dtype=torch.float32, device=dev),
             "top_p": torch.ones(max_bs, dtype=torch.float32, device=dev),
@@ -621,15 +639,11 @@ class ModelRunner:
             buf = self._graph_buffers
 
             def body(bs=bs, buf=buf):
-                # slot mapping derived IN-GRAPH from (block_tables, positions)
-                # so multi-step windows advance with zero host involvement
                 pos = buf["positions"][:bs]
                 bt = buf["block_tables"][:bs]
-                blk = torch.gather(bt, 1, (pos // bsz).unsqueeze(1)).squeeze(1)
-                slot = (blk * bsz + (pos % bsz).to(torch.int32)).to(torch.int32)
                 meta = AttentionMetadata(
                     is_prefill=False,
-                    slot_mapping=slot,
+                    slot_mapping=buf["slots"][:bs],
                     block_tables=bt,
                     context_lens=buf["context_lens"][:bs],
                 )
@@ -639,11 +653,14 @@ class ModelRunner:
                     buf["input_ids"][:bs], pos, self.kv_caches, meta
                 )
                 logits = self.model.compute_logits(hidden)
-                # greedy sample in-graph; feed back as the next step's input
+                # greedy sample in-graph; it, its position and its page slot
+                # are the next replay's input, so multi-step windows advance
+                # with zero host involvement
                 sampled = _ops.greedy_sample(logits)
-                buf["input_ids"][:bs].copy_(sampled)
-                buf["positions"][:bs].add_(1)
-                buf["context_lens"][:bs].add_(1)
+                _ops.advance_decode(
+                    sampled, buf["input_ids"], buf["positions"],
+                    buf["context_lens"], buf["slots"], bt, bsz,
+                )
                 return logits, sampled
 
             # warmup run (allocator state, rccl comms)
@@ -681,11 +698,9 @@ class ModelRunner:
         def body():
             pos = buf["positions"][:bs]
             bt = buf["block_tables"][:bs]
-            blk = torch.gather(bt, 1, (pos // bsz).unsqueeze(1)).squeeze(1)
-            slot = (blk * bsz + (pos % bsz).to(torch.int32)).to(torch.int32)
             meta = AttentionMetadata(
                 is_prefill=False,
-                slot_mapping=slot,
+                slot_mapping=buf["slots"][:bs],
                 block_tables=bt,
                 context_lens=buf["context_lens"][:bs],
             )
@@ -701,12 +716,13 @@ class ModelRunner:
                 rand, logits, buf["temps"][:bs], buf["top_p"][:bs],
                 buf["top_k"][:bs], buf["seeds"][:bs],
             )
-            sampled = torch.where(buf["greedy_mask"][:bs], greedy, rand)
-            buf["input_ids"][:bs].copy_(sampled)
-            buf["positions"][:bs].add_(1)
-            buf["context_lens"][:bs].add_(1)
-            # fresh Gumbel noise next replay, zero host involvement
-            buf["seeds"][:bs].add_(self._SEED_PRIME)
+            sampled = torch.empty_like(rand)
+            # with fresh Gumbel noise next replay, zero host involvement
+            _ops.advance_decode(
+                greedy, buf["input_ids"], buf["positions"], buf["context_lens"],
+                buf["slots"], bt, bsz, rand, buf["greedy_mask"], sampled,
+                buf["seeds"], self._SEED_PRIME,
+            )
             return sampled
 
         body()
@@ -726,57 +742,24 @@ class ModelRunner:
         return None
 
     def _run_graph(self, bucket: int, batch, block_manager) -> torch.Tensor:
-        n, nb = self._fill_pinned(batch, block_manager)
-        pin = self._pin
-        pnp = self._pin_np
-        if n < bucket:
-            # padded rows: write scratch KV to block 0 (reserved), ctx len 1
-            pnp["input_ids"][n:bucket] = 0
-            pnp["positions"][n:bucket] = 0
-            pnp["context_lens"][n:bucket] = 1
-            pnp["state_slots"][n:bucket] = 0
-            pnp["block_tables"][n:bucket, :nb] = 0
-        buf = self._graph_buffers
-        buf["state_slots"][:bucket].copy_(
-            pin["state_slots"][:bucket], non_blocking=True
-        )
-        # single async H2D per tensor, pinned -> static graph buffers
-        # (slot mapping is derived in-graph from block_tables + positions)
-        buf["input_ids"][:bucket].copy_(pin["input_ids"][:bucket], non_blocking=True)
-        buf["positions"][:bucket].copy_(pin["positions"][:bucket], non_blocking=True)
-        buf["context_lens"][:bucket].copy_(
-            pin["context_lens"][:bucket], non_blocking=True
-        )
-        buf["block_tables"][:bucket, :nb].copy_(
-            pin["block_tables"][:bucket, :nb], non_blocking=True
-        )
-        self._mark_staging()
+        n = self._stage_graph_inputs(bucket, batch, block_manager)
         self._graphs[bucket].replay()
-        return buf["logits"][bucket][:n]
+        return self._graph_buffers["logits"][bucket][:n]
 
     def _stage_graph_inputs(self, bucket: int, batch, block_manager) -> int:
+        """The batch in the graph buffers: one H2D copy, one kernel."""
         n, nb = self._fill_pinned(batch, block_manager)
-        pin = self._pin
-        pnp = self._pin_np
         if n < bucket:
-            pnp["input_ids"][n:bucket] = 0
-            pnp["positions"][n:bucket] = 0
-            pnp["context_lens"][n:bucket] = 1
-            pnp["state_slots"][n:bucket] = 0
-            pnp["block_tables"][n:bucket, :nb] = 0
+            # padded rows: write scratch KV to block 0 (reserved), ctx len 1
+            pad = self._pin[n * self._pin_stride : bucket * self._pin_stride]
+            pad.zero_()
+            self._pin_np["context_lens"][n:bucket] = 1
         buf = self._graph_buffers
-        buf["state_slots"][:bucket].copy_(
-            pin["state_slots"][:bucket], non_blocking=True
+        ops.unpack_decode_rows(
+            self._staged_rows(bucket), nb, buf["input_ids"], buf["positions"],
+            buf["context_lens"], buf["state_slots"], buf["slots"],
+            buf["block_tables"],
         )
-        buf["input_ids"][:bucket].copy_(pin["input_ids"][:bucket], non_blocking=True)
-        buf["positions"][:bucket].copy_(pin["positions"][:bucket], non_blocking=True)
-        buf["context_lens"][:bucket].copy_(
-            pin["context_lens"][:bucket], non_blocking=True
-        )
-        buf["block_tables"][:bucket, :nb].copy_(
-            pin["block_tables"][:bucket, :nb], non_blocking=True
-        )
-        self._mark_staging()
         return n
 
     def _stage_sampling_params(self, bucket: int, requests) -> None:

@@ -199,6 +199,48 @@ def greedy_sample(logits: torch.Tensor) -> torch.Tensor:
     return torch_ref.greedy_sample(logits)
 
 
+#: ints of a staged decode row before its page table: token id (64 bits),
+#: position (64 bits), context length, state slot, page slot, unused
+DECODE_ROW_HEAD = 8
+
+
+def unpack_decode_rows(
+    staged: torch.Tensor, width: int, ids, positions, context_lens, state_slots,
+    slots, tables,
+) -> None:
+    """Spreads staged decode rows (int32 [rows, DECODE_ROW_HEAD + width or
+    more]) over the buffers that a decode step reads."""
+    if staged.is_cuda:
+        _native_sampling("unpack_decode_rows").unpack_decode_rows(
+            staged, int(width), ids, positions, context_lens, state_slots, slots,
+            tables,
+        )
+        return
+    torch_ref.unpack_decode_rows(
+        staged, width, ids, positions, context_lens, state_slots, slots, tables
+    )
+
+
+def advance_decode(
+    greedy, ids, positions, context_lens, slots, tables, block: int,
+    random=None, greedy_mask=None, sampled=None, seeds=None, seed_step: int = 0,
+) -> None:
+    """The next decode step's inputs in place: the sampled token (``greedy``;
+    with ``random`` that one where ``greedy_mask`` is not set; also into
+    ``sampled``), position + 1 with its page slot, context + 1, seed +
+    ``seed_step``."""
+    if greedy.is_cuda:
+        _native_sampling("advance_decode").advance_decode(
+            greedy, random, greedy_mask, sampled, ids, positions, context_lens,
+            slots, seeds, int(seed_step), tables, int(block),
+        )
+        return
+    torch_ref.advance_decode(
+        greedy, ids, positions, context_lens, slots, tables, block, random,
+        greedy_mask, sampled, seeds, seed_step,
+    )
+
+
 def random_sample(
     logits: torch.Tensor,
     temperatures: torch.Tensor,

@@ -1,5 +1,6 @@
-// Helpers and the sampling wrappers shared by every extension module of this
-// package (each module links its own copy of sampling.hip).
+// Helpers and the sampling and decode-step wrappers shared by every extension
+// module of this package (each links its own copy of sampling.hip and
+// decode_step.hip).
 #pragma once
 
 #include <torch/extension.h>
@@ -15,10 +16,14 @@ hipError_t ks_gumbel_sample(void*, const void*, const void*, const void*,
 hipError_t ks_topk_topp_sample(void*, const void*, const void*, const void*,
                                const void*, const void*, int, int,
                                hipStream_t);
+hipError_t ks_unpack_decode_rows(const void*, long, int, int, void*, void*, void*,
+                                 void*, void*, void*, long, hipStream_t);
+hipError_t ks_advance_decode(const void*, const void*, const void*, void*, void*,
+                             void*, void*, void*, void*, long, const void*, long,
+                             int, int, int, hipStream_t);
 }
 
 namespace {
-
 
 hipStream_t current_stream() {
   return c10::hip::getCurrentHIPStream().stream();
@@ -80,7 +85,72 @@ void topk_topp_sample(at::Tensor& out, at::Tensor& logits,
             "topk_topp_sample");
 }
 
+#define CHECK_STEP(t, kind, n)                                             \
+  TORCH_CHECK((t).is_cuda() && (t).scalar_type() == kind && (t).dim() == 1 && \
+                  (t).is_contiguous() && (t).numel() >= (n),                  \
+              #t ": a dense vector of the rows expected")
+#define CHECK_TABLES(t, n)                                                   \
+  TORCH_CHECK((t).is_cuda() && (t).scalar_type() == at::kInt && (t).dim() == 2 && \
+                  (t).size(0) >= (n) && ((t).size(1) < 2 || (t).stride(1) == 1),  \
+              #t ": int32 rows expected")
+
+void unpack_decode_rows(at::Tensor& staged, int64_t width, at::Tensor& ids,
+                        at::Tensor& positions, at::Tensor& context_lens,
+                        at::Tensor& state_slots, at::Tensor& slots,
+                        at::Tensor& tables) {
+  TORCH_CHECK(staged.is_cuda() && staged.scalar_type() == at::kInt &&
+                  staged.dim() == 2 && staged.is_contiguous(),
+              "staged: int32 rows");
+  const int64_t rows = staged.size(0);
+  CHECK_STEP(ids, at::kLong, rows);
+  CHECK_STEP(positions, at::kLong, rows);
+  CHECK_STEP(context_lens, at::kInt, rows);
+  CHECK_STEP(state_slots, at::kInt, rows);
+  CHECK_STEP(slots, at::kInt, rows);
+  CHECK_TABLES(tables, rows);
+  TORCH_CHECK(width >= 0 && width <= tables.size(1), "table width");
+  check_hip(ks_unpack_decode_rows(
+                staged.data_ptr(), staged.size(1), (int)rows, (int)width,
+                ids.data_ptr(), positions.data_ptr(), context_lens.data_ptr(),
+                state_slots.data_ptr(), slots.data_ptr(), tables.data_ptr(),
+                std::max<int64_t>(tables.stride(0), tables.size(1)), current_stream()),
+            "unpack_decode_rows");
+}
+
+void advance_decode(at::Tensor& greedy, const c10::optional<at::Tensor>& random,
+                    const c10::optional<at::Tensor>& greedy_mask,
+                    const c10::optional<at::Tensor>& sampled, at::Tensor& ids,
+                    at::Tensor& positions, at::Tensor& context_lens,
+                    at::Tensor& slots, const c10::optional<at::Tensor>& seeds,
+                    int64_t seed_step, at::Tensor& tables, int64_t block) {
+  const int64_t rows = greedy.numel();
+  CHECK_STEP(greedy, at::kLong, rows);
+  CHECK_STEP(ids, at::kLong, rows);
+  CHECK_STEP(positions, at::kLong, rows);
+  CHECK_STEP(context_lens, at::kInt, rows);
+  CHECK_STEP(slots, at::kInt, rows);
+  CHECK_TABLES(tables, rows);
+  if (random) {
+    CHECK_STEP(*random, at::kLong, rows);
+    TORCH_CHECK(greedy_mask, "greedy_mask missing");
+    CHECK_STEP(*greedy_mask, at::kBool, rows);
+  }
+  if (sampled) CHECK_STEP(*sampled, at::kLong, rows);
+  if (seeds) CHECK_STEP(*seeds, at::kLong, rows);
+  check_hip(ks_advance_decode(
+                greedy.data_ptr(), random ? random->data_ptr() : nullptr,
+                greedy_mask ? greedy_mask->data_ptr() : nullptr,
+                sampled ? sampled->data_ptr() : nullptr, ids.data_ptr(),
+                positions.data_ptr(), context_lens.data_ptr(), slots.data_ptr(),
+                seeds ? seeds->data_ptr() : nullptr, (long)seed_step,
+                tables.data_ptr(), tables.stride(0), (int)tables.size(1), (int)block,
+                (int)rows, current_stream()),
+            "advance_decode");
+}
+
 void def_sampling(pybind11::module_& m) {
+  m.def("unpack_decode_rows", &unpack_decode_rows, "staged decode inputs to buffers");
+  m.def("advance_decode", &advance_decode, "the next decode step's inputs");
   m.def("greedy_sample", &greedy_sample, "argmax sampling");
   m.def("gumbel_sample", &gumbel_sample, "Gumbel-max temperature sampling");
   m.def("topk_topp_sample", &topk_topp_sample,

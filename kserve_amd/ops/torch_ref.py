@@ -1094,3 +1094,31 @@ def delta_unit_decay(
     z = torch.where(z > 30.0, z, torch.log1p(torch.exp(z)))
     A = torch.exp(a_log).repeat_interleave(a_raw.shape[1] // a_log.numel())
     return torch.exp(-A * z)
+
+
+def unpack_decode_rows(
+    staged, width, ids, positions, context_lens, state_slots, slots, tables
+) -> None:
+    n = staged.shape[0]
+    wide = staged[:, :4].contiguous().view(torch.int64)
+    ids[:n], positions[:n] = wide[:, 0], wide[:, 1]
+    context_lens[:n], state_slots[:n], slots[:n] = staged[:, 4], staged[:, 5], staged[:, 6]
+    tables[:n, :width] = staged[:, 8 : 8 + width]
+
+
+def advance_decode(
+    greedy, ids, positions, context_lens, slots, tables, block, random=None,
+    greedy_mask=None, sampled=None, seeds=None, seed_step: int = 0,
+) -> None:
+    n = greedy.shape[0]
+    token = greedy if random is None else torch.where(greedy_mask[:n], greedy, random)
+    if sampled is not None:
+        sampled[:n] = token
+    ids[:n] = token
+    positions[:n] += 1
+    context_lens[:n] += 1
+    pos = positions[:n]
+    page = (pos // block).clamp(0, tables.shape[1] - 1)
+    slots[:n] = tables[:n].gather(1, page[:, None])[:, 0] * block + (pos % block).int()
+    if seeds is not None:
+        seeds[:n] += seed_step

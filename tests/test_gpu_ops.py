@@ -863,6 +863,43 @@ class TestFusedProjections:
         torch.testing.assert_close(out.double(), norm, rtol=2.0 ** -6, atol=2.0 ** -6)
 
 
+class TestDecodeStep:
+    """The one-launch bookkeeping of a decode step against the CPU forms."""
+
+    @pytest.mark.parametrize("rows,width", [(1, 1), (3, 7), (256, 129), (257, 5000), (0, 4)])
+    def test_unpack_and_advance(self, dev, rows, width):
+        from kserve_amd import ops
+
+        torch.manual_seed(rows)
+        stride = ops.DECODE_ROW_HEAD + width + width % 2
+        staged = torch.randint(0, 1 << 20, (rows, stride), dtype=torch.int32)
+        staged[:, 1] = torch.randint(0, 3, (rows,))  # ids above 32 bits
+        staged[:, 2] = torch.randint(0, width * 16, (rows,))
+        staged[:, 3] = 0
+
+        def buffers(where):
+            v = lambda dt: torch.zeros(rows + 2, dtype=dt, device=where)  # noqa: E731
+            return [v(torch.int64), v(torch.int64), v(torch.int32), v(torch.int32),
+                    v(torch.int32), torch.zeros(rows + 2, width + 3, dtype=torch.int32, device=where)]
+
+        got, want = buffers(dev), buffers("cpu")
+        ops.unpack_decode_rows(staged.to(dev), width, *got)
+        ops.unpack_decode_rows(staged, width, *want)
+        greedy = torch.randint(0, 1 << 40, (rows,))
+        rand = torch.randint(0, 1 << 40, (rows,))
+        mask = torch.rand(rows) < 0.5
+        for random in (False, True):
+            outs = []
+            for where, (ids, pos, ctx, _, slots, tables) in ((dev, got), ("cpu", want)):
+                sampled = torch.zeros(rows, dtype=torch.int64, device=where)
+                seeds = torch.arange(rows, device=where)
+                more = (rand.to(where), mask.to(where), sampled, seeds, 77) if random else ()
+                ops.advance_decode(greedy.to(where), ids, pos, ctx, slots, tables, 16, *more)
+                outs.append((sampled, seeds))
+            assert all(torch.equal(a.cpu(), b) for a, b in zip(*outs))
+            assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
+
+
 class TestGemm8Experimental:
     """8-phase MFMA GEMM (experimental; not in the serving path).
     GPU-validated across the full SW x SCHED matrix — runs by
