@@ -199,6 +199,40 @@ class TestCausalConv:
             close(torch.cat(got[s]), want, be)
 
 
+    @pytest.mark.parametrize("taps", [2, 3, 4])
+    @pytest.mark.parametrize(
+        "lens",
+        [[1] * 5, [1, 0, 4, 7], [4, 4], [17, 1, 33], [16, 0, 15, 1, 40], [5]],
+    )
+    @pytest.mark.parametrize("bias", [False, True])
+    def test_portions_of_every_route(self, be, taps, lens, bias):
+        """Whole portions per block, tokens in blocks of 16 and the edges
+        between them; outputs and the state left, from a first portion (state
+        ignored) and a second one."""
+        C = 1028
+        T = sum(lens)
+        wide = rnd(2 * T, C + 8, seed=17, dtype=be[1])
+        w, b = rnd(C, taps, seed=18, scale=0.5), rnd(C, seed=19) if bias else None
+        slots = list(range(len(lens), 0, -1))
+        state = torch.full((len(lens) + 1, taps - 1, C), 77.0).to(be[1])
+        ref_state, dev_state = state.clone(), state.to(be[0])
+        dev_in = act(wide, be)
+        for part in (0, 1):
+            rows = slice(part * T, (part + 1) * T)
+            cu, seq, pos = layout(lens, [part * n for n in lens])
+            got = ops.causal_conv_silu(
+                dev_in[rows, 4 : 4 + C], f32(w, be), f32(b, be) if bias else None,
+                dev_state, i64(pos, be), i32(seq, be), i32(cu, be), i32(slots, be),
+            )
+            want = ops.torch_ref.causal_conv_silu(
+                wide[rows, 4 : 4 + C].double().float(), w, b, ref_state,
+                torch.tensor(pos), torch.tensor(cu), torch.tensor(slots),
+            )
+            close(got, want.double(), be)
+            used = [s for s, n in zip(slots, lens) if n]
+            assert torch.equal(dev_state.cpu()[used], ref_state[used])
+
+
 class TestScan:
     @pytest.mark.parametrize(
         "H,G,P,N",
