@@ -400,6 +400,113 @@ ssd_scan_kernel(
   }
 }
 
+// sums of V[0 .. NP) over groups of NL lanes, each level handing half of the
+// values that are left to the other half of the lanes: lane nl of a group ends
+// with the sum of V[nl / 4] (NP = NL / 4 values)
+template <int NL, int NP>
+__device__ __forceinline__ float group_sums(float (&V)[NP], const int nl) {
+  static_assert(NP == NL / 4 && (NL == 16 || NL == 32), "lanes");
+  auto dpp = [](float x, auto ctrl) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                           decltype(ctrl)::value, 0xF, 0xF, true));
+  };
+  if constexpr (NL == 32) {  // rows of 16 lanes: odd ones take V[4 ..]
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const auto r = __builtin_amdgcn_permlane16_swap(
+          __builtin_bit_cast(unsigned int, V[i]),
+          __builtin_bit_cast(unsigned int, V[i + 4]), false, false);
+      V[i] = __builtin_bit_cast(float, (unsigned int)r[0]) +
+             __builtin_bit_cast(float, (unsigned int)r[1]);
+    }
+  }
+  const bool half = nl & 8, quad = nl & 4;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)  // halves of a row, mirrored
+    V[i] = (half ? V[i + 2] : V[i]) +
+           dpp(half ? V[i] : V[i + 2], std::integral_constant<int, 0x140>{});
+  float v = (quad ? V[1] : V[0]) +  // quads of a half row, mirrored
+            dpp(quad ? V[0] : V[1], std::integral_constant<int, 0x141>{});
+  v += dpp(v, std::integral_constant<int, 0xB1>{});
+  v += dpp(v, std::integral_constant<int, 0x4E>{});
+  return v;
+}
+
+// The scan for portions of a token or two (decode steps), bound by the state's
+// way through memory: NL lanes hold a state row, 16 bytes each, so a wave reads
+// and writes whole rows, and a block's 64 columns of one head are all in flight
+// before the first token is there. What the vector units do beside it has to
+// stay below that: uniform addresses, sums that halve their values as they go
+// (with whole butterflies 770 us where this takes 401). 512 sequences of one
+// token, 64 heads of 64 x 128: 401 us = 5.4 TB/s, 594 us with the kernel above;
+// 128 sequences 83 and 153 us.
+template <int NL>  // lanes of a state row: N = 4 NL
+__global__ void __launch_bounds__(256) ssd_step_kernel(
+    float* __restrict__ y, const float* __restrict__ xbc,
+    const float* __restrict__ dt_raw_f32, const short* __restrict__ dt_raw_bf16,
+    long dt_stride, const float* __restrict__ dt_bias,
+    const float* __restrict__ a_log, const float* __restrict__ d_skip,
+    float* __restrict__ state, const long* __restrict__ positions,
+    const int* __restrict__ cu_seqlens, const int* __restrict__ slots,
+    int heads, int groups, int P) {
+  constexpr int N = 4 * NL;
+  constexpr int RP = 256 / NL;   // state rows (columns p) per pass
+  constexpr int NP = 64 / RP;    // passes
+  const int s = blockIdx.z, h = blockIdx.y, p0 = blockIdx.x * 64;
+  const int first = cu_seqlens[s], end = cu_seqlens[s + 1];
+  if (end <= first) return;
+  const unsigned nl = threadIdx.x % NL, pl = threadIdx.x / NL, n = nl * 4;
+  const bool fresh = positions[first] == 0;
+  float* sp = state + (((long)slots[s] * heads + h) * P + p0) * N;
+  const unsigned at = pl * N + n;
+  float4_t S[NP];
+  if (fresh) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) S[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+  } else {
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      S[i] = __builtin_nontemporal_load(
+          reinterpret_cast<const float4_t*>(sp + RP * i * N + at));
+  }
+  const int g = h / (heads / groups), inner = heads * P;
+  const long channels = inner + 2L * groups * N;
+  const float A = -expf(a_log[h]), bias = dt_bias[h], Dh = d_skip[h];
+  for (int t = first; t < end; ++t) {
+    const float* row = xbc + t * channels;
+    const float* xr = row + h * P + p0;
+    const float* br = row + inner + g * N;
+    const float4_t B = *reinterpret_cast<const float4_t*>(br + n);
+    const float4_t C = *reinterpret_cast<const float4_t*>(br + groups * N + n);
+    float x[NP], acc[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) x[i] = xr[RP * i + pl];
+    const long di = t * dt_stride + h;
+    const float v = (dt_raw_f32 ? dt_raw_f32[di] : bf16_bits_to_float(dt_raw_bf16[di])) + bias;
+    // softplus without a clamp; log1p(exp(v)) is v itself past v ~ 30
+    const float dt = v > 30.f ? v : log1pf(expf(v));
+    const float a = expf(A * dt);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const float dtx = dt * x[i];
+      acc[i] = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        S[i][j] = fmaf(a, S[i][j], B[j] * dtx);
+        acc[i] += S[i][j] * C[j];
+      }
+    }
+    const float sum = group_sums<NL, NP>(acc, nl);
+    const int i = nl / 4;  // the pass whose row this lane has the sum of
+    if (nl % 4 == 0)
+      y[(long)t * inner + h * P + p0 + RP * i + pl] = sum + Dh * xr[RP * i + pl];
+  }
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    *reinterpret_cast<float4_t*>(sp + RP * i * N + at) = S[i];
+}
+
 // ---------------------------------------------------------------------------
 // The scan in chunks of 64 tokens on the fp32 matrix cores
 // (v_mfma_f32_16x16x4_f32), for portions that are long enough to fill chunks.
@@ -804,6 +911,28 @@ extern "C" hipError_t ks_ssd_scan(void* y, const void* xbc, const void* dt_raw,
     else if (N <= 64) SSD_CHUNK(4);
     else SSD_CHUNK(8);
 #undef SSD_CHUNK
+    HIP_CHECK_KERNEL();
+    return hipSuccess;
+  }
+  // A token or two per sequence: whole state rows by 16-byte lanes (us, token by
+  // token in chunks of 16 -> this, 64 heads of 64 x 128: 128 x 1 token 153 ->
+  // 83, 128 x 2 159 -> 86, 64 x 8 85 -> 72; one long portion among them loses
+  // it again, 127 x 1 + 100 tokens 244 -> 183, 127 x 1 + 500 612 -> 655)
+  if (tokens <= 2L * num_seqs && (N == 64 || N == 128) && P % 64 == 0 &&
+      (((uintptr_t)xbc | (uintptr_t)state) & 15) == 0) {
+    const dim3 sgrid(P / 64, heads, num_seqs);
+#define SSD_STEP(nl)                                                          \
+  hipLaunchKernelGGL((ssd_step_kernel<nl>), sgrid, dim3(256), 0, stream,      \
+                     (float*)y, (const float*)xbc,                            \
+                     dt_is_f32 ? (const float*)dt_raw : nullptr,              \
+                     dt_is_f32 ? nullptr : (const short*)dt_raw, dt_stride,   \
+                     (const float*)dt_bias, (const float*)a_log,              \
+                     (const float*)d_skip, (float*)state,                     \
+                     (const long*)positions, (const int*)cu_seqlens,          \
+                     (const int*)slots, heads, groups, P)
+    if (N == 64) SSD_STEP(16);
+    else SSD_STEP(32);
+#undef SSD_STEP
     HIP_CHECK_KERNEL();
     return hipSuccess;
   }

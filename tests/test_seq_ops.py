@@ -270,6 +270,44 @@ class TestScan:
         close(torch.cat(outs), want, be, f32_tol=5e-5, bf16_tol=5e-5)
 
     @pytest.mark.parametrize(
+        "H,G,P,N", [(2, 1, 64, 128), (3, 3, 128, 64), (4, 2, 64, 64), (2, 2, 192, 128)]
+    )
+    def test_decode_sized_portions(self, be, H, G, P, N):
+        """Batches of a token or two per sequence, fresh and continued, one
+        with none and one long, the states handed from call to call."""
+        inner = H * P
+        calls = ((1, 2, 1, 0), (1, 1, 1, 1), (0, 5, 1, 2), (1, 1, 1, 1))
+        dt_bias = rnd(H, seed=72) - 1.0
+        a_log = rnd(H, seed=73, scale=0.5)
+        d_skip = rnd(H, seed=74)
+        total = [sum(c) for c in zip(*calls)]
+        xs = [rnd(n, inner + 2 * G * N, seed=80 + i, scale=0.7) for i, n in enumerate(total)]
+        dts = [rnd(n, H, seed=90 + i, dtype=be[1]) for i, n in enumerate(total)]
+        state = torch.full((6, H, P, N), 5.0, device=be[0])  # junk in the slots
+        at, got = [0] * 4, [[] for _ in total]
+        for lens in calls:
+            cu, _, pos = layout(lens, at)
+            part = lambda v: torch.cat([v[i][at[i] : at[i] + n] for i, n in enumerate(lens)])  # noqa: E731
+            y = ops.ssd_scan(
+                f32(part(xs), be), act(part(dts), be), f32(dt_bias, be), f32(a_log, be),
+                f32(d_skip, be), state, i64(pos, be), i32(cu, be), i32([4, 1, 5, 2], be), G,
+            )
+            for i, n in enumerate(lens):
+                got[i].append(y[cu[i] : cu[i + 1]])
+                at[i] += n
+        for i, (x, d) in enumerate(zip(xs, dts)):
+            n = x.shape[0]
+            want = O.ssd(
+                x[:, :inner].double().reshape(n, H, P),
+                x[:, inner : inner + G * N].double().reshape(n, G, N),
+                x[:, inner + G * N :].double().reshape(n, G, N),
+                O.softplus(d.double() + dt_bias.double()), a_log.double(),
+                d_skip.double(), G,
+            ).reshape(n, inner)
+            close(torch.cat(got[i]), want, be, f32_tol=5e-5, bf16_tol=5e-5)
+        assert (state[0] == 5.0).all() and (state[3] == 5.0).all()
+
+    @pytest.mark.parametrize(
         "H,G,P,N", [(2, 1, 64, 128), (4, 2, 24, 16), (2, 2, 72, 100), (3, 1, 8, 36)]
     )
     def test_long_portions(self, be, H, G, P, N):
