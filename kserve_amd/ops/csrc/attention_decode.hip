@@ -23,10 +23,12 @@
 //
 // Measured (32 query and 8 KV heads of 128; before it a wave per query head
 // walked the pages with vector dot products): 256 sequences of 2048 +- 60%
-// tokens 733 -> 389 us (5.6 TB/s of pages), all of 2048 606 -> 365 us (5.9);
-// 512 of 576 344 -> 217 us; 64 of 1000 71 -> 48 us; 24 of 900 35 -> 27 us; one
-// of 560 9.2 -> 7.4 us, of 7000 45 -> 12 us; E4M3, 96 of 3000 377 -> 128 us;
-// 64 / 8 heads, 64 of 600 71 -> 29 us.
+// tokens 739 -> 358 us (6.0 TB/s of pages), all of 2048 609 -> 330 us (6.5);
+// 512 of 576 341 -> 198 us; E4M3, 96 of 3000 385 -> 119 us; one of 560 9.4 ->
+// 7.6 us, of 7000 45 -> 12 us; 64 / 8 heads, 64 of 600 71 -> 29 us. The page
+// loads are non-temporal: a step's pages pass once and a model's do not fit
+// the caches (temporal, the first four take 392, 366, 216 and 131 us; only
+// pages still cached from the last call, 64 of 1000 alone, gain, 47 / 55).
 //
 // Splits are merged by paged_attention_reduce_kernel. Numerics oracle:
 // ops/torch_ref.paged_attention_decode.

@@ -481,6 +481,14 @@ __device__ __forceinline__ Range page_range(int ctx, int window, int chunk,
   return r;
 }
 
+constexpr int NT_AUX = 2;  // cache policy of a non-temporal load
+
+__device__ __forceinline__ uint4 load16_nt(const char* from) {
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(
+      uint4, __builtin_nontemporal_load(reinterpret_cast<const u4*>(from)));
+}
+
 struct DecodeArgs {
   void* out;                // [S, H, D]
   const void* q;            // [S, H, D] bf16 (PARTS 1) or fp32, row stride sq
@@ -613,11 +621,11 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
       __builtin_amdgcn_global_load_lds(
           reinterpret_cast<const unsigned int*>(
               src(p.k_cache, p.sk, n, pg, i, lchunk ^ k_swz<D>(r))),
-          reinterpret_cast<unsigned int*>(dst), 16, 0, 0);
+          reinterpret_cast<unsigned int*>(dst), 16, 0, NT_AUX);
       __builtin_amdgcn_global_load_lds(
           reinterpret_cast<const unsigned int*>(
               src(p.v_cache, p.sv, n, pg, i, lchunk ^ v_swz<D>(r))),
-          reinterpret_cast<unsigned int*>(dst + ROWS * D), 16, 0, 0);
+          reinterpret_cast<unsigned int*>(dst + ROWS * D), 16, 0, NT_AUX);
     }
   };
   uint4 raw[SRC == PAGES_DMA ? 1 : 2 * NI];
@@ -625,9 +633,8 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
     if constexpr (SRC != PAGES_DMA) {
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
-        raw[2 * i] = *reinterpret_cast<const uint4*>(src(p.k_cache, p.sk, n, pg, i, lchunk));
-        raw[2 * i + 1] =
-            *reinterpret_cast<const uint4*>(src(p.v_cache, p.sv, n, pg, i, lchunk));
+        raw[2 * i] = load16_nt(src(p.k_cache, p.sk, n, pg, i, lchunk));
+        raw[2 * i + 1] = load16_nt(src(p.v_cache, p.sv, n, pg, i, lchunk));
       }
     }
   };
@@ -879,7 +886,7 @@ __global__ __launch_bounds__(256) void paged_attention_reduce_kernel(
 }
 
 // Two waves per block: 64 KB of LDS, two blocks per compute unit, so one
-// block's first loads run under the other's last ones. (256 sequences of 819 to
+// block's first loads run under the other's last ones. (With temporal loads: 256 sequences of 819 to
 // 3277 tokens: 389 us with 2 waves, 390 with 4, 431 with 1; 64 of 400 to 1600:
 // 48.4 / 50.0 / 66.4.)
 constexpr int WAVES = 2;
@@ -904,7 +911,7 @@ hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) 
 }
 
 // Context splits for a launch over num_seqs x num_kv_heads: none from 512
-// blocks on, which fill the chip (64 sequences, 8 KV heads: 48.4 us unsplit,
+// blocks on, which fill the chip (temporal loads here too: 64 sequences, 8 KV heads: 48.4 us unsplit,
 // 51.4 with 2 splits, 50.4 with 4; 96 of 3000, E4M3: 128 / 140 / 129), about
 // 640 blocks below that (24 sequences of 900: 30.4 us with 3 splits, 27.4 with
 // 4, 29.8 with 6; 8 of 600: 9.3 with 8, 11.9 with 16), and at most 32 (one of
