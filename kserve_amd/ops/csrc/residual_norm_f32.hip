@@ -541,10 +541,12 @@ __global__ void gated_group_rms_norm_vec4_kernel(
   }
 }
 
-// Groups of at most 256 elements (heads of a recurrent read-out): a block
-// takes a whole row and each of its waves a group at a time, 4 elements per
-// lane, so a row costs one block instead of one block per group.
-template <typename TZ, typename TO>
+// Groups of at most 256 V elements (heads of a recurrent read-out, norm groups
+// of a state-space layer): a block takes a whole row and each of its waves a
+// group at a time, 4 V elements per lane, so a row costs one block and no
+// barrier. 8000 rows of 8 groups of 512: 50 us = 5.2 TB/s, 110 us with a block per group
+// (of whose 256 threads half had elements).
+template <typename TZ, typename TO, int V>
 __global__ void __launch_bounds__(NT) gated_group_rms_norm_wave_kernel(
     TO* __restrict__ out, const float* __restrict__ y, const TZ* __restrict__ z,
     long z_stride, const float* __restrict__ weight, int weight_n, float eps,
@@ -552,32 +554,38 @@ __global__ void __launch_bounds__(NT) gated_group_rms_norm_wave_kernel(
     int sigmoid) {
   const long row = blockIdx.x;
   const int lane = threadIdx.x & 63;
-  const int i = lane * 4;
-  const bool on = i < group_size;
   for (int g = threadIdx.x >> 6; g < groups; g += NW) {
     const int g0 = g * group_size;
-    float v[4] = {0.f, 0.f, 0.f, 0.f}, gate[4] = {1.f, 1.f, 1.f, 1.f};
+    float v[V][4], gate[V][4];
     float ss = 0.f;
-    if (on) {
-      float zv[4];
-      ld4<float>(y + row * inner + g0 + i, v);
-      ld4<TZ>(z + row * z_stride + g0 + i, zv);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float sg = gate_of(zv[j], sigmoid);
-        if (gate_after) gate[j] = sg;
-        else v[j] *= sg;
-        ss += v[j] * v[j];
+    for (int u = 0; u < V; ++u) {
+      const int i = (lane + 64 * u) * 4;
+      if (i < group_size) {
+        float zv[4];
+        ld4<float>(y + row * inner + g0 + i, v[u]);
+        ld4<TZ>(z + row * z_stride + g0 + i, zv);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float sg = gate_of(zv[j], sigmoid);
+          gate[u][j] = gate_after ? sg : 1.0f;
+          if (!gate_after) v[u][j] *= sg;
+          ss += v[u][j] * v[u][j];
+        }
       }
     }
     ss = wave_reduce_sum(ss);
-    if (on) {
-      const float inv = 1.0f / sqrtf(ss / (float)group_size + eps);
-      float w[4] = {1.f, 1.f, 1.f, 1.f}, o[4];
-      if (weight) ld4<float>(weight + (g0 + i) % weight_n, w);
+    const float inv = 1.0f / sqrtf(ss / (float)group_size + eps);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) o[j] = v[j] * inv * w[j] * gate[j];
-      st4<TO>(out + row * inner + g0 + i, o);
+    for (int u = 0; u < V; ++u) {
+      const int i = (lane + 64 * u) * 4;
+      if (i < group_size) {
+        float w[4] = {1.f, 1.f, 1.f, 1.f}, o[4];
+        if (weight) ld4<float>(weight + (g0 + i) % weight_n, w);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = v[u][j] * inv * w[j] * gate[u][j];
+        st4<TO>(out + row * inner + g0 + i, o);
+      }
     }
   }
 }
@@ -909,15 +917,22 @@ extern "C" hipError_t ks_gated_group_rms_norm(void* out, const void* y,
 #define GNORM_ARGS(TT)                                                        \
   (TT*)out, (const float*)y, (const TT*)z, z_stride, (const float*)weight,    \
       weight_n, eps, inner, gs
-  if (vec && gs <= 4 * WAVE_SIZE && groups > 1) {
-    if (is_f32)
-      hipLaunchKernelGGL((gated_group_rms_norm_wave_kernel<float, float>),
-                         dim3(rows), dim3(NT), 0, stream, GNORM_ARGS(float),
-                         groups, gate_after, gate_sigmoid);
-    else
-      hipLaunchKernelGGL((gated_group_rms_norm_wave_kernel<short, short>),
-                         dim3(rows), dim3(NT), 0, stream, GNORM_ARGS(short),
-                         groups, gate_after, gate_sigmoid);
+  // a wave per group, where a row has more than one
+  if (vec && gs <= 16 * WAVE_SIZE && groups > 1) {
+#define GNORM_WAVE(TT, V)                                                     \
+  hipLaunchKernelGGL((gated_group_rms_norm_wave_kernel<TT, TT, V>),           \
+                     dim3(rows), dim3(NT), 0, stream, GNORM_ARGS(TT), groups, \
+                     gate_after, gate_sigmoid)
+#define GNORM_WAVES(V)                \
+  do {                                \
+    if (is_f32) GNORM_WAVE(float, V); \
+    else GNORM_WAVE(short, V);        \
+  } while (0)
+    if (gs <= 4 * WAVE_SIZE) GNORM_WAVES(1);
+    else if (gs <= 8 * WAVE_SIZE) GNORM_WAVES(2);
+    else GNORM_WAVES(4);
+#undef GNORM_WAVES
+#undef GNORM_WAVE
     HIP_CHECK_KERNEL();
     return hipSuccess;
   }

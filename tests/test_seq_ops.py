@@ -135,6 +135,25 @@ class TestNorms:
         want = O.rms(v.reshape(4, groups, -1), 1e-5).reshape(4, inner) * w.double()
         close(got, want, be)
 
+    @pytest.mark.parametrize("gs", [4, 256, 260, 512, 516, 1024, 1028, 2052])
+    @pytest.mark.parametrize("groups", [1, 2, 5])
+    @pytest.mark.parametrize("gate_after", [False, True])
+    def test_gated_group_norm_by_waves(self, be, gs, groups, gate_after):
+        """Group sizes at the edges of what a wave takes, rows that are not."""
+        inner = gs * groups
+        y = rnd(3, inner, seed=8, scale=2.0)
+        wide = rnd(3, inner + 8, seed=9, dtype=be[1])
+        z = wide[:, 4 : 4 + inner]
+        w = rnd(inner, seed=10) + 1.0
+        got = ops.gated_group_rms_norm(
+            f32(y, be), act(wide, be)[:, 4 : 4 + inner], f32(w, be), 1e-5, groups,
+            be[1], gate_after=gate_after,
+        )
+        g = O.silu(z.double())
+        v = y.double() if gate_after else y.double() * g
+        want = O.rms(v.reshape(3, groups, -1), 1e-5).reshape(3, inner) * w.double()
+        close(got, want * g if gate_after else want, be)
+
 
 class TestClampedGLU:
     def test_branches_and_limits(self, be):
