@@ -84,6 +84,88 @@ __global__ void layer_norm_kernel(
   }
 }
 
+// Rows of up to 2048: a wave per row with the row in registers, read once, no
+// barrier, and the variance from the centred values. Bound by memory: 6400 rows
+// of 768 with the residual take 9.2 us, 10.1 us with a block per row (of whose
+// 256 threads 96 had a vector).
+template <bool FUSED_ADD, int V>
+__global__ __launch_bounds__(256) void layer_norm_wave_kernel(
+    short* __restrict__ out, const short* __restrict__ input,
+    const short* __restrict__ residual, const short* __restrict__ weight,
+    const short* __restrict__ bias, const float eps, const int rows,
+    const int hidden) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= rows) return;
+  const int nvec = hidden >> 3;
+  const long at = (long)row * nvec;
+  float x[V][8];
+  float sum = 0.f;
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const int i = lane + 64 * u;
+    if (i < nvec) {
+      const short8_t a = reinterpret_cast<const short8_t*>(input)[at + i];
+      short8_t r;
+      if constexpr (FUSED_ADD) r = reinterpret_cast<const short8_t*>(residual)[at + i];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        x[u][j] = bf16_bits_to_float(a[j]);
+        if constexpr (FUSED_ADD) x[u][j] += bf16_bits_to_float(r[j]);
+        sum += x[u][j];
+      }
+    }
+  }
+  const float mean = wave_reduce_sum(sum) / hidden;
+  float sq = 0.f;
+#pragma unroll
+  for (int u = 0; u < V; ++u)
+    if (lane + 64 * u < nvec) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sq += (x[u][j] - mean) * (x[u][j] - mean);
+    }
+  const float rstd = rsqrtf(wave_reduce_sum(sq) / hidden + eps);
+#pragma unroll
+  for (int u = 0; u < V; ++u) {
+    const int i = lane + 64 * u;
+    if (i < nvec) {
+      const short8_t w = reinterpret_cast<const short8_t*>(weight)[i];
+      const short8_t b = reinterpret_cast<const short8_t*>(bias)[i];
+      short8_t o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        o[j] = float_to_bf16_bits((x[u][j] - mean) * rstd * bf16_bits_to_float(w[j]) +
+                                  bf16_bits_to_float(b[j]));
+      reinterpret_cast<short8_t*>(out)[at + i] = o;
+    }
+  }
+}
+
+template <bool FUSED_ADD>
+hipError_t launch_layer_norm(void* out, const void* input, const void* residual,
+                             const void* weight, const void* bias, float eps,
+                             int rows, int hidden, hipStream_t stream) {
+  if (hidden % 8 != 0) return hipErrorInvalidValue;
+  if (rows < 1) return hipSuccess;
+#define LN_ARGS                                                           \
+  (short*)out, (const short*)input, (const short*)residual,               \
+      (const short*)weight, (const short*)bias, eps, rows, hidden
+#define LN_WAVE(V)                                                        \
+  hipLaunchKernelGGL((layer_norm_wave_kernel<FUSED_ADD, V>),              \
+                     dim3((rows + 3) / 4), dim3(256), 0, stream, LN_ARGS)
+  if (hidden <= 512) LN_WAVE(1);
+  else if (hidden <= 1024) LN_WAVE(2);
+  else if (hidden <= 2048) LN_WAVE(4);
+  else
+    hipLaunchKernelGGL((layer_norm_kernel<FUSED_ADD>),
+                       dim3(rows < 2048 ? rows : 2048), dim3(256), 0, stream,
+                       LN_ARGS);
+#undef LN_WAVE
+#undef LN_ARGS
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
+}
+
 __global__ void gelu_kernel(short* __restrict__ out,
                             const short* __restrict__ input, const long nvec) {
   const short8_t* in = reinterpret_cast<const short8_t*>(input);
@@ -215,30 +297,16 @@ hipError_t ks_embed_layer_norm(void* out, const void* word, const void* pos_tabl
 hipError_t ks_layer_norm(void* out, const void* input, const void* weight,
                          const void* bias, float eps, int rows, int hidden,
                          hipStream_t stream) {
-  if (hidden % 8 != 0) return hipErrorInvalidValue;
-  int grid = rows < 2048 ? rows : 2048;
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL((layer_norm_kernel<false>), dim3(grid), dim3(256), 0,
-                     stream, (short*)out, (const short*)input, nullptr,
-                     (const short*)weight, (const short*)bias, eps, rows,
-                     hidden);
-  HIP_CHECK_KERNEL();
-  return hipSuccess;
+  return launch_layer_norm<false>(out, input, nullptr, weight, bias, eps, rows,
+                                  hidden, stream);
 }
 
 hipError_t ks_fused_add_layer_norm(void* out, const void* input,
                                    const void* residual, const void* weight,
                                    const void* bias, float eps, int rows,
                                    int hidden, hipStream_t stream) {
-  if (hidden % 8 != 0) return hipErrorInvalidValue;
-  int grid = rows < 2048 ? rows : 2048;
-  if (grid == 0) return hipSuccess;
-  hipLaunchKernelGGL((layer_norm_kernel<true>), dim3(grid), dim3(256), 0,
-                     stream, (short*)out, (const short*)input,
-                     (const short*)residual, (const short*)weight,
-                     (const short*)bias, eps, rows, hidden);
-  HIP_CHECK_KERNEL();
-  return hipSuccess;
+  return launch_layer_norm<true>(out, input, residual, weight, bias, eps, rows,
+                                 hidden, stream);
 }
 
 hipError_t ks_gelu(void* out, const void* input, long numel,

@@ -900,6 +900,28 @@ class TestDecodeStep:
             assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
 
 
+class TestLayerNormEdges:
+    """Rows at the edges of what a wave holds, against fp64: fp32 sums of
+    ``hidden`` terms, then one rounding to bf16."""
+
+    @pytest.mark.parametrize("hidden", [8, 504, 512, 520, 768, 1024, 1032, 2048, 2056])
+    @pytest.mark.parametrize("rows", [1, 4, 5, 2051])
+    @pytest.mark.parametrize("add", [False, True])
+    def test_layer_norm(self, dev, hidden, rows, add):
+        from kserve_amd import ops
+
+        torch.manual_seed(hidden + rows)
+        x, r = (torch.randn(rows, hidden, device=dev).mul_(3).add_(1).to(torch.bfloat16) for _ in range(2))
+        w, b = (torch.randn(hidden, device=dev).to(torch.bfloat16) for _ in range(2))
+        out = (ops.fused_add_layer_norm(x, r, w, b, 1e-6) if add
+               else ops.layer_norm(x, w, b, 1e-6))
+        v = x.double() + (r.double() if add else 0)
+        n = (v - v.mean(-1, keepdim=True)) * (v.var(-1, unbiased=False, keepdim=True) + 1e-6).rsqrt()
+        want = n * w.double() + b.double()
+        lim = 2.0 ** -8 * want.abs() + hidden * 2.0 ** -22 * (n.abs() * w.double().abs() + 1)
+        assert ((out.double() - want).abs() <= lim).all()
+
+
 class TestGemm8Experimental:
     """8-phase MFMA GEMM (experimental; not in the serving path).
     GPU-validated across the full SW x SCHED matrix — runs by
