@@ -252,9 +252,9 @@ def random_sample(
 ) -> torch.Tensor:
     """Temperature/top-k/top-p/min-p sampling.
 
-    GPU: one fused HIP kernel. Plain temperature sampling is Gumbel-max;
-    top-k/top-p use a bf16 radix-histogram select (exact k-th value / mass
-    threshold, no sort) followed by Gumbel-max over the surviving set.
+    GPU: one fused HIP kernel. Rows with top-k or top-p get the exact k-th
+    value / mass threshold from counts per bf16 key (no sort); then Gumbel-max
+    over the surviving set, which is the whole row for plain temperatures.
     min_p (rare) routes to the fp32 sort path.
     """
     has_min_p = min_p is not None and bool((min_p > 0).any())
@@ -264,8 +264,13 @@ def random_sample(
         out = torch.empty(
             logits.shape[0], dtype=torch.int64, device=logits.device
         )
-        needs_trunc = bool((top_p < 1.0).any()) or bool((top_k > 0).any())
-        if needs_trunc:
+        # given one value per row on the device, the kernel sees what there is
+        # to cut: no round trip to the host to choose one
+        per_row = all(
+            t.shape == out.shape and t.device == logits.device and t.is_contiguous()
+            for t in (top_p, top_k)
+        ) and top_p.dtype == torch.float32
+        if per_row or bool((top_p < 1.0).any()) or bool((top_k > 0).any()):
             _native_sampling("random_sample").topk_topp_sample(
                 out, logits, temperatures, top_p, top_k.to(torch.int32), seeds
             )

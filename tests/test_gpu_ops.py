@@ -922,6 +922,37 @@ class TestLayerNormEdges:
         assert ((out.double() - want).abs() <= lim).all()
 
 
+class TestUncutSampling:
+    @pytest.mark.parametrize("V", [1, 7, 8, 1031, 32000, 65544, 128257])
+    def test_rows_without_limits(self, dev, V):
+        """The fused sampler's uncut rows are the plain kernel's, for any
+        logits, and the same whichever form the limits are given in."""
+        import kserve_amd_C
+        from kserve_amd import ops
+
+        torch.manual_seed(V)
+        S = 6
+        logits = (torch.randn(S, V, device=dev) * 2.5).to(torch.bfloat16)
+        logits[1] = 0.0
+        logits[2, V // 2 :] = float("-inf")
+        logits[3, V // 3] = float("nan")
+        temps = torch.rand(S, device=dev) + 0.5
+        seeds = torch.randint(0, 1 << 31, (S,), device=dev)
+        one = torch.ones(S, device=dev)
+        zero = torch.zeros(S, dtype=torch.int32, device=dev)
+        want = torch.empty(S, dtype=torch.int64, device=dev)
+        kserve_amd_C.gumbel_sample(want, logits, temps, zero, seeds)
+        for top_p, top_k in (
+            (one, zero), (one, zero.long()), (one.cpu(), zero.cpu()),
+            (one[:1].expand(S), zero), (one.double(), zero), (one[:1], zero[:1]),
+        ):
+            if top_k.device.type == "cpu":
+                top_k = top_k.to(dev)
+            assert torch.equal(
+                ops.random_sample(logits, temps, top_p, top_k, seeds=seeds), want
+            )
+
+
 class TestGemm8Experimental:
     """8-phase MFMA GEMM (experimental; not in the serving path).
     GPU-validated across the full SW x SCHED matrix — runs by
