@@ -25,7 +25,6 @@ from typing import List, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from kserve_amd import ops
 from kserve_amd.engine.config import (
@@ -205,7 +204,7 @@ class DesalixForCausalLM(nn.Module):
         )
 
     def compute_logits(self, hidden):
-        return F.linear(hidden, self.head)
+        return ops.linear(hidden, self.head)
 
     # -- weights ----------------------------------------------------------------
     @torch.no_grad()

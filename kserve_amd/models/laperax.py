@@ -24,7 +24,6 @@ from typing import List, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from kserve_amd import ops
 from kserve_amd.engine.config import HybridLayerSpec, HybridModelConfig
@@ -168,7 +167,7 @@ class LaperaxForCausalLM(nn.Module):
 
     def compute_logits(self, hidden):
         return ops.scale_softcap(
-            F.linear(hidden, self.head), self.config.logit_scale,
+            ops.linear(hidden, self.head), self.config.logit_scale,
             self.config.logit_softcap,
         )
 

@@ -25,7 +25,6 @@ from typing import List, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from kserve_amd import ops
 from kserve_amd.engine.config import HybridLayerSpec, HybridModelConfig, SiluGLUSpec
@@ -94,7 +93,7 @@ class MededraLayer(nn.Module):
         kernel: (delta, delta2, pre_w, pre_w2)."""
         if self.attn is not None:
             return self.attn(h, positions, cache, meta), None, None, None
-        proj = F.linear(h, self.fused_proj)
+        proj = ops.linear(h, self.fused_proj)
         a = self.left.proj_width
         left = self.left.mix(proj[:, :a], positions, cache, meta)
         right = self.right.mix(proj[:, a:], positions, cache, meta)
@@ -210,7 +209,7 @@ class MededraForCausalLM(nn.Module):
 
     def compute_logits(self, hidden):
         return ops.scale_softcap(
-            F.linear(hidden, self.head), self.config.logit_scale,
+            ops.linear(hidden, self.head), self.config.logit_scale,
             self.config.logit_softcap,
         )
 

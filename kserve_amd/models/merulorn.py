@@ -18,7 +18,6 @@ from typing import List, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from kserve_amd import ops
 from kserve_amd.engine.config import HybridLayerSpec, HybridModelConfig
@@ -84,7 +83,7 @@ class MerulornLayer(nn.Module):
     def mixer(self, h, positions, cache: LayerCache, meta):
         """Returns (delta0, scale0, delta1, scale1) to add to the stream."""
         if self.attn is not None and self.ssm is not None:
-            proj = F.linear(h, self.fused_proj, self.fused_bias)
+            proj = ops.linear(h, self.fused_proj, self.fused_bias)
             a = self.attn.proj_width
             left = self.attn.mix(proj[:, :a], positions, cache, meta)
             right = self.ssm.mix(proj[:, a:], positions, cache, meta)
@@ -207,7 +206,7 @@ class MerulornForCausalLM(nn.Module):
         )
 
     def compute_logits(self, hidden):
-        return F.linear(hidden, self.head)
+        return ops.linear(hidden, self.head)
 
     # -- weights ----------------------------------------------------------------
     @torch.no_grad()

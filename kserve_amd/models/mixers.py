@@ -19,7 +19,6 @@ from typing import NamedTuple, Optional, Tuple
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from kserve_amd import ops
 from kserve_amd.engine.config import (
@@ -120,10 +119,10 @@ class SSDMixer(nn.Module):
         yn = ops.gated_group_rms_norm(
             y, z, self.norm_w, self.eps, s.norm_groups, self.dtype
         )
-        return F.linear(yn, self.o_proj)
+        return ops.linear(yn, self.o_proj)
 
     def forward(self, h, positions, cache: LayerCache, meta):
-        return self.mix(F.linear(h, self.in_proj), positions, cache, meta)
+        return self.mix(ops.linear(h, self.in_proj), positions, cache, meta)
 
 
 class NormedGatedAttention(nn.Module):
@@ -176,11 +175,11 @@ class NormedGatedAttention(nn.Module):
             meta.context_lens, s.scale, meta.max_seqlen, s.heads, gate=gate,
             out_dtype=self.dtype,
         )
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
     def forward(self, h, positions, cache: LayerCache, meta):
         return self.mix(
-            F.linear(h, self.qkvg, self.qkvg_bias), positions, cache, meta
+            ops.linear(h, self.qkvg, self.qkvg_bias), positions, cache, meta
         )
 
 
@@ -250,7 +249,7 @@ class RotaryChunkSinkAttention(nn.Module):
 
     def forward(self, h, positions, cache: LayerCache, meta):
         s = self.spec
-        proj = F.linear(h, self.qkv)
+        proj = ops.linear(h, self.qkv)
         a, b = self.q_w, self.q_w + self.k_w
         qn = ops.qk_headnorm_rope_cache(
             proj[:, :a], proj[:, a:b], proj[:, b:], self.q_norm, self.k_norm,
@@ -265,7 +264,7 @@ class RotaryChunkSinkAttention(nn.Module):
             out_inv_freq=self.v_inv_freq, window=s.window,
             keep_first=s.keep_first,
         )
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
 
 class ClampedGLU(nn.Module):
@@ -289,9 +288,9 @@ class ClampedGLU(nn.Module):
 
     def forward(self, h):
         act = ops.clamped_swiglu(
-            F.linear(h, self.gate_up), self.ALPHA, self.spec.limit
+            ops.linear(h, self.gate_up), self.ALPHA, self.spec.limit
         )
-        return F.linear(act, self.down)
+        return ops.linear(act, self.down)
 
 
 class RoutedClampedMoE(nn.Module):
@@ -508,7 +507,7 @@ class LatentAttention(nn.Module):
     def forward(self, h, positions, cache: LayerCache, meta):
         """``cache.k``: this layer's pages, or those of layer ``kv_from``."""
         s = self.spec
-        proj = F.linear(h, self.in_proj)
+        proj = ops.linear(h, self.in_proj)
         turn = {"pairs": s.rot_pairs, "rot_mult": self.rot_mult}
         if s.q_rank or self.own_kv:
             cq = ops.latent_norm_rope_cache(
@@ -518,10 +517,10 @@ class LatentAttention(nn.Module):
                 positions, meta.slot_mapping, cache.k if self.own_kv else None,
                 self.eps, self.inv_freq, **turn,
             )
-        q = F.linear(cq, self.uq) if s.q_rank else proj[:, : self.q_in]
+        q = ops.linear(cq, self.uq) if s.q_rank else proj[:, : self.q_in]
         gate = proj[:, self.q_in + self.kv_cols :] if s.gate else None
         if self.expanded:
-            return F.linear(
+            return ops.linear(
                 self._expanded_attention(q, gate, positions, cache, meta),
                 self.o_proj,
             )
@@ -536,7 +535,7 @@ class LatentAttention(nn.Module):
             window=s.window,
         )
         o = ops.head_matmul_rope(o_lat, self.uv, s.heads)
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
     def _expanded_attention(self, q, gate, positions, cache: LayerCache, meta):
         """Per-head keys and values of every sequence's whole context, built
@@ -565,11 +564,11 @@ class LatentAttention(nn.Module):
         lat = rows[..., :R].reshape(-1, R)
         # one plain GEMM each: rows [n, R] against all heads' matrices
         uk = self.uk_t.transpose(1, 2).reshape(H * s.dim, R)
-        keys = F.linear(lat, uk).view(n_pages, bs, H, s.dim)
+        keys = ops.linear(lat, uk).view(n_pages, bs, H, s.dim)
         if rd:
             shared = rows[..., R:].unsqueeze(2).expand(-1, -1, H, -1)
             keys = torch.cat([keys, shared], dim=-1)
-        vals = F.linear(lat, self.uv.view(H * s.vdim, R))
+        vals = ops.linear(lat, self.uv.view(H * s.vdim, R))
         vals = vals.view(n_pages, bs, H, s.vdim)
         k_tmp = keys.transpose(1, 2).contiguous()
         v_tmp = vals.transpose(1, 2).contiguous()
@@ -606,8 +605,8 @@ class GeluMLP(nn.Module):
         self.down_b.copy_(get(prefix + "down.b").to(dt))
 
     def forward(self, h):
-        a = ops.bias_gelu_tanh(F.linear(h, self.up), self.up_b)
-        return F.linear(a, self.down, self.down_b)
+        a = ops.bias_gelu_tanh(ops.linear(h, self.up), self.up_b)
+        return ops.linear(a, self.down, self.down_b)
 
 
 class SiluGLU(nn.Module):
@@ -626,7 +625,7 @@ class SiluGLU(nn.Module):
         self.down.copy_(get(prefix + "down").to(dt))
 
     def forward(self, h):
-        return F.linear(ops.glu_silu_scale(F.linear(h, self.gate_up)), self.down)
+        return ops.linear(ops.glu_silu_scale(ops.linear(h, self.gate_up)), self.down)
 
 
 class ExpertRows(NamedTuple):
@@ -703,11 +702,11 @@ class SoftmaxRoutedMoE(nn.Module):
         T, W = h.shape
         if E == 0:
             return torch.zeros((T, W), dtype=h.dtype, device=h.device)
-        gu = F.linear(h, self.gate_up.view(E * 2 * ff, W))
+        gu = ops.linear(h, self.gate_up.view(E * 2 * ff, W))
         act = ops.glu_silu_scale(
             gu.view(T * E, 2 * ff), dense_w[:, :E].reshape(-1)
         )
-        return F.linear(act.view(T, E * ff), self.down.view(W, E * ff))
+        return ops.linear(act.view(T, E * ff), self.down.view(W, E * ff))
 
     def _sorted_rows(self, h, idx, w) -> ExpertRows:
         E, top = self.spec.experts, self.spec.top
@@ -819,7 +818,7 @@ class RetentionMixer(nn.Module):
 
     def forward(self, h, positions, cache: LayerCache, meta):
         s = self.spec
-        proj = F.linear(h, self.qkvg)
+        proj = ops.linear(h, self.qkvg)
         a, b, c = self.qk_w, 2 * self.qk_w, 2 * self.qk_w + self.v_w
         # q | k | v to fp32 in one pass: q and k rotated, k scaled
         qkv = ops.rope_scale_heads(
@@ -833,7 +832,7 @@ class RetentionMixer(nn.Module):
         on = ops.gated_group_rms_norm(
             o, proj[:, c:], None, self.eps, s.heads, self.dtype, gate_after=True
         )
-        return F.linear(on, self.o_proj)
+        return ops.linear(on, self.o_proj)
 
 
 class GatedDeltaMixer(nn.Module):
@@ -890,7 +889,7 @@ class GatedDeltaMixer(nn.Module):
 
     def forward(self, h, positions, cache: LayerCache, meta):
         s = self.spec
-        proj = F.linear(h, self.proj)
+        proj = ops.linear(h, self.proj)
         cc = s.conv_channels
         gate = proj[:, cc : cc + self.v_w]
         b_raw = proj[:, cc + self.v_w : cc + self.v_w + s.heads]
@@ -915,7 +914,7 @@ class GatedDeltaMixer(nn.Module):
         on = ops.gated_group_rms_norm(
             o, gate, self.norm_w, self.eps, s.heads, self.dtype, gate_after=True
         )
-        return F.linear(on, self.o_proj)
+        return ops.linear(on, self.o_proj)
 
 
 class GatedLinearMixer(nn.Module):
@@ -972,7 +971,7 @@ class GatedLinearMixer(nn.Module):
 
     def forward(self, h, positions, cache: LayerCache, meta):
         s = self.spec
-        proj = F.linear(h, self.proj)
+        proj = ops.linear(h, self.proj)
         a, b, c = self.qk_w, 2 * self.qk_w, 2 * self.qk_w + self.v_w
         decay = ops.lowrank_channel_decay(
             proj[:, self.low_at : self.low_at + self.a_rank], self.a2, self.a2_b,
@@ -987,7 +986,7 @@ class GatedLinearMixer(nn.Module):
             o, proj[:, c : self.low_at], self.norm_w, self.eps, s.heads,
             self.dtype, gate_after=True,
         )
-        return F.linear(on, self.o_proj)
+        return ops.linear(on, self.o_proj)
 
 
 class SquaredReluMoE(nn.Module):
@@ -1032,9 +1031,9 @@ class SquaredReluMoE(nn.Module):
     def _dense(self, h, dense_w, extra):
         E, ff = self.spec.experts, self.spec.ff
         T, W = h.shape
-        x = F.linear(h, self.up.view(E * ff, W))
+        x = ops.linear(h, self.up.view(E * ff, W))
         act = ops.relu2_scale(x.view(T * E, ff), dense_w.reshape(-1))
-        y = F.linear(act.view(T, E * ff), self.down.view(W, E * ff))
+        y = ops.linear(act.view(T, E * ff), self.down.view(W, E * ff))
         ar = torch.arange(T, dtype=torch.int32, device=h.device)
         return ops.combine_rows(y, ar, 1, extra)
 
@@ -1157,7 +1156,7 @@ class DifferentialAttention(nn.Module):
 
     def forward(self, h, positions, cache: LayerCache, meta):
         s = self.spec
-        x = F.linear(h, self.qkv)
+        x = ops.linear(h, self.qkv)
         if s.conv > 1:
             x = ops.causal_conv_silu(
                 x, self.conv_w, None, cache.conv, positions, meta.seq_of_token,
@@ -1179,7 +1178,7 @@ class DifferentialAttention(nn.Module):
             softcap=s.softcap,
         )
         o = ops.diff_combine(o, self.lam, s.heads, self.eps, 1.0 - s.diff, self.dtype)
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
 
 class TalkingHeadsAttention(nn.Module):
@@ -1273,10 +1272,10 @@ class TalkingHeadsAttention(nn.Module):
             meta.context_lens, s.scale, meta.max_seqlen, s.heads, self.talk,
             self.bias, s.window, gate=proj[:, b:], out_dtype=self.dtype,
         )
-        return F.linear(o, self.o_proj)
+        return ops.linear(o, self.o_proj)
 
     def forward(self, h, positions, cache: LayerCache, meta):
-        return self.mix(F.linear(h, self.qkg), positions, cache, meta)
+        return self.mix(ops.linear(h, self.qkg), positions, cache, meta)
 
 
 class ChannelDeltaMixer(nn.Module):
@@ -1361,7 +1360,7 @@ class ChannelDeltaMixer(nn.Module):
 
     def mix(self, proj, positions, cache: LayerCache, meta):
         s = self.spec
-        low = F.linear(proj[:, self.low_at : self.b_at], self.low2)
+        low = ops.linear(proj[:, self.low_at : self.b_at], self.low2)
         if s.conv > 1:
             qkv = ops.causal_conv_silu(
                 proj[:, : self.low_at], self.conv_w, None, cache.conv, positions,
@@ -1384,7 +1383,7 @@ class ChannelDeltaMixer(nn.Module):
             o, low[:, self.decay_w :], self.norm_w, self.eps, s.heads, self.dtype,
             gate_after=True, gate_sigmoid=True,
         )
-        return F.linear(on, self.o_proj)
+        return ops.linear(on, self.o_proj)
 
     def forward(self, h, positions, cache: LayerCache, meta):
-        return self.mix(F.linear(h, self.proj), positions, cache, meta)
+        return self.mix(ops.linear(h, self.proj), positions, cache, meta)

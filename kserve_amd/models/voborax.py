@@ -23,7 +23,6 @@ from typing import List, Optional
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from kserve_amd import ops
 from kserve_amd.engine.config import (
@@ -197,7 +196,7 @@ class VoboraxForCausalLM(nn.Module):
         )
 
     def compute_logits(self, hidden):
-        return F.linear(hidden, self.head)
+        return ops.linear(hidden, self.head)
 
     # -- weights ----------------------------------------------------------------
     @torch.no_grad()
