@@ -15,7 +15,9 @@
 //    q (fp32) out and scatter k / v into the paged cache.
 //  * ctx_attention_f32: causal attention of a flat variable-length query
 //    batch against each sequence's pages (the portion's own keys are already
-//    in the cache). Both products run on the fp32 matrix cores
+//    in the cache). bf16 pages with head sizes that mfma_attention.h has go
+//    there (fp32 operands as three exact bf16 parts); what follows is the
+//    general kernel. Both of its products run on the fp32 matrix cores
 //    (v_mfma_f32_16x16x4_f32), so q.k, the softmax weights and weights x V
 //    are all true fp32 whatever the cache dtype; K/V tiles of 64 keys are
 //    converted to fp32 while they are staged in LDS.
