@@ -29,9 +29,8 @@
 // 413 -> 149 us; 2 x 1000 queries over 13000 paged keys 2441 -> 509 us (E4M3
 // pages 2596 -> 625); 64 x 128, 12 heads of 64, bidirectional 28 -> 13 us.
 //
-// Replaces the vLLM flash prefill the reference delegates to
-// (SURVEY.md §2.7 row 1). Numerics oracles: ops/torch_ref.flash_prefill_varlen
-// and context_attention_varlen.
+// Replaces the vLLM flash prefill the reference delegates to. Numerics oracles:
+// ops/torch_ref.flash_prefill_varlen and context_attention_varlen.
 #include "mfma_attention.h"
 
 namespace {
