@@ -308,6 +308,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
 
   for (int t = t_lo; t < t_hi; ++t) {
     const int buf = (t - t_lo) & 1;
+    // The barrier publishes tile t, and does not wait for this wave's LDS-direct
+    // loads of it. The wait that the compiler puts ahead of the LDS reads is on
+    // the path of a wave that computes; one without queries here has none.
+    if constexpr (DMA) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (t + 1 < t_hi) {
       stage(t + 1, page, buf ^ 1);

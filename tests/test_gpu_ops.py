@@ -399,6 +399,45 @@ class TestPrefillAttention:
         err = (out.float().cpu() - ref).norm() / ref.norm()
         assert err < 2 * 2 ** -9, float(err)
 
+    @pytest.mark.parametrize("H,Hkv,causal", [(16, 16, False), (32, 16, True)])
+    def test_prefill_idle_waves(self, dev, H, Hkv, causal):
+        """Last blocks in which some waves have no queries and only bring key
+        rows, over K and V larger than the caches (so that loads are late) and
+        between sequences of NaN (so that a row that is read before it has
+        arrived shows)."""
+        import kserve_amd_C
+
+        D = 128
+        g = torch.Generator().manual_seed(H)
+        lens = torch.randint(129, 225, (260,), generator=g).tolist()
+        lens[8::52] = [1000 + n for n in (1, 7, 16, 30, 31)]  # even places
+        T = sum(lens)
+        assert T * Hkv * D * 4 > 320 << 20  # K and V against 256 MB of cache
+        cu = [0] + torch.tensor(lens).cumsum(0).tolist()
+        q = torch.randn(T, H, D, device=dev).to(torch.bfloat16)
+        k, v = (torch.randn(T, Hkv, D, device=dev).to(torch.bfloat16) for _ in "kv")
+        for i in range(1, len(lens), 2):
+            k[cu[i] : cu[i + 1]] = v[cu[i] : cu[i + 1]] = float("nan")
+        out = torch.empty_like(q)
+        kserve_amd_C.flash_prefill_varlen(
+            out, q, k, v, torch.tensor(cu, dtype=torch.int32, device=dev), max(lens),
+            D ** -0.5, causal, 0,
+        )
+        diff = total = 0.0
+        for i in range(0, len(lens), 2):
+            rows = slice(cu[i], cu[i + 1])
+            heads = [x[rows].float().transpose(0, 1).contiguous() for x in (q, k, v)]
+            kk, vv = (x.repeat_interleave(H // Hkv, 0) for x in heads[1:])
+            s = torch.matmul(heads[0], kk.transpose(1, 2).contiguous()) * D ** -0.5
+            if causal:
+                s += torch.full_like(s[0], float("-inf")).triu(1)
+            ref = torch.matmul(s.softmax(-1), vv).transpose(0, 1)
+            diff += (out[rows].float() - ref).square().sum()
+            total += ref.square().sum()
+        # weights and output are each rounded to bf16: 2^-9 relative twice
+        err = float(diff / total) ** 0.5
+        assert err < 2 * 2 ** -9, err
+
     @pytest.mark.parametrize("fp8", [False, True])
     @pytest.mark.parametrize("window", [0, 50])
     @pytest.mark.parametrize("H,Hkv", [(4, 1), (6, 3), (2, 2), (8, 1)])
