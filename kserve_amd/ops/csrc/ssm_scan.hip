@@ -755,7 +755,22 @@ __global__ void __launch_bounds__(CT) ssd_chunk_kernel(
       }
       f32x4s z = (acc[0] + acc[1]) + (acc[2] + acc[3]);
       const f32x4s e4 = *reinterpret_cast<const f32x4s*>(grow + tb * 16 + g * 4);
-      z += (own + part[wave ^ 4][k][lane]) * e4;
+      const f32x4s past = (own + part[wave ^ 4][k][lane]) * e4;
+      z += past;
+      // The products above take later tokens of the tile with weight 0, which
+      // is no 0 if their x is infinite or NaN: such sums are formed again, from
+      // the tokens up to each row's own only.
+      const float size = fabsf(z[0]) + fabsf(z[1]) + fabsf(z[2]) + fabsf(z[3]);
+      if (__any(!(size < INFINITY))) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int tk = tb * 16 + g * 4 + r;
+          float sum = 0.f;
+          for (int sk = 0; sk <= tk; ++sk)
+            sum = fmaf(Ms[tk * XS + sk], Xs[sk * XS + pw * 16 + col], sum);
+          z[r] = sum + past[r];
+        }
+      }
       if (p < P) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {

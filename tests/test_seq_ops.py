@@ -372,6 +372,36 @@ class TestScan:
             # fp32 sums of at most 130 + 128 terms against the largest output
             close(torch.cat(g), w, be, f32_tol=5e-6, bf16_tol=5e-6)
 
+    @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+    def test_bad_inputs_stay_behind_them(self, be, bad):
+        """An infinity or a NaN in one column at one token reaches that column
+        from that token on, no earlier token and no other column."""
+        H, G, P, N, T = 2, 1, 64, 64, 130
+        inner = H * P
+        xbc = rnd(T, inner + 2 * N, seed=45, scale=0.7)
+        dt_raw = rnd(T, H, seed=46, dtype=be[1])
+        dt_bias, a_log, d_skip = rnd(H, seed=47) - 1.0, rnd(H, seed=48), rnd(H, seed=49)
+        want = O.ssd(
+            xbc[:, :inner].double().reshape(T, H, P),
+            xbc[:, inner : inner + N].double().reshape(T, G, N),
+            xbc[:, inner + N :].double().reshape(T, G, N),
+            O.softplus(dt_raw.double() + dt_bias.double()), a_log.double(),
+            d_skip.double(), G,
+        ).reshape(T, inner)
+        at = {3: 20, 40: 63, 64: 64, 100: 127}  # column: token
+        for c, t in at.items():
+            xbc[t, c] = bad
+        state = torch.zeros(2, H, P, N, device=be[0])
+        cu, _, pos = layout([T], [0])
+        got = ops.ssd_scan(
+            f32(xbc, be), act(dt_raw, be), f32(dt_bias, be), f32(a_log, be),
+            f32(d_skip, be), state, i64(pos, be), i32(cu, be), i32([1], be), G,
+        ).cpu()
+        for c, t in at.items():
+            assert not torch.isfinite(got[t:, c]).any()
+            got[t:, c] = want[t:, c].float()
+        close(got, want, be, f32_tol=5e-6, bf16_tol=5e-6)
+
     def test_large_step_sizes_are_not_clamped(self, be):
         """softplus of a large argument is the argument itself."""
         H, P, N, T = 1, 4, 8, 3
