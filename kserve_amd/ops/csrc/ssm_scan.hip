@@ -24,6 +24,7 @@
 //    tiles x heads x sequences, so decode batches fill the chip).
 #include "dtype_io.h"
 
+#include <float.h>
 #include <type_traits>
 
 namespace {
@@ -580,7 +581,10 @@ __global__ void __launch_bounds__(CT) ssd_chunk_kernel(
   const int grp = h / (heads / groups);
   const int inner = heads * P;
   const int channels = inner + 2 * groups * N;
-  const float A = -expf(a_log[h]);
+  // finite where exp leaves the range: differences of infinite running sums
+  // would be NaN where the decay is 0
+  float A = -expf(a_log[h]);
+  if (A < -FLT_MAX) A = -FLT_MAX;
   const float bias = dt_bias[h];
   const float Dh = d_skip[h];
   const bool fresh = positions[first] == 0;

@@ -402,6 +402,28 @@ class TestScan:
             got[t:, c] = want[t:, c].float()
         close(got, want, be, f32_tol=5e-6, bf16_tol=5e-6)
 
+    @pytest.mark.parametrize("T", [3, 70])
+    def test_decay_past_the_range(self, be, T):
+        """exp(a_log) past the largest fp32 number: nothing is carried on."""
+        H, P, N = 2, 4, 8
+        xbc = rnd(T, H * P + 2 * N, seed=65)
+        dt_raw = rnd(T, H, seed=66)
+        a_log = torch.tensor([90.0, 0.0])
+        state = torch.zeros(2, H, P, N, device=be[0])
+        cu, _, pos = layout([T], [0])
+        got = ops.ssd_scan(
+            f32(xbc, be), act(dt_raw, be), f32(torch.zeros(H), be), f32(a_log, be),
+            f32(torch.ones(H), be), state, i64(pos, be), i32(cu, be), i32([1], be), 1,
+        )
+        want = O.ssd(
+            xbc[:, : H * P].double().reshape(T, H, P),
+            xbc[:, H * P : H * P + N].double().reshape(T, 1, N),
+            xbc[:, H * P + N :].double().reshape(T, 1, N),
+            O.softplus(dt_raw.to(be[1]).double()), a_log.double(),
+            torch.ones(H, dtype=F64), 1,
+        ).reshape(T, H * P)
+        close(got, want, be, f32_tol=5e-6, bf16_tol=5e-6)
+
     def test_large_step_sizes_are_not_clamped(self, be):
         """softplus of a large argument is the argument itself."""
         H, P, N, T = 1, 4, 8, 3
