@@ -46,6 +46,23 @@ __device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// Softmax weights are exp2((s pre - m) c2) with m the largest s pre. c2 > 0 is
+// the scale in powers of two, so hidden keys (MASKED) come to 0; a scale too
+// close to 0 for that goes into pre, as a negative one's sign does.
+struct ScoreScale {
+  float c2, pre = 1.f;
+  __device__ __forceinline__ explicit ScoreScale(float scale) : c2(scale * LOG2E) {
+    if (c2 < 0.f) {
+      pre = -1.f;
+      c2 = -c2;
+    }
+    if (c2 < 1e-30f) {
+      pre *= c2;
+      c2 = 1.f;
+    }
+  }
+};
+
 // x as the sum of three bf16 numbers, exactly
 struct Split3 {
   __bf16 hi, mid, lo;
@@ -292,9 +309,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
                (((4 * b + ((lane >> 4) & 1) * 2 + ((ti & 3) >> 1)) ^ v_swz<D>(vrow)) * 8) +
                (ti & 1) * 4;
 
-  float c2 = p.scale * 1.44269504088896340736f;
-  const bool flip = c2 < 0.f;
-  c2 = fabsf(c2);
+  const ScoreScale sc2(p.scale);
+  const float c2 = sc2.c2;
   float m = NO_MAX, l = 0.f;
   f32x16_t o[DB];
 #pragma unroll
@@ -343,9 +359,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
         }
         if constexpr (PARTS == 3) s[kb] += rest;
       }
-      if (flip) {
+      if (sc2.pre != 1.f) {
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) s[kb] = -s[kb];
+        for (int kb = 0; kb < NKB; ++kb) s[kb] *= sc2.pre;
       }
       // register r of block kb: key 32 kb + (r & 3) + 8 (r / 4) + 4 half
       if (t0 + KT > len || (CAUSAL && t0 + KT - 1 > pos_lo) ||
@@ -685,9 +701,8 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
     vaddr[b] = ROWS * D + vrow * D +
                ((2 * b + ((col & 3) >> 1)) ^ v_swz<D>(vrow)) * 8 + (col & 1) * 4;
 
-  float c2 = p.scale * 1.44269504088896340736f;
-  const bool flip = c2 < 0.f;
-  c2 = fabsf(c2);
+  const ScoreScale sc2(p.scale);
+  const float c2 = sc2.c2;
   const int key_lo = low_of(ctx - 1, p.window, p.x.chunk);  // first visible key
   float m = NO_MAX, l = 0.f;
   f32x4_t o[DB];
@@ -712,9 +727,9 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
       }
       if constexpr (PARTS == 3) sc[h] += rest;
     }
-    if (flip) {
-      sc[0] = -sc[0];
-      sc[1] = -sc[1];
+    if (sc2.pre != 1.f) {
+      sc[0] *= sc2.pre;
+      sc[1] *= sc2.pre;
     }
     const int key0 = (rg.first + 2 * n) * PAGE;
     if (key0 + ROWS > ctx || key0 < key_lo) {

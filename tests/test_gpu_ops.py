@@ -438,6 +438,54 @@ class TestPrefillAttention:
         err = float(diff / total) ** 0.5
         assert err < 2 * 2 ** -9, err
 
+    @pytest.mark.parametrize("scale", [0.0, 1e-38, -1e-38])
+    def test_attention_vanishing_scale(self, dev, scale):
+        """Scores that all round to the same weight: hidden keys stay hidden."""
+        import kserve_amd_C
+        from kserve_amd import ops
+
+        H, Hkv, D, T, ctx = 4, 2, 128, 90, 100
+        torch.manual_seed(3)
+        q = torch.randn(T, H, D, device=dev).to(torch.bfloat16)
+        k, v = (torch.randn(T, Hkv, D, device=dev).to(torch.bfloat16) for _ in "kv")
+        cu = torch.tensor([0, T], dtype=torch.int32)
+        out = torch.empty_like(q)
+        kserve_amd_C.flash_prefill_varlen(out, q, k, v, cu.to(dev), T, scale, True, 20)
+        ref = torch_ref.flash_prefill_varlen(
+            q.float().cpu(), k.float().cpu(), v.float().cpu(), cu, scale,
+            causal=True, window=20,
+        )
+        # weights and output are each rounded to bf16: 2^-9 relative twice
+        err = (out.float().cpu() - ref).norm() / ref.norm()
+        assert err < 2 * 2 ** -9, float(err)
+
+        pages = [torch.randn(8, Hkv, 16, D, device=dev).to(torch.bfloat16) for _ in "kv"]
+        bt = torch.tensor([[3, 1, 4, 0, 5, 2, 6]], dtype=torch.int32)
+        ctx_t = torch.tensor([ctx], dtype=torch.int32)
+        for rows in (1, 5):
+            cu = torch.tensor([0, rows], dtype=torch.int32)
+            host = (x.float().cpu() for x in (q[:rows], *pages))
+            ref = torch_ref.context_attention_varlen(
+                *host, bt, cu, ctx_t, scale, window=20
+            )
+            if rows == 1:
+                got = ops.paged_attention_decode(
+                    q[:rows], *pages, bt.to(dev), ctx_t.to(dev), scale, window=20
+                )
+            else:
+                got = ops.context_attention_varlen(
+                    q[:rows], *pages, bt.to(dev), cu.to(dev), ctx_t.to(dev), rows,
+                    scale, window=20,
+                )
+            err = (got.float().cpu() - ref).norm() / ref.norm()
+            assert err < 2 * 2 ** -9, (rows, float(err))
+            got = ops.ctx_attention_f32(
+                q[:rows].float().reshape(rows, -1), *pages, bt.to(dev), cu.to(dev),
+                ctx_t.to(dev), scale, rows, H, window=20,
+            )
+            err = (got.cpu() - ref.reshape(rows, -1)).norm() / ref.norm()
+            assert err < 1e-6, (rows, float(err))
+
     @pytest.mark.parametrize("fp8", [False, True])
     @pytest.mark.parametrize("window", [0, 50])
     @pytest.mark.parametrize("H,Hkv", [(4, 1), (6, 3), (2, 2), (8, 1)])
