@@ -111,6 +111,7 @@ class SSDMixer(nn.Module):
         xbc = ops.causal_conv_silu(
             xbc_raw, self.conv_w, self.conv_b, cache.conv, positions,
             meta.seq_of_token, meta.cu_seqlens, meta.state_slots,
+            longest=meta.max_seqlen,
         )
         y = ops.ssd_scan(
             xbc, dt_raw, self.dt_bias, self.a_log, self.d_skip, cache.ssm,
@@ -898,6 +899,7 @@ class GatedDeltaMixer(nn.Module):
             qkv = ops.causal_conv_silu(
                 proj[:, :cc], self.conv_w, None, cache.conv, positions,
                 meta.seq_of_token, meta.cu_seqlens, meta.state_slots,
+                longest=meta.max_seqlen,
             )
         else:
             x = proj[:, :cc].float() * self.conv_w[:, 0]
@@ -1161,6 +1163,7 @@ class DifferentialAttention(nn.Module):
             x = ops.causal_conv_silu(
                 x, self.conv_w, None, cache.conv, positions, meta.seq_of_token,
                 meta.cu_seqlens, meta.state_slots, silu=False,
+                longest=meta.max_seqlen,
             )
         elif s.conv:
             x = x.float() * self.conv_w[:, 0]
@@ -1365,6 +1368,7 @@ class ChannelDeltaMixer(nn.Module):
             qkv = ops.causal_conv_silu(
                 proj[:, : self.low_at], self.conv_w, None, cache.conv, positions,
                 meta.seq_of_token, meta.cu_seqlens, meta.state_slots,
+                longest=meta.max_seqlen,
             )
         else:
             x = proj[:, : self.low_at].float() * self.conv_w[:, 0]

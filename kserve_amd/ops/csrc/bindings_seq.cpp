@@ -19,7 +19,7 @@ hipError_t ks_gated_group_rms_norm(void*, const void*, const void*, long,
 hipError_t ks_causal_conv_silu(void*, const void*, long, const void*,
                                const void*, void*, const void*, const void*,
                                const void*, const void*, int, int, int, int,
-                               int, int, hipStream_t);
+                               int, int, int, hipStream_t);
 hipError_t ks_ssd_scan(void*, const void*, const void*, long, int, const void*,
                        const void*, const void*, void*, const void*,
                        const void*, const void*, int, int, int, int, int, int,
@@ -277,7 +277,8 @@ void causal_conv_silu(at::Tensor& out, at::Tensor& in, at::Tensor& w,
                       const c10::optional<at::Tensor>& bias_opt,
                       at::Tensor& conv_state,
                       at::Tensor& positions, at::Tensor& seq_of_token,
-                      at::Tensor& cu_seqlens, at::Tensor& slots, bool silu) {
+                      at::Tensor& cu_seqlens, at::Tensor& slots, bool silu,
+                      bool whole_portions) {
   CHECK_F32(out);
   CHECK_F32(w);
   const void* bias_ptr = nullptr;
@@ -310,7 +311,8 @@ void causal_conv_silu(at::Tensor& out, at::Tensor& in, at::Tensor& w,
                                 conv_state.data_ptr(), positions.data_ptr(),
                                 seq_of_token.data_ptr(), cu_seqlens.data_ptr(),
                                 slots.data_ptr(), tokens, num_seqs, channels,
-                                taps, silu ? 1 : 0, f32, current_stream()),
+                                taps, silu ? 1 : 0, f32, whole_portions ? 1 : 0,
+                                current_stream()),
             "causal_conv_silu");
 }
 

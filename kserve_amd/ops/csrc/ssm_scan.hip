@@ -805,7 +805,8 @@ extern "C" hipError_t ks_causal_conv_silu(
     void* out, const void* in, long in_stride, const void* w, const void* bias,
     void* conv_state, const void* positions, const void* seq_of_token,
     const void* cu_seqlens, const void* slots, int tokens, int num_seqs,
-    int channels, int taps, int silu, int is_f32, hipStream_t stream) {
+    int channels, int taps, int silu, int is_f32, int whole_portions,
+    hipStream_t stream) {
   if (tokens == 0) return hipSuccess;
   if (taps < 1 || taps > MAX_TAPS) return hipErrorInvalidValue;
   dim3 grid(cdiv(channels, 256), tokens);
@@ -822,9 +823,7 @@ extern "C" hipError_t ks_causal_conv_silu(
   (float*)out, (const TT*)in, in_stride, (const float*)w, (const float*)bias, \
       (const TT*)conv_state, (const long*)positions,                          \
       (const int*)seq_of_token, (const int*)cu_seqlens, (const int*)slots
-  // whole portions per block up to four tokens a sequence (a walk of n tokens
-  // is n loads in a row; above, tokens in parallel are worth a second launch)
-  if (vec && tokens <= 4L * num_seqs) {
+  if (vec && whole_portions) {
     const dim3 grid_s(cdiv(channels / 4, 256), num_seqs);
 #define CONV_SEQ_K(TT, K)                                                     \
   hipLaunchKernelGGL((causal_conv_silu_seq_kernel<TT, K>), grid_s, dim3(256), \

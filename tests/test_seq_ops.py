@@ -252,6 +252,26 @@ class TestCausalConv:
             assert torch.equal(dev_state.cpu()[used], ref_state[used])
 
 
+    @pytest.mark.parametrize("taps", [2, 3, 4])
+    @pytest.mark.parametrize("lens", [[1] * 5, [1, 0, 4, 7], [4, 4], [32] + [0, 1] * 6])
+    @pytest.mark.parametrize("bias", [False, True])
+    def test_portions_with_longest_known(self, be, taps, lens, bias, monkeypatch):
+        """The same in one launch, a block per portion."""
+        conv = ops.causal_conv_silu
+        assert ops._conv_whole_portions(sum(lens), len(lens), max(lens))
+        monkeypatch.setattr(
+            ops, "causal_conv_silu", lambda *a: conv(*a, longest=max(lens))
+        )
+        self.test_portions_of_every_route(be, taps, lens, bias)
+
+    def test_one_long_portion_is_not_walked(self):
+        """127 decode tokens beside a prompt portion: the average says decode."""
+        assert ops._conv_whole_portions(128, 128, 1)
+        assert not ops._conv_whole_portions(512, 128, 385)
+        assert not ops._conv_whole_portions(191, 128, 64)
+        assert not ops._conv_whole_portions(128, 128, 0)  # not known
+
+
 class TestScan:
     @pytest.mark.parametrize(
         "H,G,P,N",
