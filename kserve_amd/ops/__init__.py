@@ -650,10 +650,11 @@ def gated_group_rms_norm(
 def _conv_whole_portions(tokens: int, seqs: int, longest: int) -> bool:
     """Whether a block walks the whole portion of a sequence and leaves its conv
     state, in one launch: 0.5 us per token of the longest portion, against two
-    launches over blocks of 16 tokens (MI355X, 6144 channels, us, one launch /
-    two: 128 sequences of 1 token 7 / 38, of 4 8 / 28, 127 of 1 and one of 30
-    18 / 38, of 64 34 / 38, of 385 191 / 39; 7 of 1 and one of 25 14 / 20)."""
-    return (tokens <= 4 * seqs and 0 < longest <= 32) or tokens <= 4
+    launches over blocks of 4 tokens (MI355X, 6144 channels, us, one launch /
+    two: 128 sequences of 1 token 8 / 21, of 4 8 / 21, 127 of 1 and one of 16
+    12 / 21, of 30 18 / 21, of 64 34 / 21, of 385 186 / 23; 7 of 1 and one of 16
+    10 / 11, of 26 15 / 11; 2048 channels, 127 of 1 and one of 30 17 / 14)."""
+    return (tokens <= 4 * seqs and 0 < longest <= 16) or tokens <= 4
 
 
 def causal_conv_silu(

@@ -100,11 +100,15 @@ __device__ __forceinline__ void load4<float>(const float* p, float* v) {
   for (int i = 0; i < 4; ++i) v[i] = x[i];
 }
 
-constexpr int CONV_TT = 16;  // tokens per block of the vector kernel
+constexpr int CONV_TT = 4;  // tokens per block of the vector kernel
 
 // The last TAPS - 1 inputs stay in registers while a lane walks its tokens, so
 // a token costs one load. Bound by memory (bf16 in, fp32 out): 8000 tokens of
-// 6144 channels take 61 us = 4.8 TB/s, 93 us when every tap was loaded.
+// 6144 channels take 61 us = 4.8 TB/s, 93 us when every tap was loaded. Four
+// tokens a block: the loads of a walk are one after the other, and short
+// portions start it anew (with the state update, us, blocks of 1 / 4 / 16
+// tokens, 6144 channels: 8000 tokens 113 / 72 / 73, 500 14 / 11 / 15, 127
+// sequences of 1 and one of 385 23 / 23 / 39; 2048 channels 11 / 14 / 31).
 template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void causal_conv_silu_vec4_kernel(
     float* __restrict__ out, const T* __restrict__ in, long in_stride,
@@ -164,8 +168,8 @@ __global__ __launch_bounds__(256) void causal_conv_silu_vec4_kernel(
 
 // A block walks the whole portion of one sequence and leaves its conv state:
 // one launch where the portions are short (decode steps), with the state read
-// once. 128 sequences of one token, 6144 channels: 6.4 us, 21 + 14 for the
-// kernel above (before its window) and the state update.
+// once. 128 sequences of one token, 6144 channels: 7.6 us, 21 for the kernel
+// above and the state update.
 template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void causal_conv_silu_seq_kernel(
     float* __restrict__ out, const T* __restrict__ in, long in_stride,

@@ -225,7 +225,7 @@ class TestCausalConv:
     )
     @pytest.mark.parametrize("bias", [False, True])
     def test_portions_of_every_route(self, be, taps, lens, bias):
-        """Whole portions per block, tokens in blocks of 16 and the edges
+        """Whole portions per block, tokens in blocks of 4 and the edges
         between them; outputs and the state left, from a first portion (state
         ignored) and a second one."""
         C = 1028
@@ -253,7 +253,7 @@ class TestCausalConv:
 
 
     @pytest.mark.parametrize("taps", [2, 3, 4])
-    @pytest.mark.parametrize("lens", [[1] * 5, [1, 0, 4, 7], [4, 4], [32] + [0, 1] * 6])
+    @pytest.mark.parametrize("lens", [[1] * 5, [1, 0, 4, 7], [4, 4], [16] + [0, 1] * 6])
     @pytest.mark.parametrize("bias", [False, True])
     def test_portions_with_longest_known(self, be, taps, lens, bias, monkeypatch):
         """The same in one launch, a block per portion."""
@@ -269,6 +269,7 @@ class TestCausalConv:
         assert ops._conv_whole_portions(128, 128, 1)
         assert not ops._conv_whole_portions(512, 128, 385)
         assert not ops._conv_whole_portions(191, 128, 64)
+        assert not ops._conv_whole_portions(33, 8, 26)
         assert not ops._conv_whole_portions(128, 128, 0)  # not known
 
 
