@@ -271,6 +271,13 @@ void embed_layer_norm(at::Tensor& out, at::Tensor& word, at::Tensor& pos_table,
                   pos_table.size(1) == hidden && type_table.size(1) == hidden &&
                   weight.numel() == hidden && bias.numel() == hidden,
               "embed_layer_norm: shape mismatch");
+  const c10::Device dev = word.device();
+  TORCH_CHECK(out.device() == dev && pos_table.device() == dev &&
+                  type_table.device() == dev && ids.device() == dev &&
+                  cu_seqlens.device() == dev && weight.device() == dev &&
+                  bias.device() == dev && (!types || types->device() == dev),
+              "operands on different devices");
+  const c10::DeviceGuard guard(dev);
   check_hip(ks_embed_layer_norm(
                 out.data_ptr(), word.data_ptr(), pos_table.data_ptr(),
                 type_table.data_ptr(), ids.data_ptr(),
@@ -412,6 +419,11 @@ static void rope_cache_run(at::Tensor& q, at::Tensor& k, at::Tensor& v,
                   positions.numel() == T && positions.is_contiguous() &&
                   cos_sin.size(-1) == D,
               "rope_and_cache: shape mismatch");
+  const c10::Device dev = q.device();
+  TORCH_CHECK(k.device() == dev && v.device() == dev && positions.device() == dev &&
+                  cos_sin.device() == dev,
+              "operands on different devices");
+  const c10::DeviceGuard guard(dev);
   const bool cached = k_cache.numel() > 0;
   bool fp8 = false;
   int block = 1;
@@ -421,6 +433,9 @@ static void rope_cache_run(at::Tensor& q, at::Tensor& k, at::Tensor& v,
     TORCH_CHECK(slot_mapping.scalar_type() == at::kInt && slot_mapping.is_contiguous() &&
                     slot_mapping.numel() >= T,
                 "slot_mapping int32");
+    TORCH_CHECK(k_cache.device() == dev && v_cache.device() == dev &&
+                    slot_mapping.device() == dev,
+                "pages and slots on another device");
     TORCH_CHECK(k_cache.dim() == 4 && k_cache.size(1) == Hk && k_cache.size(3) == D &&
                     v_cache.sizes() == k_cache.sizes() &&
                     v_cache.scalar_type() == k_cache.scalar_type(),
@@ -454,6 +469,8 @@ void skinny_rope_cache(at::Tensor& q, at::Tensor& k, at::Tensor& v, at::Tensor& 
   TORCH_CHECK(x.size(0) == q.size(0) &&
                   w.size(0) == (q.size(1) + k.size(1) + v.size(1)) * q.size(2),
               "shape mismatch");
+  TORCH_CHECK(x.device() == q.device(), "operands on different devices");
+  const c10::DeviceGuard guard(x.device());
   const at::Tensor part = skinny_sums(x, w);
   rope_cache_run(q, k, v, &part, positions, cos_sin, k_cache, v_cache,
                  slot_mapping);

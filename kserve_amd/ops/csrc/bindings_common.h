@@ -85,12 +85,13 @@ void topk_topp_sample(at::Tensor& out, at::Tensor& logits,
             "topk_topp_sample");
 }
 
+// operands of a decode step: on device `dev`
 #define CHECK_STEP(t, kind, n)                                             \
-  TORCH_CHECK((t).is_cuda() && (t).scalar_type() == kind && (t).dim() == 1 && \
+  TORCH_CHECK((t).device() == dev && (t).scalar_type() == kind && (t).dim() == 1 && \
                   (t).is_contiguous() && (t).numel() >= (n),                  \
               #t ": a dense vector of the rows expected")
 #define CHECK_TABLES(t, n)                                                   \
-  TORCH_CHECK((t).is_cuda() && (t).scalar_type() == at::kInt && (t).dim() == 2 && \
+  TORCH_CHECK((t).device() == dev && (t).scalar_type() == at::kInt && (t).dim() == 2 && \
                   (t).size(0) >= (n) && ((t).size(1) < 2 || (t).stride(1) == 1),  \
               #t ": int32 rows expected")
 
@@ -101,6 +102,8 @@ void unpack_decode_rows(at::Tensor& staged, int64_t width, at::Tensor& ids,
   TORCH_CHECK(staged.is_cuda() && staged.scalar_type() == at::kInt &&
                   staged.dim() == 2 && staged.is_contiguous(),
               "staged: int32 rows");
+  const c10::Device dev = staged.device();
+  const c10::DeviceGuard guard(dev);
   const int64_t rows = staged.size(0);
   CHECK_STEP(ids, at::kLong, rows);
   CHECK_STEP(positions, at::kLong, rows);
@@ -123,6 +126,9 @@ void advance_decode(at::Tensor& greedy, const c10::optional<at::Tensor>& random,
                     at::Tensor& positions, at::Tensor& context_lens,
                     at::Tensor& slots, const c10::optional<at::Tensor>& seeds,
                     int64_t seed_step, at::Tensor& tables, int64_t block) {
+  TORCH_CHECK(greedy.is_cuda(), "greedy: a GPU tensor expected");
+  const c10::Device dev = greedy.device();
+  const c10::DeviceGuard guard(dev);
   const int64_t rows = greedy.numel();
   CHECK_STEP(greedy, at::kLong, rows);
   CHECK_STEP(ids, at::kLong, rows);

@@ -950,6 +950,51 @@ class TestFusedProjections:
         torch.testing.assert_close(out.double(), norm, rtol=2.0 ** -6, atol=2.0 ** -6)
 
 
+class TestOperandDevices:
+    """The entry points that took over from guarded torch calls."""
+
+    def _calls(self, dev):
+        import kserve_amd_C as C
+
+        def z(*shape, dtype=torch.bfloat16, at=dev):
+            return torch.zeros(*shape, dtype=dtype, device=at)
+
+        qkv = [z(2, h, 64) for h in (4, 1, 1)]
+        pages, slots = [z(1, 1, 16, 64) for _ in "kv"], z(2, dtype=torch.int32)
+        pos, cs = z(2, dtype=torch.int64), z(8, 64, dtype=torch.float32)
+        x, w = z(2, 64), z(6 * 64, 64)
+        ids, cu = z(2, dtype=torch.int64), torch.tensor([0, 2], dtype=torch.int32, device=dev)
+        tables, vec = z(2, 1, dtype=torch.int32), z(64)
+        ints = [z(2, dtype=torch.int32) for _ in range(3)]
+        staged = z(2, 10, dtype=torch.int32)
+        yield C.rope_and_cache, [pos, *qkv, cs, *pages, slots]
+        yield C.skinny_rope_cache, [*qkv, x, w, pos, cs, *pages, slots]
+        yield C.embed_layer_norm, [
+            z(2, 64), z(4, 64), z(4, 64), z(2, 64), ids, None, cu, vec, vec, 1e-5
+        ]
+        yield C.unpack_decode_rows, [staged, 1, ids, pos, *ints, tables]
+        yield C.advance_decode, [
+            ids, None, None, None, ids.clone(), pos, ints[0], ints[1], None, 0, tables, 16
+        ]
+
+    def test_host_operands_are_refused(self, dev):
+        for call, args in self._calls(dev):
+            call(*args)
+            for i, a in enumerate(args):
+                if torch.is_tensor(a):
+                    with pytest.raises(RuntimeError):
+                        call(*args[:i], a.cpu(), *args[i + 1 :])
+
+    def test_other_current_device(self, dev):
+        if torch.cuda.device_count() < 2:
+            pytest.skip("needs two GPUs")
+        other = torch.device("cuda:1")
+        assert torch.cuda.current_device() != other.index
+        for call, args in self._calls(other):
+            call(*args)
+        torch.cuda.synchronize(other)
+
+
 class TestDecodeStep:
     """The one-launch bookkeeping of a decode step against the CPU forms."""
 
