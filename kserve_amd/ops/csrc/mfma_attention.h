@@ -46,9 +46,10 @@ __device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// Softmax weights are exp2((s pre - m) c2) with m the largest s pre. c2 > 0 is
-// the scale in powers of two, so hidden keys (MASKED) come to 0; a scale too
-// close to 0 for that goes into pre, as a negative one's sign does.
+// Softmax weights are exp2((s - m) c2) with m the largest score. c2 > 0 is the
+// scale in powers of two, so hidden keys (MASKED) come to 0; the query is
+// multiplied by `pre`, which has a negative scale's sign, or the scale itself
+// where it is too close to 0 for that (the scores are all next to 0 then).
 struct ScoreScale {
   float c2, pre = 1.f;
   __device__ __forceinline__ explicit ScoreScale(float scale) : c2(scale * LOG2E) {
@@ -60,6 +61,13 @@ struct ScoreScale {
       pre *= c2;
       c2 = 1.f;
     }
+  }
+  __device__ __forceinline__ bf16x8_t apply(bf16x8_t q) const {
+    if (pre != 1.f) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = (__bf16)((float)q[j] * pre);
+    }
+    return q;
   }
 };
 
@@ -186,6 +194,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   __shared__ __attribute__((aligned(16))) short lds[2][2][TILE];  // [buffer][K, V]
 
   // ---- queries: B operands, 8 consecutive columns per lane ----
+  const ScoreScale scale(p.scale);
+  const float c2 = scale.c2;
   bf16x8_t qf[PARTS][KC];
   {
     const int qrow = min(q0 + (lane & 31), q_len - 1);
@@ -194,7 +204,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
       const short* qp = reinterpret_cast<const short*>(p.q) + at;
 #pragma unroll
       for (int c = 0; c < KC; ++c)
-        qf[0][c] = *reinterpret_cast<const bf16x8_t*>(qp + c * 16);
+        qf[0][c] = scale.apply(*reinterpret_cast<const bf16x8_t*>(qp + c * 16));
     } else {
       const float* qp = reinterpret_cast<const float*>(p.q) + at;
 #pragma unroll
@@ -204,7 +214,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
           const f32x4_t x = *reinterpret_cast<const f32x4_t*>(qp + c * 16 + j);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const Split3 w(x[e]);
+            const Split3 w(x[e] * scale.pre);
             qf[0][c][j + e] = w.hi;
             qf[1][c][j + e] = w.mid;
             qf[2][c][j + e] = w.lo;
@@ -309,8 +319,6 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
                (((4 * b + ((lane >> 4) & 1) * 2 + ((ti & 3) >> 1)) ^ v_swz<D>(vrow)) * 8) +
                (ti & 1) * 4;
 
-  const ScoreScale sc2(p.scale);
-  const float c2 = sc2.c2;
   float m = NO_MAX, l = 0.f;
   f32x16_t o[DB];
 #pragma unroll
@@ -358,10 +366,6 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
           s[kb] = mfma32(a, qf[0][c], s[kb]);
         }
         if constexpr (PARTS == 3) s[kb] += rest;
-      }
-      if (sc2.pre != 1.f) {
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) s[kb] *= sc2.pre;
       }
       // register r of block kb: key 32 kb + (r & 3) + 8 (r / 4) + 4 half
       if (t0 + KT > len || (CAUSAL && t0 + KT - 1 > pos_lo) ||
@@ -552,8 +556,11 @@ __device__ __forceinline__ float final_factor(const DecodeArgs& p, long tok, int
   }
 }
 
+// E4M3 pages: two waves per SIMD at least, or the compiler keeps the output in
+// accumulation registers and copies it out and back for every rescale (96 x
+// 3000 +- 60%: 114 us, 108 so; bf16 pages 353 and 360 the other way round)
 template <int D, int NW, int SRC, bool WIDE, int PARTS = 1>  // WIDE: groups of 6 to 8
-__global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
+__global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_attention_kernel(
     const DecodeArgs p) {
   constexpr int KC = D / 32;           // contraction chunks of K Q^T
   constexpr int DB = D / 16;           // 16-column blocks of the output
@@ -581,6 +588,8 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
   __shared__ __attribute__((aligned(16))) short lds[NW][RING][STAGE];
   static_assert(RING * STAGE * 2 >= 8 * (D + 4) * 4 + 64, "merge area");
 
+  const ScoreScale scale(p.scale);
+  const float c2 = scale.c2;
   bf16x8_t qf[PARTS][KC];
   {
     const long at = (long)tok * p.sq + (long)(kvh * G + col % G) * D + g * 8;
@@ -591,7 +600,7 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
         short8_t x = *reinterpret_cast<const short8_t*>(qp + c * 32);
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = used ? x[j] : 0;
-        qf[0][c] = __builtin_bit_cast(bf16x8_t, x);
+        qf[0][c] = scale.apply(__builtin_bit_cast(bf16x8_t, x));
       }
     } else {
       const float* qp = reinterpret_cast<const float*>(p.q) + at;
@@ -602,7 +611,7 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
           const f32x4_t x = *reinterpret_cast<const f32x4_t*>(qp + c * 32 + j);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const Split3 w(used ? x[e] : 0.f);
+            const Split3 w(used ? x[e] * scale.pre : 0.f);
             qf[0][c][j + e] = w.hi;
             qf[1][c][j + e] = w.mid;
             qf[2][c][j + e] = w.lo;
@@ -701,8 +710,6 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
     vaddr[b] = ROWS * D + vrow * D +
                ((2 * b + ((col & 3) >> 1)) ^ v_swz<D>(vrow)) * 8 + (col & 1) * 4;
 
-  const ScoreScale sc2(p.scale);
-  const float c2 = sc2.c2;
   const int key_lo = low_of(ctx - 1, p.window, p.x.chunk);  // first visible key
   float m = NO_MAX, l = 0.f;
   f32x4_t o[DB];
@@ -726,10 +733,6 @@ __global__ __launch_bounds__(NW * 64) void paged_attention_kernel(
         sc[h] = mfma16x16x32(a, qf[0][c], sc[h]);
       }
       if constexpr (PARTS == 3) sc[h] += rest;
-    }
-    if (sc2.pre != 1.f) {
-      sc[0] *= sc2.pre;
-      sc[1] *= sc2.pre;
     }
     const int key0 = (rg.first + 2 * n) * PAGE;
     if (key0 + ROWS > ctx || key0 < key_lo) {
