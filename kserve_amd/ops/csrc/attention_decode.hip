@@ -6,9 +6,14 @@
 //
 // A block takes the query heads of one KV head of one sequence (or of one of
 // several splits of its context) and its waves take pairs of pages in turn,
-// each wave in LDS of its own: bf16 pages arrive by LDS-direct loads, two
-// pairs (32 KB) in flight per wave without a register or a barrier; E4M3 pages
-// pass through registers and are widened (exactly) on the way.
+// each wave in LDS of its own, without a barrier: a pair's rows pass through
+// registers, and the next pair's loads are under way while one is multiplied.
+// E4M3 pages are widened (exactly) on the way. LDS-direct loads into a ring of
+// two pairs were slower, the more so the shorter the contexts (500 sequences of
+// 100, 8 heads: 60 us, 39 here; 24 of 900 29 / 22; 256 of 2048 328 / 332): the
+// ring takes twice the LDS, so half the blocks were resident, and the compiler
+// waits for all LDS-direct loads before the transposing LDS reads, so it never
+// held more than one pair.
 //
 // The tiles are transposed: S^T = K Q^T on v_mfma_f32_16x16x32_bf16 puts one
 // query head per lane column, and the score registers of a page pair are
@@ -21,14 +26,15 @@
 // side in the 16 columns of one product (the query is repeated); six to eight
 // heads put two parts there and the third through a second product.
 //
-// Measured (32 query and 8 KV heads of 128; before it a wave per query head
-// walked the pages with vector dot products): 256 sequences of 2048 +- 60%
-// tokens 739 -> 358 us (6.0 TB/s of pages), all of 2048 609 -> 330 us (6.5);
-// 512 of 576 341 -> 198 us; E4M3, 96 of 3000 385 -> 119 us; one of 560 9.4 ->
-// 7.6 us, of 7000 45 -> 12 us; 64 / 8 heads, 64 of 600 71 -> 29 us. The page
-// loads are non-temporal: a step's pages pass once and a model's do not fit
-// the caches (temporal, the first four take 392, 366, 216 and 131 us; only
-// pages still cached from the last call, 64 of 1000 alone, gain, 47 / 55).
+// Measured (32 query and 8 KV heads of 128, pages not in a cache; before it a
+// wave per query head walked the pages with vector dot products): 256 sequences
+// of 2048 +- 60% tokens 741 -> 352 us (6.2 TB/s of pages), all of 2048 606 ->
+// 332 us (6.5); 512 of 576 341 -> 189 us; E4M3, 96 of 3000 268 -> 93 us, 3000 +-
+// 60% 390 -> 108 us; one of 560 12.5 -> 9.7 us, of 7000 66 -> 14.5 us; 64 / 8
+// heads, 64 of 600 83 -> 29 us. Short contexts are bound by a block's fixed work
+// (about 5 us) and not by the pages; there E4M3 pages under one query head each
+// are slower than before (500 of 100: 24 -> 31 us, 8 heads). The page loads are
+// non-temporal: a step's pages pass once and a model's do not fit the caches.
 //
 // Splits are merged by paged_attention_reduce_kernel. Numerics oracle:
 // ops/torch_ref.paged_attention_decode.
@@ -57,15 +63,9 @@ extern "C" hipError_t ks_paged_attention_decode(
                      num_heads, num_kv_heads, group, max_blocks, q_row_stride,
                      n_splits, (float*)part_out, (float*)part_ml, window,
                      head_dim, head_dim, nullptr, Extra{}};
-  const bool aligned = (((uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
-  if (head_dim == 128) {
-    if (fp8) return launch_decode<128, PAGES_FP8>(p, num_seqs, stream);
-    if (aligned) return launch_decode<128, PAGES_DMA>(p, num_seqs, stream);
-    return launch_decode<128, PAGES_REG>(p, num_seqs, stream);
-  }
-  if (head_dim == 64 && !fp8) {
-    if (aligned) return launch_decode<64, PAGES_DMA>(p, num_seqs, stream);
-    return launch_decode<64, PAGES_REG>(p, num_seqs, stream);
-  }
+  if (head_dim == 128)
+    return fp8 ? launch_decode<128, PAGES_FP8>(p, num_seqs, stream)
+               : launch_decode<128, PAGES_REG>(p, num_seqs, stream);
+  if (head_dim == 64 && !fp8) return launch_decode<64, PAGES_REG>(p, num_seqs, stream);
   return hipErrorInvalidValue;
 }

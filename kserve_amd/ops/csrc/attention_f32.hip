@@ -999,7 +999,7 @@ hipError_t dispatch_d(const CtxArgs& a) {
 // Times (us, fp32 products -> this), heads of 128: prefill 4 x 2000, 16/4 heads
 // 1428 -> 237, 8 x 2048, 32/8 heads 5912 -> 837, windowed (1024, 16/4 heads)
 // 1675 -> 351, 500 after 1500 266 -> 106; decode 128 of 1500 +- 60%, 16/4 heads
-// 278 -> 96, 256 of 2048, 32/8 heads 987 -> 390, one of 600 23 -> 10.
+// 281 -> 78, 256 of 2048, 32/8 heads 985 -> 340, one of 600 27 -> 10.
 extern "C" int ks_ctx_attention_mfma(const void* out, const void* q,
                                      const void* k_cache, const void* v_cache,
                                      int max_q_len, int heads, int kv_heads,
@@ -1033,8 +1033,8 @@ static hipError_t ctx_attention_mfma(const CtxArgs& a) {
                        a.bt_stride, (long)a.heads * a.D, a.nsplit, ws,
                        ws ? ws + rows * a.DV : nullptr, a.window, a.D,
                        a.v_row_stride, (const int*)a.cu_q, x};
-    return a.D == 128 ? launch_decode<128, PAGES_DMA, 3>(p, a.num_seqs, a.stream)
-                      : launch_decode<64, PAGES_DMA, 3>(p, a.num_seqs, a.stream);
+    return a.D == 128 ? launch_decode<128, PAGES_REG, 3>(p, a.num_seqs, a.stream)
+                      : launch_decode<64, PAGES_REG, 3>(p, a.num_seqs, a.stream);
   }
   const int group = a.heads / a.kv_heads;
   const int hpb = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;

@@ -25,8 +25,8 @@ constexpr int PAGE = 16;
 enum Src {
   ROWS_DMA,   // flat rows, 16-byte aligned: loaded straight into LDS
   ROWS_REG,   // flat rows at any alignment: through registers
-  PAGES_DMA,  // bf16 pages of 16 tokens
-  PAGES_REG,  // bf16 pages at any alignment
+  PAGES_DMA,  // bf16 pages of 16 tokens, 16-byte aligned: straight into LDS
+  PAGES_REG,  // bf16 pages at any alignment: through registers
   PAGES_FP8,  // E4M3 pages, widened to bf16 on the way
 };
 
@@ -505,8 +505,6 @@ __device__ __forceinline__ Range page_range(int ctx, int window, int chunk,
   return r;
 }
 
-constexpr int NT_AUX = 2;  // cache policy of a non-temporal load
-
 __device__ __forceinline__ uint4 load16_nt(const char* from) {
   typedef unsigned int u4 __attribute__((ext_vector_type(4)));
   return __builtin_bit_cast(
@@ -566,7 +564,6 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
   constexpr int DB = D / 16;           // 16-column blocks of the output
   constexpr int ROWS = 2 * PAGE;       // rows of a stage (a pair of pages)
   constexpr int STAGE = 2 * ROWS * D;  // K rows, then V rows
-  constexpr int RING = SRC == PAGES_DMA ? 2 : 1;
   // elements per lane and load, loads per stage and tensor
   constexpr int EPL = SRC == PAGES_FP8 ? 16 : 8;
   constexpr int LPR = D / EPL;  // lanes per row
@@ -585,8 +582,8 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
   const int part = col / G;  // of the weights: high, middle, low
   const bool used = part < (WIDE ? 2 : 3);
 
-  __shared__ __attribute__((aligned(16))) short lds[NW][RING][STAGE];
-  static_assert(RING * STAGE * 2 >= 8 * (D + 4) * 4 + 64, "merge area");
+  __shared__ __attribute__((aligned(16))) short lds[NW][STAGE];
+  static_assert(STAGE * 2 >= 8 * (D + 4) * 4 + 64, "merge area");
 
   const ScoreScale scale(p.scale);
   const float c2 = scale.c2;
@@ -642,54 +639,36 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
            ((long)(second ? pg.b : pg.a) * p.Hkv + kvh) * PAGE * st * ES +
            (row * (int)st + chunk * EPL) * ES;
   };
-  auto load_dma = [&](int n, Pages pg, int slot) {
+  uint4 raw[2 * NI];
+  auto load = [&](int n) {
+    const Pages pg = pages_of(n);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int r = i * RPI + lrow;
-      short* dst = &lds[wave][slot][i * RPI * D];
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const unsigned int*>(
-              src(p.k_cache, p.sk, n, pg, i, lchunk ^ k_swz<D>(r))),
-          reinterpret_cast<unsigned int*>(dst), 16, 0, NT_AUX);
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const unsigned int*>(
-              src(p.v_cache, p.sv, n, pg, i, lchunk ^ v_swz<D>(r))),
-          reinterpret_cast<unsigned int*>(dst + ROWS * D), 16, 0, NT_AUX);
-    }
-  };
-  uint4 raw[SRC == PAGES_DMA ? 1 : 2 * NI];
-  auto load_reg = [&](int n, Pages pg) {
-    if constexpr (SRC != PAGES_DMA) {
-#pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        raw[2 * i] = load16_nt(src(p.k_cache, p.sk, n, pg, i, lchunk));
-        raw[2 * i + 1] = load16_nt(src(p.v_cache, p.sv, n, pg, i, lchunk));
-      }
+      raw[2 * i] = load16_nt(src(p.k_cache, p.sk, n, pg, i, lchunk));
+      raw[2 * i + 1] = load16_nt(src(p.v_cache, p.sv, n, pg, i, lchunk));
     }
   };
   auto commit = [&]() {
-    if constexpr (SRC != PAGES_DMA) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i) {
-        const int r = i * RPI + lrow;
+    for (int i = 0; i < NI; ++i) {
+      const int r = i * RPI + lrow;
 #pragma unroll
-        for (int kv = 0; kv < 2; ++kv) {
-          short* row = &lds[wave][0][kv * ROWS * D + r * D];
-          const int sw = kv ? v_swz<D>(r) : k_swz<D>(r);
-          const uint4 x = raw[2 * i + kv];
-          if constexpr (SRC == PAGES_REG) {
-            *reinterpret_cast<uint4*>(row + (lchunk ^ sw) * 8) = x;
-          } else {
-            const unsigned int w[4] = {x.x, x.y, x.z, x.w};
+      for (int kv = 0; kv < 2; ++kv) {
+        short* row = &lds[wave][kv * ROWS * D + r * D];
+        const int sw = kv ? v_swz<D>(r) : k_swz<D>(r);
+        const uint4 x = raw[2 * i + kv];
+        if constexpr (SRC == PAGES_REG) {
+          *reinterpret_cast<uint4*>(row + (lchunk ^ sw) * 8) = x;
+        } else {
+          const unsigned int w[4] = {x.x, x.y, x.z, x.w};
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              uint4 o;
-              o.x = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h], 1.0f, false));
-              o.y = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h], 1.0f, true));
-              o.z = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h + 1], 1.0f, false));
-              o.w = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h + 1], 1.0f, true));
-              *reinterpret_cast<uint4*>(row + ((2 * lchunk + h) ^ sw) * 8) = o;
-            }
+          for (int h = 0; h < 2; ++h) {
+            uint4 o;
+            o.x = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h], 1.0f, false));
+            o.y = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h], 1.0f, true));
+            o.z = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h + 1], 1.0f, false));
+            o.w = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h + 1], 1.0f, true));
+            *reinterpret_cast<uint4*>(row + ((2 * lchunk + h) ^ sw) * 8) = o;
           }
         }
       }
@@ -788,34 +767,12 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
 
   const int n_lo = split * rg.per + wave;
   const int n_hi = min((split + 1) * rg.per, rg.pairs);
-  if constexpr (SRC == PAGES_DMA) {
-    // s_waitcnt immediates (vmcnt in bits 3:0 and 15:14; no wait on the rest)
-    constexpr int NL = 2 * NI;  // loads of one stage
-    constexpr int WAIT_STAGE = (0xF << 8) | (0x7 << 4) | (NL & 0xF) | ((NL >> 4) << 14);
-    constexpr int WAIT_ALL = (0xF << 8) | (0x7 << 4);
-    if (n_lo < n_hi) load_dma(n_lo, pages_of(n_lo), 0);
-    if (n_lo + NW < n_hi) load_dma(n_lo + NW, pages_of(n_lo + NW), 1);
-    int slot = 0;
-    for (int n = n_lo; n < n_hi; n += NW, slot ^= 1) {
-      const int next = n + 2 * NW;
-      Pages pg{0, 0};
-      if (next < n_hi) pg = pages_of(next);
-      if (n + NW < n_hi) __builtin_amdgcn_s_waitcnt(WAIT_STAGE);
-      else __builtin_amdgcn_s_waitcnt(WAIT_ALL);
-      __builtin_amdgcn_sched_barrier(0);
-      asm volatile("" ::: "memory");
-      compute(n, lds[wave][slot]);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      if (next < n_hi) load_dma(next, pg, slot);
-    }
-  } else {
-    if (n_lo < n_hi) load_reg(n_lo, pages_of(n_lo));
-    for (int n = n_lo; n < n_hi; n += NW) {
-      commit();
-      if (n + NW < n_hi) load_reg(n + NW, pages_of(n + NW));
-      compute(n, lds[wave][0]);
-    }
+  if (n_lo < n_hi) load(n_lo);
+  // the next pair's loads are under way while this one is multiplied
+  for (int n = n_lo; n < n_hi; n += NW) {
+    commit();
+    if (n + NW < n_hi) load(n + NW);
+    compute(n, lds[wave]);
   }
 
   // ---- merge: the parts of the weights, then the waves ----
@@ -838,7 +795,7 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
     mm[8 + lane] = l;
   }
   __syncthreads();
-  constexpr int WF = RING * STAGE / 2;  // floats between the waves' areas
+  constexpr int WF = STAGE / 2;  // floats between the waves' areas
   const float* all = reinterpret_cast<const float*>(lds);
   for (int i = threadIdx.x; i < G * (D / 4); i += NW * 64) {
     const int h = i / (D / 4), d = i % (D / 4) * 4;
@@ -907,10 +864,11 @@ __global__ __launch_bounds__(256) void paged_attention_reduce_kernel(
   }
 }
 
-// Two waves per block: 64 KB of LDS, two blocks per compute unit, so one
-// block's first loads run under the other's last ones. (With temporal loads: 256 sequences of 819 to
-// 3277 tokens: 389 us with 2 waves, 390 with 4, 431 with 1; 64 of 400 to 1600:
-// 48.4 / 50.0 / 66.4.)
+// Two waves per block: 32 KB of LDS, five blocks per compute unit, so one
+// block's first loads run under the others' last ones (32 / 8 heads of 128, us
+// with 1 / 2 / 4 waves: 256 sequences of 2048 +- 60% 364 / 349 / 338, 64 of 1000
+// +- 60% 56 / 48 / 48, 500 of 100 37 / 38 / 46; E4M3, 96 of 3000 +- 60% 182 /
+// 122 / 115, without the launch bound above).
 constexpr int WAVES = 2;
 
 template <int D, int SRC, int PARTS = 1>
@@ -933,12 +891,13 @@ hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) 
 }
 
 // Context splits for a launch over num_seqs x num_kv_heads: none from 512
-// blocks on, which fill the chip (temporal loads here too: 64 sequences, 8 KV heads: 48.4 us unsplit,
-// 51.4 with 2 splits, 50.4 with 4; 96 of 3000, E4M3: 128 / 140 / 129), about
-// 640 blocks below that (24 sequences of 900: 30.4 us with 3 splits, 27.4 with
-// 4, 29.8 with 6; 8 of 600: 9.3 with 8, 11.9 with 16), and at most 32 (one of
-// 7000: 12.0 us with 32, 12.8 with 64, 14.7 with 16). A sequence uses as many
-// of them as it has page pairs for every wave.
+// blocks on (8 KV heads, us: 64 sequences of 1500 61.5 unsplit, 65 with 2 splits,
+// 69 with 4), about 640 blocks below that. Splits cost even contexts up to a
+// tenth there (48 of 900: 32 unsplit, 35 with 2; 24 of 900: 21 and 22 with 4) and
+// keep one long context from being what the launch waits for (40 of 500 and one
+// of 7000: 118 unsplit, 71 with 2; 24 of 1000 to 4000: 63, 45 with 4). At most 32
+// (one of 7000: 14 us with 32, 16 with 16). A sequence uses as many of them as it
+// has page pairs for every wave.
 inline int decode_splits(int num_seqs, int num_kv_heads, int max_blocks) {
   const long base = (long)num_seqs * num_kv_heads;
   if (base <= 0 || base >= 512) return 1;
