@@ -320,41 +320,57 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     """Whether the few-row kernel beats the library at [n, k] x [m, k]^T
     (MI355X, us, kernel / library, reduction of the K splits included).
 
-    Up to 48 rows it streams weights faster (k 4096, m 32000 at 1 row 48 / 60,
-    at 24 rows 50 / 60; k 14336, m 4096 at 24 rows 27 / 32; level on small
-    ones, 512 x 512 4.6 / 4.2), up to 64 rows but for the widest (m 16384
-    38 / 35). So far a row's sums do not depend on the rows beside it, and
-    small weights stay here for that. Above, it gains where the library does
-    not split K over the chip: k 14336, m 4096 at 128 rows 36 / 76, k 4096,
-    m 6144 22 / 26; and loses on small weights (2048 x 2048 15 / 11) and wide
-    ones (m 16384 44 / 38). Past 192 rows the lighter of the former turn
-    (4096 x 4096 27 / 23 at 256 rows; m 6144 33 / 40)."""
-    if m % 4:
+    Up to 48 rows it streams weights faster (k 4096, m 32000 at 1 row 49 / 61,
+    at 24 rows 50 / 60; k 14336, m 4096 at 24 rows 24 / 32; level on small
+    ones, 768 x 768 5.3 / 4.9; not everywhere on wide ones past 16 rows: k 5120,
+    m 27648 at 32 rows 57 / 53, at 48 rows 63 / 83), up to 64 rows but for the
+    widest (m 14336 28.3 / 27.5). So far a row's sums do not depend on the rows
+    beside it, and small weights stay here for that. Above, it gains where the
+    library does not split K over the chip: k 14336, m 4096 at 128 rows 35 / 76,
+    k 4096, m 6144 22 / 26, k 3072, m 6144 20 / 21; and loses on short K (k 2048,
+    m 8192 18.7 / 16.3, k 2560, m 8192 21.0 / 19.9), small weights (2048 x 2048
+    15 / 11) and wide ones (m 16384 44 / 38). Past 192 rows the lighter of the
+    former turn (4096 x 4096 27 / 23 at 256 rows; m 6144 33 / 40)."""
+    if m % 4 or n > 256:
         return False
     if n <= 48 or (n <= 64 and m <= 8192):
         return True
-    return 4096 <= m <= 10240 and k * m >= (16 if n <= 192 else 24) << 20
+    return (
+        4096 <= m <= 10240
+        and k >= 3072
+        and k * m >= (16 if n <= 192 else 24) << 20
+    )
 
 
 def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     """The same for the gate|up product with silu(gate) * up on its sums,
     against the library's product and the activation kernel (k 4096, m 14336:
-    1 row 43 / 66, 48 rows 49 / 69, 96 rows 58 / 60, 192 rows 73 / 72). A
-    block takes 32 or, above 64 rows, 64 features and K is not split, so m
-    has to fill the chip (k 4096, m 3584 24 / 21 at 64 rows); above 16384
-    features the library is level (k 8192, m 28672 at 1 row 182 / 180)."""
-    if m % 4 or m > 16384:
+    1 row 46 / 67, 48 rows 50 / 67, 64 rows 56 / 59, 96 rows 60 / 60). A block
+    takes 32 or, above 64 rows, 64 features and K is not split, so m has to fill
+    the chip (k 4096, m 3584 24 / 21 at 64 rows), the more so the longer K is (k
+    8192, m 7168 at 1 row 56 / 50, m 14336 88 / 129). Past 48 rows the block's
+    LDS reads bound it: it stays where the blocks come out even and K is not
+    longer (k 3072, m 8192 25 / 28; k 2560, m 9728 35 / 31, k 5120, m 13824
+    71 / 62, k 8192, m 14336 at 96 rows 114 / 110). Above 16384 features the
+    library is level (k 8192, m 28672 at 1 row 182 / 180)."""
+    if m % 4 or m > 16384 or n > 112:
         return False
-    return (n <= 64 and m >= 4608) or (n <= 112 and m >= 12288)
+    if k > 4096:
+        return n <= 48 and m >= 12288
+    if n > 64:
+        return m >= 12288
+    return m >= 4608 and (n <= 48 or m <= 8192 or m >= 10240)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
     """x @ weight^T (+ bias): a kernel of our own for the few rows of a decode
     batch where it is the faster one, the library otherwise."""
+    # sizes first: most calls that are not for the kernel end there
     if (
         bias is None
-        and _skinny_operands(x, weight)
+        and x.dim() == 2
         and _skinny_rows(x.shape[0], x.shape[1], weight.shape[0])
+        and _skinny_operands(x, weight)
     ):
         out = torch.empty(
             (x.shape[0], weight.shape[0]), dtype=x.dtype, device=x.device
@@ -370,9 +386,10 @@ def linear_silu_and_mul(
     """silu(gate) * up for [gate | up] = x @ weight^T (+ bias)."""
     if (
         bias is None
-        and _skinny_operands(x, weight)
+        and x.dim() == 2
         and weight.shape[0] % 2 == 0
         and _skinny_glu_rows(x.shape[0], x.shape[1], weight.shape[0] // 2)
+        and _skinny_operands(x, weight)
     ):
         out = torch.empty(
             (x.shape[0], weight.shape[0] // 2), dtype=x.dtype, device=x.device
@@ -390,9 +407,10 @@ def linear_add_rms_norm(
     in place on the GPU. Few rows: the norm's kernel adds the GEMM's splits."""
     m = weight.shape[0]
     if (
-        _skinny_operands(x, weight)
+        m <= 16384
+        and x.dim() == 2
         and _skinny_rows(x.shape[0], x.shape[1], m)
-        and m <= 16384
+        and _skinny_operands(x, weight)
         and residual.shape == (x.shape[0], m)
         and norm_weight.shape == (m,)
         and residual.dtype == norm_weight.dtype == torch.bfloat16
@@ -480,8 +498,9 @@ def linear_rope_and_cache(
 
     if (
         bias is None
-        and _skinny_operands(x, weight)
+        and x.dim() == 2
         and _skinny_rows(T, x.shape[1], weight.shape[0])
+        and _skinny_operands(x, weight)
     ):
         q, k, v = parts(
             torch.empty((T, weight.shape[0]), dtype=x.dtype, device=x.device)

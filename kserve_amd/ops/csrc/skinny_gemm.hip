@@ -11,9 +11,9 @@
 // gate as up features and silu(gate) * up leaves it directly.
 //
 // Measured (us with the reduction, weights not in cache; the library's in
-// parentheses): K 4096, M 14336 GLU at 1 row 43 = 5.4 TB/s (66 with the
-// activation kernel), at 24 rows 46; K 4096, M 32000 at 1 row 48 (60); K
-// 14336, M 4096 at 1 / 24 / 96 / 256 rows 26 / 27 / 32 / 53 (27 / 32 / 63 / 62).
+// parentheses): K 4096, M 14336 GLU at 1 row 46 = 5.1 TB/s (67 with the
+// activation kernel), at 24 rows 47; K 4096, M 32000 at 1 row 49 (61); K
+// 14336, M 4096 at 1 / 24 / 96 / 256 rows 24 / 24 / 32 / 54 (27 / 32 / 63 / 62).
 // Up to 48 rows the loads bound it (non-temporal ones took 5 to 10 % off; no
 // gain above); above, LDS reads and the matrix cores of the few blocks that
 // fit, so wide M goes back to the library. The kernel before kept a barrier
@@ -222,18 +222,45 @@ int feature_tile(int N) { return N <= 64 ? 64 : 128; }
 
 }  // namespace
 
-// K splits for [N][K] x [M][K]: until every slot for a block is taken, with
-// four steps per split at least
+// K splits for [N][K] x [M][K]: as many as keep one block on each of the 256
+// compute units, with at least 8 steps a split where there are more than four (4
+// above 64 rows, where a block has twice the features). A block's ring covers
+// the latency by itself, and a second block per unit only added partial sums (us
+// with the reduction, 512 / 256 blocks, 24 rows: 4096 x 4096 12.5 / 10.9, K 8192,
+// M 2048 14.6 / 12.2, K 4096, M 11008 24.7 / 20.6, M 14336 27.0 / 24.0, 2048 x
+// 2048 8.4 / 7.4).
+// Up to 64 rows a later count is taken where the units end more evenly, by a
+// fifth: K 8192, M 10240 (160 tiles) at 48 rows 47 with 1, 38 with 3; K 3584, M
+// 18944 (296) at 1 row 31 with 1, 29 with 2. Splits that lie a multiple of 4 KB
+// apart fall on the same memory channels as the rows below them: up to twice as
+// many are taken if that avoids it as evenly (K 28672, M 8192 at 1 row 90 with 2,
+// 77 with 4), or three for four above 64 rows (8192 x 8192 at 72 rows 43.5 /
+// 37.4, 128 rows 45 / 43; past that the matrix cores want the blocks, 50 / 56 at
+// 192). Up to 64 rows the count does not depend on N, so neither do a row's sums.
 extern "C" int ks_skinny_splits(int M, int K, int N, int glu) {
-  const int bm = feature_tile(N);
-  const long tiles = glu ? (M + bm / 2 - 1) / (bm / 2) : (M + bm - 1) / bm;
+  constexpr int UNITS = 256;
   if (glu) return 1;
-  const long want = N <= 64 ? 512 : 256;
-  long s = want / (tiles > 0 ? tiles : 1);
-  const long most = K / BK / 4;
+  const int bm = feature_tile(N);
+  const int tiles = (M + bm - 1) / bm, steps = K / BK;
+  if (tiles < 1) return 1;
+  int most = steps / 4, s = UNITS / tiles;
+  if (N <= 64 && most > 4) most = steps / 8 > 4 ? steps / 8 : 4;
   if (s > most) s = most;
   if (s > 16) s = 16;
-  return s < 1 ? 1 : (int)s;
+  if (s < 1) s = 1;
+  if (N > 64) return s == 4 && K % 8192 == 0 && N <= 128 ? 3 : s;
+  // rounds of blocks on a unit with t splits, each of 1 / t of K
+  auto rounds = [&](int t) { return ((long)tiles * t + UNITS - 1) / UNITS; };
+  auto aliased = [&](int t) { return K % 2048 == 0 && K * 2L % (t * 4096L) == 0; };
+  for (int t = s + 1; t <= 16 && steps / t >= 12; ++t)
+    if (5 * rounds(t) * s <= 4 * rounds(s) * t) {
+      s = t;
+      break;
+    }
+  if (s > 1 && aliased(s))
+    for (int t = s + 1; t <= 2 * s && t <= 16 && steps / t >= 12; ++t)
+      if (!aliased(t) && rounds(t) * s <= rounds(s) * t) return t;
+  return s;
 }
 
 // `out` null: the sums of the splits stay in `partial` for the caller's kernel.

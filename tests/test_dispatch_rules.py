@@ -1,0 +1,35 @@
+"""Dispatch rules of the products at sizes on both sides of their lines, where the
+times of both kernels are known (no GPU needed: the rules take sizes only)."""
+
+import pytest
+
+from kserve_amd import ops
+
+
+@pytest.mark.parametrize(
+    "n,k,m,own",
+    [
+        (1, 4096, 4096, True), (48, 4096, 32000, True), (64, 4096, 8192, True),
+        (64, 4096, 14336, False),                        # 28.3 us, library 27.5
+        (96, 4096, 4096, True), (128, 3072, 6144, True),
+        (96, 2048, 8192, False), (160, 2560, 8192, False),  # 21.7 / 17.5
+        (192, 4096, 4096, True), (256, 4096, 4096, False),
+        (257, 4096, 8192, False), (8, 4096, 4098, False),
+    ],
+)
+def test_few_row_product(n, k, m, own):
+    assert ops._skinny_rows(n, k, m) is own
+
+
+@pytest.mark.parametrize(
+    "n,k,m,own",
+    [
+        (1, 4096, 14336, True), (64, 4096, 14336, True), (96, 4096, 14336, True),
+        (1, 8192, 14336, True), (1, 8192, 7168, False),  # 56 us, library 50
+        (64, 2560, 9728, False), (64, 5120, 13824, False),  # 71 / 62
+        (96, 8192, 14336, False), (128, 4096, 14336, False),
+        (1, 4096, 3584, False), (1, 4096, 18944, False),
+    ],
+)
+def test_few_row_gate_up(n, k, m, own):
+    assert ops._skinny_glu_rows(n, k, m) is own

@@ -793,6 +793,15 @@ class TestSkinnyGemmEdges:
             ref, off = sg * u, 1.1 * og * (u.abs() + ou) + sg.abs() * ou
         assert ((out.double() - ref).abs() <= off + ref.abs() * 2.0 ** -8).all()
 
+    @pytest.mark.parametrize(
+        "N,K,M", [(33, 8192, 4096), (48, 8192, 10240), (17, 3584, 18944),
+                  (72, 8192, 8192), (5, 28672, 2048), (64, 2112, 768)]
+    )
+    def test_uneven_splits(self, dev, N, K, M):
+        """Counts of K splits beside one block per compute unit, and splits of
+        unequal length."""
+        self.test_against_fp64(dev, N, K, M, False)
+
     def test_dispatch_takes_every_form(self, dev):
         from kserve_amd import ops
 
