@@ -50,9 +50,11 @@ __device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
 // scale in powers of two, so hidden keys (MASKED) come to 0; the query is
 // multiplied by `pre`, which has a negative scale's sign, or the scale itself
 // where it is too close to 0 for that (the scores are all next to 0 then).
+// Formed on the host: kernel arguments are scalar registers, and the vector
+// registers of the forms with three parts are full.
 struct ScoreScale {
   float c2, pre = 1.f;
-  __device__ __forceinline__ explicit ScoreScale(float scale) : c2(scale * LOG2E) {
+  ScoreScale(float scale) : c2(scale * LOG2E) {
     if (c2 < 0.f) {
       pre = -1.f;
       c2 = -c2;
@@ -154,7 +156,7 @@ struct PrefillArgs {
   const int* block_tables;  // [S, max_nb] (pages, row stride max_nb)
   int Hq, Hkv, max_nb;
   int hpb;  // query heads per block: 1, 2 or 4, divides the group
-  float scale;
+  ScoreScale scale;
   long sq, sk, sv;
   int window;
   Extra x;
@@ -194,8 +196,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   __shared__ __attribute__((aligned(16))) short lds[2][2][TILE];  // [buffer][K, V]
 
   // ---- queries: B operands, 8 consecutive columns per lane ----
-  const ScoreScale scale(p.scale);
-  const float c2 = scale.c2;
+  const float c2 = p.scale.c2;
   bf16x8_t qf[PARTS][KC];
   {
     const int qrow = min(q0 + (lane & 31), q_len - 1);
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
       const short* qp = reinterpret_cast<const short*>(p.q) + at;
 #pragma unroll
       for (int c = 0; c < KC; ++c)
-        qf[0][c] = scale.apply(*reinterpret_cast<const bf16x8_t*>(qp + c * 16));
+        qf[0][c] = p.scale.apply(*reinterpret_cast<const bf16x8_t*>(qp + c * 16));
     } else {
       const float* qp = reinterpret_cast<const float*>(p.q) + at;
 #pragma unroll
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
           const f32x4_t x = *reinterpret_cast<const f32x4_t*>(qp + c * 16 + j);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const Split3 w(x[e] * scale.pre);
+            const Split3 w(x[e]);
             qf[0][c][j + e] = w.hi;
             qf[1][c][j + e] = w.mid;
             qf[2][c][j + e] = w.lo;
@@ -367,6 +368,14 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
         }
         if constexpr (PARTS == 3) s[kb] += rest;
       }
+      // Three parts: the scale's sign here and not in the query. The branch also
+      // keeps the products apart from the softmax; scheduled as one block the two
+      // need 13 registers more than there are (4 x 2000 tokens, 16 / 4 heads of
+      // 128: 237 us with the spills, 215 so).
+      if (PARTS == 3 && p.scale.pre != 1.f) {
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb) s[kb] *= p.scale.pre;
+      }
       // register r of block kb: key 32 kb + (r & 3) + 8 (r / 4) + 4 half
       if (t0 + KT > len || (CAUSAL && t0 + KT - 1 > pos_lo) ||
           (WIN && t0 < low_hi)) {
@@ -518,7 +527,7 @@ struct DecodeArgs {
   const void* v_cache;      // likewise, sv
   const int* block_tables;  // [S, max_blocks]
   const int* ctx_lens;      // [S]
-  float scale;
+  ScoreScale scale;
   int H, Hkv, group, max_blocks;
   long sq;
   int n_splits;
@@ -585,8 +594,7 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
   __shared__ __attribute__((aligned(16))) short lds[NW][STAGE];
   static_assert(STAGE * 2 >= 8 * (D + 4) * 4 + 64, "merge area");
 
-  const ScoreScale scale(p.scale);
-  const float c2 = scale.c2;
+  const float c2 = p.scale.c2;
   bf16x8_t qf[PARTS][KC];
   {
     const long at = (long)tok * p.sq + (long)(kvh * G + col % G) * D + g * 8;
@@ -597,7 +605,7 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
         short8_t x = *reinterpret_cast<const short8_t*>(qp + c * 32);
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = used ? x[j] : 0;
-        qf[0][c] = scale.apply(__builtin_bit_cast(bf16x8_t, x));
+        qf[0][c] = p.scale.apply(__builtin_bit_cast(bf16x8_t, x));
       }
     } else {
       const float* qp = reinterpret_cast<const float*>(p.q) + at;
@@ -608,7 +616,7 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
           const f32x4_t x = *reinterpret_cast<const f32x4_t*>(qp + c * 32 + j);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const Split3 w(used ? x[e] * scale.pre : 0.f);
+            const Split3 w(used ? x[e] * p.scale.pre : 0.f);
             qf[0][c][j + e] = w.hi;
             qf[1][c][j + e] = w.mid;
             qf[2][c][j + e] = w.lo;
