@@ -100,16 +100,19 @@ __device__ __forceinline__ void load4<float>(const float* p, float* v) {
   for (int i = 0; i < 4; ++i) v[i] = x[i];
 }
 
-constexpr int CONV_TT = 4;  // tokens per block of the vector kernel
+// A block of the vector kernel takes 4 tokens, or 16 where inputs and outputs
+// are more than the memory-side cache holds (256 MB: 6 bytes an element with
+// bf16 in). The last TAPS - 1 inputs stay in registers while a lane walks its
+// tokens, so a token costs one load and a block TAPS - 1 more; these come from a
+// cache up to there, while the loads of a walk are one after the other and short
+// portions start it anew (with the state update, us, 4 / 16 tokens, 6144
+// channels: 500 tokens 11 / 16, 6000 48 / 48, 8000 75 / 70; 127 sequences of 1
+// and one of 385 23 / 39; 10240 channels, 6000 tokens 103 / 85). Bound by memory:
+// 8000 tokens of 6144 channels 61 us = 4.8 TB/s without the update.
+constexpr int CONV_TT = 4, CONV_TT_LONG = 16;
+constexpr long CONV_LONG = 42L << 20;  // tokens x channels
 
-// The last TAPS - 1 inputs stay in registers while a lane walks its tokens, so
-// a token costs one load. Bound by memory (bf16 in, fp32 out): 8000 tokens of
-// 6144 channels take 61 us = 4.8 TB/s, 93 us when every tap was loaded. Four
-// tokens a block: the loads of a walk are one after the other, and short
-// portions start it anew (with the state update, us, blocks of 1 / 4 / 16
-// tokens, 6144 channels: 8000 tokens 113 / 72 / 73, 500 14 / 11 / 15, 127
-// sequences of 1 and one of 385 23 / 23 / 39; 2048 channels 11 / 14 / 31).
-template <typename T, int TAPS>
+template <typename T, int TAPS, int TT>
 __global__ __launch_bounds__(256) void causal_conv_silu_vec4_kernel(
     float* __restrict__ out, const T* __restrict__ in, long in_stride,
     const float* __restrict__ w, const float* __restrict__ bias,
@@ -127,8 +130,8 @@ __global__ __launch_bounds__(256) void causal_conv_silu_vec4_kernel(
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) wt[i][j] = w[(long)(c + i) * TAPS + j];
-  const int t0 = blockIdx.y * CONV_TT;
-  const int t_end = min(tokens, t0 + CONV_TT);
+  const int t0 = blockIdx.y * TT;
+  const int t_end = min(tokens, t0 + TT);
   float win[TAPS][4];  // inputs of tokens t - hist .. t
   int end = 0;         // first token after the sequence that t is in
   for (int t = t0; t < t_end; ++t) {
@@ -822,7 +825,9 @@ extern "C" hipError_t ks_causal_conv_silu(
                    ((uintptr_t)conv_state % (4 * esz)) == 0 &&
                    ((uintptr_t)out % 16) == 0 && ((uintptr_t)bias % 16) == 0 &&
                    taps >= 2 && taps <= 4;
-  dim3 grid_v(cdiv(channels / 4, 256), cdiv(tokens, CONV_TT));
+  const bool longer = (long)tokens * channels > CONV_LONG;
+  dim3 grid_v(cdiv(channels / 4, 256),
+              cdiv(tokens, longer ? CONV_TT_LONG : CONV_TT));
 #define CONV_ARGS(TT)                                                         \
   (float*)out, (const TT*)in, in_stride, (const float*)w, (const float*)bias, \
       (const TT*)conv_state, (const long*)positions,                          \
@@ -846,9 +851,14 @@ extern "C" hipError_t ks_causal_conv_silu(
     HIP_CHECK_KERNEL();
     return hipSuccess;
   }
-#define CONV_VEC_K(TT, K)                                                     \
-  hipLaunchKernelGGL((causal_conv_silu_vec4_kernel<TT, K>), grid_v,           \
+#define CONV_VEC_N(TT, K, N)                                                  \
+  hipLaunchKernelGGL((causal_conv_silu_vec4_kernel<TT, K, N>), grid_v,        \
                      dim3(256), 0, stream, CONV_ARGS(TT), tokens, channels, silu)
+#define CONV_VEC_K(TT, K)                        \
+  do {                                           \
+    if (longer) CONV_VEC_N(TT, K, CONV_TT_LONG); \
+    else CONV_VEC_N(TT, K, CONV_TT);             \
+  } while (0)
 #define CONV_VEC(TT)                                                          \
   do {                                                                        \
     if (taps == 2) CONV_VEC_K(TT, 2);                                         \

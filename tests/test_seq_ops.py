@@ -264,6 +264,28 @@ class TestCausalConv:
         )
         self.test_portions_of_every_route(be, taps, lens, bias)
 
+    @pytest.mark.gpu
+    def test_more_than_the_cache(self):
+        """Blocks of 16 tokens, portions that end inside and on their edges."""
+        C, lens = 14336, [1601, 1, 15, 16, 17, 1550]
+        assert sum(lens) * C > 42 << 20
+        cu, seq, pos = layout(lens, [0, 5, 0, 7, 9, 1])
+        be = ("cuda", torch.bfloat16)
+        x, w = rnd(sum(lens), C, seed=21, dtype=be[1]), rnd(C, 4, seed=22, scale=0.5)
+        state = rnd(len(lens), 3, C, seed=23, dtype=be[1]).to(be[1])
+        ref_state, dev_state = state.clone(), state.to(be[0])
+        slots = list(range(len(lens)))
+        got = ops.causal_conv_silu(
+            act(x, be), f32(w, be), None, dev_state, i64(pos, be), i32(seq, be),
+            i32(cu, be), i32(slots, be),
+        )
+        want = ops.torch_ref.causal_conv_silu(
+            x, w, None, ref_state, torch.tensor(pos), torch.tensor(cu),
+            torch.tensor(slots),
+        )
+        close(got, want.double(), be, bf16_tol=1e-6)  # four fp32 products
+        assert torch.equal(dev_state.cpu(), ref_state)
+
     def test_one_long_portion_is_not_walked(self):
         """127 decode tokens beside a prompt portion: the average says decode."""
         assert ops._conv_whole_portions(128, 128, 1)
