@@ -351,12 +351,13 @@ def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     8192, m 7168 at 1 row 56 / 50, m 14336 88 / 129). Past 48 rows the block's
     LDS reads bound it: it stays where the blocks come out even and K is not
     longer (k 3072, m 8192 25 / 28; k 2560, m 9728 35 / 31, k 5120, m 13824
-    71 / 62, k 8192, m 14336 at 96 rows 114 / 110). Above 16384 features the
-    library is level (k 8192, m 28672 at 1 row 182 / 180)."""
+    71 / 62). Above 64 rows it is level with the library (k 5120, m 13824 at 72 /
+    112 rows 66 / 70, 74 / 69) and keeps gate and up in 32 bits. Above 16384
+    features the library is level (k 8192, m 28672 at 1 row 182 / 180)."""
     if m % 4 or m > 16384 or n > 112:
         return False
-    if k > 4096:
-        return n <= 48 and m >= 12288
+    if k > 4096 and (m < 12288 or 48 < n <= 64):
+        return False
     if n > 64:
         return m >= 12288
     return m >= 4608 and (n <= 48 or m <= 8192 or m >= 10240)

@@ -59,7 +59,8 @@ extern "C" hipError_t ks_paged_attention_decode(
   if (num_seqs == 0) return hipSuccess;
   if (n_splits < 1 || !part_out || !part_ml) n_splits = 1;
   const DecodeArgs p{out, q, k_cache, v_cache,
-                     (const int*)block_tables, (const int*)context_lens, scale,
+                     (const int*)block_tables, (const int*)context_lens,
+                     score_scale(scale),
                      num_heads, num_kv_heads, group, max_blocks, q_row_stride,
                      n_splits, (float*)part_out, (float*)part_ml, window,
                      head_dim, head_dim, nullptr, Extra{}};

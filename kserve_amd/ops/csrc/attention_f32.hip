@@ -1029,7 +1029,7 @@ static hipError_t ctx_attention_mfma(const CtxArgs& a) {
     const long rows = (long)a.num_seqs * a.heads * a.nsplit;
     const DecodeArgs p{a.out, a.q, a.k_cache, a.v_cache,
                        (const int*)a.block_tables, (const int*)a.ctx_lens,
-                       a.scale, a.heads, a.kv_heads, a.heads / a.kv_heads,
+                       score_scale(a.scale), a.heads, a.kv_heads, a.heads / a.kv_heads,
                        a.bt_stride, (long)a.heads * a.D, a.nsplit, ws,
                        ws ? ws + rows * a.DV : nullptr, a.window, a.D,
                        a.v_row_stride, (const int*)a.cu_q, x};
@@ -1040,7 +1040,7 @@ static hipError_t ctx_attention_mfma(const CtxArgs& a) {
   const int hpb = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
   const PrefillArgs p{a.out, a.q, a.k_cache, a.v_cache, (const int*)a.cu_q,
                       (const int*)a.ctx_lens, (const int*)a.block_tables,
-                      a.heads, a.kv_heads, a.bt_stride, hpb, a.scale,
+                      a.heads, a.kv_heads, a.bt_stride, hpb, score_scale(a.scale),
                       (long)a.heads * a.D, a.D, a.v_row_stride, a.window, x};
   const dim3 grid(a.heads / hpb, cdiv(a.max_q_len, NWAVES * QW / hpb), a.num_seqs);
 #define GO(DD, WW)                                                             \

@@ -80,7 +80,7 @@ extern "C" hipError_t ks_context_prefill_varlen(
   if (Hq % Hkv != 0) return hipErrorInvalidValue;
   PrefillArgs p{out, q, k_cache, v_cache,
                 (const int*)cu_seqlens_q, (const int*)ctx_lens,
-                (const int*)block_tables, Hq, Hkv, max_nb, 1, scale, sq,
+                (const int*)block_tables, Hq, Hkv, max_nb, 1, score_scale(scale), sq,
                 head_dim, head_dim, window, Extra{}};
   if (fp8_cache) return launch<128, PAGES_FP8>(p, num_seqs, max_q_len, true, stream);
   if (aligned16(k_cache, v_cache))
@@ -96,7 +96,7 @@ extern "C" hipError_t ks_flash_prefill_varlen(
   if (head_dim != 128 && head_dim != 64) return hipErrorInvalidValue;
   if (Hq % Hkv != 0) return hipErrorInvalidValue;
   PrefillArgs p{out, q, k, v, (const int*)cu_seqlens,
-                nullptr, nullptr, Hq, Hkv, 0, 1, scale, sq, sk, sv, window,
+                nullptr, nullptr, Hq, Hkv, 0, 1, score_scale(scale), sq, sk, sv, window,
                 Extra{}};
   // LDS-direct loads move 16 aligned bytes per lane
   const bool dma = aligned16(k, v) && sk % 8 == 0 && sv % 8 == 0;

@@ -46,32 +46,12 @@ __device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// Softmax weights are exp2((s - m) c2) with m the largest score. c2 > 0 is the
-// scale in powers of two, so hidden keys (MASKED) come to 0; the query is
-// multiplied by `pre`, which has a negative scale's sign, or the scale itself
-// where it is too close to 0 for that (the scores are all next to 0 then).
-// Formed on the host: kernel arguments are scalar registers, and the vector
-// registers of the forms with three parts are full.
-struct ScoreScale {
-  float c2, pre = 1.f;
-  ScoreScale(float scale) : c2(scale * LOG2E) {
-    if (c2 < 0.f) {
-      pre = -1.f;
-      c2 = -c2;
-    }
-    if (c2 < 1e-30f) {
-      pre *= c2;
-      c2 = 1.f;
-    }
-  }
-  __device__ __forceinline__ bf16x8_t apply(bf16x8_t q) const {
-    if (pre != 1.f) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) q[j] = (__bf16)((float)q[j] * pre);
-    }
-    return q;
-  }
-};
+// What the launchers hand the kernels as their scale: scores are masked before
+// they are scaled, and the scaled mask has to give weight 0. Below 1e-30 all
+// scores are level whatever the scale.
+inline float score_scale(float scale) {
+  return fabsf(scale) < 1e-30f ? copysignf(1e-30f, scale) : scale;
+}
 
 // x as the sum of three bf16 numbers, exactly
 struct Split3 {
@@ -156,7 +136,7 @@ struct PrefillArgs {
   const int* block_tables;  // [S, max_nb] (pages, row stride max_nb)
   int Hq, Hkv, max_nb;
   int hpb;  // query heads per block: 1, 2 or 4, divides the group
-  ScoreScale scale;
+  float scale;
   long sq, sk, sv;
   int window;
   Extra x;
@@ -196,7 +176,6 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   __shared__ __attribute__((aligned(16))) short lds[2][2][TILE];  // [buffer][K, V]
 
   // ---- queries: B operands, 8 consecutive columns per lane ----
-  const float c2 = p.scale.c2;
   bf16x8_t qf[PARTS][KC];
   {
     const int qrow = min(q0 + (lane & 31), q_len - 1);
@@ -205,7 +184,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
       const short* qp = reinterpret_cast<const short*>(p.q) + at;
 #pragma unroll
       for (int c = 0; c < KC; ++c)
-        qf[0][c] = p.scale.apply(*reinterpret_cast<const bf16x8_t*>(qp + c * 16));
+        qf[0][c] = *reinterpret_cast<const bf16x8_t*>(qp + c * 16);
     } else {
       const float* qp = reinterpret_cast<const float*>(p.q) + at;
 #pragma unroll
@@ -320,6 +299,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
                (((4 * b + ((lane >> 4) & 1) * 2 + ((ti & 3) >> 1)) ^ v_swz<D>(vrow)) * 8) +
                (ti & 1) * 4;
 
+  float c2 = p.scale * LOG2E;
+  const bool flip = c2 < 0.f;
+  c2 = fabsf(c2);
   float m = NO_MAX, l = 0.f;
   f32x16_t o[DB];
 #pragma unroll
@@ -368,13 +350,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
         }
         if constexpr (PARTS == 3) s[kb] += rest;
       }
-      // Three parts: the scale's sign here and not in the query. The branch also
-      // keeps the products apart from the softmax; scheduled as one block the two
-      // need 13 registers more than there are (4 x 2000 tokens, 16 / 4 heads of
-      // 128: 237 us with the spills, 215 so).
-      if (PARTS == 3 && p.scale.pre != 1.f) {
+      if (flip) {
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) s[kb] *= p.scale.pre;
+        for (int kb = 0; kb < NKB; ++kb) s[kb] = -s[kb];
       }
       // register r of block kb: key 32 kb + (r & 3) + 8 (r / 4) + 4 half
       if (t0 + KT > len || (CAUSAL && t0 + KT - 1 > pos_lo) ||
@@ -527,7 +505,7 @@ struct DecodeArgs {
   const void* v_cache;      // likewise, sv
   const int* block_tables;  // [S, max_blocks]
   const int* ctx_lens;      // [S]
-  ScoreScale scale;
+  float scale;
   int H, Hkv, group, max_blocks;
   long sq;
   int n_splits;
@@ -594,7 +572,6 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
   __shared__ __attribute__((aligned(16))) short lds[NW][STAGE];
   static_assert(STAGE * 2 >= 8 * (D + 4) * 4 + 64, "merge area");
 
-  const float c2 = p.scale.c2;
   bf16x8_t qf[PARTS][KC];
   {
     const long at = (long)tok * p.sq + (long)(kvh * G + col % G) * D + g * 8;
@@ -605,7 +582,7 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
         short8_t x = *reinterpret_cast<const short8_t*>(qp + c * 32);
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[j] = used ? x[j] : 0;
-        qf[0][c] = p.scale.apply(__builtin_bit_cast(bf16x8_t, x));
+        qf[0][c] = __builtin_bit_cast(bf16x8_t, x);
       }
     } else {
       const float* qp = reinterpret_cast<const float*>(p.q) + at;
@@ -616,7 +593,7 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
           const f32x4_t x = *reinterpret_cast<const f32x4_t*>(qp + c * 32 + j);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const Split3 w(used ? x[e] * p.scale.pre : 0.f);
+            const Split3 w(used ? x[e] : 0.f);
             qf[0][c][j + e] = w.hi;
             qf[1][c][j + e] = w.mid;
             qf[2][c][j + e] = w.lo;
@@ -697,6 +674,9 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
     vaddr[b] = ROWS * D + vrow * D +
                ((2 * b + ((col & 3) >> 1)) ^ v_swz<D>(vrow)) * 8 + (col & 1) * 4;
 
+  float c2 = p.scale * LOG2E;
+  const bool flip = c2 < 0.f;
+  c2 = fabsf(c2);
   const int key_lo = low_of(ctx - 1, p.window, p.x.chunk);  // first visible key
   float m = NO_MAX, l = 0.f;
   f32x4_t o[DB];
@@ -720,6 +700,10 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
         sc[h] = mfma16x16x32(a, qf[0][c], sc[h]);
       }
       if constexpr (PARTS == 3) sc[h] += rest;
+    }
+    if (flip) {
+      sc[0] = -sc[0];
+      sc[1] = -sc[1];
     }
     const int key0 = (rg.first + 2 * n) * PAGE;
     if (key0 + ROWS > ctx || key0 < key_lo) {

@@ -231,7 +231,8 @@ int feature_tile(int N) { return N <= 64 ? 64 : 128; }
 // 2048 8.4 / 7.4).
 // Up to 64 rows a later count is taken where the units end more evenly, by a
 // fifth: K 8192, M 10240 (160 tiles) at 48 rows 47 with 1, 38 with 3; K 3584, M
-// 18944 (296) at 1 row 31 with 1, 29 with 2. Splits that lie a multiple of 4 KB
+// 18944 (296) at 1 row 31 with 1, 29 with 2; not from two blocks a unit on (M
+// 37888 at 33 rows 56 with 1, 62 with 3). Splits that lie a multiple of 4 KB
 // apart fall on the same memory channels as the rows below them: up to twice as
 // many are taken if that avoids it as evenly (K 28672, M 8192 at 1 row 90 with 2,
 // 77 with 4), or three for four above 64 rows (8192 x 8192 at 72 rows 43.5 /
@@ -252,7 +253,7 @@ extern "C" int ks_skinny_splits(int M, int K, int N, int glu) {
   // rounds of blocks on a unit with t splits, each of 1 / t of K
   auto rounds = [&](int t) { return ((long)tiles * t + UNITS - 1) / UNITS; };
   auto aliased = [&](int t) { return K % 2048 == 0 && K * 2L % (t * 4096L) == 0; };
-  for (int t = s + 1; t <= 16 && steps / t >= 12; ++t)
+  for (int t = s + 1; tiles < 2 * UNITS && t <= 16 && steps / t >= 12; ++t)
     if (5 * rounds(t) * s <= 4 * rounds(s) * t) {
       s = t;
       break;

@@ -27,7 +27,7 @@ def test_few_row_product(n, k, m, own):
         (1, 4096, 14336, True), (64, 4096, 14336, True), (96, 4096, 14336, True),
         (1, 8192, 14336, True), (1, 8192, 7168, False),  # 56 us, library 50
         (64, 2560, 9728, False), (64, 5120, 13824, False),  # 71 / 62
-        (96, 8192, 14336, False), (128, 4096, 14336, False),
+        (96, 8192, 14336, True), (64, 8192, 14336, False), (128, 4096, 14336, False),
         (1, 4096, 3584, False), (1, 4096, 18944, False),
     ],
 )
