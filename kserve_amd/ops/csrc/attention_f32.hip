@@ -997,8 +997,8 @@ hipError_t dispatch_d(const CtxArgs& a) {
 // pages of 16, everything 16-byte aligned. Error against 64 bits (fp32 output,
 // 1 to 2000 keys): 0.9e-7 to 3.9e-7 with fp32 products, 0.6e-7 to 2.6e-7 here.
 // Times (us, fp32 products -> this), heads of 128: prefill 4 x 2000, 16/4 heads
-// 1428 -> 237, 8 x 2048, 32/8 heads 5912 -> 837, windowed (1024, 16/4 heads)
-// 1675 -> 351, 500 after 1500 266 -> 106; decode 128 of 1500 +- 60%, 16/4 heads
+// 1428 -> 226, 8 x 2048, 32/8 heads 5912 -> 798, windowed (1024, 16/4 heads)
+// 1675 -> 322, 500 after 1500 266 -> 104; decode 128 of 1500 +- 60%, 16/4 heads
 // 281 -> 78, 256 of 2048, 32/8 heads 985 -> 340, one of 600 27 -> 10.
 extern "C" int ks_ctx_attention_mfma(const void* out, const void* q,
                                      const void* k_cache, const void* v_cache,

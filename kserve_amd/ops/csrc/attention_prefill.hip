@@ -12,8 +12,10 @@
 // never leave registers.
 //
 // A block is 4 waves of 32 queries and shares double-buffered tiles of 64 keys
-// that the LDS-direct loads fill while the other buffer is computed on; the
-// XOR swizzles below are on the source side of those loads. With several query
+// that the LDS-direct loads fill while the other buffer is computed on (they run
+// under K Q^T and the softmax: the compiler waits for them ahead of the
+// transposing reads of V); the XOR swizzles are on the source side of those
+// loads. With several query
 // heads per KV head the waves take up to four heads of one group over the same
 // queries (equal causal ranges, and a K/V tile is fetched once for the group);
 // otherwise consecutive queries of one head.
@@ -25,9 +27,9 @@
 // overlap the three. Measured (32 query and 8 KV heads of 128, causal; the
 // 16x16x32 kernel with one head per block, V transposed by 2-byte LDS stores and
 // a barrier on each side of the staging, before this one): 1 x 8191 tokens
-// 2497 -> 652 us (220 -> 843 TFLOP/s), 8 x 2048 1280 -> 387 us, 32 x 512
-// 413 -> 149 us; 2 x 1000 queries over 13000 paged keys 2441 -> 509 us (E4M3
-// pages 2596 -> 625); 64 x 128, 12 heads of 64, bidirectional 28 -> 13 us.
+// 2497 -> 597 us (220 -> 921 TFLOP/s), 8 x 2048 1280 -> 365 us, 32 x 512
+// 413 -> 141 us; 2 x 1000 queries over 13000 paged keys 2441 -> 460 us (E4M3
+// pages 2596 -> 557); 64 x 128, 12 heads of 64, bidirectional 28 -> 12 us.
 //
 // Replaces the vLLM flash prefill the reference delegates to. Numerics oracles:
 // ops/torch_ref.flash_prefill_varlen and context_attention_varlen.

@@ -947,9 +947,13 @@ extern "C" hipError_t ks_ssd_scan(void* y, const void* xbc, const void* dt_raw,
     return hipSuccess;
   }
   // A token or two per sequence: whole state rows by 16-byte lanes (us, token by
-  // token in chunks of 16 -> this, 64 heads of 64 x 128: 128 x 1 token 153 ->
-  // 83, 128 x 2 159 -> 86, 64 x 8 85 -> 72; one long portion among them loses
-  // it again, 127 x 1 + 100 tokens 244 -> 183, 127 x 1 + 500 612 -> 655)
+  // token in chunks of 16 -> this, 64 heads of 64 x 128, states not in a cache:
+  // 128 x 1 token 162 -> 105, 128 x 2 164 -> 108, 4 of 1 to 5 18 -> 13). One long
+  // portion among them is walked at 1.0 to 1.7 us per token here and there, and
+  // the rule keeps it to about as many tokens as there are sequences, whose
+  // states cost more than the walk gains there: 127 x 1 + 100 254 -> 214, 127 x 1
+  // + 129 277 -> 250, 399 x 1 + 401 817 -> 764, 1019 x 1 + 1020 2060 -> 1920
+  // (with 500 beside 127 it would be 612 -> 655, past the rule)
   if (tokens <= 2L * num_seqs && (N == 64 || N == 128) && P % 64 == 0 &&
       (((uintptr_t)xbc | (uintptr_t)state) & 15) == 0) {
     const dim3 sgrid(P / 64, heads, num_seqs);
