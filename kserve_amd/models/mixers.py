@@ -116,6 +116,7 @@ class SSDMixer(nn.Module):
         y = ops.ssd_scan(
             xbc, dt_raw, self.dt_bias, self.a_log, self.d_skip, cache.ssm,
             positions, meta.cu_seqlens, meta.state_slots, s.groups,
+            longest=meta.max_seqlen,
         )
         yn = ops.gated_group_rms_norm(
             y, z, self.norm_w, self.eps, s.norm_groups, self.dtype

@@ -698,17 +698,54 @@ def causal_conv_silu(
     )
 
 
+def _scan_in_chunks(
+    tokens: int, seqs: int, longest: int, heads: int, P: int, N: int
+) -> bool:
+    """Whether the scan takes chunks of 64 tokens (a block per 64 columns, head
+    and sequence, one on each of the 256 compute units at a time) rather than
+    token by token. Both times are estimated, in us, from measurements over 8 to
+    128 heads, P 32 to 128, N 16 to 128, 1 to 256 sequences of 8 to 256 tokens:
+    the walk costs the longest portion its latencies and the chip its tokens, a
+    chunk much the same however few tokens it has. (Token by token / chunks, 64
+    heads of 64 x 128: 4 x 16 tokens 23 / 15, 8 x 20 31 / 25, 16 x 24 46 / 50,
+    32 x 32 104 / 97, 128 x 32 371 / 395, 128 x 40 466 / 400; 16 heads of 64 x 16:
+    32 x 24 15 / 15, 128 x 48 52 / 56, 256 x 56 99 / 110; 8 heads of 32 x 16, 256 x
+    32 23 / 53, 64 x 80 27 / 23.)"""
+    longest = max(longest, -(-tokens // max(seqs, 1)))
+    if longest < 16:
+        return False
+    cols = -(-P // 64)
+    rounds = -(-cols * heads * seqs // 256)
+    average = tokens / seqs
+    # columns that do not fill a block of 64 cost the walk less
+    fill = max(0.3, 1 - 1.3 * (1 - P / (64 * cols)) ** 2)
+    latency = fill * (0.35 + 0.0047 * N)
+    work = fill * rounds * (0.075 + 0.0021 * N)
+    walk = 3 + 0.04 * N + max(
+        longest * latency, average * max(work, 0.6 * (latency + work))
+    )
+    chunk = 6.7 if N <= 32 else 8.2 if N <= 64 else 11.8
+    chunks = min(-(-longest // 64), average / 64 + 1)
+    last = -(-longest // 64) * chunk
+    return max(rounds * chunk * (1 + 0.75 * (chunks - 1)), last) < walk
+
+
 def ssd_scan(
     xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, cu_seqlens, slots,
-    groups: int,
+    groups: int, longest: int = 0,
 ):
-    """State-space scan; carries ``state[slot]`` ([heads, P, N] fp32)."""
+    """State-space scan; carries ``state[slot]`` ([heads, P, N] fp32).
+    ``longest``: tokens of the longest portion (0: taken as the average), which
+    chooses between kernels."""
     if xbc.is_cuda:
         heads, P = state.shape[1], state.shape[2]
         y = _f32_like(xbc.shape[0], heads * P, xbc)
         _native_seq("ssd_scan").ssd_scan(
             y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions,
             cu_seqlens, slots, int(groups),
+            _scan_in_chunks(
+                xbc.shape[0], slots.numel(), longest, heads, P, state.shape[3]
+            ),
         )
         return y
     return torch_ref.ssd_scan(

@@ -23,7 +23,7 @@ hipError_t ks_causal_conv_silu(void*, const void*, long, const void*,
 hipError_t ks_ssd_scan(void*, const void*, const void*, long, int, const void*,
                        const void*, const void*, void*, const void*,
                        const void*, const void*, int, int, int, int, int, int,
-                       hipStream_t);
+                       int, hipStream_t);
 hipError_t ks_qk_norm_temp_cache(void*, const void*, const void*, const void*,
                                  long, const void*, const void*, const void*,
                                  const void*, void*, void*, float, float, int,
@@ -319,7 +319,7 @@ void causal_conv_silu(at::Tensor& out, at::Tensor& in, at::Tensor& w,
 void ssd_scan(at::Tensor& y, at::Tensor& xbc, at::Tensor& dt_raw,
               at::Tensor& dt_bias, at::Tensor& a_log, at::Tensor& d_skip,
               at::Tensor& state, at::Tensor& positions, at::Tensor& cu_seqlens,
-              at::Tensor& slots, int64_t groups) {
+              at::Tensor& slots, int64_t groups, bool chunks) {
   CHECK_F32(y);
   CHECK_F32(xbc);
   CHECK_F32(dt_bias);
@@ -347,7 +347,7 @@ void ssd_scan(at::Tensor& y, at::Tensor& xbc, at::Tensor& dt_raw,
                         d_skip.data_ptr(), state.data_ptr(),
                         positions.data_ptr(), cu_seqlens.data_ptr(),
                         slots.data_ptr(), tokens, num_seqs, heads, (int)groups,
-                        P, N, current_stream()),
+                        P, N, chunks ? 1 : 0, current_stream()),
             "ssd_scan");
 }
 

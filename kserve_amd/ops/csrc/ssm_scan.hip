@@ -916,18 +916,12 @@ extern "C" hipError_t ks_ssd_scan(void* y, const void* xbc, const void* dt_raw,
                                   const void* positions,
                                   const void* cu_seqlens, const void* slots,
                                   int tokens, int num_seqs, int heads,
-                                  int groups, int P, int N,
+                                  int groups, int P, int N, int chunks,
                                   hipStream_t stream) {
   if (num_seqs == 0) return hipSuccess;
   if (groups <= 0 || heads % groups != 0 || N < 1 || N > 256)
     return hipErrorInvalidValue;
-  // Chunks of 64 tokens pay off from 32 tokens per sequence on, and from 16
-  // where blocks are few enough to be in flight at once (us, token by token ->
-  // chunks, 64 heads: 64 x 16 tokens 108 -> 193, 64 x 32 197 -> 188, 16 x 24
-  // 47 -> 48; 8 x 16 25 -> 24, 8 x 8 18 -> 24; 1 x 24 29 -> 13)
-  const long chunk_blocks = (long)cdiv(P, 64) * heads * num_seqs;
-  if (tokens >= (chunk_blocks <= 512 ? 16L : 32L) * num_seqs && N % 4 == 0 &&
-      N <= 128 && P % 4 == 0 &&
+  if (chunks && N % 4 == 0 && N <= 128 && P % 4 == 0 &&
       (((uintptr_t)xbc | (uintptr_t)state) & 15) == 0) {
     const dim3 cgrid(cdiv(P, 64), heads, num_seqs);
 #define SSD_CHUNK(nb)                                                         \

@@ -33,3 +33,26 @@ def test_few_row_product(n, k, m, own):
 )
 def test_few_row_gate_up(n, k, m, own):
     assert ops._skinny_glu_rows(n, k, m) is own
+
+
+@pytest.mark.parametrize(
+    "lens,heads,P,N,chunks",
+    [
+        ([15], 64, 64, 128, False), ([16] * 4, 64, 64, 128, True),
+        ([20] * 8, 64, 64, 128, True), ([24] * 16, 64, 64, 128, False),
+        ([32] * 32, 64, 64, 128, True), ([32] * 128, 64, 64, 128, False),
+        ([40] * 128, 64, 64, 128, True), ([2000] * 4, 64, 64, 128, True),
+        ([16] * 64, 8, 32, 16, False),       # 8 us token by token, 14 in chunks
+        ([32] * 256, 8, 32, 16, False),      # 23 / 53
+        ([80] * 64, 8, 32, 16, True),        # 27 / 23
+        ([56] * 256, 16, 64, 16, False), ([65] * 256, 24, 64, 64, False),
+        ([1] * 128, 64, 64, 128, False), ([1] * 127 + [129], 64, 64, 128, False),
+        ([1] * 127 + [500], 64, 64, 128, True),  # the long one is not walked
+        ([1] * 63 + [2000], 64, 64, 128, True),
+        ([], 64, 64, 128, False),
+    ],
+)
+def test_scan_in_chunks(lens, heads, P, N, chunks):
+    assert ops._scan_in_chunks(
+        sum(lens), len(lens), max(lens, default=0), heads, P, N
+    ) is chunks
