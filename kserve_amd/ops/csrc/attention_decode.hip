@@ -32,8 +32,10 @@
 // 332 us (6.5); 512 of 576 341 -> 189 us; E4M3, 96 of 3000 268 -> 93 us, 3000 +-
 // 60% 390 -> 108 us; one of 560 12.5 -> 9.7 us, of 7000 66 -> 14.5 us; 64 / 8
 // heads, 64 of 600 83 -> 29 us. Short contexts are bound by a block's fixed work
-// (about 5 us) and not by the pages; there E4M3 pages under one query head each
-// are slower than before (500 of 100: 24 -> 31 us, 8 heads). The page loads are
+// (about 5 us) and not by the pages: 500 of 100 tokens, 8 heads 98 -> 42 us, E4M3
+// 50 -> 31; one or two pages under one query head each are the only ones slower
+// than before (1000 of 16, 32 heads 97 -> 83 us where the table is as short, 138
+// in a wide one; E4M3 53 -> 72 and 133). The page loads are
 // non-temporal: a step's pages pass once and a model's do not fit the caches.
 //
 // Splits are merged by paged_attention_reduce_kernel. Numerics oracle:

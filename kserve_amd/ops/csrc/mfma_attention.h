@@ -861,17 +861,35 @@ __global__ __launch_bounds__(256) void paged_attention_reduce_kernel(
 // with 1 / 2 / 4 waves: 256 sequences of 2048 +- 60% 364 / 349 / 338, 64 of 1000
 // +- 60% 56 / 48 / 48, 500 of 100 37 / 38 / 46; E4M3, 96 of 3000 +- 60% 182 /
 // 122 / 115, without the launch bound above).
+//
+// One wave where a table holds a page pair or two per wave (four of E4M3) and
+// the blocks are more than the chip takes at once: the second wave has little or
+// nothing to do there and its LDS keeps other blocks out (us, 2 waves / 1: 1000
+// of 16 tokens, 32 heads 136 / 82, E4M3 130 / 72, of 32 E4M3 137 / 78; 512 of 64,
+// 16 heads 58 / 52; 256 of 16, 32 / 8 heads 16 / 12; level at 1024 blocks). Above,
+// the longest sequence's block takes its time (400 +- 60% of 4096 blocks 4% to
+// 10% slower).
 constexpr int WAVES = 2;
+constexpr long ONE_WAVE_BLOCKS = 2048;
+
+template <int D, int SRC, int PARTS, int NW>
+void launch_decode_waves(const DecodeArgs& p, int num_seqs, hipStream_t stream) {
+  const dim3 grid(p.Hkv, num_seqs, p.n_splits);
+  if (3 * p.group <= 16)
+    hipLaunchKernelGGL((paged_attention_kernel<D, NW, SRC, false, PARTS>), grid,
+                       dim3(NW * 64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((paged_attention_kernel<D, NW, SRC, true, PARTS>), grid,
+                       dim3(NW * 64), 0, stream, p);
+}
 
 template <int D, int SRC, int PARTS = 1>
 hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) {
-  const dim3 grid(p.Hkv, num_seqs, p.n_splits);
-  if (3 * p.group <= 16)
-    hipLaunchKernelGGL((paged_attention_kernel<D, WAVES, SRC, false, PARTS>), grid,
-                       dim3(WAVES * 64), 0, stream, p);
+  const bool few = p.max_blocks <= (SRC == PAGES_FP8 ? 8 : 4);
+  if (few && p.n_splits == 1 && (long)num_seqs * p.Hkv >= ONE_WAVE_BLOCKS)
+    launch_decode_waves<D, SRC, PARTS, 1>(p, num_seqs, stream);
   else
-    hipLaunchKernelGGL((paged_attention_kernel<D, WAVES, SRC, true, PARTS>), grid,
-                       dim3(WAVES * 64), 0, stream, p);
+    launch_decode_waves<D, SRC, PARTS, WAVES>(p, num_seqs, stream);
   HIP_CHECK_KERNEL();
   if (p.n_splits > 1) {
     const long sh = (long)num_seqs * p.H;

@@ -208,6 +208,57 @@ class TestDecodeAttention:
             assert (err <= 2 ** -8 * ref.abs() + 1e-5).all(), float(err.max())
             assert err.norm() < 2 ** -9 * ref.norm()
 
+    @pytest.mark.parametrize("window", [0, 20])
+    @pytest.mark.parametrize(
+        "H,Hkv,D,fp8", [(4, 4, 128, False), (8, 1, 128, False), (6, 3, 64, False),
+                        (4, 4, 128, True), (4, 1, 128, True)]
+    )
+    def test_one_wave_per_block(self, dev, H, Hkv, D, fp8, window):
+        """Tables of at most four pages (eight of E4M3) and just enough blocks for
+        the form with one wave, in both precisions of the scores."""
+        from kserve_amd import ops
+
+        ctx = [1, 15, 16, 17, 31, 32, 33, 48, 63, 64] + [65, 100, 127, 128] * fp8
+        torch.manual_seed(H + D)
+        width = -(-max(ctx) // 16)
+        NB = len(ctx) * width
+        kc, vc = (torch.randn(NB, Hkv, 16, D, device=dev).to(torch.bfloat16) for _ in "kv")
+        bt = torch.randperm(NB).view(len(ctx), width).to(torch.int32)
+        for row, c in zip(bt.long(), ctx):
+            for x in (kc, vc):  # rows that no sequence owns
+                x[row[-(-c // 16) :]] = float("nan")
+                if c % 16:
+                    x[row[c // 16], :, c % 16 :] = float("nan")
+        if fp8:
+            kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
+        ctx_t = torch.tensor(ctx, dtype=torch.int32)
+        q = (torch.randn(len(ctx), H, D, device=dev) * 1.5).to(torch.bfloat16)
+        ref = torch_ref.paged_attention_decode(
+            q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt, ctx_t,
+            D ** -0.5, window=window,
+        )
+        n = -(-2048 // (len(ctx) * Hkv))
+        many = [x.to(dev) for x in (bt.repeat(n, 1), ctx_t.repeat(n))]
+        got = ops.paged_attention_decode(
+            q.repeat(n, 1, 1), kc, vc, *many, D ** -0.5, window=window
+        )
+        for part in got.float().cpu().split(len(ctx)):
+            # fp32 weights and sums, the output rounded to bf16
+            err = (part - ref).abs()
+            assert (err <= 2 ** -8 * ref.abs() + 1e-5).all(), float(err.max())
+        if fp8:
+            return
+        rows = n * len(ctx)
+        cu = torch.arange(rows + 1, dtype=torch.int32, device=dev)
+        got = ops.ctx_attention_f32(
+            q.float().reshape(len(ctx), -1).repeat(n, 1), kc, vc, many[0], cu, many[1],
+            D ** -0.5, 1, H, window=window,
+        )
+        for part in got.cpu().split(len(ctx)):
+            # fp32 sums of at most 64 terms on both sides
+            err = (part - ref.reshape(len(ctx), -1)).norm() / ref.norm()
+            assert err < 1e-6, float(err)
+
 
 class TestPrefillAttention:
     @pytest.mark.parametrize(
