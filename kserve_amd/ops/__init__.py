@@ -711,7 +711,9 @@ def _scan_in_chunks(
     32 x 32 104 / 97, 128 x 32 371 / 395, 128 x 40 466 / 400; 16 heads of 64 x 16:
     32 x 24 15 / 15, 128 x 48 52 / 56, 256 x 56 99 / 110; 8 heads of 32 x 16, 256 x
     32 23 / 53, 64 x 80 27 / 23.)"""
-    longest = max(longest, -(-tokens // max(seqs, 1)))
+    if seqs == 0:
+        return False
+    longest = max(longest, -(-tokens // seqs))
     if longest < 16:
         return False
     cols = -(-P // 64)

@@ -56,3 +56,7 @@ def test_scan_in_chunks(lens, heads, P, N, chunks):
     assert ops._scan_in_chunks(
         sum(lens), len(lens), max(lens, default=0), heads, P, N
     ) is chunks
+
+
+def test_scan_of_no_sequences():
+    assert not ops._scan_in_chunks(100, 0, 100, 64, 64, 128)

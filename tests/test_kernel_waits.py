@@ -96,7 +96,7 @@ def test_prefill_attention_waits_for_lds_loads(tmp_path, fast_math):
         assert not unwaited_barriers(lines), name
 
 
-def test_checker_sees_a_skipped_wait():
+def test_skipped_wait_is_seen():
     body = """
  global_load_lds_dwordx4 v[2:3], off
  s_cbranch_vccz .LBB0_2
