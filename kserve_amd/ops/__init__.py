@@ -326,8 +326,9 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     need their second launch, k 1024 to 2048, m up to 256: at 48 rows 6.9 / 4.8;
     over 64 to 4096 x 16 to 8192 it takes 0.82 of the time; not everywhere ahead
     on wide ones past 16 rows: k 5120, m 27648 at 32 rows 57 / 53, at 48 rows 63 /
-    83), up to 64 rows but for the widest (m 14336 28.3 / 27.5). So far a row's sums do not depend on the rows
-    beside it, and small weights stay here for that. Above, it gains where the
+    83), up to 64 rows but for the widest (m 14336 28.3 / 27.5). So far a row's
+    sums do not depend on the rows beside it, and small weights stay here for
+    that. Above, it gains where the
     library does not split K over the chip: k 14336, m 4096 at 128 rows 35 / 76,
     k 4096, m 6144 22 / 26, k 3072, m 6144 20 / 21; and loses on short K (k 2048,
     m 8192 18.7 / 16.3, k 2560, m 8192 21.0 / 19.9), small weights (2048 x 2048
