@@ -4,14 +4,20 @@
 // softmax(logit/T) distribution exactly, without materializing probabilities
 // or sorting. Per-element U_i comes from a counter-based hash (seed, idx) so
 // the kernel is stateless and hipGraph-replayable.
-// (SURVEY.md §2.7 sampling row; north star: hand-written sampling kernel.)
 #include "common.h"
+
+#include <type_traits>
 
 namespace {
 
-// xxhash-like 2x32 mix: deterministic per (seed, idx)
-__device__ __forceinline__ unsigned int hash2(unsigned int a, unsigned int b) {
-  unsigned int h = a * 0x9E3779B1u + b * 0x85EBCA77u + 0x165667B1u;
+// xxhash-like 2x32 mix, deterministic per (seed, idx): hash_end of
+// hash_start(seed) + idx * HASH_STEP
+constexpr unsigned int HASH_STEP = 0x85EBCA77u;
+
+__device__ __forceinline__ unsigned int hash_start(unsigned int seed) {
+  return seed * 0x9E3779B1u + 0x165667B1u;
+}
+__device__ __forceinline__ unsigned int hash_end(unsigned int h) {
   h ^= h >> 15;
   h *= 0x2C1B3C6Du;
   h ^= h >> 12;
@@ -39,20 +45,36 @@ struct Bf16Row {
     const int tail0 = head + nvec * 8;
     ex = tid < head ? tid : (tid >= 8 && tail0 + tid - 8 < V) ? tail0 + tid - 8 : -1;
   }
-  // f(eight elements, index of the first) with four loads in flight, then
-  // one(element, index) for this thread's extra element
-  template <typename F, typename G>
-  __device__ __forceinline__ void each8(F f, G one) const {
+  // group(vectors, integral_constant of their number (4 or 1), index of the
+  // first element; the vectors are NT * 8 elements apart) by whole waves, with
+  // four loads in flight; rest(vector, index of its first element) for the last
+  // nvec % 64; then one(element, index) for this thread's extra element
+  template <typename F, typename R, typename G>
+  __device__ __forceinline__ void groups(F group, R rest, G one) const {
+    const int whole = nvec & ~63;
     int i = threadIdx.x;
-    for (; i + 3 * NT < nvec; i += 4 * NT) {
+    for (; i + 3 * NT < whole; i += 4 * NT) {
       short8_t v[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) v[u] = rv[i + u * NT];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) f(v[u], head + (i + u * NT) * 8);
+      group(v, std::integral_constant<int, 4>{}, head + i * 8);
     }
-    for (; i < nvec; i += NT) f(rv[i], head + i * 8);
+    for (; i < whole; i += NT) {
+      const short8_t v[1] = {rv[i]};
+      group(v, std::integral_constant<int, 1>{}, head + i * 8);
+    }
+    if (i < nvec) rest(rv[i], head + i * 8);
     if (ex >= 0) one(row[ex], ex);
+  }
+  // f(eight elements, index of the first)
+  template <typename F, typename G>
+  __device__ __forceinline__ void each8(F f, G one) const {
+    groups(
+        [&](const short8_t* v, auto count, int i0) {
+#pragma unroll
+          for (int u = 0; u < decltype(count)::value; ++u) f(v[u], i0 + u * NT * 8);
+        },
+        f, one);
   }
   template <typename F>
   __device__ __forceinline__ void each(F f) const {
@@ -91,11 +113,97 @@ __device__ __forceinline__ void block_argmax(float best, int best_idx, long* out
   }
 }
 
-__device__ __forceinline__ float gumbel_noise(unsigned int seed, int idx) {
-  const unsigned int h = hash2(seed, (unsigned int)idx);
+__device__ __forceinline__ float noise_of_hash(unsigned int h) {
   // u in (0,1): (h + 1) / 2^32
   const float u = ((float)h + 1.0f) * 2.3283064e-10f;
   return __logf(-__logf(u));
+}
+// Whether x / T + G can reach the best score that the wave has seen. With u = 1 -
+// r / 2^32 the noise is at most ln(2^32 / r), so an element whose r is above 2^32
+// exp(x / T - best) cannot. r's float pattern is a logarithm of it to within 0.09,
+// so the test is a multiply-add, two conversions and a compare beside the hash, in
+// place of two logarithms.
+//
+// Margin in log2: over all 2^32 hashes with r past 4096 (below, an element always
+// passes) pattern, u's rounding and the two hardware logarithms are off by 0.031 at
+// most; the rest of the 0.15 and the term in |best| are for the fp32 sums of scores.
+struct GumbelBound {
+  static constexpr float ONE = 8388608.f;  // 2^23: 1 in log2 as a pattern
+  float c1, c0 = 3e38f;                    // everything passes at first
+
+  __device__ __forceinline__ explicit GumbelBound(float inv_t)
+      : c1(inv_t * 1.44269504f * ONE) {}
+  __device__ __forceinline__ bool passes(float x, unsigned int hash) const {
+    const float r = (float)(~hash);
+    // at least the pattern of 4096, and within the range of an int
+    const float t = __builtin_amdgcn_fmed3f(x * c1 + c0, 1166016512.f, 2.1e9f);
+    return __builtin_bit_cast(int, r) <= (int)t;
+  }
+  // by a whole wave
+  __device__ __forceinline__ void raise(float best) {
+    const float b = fminf(wave_reduce_max(best), 1e30f);
+    c0 = (32.f + 127.f - b * 1.44269504f + (0.15f + 2e-6f * fabsf(b))) * ONE;
+  }
+};
+
+// A thread's part of argmax(x / T + G) over a whole row, ties to the lower index.
+// Bound by arithmetic, 20 operations an element with the hash's two multiplies at
+// a quarter of the rate. 256 x 128256: 37.7 us with two logarithms for every
+// element, 26.9 with the bound; 256 x 32000 17.1 -> 13.1. Blocks of few waves walk
+// short rows, where the score to beat is found too late to pay for the bound.
+template <int NT>
+__device__ __forceinline__ void gumbel_row(const Bf16Row<NT>& row, const float inv_t,
+                                           const unsigned int seed, float& best,
+                                           int& best_idx) {
+  const unsigned int h0 = hash_start(seed);
+  GumbelBound bound(inv_t);
+  bool started = false;
+  auto take = [&](float x, unsigned int h, int i) {
+    const float val = x * inv_t - noise_of_hash(h);
+    if (val > best || (val == best && i < best_idx)) {
+      best = val;
+      best_idx = i;
+    }
+  };
+  auto vec = [&](const short8_t& v, const int i0) {
+    const unsigned int hi = h0 + (unsigned int)i0 * HASH_STEP;
+    if (!started) {  // the wave's first elements give it a score to beat
+      take(bf16_bits_to_float(v[0]), hash_end(hi), i0);
+      bound.raise(best);
+      started = true;
+    }
+    unsigned int in = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      in |= (bound.passes(bf16_bits_to_float(v[j]), hash_end(hi + j * HASH_STEP)) ? 1u : 0u)
+            << j;
+    if (__ballot(in != 0)) {
+      while (in) {
+        const int j = __builtin_ctz(in);
+        in &= in - 1;
+        short b = v[0];
+#pragma unroll
+        for (int q = 1; q < 8; ++q) b = j == q ? v[q] : b;
+        take(bf16_bits_to_float(b), hash_end(hi + j * HASH_STEP), i0 + j);
+      }
+      bound.raise(best);
+    }
+  };
+  // the wave's maximum takes whole waves: the rest is evaluated in full
+  row.groups(
+      [&](const short8_t* v, auto count, int i0) {
+#pragma unroll
+        for (int u = 0; u < decltype(count)::value; ++u) vec(v[u], i0 + u * NT * 8);
+      },
+      [&](const short8_t& v, int i0) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          take(bf16_bits_to_float(v[j]),
+               hash_end(h0 + (unsigned int)(i0 + j) * HASH_STEP), i0 + j);
+      },
+      [&](short b, int i) {
+        take(bf16_bits_to_float(b), hash_end(h0 + (unsigned int)i * HASH_STEP), i);
+      });
 }
 
 // logits bf16 [S, V]; one block of NT threads per row.
@@ -108,41 +216,36 @@ __global__ __launch_bounds__(NT) void argmax_kernel(
     const int V) {
   const int s = blockIdx.x;
   const short* row = logits + (long)s * V;
+
   const float inv_t = GUMBEL ? 1.f / fmaxf(temperatures[s], 1e-5f) : 1.f;
   const unsigned int seed = GUMBEL ? (unsigned int)(seeds[s] & 0xFFFFFFFF) : 0;
 
   float best = -1e38f;
   int best_idx = 0;
-  // vectorized short8 loads over the vocab row
-  const int nvec = V >> 3;
-  const short8_t* rv = reinterpret_cast<const short8_t*>(row);
-  for (int i = threadIdx.x; i < nvec; i += NT) {
-    short8_t v = rv[i];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int idx = i * 8 + j;
-      float val = bf16_bits_to_float(v[j]);
+  if constexpr (GUMBEL && NT >= 1024) {
+    gumbel_row<NT>(Bf16Row<NT>(row, V), inv_t, seed, best, best_idx);
+  } else {
+    auto take = [&](short b, int idx) {
+      float val = bf16_bits_to_float(b);
       if constexpr (GUMBEL) {
         val *= inv_t;
-        val -= gumbel_noise(seed, idx);
+        val -= noise_of_hash(hash_end(hash_start(seed) + (unsigned int)idx * HASH_STEP));
       }
-      if (val > best) {
+      if (val > best) {  // a thread's indexes only grow
         best = val;
         best_idx = idx;
       }
+    };
+    // vectorized short8 loads over the vocab row
+    const int nvec = V >> 3;
+    const short8_t* rv = reinterpret_cast<const short8_t*>(row);
+    for (int i = threadIdx.x; i < nvec; i += NT) {
+      const short8_t v = rv[i];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) take(v[j], i * 8 + j);
     }
-  }
-  // tail (V not divisible by 8)
-  for (int idx = nvec * 8 + threadIdx.x; idx < V; idx += NT) {
-    float val = bf16_bits_to_float(row[idx]);
-    if constexpr (GUMBEL) {
-      val *= inv_t;
-      val -= gumbel_noise(seed, idx);
-    }
-    if (val > best) {
-      best = val;
-      best_idx = idx;
-    }
+    // tail (V not divisible by 8)
+    for (int idx = nvec * 8 + threadIdx.x; idx < V; idx += NT) take(row[idx], idx);
   }
   block_argmax<NT>(best, best_idx, out + s);
 }
@@ -228,20 +331,54 @@ __global__ __launch_bounds__(AM_NT) void argmax_f32_kernel(
 // coarser histograms find it: the keys' upper 12 bits, then the lower 4 inside
 // the bin that the limit falls into.
 //
-// What bounds it: one pass of LDS atomics, an exponential per element and the
-// three passes over the row, which come from the L2 and the memory-side cache.
-// A histogram over the keys' upper byte puts a model's logits into half a
-// dozen bins and serialises a wave's 64 adds, for count and mass each. Rows of
-// N(0, 2.5) logits, top-k and top-p mixed, that form -> this one: 256 x 128256
-// 704 -> 78 us, 256 x 32000 141 -> 34 us, 1 x 128256 465 -> 44 us; limits
-// below the window (k of the order of the row) 702 -> 156 us. Holding the row
-// in registers over the passes is not faster (80 us). Rows with nothing to cut
-// go straight to the last pass (256 x 128256: 38 us; the plain kernel's 31 need
-// the host to know that no row has a limit, a synchronisation of 15).
+// The usual row takes one pass for all of it ("first pass"): counts of the keys
+// between 2^-16 and 2^16 of either sign in 8193 bins (those closer to 0 share one)
+// and the first and last bin, by 16-bit packed operations while the row comes from
+// memory. The mass is formed from the counts, and the bins are scanned from the
+// row's largest, 1024 at a time, until both limits are found; one scan nearly always
+// does. Rows with NaNs or numbers past 2^16, and limits
+// among the numbers closer to 0 than 2^-16 go through the passes above.
+//
+// The last pass queues a wave's survivors in LDS and evaluates them 64 at a time,
+// so a set of any density costs what it holds.
+//
+// What bounds it: the first pass runs at memory speed (8 operations an element
+// hide under it), the last at the vector units' and the queue's. Rows of N(0, 2.5)
+// logits, one per compute unit (us, three passes / this): 256 x 128256 top-p 0.9 75
+// / 41, top-k 50 49 / 29, both 52 / 30; 15 x 128256 66 / 34, 40 / 20, 45 / 22; 256 x
+// 32000 33 / 20, 23 / 14, 29 / 16; limits below zero 131 / 68 (a histogram by the
+// keys' upper byte took 704 at 256 x 128256). Holding the row in registers over the
+// passes was no faster.
 // ---------------------------------------------------------------------------
 constexpr int RT = 1024;
 constexpr int WIN = 16384;
 constexpr int KBINS = 4096;
+
+// First pass: a 16-bit pattern as a signed number in the logits' order, with the
+// patterns of +-2^-16 .. 0 taken out of the middle: bin FSPAN - that, FBINS in all
+constexpr int FSPAN = 4096, FBINS = 2 * FSPAN + 1;
+constexpr short NEAR_HI = 0x377f, NEAR_LO = -0x3780;
+constexpr int MINUS_INF_BIN = FSPAN + 0x7f81 + NEAR_LO;
+typedef short short2_v __attribute__((ext_vector_type(2)));
+typedef unsigned short ushort2_v __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ short2_v ordered(short2_v b) {
+  const short2_v sign = b >> 15;
+  return b ^ __builtin_bit_cast(short2_v, __builtin_bit_cast(ushort2_v, sign) >> 1);
+}
+__device__ __forceinline__ ushort2_v first_bin(short2_v s) {
+  const short2_v lo = {NEAR_LO, NEAR_LO}, hi = {NEAR_HI, NEAR_HI};
+  const short2_v mid = __builtin_elementwise_min(__builtin_elementwise_max(s, lo), hi);
+  return __builtin_bit_cast(ushort2_v, (short2_v)(short2_v{FSPAN, FSPAN} - (s - mid)));
+}
+// the number of an ordered pattern, and the ordered pattern of a bin
+__device__ __forceinline__ float ordered_value(int s) {
+  return bf16_bits_to_float((short)(s ^ ((s >> 15) & 0x7fff)));
+}
+__device__ __forceinline__ int bin_ordered(int bin) {
+  const int d = FSPAN - bin;
+  return d > 0 ? d + NEAR_HI : d < 0 ? d + NEAR_LO : 0;
+}
 
 __device__ __forceinline__ unsigned int bf16_sort_key(short bits) {
   const unsigned short u = (unsigned short)bits;
@@ -308,6 +445,7 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
   const int lane = tid & 63, wave = tid >> 6;
   constexpr int NWV = RT / 64;
   constexpr int NONE = 0x7fffffff;
+  constexpr int QUEUE = 63 + 8 * 64;  // survivors of a wave on their way
 
   __shared__ union {
     unsigned int win[WIN];
@@ -315,6 +453,7 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
       unsigned int cnt[KBINS];
       u64 mass[KBINS];
     } h;
+    uint2 queue[NWV][QUEUE];
   } lds;
   __shared__ unsigned int f_cnt[16];
   __shared__ u64 f_mass[16];
@@ -331,6 +470,127 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
   const Bf16Row<RT> row(logits + (long)s * V, V);
   unsigned int thr = 0;
   if (use_k || use_p) {
+    // ---- first pass: counts per bin, extremes, mass ----
+    for (int i = tid; i < FBINS; i += RT) lds.win[i] = 0;
+    if (tid < 4) sh_bin[tid] = NONE;
+    __syncthreads();
+    const float c2 = inv_t * 1.44269504f;
+    ushort2_v lo2 = {65535, 65535}, hi2 = {0, 0};  // first and last bin
+    auto add = [&](short2_v b) {
+      const ushort2_v at = first_bin(ordered(b));
+      lo2 = __builtin_elementwise_min(lo2, at);
+      hi2 = __builtin_elementwise_max(hi2, at);
+      if (at.x < FBINS) atomicAdd(&lds.win[at.x], 1u);
+      if (at.y < FBINS) atomicAdd(&lds.win[at.y], 1u);
+    };
+    auto add8 = [&](const short8_t& v, int) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) add(short2_v{v[2 * q], v[2 * q + 1]});
+    };
+    row.each8(add8, [&](short b, int) {
+      const unsigned short at = first_bin(ordered(short2_v{b, b})).x;
+      lo2 = __builtin_elementwise_min(lo2, ushort2_v{at, at});
+      hi2 = __builtin_elementwise_max(hi2, ushort2_v{at, at});
+      if (at < FBINS) atomicAdd(&lds.win[at], 1u);
+    });
+    unsigned int lo = min((unsigned int)lo2.x, (unsigned int)lo2.y);
+    unsigned int hi = max((unsigned int)hi2.x, (unsigned int)hi2.y);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      lo = min(lo, (unsigned int)__shfl_xor((int)lo, off, 64));
+      hi = max(hi, (unsigned int)__shfl_xor((int)hi, off, 64));
+    }
+    if (lane == 0) {
+      s_key[wave] = lo;
+      s_bad[wave] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NWV; ++w) {
+      lo = min(lo, s_key[w]);
+      hi = max(hi, s_bad[w]);
+    }
+    // past the last bin come numbers below -2^16, -inf, NaNs, then what is above
+    // 2^16; the largest number has a bin
+    const bool direct = hi <= MINUS_INF_BIN && lo < FBINS;
+    const float most = direct ? ordered_value(bin_ordered(lo)) : 0.f;
+    auto weight_of_bin = [&](int bin) {
+      return (double)__builtin_amdgcn_exp2f((ordered_value(bin_ordered(bin)) - most) * c2);
+    };
+    if (direct) {
+      double zz = 0;
+      if (use_p) {
+#pragma unroll
+        for (int i = 0; i < (FBINS + RT - 1) / RT; ++i) {
+          const int bin = tid + i * RT;
+          const unsigned int n = bin < FBINS ? lds.win[bin] : 0u;
+          if (n) zz += n * weight_of_bin(bin);
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) zz += __shfl_xor(zz, off, 64);
+        if (lane == 0) w_mass[wave] = zz;
+        __syncthreads();
+        zz = 0;
+#pragma unroll
+        for (int w = 0; w < NWV; ++w) zz += w_mass[w];
+      }
+      const double want = (double)p * zz;
+      bool find_k = use_k, find_p = use_p && want > 0;
+      unsigned int over_k = 0;  // elements and mass of the bins before
+      double over_p = 0;
+      for (int b0 = lo; b0 < FBINS && (find_k || find_p); b0 += RT) {
+        __syncthreads();  // the sums of the round before are read
+        const int bin = b0 + tid;
+        const unsigned int n = bin < FBINS ? lds.win[bin] : 0u;
+        const double m = find_p && n ? n * weight_of_bin(bin) : 0.0;
+        unsigned int nk = n;
+        double mp = m;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const unsigned int a = __shfl_up(nk, off, 64);
+          const double b = __shfl_up(mp, off, 64);
+          if (lane >= off) {
+            nk += a;
+            mp += b;
+          }
+        }
+        if (lane == 63) {
+          w_cnt[wave] = nk;
+          w_mass[wave] = mp;
+        }
+        __syncthreads();
+        unsigned int ck = over_k + nk - n;
+        double cp = over_p + (mp - m);
+#pragma unroll
+        for (int w = 0; w < NWV; ++w) {
+          ck += w < wave ? w_cnt[w] : 0u;
+          cp += w < wave ? w_mass[w] : 0.0;
+          over_k += w_cnt[w];
+          over_p += w_mass[w];
+        }
+        // the first bin at which the running sum reaches its target; in
+        // floating point a thread's end need not be the next one's start
+        if (find_k && n && ck < (unsigned int)k && ck + n >= (unsigned int)k)
+          atomicMin(&sh_bin[0], bin);
+        if (find_p && n && cp < want && cp + m >= want) atomicMin(&sh_bin[1], bin);
+        __syncthreads();
+        if (sh_bin[0] != NONE) find_k = false;
+        if (sh_bin[1] != NONE) find_p = false;
+      }
+      // the smaller bin is the higher limit; a limit that was not found lies
+      // below one that was
+      const int bin = min(sh_bin[0], sh_bin[1]);
+      // What the mass is not exact in has to be nothing beside it: numbers closer
+      // to 0 than 2^-16 (known to 2^-16 / T of theirs) and those below -2^16.
+      const double off =
+          lds.win[FSPAN] * weight_of_bin(FSPAN) * c2 * 1.6e-5 +
+          (hi < FBINS ? 0.0 : V * (double)__builtin_amdgcn_exp2f((-65536.f - most) * c2));
+      if (bin != NONE && bin != FSPAN && (!use_p || off <= 3e-8 * zz))
+        thr = (unsigned int)(bin_ordered(bin) + 32768);
+    }
+    __syncthreads();
+  }
+  if ((use_k || use_p) && thr == 0) {
     // ---- largest number (exp stability), and whether a mass can be formed ----
     unsigned int mk = 0;
     unsigned int bad = 0;  // a NaN or +inf: no mass, as its sum would be NaN
@@ -468,48 +728,95 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
     }
   }
 
-  // ---- Gumbel-argmax over the surviving set: the lanes of a wave go through
-  // their own survivors, so a sparse set costs few rounds of hash and logs ----
+  // ---- Gumbel-argmax over the surviving set ----
   float best = -1e38f;
   int best_idx = 0;
-  auto take = [&](short b, int i) {
+  if (thr == 0 && k != 1) {
+    gumbel_row<RT>(row, inv_t, seed, best, best_idx);
+  } else {
+    const unsigned int h0 = hash_start(seed);
+    GumbelBound bound(inv_t);
     // top-k of one is the greedy choice, ties included: no noise
-    float val = bf16_bits_to_float(b) * inv_t;
-    if (k != 1) val -= gumbel_noise(seed, i);
-    if (val > best || (val == best && i < best_idx)) {
-      best = val;
-      best_idx = i;
+    auto take = [&](float x, unsigned int h, int i) {
+      const float val = k == 1 ? x * inv_t : x * inv_t - noise_of_hash(h);
+      if (val > best || (val == best && i < best_idx)) {
+        best = val;
+        best_idx = i;
+      }
+    };
+    auto take_one = [&](short b, int i) {
+      if (bf16_sort_key(b) >= thr)
+        take(bf16_bits_to_float(b), hash_end(h0 + (unsigned int)i * HASH_STEP), i);
+    };
+    __syncthreads();  // the counts are read
+    uint2* queue = lds.queue[wave];
+    int queued = 0;
+    auto drain = [&](int from) {  // 64 of the queue, by a whole wave
+      const uint2 e = queue[from + lane];
+      const float x = __builtin_bit_cast(float, e.y);
+      const unsigned int h = hash_end(h0 + e.x * HASH_STEP);
+      if (__ballot(k == 1 || bound.passes(x, h))) {
+        take(x, h, (int)e.x);
+        if (k != 1) bound.raise(best);
+      }
+    };
+    // key >= thr as one unsigned comparison per half of a dword: the patterns
+    // of positive limits are ordered once the sign is flipped, those of negative
+    // ones once all bits are (positive numbers come out on top either way)
+    const bool pos = thr & 0x8000u;
+    const unsigned int flip = pos ? 0x80008000u : 0xffffffffu;
+    const unsigned int lim = thr;
+    row.groups(
+        [&](const short8_t* v, auto count, int i0) {
+#pragma unroll
+          for (int u = 0; u < decltype(count)::value; ++u) {
+            const uint4 d = __builtin_bit_cast(uint4, v[u]);
+            const unsigned int dw[4] = {d.x, d.y, d.z, d.w};
+            ushort2_v m = {0, 0};
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              m = __builtin_elementwise_max(
+                  m, __builtin_bit_cast(ushort2_v, dw[q] ^ flip));
+            if (!__ballot(max((unsigned int)m.x, (unsigned int)m.y) >= lim)) continue;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const unsigned int w = dw[j / 2] ^ flip;
+              const bool in = j & 1 ? w >= lim << 16
+                                    : (unsigned short)w >= (unsigned short)lim;
+              const u64 set = __ballot(in);
+              if (set) {
+                if (in)
+                  queue[queued + __builtin_amdgcn_mbcnt_hi(
+                                     (unsigned int)(set >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((unsigned int)set, 0))] =
+                      uint2{(unsigned int)(i0 + u * RT * 8 + j),
+                            j & 1 ? dw[j / 2] & 0xffff0000u : dw[j / 2] << 16};
+                queued += __builtin_popcountll(set);
+              }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            while (queued >= 64) drain(queued -= 64);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          }
+        },
+        [&](const short8_t& v, int i0) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) take_one(v[j], i0 + j);
+        },
+        take_one);
+    if (lane < queued) {
+      const uint2 e = queue[lane];
+      take(__builtin_bit_cast(float, e.y), hash_end(h0 + e.x * HASH_STEP), (int)e.x);
     }
-  };
-  row.each8(
-      [&](const short8_t& v, int i0) {
-        if (thr == 0) {  // nothing cut: every element, without the detour
-#pragma unroll
-          for (int j = 0; j < 8; ++j) take(v[j], i0 + j);
-          return;
-        }
-        unsigned int in = 0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) in |= (bf16_sort_key(v[j]) >= thr ? 1u : 0u) << j;
-        while (in) {
-          const int j = __builtin_ctz(in);
-          in &= in - 1;
-          short b = v[0];
-#pragma unroll
-          for (int q = 1; q < 8; ++q) b = j == q ? v[q] : b;
-          take(b, i0 + j);
-        }
-      },
-      [&](short b, int i) {
-        if (bf16_sort_key(b) >= thr) take(b, i);
-      });
+  }
   block_argmax<RT>(best, best_idx, out + s);
 }
 
 // 1024 threads for rows past 64k elements (256 rows of 128256, greedy 24.7 ->
-// 12.3 us, with noise 36.5 -> 30.8); shorter rows are over before a block that
+// 12.3 us, with noise 36.5 -> 26.2); shorter rows are over before a block that
 // size has merged its waves (256 x 32000, greedy: 5.9 us with 256 threads, 7.0
-// with 1024)
+// with 1024; with noise 10.5 with 256 threads that evaluate every element, 11.9
+// with 512 and the bound)
 template <bool GUMBEL>
 void launch_argmax(void* out, const void* logits, const void* temperatures,
                    const void* seeds, int num_seqs, int vocab, hipStream_t stream) {

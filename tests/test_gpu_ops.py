@@ -762,6 +762,70 @@ class TestSampling:
             assert x[r][got] >= least, (r, got)
             assert s[got] >= s.max() - 1e-4, (r, got, int(s.argmax()))
 
+    @pytest.mark.parametrize(
+        "mode", ["near_zero", "huge", "lowest", "below_zero", "zeros", "warm"]
+    )
+    @pytest.mark.parametrize("vocab", [9, 1031, 8200, 40003])
+    def test_limits_of_the_first_pass(self, dev, vocab, mode):
+        """Rows at the edges of the bins from 2^-16 to 2^16: limits closer to 0,
+        numbers past the bins on either side, limits among negative numbers,
+        survivors from a handful to nearly all. Every token is one that the
+        float64 limits leave, and the best of them by the kernel's noise."""
+        import kserve_amd_C
+
+        n = 8
+        g = torch.Generator().manual_seed(vocab)
+        logits = torch.randn(n, vocab, generator=g) * 2.5
+        top_p = torch.tensor([1.0, 0.9, 0.99, 0.5] * 2)
+        top_k = torch.tensor([5, 0, 40, 0, 0, 3, 0, 1000], dtype=torch.int32)
+        temps = torch.rand(n, generator=g) * 0.6 + 0.6
+        if mode == "near_zero":
+            logits = logits * 1e-6
+        if mode == "huge":
+            logits, temps = logits * 4e4, temps * 3e4
+        if mode == "lowest":
+            logits[:, ::3] = torch.finfo(torch.bfloat16).min
+            logits[1, 1:] = float("-inf")
+        if mode == "below_zero":
+            logits = logits - 20.0
+        if mode == "zeros":
+            logits[:, ::2] = 0.0
+        if mode == "warm":
+            temps = temps * 40
+        logits = logits.to(torch.bfloat16)
+        seeds = torch.randint(0, 1 << 31, (n,), generator=g)
+        out = torch.empty(n, dtype=torch.int64, device=dev)
+        kserve_amd_C.topk_topp_sample(
+            out, logits.to(dev), temps.to(dev), top_p.to(dev), top_k.to(dev),
+            seeds.to(dev),
+        )
+        M = 0xFFFFFFFF
+        h = ((seeds[:, None] * 0x9E3779B1) & M) + ((torch.arange(vocab) * 0x85EBCA77) & M)
+        h = (h + 0x165667B1) & M
+        for mul, shift in ((0x2C1B3C6D, 12), (0x297A2D39, 15)):
+            h = ((h ^ (h >> 15)) * mul & M) if shift == 12 else h * mul & M
+            h = h ^ (h >> shift)
+        u = (h.float() + 1.0) * 2.3283064e-10
+        x = logits.double() / temps[:, None].double()
+        score = x - torch.log(-torch.log(u.double()))
+        for r in range(n):
+            vals, order = x[r].sort(descending=True)
+            least = torch.tensor([float("-inf")], dtype=torch.float64)
+            if 0 < top_k[r] < vocab:
+                least = vals[top_k[r] - 1 : top_k[r]]
+            if top_p[r] < 1:
+                c = torch.softmax(x[r], 0)[order].cumsum(0)
+                # either side of the limit where the sum meets it within its rounding
+                at = [int((c < float(top_p[r]) * f).sum()) for f in (1 - 1e-6, 1 + 1e-6)]
+                ps = vals[[min(a, vocab - 1) for a in at]]
+                least = torch.maximum(least, ps)
+            got = int(out[r])
+            assert x[r][got] >= least.min(), (r, got)
+            s = score[r].masked_fill(x[r] < least.max(), float("-inf"))
+            # fast fp32 logarithms and the fp32 score itself: a few ulp of it
+            near = 1e-4 + 4 * 2.0 ** -24 * float(x[r][got].abs())
+            assert s.max() <= score[r][got] + near, (r, got, int(s.argmax()))
+
     @pytest.mark.parametrize("vocab", [5, 32000, 70001])
     def test_topk1_ties_are_greedy(self, dev, vocab):
         """Equal largest logits: top_k 1 takes the one that greedy takes."""
