@@ -1008,7 +1008,7 @@ extern "C" int ks_ctx_attention_mfma(const void* out, const void* q,
                                      int maps, float softcap, int keep_first) {
   return !is_f32 && (D == 64 || D == 128) && DV == D && maps == 1 &&
          block_size == mfma_attn::PAGE && softcap == 0.f && !out_inv_freq &&
-         keep_first == 0 && v_row_stride % 8 == 0 &&
+         keep_first == 0 && v_row_stride % 8 == 0 && v_row_stride < (1L << 26) &&
          (max_q_len > 1 || heads / (kv_heads > 0 ? kv_heads : 1) <= 8) &&
          (((uintptr_t)out | (uintptr_t)q | (uintptr_t)k_cache |
            (uintptr_t)v_cache) & 15) == 0;
@@ -1041,7 +1041,8 @@ static hipError_t ctx_attention_mfma(const CtxArgs& a) {
   const PrefillArgs p{a.out, a.q, a.k_cache, a.v_cache, (const int*)a.cu_q,
                       (const int*)a.ctx_lens, (const int*)a.block_tables,
                       a.heads, a.kv_heads, a.bt_stride, hpb, score_scale(a.scale),
-                      (long)a.heads * a.D, a.D, a.v_row_stride, a.window, x};
+                      (long)a.heads * a.D, a.D, a.v_row_stride, a.window, x,
+                      1, 0, nullptr, nullptr};
   const dim3 grid(a.heads / hpb, cdiv(a.max_q_len, NWAVES * QW / hpb), a.num_seqs);
 #define GO(DD, WW)                                                             \
   hipLaunchKernelGGL((prefill_attention_kernel<DD, PAGES_DMA, true, WW, 3>),   \

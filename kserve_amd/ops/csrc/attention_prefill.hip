@@ -14,22 +14,26 @@
 // A block is 4 waves of 32 queries and shares double-buffered tiles of 64 keys
 // that the LDS-direct loads fill while the other buffer is computed on (they run
 // under K Q^T and the softmax: the compiler waits for them ahead of the
-// transposing reads of V); the XOR swizzles are on the source side of those
-// loads. With several query
-// heads per KV head the waves take up to four heads of one group over the same
-// queries (equal causal ranges, and a K/V tile is fetched once for the group);
-// otherwise consecutive queries of one head.
+// transposing reads of V; without that wait it moves those reads up and the tile
+// takes 10% longer); the XOR swizzles are on the source side of those loads. With
+// several query heads per KV head the waves take up to four heads of one group
+// over the same queries (equal causal ranges, and a K/V tile is fetched once for
+// the group); otherwise consecutive queries of one head. Few queries behind a long
+// context are split over its keys.
 //
-// What bounds it: per 64 keys and 32 queries a wave issues 32 MFMAs (1024
-// cycles of its matrix core), reads 32 KB of LDS operands (a quarter of the
-// LDS bandwidth for the same time, times four waves) and has 32 exponentials
-// and about 130 further vector instructions per lane; two waves per SIMD
-// overlap the three. Measured (32 query and 8 KV heads of 128, causal; the
-// 16x16x32 kernel with one head per block, V transposed by 2-byte LDS stores and
-// a barrier on each side of the staging, before this one): 1 x 8191 tokens
-// 2497 -> 597 us (220 -> 921 TFLOP/s), 8 x 2048 1280 -> 365 us, 32 x 512
-// 413 -> 141 us; 2 x 1000 queries over 13000 paged keys 2441 -> 460 us (E4M3
-// pages 2596 -> 557); 64 x 128, 12 heads of 64, bidirectional 28 -> 12 us.
+// What bounds it: per 64 keys and 32 queries a wave issues 32 MFMAs (1024 cycles of
+// its matrix core), reads 32 KB of LDS operands (256 cycles of the unit's LDS, for 8
+// waves as much as the products of two) and has 32 exponentials and about 130 further
+// vector instructions per lane (1050 cycles); two waves per SIMD overlap the three.
+// The sign of the scale in the query, the exponent as one multiply-add, a maximum
+// that is followed in steps of 2^8, tile addresses from scalars, and keys read six
+// products ahead took 700 vector cycles and most waits off a tile. Measured (32 query
+// and 8 KV heads of 128, causal; the 16x16x32 kernel with one head per block before,
+// then before and with those): 1 x 8191 tokens 2497 / 620 / 518 us (1060 TFLOP/s), 8 x
+// 2048 1280 / 367 / 319 us, 16 x 500 74 / 67 us; 2 x 1000 queries over 13000 paged
+// keys 2441 / 479 / 420 us (E4M3 pages 2596 / 572 / 500); 8 x 500, 12 heads of 64,
+// bidirectional 18 / 15 us, 64 x 128 level at 13; fp32 scores, 4 x 2000, 16 / 4 heads
+// 239 / 223 us.
 //
 // Replaces the vLLM flash prefill the reference delegates to. Numerics oracles:
 // ops/torch_ref.flash_prefill_varlen and context_attention_varlen.
@@ -39,15 +43,17 @@ namespace {
 
 using namespace mfma_attn;
 
+// query heads that a block takes
+int heads_per_block(int group) { return group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1; }
+
 template <int D, int SRC>
 hipError_t launch(PrefillArgs p, int num_seqs, int max_q_len, bool causal,
                   hipStream_t stream) {
-  const int group = p.Hq / p.Hkv;
-  p.hpb = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
+  p.hpb = heads_per_block(p.Hq / p.Hkv);
   const int qpb = NWAVES * QW / p.hpb;
   const int tiles = (max_q_len + qpb - 1) / qpb;
   if (tiles == 0 || num_seqs == 0) return hipSuccess;
-  const dim3 grid(p.Hq / p.hpb, tiles, num_seqs);
+  const dim3 grid(p.Hq / p.hpb, tiles, num_seqs * p.n_splits);
 #define GO(CC, WW)                                                             \
   hipLaunchKernelGGL((prefill_attention_kernel<D, SRC, CC, WW>), grid,         \
                      dim3(256), 0, stream, p)
@@ -64,6 +70,12 @@ hipError_t launch(PrefillArgs p, int num_seqs, int max_q_len, bool causal,
   }
 #undef GO
   HIP_CHECK_KERNEL();
+  if (p.n_splits > 1) {
+    hipLaunchKernelGGL(prefill_attention_merge_kernel, dim3((unsigned)((p.rows + 7) / 8)),
+                       dim3(256), 0, stream, (short*)p.out, p.part_out, p.part_ml,
+                       p.n_splits, p.rows);
+    HIP_CHECK_KERNEL();
+  }
   return hipSuccess;
 }
 
@@ -73,17 +85,31 @@ bool aligned16(const void* a, const void* b) {
 
 }  // namespace
 
+// key parts for such a call (what its workspace is sized for)
+extern "C" int ks_context_prefill_splits(int num_seqs, long rows, int max_q_len, int Hq,
+                                         int Hkv, int max_nb, int window) {
+  if (num_seqs < 1 || max_q_len < 1 || Hkv < 1 || Hq % Hkv != 0) return 1;
+  const int hpb = heads_per_block(Hq / Hkv), qpb = NWAVES * QW / hpb;
+  const long blocks = (long)(Hq / hpb) * ((max_q_len + qpb - 1) / qpb) * num_seqs;
+  long keys = (long)max_nb * PAGE;
+  if (window > 0 && keys > (long)window + qpb) keys = (long)window + qpb;
+  return prefill_splits(blocks, (int)((keys + KT - 1) / KT), rows);
+}
+
 extern "C" hipError_t ks_context_prefill_varlen(
     void* out, const void* q, const void* k_cache, const void* v_cache,
     const void* block_tables, const void* ctx_lens, const void* cu_seqlens_q,
     int num_seqs, int max_q_len, int Hq, int Hkv, int head_dim, int max_nb,
-    float scale, long sq, int fp8_cache, int window, hipStream_t stream) {
+    float scale, long sq, int fp8_cache, int window, long rows, int n_splits,
+    void* part_out, void* part_ml, hipStream_t stream) {
   if (head_dim != 128) return hipErrorInvalidValue;
+  if (n_splits < 1 || !part_out || !part_ml) n_splits = 1;
   if (Hq % Hkv != 0) return hipErrorInvalidValue;
   PrefillArgs p{out, q, k_cache, v_cache,
                 (const int*)cu_seqlens_q, (const int*)ctx_lens,
                 (const int*)block_tables, Hq, Hkv, max_nb, 1, score_scale(scale), sq,
-                head_dim, head_dim, window, Extra{}};
+                head_dim, head_dim, window, Extra{}, n_splits, rows,
+                (float*)part_out, (float*)part_ml};
   if (fp8_cache) return launch<128, PAGES_FP8>(p, num_seqs, max_q_len, true, stream);
   if (aligned16(k_cache, v_cache))
     return launch<128, PAGES_DMA>(p, num_seqs, max_q_len, true, stream);
@@ -99,7 +125,8 @@ extern "C" hipError_t ks_flash_prefill_varlen(
   if (Hq % Hkv != 0) return hipErrorInvalidValue;
   PrefillArgs p{out, q, k, v, (const int*)cu_seqlens,
                 nullptr, nullptr, Hq, Hkv, 0, 1, score_scale(scale), sq, sk, sv, window,
-                Extra{}};
+                Extra{}, 1, 0, nullptr, nullptr};
+  if (sk >= 1L << 26 || sv >= 1L << 26) return hipErrorInvalidValue;
   // LDS-direct loads move 16 aligned bytes per lane
   const bool dma = aligned16(k, v) && sk % 8 == 0 && sv % 8 == 0;
   if (head_dim == 128) {

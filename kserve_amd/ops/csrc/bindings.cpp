@@ -27,8 +27,9 @@ hipError_t ks_flash_prefill_varlen(void*, const void*, const void*,
 hipError_t ks_context_prefill_varlen(void*, const void*, const void*,
                                      const void*, const void*, const void*,
                                      const void*, int, int, int, int, int,
-                                     int, float, long, int, int,
-                                     hipStream_t);
+                                     int, float, long, int, int, long, int,
+                                     void*, void*, hipStream_t);
+int ks_context_prefill_splits(int, long, int, int, int, int, int);
 hipError_t ks_reshape_and_cache_fp8(const void*, const void*, void*, void*,
                                     const void*, int, int, int, int, long,
                                     long, hipStream_t);
@@ -206,11 +207,14 @@ void flash_prefill_varlen(at::Tensor& out, at::Tensor& q, at::Tensor& k,
   int Hq = q.size(1);
   int Hkv = k.size(1);
   int D = q.size(2);
-  check_hip(ks_flash_prefill_varlen(out.data_ptr(), q.data_ptr(), k.data_ptr(),
-                                    v.data_ptr(), cu_seqlens.data_ptr(),
+  // the kernel's lane offsets are 32 bits wide
+  const at::Tensor kk = k.stride(0) < (1L << 26) ? k : k.contiguous();
+  const at::Tensor vv = v.stride(0) < (1L << 26) ? v : v.contiguous();
+  check_hip(ks_flash_prefill_varlen(out.data_ptr(), q.data_ptr(), kk.data_ptr(),
+                                    vv.data_ptr(), cu_seqlens.data_ptr(),
                                     num_seqs, (int)max_seqlen, Hq, Hkv, D,
                                     (float)scale, (long)q.stride(0),
-                                    (long)k.stride(0), (long)v.stride(0),
+                                    (long)kk.stride(0), (long)vv.stride(0),
                                     causal ? 1 : 0, (int)window,
                                     current_stream()),
             "flash_prefill_varlen");
@@ -235,13 +239,26 @@ void context_prefill_varlen(at::Tensor& out, at::Tensor& q,
   int Hkv = k_cache.size(1);
   int D = q.size(2);
   int fp8 = k_cache.scalar_type() == at::kFloat8_e4m3fn ? 1 : 0;
+  const long rows = (long)q.size(0) * Hq;
+  const int n_splits =
+      ks_context_prefill_splits(num_seqs, rows, (int)max_q_len, Hq, Hkv,
+                                (int)block_tables.size(1), (int)window);
+  at::Tensor part_out, part_ml;
+  void *po = nullptr, *pml = nullptr;
+  if (n_splits > 1) {
+    auto opts = at::TensorOptions().dtype(at::kFloat).device(q.device());
+    part_out = at::empty({n_splits, rows, D}, opts);
+    part_ml = at::empty({n_splits, rows, 2}, opts);
+    po = part_out.data_ptr();
+    pml = part_ml.data_ptr();
+  }
   check_hip(ks_context_prefill_varlen(
                 out.data_ptr(), q.data_ptr(), k_cache.data_ptr(),
                 v_cache.data_ptr(), block_tables.data_ptr(),
                 ctx_lens.data_ptr(), cu_seqlens_q.data_ptr(), num_seqs,
                 (int)max_q_len, Hq, Hkv, D, (int)block_tables.size(1),
-                (float)scale, (long)q.stride(0), fp8, (int)window,
-                current_stream()),
+                (float)scale, (long)q.stride(0), fp8, (int)window, rows, n_splits, po,
+                pml, current_stream()),
             "context_prefill_varlen");
 }
 

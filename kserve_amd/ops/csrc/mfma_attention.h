@@ -46,6 +46,11 @@ __device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
+// for buffer loads from a uniform address, offsets below 2^32
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00027000);
+}
+
 // What the launchers hand the kernels as their scale: scores are masked before
 // they are scaled, and the scaled mask has to give weight 0. Below 1e-30 all
 // scores are level whatever the scale.
@@ -140,6 +145,11 @@ struct PrefillArgs {
   long sq, sk, sv;
   int window;
   Extra x;
+  // keys in n_splits parts (pages, one part per value): sums of the parts
+  int n_splits;
+  long rows;        // T * Hq
+  float* part_out;  // [n_splits, T, Hq, D]
+  float* part_ml;   // [n_splits, T, Hq, 2]: exponent, sum of weights
 };
 
 template <int D, int SRC, bool CAUSAL, bool WIN, int PARTS = 1>
@@ -157,7 +167,9 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   constexpr int KC = D / 16;          // contraction chunks of Q K^T
   constexpr int DB = D / 32;          // 32-column blocks of the output
 
-  const int seq = blockIdx.z;
+  constexpr bool SPLITS = PAGED && PARTS == 1;
+  const int seq = SPLITS ? blockIdx.z / p.n_splits : blockIdx.z;
+  const int split = SPLITS ? blockIdx.z % p.n_splits : 0;
   const int q_start = p.cu_q[seq];
   const int q_len = p.cu_q[seq + 1] - q_start;
   const int qpb = NWAVES * QW / p.hpb;  // queries per block
@@ -175,6 +187,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
 
   __shared__ __attribute__((aligned(16))) short lds[2][2][TILE];  // [buffer][K, V]
 
+  // The scale's sign goes into the query, exactly. With three parts it is applied to
+  // the scores: as a branch between products and softmax it keeps the compiler from
+  // moving one into the other, for which there are no registers.
+  float c2 = p.scale * LOG2E;
+  const bool flip = c2 < 0.f;
+  c2 = fabsf(c2);
+
   // ---- queries: B operands, 8 consecutive columns per lane ----
   bf16x8_t qf[PARTS][KC];
   {
@@ -183,8 +202,11 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
     if constexpr (PARTS == 1) {
       const short* qp = reinterpret_cast<const short*>(p.q) + at;
 #pragma unroll
-      for (int c = 0; c < KC; ++c)
-        qf[0][c] = *reinterpret_cast<const bf16x8_t*>(qp + c * 16);
+      for (int c = 0; c < KC; ++c) {
+        short8_t x = *reinterpret_cast<const short8_t*>(qp + c * 16);
+        if (flip) x ^= (short)0x8000;
+        qf[0][c] = __builtin_bit_cast(bf16x8_t, x);
+      }
     } else {
       const float* qp = reinterpret_cast<const float*>(p.q) + at;
 #pragma unroll
@@ -208,8 +230,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   const int hi = CAUSAL ? min(len, start_pos + last_q + 1) : len;
   auto low = [&](int pos) { return low_of(pos, p.window, p.x.chunk); };
   const int lo = WIN ? max(0, low(start_pos + tile_base)) : 0;
-  const int t_lo = lo / KT;
-  const int t_hi = (hi + KT - 1) / KT;
+  int t_lo = lo / KT;
+  int t_hi = (hi + KT - 1) / KT;
+  if (SPLITS && p.n_splits > 1) {
+    const int per = (t_hi - t_lo + p.n_splits - 1) / p.n_splits;
+    t_lo += split * per;
+    t_hi = min(t_hi, t_lo + per);
+  }
   const int pos_lo = start_pos + q0;
   const int pos_hi = start_pos + min(q0 + QW, q_len) - 1;
   const int my_pos = start_pos + q0 + (lane & 31);
@@ -224,47 +251,69 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   const int lrow = lane / CPR, lchunk = lane % CPR;
   auto group_of = [&](int t) { return min(t * KT + wave * 16, len - 1); };
   auto page_of = [&](int t) { return PAGED ? bt[group_of(t) >> 4] : 0; };
-  // address of this lane's chunk (c, already unswizzled) of row r of tile t
-  auto src = [&](const void* base, long stride, int t, int page, int r, int c) {
-    const int g0 = PAGED ? group_of(t) & ~15 : group_of(t);
-    const int row = min(r, len - 1 - g0);
-    if constexpr (PAGED) {
-      constexpr int ES = SRC == PAGES_FP8 ? 1 : 2;
-      const long st = PARTS == 1 ? D : stride;  // bf16 queries: whole rows
-      return reinterpret_cast<const char*>(base) +
-             ((long)page * p.Hkv + kvh) * PAGE * st * ES +
-             (row * (int)st + c * 8) * ES;
-    } else {
-      return reinterpret_cast<const char*>(base) +
-             ((long)(q_start + g0) * stride + (long)kvh * D) * 2 +
-             (long)row * stride * 2 + c * 16;
-    }
+  // A scalar base per tile and 32-bit lane offsets (the launchers see to strides
+  // below 2^26): tiles with all their keys cost no vector arithmetic, where 64-bit
+  // addresses per lane and load took 500 of a tile's 1800 vector cycles. The
+  // LDS-direct loads are buffer loads: after the global form the compiler waits
+  // for all of a wave's LDS reads at once instead of one after the other.
+  constexpr int ES = SRC == PAGES_FP8 ? 1 : 2;
+  const int krs = PAGED && PARTS == 1 ? D : (int)p.sk;  // bf16 queries: whole rows
+  const int vrs = PAGED && PARTS == 1 ? D : (int)p.sv;
+  // (three parts leave no registers for them: there they are formed per tile)
+  constexpr bool KEEP = PARTS == 1;
+  unsigned int koff[NI], voff[NI];
+#pragma unroll
+  for (int i = 0; KEEP && i < NI; ++i) {
+    const int r = i * RPI + lrow;
+    koff[i] = (unsigned int)(r * krs + (lchunk ^ k_swz<D>(r)) * 8) * ES;
+    voff[i] = (unsigned int)(r * vrs + (lchunk ^ v_swz<D>(r)) * 8) * ES;
+  }
+  auto base_of = [&](const void* base, int stride, int g0, int page) {
+    const long at = PAGED ? ((long)page * p.Hkv + kvh) * PAGE * stride
+                          : (long)(q_start + g0) * stride + kvh * D;
+    return reinterpret_cast<const char*>(base) + at * ES;
   };
   uint2 raw8[SRC == PAGES_FP8 ? 2 * NI : 1];
   short8_t raw16[!DMA && SRC != PAGES_FP8 ? 2 * NI : 1];
   // DMA: fills buffer `buf`; otherwise the rows wait in registers for commit()
-  auto stage = [&](int t, int page, int buf) {
+  auto stage_rows = [&](const char* kb, const char* vb, auto k_at, auto v_at, int buf) {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int r = i * RPI + lrow;
-      const char* ks = src(p.k, p.sk, t, page, r, lchunk ^ k_swz<D>(r));
-      const char* vs = src(p.v, p.sv, t, page, r, lchunk ^ v_swz<D>(r));
+      const unsigned int ka = k_at(i), va = v_at(i);
       if constexpr (DMA) {
+        typedef __attribute__((address_space(3))) void lds_t;
         const int at = (wave * 16 + i * RPI) * D;
-        __builtin_amdgcn_global_load_lds(
-            reinterpret_cast<const unsigned int*>(ks),
-            reinterpret_cast<unsigned int*>(&lds[buf][0][at]), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds(
-            reinterpret_cast<const unsigned int*>(vs),
-            reinterpret_cast<unsigned int*>(&lds[buf][1][at]), 16, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(raw_buffer(kb), (lds_t*)&lds[buf][0][at],
+                                                 16, ka, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(raw_buffer(vb), (lds_t*)&lds[buf][1][at],
+                                                 16, va, 0, 0, 0);
       } else if constexpr (SRC == PAGES_FP8) {
-        raw8[2 * i] = *reinterpret_cast<const uint2*>(ks);
-        raw8[2 * i + 1] = *reinterpret_cast<const uint2*>(vs);
+        raw8[2 * i] = *reinterpret_cast<const uint2*>(kb + ka);
+        raw8[2 * i + 1] = *reinterpret_cast<const uint2*>(vb + va);
       } else {
-        raw16[2 * i] = *reinterpret_cast<const short8_t*>(ks);
-        raw16[2 * i + 1] = *reinterpret_cast<const short8_t*>(vs);
+        raw16[2 * i] = *reinterpret_cast<const short8_t*>(kb + ka);
+        raw16[2 * i + 1] = *reinterpret_cast<const short8_t*>(vb + va);
       }
     }
+  };
+  auto stage = [&](int t, int page, int buf) {
+    const int g0 = PAGED ? group_of(t) & ~15 : group_of(t);
+    const char* kb = base_of(p.k, krs, g0, page);
+    const char* vb = base_of(p.v, vrs, g0, page);
+    if (KEEP && (t + 1) * KT <= len)
+      stage_rows(kb, vb, [&](int i) { return koff[i]; }, [&](int i) { return voff[i]; }, buf);
+    else
+      stage_rows(
+          kb, vb,
+          [&](int i) {
+            const int r = i * RPI + lrow;
+            return (unsigned int)(min(r, len - 1 - g0) * krs + (lchunk ^ k_swz<D>(r)) * 8) * ES;
+          },
+          [&](int i) {
+            const int r = i * RPI + lrow;
+            return (unsigned int)(min(r, len - 1 - g0) * vrs + (lchunk ^ v_swz<D>(r)) * 8) * ES;
+          },
+          buf);
   };
   auto commit = [&](int buf) {
     if constexpr (!DMA) {
@@ -299,10 +348,11 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
                (((4 * b + ((lane >> 4) & 1) * 2 + ((ti & 3) >> 1)) ^ v_swz<D>(vrow)) * 8) +
                (ti & 1) * 4;
 
-  float c2 = p.scale * LOG2E;
-  const bool flip = c2 < 0.f;
-  c2 = fabsf(c2);
-  float m = NO_MAX, l = 0.f;
+  // Weights are 2^(score c2 - mc). mc follows the row's largest score only once it
+  // is passed by 2^8: the sums have the room, and the rescaling of the output that
+  // each new maximum of any of the 32 rows costs becomes rare.
+  constexpr float ROOM = 8.f;
+  float mc = fmaxf(NO_MAX * c2, -3e38f), l = 0.f;
   f32x16_t o[DB];
 #pragma unroll
   for (int b = 0; b < DB; ++b)
@@ -333,6 +383,27 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
 #pragma unroll
       for (int kg = 0; kg < 2; kg += NKB) {
       f32x16_t s[NKB];
+      if constexpr (PARTS == 1) {
+#pragma unroll
+        for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[kb][r] = 0.f;
+        // both key blocks' chains side by side, keys read ahead of the products
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+#pragma unroll
+          for (int kb = 0; kb < NKB; ++kb)
+            s[kb] = mfma32(*reinterpret_cast<const bf16x8_t*>(kt + kb * 32 * D + kaddr[c]),
+                           qf[0][c], s[kb]);
+        constexpr int READS = NKB * KC, AHEAD = READS < 6 ? READS : 6;
+        __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);  // LDS reads
+#pragma unroll
+        for (int i = 0; i < READS - AHEAD; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // matrix products
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+      } else {
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb) {
         f32x16_t rest;  // the products with the query's lower parts
@@ -342,17 +413,16 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
         for (int c = 0; c < KC; ++c) {
           const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(
               kt + (kg + kb) * 32 * D + kaddr[c]);
-          if constexpr (PARTS == 3) {
-            rest = mfma32(a, qf[PARTS - 1][c], rest);
-            rest = mfma32(a, qf[PARTS - 2][c], rest);
-          }
+          rest = mfma32(a, qf[PARTS - 1][c], rest);
+          rest = mfma32(a, qf[PARTS - 2][c], rest);
           s[kb] = mfma32(a, qf[0][c], s[kb]);
         }
-        if constexpr (PARTS == 3) s[kb] += rest;
+        s[kb] += rest;
       }
       if (flip) {
 #pragma unroll
         for (int kb = 0; kb < NKB; ++kb) s[kb] = -s[kb];
+      }
       }
       // register r of block kb: key 32 kb + (r & 3) + 8 (r / 4) + 4 half
       if (t0 + KT > len || (CAUSAL && t0 + KT - 1 > pos_lo) ||
@@ -372,25 +442,24 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
       for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
-      mx = half_max(mx);
-      if (__any(mx > m)) {
-        const float mn = fmaxf(m, mx);
-        const float f = __builtin_amdgcn_exp2f((m - mn) * c2);
-        m = mn;
+      mx = half_max(mx) * c2;
+      if (__any(mx > mc + ROOM)) {
+        const float mn = fmaxf(mc, mx);
+        const float f = __builtin_amdgcn_exp2f(mc - mn);
+        mc = mn;
         l *= f;
 #pragma unroll
         for (int b = 0; b < DB; ++b)
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[b][r] *= f;
       }
-      const float mc = m * c2;
       bf16x8_t pf[PARTS][NKB * 2];
       float sum = 0.f;
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float w = __builtin_amdgcn_exp2f(s[kb][r] * c2 - mc);
+          const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][r], c2, -mc));
           sum += w;
           if constexpr (PARTS == 1) {
             pf[0][kb * 2 + (r >> 3)][r & 7] = (__bf16)w;
@@ -431,13 +500,28 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   l = half_sum(l);
   if (qrow >= q_len) return;
   const long tok = q_start + qrow;
+  if (SPLITS && p.n_splits > 1) {
+    const long row = split * p.rows + tok * p.Hq + head;
+    if (half == 0) *reinterpret_cast<float2_t*>(p.part_ml + row * 2) = float2_t{mc, l};
+    if (t_lo >= t_hi) return;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4_t w;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) w[r] = o[b][g * 4 + r];
+        store4(p.part_out, row * D + half * 4 + b * 32 + g * 8, w, 1);
+      }
+    return;
+  }
   float inv;
   if constexpr (PARTS == 1) {
     inv = l > 0.f ? 1.f / l : 0.f;
   } else {
     if (p.x.sink) {
       // exp(sink) joins the denominator; the larger of the two maxima scales
-      const float sl = p.x.sink[head] * LOG2E, ml = m * c2, top = fmaxf(ml, sl);
+      const float sl = p.x.sink[head] * LOG2E, ml = mc, top = fmaxf(ml, sl);
       const float f = exp2f(ml - top);
       l = l * f + exp2f(sl - top);
       inv = f / l;
@@ -456,6 +540,57 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
       store4(p.out, (tok * p.Hq + head) * D + half * 4 + b * 32 + g * 8, w,
              PARTS == 1 ? 0 : p.x.out_f32);
     }
+}
+
+// adds the parts of prefill_attention_kernel's keys: 32 lanes per (token, head),
+// 4 of 128 columns each. Parts without a visible key wrote no sums (weight 0).
+__global__ __launch_bounds__(256) void prefill_attention_merge_kernel(
+    short* __restrict__ out, const float* __restrict__ part_out,
+    const float* __restrict__ part_ml, const int n_splits, const long rows) {
+  constexpr int D = 128;
+  const long row = blockIdx.x * 8L + (threadIdx.x >> 5);
+  if (row >= rows) return;
+  const int d = (threadIdx.x & 31) * 4;
+  float top = -3.4e38f;
+  for (int s = 0; s < n_splits; ++s) {
+    const float2_t ml = *reinterpret_cast<const float2_t*>(part_ml + (s * rows + row) * 2);
+    if (ml[1] > 0.f) top = fmaxf(top, ml[0]);
+  }
+  float sum = 0.f;
+  f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < n_splits; ++s) {
+    const float2_t ml = *reinterpret_cast<const float2_t*>(part_ml + (s * rows + row) * 2);
+    if (ml[1] > 0.f) {
+      const float f = __builtin_amdgcn_exp2f(ml[0] - top);
+      sum += f * ml[1];
+      acc += f * *reinterpret_cast<const f32x4_t*>(part_out + (s * rows + row) * D + d);
+    }
+  }
+  store4(out, row * D + d, acc * (sum > 0.f ? 1.f / sum : 0.f), 0);
+}
+
+// Key parts of a prefill over pages. A block walks its tiles of 64 keys one after
+// the other, 1.4 us each where a compute unit has one block and 2.2 with two, so
+// few queries behind a long context leave most of the chip waiting; parts cost a
+// launch and fp32 sums that are written and read. The estimate of both is taken
+// from what was measured (32 / 8 heads, us, one part / chosen): 4 x 48 queries
+// after 12900 keys 294 / 70, 3 x 56 after 1844 42 / 25, 2 x 200 after 14000 321 / 119,
+// 700 after 5000 121 / 86, 32 after 600 17.5 / 13.8; 4 x 382 after 462 stays one).
+inline int prefill_splits(long blocks, int tiles, long rows) {
+  if (blocks <= 0 || tiles <= 0 || rows <= 0) return 1;
+  int best = 1;
+  double least = 0;
+  for (int n = 1; n <= 32 && n <= tiles; ++n) {
+    const long all = blocks * n, rounds = (all + 511) / 512;
+    const double tile = all <= 256 ? 1.4 : 2.2 * rounds;
+    const double us = (tiles + n - 1) / n * tile + 2.0 * rounds +
+                      (n > 1 ? 4.0 + rows * 128 * 4.0 * 2 * n / 3e6 : 0.0);
+    if (n == 1 || us < 0.95 * least) {
+      best = n;
+      least = us;
+    }
+  }
+  return best;
 }
 
 // over the four lanes that share a column (lane & 15)

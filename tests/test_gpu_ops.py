@@ -537,6 +537,57 @@ class TestPrefillAttention:
             err = (got.cpu() - ref.reshape(rows, -1)).norm() / ref.norm()
             assert err < 1e-6, (rows, float(err))
 
+    @pytest.mark.parametrize("rise", [0.02, 0.5, -0.5])
+    @pytest.mark.parametrize("scale", [0.088, -0.088])
+    def test_prefill_rising_scores(self, dev, scale, rise):
+        """Largest scores that move by less and by more than the room that the
+        weights leave them before the output is rescaled, from tile to tile and
+        from one part of the keys to the next."""
+        import kserve_amd_C
+        from kserve_amd import ops
+
+        H, Hkv, D, T, ctx = 4, 2, 128, 70, 1500
+        torch.manual_seed(5)
+        q = torch.randn(T, H, D, device=dev)
+        # every key has a share of the queries' common direction, by its position
+        along = q.mean((0, 1))
+        along /= along.norm()
+        q = (q + 8 * along).to(torch.bfloat16)
+        steps = torch.arange(ctx + 4, device=dev).float()[:, None, None]
+        k = torch.randn(ctx + 4, Hkv, D, device=dev)
+        k = (k + steps * along * (rise * (1 if scale > 0 else -1))).to(torch.bfloat16)
+        v = torch.randn(ctx + 4, Hkv, D, device=dev).to(torch.bfloat16)
+        cu = torch.tensor([0, T], dtype=torch.int32)
+        limit = 2 * 2 ** -9  # weights and output are each rounded to bf16
+
+        out = torch.empty_like(q)
+        kserve_amd_C.flash_prefill_varlen(
+            out, q, k[:T], v[:T], cu.to(dev), T, scale, True, 0
+        )
+        ref = torch_ref.flash_prefill_varlen(
+            q.double().cpu(), k[:T].double().cpu(), v[:T].double().cpu(), cu, scale
+        )
+        assert (out.double().cpu() - ref).norm() < limit * ref.norm()
+
+        pages = [x.view(-1, 16, Hkv, D).transpose(1, 2).contiguous() for x in (k, v)]
+        bt = torch.arange(pages[0].shape[0], dtype=torch.int32)[None]
+        ctx_t = torch.tensor([ctx], dtype=torch.int32)
+        ref = torch_ref.context_attention_varlen(
+            q.double().cpu(), *(x.double().cpu() for x in pages), bt, cu, ctx_t, scale
+        )
+        got = ops.context_attention_varlen(
+            q, *pages, bt.to(dev), cu.to(dev), ctx_t.to(dev), T, scale
+        )
+        assert (got.double().cpu() - ref).norm() < limit * ref.norm()
+        got = ops.ctx_attention_f32(
+            q.float().reshape(T, -1), *pages, bt.to(dev), cu.to(dev), ctx_t.to(dev),
+            scale, T, H,
+        )
+        # q . k up to 6000 in fp32, here and in the reference: 6000 * 2^-23 * 0.088 =
+        # 6e-5 in an exponent for each rounding of the sum
+        ref = ref.reshape(T, -1)
+        assert (got.double().cpu() - ref).norm() < 5e-4 * ref.norm()
+
     @pytest.mark.parametrize("fp8", [False, True])
     @pytest.mark.parametrize("window", [0, 50])
     @pytest.mark.parametrize("H,Hkv", [(4, 1), (6, 3), (2, 2), (8, 1)])
