@@ -37,6 +37,7 @@ MODULES = {
             "sampling.hip",
             "decode_step.hip",
             "skinny_gemm.hip",
+            "dense_gemm.hip",
             "gemm8.hip",
             "mfma_probe.hip",
         ],

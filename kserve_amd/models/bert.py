@@ -103,7 +103,7 @@ class BertLayer(nn.Module):
         hidden = ops.fused_add_layer_norm(
             attn, hidden, self.attn_ln_w, self.attn_ln_b, self.eps
         )
-        inter = ops.gelu(ops.linear(hidden, self.inter_w, self.inter_b))
+        inter = ops.linear_gelu(hidden, self.inter_w, self.inter_b)
         out = ops.linear(inter, self.out_w, self.out_b)
         return ops.fused_add_layer_norm(
             out, hidden, self.out_ln_w, self.out_ln_b, self.eps
@@ -241,7 +241,7 @@ class BertForMaskedLM(nn.Module):
 
     def forward(self, input_ids, cu_seqlens, token_type_ids=None):
         hidden = self.bert(input_ids, cu_seqlens, token_type_ids)
-        t = ops.gelu(ops.linear(hidden, self.transform_w, self.transform_b))
+        t = ops.linear_gelu(hidden, self.transform_w, self.transform_b)
         t = ops.layer_norm(t, self.transform_ln_w, self.transform_ln_b, self.eps)
         return ops.linear(t, self.bert.word_embeddings, self.decoder_bias)
 

@@ -286,8 +286,12 @@ def random_sample(
 
 
 def _skinny_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """What the few-row kernels read directly: plain bf16 matrices on one GPU
-    with 16-byte aligned rows, outside autograd and its transforms."""
+    return x.shape[0] <= 256 and _plain_operands(x, weight)
+
+
+def _plain_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """What the GEMM kernels read directly: plain bf16 matrices on one GPU with
+    16-byte aligned rows, outside autograd and its transforms."""
     return (
         _C is not None
         and x.is_cuda
@@ -296,7 +300,7 @@ def _skinny_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
         and x.dtype == torch.bfloat16
         and weight.dtype == torch.bfloat16
         and x.device == weight.device
-        and 0 < x.shape[0] <= 256
+        and x.shape[0] > 0
         and x.shape[1] == weight.shape[1]
         and x.shape[1] > 0
         and x.shape[1] % 64 == 0
@@ -366,9 +370,51 @@ def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     return m >= 4608 and (n <= 48 or m <= 8192 or m >= 10240)
 
 
+def _dense_rows(n: int, k: int, m: int) -> bool:
+    """Whether the encoder kernel beats the library at [n, k] x [m, k]^T + bias
+    (MI355X, us, kernel / library). Up to k 768 it does from one row to 30000 (m
+    768 at 100 / 7864 / 30000 rows 4.8 / 5.1, 13.9 / 15.1, 48 / 60; level at 8 rows,
+    4.6 / 4.4, where it is the shorter call by 14 us of host time); at k 1024 while
+    the rows leave the library short of tiles (m 1024 at 1000 / 3500 / 16384 rows 6.7 /
+    9.4, 12.3 / 12.8, 43 / 30); past that the library's larger tiles win (k 3072, m
+    768 at 200 / 3500 rows 12.0 / 9.4, 29 / 22)."""
+    return m % 8 == 0 and 8 <= m <= 4096 and (k <= 768 or (k <= 1024 and n <= 3584))
+
+
+def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
+    """The encoder kernel's product, or None for operands that it does not take."""
+    m = weight.shape[0]
+    if not (
+        bias is not None
+        and x.dim() == 2
+        and _dense_rows(x.shape[0], x.shape[1], m)
+        and _plain_operands(x, weight)
+        and x.shape[0] < 1 << 30
+        and x.shape[1] <= x.stride(0) < 1 << 22
+        and type(bias) in (torch.Tensor, torch.nn.Parameter)
+        and bias.shape == (m,)
+        and bias.dtype == torch.bfloat16
+        and bias.device == x.device
+        and bias.is_contiguous()
+        and bias.data_ptr() % 16 == 0
+        and not torch._C._functorch.is_functorch_wrapped_tensor(bias)
+        and not (torch.is_grad_enabled() and bias.requires_grad)
+        and not torch.is_autocast_enabled("cuda")
+    ):
+        return None
+    out = torch.empty((x.shape[0], m), dtype=x.dtype, device=x.device)
+    _C.dense_gemm(out, x, weight, bias, gelu)
+    return out
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x @ weight^T (+ bias): a kernel of our own for the few rows of a decode
-    batch where it is the faster one, the library otherwise."""
+    """x @ weight^T (+ bias): kernels of our own for the few rows of a decode
+    batch and for the encoder's short K where they are the faster ones, the
+    library otherwise."""
+    if bias is not None:
+        out = _dense(x, weight, bias, False)
+        if out is not None:
+            return out
     # sizes first: most calls that are not for the kernel end there
     if (
         bias is None
@@ -382,6 +428,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         _C.skinny_gemm(out, x, weight)
         return out
     return torch.nn.functional.linear(x, weight, bias)
+
+
+def linear_gelu(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+    """gelu (erf form) of x @ weight^T + bias, on the sums in 32 bits where the
+    encoder kernel takes the product."""
+    out = _dense(x, weight, bias, True)
+    return gelu(linear(x, weight, bias)) if out is None else out
 
 
 def linear_silu_and_mul(

@@ -50,6 +50,8 @@ hipError_t ks_rope_cache(void*, void*, void*, const void*, int, const void*,
 hipError_t ks_add_splits_rms_norm(void*, void*, const void*, const void*, float,
                                   int, int, int, hipStream_t);
 int ks_skinny_splits(int, int, int, int);
+hipError_t ks_dense_gemm(void*, const void*, const void*, const void*, int, int, int,
+                         long, int, int, hipStream_t);
 hipError_t ks_skinny_gemm(void*, void*, const void*, const void*, int, int,
                           int, long, int, int, hipStream_t);
 hipError_t ks_gemm8(void*, const void*, const void*, int, int, int, int,
@@ -398,6 +400,32 @@ void skinny_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
   skinny_product(out, x, w, true);
 }
 
+void dense_gemm(at::Tensor& out, at::Tensor& x, at::Tensor& w,
+                const c10::optional<at::Tensor>& bias, bool gelu, int64_t tile) {
+  // out [N, M] = act(x [N, K] @ w [M, K]^T + bias), bf16
+  CHECK_BF16_CONTIG(out);
+  CHECK_BF16_CONTIG(w);
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && x.is_cuda() && x.dim() == 2 &&
+                  w.dim() == 2 && out.dim() == 2 && x.stride(1) == 1,
+              "x must be bf16 row-dense");
+  const long N = x.size(0), K = x.size(1), M = w.size(0);
+  TORCH_CHECK(w.size(1) == K && out.size(0) == N && out.size(1) == M, "shape mismatch");
+  TORCH_CHECK(x.device() == w.device() && out.device() == x.device(),
+              "operands on different devices");
+  TORCH_CHECK(N < (1L << 30) && M < (1L << 30) && K < (1L << 30), "size out of range");
+  const void* b = nullptr;
+  if (bias.has_value()) {
+    CHECK_BF16_CONTIG(*bias);
+    TORCH_CHECK(bias->numel() == M && bias->device() == x.device(), "bias mismatch");
+    b = bias->data_ptr();
+  }
+  const c10::DeviceGuard guard(x.device());
+  check_hip(ks_dense_gemm(out.data_ptr(), x.data_ptr(), w.data_ptr(), b, (int)M, (int)K,
+                          (int)N, (long)x.stride(0), gelu ? 1 : 0, (int)tile,
+                          current_stream()),
+            "dense_gemm");
+}
+
 void skinny_add_rms_norm(at::Tensor& out, at::Tensor& residual, at::Tensor& x,
                          at::Tensor& w, at::Tensor& norm_weight, double eps) {
   // residual += x @ w^T; out = RMS norm of residual
@@ -546,6 +574,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_rope_cache", &skinny_rope_cache,
         "few-row qkv GEMM, rotary embedding and K/V scatter");
   m.def("skinny_glu", &skinny_glu, "gate|up GEMM (N<=256) with silu(gate) * up");
+  m.def("dense_gemm", &dense_gemm, "GEMM with bias and, if asked for, erf GELU",
+        pybind11::arg("out"), pybind11::arg("x"), pybind11::arg("w"),
+        pybind11::arg("bias"), pybind11::arg("gelu"), pybind11::arg("tile") = -1);
   m.def("gemm8", &gemm8,
         "EXPERIMENTAL 8-phase 256x256 MFMA GEMM");
   m.def("mfma_probe", &mfma_probe, "MFMA layout probe (tests)");

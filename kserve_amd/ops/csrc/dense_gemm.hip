@@ -1,0 +1,269 @@
+// Products of an encoder's layers: out[N][M] = act(x[N][K] w[M][K]^T + bias), bf16
+// with fp32 sums, act the identity or gelu (erf form) on the fp32 sums.
+//
+// K is short here (768: twelve steps), so a tile's first loads, its epilogue and
+// the last, uneven round of tiles weigh as much as the products, and the library,
+// whose choice of tile changes from one token count to the next, ran at 0.4 to 0.9
+// PFLOP/s with a pass over memory of its own for gelu. Each step's token and
+// weight rows come by LDS-direct loads into one slot of a ring; a wave reads the
+// fragments of a half step while it multiplies those of the half before, with one
+// barrier per step. What bounds it is the rate at which one compute unit takes
+// lines in, about 27 bytes a cycle whatever the tile or the depth of the ring (a
+// ring of 32-wide steps, 64-byte rows, took 20): so tiles are as large as the
+// token count lets them be, and where two blocks fit a unit one multiplies while
+// the other starts or ends. No two steps of a row share a bank (0 conflicts).
+//
+// us, this / the library (and gelu's kernel): 7864 x 768 to 2304 33 / 63, to 768
+// 13.9 / 15.1, to 3072 with gelu 50 / 68; 1500 rows to 768 7.2 / 8.7, to 3072 with
+// gelu 15.8 / 20.9; 200 rows to 2304 5.8 / 7.9.
+#include "common.h"
+#include "mfma_layouts.h"
+
+namespace {
+
+constexpr int UNITS = 256;  // compute units
+constexpr int BK = 64;  // K per step
+
+struct DenseArgs {
+  short* out;         // [N][M]
+  const short* x;     // [N][K], row stride xs
+  const short* w;     // [M][K]
+  const short* bias;  // [M] or null
+  int M, K, N, xs;
+  int ftiles, tiles;  // tiles along M, in all
+};
+
+typedef __attribute__((address_space(3))) void lds_t;
+
+// 16 bytes per lane from a uniform address (lane and step offsets below 2^32)
+// straight to 1 KB of LDS
+__device__ __forceinline__ void load_lds(const short* from, short* to, unsigned int lane_at,
+                                         int step_at) {
+  const __amdgpu_buffer_rsrc_t rows =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<short*>(from), 0, -1, 0x00027000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_t*)to, 16, lane_at, step_at, 0, 0);
+}
+
+// s_waitcnt with vmcnt <= n (bits 3:0 and 15:14), lgkmcnt 0, expcnt free
+constexpr int wait_imm(int n) { return (0x7 << 4) | (n & 0xF) | ((n >> 4) << 14); }
+
+// x Phi(x) with the tail Phi(-|x|) = exp(-x^2 / 2) t Q(t), t = 1 / (1 + c |x|), Q a
+// polynomial fitted to a relative 6.5e-7 of it over |x| < 13.4 (least squares,
+// reweighted towards the largest error): a third of erff's instructions, which
+// would cost as much as the products.
+__device__ __forceinline__ float gelu_f(float x) {
+  const float a = fabsf(x);
+  const float t = __builtin_amdgcn_rcpf(1.f + 0.265165043f * a);
+  float q = -0.0675466018f;
+  q = q * t + 0.193964045f;
+  q = q * t - 0.0647915465f;
+  q = q * t + 0.141525405f;
+  q = q * t + 0.0833345009f;
+  q = q * t + 0.107844114f;
+  q = q * t + 0.105669766f;
+  const float tail = q * t * __builtin_amdgcn_exp2f(x * x * -0.721347520f);
+  return x * (x > 0.f ? 1.f - tail : tail);
+}
+
+template <int TN, int TM, int WN, int WM, int S, bool GELU>
+__global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const DenseArgs p) {
+  constexpr int NW = WN * WM;
+  constexpr int FN = TN / WN / 16, FM = TM / WM / 16;  // fragments of a wave
+  constexpr int STAGE = (TN + TM) * BK;                // elements
+  constexpr int NX = TN / 8 / NW, NI = (TN + TM) / 8 / NW;  // 1 KB loads of a wave
+  static_assert(TN % (8 * NW) == 0 && TM % (8 * NW) == 0 && FM % 2 == 0 && S >= 2 &&
+                    S * STAGE * 2 <= 160 * 1024,
+                "tile");
+  __shared__ __attribute__((aligned(16))) short ring[S * STAGE];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+
+  // blocks go to the 8 XCDs in turn: each takes a run of tiles, features first
+  const int xcd = blockIdx.x & 7, nth = blockIdx.x >> 3;
+  const int tile = xcd * (p.tiles >> 3) + min(xcd, p.tiles & 7) + nth;
+  const int n0 = tile / p.ftiles * TN, m0 = tile % p.ftiles * TM;
+
+  // a load is 8 rows of 128 bytes; 16-byte chunk c of a row sits at c ^ key, the
+  // key such that the rows of a fragment at one chunk hit different banks
+  const short *xb = p.x + (long)n0 * p.xs, *wb = p.w + (long)m0 * p.K;
+  unsigned int at[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = ((i < NX ? i : i - NX) * NW + wave) * 8 + (lane >> 3);
+    const int key = i < NX ? (r >> 1) & 7 : ((r >> 1) & 1) | ((r >> 2) & 6);
+    const int row = i < NX ? min(r, p.N - 1 - n0) * p.xs : min(r, p.M - 1 - m0) * p.K;
+    at[i] = (unsigned int)(row + ((lane & 7) ^ key) * 8) * 2;
+  }
+  auto issue = [&](int step, int slot) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      load_lds(i < NX ? xb : wb, &ring[slot * STAGE + (i * NW + wave) * 8 * BK], at[i],
+               step * BK * 2);
+  };
+
+  f32x4_t acc[FM][FN];
+#pragma unroll
+  for (int f = 0; f < FM; ++f)
+#pragma unroll
+    for (int t = 0; t < FN; ++t) acc[f][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // fragment rows: tokens in order; features so that a lane's rows of two
+  // fragments are 8 consecutive ones, 16 bytes of the output
+  const int wn = wave % WN, wm = wave / WN;
+  const int xrow = wn * FN * 16 + col, xkey = (col >> 1) & 7;
+  const int frow = TN + wm * FM * 16 + (col >> 2) * 8 + (col & 3);
+  const int fkey = ((col >> 1) & 1) | ((col >> 2) << 1);
+
+  bf16x8_t a0[FM], b0[FN], a1[FM], b1[FN];  // the two halves of a step
+  auto fetch = [&](int slot, int half, bf16x8_t(&a)[FM], bf16x8_t(&b)[FN]) {
+    const short* st = &ring[slot * STAGE];
+    const short* fp = st + frow * BK + ((half * 4 + g) ^ fkey) * 8;
+    const short* xp = st + xrow * BK + ((half * 4 + g) ^ xkey) * 8;
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+      a[f] = *reinterpret_cast<const bf16x8_t*>(fp + ((f >> 1) * 32 + (f & 1) * 4) * BK);
+#pragma unroll
+    for (int t = 0; t < FN; ++t) b[t] = *reinterpret_cast<const bf16x8_t*>(xp + t * 16 * BK);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](bf16x8_t(&a)[FM], bf16x8_t(&b)[FN]) {
+#pragma unroll
+    for (int t = 0; t < FN; ++t)
+#pragma unroll
+      for (int f = 0; f < FM; ++f) acc[f][t] = mfma16x16x32(a[f], b[t], acc[f][t]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto barrier = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  const int steps = p.K / BK;
+#pragma unroll
+  for (int j = 0; j < S; ++j)
+    if (j < steps) issue(j, j);
+  if (steps >= S) __builtin_amdgcn_s_waitcnt(wait_imm(NI * (S - 1)));
+  else __builtin_amdgcn_s_waitcnt(wait_imm(0));
+  barrier();
+  fetch(0, 0, a0, b0);
+  // In a step, this wave has read all of it and its own loads of the next have
+  // landed before the barrier, which covers the other waves'; then the slot is
+  // free. (A loop of its own for the steps that load no more: with the loads under
+  // a condition the compiler moves every accumulator once a step.)
+  int slot = 0, j = 0;
+  for (; j + S < steps; ++j) {
+    fetch(slot, 1, a1, b1);
+    multiply(a0, b0);
+    __builtin_amdgcn_s_waitcnt(wait_imm(NI * (S - 2)));
+    barrier();
+    issue(j + S, slot);
+    slot = slot + 1 == S ? 0 : slot + 1;
+    fetch(slot, 0, a0, b0);
+    multiply(a1, b1);
+  }
+  for (; j + 1 < steps; ++j) {
+    fetch(slot, 1, a1, b1);
+    multiply(a0, b0);
+    __builtin_amdgcn_s_waitcnt(wait_imm(0));
+    barrier();
+    slot = slot + 1 == S ? 0 : slot + 1;
+    fetch(slot, 0, a0, b0);
+    multiply(a1, b1);
+  }
+  fetch(slot, 1, a1, b1);
+  multiply(a0, b0);
+  multiply(a1, b1);
+
+#pragma unroll
+  for (int f = 0; f < FM; f += 2) {
+    const int feat = m0 + wm * FM * 16 + f * 16 + g * 8;
+    if (feat >= p.M) continue;
+    float b[8];
+    const short8_t bv = p.bias ? *reinterpret_cast<const short8_t*>(p.bias + feat) : short8_t{};
+#pragma unroll
+    for (int r = 0; r < 8; ++r) b[r] = bf16_bits_to_float(bv[r]);
+#pragma unroll
+    for (int t = 0; t < FN; ++t) {
+      const int tok = n0 + wn * FN * 16 + t * 16 + col;
+      if (tok >= p.N) continue;
+      bf16x8_t o;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        float v = acc[f + r / 4][t][r % 4] + b[r];
+        if constexpr (GELU) v = gelu_f(v);
+        o[r] = (__bf16)v;
+      }
+      *reinterpret_cast<bf16x8_t*>(p.out + (long)tok * p.M + feat) = o;
+    }
+  }
+}
+
+// Which tile: the least a n + b, for n tiles on the busiest unit. a and b are us at
+// K 768, between those with and without gelu; all grow with K alike, so the order
+// holds. Where a unit has a single tile, one block of eight waves with a deeper
+// ring beats one of four (7864 x 768 to 768 13.9 / 15.1, 1000 to 2304 10.1 / 12.3).
+struct Tile {
+  int tn, tm;
+  float a, b;
+};
+constexpr int NTILES = 6;
+constexpr Tile TILES[NTILES] = {
+    {128, 192, 12.f, 0.f},   {128, 192, 11.f, 2.f},  {128, 128, 9.8f, 0.f},
+    {128, 128, 8.2f, 2.5f}, {64, 128, 4.3f, 3.5f},  {64, 64, 2.8f, 2.8f}};
+
+}  // namespace
+
+extern "C" int ks_dense_tile(int M, int N) {
+  int best = 0;
+  float least = 0.f;
+  for (int i = 0; i < NTILES; ++i) {
+    const Tile& t = TILES[i];
+    const long tiles = (long)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
+    const long n = (tiles + UNITS - 1) / UNITS;
+    const float us = t.a * (float)n + t.b;
+    if (i == 0 || us < least) {
+      least = us;
+      best = i;
+    }
+  }
+  return best;
+}
+
+// `tile` < 0: by the rule above
+extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
+                                    const void* bias, int M, int K, int N, long xs,
+                                    int gelu, int tile, hipStream_t stream) {
+  // (rows within a tile and steps along K by 32-bit offsets)
+  if (N < 1 || M < 8 || M % 8 != 0 || K < BK || K % BK != 0 || K >= 1 << 22 ||
+      xs % 8 != 0 || xs < K || xs >= 1 << 22 || tile >= NTILES ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)bias) & 15) != 0)
+    return hipErrorInvalidValue;
+  if (tile < 0) tile = ks_dense_tile(M, N);
+  const Tile& t = TILES[tile];
+  const long ftiles = (M + t.tm - 1) / t.tm, tiles = ftiles * ((N + t.tn - 1) / t.tn);
+  if (tiles > 0x7fffffff) return hipErrorInvalidValue;
+  const DenseArgs p{(short*)out, (const short*)x, (const short*)w, (const short*)bias,
+                    M, K, N, (int)xs, (int)ftiles, (int)tiles};
+#define GO(tn, tm, wn, wm, s)                                                         \
+  if (gelu)                                                                           \
+    hipLaunchKernelGGL((dense_gemm_kernel<tn, tm, wn, wm, s, true>), dim3(p.tiles),   \
+                       dim3(wn * wm * 64), 0, stream, p);                             \
+  else                                                                                \
+    hipLaunchKernelGGL((dense_gemm_kernel<tn, tm, wn, wm, s, false>), dim3(p.tiles),  \
+                       dim3(wn * wm * 64), 0, stream, p);
+  switch (tile) {
+    case 0: GO(128, 192, 4, 2, 3) break;
+    case 1: GO(128, 192, 2, 2, 2) break;
+    case 2: GO(128, 128, 4, 2, 4) break;
+    case 3: GO(128, 128, 2, 2, 2) break;
+    case 4: GO(64, 128, 2, 2, 3) break;
+    default: GO(64, 64, 2, 2, 4) break;
+  }
+#undef GO
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
+}

@@ -2,6 +2,7 @@
 times of both kernels are known (no GPU needed: the rules take sizes only)."""
 
 import pytest
+import torch
 
 from kserve_amd import ops
 
@@ -60,3 +61,29 @@ def test_scan_in_chunks(lens, heads, P, N, chunks):
 
 def test_scan_of_no_sequences():
     assert not ops._scan_in_chunks(100, 0, 100, 64, 64, 128)
+
+
+@pytest.mark.parametrize(
+    "n,k,m,own",
+    [
+        (1, 768, 768, True), (30000, 768, 3072, True), (7864, 384, 1536, True),
+        (3584, 1024, 4096, True), (3585, 1024, 4096, False),  # 16384 rows 183 / 169
+        (200, 3072, 768, False), (64, 768, 30522, False), (64, 768, 4, False),
+        (64, 768, 4104, False),
+    ],
+)
+def test_encoder_product(n, k, m, own):
+    assert ops._dense_rows(n, k, m) is own
+
+
+def test_encoder_product_on_cpu_is_the_librarys():
+    x, w, b = torch.randn(5, 64), torch.randn(16, 64), torch.randn(16)
+    y = torch.nn.functional.linear(x, w, b)
+    assert torch.equal(ops.linear(x, w, b), y)
+    assert torch.equal(ops.linear_gelu(x, w, b), ops.gelu(y))
+    # rows of rows, gradients and transforms stay with it too
+    x3 = torch.randn(2, 5, 64, requires_grad=True)
+    ops.linear_gelu(x3, w, b).sum().backward()
+    assert x3.grad is not None
+    z = torch.vmap(lambda v: ops.linear(v, w, b))(torch.randn(3, 5, 64))
+    assert z.shape == (3, 5, 16)

@@ -1014,6 +1014,76 @@ class TestSkinnyGemmEdges:
         torch.testing.assert_close(got, want, rtol=2.0 ** -6, atol=2e-2)
 
 
+class TestDenseGemm:
+    """Encoder products: every tile at its edges, strided rows, both epilogues."""
+
+    @staticmethod
+    def _check(out, x, w, b, gelu):
+        y = x.double().cpu() @ w.double().cpu().t() + b.double().cpu()
+        if gelu:
+            y = torch.nn.functional.gelu(y)
+        # one rounding to bf16 of a sum of K products in 32 bits
+        tol = 2.0**-8 * y.abs() + 1e-5 * x.shape[1] ** 0.5
+        assert ((out.double().cpu() - y).abs() <= tol).all()
+
+    @pytest.mark.parametrize("tile", range(6))
+    @pytest.mark.parametrize(
+        "N,K,M",
+        [(1, 64, 8), (63, 128, 200), (129, 192, 72), (130, 256, 392), (257, 320, 1160)],
+    )
+    def test_every_tile(self, dev, tile, N, K, M):
+        import kserve_amd_C
+
+        torch.manual_seed(N + K)
+        x = torch.randn(N, K + 8, device=dev, dtype=torch.bfloat16)[:, :K]
+        w = (torch.randn(M, K, device=dev) * K**-0.5).to(torch.bfloat16)
+        b = torch.randn(M, device=dev, dtype=torch.bfloat16)
+        for gelu in (False, True):
+            # a row past the end must stay as it is
+            out = torch.full((N + 1, M), 7.0, device=dev, dtype=torch.bfloat16)
+            kserve_amd_C.dense_gemm(out[:N], x, w, b, gelu, tile)
+            self._check(out[:N], x, w, b, gelu)
+            assert (out[N] == 7.0).all()
+        out = torch.empty(N, M, device=dev, dtype=torch.bfloat16)
+        kserve_amd_C.dense_gemm(out, x, w, None, False, tile)
+        self._check(out, x, w, torch.zeros_like(b), False)
+
+    @pytest.mark.parametrize("N", [7, 700, 2600])
+    def test_entry_points(self, dev, N):
+        from kserve_amd import ops
+
+        torch.manual_seed(N)
+        x = torch.randn(N, 768, device=dev, dtype=torch.bfloat16)
+        w = (torch.randn(768, 768, device=dev) * 768**-0.5).to(torch.bfloat16)
+        b = torch.randn(768, device=dev, dtype=torch.bfloat16)
+        self._check(ops.linear(x, w, b), x, w, b, False)
+        self._check(ops.linear_gelu(x, w, b), x, w, b, True)
+        # what the kernel does not read: odd offsets, rows of rows, gradients
+        odd = torch.randn(N * 768 + 1, device=dev, dtype=torch.bfloat16)[1:].view(N, 768)
+        self._check(ops.linear(odd, w, b), odd, w, b, False)
+        assert ops.linear(x.view(1, N, 768), w, b).shape == (1, N, 768)
+        xg = x.clone().requires_grad_()
+        assert ops.linear(xg, w, b).requires_grad
+
+    def test_gelu_tails(self, dev):
+        """gelu alone: the product passes x through one column of ones."""
+        import kserve_amd_C
+
+        v = torch.cat([torch.linspace(-14, 14, 4001), torch.tensor([0.0, -0.0, 40.0, 3e38])])
+        x = torch.zeros(v.numel(), 64, device=dev, dtype=torch.bfloat16)
+        x[:, 0] = v.to(dev, torch.bfloat16)
+        w = torch.zeros(8, 64, device=dev, dtype=torch.bfloat16)
+        w[:, 0] = 1.0
+        out = torch.empty(v.numel(), 8, device=dev, dtype=torch.bfloat16)
+        kserve_amd_C.dense_gemm(out, x, w, None, True)
+        z = x[:, 0].double().cpu()
+        y = z * 0.5 * torch.special.erfc(-z / 2**0.5)
+        # the fit's 6.5e-7, 32-bit exponents up to 100 and bf16's rounding; results
+        # below the smallest normal number may vanish
+        err = (out[:, 0].double().cpu() - y).abs()
+        assert (err <= 2.0**-8 * y.abs() + 2e-38).all()
+
+
 class TestFusedProjections:
     """The kernels that take a few-row GEMM's K splits, and the one-pass
     rotation and scatter, against fp64 and against the separate ops."""
