@@ -788,6 +788,24 @@ def _scan_in_chunks(
     return max(rounds * chunk * (1 + 0.75 * (chunks - 1)), last) < walk
 
 
+def _scan_chunks_apart(tokens: int, seqs: int, longest: int, heads: int, P: int) -> bool:
+    """Whether the scan in chunks forms what needs no state in a launch of its own.
+    Both times are estimated, in us, for 64 heads of 64 columns and 128 states: one
+    launch pays every chunk its chain of barriers, a block a compute unit; two pay the
+    launch and run two blocks a unit, or smaller ones on units that would be idle.
+    (One / two launches: 1 x 64 tokens 12.8 / 17.4, 1 x 100 21.6 / 20.2, 2 x 100 22.3
+    / 25.1, 4 x 200 46.0 / 47.3, 8 x 128 51.9 / 51.0, 6 x 130 64.9 / 53.5, 32 x 64 104 /
+    100, 32 x 100 179 / 153, 40 + 300 49.4 / 33.2.)"""
+    if seqs == 0:
+        return False
+    blocks = -(-P // 64) * heads * seqs
+    most = -(-max(longest, -(-tokens // seqs)) // 64)  # chunks
+    average = min(most, tokens / seqs / 64 + 0.5)
+    one = 4 + 0.0133 * blocks + 9.3 * max(most, average * -(-blocks // 256))
+    a_chunk = max(1.5 + 0.0245 * blocks, 0.031 * blocks)
+    return 14 + 0.012 * blocks + max(3.1 * most, average * a_chunk) < one
+
+
 def ssd_scan(
     xbc, dt_raw, dt_bias, a_log, d_skip, state, positions, cu_seqlens, slots,
     groups: int, longest: int = 0,
@@ -801,9 +819,10 @@ def ssd_scan(
         _native_seq("ssd_scan").ssd_scan(
             y, xbc, dt_raw, dt_bias, a_log, d_skip, state, positions,
             cu_seqlens, slots, int(groups),
-            _scan_in_chunks(
+            0 if not _scan_in_chunks(
                 xbc.shape[0], slots.numel(), longest, heads, P, state.shape[3]
-            ),
+            )
+            else 1 + _scan_chunks_apart(xbc.shape[0], slots.numel(), longest, heads, P),
         )
         return y
     return torch_ref.ssd_scan(

@@ -20,10 +20,11 @@ hipError_t ks_causal_conv_silu(void*, const void*, long, const void*,
                                const void*, void*, const void*, const void*,
                                const void*, const void*, int, int, int, int,
                                int, int, int, hipStream_t);
+long ks_ssd_work_bytes(int, int, int);
 hipError_t ks_ssd_scan(void*, const void*, const void*, long, int, const void*,
                        const void*, const void*, void*, const void*,
                        const void*, const void*, int, int, int, int, int, int,
-                       int, hipStream_t);
+                       int, void*, hipStream_t);
 hipError_t ks_qk_norm_temp_cache(void*, const void*, const void*, const void*,
                                  long, const void*, const void*, const void*,
                                  const void*, void*, void*, float, float, int,
@@ -319,7 +320,7 @@ void causal_conv_silu(at::Tensor& out, at::Tensor& in, at::Tensor& w,
 void ssd_scan(at::Tensor& y, at::Tensor& xbc, at::Tensor& dt_raw,
               at::Tensor& dt_bias, at::Tensor& a_log, at::Tensor& d_skip,
               at::Tensor& state, at::Tensor& positions, at::Tensor& cu_seqlens,
-              at::Tensor& slots, int64_t groups, bool chunks) {
+              at::Tensor& slots, int64_t groups, int64_t chunks) {
   CHECK_F32(y);
   CHECK_F32(xbc);
   CHECK_F32(dt_bias);
@@ -341,13 +342,20 @@ void ssd_scan(at::Tensor& y, at::Tensor& xbc, at::Tensor& dt_raw,
                   d_skip.numel() == heads && positions.numel() >= tokens &&
                   cu_seqlens.numel() == num_seqs + 1,
               "ssd_scan: shape mismatch");
+  // chunks: 0 token by token, 1 in chunks in one launch, 2 in two launches (3, 4: with
+  // 16 or 32 columns a block)
+  TORCH_CHECK(chunks >= 0 && chunks <= 4, "chunks");
+  at::Tensor work;
+  if (chunks > 1)
+    work = at::empty({ks_ssd_work_bytes(tokens, num_seqs, heads)}, y.options().dtype(at::kByte));
   check_hip(ks_ssd_scan(y.data_ptr(), xbc.data_ptr(), dt_raw.data_ptr(),
                         dt_raw.stride(0), act_is_f32(dt_raw, "dt_raw"),
                         dt_bias.data_ptr(), a_log.data_ptr(),
                         d_skip.data_ptr(), state.data_ptr(),
                         positions.data_ptr(), cu_seqlens.data_ptr(),
                         slots.data_ptr(), tokens, num_seqs, heads, (int)groups,
-                        P, N, chunks ? 1 : 0, current_stream()),
+                        P, N, (int)chunks, chunks > 1 ? work.data_ptr() : nullptr,
+                        current_stream()),
             "ssd_scan");
 }
 

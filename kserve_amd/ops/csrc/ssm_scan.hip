@@ -517,8 +517,8 @@ __global__ void __launch_bounds__(256) ssd_step_kernel(
 
 // ---------------------------------------------------------------------------
 // The scan in chunks of 64 tokens on the fp32 matrix cores
-// (v_mfma_f32_16x16x4_f32), for portions that are long enough to fill chunks.
-// With c_t the running sum of A dt inside the chunk and S the state at its
+// (v_mfma_f32_16x16x4_f32), in one launch: for portions of one or two chunks (the
+// form after it takes the longer ones). With c_t the running sum of A dt inside the chunk and S the state at its
 // start:
 //     y_t = exp(c_t) S^T C_t + sum_{s <= t} (C_t . B_s) exp(c_t - c_s) dt_s x_s
 //           + D x_t
@@ -537,10 +537,7 @@ __global__ void __launch_bounds__(256) ssd_step_kernel(
 // cycles each, two waves per SIMD (5.6 us of the 10 us that a chunk takes).
 // Token by token a chunk took 64 times the latency of one step (LDS reads,
 // update, lane tree), whatever the arithmetic. 64 heads of 64 columns, 128
-// states: 4 x 2000 tokens 1855 -> 320 us, 8 x 2000 1962 -> 627 us, 1 x 2000
-// 1793 -> 299 us, 1 x 40 43 -> 13 us; one wave per column block with all states
-// (4 waves) took 391 us for 4 x 2000. Error against 64 bits, mean over portions
-// of 50 to 400 tokens: y 8.0e-8 both, state 8.3e-8 -> 7.9e-8.
+// states: 1 x 40 tokens 43 -> 13 us, 4 x 64 16, 8 x 20 25.
 // ---------------------------------------------------------------------------
 constexpr int CQ = 64;  // tokens per chunk
 constexpr int CT = 512;
@@ -806,7 +803,440 @@ __global__ void __launch_bounds__(CT) ssd_chunk_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same in two launches, for longer portions. What needs no state comes first,
+// for all chunks at once: the products C_t . B_s of a group of heads (the 10 16 x 16
+// tiles on and below the diagonal) and, per head, the running sums, these products
+// with decay and step size, and the weights of the recurrence. The scan is then a
+// chain of three products a chunk. A block takes 16 CB columns (p) of one head of
+// one sequence. Each of its 4 waves owns a quarter of the states, S^T in
+// accumulator layout, and a quarter of a chunk's tokens: it moves its states on with
+// B and x from LDS, hands them to the others through LDS and forms its own tokens'
+// y with C and the decayed products from registers. Two barriers a chunk; the next
+// chunk's rows are on their way in registers meanwhile.
+//
+// The one-launch form took 10 us a chunk, 5.6 of them products: an inclusive sum in
+// 64 bits, 64 x 64 exponentials and three barriers stood between them, with one
+// block a compute unit. Here two blocks of 32 columns share a unit (7.8 us a chunk
+// of both, 4.2 of them products, 160 per wave and block) and a block alone takes
+// 4.7 us, of 16 columns 3.0. The first launch moves 19 KB a chunk and head at 3.5
+// TB/s (44 us for 8000 tokens of 64 heads). us, one launch / two (64 heads of 64
+// columns, 128 states): 4 x 2000 tokens 308 / 260, 1 x 2000 296 / 107, 1 x 8000
+// 1154 / 398, 8 x 2000 628 / 518, 32 x 128 187 / 164, 1 x 100 21.6 / 20.2, 4 x 64
+// 15.5 / 27. Error of y against 64 bits 8.5e-8 both.
+// ---------------------------------------------------------------------------
+constexpr int CTILES = 10;
+
+// Chunks are numbered over the batch with gaps: those of sequence s from here on.
+__device__ __forceinline__ int chunk_base(int first, int s) { return first / CQ + s; }
+
+// 16 bytes at a byte offset from a uniform address, 0 past `bytes`: rows after a
+// portion and columns after a head cost no branch and no address registers
+__device__ __forceinline__ f32x4s load_or_zero(const float* base, unsigned int bytes,
+                                               unsigned int at) {
+  const __amdgpu_buffer_rsrc_t rows =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, bytes, 0x00027000);
+  return __builtin_bit_cast(f32x4s, __builtin_amdgcn_raw_buffer_load_b128(rows, at, 0, 0));
+}
+__device__ __forceinline__ void store_or_drop(float* base, unsigned int bytes,
+                                              unsigned int at, float v) {
+  const __amdgpu_buffer_rsrc_t rows =
+      __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000);
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), rows, at, 0, 0);
+}
+constexpr unsigned int OUTSIDE = 0x80000000u;
+
+// tile i of the 64 x 64 products: token block tb, and the block sb <= tb before it
+__device__ __forceinline__ void chunk_tile(int i, int& tb, int& sb) {
+  tb = i < 1 ? 0 : i < 3 ? 1 : i < 6 ? 2 : 3;
+  sb = i - tb * (tb + 1) / 2;
+}
+
+// what the scan takes per chunk and head from the pass before it
+struct ChunkWork {
+  f32x4s m[CTILES][64];  // tile (tb, sb) at tb (tb + 1) / 2 + sb: lane 16 g + t has
+                         // (C_t . B_s) exp(c_t - c_s) dt_s for s = 4 g .. 4 g + 3
+  float grow[CQ];        // exp(c_t)
+  float left[CQ];        // exp(c_end - c_t) dt_t
+};
+constexpr int ST = 256, DT = 512, HEADS_PER_BLOCK = DT / 64;
+
+template <int NB>  // blocks of 16 states: N <= 16 NB
+__global__ void __launch_bounds__(DT) ssd_decays_kernel(
+    ChunkWork* __restrict__ work, const float* __restrict__ xbc,
+    const float* __restrict__ dt_raw_f32, const short* __restrict__ dt_raw_bf16,
+    long dt_stride, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
+    const int* __restrict__ cu_seqlens, int seqs, int heads, int groups, int P, int N) {
+  constexpr int NW = DT / 64;
+  constexpr int NG = (CTILES + NW - 1) / NW;
+  // running sums in 64 bits, for powers of two: their differences are exponents, and
+  // a sum over a chunk may be far larger than the difference of two neighbours
+  __shared__ double cum[NW][CQ];
+  __shared__ float dts[NW][CQ];
+  const int chunk = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  int s = -1;  // the last sequence that starts at or before this chunk
+  for (int i = 0; i < seqs; i += 64) {
+    const int k = i + lane;
+    s += __popcll(__ballot(k < seqs && chunk_base(cu_seqlens[min(k, seqs - 1)], k) <= chunk));
+  }
+  if (s < 0) return;
+  const int first = cu_seqlens[s], end = cu_seqlens[s + 1];
+  const int t0 = first + (chunk - chunk_base(first, s)) * CQ;
+  if (t0 < first || t0 >= end) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  const int per = heads / groups;
+  const int parts = cdiv(per, HEADS_PER_BLOCK);
+  const int grp = blockIdx.y / parts;
+  const int h0 = grp * per + blockIdx.y % parts * HEADS_PER_BLOCK;
+  const int h_end = min(h0 + HEADS_PER_BLOCK, (grp + 1) * per);
+  const int inner = heads * P;
+  const long channels = inner + 2L * groups * N;
+
+  f32x4s cb[NG];  // B_s . C_t: row s, column t
+#pragma unroll
+  for (int i = 0; i < NG; ++i) {
+    if (wave + i * NW >= CTILES) continue;
+    int tb, sb;
+    chunk_tile(wave + i * NW, tb, sb);
+    const int t = t0 + tb * 16 + col, u = t0 + sb * 16 + col;
+    const float* cr = xbc + t * channels + inner + (groups + grp) * N + g * 4;
+    const float* br = xbc + u * channels + inner + grp * N + g * 4;
+    const f32x4s zero = f32x4s{0.f, 0.f, 0.f, 0.f};
+    f32x4s c4[NB], b4[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const bool ok = b * 16 + g * 4 < N;
+      c4[b] = ok && t < end ? *reinterpret_cast<const f32x4s*>(cr + b * 16) : zero;
+      b4[b] = ok && u < end ? *reinterpret_cast<const f32x4s*>(br + b * 16) : zero;
+    }
+    // eight chains: fewer roundings in a row than one sum over the states
+    f32x4s acc[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) acc[r] = zero;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        f32x4s& to = acc[r + (b & 1) * 4];
+        to = mfma4(b4[b][r], c4[b][r], to);
+      }
+    cb[i] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
+  }
+
+  for (int hb = h0; hb < h_end; hb += NW) {
+    __syncthreads();
+    if (hb + wave < h_end) {
+      const int h = hb + wave;
+      // finite where exp leaves the range: differences of infinite running sums
+      // would be NaN where the decay is 0
+      float A = -expf(a_log[h]);
+      if (A < -FLT_MAX) A = -FLT_MAX;
+      const long i = (long)min(t0 + lane, end - 1) * dt_stride + h;
+      const float v =
+          (dt_raw_f32 ? dt_raw_f32[i] : bf16_bits_to_float(dt_raw_bf16[i])) + dt_bias[h];
+      // softplus without a clamp; log1p(exp(v)) is v itself past v ~ 30.
+      // Rows past the portion: dt 0, so they change nothing
+      const float dt = t0 + lane < end ? (v > 30.f ? v : log1pf(expf(v))) : 0.f;
+      double c = (double)A * dt * 1.4426950408889634;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_up(c, off, 64);
+        if (lane >= off) c += o;
+      }
+      const double last = __shfl(c, 63, 64);
+      cum[wave][lane] = c;
+      dts[wave][lane] = dt;
+      ChunkWork& to = work[(long)chunk * heads + h];
+      to.grow[lane] = __builtin_amdgcn_exp2f((float)c);
+      to.left[lane] = dt * __builtin_amdgcn_exp2f((float)(last - c));
+    }
+    __syncthreads();
+    for (int k = 0; k < NW && hb + k < h_end; ++k) {
+      ChunkWork& to = work[(long)chunk * heads + hb + k];
+#pragma unroll
+      for (int i = 0; i < NG; ++i) {
+        if (wave + i * NW >= CTILES) continue;
+        int tb, sb;
+        chunk_tile(wave + i * NW, tb, sb);
+        const int t = tb * 16 + col;
+        f32x4s m;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int u = sb * 16 + g * 4 + r;
+          const float d = (float)(cum[k][t] - cum[k][u]);
+          // (later tokens: whatever it is, it is not taken)
+          const float e = cb[i][r] * __builtin_amdgcn_exp2f(d) * dts[k][u];
+          m[r] = u <= t ? e : 0.f;
+        }
+        to.m[wave + i * NW][lane] = m;
+      }
+    }
+  }
+}
+
+template <int NB, int CB>  // blocks of 16 states and columns
+__global__ void __launch_bounds__(ST, 2) ssd_chain_kernel(
+    float* __restrict__ y, const float* __restrict__ xbc, const ChunkWork* __restrict__ work,
+    const float* __restrict__ d_skip, float* __restrict__ state,
+    const long* __restrict__ positions, const int* __restrict__ cu_seqlens,
+    const int* __restrict__ slots, int heads, int groups, int P, int N) {
+  constexpr int NW = ST / 64;
+  constexpr int NP = NB * 16, PB = CB * 16;
+  constexpr int RS = NP + 4;  // B and state rows: 4 rows apart fall 16 banks apart
+  constexpr int XS = PB + 4;
+  constexpr int NH = NB / NW;           // state blocks of a wave
+  constexpr int NV = CQ * NP / 4 / ST;  // float4 per thread of a B tile
+  constexpr int XV = CQ * PB / 4 / ST;
+  static_assert(NH * NW == NB && XV * ST * 4 == CQ * PB && CQ == 16 * NW, "tile");
+  __shared__ __attribute__((aligned(16))) float Bs[CQ * RS];
+  __shared__ __attribute__((aligned(16))) float Xs[CQ * XS];
+  __shared__ __attribute__((aligned(16))) float Ss[PB * RS];  // by column
+  __shared__ __attribute__((aligned(16))) float left[CQ];
+
+  const int s = blockIdx.z, h = blockIdx.y;
+  const int first = cu_seqlens[s];
+  const int len = cu_seqlens[s + 1] - first;
+  if (len <= 0) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p0 = blockIdx.x * PB;
+  const int grp = h / (heads / groups);
+  const int inner = heads * P;
+  const int channels = inner + 2 * groups * N;
+  const float Dh = d_skip[h];
+  const f32x4s zero = f32x4s{0.f, 0.f, 0.f, 0.f};
+  float* sp = state + ((slots[s] * (long)heads + h) * P + p0) * N;
+
+  // byte offsets within a chunk's rows: of B, of x, of C (this wave's tokens)
+  const unsigned int row4 = (unsigned int)channels * 4;
+  const int bn = threadIdx.x % (NP / 4) * 4, xn = threadIdx.x % (PB / 4) * 4;
+  const unsigned int b_at = bn < N ? threadIdx.x / (NP / 4) * row4 + bn * 4 : OUTSIDE;
+  const unsigned int x_at =
+      p0 + xn < P ? threadIdx.x / (PB / 4) * row4 + xn * 4 : OUTSIDE;
+  const int c_n = (threadIdx.x & 63) / 16 * 4;
+  const unsigned int c_at = (wave * 16 + (threadIdx.x & 15)) * row4 + c_n * 4;
+  const float* seq_rows = xbc + (long)first * channels;
+  const ChunkWork* seq_work = work + (long)chunk_base(first, s) * heads + h;
+
+  f32x4s rB[NV], rX[XV], rC[NB], rM[NW], rE;
+  float rL = 0.f, keep = 0.f, keep_next;
+  auto fetch_rows = [&](int t0) {
+    const float* rows = seq_rows + (long)t0 * channels;
+    const unsigned int last = (unsigned int)(min(len - t0, CQ) - 1) * row4;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      rB[i] = load_or_zero(rows + inner + grp * N, last + N * 4,
+                           b_at + i * (ST / (NP / 4)) * row4);
+#pragma unroll
+    for (int i = 0; i < XV; ++i)
+      rX[i] = load_or_zero(rows + h * P + p0, last + (P - p0) * 4,
+                           x_at + i * (ST / (PB / 4)) * row4);
+    const ChunkWork& w = seq_work[(long)(t0 / CQ) * heads];
+    rL = w.left[threadIdx.x % CQ];
+    keep_next = w.grow[CQ - 1];
+  };
+  auto fetch_c = [&](int t0) {
+    const float* rows = seq_rows + (long)t0 * channels + inner + (groups + grp) * N;
+    const unsigned int last = (unsigned int)(min(len - t0, CQ) - 1) * row4;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      rC[b] = load_or_zero(rows, last + N * 4, c_n + b * 16 < N ? c_at + b * 64 : OUTSIDE);
+  };
+  auto fetch_products = [&](int t0) {
+    const ChunkWork& w = seq_work[(long)(t0 / CQ) * heads];
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int sb = 0; sb < NW; ++sb)
+      rM[sb] = w.m[wave * (wave + 1) / 2 + min(sb, wave)][lane];
+    rE = *reinterpret_cast<const f32x4s*>(w.grow + wave * 16 + lane / 16 * 4);
+  };
+
+  f32x4s S[NH][CB];
+  {
+    const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+    const bool fresh = positions[first] == 0;
+#pragma unroll
+    for (int b = 0; b < NH; ++b)
+#pragma unroll
+      for (int k = 0; k < CB; ++k) {
+        const int n = (wave * NH + b) * 16 + g * 4, c = k * 16 + col;
+        S[b][k] = (!fresh && p0 + c < P && n < N)
+                      ? *reinterpret_cast<const f32x4s*>(sp + (long)c * N + n)
+                      : zero;
+      }
+  }
+
+  // (in the loop's order, which its waits count by)
+  fetch_rows(0);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_c(0);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch_products(0);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int t0 = 0; t0 < len; t0 += CQ) {
+    const int cnt = min(CQ, len - t0);
+    // (the last chunk fetches itself again: were its loads left out, the waits for
+    // the others would have to assume so in every chunk)
+    const int next = t0 + CQ < len ? t0 + CQ : t0;
+    // (lane numbers that the compiler takes for new ones: it keeps every address of
+    // the chunk in a register from before the loop otherwise, more than there are)
+    unsigned int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, col = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const unsigned int e = tid + i * ST;
+      *reinterpret_cast<f32x4s*>(Bs + e / (NP / 4) * RS + e % (NP / 4) * 4) = rB[i];
+    }
+#pragma unroll
+    for (int i = 0; i < XV; ++i) {
+      const unsigned int e = tid + i * ST;
+      *reinterpret_cast<f32x4s*>(Xs + e / (PB / 4) * XS + e % (PB / 4) * 4) = rX[i];
+    }
+    if (wave == 0) left[lane] = rL;
+    keep = keep_next;
+#pragma unroll
+    for (int b = 0; b < NH; ++b)
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        *reinterpret_cast<f32x4s*>(Ss + (k * 16 + col) * RS + (wave * NH + b) * 16 + g * 4) =
+            S[b][k];
+    __syncthreads();
+    fetch_rows(next);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // LDS reads go a step ahead of the products that want them, 8 or 16 products of
+    // 32 cycles: left to itself the compiler reads each operand as it is wanted
+    f32x4s X[4][CB];  // tokens 16 tb + 4 g + r, this lane's columns
+    {
+      const float* xrow = Xs + g * 4 * XS + col;
+#pragma unroll
+      for (int tb = 0; tb < 4; ++tb)
+#pragma unroll
+        for (int k = 0; k < CB; ++k)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) X[tb][k][r] = xrow[(tb * 16 + r) * XS + k * 16];
+    }
+
+    // ---- what the state at the chunk's start contributes to this wave's tokens ----
+    f32x4s Y[CB][4];  // four chains: fewer roundings in a row
+#pragma unroll
+    for (int k = 0; k < CB; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) Y[k][r] = zero;
+    f32x4s s4[2][CB];
+    auto states = [&](int b) {
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        s4[b & 1][k] =
+            *reinterpret_cast<const f32x4s*>(Ss + (k * 16 + col) * RS + b * 16 + g * 4);
+    };
+    states(0);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (b + 1 < NB) states(b + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int k = 0; k < CB; ++k) Y[k][r] = mfma4(rC[b][r], s4[b & 1][k][r], Y[k][r]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    fetch_c(next);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- and the chunk's own tokens ----
+#pragma unroll
+    for (int k = 0; k < CB; ++k) {
+      f32x4s acc[4], x = zero;  // x ends as this wave's tokens' own
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = zero;
+#pragma unroll
+      for (int sb = 0; sb < NW; ++sb) {
+        if (sb > wave) continue;
+        x = X[sb][k];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[r] = mfma4(rM[sb][r], x[r], acc[r]);
+      }
+      f32x4s z = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+      const f32x4s past = ((Y[k][0] + Y[k][1]) + (Y[k][2] + Y[k][3])) * rE;
+      z += past;
+      // The products above take later tokens of the tile with weight 0, which
+      // is no 0 if their x is infinite or NaN: such sums are formed again, from
+      // the tokens up to each row's own only.
+      const float size = fabsf(z[0]) + fabsf(z[1]) + fabsf(z[2]) + fabsf(z[3]);
+      if (__any(!(size < INFINITY))) {
+        const ChunkWork& w = seq_work[(long)(t0 / CQ) * heads];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int t = g * 4 + r;
+          float sum = 0.f;
+          for (int u = 0; u <= wave * 16 + t; ++u)
+            sum = fmaf(w.m[wave * (wave + 1) / 2 + u / 16][u % 16 / 4 * 16 + t][u % 4],
+                       Xs[u * XS + k * 16 + col], sum);
+          z[r] = sum + past[r];
+        }
+      }
+      float* yrows = y + (long)(first + t0) * inner + h * P + p0;
+      const unsigned int ybytes = ((cnt - 1) * inner + (P - p0)) * 4;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const unsigned int at = ((wave * 16 + g * 4 + r) * inner + k * 16 + col) * 4;
+        store_or_drop(yrows, ybytes, p0 + k * 16 + col < P ? at : OUTSIDE, z[r] + Dh * x[r]);
+      }
+    }
+    fetch_products(next);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the state moves on ----
+    f32x4s w4[2], b4[2][NH];  // of a block of 16 tokens: weights, B by token
+    auto tokens = [&](int tb) {
+      w4[tb & 1] = *reinterpret_cast<const f32x4s*>(left + tb * 16 + g * 4);
+      const float* brow = Bs + (tb * 16 + g * 4) * RS + wave * NH * 16 + col;
+#pragma unroll
+      for (int b = 0; b < NH; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) b4[tb & 1][b][r] = brow[r * RS + b * 16];
+    };
+    tokens(0);
+#pragma unroll
+    for (int b = 0; b < NH; ++b)
+#pragma unroll
+      for (int k = 0; k < CB; ++k) S[b][k] *= keep;
+#pragma unroll
+    for (int tb = 0; tb < 4; ++tb) {
+      if (tb < 3) tokens(tb + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < CB; ++k) X[tb][k] *= w4[tb & 1];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int k = 0; k < CB; ++k)
+#pragma unroll
+          for (int b = 0; b < NH; ++b)
+            S[b][k] = mfma4(b4[tb & 1][b][r], X[tb][k][r], S[b][k]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // the chunk's tiles are consumed
+  }
+  const int lane = threadIdx.x & 63, col = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int b = 0; b < NH; ++b)
+#pragma unroll
+    for (int k = 0; k < CB; ++k) {
+      const int n = (wave * NH + b) * 16 + g * 4, c = k * 16 + col;
+      if (p0 + c < P && n < N) *reinterpret_cast<f32x4s*>(sp + (long)c * N + n) = S[b][k];
+    }
+}
+
 }  // namespace
+
+// bytes that the scan in chunks takes for what needs no state
+extern "C" long ks_ssd_work_bytes(int tokens, int num_seqs, int heads) {
+  return ((long)tokens / CQ + num_seqs) * heads * (long)sizeof(ChunkWork);
+}
 
 extern "C" hipError_t ks_causal_conv_silu(
     void* out, const void* in, long in_stride, const void* w, const void* bias,
@@ -917,26 +1347,61 @@ extern "C" hipError_t ks_ssd_scan(void* y, const void* xbc, const void* dt_raw,
                                   const void* cu_seqlens, const void* slots,
                                   int tokens, int num_seqs, int heads,
                                   int groups, int P, int N, int chunks,
-                                  hipStream_t stream) {
+                                  void* work, hipStream_t stream) {
   if (num_seqs == 0) return hipSuccess;
   if (groups <= 0 || heads % groups != 0 || N < 1 || N > 256)
     return hipErrorInvalidValue;
   if (chunks && N % 4 == 0 && N <= 128 && P % 4 == 0 &&
       (((uintptr_t)xbc | (uintptr_t)state) & 15) == 0) {
-    const dim3 cgrid(cdiv(P, 64), heads, num_seqs);
+#define SSD_DT                                                                \
+  dt_is_f32 ? (const float*)dt_raw : nullptr,                                 \
+      dt_is_f32 ? nullptr : (const short*)dt_raw, dt_stride,                  \
+      (const float*)dt_bias, (const float*)a_log
+    if (!work) {
+      const dim3 cgrid(cdiv(P, 64), heads, num_seqs);
 #define SSD_CHUNK(nb)                                                         \
   hipLaunchKernelGGL((ssd_chunk_kernel<nb>), cgrid, dim3(CT), 0, stream,      \
-                     (float*)y, (const float*)xbc,                            \
-                     dt_is_f32 ? (const float*)dt_raw : nullptr,              \
-                     dt_is_f32 ? nullptr : (const short*)dt_raw, dt_stride,   \
-                     (const float*)dt_bias, (const float*)a_log,              \
+                     (float*)y, (const float*)xbc, SSD_DT,                    \
                      (const float*)d_skip, (float*)state,                     \
                      (const long*)positions, (const int*)cu_seqlens,          \
                      (const int*)slots, heads, groups, P, N)
-    if (N <= 32) SSD_CHUNK(2);
-    else if (N <= 64) SSD_CHUNK(4);
-    else SSD_CHUNK(8);
+      if (N <= 32) SSD_CHUNK(2);
+      else if (N <= 64) SSD_CHUNK(4);
+      else SSD_CHUNK(8);
 #undef SSD_CHUNK
+      HIP_CHECK_KERNEL();
+      return hipSuccess;
+    }
+    if (((uintptr_t)work & 15) != 0) return hipErrorInvalidValue;
+    const dim3 pgrid((unsigned)(tokens / CQ + num_seqs),
+                     groups * cdiv(heads / groups, HEADS_PER_BLOCK));
+    // 32 columns a block, or 16 where the chip has room for twice the blocks
+    // (64 heads of 64 columns, 8000 tokens of 1 / 2 / 4 sequences: 568 / 398, 157 /
+    // 158, 260 / 327 us)
+    const int cb =
+        chunks > 2 ? chunks - 2 : P <= 16 || cdiv(P, 32) * (long)heads * num_seqs <= 192 ? 1 : 2;
+    const dim3 cgrid(cdiv(P, 16 * cb), heads, num_seqs);
+#define SSD_CHAIN(nb, cbs)                                                    \
+  hipLaunchKernelGGL((ssd_chain_kernel<nb, cbs>), cgrid, dim3(ST), 0, stream, \
+                     (float*)y, (const float*)xbc, (const ChunkWork*)work,    \
+                     (const float*)d_skip, (float*)state,                     \
+                     (const long*)positions, (const int*)cu_seqlens,          \
+                     (const int*)slots, heads, groups, P, N)
+#define SSD_CHAINS(nb)                                                        \
+  do {                                                                        \
+    hipLaunchKernelGGL((ssd_decays_kernel<nb>), pgrid, dim3(DT), 0, stream,   \
+                       (ChunkWork*)work, (const float*)xbc, SSD_DT,           \
+                       (const int*)cu_seqlens, num_seqs, heads, groups, P,    \
+                       N);                                                    \
+    HIP_CHECK_KERNEL();                                                       \
+    if (cb == 1) SSD_CHAIN(nb, 1);                                            \
+    else SSD_CHAIN(nb, 2);                                                    \
+  } while (0)
+    if (N <= 64) SSD_CHAINS(4);
+    else SSD_CHAINS(8);
+#undef SSD_CHAINS
+#undef SSD_CHAIN
+#undef SSD_DT
     HIP_CHECK_KERNEL();
     return hipSuccess;
   }

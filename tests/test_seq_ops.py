@@ -415,6 +415,48 @@ class TestScan:
             # fp32 sums of at most 130 + 128 terms against the largest output
             close(torch.cat(g), w, be, f32_tol=5e-6, bf16_tol=5e-6)
 
+    @pytest.mark.gpu
+    @pytest.mark.parametrize("form", [1, 2, 3, 4])
+    @pytest.mark.parametrize(
+        "H,G,P,N", [(2, 1, 64, 128), (9, 1, 20, 16), (4, 2, 72, 100), (3, 3, 8, 36)]
+    )
+    def test_every_form_in_chunks(self, form, H, G, P, N):
+        """Portions at the chunks' edges, one empty and one of a single token among
+        them, fresh and continued; y and the states left behind."""
+        import kserve_amd_seq_C
+
+        be = ("cuda", torch.bfloat16)
+        lens, had = (64, 0, 1, 129, 63, 200), (0, 0, 7, 0, 64, 3)
+        inner = H * P
+        dt_bias, a_log, d_skip = rnd(H, seed=102) - 1.0, rnd(H, seed=103), rnd(H, seed=104)
+        T = sum(lens)
+        xbc, dt_raw = rnd(T, inner + 2 * G * N, seed=105, scale=0.7), rnd(T, H, seed=106, dtype=be[1])
+        before = rnd(7, H, P, N, seed=107)
+        slots = [3, 1, 6, 5, 2, 4]
+        cu, _, pos = layout(list(lens), list(had))
+        state, y = f32(before, be), torch.full((T + 1, inner), 9.0, device="cuda")
+        kserve_amd_seq_C.ssd_scan(
+            y[:T], f32(xbc, be), act(dt_raw, be), f32(dt_bias, be), f32(a_log, be),
+            f32(d_skip, be), state, i64(pos, be), i32(cu, be), i32(slots, be), G, form,
+        )
+        dt = O.softplus(dt_raw.double() + dt_bias.double())
+        want, after = torch.empty(T, inner, dtype=F64), before.double()
+        for n, h0, a, slot in zip(lens, had, cu, slots):
+            S = after[slot] if h0 else torch.zeros(H, P, N, dtype=F64)
+            for t in range(a, a + n):
+                x = xbc[t, :inner].double().view(H, P)
+                B = xbc[t, inner:inner + G * N].double().view(G, N).repeat_interleave(H // G, 0)
+                C = xbc[t, inner + G * N:].double().view(G, N).repeat_interleave(H // G, 0)
+                S = S * torch.exp(-a_log.double().exp() * dt[t])[:, None, None] + (
+                    dt[t][:, None] * x)[:, :, None] * B[:, None]
+                want[t] = ((S * C[:, None]).sum(-1) + d_skip.double()[:, None] * x).view(-1)
+            if n:
+                after[slot] = S
+        # fp32 sums of at most 200 + 128 terms against the largest output
+        close(y[:T], want, be, bf16_tol=5e-6)
+        close(state, after, be, bf16_tol=5e-6)
+        assert (y[T] == 9.0).all()
+
     @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
     def test_bad_inputs_stay_behind_them(self, be, bad):
         """An infinity or a NaN in one column at one token reaches that column
