@@ -286,7 +286,9 @@ def random_sample(
 
 
 def _skinny_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    return x.shape[0] <= 256 and _plain_operands(x, weight)
+    n = x.shape[0]
+    # (above 64 rows: 32-bit offsets within a tile; the rules bound K)
+    return (n <= 64 or n <= 256 and x.stride(0) < 1 << 22) and _plain_operands(x, weight)
 
 
 def _plain_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
@@ -333,18 +335,21 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     83), up to 64 rows but for the widest (m 14336 28.3 / 27.5). So far a row's
     sums do not depend on the rows beside it, and small weights stay here for
     that. Above, it gains where the
-    library does not split K over the chip: k 14336, m 4096 at 128 rows 35 / 76,
-    k 4096, m 6144 22 / 26, k 3072, m 6144 20 / 21; and loses on short K (k 2048,
-    m 8192 18.7 / 16.3, k 2560, m 8192 21.0 / 19.9), small weights (2048 x 2048
-    15 / 11) and wide ones (m 16384 44 / 38). Past 192 rows the lighter of the
-    former turn (4096 x 4096 27 / 23 at 256 rows; m 6144 33 / 40)."""
+    library does not split K over the chip: k 14336, m 4096 at 128 / 256 rows 34 / 74,
+    46 / 62, k 8192, m 2048 at 77 / 256 rows 15 / 21, 21 / 27, k 4096, m 4096 at 128
+    rows 16 / 25, k 4096, m 6144 22 / 25, at 256 rows 32 / 40, k 3072, m 6144 20 / 21;
+    and loses on short K (k 2048, m 8192 18.7 / 16.3, k 2560, m 8192 21.0 / 19.9), small
+    weights (2048 x 2048 15 / 11) and wide ones (m 16384 27 / 21). Past 192 rows the
+    lighter of the former turn (4096 x 4096 level at 256 rows)."""
     if m % 4 or n > 256:
         return False
     if n <= 48 or (n <= 64 and m <= 8192):
         return True
+    if 2048 <= m < 4096:
+        return 8192 <= k < 1 << 22
     return (
         4096 <= m <= 10240
-        and k >= 3072
+        and 3072 <= k < 1 << 22
         and k * m >= (16 if n <= 192 else 24) << 20
     )
 

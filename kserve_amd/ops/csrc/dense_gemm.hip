@@ -7,14 +7,16 @@
 // PFLOP/s with a pass over memory of its own for gelu. Each step's token and
 // weight rows come by LDS-direct loads into one slot of a ring; a wave reads the
 // fragments of a half step while it multiplies those of the half before, with one
-// barrier per step. What bounds it is the rate at which one compute unit takes
-// lines in, about 27 bytes a cycle whatever the tile or the depth of the ring (a
-// ring of 32-wide steps, 64-byte rows, took 20): so tiles are as large as the
-// token count lets them be, and where two blocks fit a unit one multiplies while
-// the other starts or ends. No two steps of a row share a bank (0 conflicts).
+// barrier per step, and its reads and loads go between the products. Where a unit
+// has one block, LDS bounds it: 128 bytes a cycle for reads and loads (128 x 192 in
+// 8 waves: 1344 cycles a step, 768 of them products; 1310 measured, 1400 with the
+// reads and loads in a row). Where it has two, the latency of the one step that two
+// slots hold in flight does (1.7 us a step of both); 32-wide steps in four slots took
+// 41 us for 34, their 64-byte rows come at two thirds of the rate. The rows of a
+// fragment never share a bank (0 conflicts).
 //
 // us, this / the library (and gelu's kernel): 7864 x 768 to 2304 33 / 63, to 768
-// 13.9 / 15.1, to 3072 with gelu 50 / 68; 1500 rows to 768 7.2 / 8.7, to 3072 with
+// 13.5 / 15.1, to 3072 with gelu 50 / 68; 1500 rows to 768 7.2 / 8.7, to 3072 with
 // gelu 15.8 / 20.9; 200 rows to 2304 5.8 / 7.9.
 #include "common.h"
 #include "mfma_layouts.h"
@@ -24,8 +26,11 @@ namespace {
 constexpr int UNITS = 256;  // compute units
 constexpr int BK = 64;  // K per step
 
+// sums + bias in bf16; gelu of it; fp32 sums of the K splits
+enum Epilogue { BIAS, BIAS_GELU, PARTIAL };
+
 struct DenseArgs {
-  short* out;         // [N][M]
+  void* out;          // [N][M] bf16; PARTIAL: [splits][N][M] fp32
   const short* x;     // [N][K], row stride xs
   const short* w;     // [M][K]
   const short* bias;  // [M] or null
@@ -65,12 +70,14 @@ __device__ __forceinline__ float gelu_f(float x) {
   return x * (x > 0.f ? 1.f - tail : tail);
 }
 
-template <int TN, int TM, int WN, int WM, int S, bool GELU>
+template <int TN, int TM, int WN, int WM, int S, int EPI>
 __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const DenseArgs p) {
   constexpr int NW = WN * WM;
   constexpr int FN = TN / WN / 16, FM = TM / WM / 16;  // fragments of a wave
   constexpr int STAGE = (TN + TM) * BK;                // elements
   constexpr int NX = TN / 8 / NW, NI = (TN + TM) / 8 / NW;  // 1 KB loads of a wave
+  constexpr int LAG = (FM + FN) / 2;  // a half step's reads end by 2/3 of its products
+  constexpr int N1 = S == 2 ? NI : (NI + 1) / 2;  // of them, right after the barrier
   static_assert(TN % (8 * NW) == 0 && TM % (8 * NW) == 0 && FM % 2 == 0 && S >= 2 &&
                     S * STAGE * 2 <= 160 * 1024,
                 "tile");
@@ -84,23 +91,26 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
   const int xcd = blockIdx.x & 7, nth = blockIdx.x >> 3;
   const int tile = xcd * (p.tiles >> 3) + min(xcd, p.tiles & 7) + nth;
   const int n0 = tile / p.ftiles * TN, m0 = tile % p.ftiles * TM;
+  const int all = p.K / BK;
+  const int lo = (int)((long)all * blockIdx.y / gridDim.y);  // of this K split
+  const int steps = (int)((long)all * (blockIdx.y + 1) / gridDim.y) - lo;
 
   // a load is 8 rows of 128 bytes; 16-byte chunk c of a row sits at c ^ key, the
   // key such that the rows of a fragment at one chunk hit different banks
-  const short *xb = p.x + (long)n0 * p.xs, *wb = p.w + (long)m0 * p.K;
+  const short* xb = p.x + (long)n0 * p.xs + lo * BK;
+  const short* wb = p.w + (long)m0 * p.K + lo * BK;
   unsigned int at[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
     const int r = ((i < NX ? i : i - NX) * NW + wave) * 8 + (lane >> 3);
     const int key = i < NX ? (r >> 1) & 7 : ((r >> 1) & 1) | ((r >> 2) & 6);
-    const int row = i < NX ? min(r, p.N - 1 - n0) * p.xs : min(r, p.M - 1 - m0) * p.K;
-    at[i] = (unsigned int)(row + ((lane & 7) ^ key) * 8) * 2;
+    const unsigned int row =
+        i < NX ? min(r, p.N - 1 - n0) * p.xs : min(r, p.M - 1 - m0) * p.K;
+    at[i] = (row + ((lane & 7) ^ key) * 8) * 2;
   }
-  auto issue = [&](int step, int slot) {
-#pragma unroll
-    for (int i = 0; i < NI; ++i)
-      load_lds(i < NX ? xb : wb, &ring[slot * STAGE + (i * NW + wave) * 8 * BK], at[i],
-               step * BK * 2);
+  auto issue = [&](int step, int slot, int i) {
+    load_lds(i < NX ? xb : wb, &ring[slot * STAGE + (i * NW + wave) * 8 * BK], at[i],
+             step * BK * 2);
   };
 
   f32x4_t acc[FM][FN];
@@ -117,23 +127,45 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
   const int fkey = ((col >> 1) & 1) | ((col >> 2) << 1);
 
   bf16x8_t a0[FM], b0[FN], a1[FM], b1[FN];  // the two halves of a step
-  auto fetch = [&](int slot, int half, bf16x8_t(&a)[FM], bf16x8_t(&b)[FN]) {
+  auto fetch_one = [&](int slot, int half, bf16x8_t(&a)[FM], bf16x8_t(&b)[FN], int i) {
     const short* st = &ring[slot * STAGE];
     const short* fp = st + frow * BK + ((half * 4 + g) ^ fkey) * 8;
     const short* xp = st + xrow * BK + ((half * 4 + g) ^ xkey) * 8;
+    if (i >= 1 && i <= FM)
+      a[i - 1] = *reinterpret_cast<const bf16x8_t*>(
+          fp + (((i - 1) >> 1) * 32 + ((i - 1) & 1) * 4) * BK);
+    else
+      b[i ? i - FM : 0] =
+          *reinterpret_cast<const bf16x8_t*>(xp + (i ? i - FM : 0) * 16 * BK);
+  };
+  auto fetch = [&](int slot, int half, bf16x8_t(&a)[FM], bf16x8_t(&b)[FN]) {
 #pragma unroll
-    for (int f = 0; f < FM; ++f)
-      a[f] = *reinterpret_cast<const bf16x8_t*>(fp + ((f >> 1) * 32 + (f & 1) * 4) * BK);
-#pragma unroll
-    for (int t = 0; t < FN; ++t) b[t] = *reinterpret_cast<const bf16x8_t*>(xp + t * 16 * BK);
+    for (int i = 0; i < FM + FN; ++i) fetch_one(slot, half, a, b, i);
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto multiply = [&](bf16x8_t(&a)[FM], bf16x8_t(&b)[FN]) {
+  // A half step's products, between them the reads of the next half step and loads
+  // first .. last - 1 of a step to come: a wave that issues those in a row waits for
+  // each to be taken while its matrix core idles.
+  auto multiply = [&](bf16x8_t(&a)[FM], bf16x8_t(&b)[FN], bf16x8_t(&an)[FM],
+                      bf16x8_t(&bn)[FN], int slot, int half, int step, int free_slot,
+                      int first, int last) {
+    constexpr int T = FM * FN;
 #pragma unroll
     for (int t = 0; t < FN; ++t)
 #pragma unroll
-      for (int f = 0; f < FM; ++f) acc[f][t] = mfma16x16x32(a[f], b[t], acc[f][t]);
-    __builtin_amdgcn_sched_barrier(0);
+      for (int f = 0; f < FM; ++f) {
+        const int m = t * FM + f;
+        acc[f][t] = mfma16x16x32(a[f], b[t], acc[f][t]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < FM + FN; ++i)
+          if (i * T / (FM + FN + LAG) == m) fetch_one(slot, half, an, bn, i);
+#pragma unroll
+        for (int i = first; i < last; ++i)
+          if (m == (i - first) * T / (last > first ? last - first : 1))
+            issue(step, free_slot, i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
   };
   auto barrier = [&]() {
     __builtin_amdgcn_sched_barrier(0);
@@ -142,11 +174,13 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
     asm volatile("" ::: "memory");
   };
 
-  const int steps = p.K / BK;
+  const bool ring_full = steps >= S;
 #pragma unroll
   for (int j = 0; j < S; ++j)
-    if (j < steps) issue(j, j);
-  if (steps >= S) __builtin_amdgcn_s_waitcnt(wait_imm(NI * (S - 1)));
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+      if (j < steps && (i < N1 || j < S - 1)) issue(j, j, i);
+  if (ring_full) __builtin_amdgcn_s_waitcnt(wait_imm(NI * (S - 2) + N1));
   else __builtin_amdgcn_s_waitcnt(wait_imm(0));
   barrier();
   fetch(0, 0, a0, b0);
@@ -154,50 +188,73 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
   // landed before the barrier, which covers the other waves'; then the slot is
   // free. (A loop of its own for the steps that load no more: with the loads under
   // a condition the compiler moves every accumulator once a step.)
-  int slot = 0, j = 0;
+  int slot = 0, before = S - 1, j = 0;
   for (; j + S < steps; ++j) {
-    fetch(slot, 1, a1, b1);
-    multiply(a0, b0);
+    multiply(a0, b0, a1, b1, slot, 1, j + S - 1, before, N1, NI);
     __builtin_amdgcn_s_waitcnt(wait_imm(NI * (S - 2)));
     barrier();
-    issue(j + S, slot);
+    before = slot;
     slot = slot + 1 == S ? 0 : slot + 1;
-    fetch(slot, 0, a0, b0);
-    multiply(a1, b1);
+    multiply(a1, b1, a0, b0, slot, 0, j + S, before, 0, N1);
   }
+  if (ring_full)
+#pragma unroll
+    for (int i = N1; i < NI; ++i) issue(j + S - 1, before, i);
   for (; j + 1 < steps; ++j) {
-    fetch(slot, 1, a1, b1);
-    multiply(a0, b0);
+    multiply(a0, b0, a1, b1, slot, 1, 0, 0, 0, 0);
     __builtin_amdgcn_s_waitcnt(wait_imm(0));
     barrier();
     slot = slot + 1 == S ? 0 : slot + 1;
-    fetch(slot, 0, a0, b0);
-    multiply(a1, b1);
+    multiply(a1, b1, a0, b0, slot, 0, 0, 0, 0, 0);
   }
-  fetch(slot, 1, a1, b1);
-  multiply(a0, b0);
-  multiply(a1, b1);
+  multiply(a0, b0, a1, b1, slot, 1, 0, 0, 0, 0);
+#pragma unroll
+  for (int t = 0; t < FN; ++t)
+#pragma unroll
+    for (int f = 0; f < FM; ++f) acc[f][t] = mfma16x16x32(a1[f], b1[t], acc[f][t]);
 
 #pragma unroll
   for (int f = 0; f < FM; f += 2) {
     const int feat = m0 + wm * FM * 16 + f * 16 + g * 8;
     if (feat >= p.M) continue;
-    float b[8];
-    const short8_t bv = p.bias ? *reinterpret_cast<const short8_t*>(p.bias + feat) : short8_t{};
+    if constexpr (EPI == PARTIAL) {
 #pragma unroll
-    for (int r = 0; r < 8; ++r) b[r] = bf16_bits_to_float(bv[r]);
-#pragma unroll
-    for (int t = 0; t < FN; ++t) {
-      const int tok = n0 + wn * FN * 16 + t * 16 + col;
-      if (tok >= p.N) continue;
-      bf16x8_t o;
-#pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        float v = acc[f + r / 4][t][r % 4] + b[r];
-        if constexpr (GELU) v = gelu_f(v);
-        o[r] = (__bf16)v;
+      for (int t = 0; t < FN; ++t) {
+        const int tok = n0 + wn * FN * 16 + t * 16 + col;
+        if (tok >= p.N) continue;
+        f32x4_t* o = reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.out) +
+                                                ((long)blockIdx.y * p.N + tok) * p.M + feat);
+        o[0] = acc[f][t];
+        if (feat + 4 < p.M) o[1] = acc[f + 1][t];
       }
-      *reinterpret_cast<bf16x8_t*>(p.out + (long)tok * p.M + feat) = o;
+    } else {
+      float b[8] = {};
+      if (p.bias) {
+        const short8_t bv = *reinterpret_cast<const short8_t*>(p.bias + feat);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) b[r] = bf16_bits_to_float(bv[r]);
+      }
+#pragma unroll
+      for (int t = 0; t < FN; ++t) {
+        const int tok = n0 + wn * FN * 16 + t * 16 + col;
+        if (tok >= p.N) continue;
+        bf16x8_t o;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          float v = acc[f + r / 4][t][r % 4] + b[r];
+          if constexpr (EPI == BIAS_GELU) v = gelu_f(v);
+          o[r] = (__bf16)v;
+        }
+        short* to = reinterpret_cast<short*>(p.out) + (long)tok * p.M + feat;
+        if (p.M % 8 == 0) {
+          *reinterpret_cast<bf16x8_t*>(to) = o;
+        } else {  // (M a multiple of 4)
+          typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+          *reinterpret_cast<bf16x4_t*>(to) = bf16x4_t{o[0], o[1], o[2], o[3]};
+          if (feat + 4 < p.M)
+            *reinterpret_cast<bf16x4_t*>(to + 4) = bf16x4_t{o[4], o[5], o[6], o[7]};
+        }
+      }
     }
   }
 }
@@ -246,14 +303,14 @@ extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
   const Tile& t = TILES[tile];
   const long ftiles = (M + t.tm - 1) / t.tm, tiles = ftiles * ((N + t.tn - 1) / t.tn);
   if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-  const DenseArgs p{(short*)out, (const short*)x, (const short*)w, (const short*)bias,
+  const DenseArgs p{out, (const short*)x, (const short*)w, (const short*)bias,
                     M, K, N, (int)xs, (int)ftiles, (int)tiles};
 #define GO(tn, tm, wn, wm, s)                                                         \
   if (gelu)                                                                           \
-    hipLaunchKernelGGL((dense_gemm_kernel<tn, tm, wn, wm, s, true>), dim3(p.tiles),   \
-                       dim3(wn * wm * 64), 0, stream, p);                             \
+    hipLaunchKernelGGL((dense_gemm_kernel<tn, tm, wn, wm, s, BIAS_GELU>),             \
+                       dim3(p.tiles), dim3(wn * wm * 64), 0, stream, p);              \
   else                                                                                \
-    hipLaunchKernelGGL((dense_gemm_kernel<tn, tm, wn, wm, s, false>), dim3(p.tiles),  \
+    hipLaunchKernelGGL((dense_gemm_kernel<tn, tm, wn, wm, s, BIAS>), dim3(p.tiles),   \
                        dim3(wn * wm * 64), 0, stream, p);
   switch (tile) {
     case 0: GO(128, 192, 4, 2, 3) break;
@@ -262,6 +319,56 @@ extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
     case 3: GO(128, 128, 2, 2, 2) break;
     case 4: GO(64, 128, 2, 2, 3) break;
     default: GO(64, 64, 2, 2, 4) break;
+  }
+#undef GO
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
+}
+
+// Products of 65 to 256 rows for the few-row entry points, K in parts so that the
+// blocks come to one or two a compute unit. Where M is narrow a block takes 64
+// features (few parts, so few sums to add); otherwise, above 128 rows, 128 features
+// and all rows. us, here / the few-row kernel, with the sums added: K 4096, M 4096 at
+// 128 rows 15.9 / 18.9 (level at 77, the products alone); K 8192, M 2048 at 77 / 256 15.4 / 18.4, 21.3 /
+// 29.2; K 14336, M 4096 at 200 / 256 41.4 / 49.5, 45.8 / 54.7 (54.9 with 64 features); K
+// 4096, M 6144 at 256 31.9 / 33.6. Up to 128 rows the few-row kernel keeps wide M and
+// long K (K 14336, M 4096 at 77 rows 29.7, 128 x 128 here 34.1).
+static bool mid_narrow(int M, int K) { return M <= 4096 && K <= 8192; }
+
+extern "C" int ks_mid_takes(int M, int K, int N) {
+  return N > 128 || (N > (M < 4096 ? 64 : 96) && mid_narrow(M, K));
+}
+
+extern "C" int ks_mid_splits(int M, int K, int N) {
+  const int tm = mid_narrow(M, K) ? 64 : 128;
+  const int tiles = (M + tm - 1) / tm * (tm == 64 && N > 128 ? 2 : 1);
+  int s = UNITS / (tiles > 0 ? tiles : 1);
+  if (s > K / BK / 4) s = K / BK / 4;
+  return s < 1 ? 1 : s > 16 ? 16 : s;
+}
+
+// out: fp32 sums of the parts (sums) or bf16
+extern "C" hipError_t ks_mid_gemm(void* out, const void* x, const void* w, int M, int K,
+                                  int N, long xs, int splits, int sums,
+                                  hipStream_t stream) {
+  if (N < 1 || N > 256 || M < 4 || M % 4 != 0 || K < BK || K % BK != 0 ||
+      K >= 1 << 22 || xs % 8 != 0 || xs >= 1 << 22 || splits < 1 || splits > K / BK ||
+      (splits > 1 && !sums) || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
+    return hipErrorInvalidValue;
+  DenseArgs p{out, (const short*)x, (const short*)w, nullptr, M, K, N, (int)xs, 0, 0};
+#define GO(tn, tm, wn, wm, s, epi)                                                    \
+  {                                                                                   \
+    p.ftiles = (M + tm - 1) / tm;                                                     \
+    p.tiles = p.ftiles * ((N + tn - 1) / tn);                                         \
+    hipLaunchKernelGGL((dense_gemm_kernel<tn, tm, wn, wm, s, epi>),                   \
+                       dim3(p.tiles, splits), dim3(wn * wm * 64), 0, stream, p);      \
+  }
+  if (mid_narrow(M, K)) {
+    if (sums) GO(128, 64, 2, 2, 3, PARTIAL)
+    else GO(128, 64, 2, 2, 3, BIAS)
+  } else {
+    if (sums) GO(256, 128, 4, 2, 3, PARTIAL)
+    else GO(256, 128, 4, 2, 3, BIAS)
   }
 #undef GO
   HIP_CHECK_KERNEL();

@@ -1,6 +1,7 @@
 // Products of few rows with a weight matrix: out[N][M] = x[N][K] w[M][K]^T for
 // N <= 256 tokens (decode batches, short prompts), where reading the weights
-// is what bounds them.
+// is what bounds them. The kernel here takes up to 64, and up to 128 of wide
+// weights; the rest goes to the tiles of dense_gemm.hip.
 //
 // A block takes 64 F features (16 F per wave) and all tokens over a range of
 // K, in steps of 64: each step's weight and token rows come by LDS-direct
@@ -13,10 +14,9 @@
 // Measured (us with the reduction, weights not in cache; the library's in
 // parentheses): K 4096, M 14336 GLU at 1 row 46 = 5.1 TB/s (67 with the
 // activation kernel), at 24 rows 47; K 4096, M 32000 at 1 row 49 (61); K
-// 14336, M 4096 at 1 / 24 / 96 / 256 rows 24 / 24 / 32 / 54 (27 / 32 / 63 / 62).
-// Up to 48 rows the loads bound it (non-temporal ones took 5 to 10 % off; no
-// gain above); above, LDS reads and the matrix cores of the few blocks that
-// fit, so wide M goes back to the library. The kernel before kept a barrier
+// 14336, M 4096 at 1 / 24 rows 24 / 24 (27 / 32). Up to 48 rows the loads bound it
+// (non-temporal ones took 5 to 10 % off; no gain above); above, LDS reads and the
+// matrix cores of the few blocks that fit, so wide M goes back to the library. The kernel before kept a barrier
 // per step behind one load in flight and rounded the splits to bf16.
 //
 // C = W X^T on v_mfma_f32_16x16x32_bf16: a lane ends with four consecutive
@@ -214,13 +214,16 @@ __global__ __launch_bounds__(256) void reduce_splits_kernel(
   else if ((N) <= 48) GO(3, 1, 5)       \
   else if ((N) <= 64) GO(4, 1, 5)       \
   else if ((N) <= 96) GO(6, 2, 5)       \
-  else if ((N) <= 128) GO(8, 2, 5)      \
-  else if ((N) <= 192) GO(12, 2, 4)     \
-  else GO(16, 2, 3)
+  else GO(8, 2, 5)
 
 int feature_tile(int N) { return N <= 64 ? 64 : 128; }
 
 }  // namespace
+
+extern "C" int ks_mid_splits(int, int, int);
+extern "C" int ks_mid_takes(int, int, int);
+extern "C" hipError_t ks_mid_gemm(void*, const void*, const void*, int, int, int, long,
+                                  int, int, hipStream_t);
 
 // K splits for [N][K] x [M][K]: as many as keep one block on each of the 256
 // compute units, with at least 8 steps a split where there are more than four (4
@@ -236,11 +239,11 @@ int feature_tile(int N) { return N <= 64 ? 64 : 128; }
 // apart fall on the same memory channels as the rows below them: up to twice as
 // many are taken if that avoids it as evenly (K 28672, M 8192 at 1 row 90 with 2,
 // 77 with 4), or three for four above 64 rows (8192 x 8192 at 72 rows 43.5 /
-// 37.4, 128 rows 45 / 43; past that the matrix cores want the blocks, 50 / 56 at
-// 192). Up to 64 rows the count does not depend on N, so neither do a row's sums.
+// 37.4, 128 rows 45 / 43). Up to 64 rows the count does not depend on N, so neither do a row's sums.
 extern "C" int ks_skinny_splits(int M, int K, int N, int glu) {
   constexpr int UNITS = 256;
   if (glu) return 1;
+  if (ks_mid_takes(M, K, N)) return ks_mid_splits(M, K, N);
   const int bm = feature_tile(N);
   const int tiles = (M + bm - 1) / bm, steps = K / BK;
   if (tiles < 1) return 1;
@@ -249,7 +252,7 @@ extern "C" int ks_skinny_splits(int M, int K, int N, int glu) {
   if (s > most) s = most;
   if (s > 16) s = 16;
   if (s < 1) s = 1;
-  if (N > 64) return s == 4 && K % 8192 == 0 && N <= 128 ? 3 : s;
+  if (N > 64) return s == 4 && K % 8192 == 0 ? 3 : s;
   // rounds of blocks on a unit with t splits, each of 1 / t of K
   auto rounds = [&](int t) { return ((long)tiles * t + UNITS - 1) / UNITS; };
   auto aliased = [&](int t) { return K % 2048 == 0 && K * 2L % (t * 4096L) == 0; };
@@ -275,8 +278,12 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
   const bool sums = splits > 1 || !out;
   const GemmArgs p{sums ? partial : out, (const short*)x, (const short*)w, M,
                    K, N, xs};
-  const int bm = feature_tile(N) / (glu ? 2 : 1);
-  const dim3 grid((M + bm - 1) / bm, splits);
+  if (!glu && ks_mid_takes(M, K, N)) {
+    const hipError_t e = ks_mid_gemm(p.out, x, w, M, K, N, xs, splits, sums, stream);
+    if (e != hipSuccess) return e;
+  } else {
+    const int bm = feature_tile(N) / (glu ? 2 : 1);
+    const dim3 grid((M + bm - 1) / bm, splits);
 #define GO(nt, f, s)                                                           \
   {                                                                            \
     if (glu)                                                                   \
@@ -289,9 +296,17 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
       hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, BF16_OUT>), grid,       \
                          dim3(256), 0, stream, p);                             \
   }
-  FOR_TILE(N, GO)
+    if (N <= 128) {
+      FOR_TILE(N, GO)
+    } else if (glu) {
+      if (N <= 192)
+        hipLaunchKernelGGL((skinny_gemm_kernel<12, 2, 4, GLU>), grid, dim3(256), 0, stream, p);
+      else
+        hipLaunchKernelGGL((skinny_gemm_kernel<16, 2, 3, GLU>), grid, dim3(256), 0, stream, p);
+    }
 #undef GO
-  HIP_CHECK_KERNEL();
+    HIP_CHECK_KERNEL();
+  }
   if (sums && out) {
     const long nm = (long)N * M;
     hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)((nm / 4 + 255) / 256)),

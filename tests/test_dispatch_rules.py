@@ -16,6 +16,8 @@ from kserve_amd import ops
         (96, 2048, 8192, False), (160, 2560, 8192, False),  # 21.7 / 17.5
         (192, 4096, 4096, True), (256, 4096, 4096, False),
         (257, 4096, 8192, False), (8, 4096, 4098, False),
+        (65, 8192, 2048, True), (256, 8192, 2048, True), (128, 4096, 2048, False),
+        (128, 8192, 2044, False),
     ],
 )
 def test_few_row_product(n, k, m, own):

@@ -968,6 +968,14 @@ class TestSkinnyGemmEdges:
         unequal length."""
         self.test_against_fp64(dev, N, K, M, False)
 
+    @pytest.mark.parametrize(
+        "N,K,M", [(65, 8192, 2048), (129, 8192, 2052), (256, 2112, 772),
+                  (128, 4096, 4096), (129, 14336, 4100), (200, 4096, 6144)]
+    )
+    def test_parts_of_many_rows(self, dev, N, K, M):
+        """Narrow and wide weights above 64 and 128 rows, in parts of K."""
+        self.test_against_fp64(dev, N, K, M, False)
+
     def test_dispatch_takes_every_form(self, dev):
         from kserve_amd import ops
 
