@@ -375,15 +375,27 @@ def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     return m >= 4608 and (n <= 48 or m <= 8192 or m >= 10240)
 
 
-def _dense_rows(n: int, k: int, m: int) -> bool:
+def _dense_rows(n: int, k: int, m: int, gelu: bool) -> bool:
     """Whether the encoder kernel beats the library at [n, k] x [m, k]^T + bias
-    (MI355X, us, kernel / library). Up to k 768 it does from one row to 30000 (m
-    768 at 100 / 7864 / 30000 rows 4.8 / 5.1, 13.9 / 15.1, 48 / 60; level at 8 rows,
-    4.6 / 4.4, where it is the shorter call by 14 us of host time); at k 1024 while
-    the rows leave the library short of tiles (m 1024 at 1000 / 3500 / 16384 rows 6.7 /
-    9.4, 12.3 / 12.8, 43 / 30); past that the library's larger tiles win (k 3072, m
-    768 at 200 / 3500 rows 12.0 / 9.4, 29 / 22)."""
-    return m % 8 == 0 and 8 <= m <= 4096 and (k <= 768 or (k <= 1024 and n <= 3584))
+    (MI355X, us, kernel / library). Up to k 768 with gelu always (m 3072 at 200 / 4500 /
+    7864 / 30000 rows 6.8 / 11.3, 36 / 38, 50 / 69, 211 / 230). Without, on small
+    products (m 768 at 100 / 2000 / 7000 rows 4.8 / 5.1, 7.6 / 9.9, 12.9 / 15.4; m 2304 at
+    1200 / 3200 rows 10.5 / 10.9, 16.9 / 17.8) and again where the library's choice of
+    tile turns (m 2304 at 3700 / 7000 rows 20.8 / 19.7, 31 / 26, but at 7864 / 10000 /
+    12000 33 / 63, 40 / 54, 51 / 61). At k 1024 while the rows leave the library short
+    of tiles (m 1024 at 1000 / 3500 rows 6.7 / 9.4, 11.6 / 12.8, with gelu m 4096 at 2500
+    30 / 35; m 1024 at 16384 rows 43 / 30). Up to k 3072 where one round of the smallest
+    tiles holds the product (m 768 at 350 / 1200 rows 12.4 / 12.5, 12.9 / 15.1; at 100
+    rows 11.7 / 8.4, which the shorter call's 14 us of host time outweigh); past that
+    the library's larger tiles win (m 768 at 2000 / 3200 rows 19.8 / 18.6, 29 / 25)."""
+    if m % 8 or not 8 <= m <= 4096 or k > 3072:
+        return False
+    if -(-n // 64) * -(-m // 64) <= 256:
+        return True
+    work = n * m * k  # multiply-adds
+    if k <= 768:
+        return gelu or work <= 5.8e9 or work >= 13.1e9
+    return k <= 1024 and n <= 3584 and (gelu or work <= 5.8e9)
 
 
 def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
@@ -392,7 +404,7 @@ def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
     if not (
         bias is not None
         and x.dim() == 2
-        and _dense_rows(x.shape[0], x.shape[1], m)
+        and _dense_rows(x.shape[0], x.shape[1], m, gelu)
         and _plain_operands(x, weight)
         and x.shape[0] < 1 << 30
         and x.shape[1] <= x.stride(0) < 1 << 22

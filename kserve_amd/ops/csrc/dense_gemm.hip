@@ -259,18 +259,22 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
   }
 }
 
-// Which tile: the least a n + b, for n tiles on the busiest unit. a and b are us at
-// K 768, between those with and without gelu; all grow with K alike, so the order
-// holds. Where a unit has a single tile, one block of eight waves with a deeper
-// ring beats one of four (7864 x 768 to 768 13.9 / 15.1, 1000 to 2304 10.1 / 12.3).
+// Which tile: the least a n + b, for n tiles on the busiest unit (a quarter more for
+// an odd one where two blocks share a unit: alone it hides less of its latency). a
+// and b are us at K 768 without gelu, fitted over 768 to 3072 features and 1200 to
+// 12000 rows; all grow with K and gelu alike, so the order holds. Where a unit has a
+// single tile, one block of eight waves with a deeper ring beats one of four (7864 x
+// 768 to 768 13.5 / 15.0, 1200 to 2304 10.5 / 12.8).
 struct Tile {
   int tn, tm;
   float a, b;
+  bool pairs;
 };
 constexpr int NTILES = 6;
 constexpr Tile TILES[NTILES] = {
-    {128, 192, 12.f, 0.f},   {128, 192, 11.f, 2.f},  {128, 128, 9.8f, 0.f},
-    {128, 128, 8.2f, 2.5f}, {64, 128, 4.3f, 3.5f},  {64, 64, 2.8f, 2.8f}};
+    {128, 192, 12.6f, 0.5f, false}, {128, 192, 9.8f, 2.f, true},
+    {128, 128, 9.5f, 0.f, false},   {128, 128, 7.2f, 2.2f, true},
+    {64, 128, 4.4f, 2.6f, false},   {64, 64, 2.9f, 2.5f, false}};
 
 }  // namespace
 
@@ -281,7 +285,7 @@ extern "C" int ks_dense_tile(int M, int N) {
     const Tile& t = TILES[i];
     const long tiles = (long)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
     const long n = (tiles + UNITS - 1) / UNITS;
-    const float us = t.a * (float)n + t.b;
+    const float us = t.a * ((float)n + (t.pairs && n % 2 ? 0.25f : 0.f)) + t.b;
     if (i == 0 || us < least) {
       least = us;
       best = i;

@@ -82,16 +82,21 @@ def test_scan_apart(lens, heads, P, apart):
 
 
 @pytest.mark.parametrize(
-    "n,k,m,own",
+    "n,k,m,gelu,own",
     [
-        (1, 768, 768, True), (30000, 768, 3072, True), (7864, 384, 1536, True),
-        (3584, 1024, 4096, True), (3585, 1024, 4096, False),  # 16384 rows 183 / 169
-        (200, 3072, 768, False), (64, 768, 30522, False), (64, 768, 4, False),
-        (64, 768, 4104, False),
+        (1, 768, 768, False, True), (30000, 768, 3072, True, True),
+        (7000, 768, 768, False, True), (3200, 768, 2304, False, True),
+        (3700, 768, 2304, False, False), (7000, 768, 2304, False, False),  # 31 / 26 us
+        (7864, 768, 2304, False, True), (7864, 384, 1536, True, True),
+        (3584, 1024, 4096, True, True), (3585, 1024, 4096, True, False),
+        (16384, 1024, 1024, False, False),                                 # 43 / 30
+        (1344, 3072, 768, False, True), (1345, 3072, 768, False, False),
+        (64, 3136, 768, False, False), (64, 768, 30522, False, False),
+        (64, 768, 4, False, False), (64, 768, 4104, False, False),
     ],
 )
-def test_encoder_product(n, k, m, own):
-    assert ops._dense_rows(n, k, m) is own
+def test_encoder_product(n, k, m, gelu, own):
+    assert ops._dense_rows(n, k, m, gelu) is own
 
 
 def test_encoder_product_on_cpu_is_the_librarys():
