@@ -81,16 +81,17 @@ class MerulornLayer(nn.Module):
             self.ssm.in_proj.data = self.fused_proj.data[a:]
 
     def mixer(self, h, positions, cache: LayerCache, meta):
-        """Returns (delta0, scale0, delta1, scale1) to add to the stream."""
+        """Returns (delta0, scale0, delta1, scale1) to add to the stream; the
+        deltas may be in parts, summed over a first dimension."""
         if self.attn is not None and self.ssm is not None:
             proj = ops.linear(h, self.fused_proj, self.fused_bias)
             a = self.attn.proj_width
-            left = self.attn.mix(proj[:, :a], positions, cache, meta)
-            right = self.ssm.mix(proj[:, a:], positions, cache, meta)
+            left = self.attn.mix(proj[:, :a], positions, cache, meta, parts=True)
+            right = self.ssm.mix(proj[:, a:], positions, cache, meta, parts=True)
             return left, self.spec.attention_scale, right, self.spec.ssm_scale
         if self.ssm is not None:
-            return self.ssm(h, positions, cache, meta), 1.0, None, 1.0
-        return self.attn(h, positions, cache, meta), 1.0, None, 1.0
+            return self.ssm(h, positions, cache, meta, parts=True), 1.0, None, 1.0
+        return self.attn(h, positions, cache, meta, parts=True), 1.0, None, 1.0
 
 
 class MerulornForCausalLM(nn.Module):
@@ -190,12 +191,12 @@ class MerulornForCausalLM(nn.Module):
             pending = layer.mixer(h, positions, cache, meta)
             if layer.mlp is not None:
                 h = self._add_norm(x, layer.norm2, pending)
-                pending = (layer.mlp(h), 1.0, None, 1.0)
+                pending = (layer.mlp(h, parts=True), 1.0, None, 1.0)
             if dbg is not None:
                 r = x.clone()
                 for d, s in ((pending[0], pending[1]), (pending[2], pending[3])):
                     if d is not None:
-                        r += s * d.float()
+                        r += s * (d.sum(0) if d.dim() == 3 else d.float())
                 dbg.append(r)
         return self._add_norm(x, self.final_norm, pending)
 

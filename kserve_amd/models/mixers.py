@@ -101,9 +101,10 @@ class SSDMixer(nn.Module):
         self.norm_w.copy_(get(prefix + "norm").float())
         self.o_proj.copy_(get(prefix + "o").to(self.dtype))
 
-    def mix(self, proj, positions, cache: LayerCache, meta):
+    def mix(self, proj, positions, cache: LayerCache, meta, parts: bool = False):
         """``proj``: [T, proj_width] rows of this mixer's in-projection (may be
-        a column slice of a wider fused projection)."""
+        a column slice of a wider fused projection). ``parts``: the output may
+        come in parts (``ops.linear_parts``)."""
         s = self.spec
         z = proj[:, : s.inner]
         xbc_raw = proj[:, s.inner : s.inner + s.conv_channels]
@@ -121,10 +122,10 @@ class SSDMixer(nn.Module):
         yn = ops.gated_group_rms_norm(
             y, z, self.norm_w, self.eps, s.norm_groups, self.dtype
         )
-        return ops.linear(yn, self.o_proj)
+        return (ops.linear_parts if parts else ops.linear)(yn, self.o_proj)
 
-    def forward(self, h, positions, cache: LayerCache, meta):
-        return self.mix(ops.linear(h, self.in_proj), positions, cache, meta)
+    def forward(self, h, positions, cache: LayerCache, meta, parts: bool = False):
+        return self.mix(ops.linear(h, self.in_proj), positions, cache, meta, parts)
 
 
 class NormedGatedAttention(nn.Module):
@@ -164,7 +165,7 @@ class NormedGatedAttention(nn.Module):
         self.k_norm.copy_(get(prefix + "k.norm").float())
         self.o_proj.copy_(get(prefix + "o").to(dt))
 
-    def mix(self, proj, positions, cache: LayerCache, meta):
+    def mix(self, proj, positions, cache: LayerCache, meta, parts: bool = False):
         s = self.spec
         a, b, c = self.q_w, self.q_w + self.k_w, self.q_w + self.k_w + self.v_w
         q, k, v, gate = proj[:, :a], proj[:, a:b], proj[:, b:c], proj[:, c:]
@@ -177,11 +178,11 @@ class NormedGatedAttention(nn.Module):
             meta.context_lens, s.scale, meta.max_seqlen, s.heads, gate=gate,
             out_dtype=self.dtype,
         )
-        return ops.linear(o, self.o_proj)
+        return (ops.linear_parts if parts else ops.linear)(o, self.o_proj)
 
-    def forward(self, h, positions, cache: LayerCache, meta):
+    def forward(self, h, positions, cache: LayerCache, meta, parts: bool = False):
         return self.mix(
-            ops.linear(h, self.qkvg, self.qkvg_bias), positions, cache, meta
+            ops.linear(h, self.qkvg, self.qkvg_bias), positions, cache, meta, parts
         )
 
 
@@ -288,11 +289,11 @@ class ClampedGLU(nn.Module):
         )
         self.down.copy_(get(prefix + "down").to(dt))
 
-    def forward(self, h):
+    def forward(self, h, parts: bool = False):
         act = ops.clamped_swiglu(
             ops.linear(h, self.gate_up), self.ALPHA, self.spec.limit
         )
-        return ops.linear(act, self.down)
+        return (ops.linear_parts if parts else ops.linear)(act, self.down)
 
 
 class RoutedClampedMoE(nn.Module):

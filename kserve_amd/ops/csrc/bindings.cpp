@@ -364,6 +364,7 @@ static SkinnyShape skinny_shape(const at::Tensor& x, const at::Tensor& w, int ha
 // fp32 sums of the K splits of x @ w^T, [splits][N][M]
 static at::Tensor skinny_sums(const at::Tensor& x, const at::Tensor& w) {
   const SkinnyShape z = skinny_shape(x, w, 1);
+  const c10::DeviceGuard guard(x.device());
   const int splits = ks_skinny_splits(z.M, z.K, z.N, 0);
   at::Tensor part = at::empty({splits, z.N, z.M}, x.options().dtype(at::kFloat));
   check_hip(ks_skinny_gemm(nullptr, part.data_ptr(), x.data_ptr(), w.data_ptr(), z.M,
@@ -567,6 +568,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gelu", &gelu, "erf GELU");
   def_sampling(m);
   m.def("skinny_gemm", &skinny_gemm, "decode GEMM (N<=256, MFMA streaming)");
+  m.def("skinny_sums", &skinny_sums, "few-row GEMM as fp32 sums of parts of K");
   m.def("skinny_add_rms_norm", &skinny_add_rms_norm,
         "few-row GEMM into a residual and its RMS norm");
   m.def("rope_and_cache", &rope_and_cache,

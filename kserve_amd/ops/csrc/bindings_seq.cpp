@@ -8,6 +8,9 @@ extern "C" {
 hipError_t ks_embed_scale_sinpos(void*, const void*, const void*, const void*,
                                  const void*, float, int, int, int,
                                  hipStream_t);
+hipError_t ks_add_parts_rms_norm_f32res(void*, const void*, long, int, float, const void*,
+                                        long, int, float, const void*, float, float,
+                                        void*, int, int, hipStream_t);
 hipError_t ks_add_rms_norm_f32res(void*, const void*, long, float, const void*,
                                   long, float, const void*, const void*,
                                   const void*, const void*, int, const void*,
@@ -244,6 +247,48 @@ void add_rms_norm_f32res(at::Tensor& residual,
                 out.has_value() ? out->data_ptr() : nullptr, rows, width, f32,
                 df32, current_stream()),
             "add_rms_norm_f32res");
+}
+
+void add_parts_rms_norm_f32res(at::Tensor& residual, const c10::optional<at::Tensor>& d0,
+                               double s0, const c10::optional<at::Tensor>& d1, double s1,
+                               at::Tensor& weight, double w_offset, double eps,
+                               at::Tensor& out) {
+  // deltas: bf16 [T, W] or fp32 [parts, T, W]
+  CHECK_F32(residual);
+  CHECK_F32(weight);
+  TORCH_CHECK(residual.dim() == 2 && weight.numel() == residual.size(1) &&
+                  out.scalar_type() == at::kBFloat16 && out.is_contiguous() &&
+                  out.device() == residual.device() && out.numel() == residual.numel(),
+              "add_parts_rms_norm_f32res: shape mismatch");
+  const int64_t rows = residual.size(0), width = residual.size(1);
+  const void* p[2] = {nullptr, nullptr};
+  long stride[2] = {0, 0};
+  int parts[2] = {0, 0};
+  const c10::optional<at::Tensor>* d[2] = {&d0, &d1};
+  for (int i = 0; i < 2; ++i) {
+    if (!d[i]->has_value()) continue;
+    const at::Tensor& t = **d[i];
+    TORCH_CHECK(t.device() == residual.device(), "deltas on another device");
+    if (t.dim() == 3) {
+      TORCH_CHECK(t.scalar_type() == at::kFloat && t.is_contiguous() && t.size(0) >= 1 &&
+                      t.size(1) == rows && t.size(2) == width,
+                  "parts: fp32 [parts, T, W]");
+      parts[i] = (int)t.size(0);
+    } else {
+      CHECK_ROWS(t);
+      TORCH_CHECK(t.scalar_type() == at::kBFloat16 && t.size(0) == rows &&
+                      t.size(1) == width,
+                  "delta: bf16 [T, W]");
+      stride[i] = t.stride(0);
+    }
+    p[i] = t.data_ptr();
+  }
+  const c10::DeviceGuard guard(residual.device());
+  check_hip(ks_add_parts_rms_norm_f32res(
+                residual.data_ptr(), p[0], stride[0], parts[0], (float)s0, p[1], stride[1],
+                parts[1], (float)s1, weight.data_ptr(), (float)w_offset, (float)eps,
+                out.data_ptr(), (int)rows, (int)width, current_stream()),
+            "add_parts_rms_norm_f32res");
 }
 
 void gated_group_rms_norm(at::Tensor& out, at::Tensor& y, at::Tensor& z,
@@ -1333,6 +1378,8 @@ void bias_gelu_tanh(at::Tensor& out, at::Tensor& input, at::Tensor& bias) {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("embed_scale_sinpos", &embed_scale_sinpos,
         "scaled embedding + interleaved sinusoidal positions (fp32 out)");
+  m.def("add_parts_rms_norm_f32res", &add_parts_rms_norm_f32res,
+        "add_rms_norm_f32res of deltas that may be in parts");
   m.def("add_rms_norm_f32res", &add_rms_norm_f32res,
         "fp32 residual += scaled deltas, then offset-weight RMS norm");
   m.def("gated_group_rms_norm", &gated_group_rms_norm,

@@ -205,6 +205,74 @@ __global__ void add_rms_norm_f32res_vec4_kernel(
   }
 }
 
+// The same for deltas that may still be in parts, as the few-row products leave
+// them: [parts][rows][width] fp32 sums, added here in order. That saves a decode
+// layer a launch of 3.5 us and a pass over the rows for each such product (16
+// sequences, 64 state-space heads: step 451 -> 423 us).
+struct Delta {
+  const void* p;  // null: none
+  long stride;    // of bf16 rows
+  int parts;      // 0: bf16 rows
+  float scale;
+};
+
+__device__ __forceinline__ void add_delta(const Delta& d, long row, long rows, int width,
+                                          int i, float* v) {
+  if (!d.p) return;
+  float sum[4];
+  if (d.parts == 0) {
+    ld4<short>(reinterpret_cast<const short*>(d.p) + row * d.stride + i, sum);
+  } else {
+    const float* at = reinterpret_cast<const float*>(d.p) + row * width + i;
+    ld4<float>(at, sum);
+#pragma unroll 4
+    for (int q = 1; q < d.parts; ++q) {
+      float x[4];
+      ld4<float>(at + q * rows * width, x);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum[j] += x[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] += d.scale * sum[j];
+}
+
+__global__ __launch_bounds__(NT) void add_parts_rms_norm_f32res_kernel(
+    float* __restrict__ residual, const Delta d0, const Delta d1,
+    const float* __restrict__ weight, float w_offset, float eps, short* __restrict__ out,
+    long rows, int width) {
+  __shared__ float scratch[NW];
+  const long row = blockIdx.x;
+  float* r = residual + row * width;
+  float keep[VEC_STEPS][4];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < VEC_STEPS; ++k) {
+    const int i = (threadIdx.x + NT * k) * 4;
+    if (i < width) {
+      ld4<float>(r + i, keep[k]);
+      add_delta(d0, row, rows, width, i, keep[k]);
+      add_delta(d1, row, rows, width, i, keep[k]);
+      st4<float>(r + i, keep[k]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ss += keep[k][j] * keep[k][j];
+    }
+  }
+  ss = block_sum_sync<NW>(ss, scratch);
+  const float inv = 1.0f / sqrtf(ss / (float)width + eps);
+#pragma unroll
+  for (int k = 0; k < VEC_STEPS; ++k) {
+    const int i = (threadIdx.x + NT * k) * 4;
+    if (i < width) {
+      float w[4], o[4];
+      ld4<float>(weight + i, w);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = keep[k][j] * inv * (w_offset + w[j]);
+      st4<short>(out + row * width + i, o);
+    }
+  }
+}
+
 template <typename TD, typename TO>
 __global__ void post_layer_norm_add_kernel(
     float* __restrict__ residual, const TD* __restrict__ delta,
@@ -759,6 +827,25 @@ extern "C" hipError_t ks_embed_scale_sinpos(void* out, const void* table,
                        0, stream, (float*)out, (const short*)table,
                        (const long*)tokens, (const long*)positions,
                        (const float*)inv_freq, scale, width);
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
+}
+
+// parts: 0 for bf16 rows of a stride, else fp32 [parts][rows][width]
+extern "C" hipError_t ks_add_parts_rms_norm_f32res(
+    void* residual, const void* d0, long stride0, int parts0, float s0, const void* d1,
+    long stride1, int parts1, float s1, const void* weight, float w_offset, float eps,
+    void* out, int rows, int width, hipStream_t stream) {
+  if (rows == 0) return hipSuccess;
+  if (width < 4 || width % 4 != 0 || width > NT * 4 * VEC_STEPS || stride0 % 4 != 0 ||
+      stride1 % 4 != 0 || parts0 < 0 || parts1 < 0 ||
+      (((uintptr_t)residual | (uintptr_t)weight) & 15) != 0 || ((uintptr_t)out & 7) != 0 ||
+      ((uintptr_t)d0 & (parts0 ? 15 : 7)) != 0 || ((uintptr_t)d1 & (parts1 ? 15 : 7)) != 0)
+    return hipErrorInvalidValue;
+  const Delta a{d0, stride0, parts0, s0}, b{d1, stride1, parts1, s1};
+  hipLaunchKernelGGL(add_parts_rms_norm_f32res_kernel, dim3(rows), dim3(NT), 0, stream,
+                     (float*)residual, a, b, (const float*)weight, w_offset, eps,
+                     (short*)out, (long)rows, width);
   HIP_CHECK_KERNEL();
   return hipSuccess;
 }

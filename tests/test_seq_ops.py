@@ -75,6 +75,47 @@ def layout(lens, starts):
     return cu, seq, pos
 
 
+class TestResidualNormInParts:
+    @pytest.mark.parametrize(
+        "rows,width,parts0,parts1",
+        [(1, 4, 1, None), (3, 1028, 5, 0), (70, 2048, 0, 16), (2, 8192, 3, 2), (5, 36, None, 4)],
+    )
+    def test_against_oracle(self, be, rows, width, parts0, parts1):
+        """Deltas as bf16 rows (0), in parts, or absent; the residual in place."""
+        x, w = rnd(rows, width, seed=1), rnd(width, seed=2, scale=0.1)
+        deltas, want = [], x.double()
+        for parts, s, seed in ((parts0, 0.5, 3), (parts1, 2.0, 4)):
+            if parts is None:
+                deltas.append(None)
+                continue
+            d = rnd(max(parts, 1), rows, width, seed=seed, dtype=torch.bfloat16)
+            deltas.append(f32(d, be) if parts else d[0].to(be[1]).to(be[0]))
+            want = want + s * d.double().sum(0)
+        r = f32(x, be)
+        got = ops.add_rms_norm_f32res(
+            r, f32(w, be), 1e-5, 1.0, be[1], deltas[0], 0.5, deltas[1], 2.0
+        )
+        assert got.dtype == be[1]
+        # at most 18 fp32 additions a value; without the kernel a sum passes through
+        # the activation's type on its way
+        close(r, want, be, f32_tol=4e-6, bf16_tol=4e-6)
+        close(got, O.rms(want, 1e-5) * (1 + w.double()), be, f32_tol=4e-6, bf16_tol=2.0**-8)
+
+    @pytest.mark.gpu
+    @pytest.mark.parametrize(
+        "n,k,m", [(1, 4096, 2048), (64, 8192, 2048), (65, 4096, 2048), (200, 4096, 2052), (300, 4096, 2048)]
+    )
+    def test_products_in_parts(self, n, k, m):
+        x = rnd(n, k, seed=5, dtype=torch.bfloat16)
+        w = rnd(m, k, seed=6, scale=k**-0.5, dtype=torch.bfloat16)
+        got = ops.linear_parts(x.cuda().bfloat16(), w.cuda().bfloat16())
+        want = x.double() @ w.double().t()
+        assert (got.dim() == 3) == (n <= 256)
+        got = got.double().sum(0) if got.dim() == 3 else got.double()
+        tol = 1e-5 if n <= 256 else 2.0**-8  # fp32 sums, or rounded to bf16
+        assert ((got.cpu() - want).abs() <= tol * (1 + want.abs())).all()
+
+
 class TestEmbedding:
     @pytest.mark.parametrize("width", [16, 50, 256])
     def test_scaled_embedding_with_sinusoid(self, be, width):
