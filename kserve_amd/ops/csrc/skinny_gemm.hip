@@ -61,6 +61,13 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
   const int steps = p.K / BK;
   const int lo = (int)((long)steps * blockIdx.y / gridDim.y);
   const int n = (int)((long)steps * (blockIdx.y + 1) / gridDim.y) - lo;
+  // Blocks run through their K range in step, and where a row of W is a multiple of
+  // 4 KB they would all read the same few memory channels at a time: each pair of
+  // blocks starts a step further on and wraps around (us at 1 / 77 rows: K 4096, M
+  // 14336 GLU 46.3 / 53.5 -> 40.1 / 45.6, M 32000 47.8 / 59.7 -> 42.2 / 51.0 = 6.2 TB/s;
+  // K 2048, M 16384 15.5 -> 13.2; 8192 x 8192 30.4 -> 23.7; level at K 5120; a step a
+  // block, or four, leaves some as they were or slower).
+  const int rot = (int)(blockIdx.x / 2) % n;
 
   // first feature of the block's W rows (GLU: of gate and up rows)
   const int f0 = blockIdx.x * (EPI == GLU ? BM / 2 : BM);
@@ -81,9 +88,9 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
     const int c = (lane & 7) ^ ((r >> 1) & 7);
     const short* row = r < BN ? p.x + (long)min(r, p.N - 1) * p.xs
                               : p.w + (long)w_row(r - BN) * p.K;
-    src[i] = reinterpret_cast<const char*>(row + (long)lo * BK + c * 8);
+    src[i] = reinterpret_cast<const char*>(row + (long)(lo + rot) * BK + c * 8);
   }
-  int issue_slot = 0;
+  int issue_slot = 0, to_end = n - rot;
   auto issue = [&]() {  // the next step's loads
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
@@ -99,6 +106,10 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
       }
     }
     issue_slot = issue_slot + 1 == S ? 0 : issue_slot + 1;
+    if (--to_end == 0) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) src[i] -= (long)n * BK * 2;
+    }
   };
 
   f32x4_t acc[F][NT];
