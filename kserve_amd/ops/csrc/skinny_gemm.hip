@@ -66,8 +66,10 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
   // blocks starts a step further on and wraps around (us at 1 / 77 rows: K 4096, M
   // 14336 GLU 46.3 / 53.5 -> 40.1 / 45.6, M 32000 47.8 / 59.7 -> 42.2 / 51.0 = 6.2 TB/s;
   // K 2048, M 16384 15.5 -> 13.2; 8192 x 8192 30.4 -> 23.7; level at K 5120; a step a
-  // block, or four, leaves some as they were or slower).
-  const int rot = (int)(blockIdx.x / 2) % n;
+  // block, or four, leaves some as they were or slower). Not above 64 rows in many
+  // parts: the token rows, then as many as W's, are shared through the L2 by blocks
+  // at one step (K 14336, M 4096 at 96 / 128 rows 28.1 / 30.0, 29.3 / 34.5 with it).
+  const int rot = NT > 4 && gridDim.y > 3 ? 0 : (int)(blockIdx.x / 2) % n;
 
   // first feature of the block's W rows (GLU: of gate and up rows)
   const int f0 = blockIdx.x * (EPI == GLU ? BM / 2 : BM);
