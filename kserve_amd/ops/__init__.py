@@ -326,15 +326,19 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     """Whether the few-row kernel beats the library at [n, k] x [m, k]^T
     (MI355X, us, kernel / library, reduction of the K splits included).
 
-    Up to 48 rows it streams weights faster (k 4096, m 32000 at 1 row 49 / 61,
-    at 24 rows 50 / 60; k 14336, m 4096 at 24 rows 24 / 32; level on small
+    Up to 48 rows it streams weights faster (k 4096, m 32000 at 1 row 42 / 61, at 32
+    rows 40 / 55; k 14336, m 4096 at 24 rows 24 / 32; level on small
     ones, 768 x 768 5.3 / 4.9, and up to 2 us behind where splits of a short K
     need their second launch, k 1024 to 2048, m up to 256: at 48 rows 6.9 / 4.8;
     over 64 to 4096 x 16 to 8192 it takes 0.82 of the time; not everywhere ahead
-    on wide ones past 16 rows: k 5120, m 27648 at 32 rows 57 / 53, at 48 rows 63 /
-    83), up to 64 rows but for the widest (m 14336 28.3 / 27.5). So far a row's
+    on wide ones past 16 rows: k 5120, m 27648 at 32 rows 54 / 51, at 48 rows 60 /
+    75), up to 64 rows but for wide ones with rows off a multiple of 4 KB (k 5120, m
+    27648 68 / 55). So far a row's
     sums do not depend on the rows beside it, and small weights stay here for
-    that. Above, it gains where the
+    that. The widest stay to 112 rows (k 4096, m 32000 at 64 / 80 / 96 / 112 rows 50 / 51,
+    48 / 63, 49 / 53, 55 / 73, m 16384 at 80 / 112 33 / 36, 36 / 38, k 2048, m 32000 at 96
+    rows 27 / 35; but m 16384 22 / 19).
+    Otherwise it gains above where the
     library does not split K over the chip: k 14336, m 4096 at 128 / 256 rows 34 / 74,
     46 / 62, k 8192, m 2048 at 77 / 256 rows 15 / 21, 21 / 27, k 4096, m 4096 at 128
     rows 16 / 25, k 4096, m 6144 22 / 25, at 256 rows 32 / 40, k 3072, m 6144 20 / 21;
@@ -345,6 +349,8 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
         return False
     if n <= 48 or (n <= 64 and m <= 8192):
         return True
+    if m >= 16384 and n <= 112:
+        return k % 2048 == 0 and (n <= 64 or k * m >= 60 << 20)
     if 2048 <= m < 4096:
         return 8192 <= k < 1 << 22
     return (
@@ -357,7 +363,7 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
 def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     """The same for the gate|up product with silu(gate) * up on its sums,
     against the library's product and the activation kernel (k 4096, m 14336:
-    1 row 46 / 67, 48 rows 50 / 67, 64 rows 56 / 59, 96 rows 60 / 60). A block
+    1 row 40 / 67, 48 rows 47 / 67, 64 rows 52 / 59, 96 rows 47 / 60). A block
     takes 32 or, above 64 rows, 64 features and K is not split, so m has to fill
     the chip (k 4096, m 3584 24 / 21 at 64 rows), the more so the longer K is (k
     8192, m 7168 at 1 row 56 / 50, m 14336 88 / 129). Past 48 rows the block's

@@ -12,12 +12,13 @@
 // gate as up features and silu(gate) * up leaves it directly.
 //
 // Measured (us with the reduction, weights not in cache; the library's in
-// parentheses): K 4096, M 14336 GLU at 1 row 46 = 5.1 TB/s (67 with the
-// activation kernel), at 24 rows 47; K 4096, M 32000 at 1 row 49 (61); K
-// 14336, M 4096 at 1 / 24 rows 24 / 24 (27 / 32). Up to 48 rows the loads bound it
+// parentheses): K 4096, M 14336 GLU at 1 row 40 = 5.9 TB/s (67 with the
+// activation kernel), at 24 rows 41; K 4096, M 32000 at 1 row 42 (61); K
+// 14336, M 4096 at 1 / 24 rows 23 / 24 (27 / 32). Up to 48 rows the loads bound it
 // (non-temporal ones took 5 to 10 % off; no gain above); above, LDS reads and the
-// matrix cores of the few blocks that fit, so wide M goes back to the library. The kernel before kept a barrier
-// per step behind one load in flight and rounded the splits to bf16.
+// matrix cores of the few blocks that fit, so M of a few thousand or off a multiple of
+// 4 KB a row goes back to the library. The kernel before kept a barrier per step behind
+// one load in flight and rounded the splits to bf16.
 //
 // C = W X^T on v_mfma_f32_16x16x32_bf16: a lane ends with four consecutive
 // features of one token. LDS rows are 128 bytes; the 16-byte chunk c of row r

@@ -18,6 +18,9 @@ from kserve_amd import ops
         (257, 4096, 8192, False), (8, 4096, 4098, False),
         (65, 8192, 2048, True), (256, 8192, 2048, True), (128, 4096, 2048, False),
         (128, 8192, 2044, False),
+        (64, 4096, 32000, True), (112, 4096, 32000, True), (113, 4096, 32000, False),
+        (64, 2048, 16384, True), (65, 2048, 16384, False),   # 22 us, library 19
+        (64, 5120, 27648, False),                            # 68 / 55
     ],
 )
 def test_few_row_product(n, k, m, own):
