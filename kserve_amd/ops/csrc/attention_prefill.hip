@@ -29,10 +29,10 @@
 // that is followed in steps of 2^8, tile addresses from scalars, and keys read six
 // products ahead took 700 vector cycles and most waits off a tile. Measured (32 query
 // and 8 KV heads of 128, causal; the 16x16x32 kernel with one head per block before,
-// then before and with those): 1 x 8191 tokens 2497 / 620 / 518 us (1060 TFLOP/s), 8 x
-// 2048 1280 / 367 / 319 us, 16 x 500 74 / 67 us; 2 x 1000 queries over 13000 paged
-// keys 2441 / 479 / 420 us (E4M3 pages 2596 / 572 / 500); 8 x 500, 12 heads of 64,
-// bidirectional 18 / 15 us, 64 x 128 level at 13; fp32 scores, 4 x 2000, 16 / 4 heads
+// then before and with those): 1 x 8191 tokens 2497 / 621 / 557 us (990 TFLOP/s), 8 x
+// 2048 1280 / 373 / 329 us, 16 x 500 77 / 72 us; 2 x 1000 queries over 13000 paged
+// keys 2441 / 484 / 438 us (E4M3 pages 2596 / 567 / 500); 8 x 500, 12 heads of 64,
+// bidirectional 20 / 17 us, 64 x 123 level at 13; fp32 scores, 4 x 2000, 16 / 4 heads
 // 239 / 223 us.
 //
 // Replaces the vLLM flash prefill the reference delegates to. Numerics oracles:
@@ -42,6 +42,33 @@
 namespace {
 
 using namespace mfma_attn;
+
+// adds the parts of prefill_attention_kernel's keys: 32 lanes per (token, head),
+// 4 of 128 columns each. Parts without a visible key wrote no sums (weight 0).
+__global__ __launch_bounds__(256) void prefill_attention_merge_kernel(
+    short* __restrict__ out, const float* __restrict__ part_out,
+    const float* __restrict__ part_ml, const int n_splits, const long rows) {
+  constexpr int D = 128;
+  const long row = blockIdx.x * 8L + (threadIdx.x >> 5);
+  if (row >= rows) return;
+  const int d = (threadIdx.x & 31) * 4;
+  float top = -3.4e38f;
+  for (int s = 0; s < n_splits; ++s) {
+    const float2_t ml = *reinterpret_cast<const float2_t*>(part_ml + (s * rows + row) * 2);
+    if (ml[1] > 0.f) top = fmaxf(top, ml[0]);
+  }
+  float sum = 0.f;
+  f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < n_splits; ++s) {
+    const float2_t ml = *reinterpret_cast<const float2_t*>(part_ml + (s * rows + row) * 2);
+    if (ml[1] > 0.f) {
+      const float f = __builtin_amdgcn_exp2f(ml[0] - top);
+      sum += f * ml[1];
+      acc += f * *reinterpret_cast<const f32x4_t*>(part_out + (s * rows + row) * D + d);
+    }
+  }
+  store4(out, row * D + d, acc * (sum > 0.f ? 1.f / sum : 0.f), 0);
+}
 
 // query heads that a block takes
 int heads_per_block(int group) { return group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1; }

@@ -46,11 +46,6 @@ __device__ __forceinline__ f32x16_t mfma32(bf16x8_t a, bf16x8_t b, f32x16_t c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// for buffer loads from a uniform address, offsets below 2^32
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const void* base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00027000);
-}
-
 // What the launchers hand the kernels as their scale: scores are masked before
 // they are scaled, and the scaled mask has to give weight 0. Below 1e-30 all
 // scores are level whatever the scale.
@@ -253,9 +248,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   auto page_of = [&](int t) { return PAGED ? bt[group_of(t) >> 4] : 0; };
   // A scalar base per tile and 32-bit lane offsets (the launchers see to strides
   // below 2^26): tiles with all their keys cost no vector arithmetic, where 64-bit
-  // addresses per lane and load took 500 of a tile's 1800 vector cycles. The
-  // LDS-direct loads are buffer loads: after the global form the compiler waits
-  // for all of a wave's LDS reads at once instead of one after the other.
+  // addresses per lane and load took 500 of a tile's 1800 vector cycles. (As buffer
+  // loads they would leave the compiler's waits for a wave's LDS reads one after the
+  // other: 1 x 8191 tokens 564 -> 550 us, 64 texts of 123 tokens with heads of 64 13.3 ->
+  // 14.1; the check of the waits ahead of the barriers reads the global form.)
   constexpr int ES = SRC == PAGES_FP8 ? 1 : 2;
   const int krs = PAGED && PARTS == 1 ? D : (int)p.sk;  // bf16 queries: whole rows
   const int vrs = PAGED && PARTS == 1 ? D : (int)p.sv;
@@ -281,12 +277,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
     for (int i = 0; i < NI; ++i) {
       const unsigned int ka = k_at(i), va = v_at(i);
       if constexpr (DMA) {
-        typedef __attribute__((address_space(3))) void lds_t;
         const int at = (wave * 16 + i * RPI) * D;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(raw_buffer(kb), (lds_t*)&lds[buf][0][at],
-                                                 16, ka, 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(raw_buffer(vb), (lds_t*)&lds[buf][1][at],
-                                                 16, va, 0, 0, 0);
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const unsigned int*>(kb + ka),
+                                         reinterpret_cast<unsigned int*>(&lds[buf][0][at]),
+                                         16, 0, 0);
+        __builtin_amdgcn_global_load_lds(reinterpret_cast<const unsigned int*>(vb + va),
+                                         reinterpret_cast<unsigned int*>(&lds[buf][1][at]),
+                                         16, 0, 0);
       } else if constexpr (SRC == PAGES_FP8) {
         raw8[2 * i] = *reinterpret_cast<const uint2*>(kb + ka);
         raw8[2 * i + 1] = *reinterpret_cast<const uint2*>(vb + va);
@@ -540,33 +537,6 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
       store4(p.out, (tok * p.Hq + head) * D + half * 4 + b * 32 + g * 8, w,
              PARTS == 1 ? 0 : p.x.out_f32);
     }
-}
-
-// adds the parts of prefill_attention_kernel's keys: 32 lanes per (token, head),
-// 4 of 128 columns each. Parts without a visible key wrote no sums (weight 0).
-__global__ __launch_bounds__(256) void prefill_attention_merge_kernel(
-    short* __restrict__ out, const float* __restrict__ part_out,
-    const float* __restrict__ part_ml, const int n_splits, const long rows) {
-  constexpr int D = 128;
-  const long row = blockIdx.x * 8L + (threadIdx.x >> 5);
-  if (row >= rows) return;
-  const int d = (threadIdx.x & 31) * 4;
-  float top = -3.4e38f;
-  for (int s = 0; s < n_splits; ++s) {
-    const float2_t ml = *reinterpret_cast<const float2_t*>(part_ml + (s * rows + row) * 2);
-    if (ml[1] > 0.f) top = fmaxf(top, ml[0]);
-  }
-  float sum = 0.f;
-  f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < n_splits; ++s) {
-    const float2_t ml = *reinterpret_cast<const float2_t*>(part_ml + (s * rows + row) * 2);
-    if (ml[1] > 0.f) {
-      const float f = __builtin_amdgcn_exp2f(ml[0] - top);
-      sum += f * ml[1];
-      acc += f * *reinterpret_cast<const f32x4_t*>(part_out + (s * rows + row) * D + d);
-    }
-  }
-  store4(out, row * D + d, acc * (sum > 0.f ? 1.f / sum : 0.f), 0);
 }
 
 // Key parts of a prefill over pages. A block walks its tiles of 64 keys one after
