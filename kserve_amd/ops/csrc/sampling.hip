@@ -817,10 +817,13 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
 // size has merged its waves (256 x 32000, greedy: 5.9 us with 256 threads, 7.0
 // with 1024; with noise 10.5 with 256 threads that evaluate every element, 11.9
 // with 512 and the bound)
+// Rows that fill 1024 threads a few times over take as many: a row's time is the
+// latency of its loads one after the other (1 / 96 rows of 32000 5.6 / 8.7 -> 4.7 / 5.8
+// us; noise for every element keeps 256 busy up to 65536).
 template <bool GUMBEL>
 void launch_argmax(void* out, const void* logits, const void* temperatures,
                    const void* seeds, int num_seqs, int vocab, hipStream_t stream) {
-  if (vocab > 65536)
+  if (vocab > (GUMBEL ? 65536 : 8192))
     hipLaunchKernelGGL((argmax_kernel<GUMBEL, 1024>), dim3(num_seqs), dim3(1024), 0,
                        stream, (long*)out, (const short*)logits,
                        (const float*)temperatures, (const long*)seeds, vocab);
