@@ -873,6 +873,10 @@ __global__ void __launch_bounds__(DT) ssd_decays_kernel(
   // a sum over a chunk may be far larger than the difference of two neighbours
   __shared__ double cum[NW][CQ];
   __shared__ float dts[NW][CQ];
+  constexpr int NP = NB * 16;
+  constexpr int RS = NP + 4;  // 4 rows apart fall 16 banks apart
+  __shared__ __attribute__((aligned(16))) float Bs[CQ * RS];
+  __shared__ __attribute__((aligned(16))) float Cs[CQ * RS];
   const int chunk = blockIdx.x;
   const int lane = threadIdx.x & 63;
   if (order && chunk == 0 && blockIdx.y == 0 && threadIdx.x < 64) {
@@ -903,34 +907,44 @@ __global__ void __launch_bounds__(DT) ssd_decays_kernel(
   const int inner = heads * P;
   const long channels = inner + 2L * groups * N;
 
+  // rows through LDS: as fragments straight from memory, 16 rows to a load with
+  // neighbouring lanes in different ones, they come at a quarter of the rate
+#pragma unroll
+  for (int i = 0; i < CQ * NP / 4 / DT; ++i) {
+    const int e = threadIdx.x + i * DT;
+    const int t = e / (NP / 4), n = e % (NP / 4) * 4;
+    const bool ok = t0 + t < end && n < N;
+    const float* row = xbc + (t0 + t) * channels + inner + grp * N + n;
+    const f32x4s zero = f32x4s{0.f, 0.f, 0.f, 0.f};
+    *reinterpret_cast<f32x4s*>(Bs + t * RS + n) =
+        ok ? *reinterpret_cast<const f32x4s*>(row) : zero;
+    *reinterpret_cast<f32x4s*>(Cs + t * RS + n) =
+        ok ? *reinterpret_cast<const f32x4s*>(row + groups * N) : zero;
+  }
+  __syncthreads();
+
   f32x4s cb[NG];  // B_s . C_t: row s, column t
 #pragma unroll
   for (int i = 0; i < NG; ++i) {
     if (wave + i * NW >= CTILES) continue;
     int tb, sb;
     chunk_tile(wave + i * NW, tb, sb);
-    const int t = t0 + tb * 16 + col, u = t0 + sb * 16 + col;
-    const float* cr = xbc + t * channels + inner + (groups + grp) * N + g * 4;
-    const float* br = xbc + u * channels + inner + grp * N + g * 4;
-    const f32x4s zero = f32x4s{0.f, 0.f, 0.f, 0.f};
-    f32x4s c4[NB], b4[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const bool ok = b * 16 + g * 4 < N;
-      c4[b] = ok && t < end ? *reinterpret_cast<const f32x4s*>(cr + b * 16) : zero;
-      b4[b] = ok && u < end ? *reinterpret_cast<const f32x4s*>(br + b * 16) : zero;
-    }
+    const float* cr = Cs + (tb * 16 + col) * RS + g * 4;
+    const float* br = Bs + (sb * 16 + col) * RS + g * 4;
     // eight chains: fewer roundings in a row than one sum over the states
     f32x4s acc[8];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) acc[r] = zero;
+    for (int r = 0; r < 8; ++r) acc[r] = f32x4s{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int b = 0; b < NB; ++b)
+    for (int b = 0; b < NB; ++b) {
+      const f32x4s c4 = *reinterpret_cast<const f32x4s*>(cr + b * 16);
+      const f32x4s b4 = *reinterpret_cast<const f32x4s*>(br + b * 16);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         f32x4s& to = acc[r + (b & 1) * 4];
-        to = mfma4(b4[b][r], c4[b][r], to);
+        to = mfma4(b4[r], c4[r], to);
       }
+    }
     cb[i] = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
   }
 
