@@ -850,9 +850,9 @@ def _scan_chunks_apart(tokens: int, seqs: int, longest: int, heads: int, P: int)
     Both times are estimated, in us, for 64 heads of 64 columns and 128 states: one
     launch pays every chunk its chain of barriers, a block a compute unit; two pay the
     launch and run two blocks a unit, or smaller ones on units that would be idle.
-    (One / two launches: 1 x 64 tokens 12.8 / 17.4, 1 x 100 21.6 / 20.2, 2 x 100 22.3
-    / 25.1, 4 x 200 46.0 / 47.3, 8 x 128 51.9 / 51.0, 6 x 130 64.9 / 53.5, 32 x 64 104 /
-    100, 32 x 100 179 / 153, 40 + 300 49.4 / 33.2.)"""
+    (One / two launches: 1 x 64 tokens 12.7 / 15.1, 1 x 100 21.8 / 18.0, 2 x 100 22.4
+    / 23.4, 4 x 200 46.0 / 46.2, 8 x 128 52.9 / 50.3, 6 x 130 64.7 / 53.1, 32 x 64 104 /
+    97, 32 x 100 180 / 149, 40 + 300 49.2 / 36.7.)"""
     if seqs == 0:
         return False
     blocks = -(-P // 64) * heads * seqs

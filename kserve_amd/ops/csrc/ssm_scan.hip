@@ -819,11 +819,11 @@ __global__ void __launch_bounds__(CT) ssd_chunk_kernel(
 // 64 bits, 64 x 64 exponentials and three barriers stood between them, with one
 // block a compute unit. Here two blocks of 32 columns share a unit (7.8 us a chunk
 // of both, 4.2 of them products, 160 per wave and block) and a block alone takes
-// 4.7 us, of 16 columns 3.0. The first launch moves 19 KB a chunk and head at 3.5
-// TB/s (44 us for 8000 tokens of 64 heads). us, one launch / two (64 heads of 64
-// columns, 128 states): 4 x 2000 tokens 308 / 260, 1 x 2000 296 / 107, 1 x 8000
-// 1154 / 398, 8 x 2000 628 / 518, 32 x 128 187 / 164, 1 x 100 21.6 / 20.2, 4 x 64
-// 15.5 / 27. Error of y against 64 bits 8.5e-8 both.
+// 4.7 us, of 16 columns 3.0. The first launch moves 19 KB a chunk and head at 4.0
+// TB/s (38 us for 8000 tokens of 64 heads). us, one launch / two (64 heads of 64
+// columns, 128 states): 4 x 2000 tokens 310 / 257, 1 x 2000 291 / 106, 1 x 8000
+// 1156 / 390, 8 x 2000 630 / 521, 32 x 128 188 / 162, 1 x 100 21.8 / 18.0, 4 x 64
+// 15.4 / 25.7. Error of y against 64 bits 8.5e-8 both.
 // ---------------------------------------------------------------------------
 constexpr int CTILES = 10;
 
