@@ -729,9 +729,13 @@ def add_rms_norm_f32res(
     returns the normed rows in ``out_dtype`` (``weight`` None: the new residual
     itself; ``want_out`` off: nothing). With ``d1_index`` [T*d1_top] int32 the
     second delta of token t is the sum over k of d1_weights[t*d1_top + k] *
-    d1[d1_index[t*d1_top + k]] (fp32 weights or None for 1). A delta of three
-    dimensions is the sum over the first (``linear_parts``)."""
-    if (d0 is not None and d0.dim() == 3) or (d1 is not None and d1.dim() == 3):
+    d1[d1_index[t*d1_top + k]] (fp32 weights or None for 1). A delta of one
+    dimension more than the residual is the sum over its first (``linear_parts``)."""
+
+    def in_parts(d):
+        return d is not None and d.dim() == residual.dim() + 1
+
+    if in_parts(d0) or (d1_index is None and in_parts(d1)):
         plain = c0 is None and c1 is None and d1_index is None and weight is not None
         if plain and want_out and out_dtype == torch.bfloat16 and residual.is_cuda:
             out = torch.empty(residual.shape, dtype=out_dtype, device=residual.device)
@@ -740,9 +744,7 @@ def add_rms_norm_f32res(
                 float(eps), out,
             )
             return out
-        d0, d1 = (
-            d if d is None or d.dim() < 3 else d.sum(0).to(out_dtype) for d in (d0, d1)
-        )
+        d0, d1 = (d.sum(0).to(out_dtype) if in_parts(d) else d for d in (d0, d1))
     if residual.is_cuda:
         out = (
             torch.empty(residual.shape, dtype=out_dtype, device=residual.device)

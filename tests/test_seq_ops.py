@@ -101,6 +101,17 @@ class TestResidualNormInParts:
         close(r, want, be, f32_tol=4e-6, bf16_tol=4e-6)
         close(got, O.rms(want, 1e-5) * (1 + w.double()), be, f32_tol=4e-6, bf16_tol=2.0**-8)
 
+    def test_rows_of_rows(self):
+        """A residual of three dimensions has deltas of three: rows, not parts."""
+        x, w = rnd(3, 5, 16, seed=1), rnd(16, seed=2, scale=0.1)
+        d = rnd(3, 5, 16, seed=3)
+        r = x.clone()
+        got = ops.add_rms_norm_f32res(r, w, 1e-5, 1.0, torch.float32, d, 0.5, d, 2.0)
+        want = x.double() + 2.5 * d.double()
+        torch.testing.assert_close(r.double(), want, rtol=1e-6, atol=1e-6)
+        want = O.rms(want.view(15, 16), 1e-5).view_as(want) * (1 + w.double())
+        torch.testing.assert_close(got.double(), want, rtol=4e-6, atol=4e-6)
+
     @pytest.mark.gpu
     @pytest.mark.parametrize(
         "n,k,m", [(1, 4096, 2048), (64, 8192, 2048), (65, 4096, 2048), (200, 4096, 2052), (300, 4096, 2048)]
