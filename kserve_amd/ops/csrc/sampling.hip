@@ -114,8 +114,9 @@ __device__ __forceinline__ void block_argmax(float best, int best_idx, long* out
 }
 
 __device__ __forceinline__ float noise_of_hash(unsigned int h) {
-  // u in (0,1): (h + 1) / 2^32
-  const float u = ((float)h + 1.0f) * 2.3283064e-10f;
+  // u in (0,1): (h + 1) / 2^32, which rounds to 1 for the last 128 hashes: their
+  // noise would be infinite, and win the row whatever the logit
+  const float u = fminf(((float)h + 1.0f) * 2.3283064e-10f, 0.99999994f);
   return __logf(-__logf(u));
 }
 // Whether x / T + G can reach the best score that the wave has seen. With u = 1 -

@@ -790,7 +790,7 @@ class TestSampling:
         h = h ^ (h >> 12)
         h = (h * 0x297A2D39) & M
         h = h ^ (h >> 15)
-        u = (h.float() + 1.0) * 2.3283064e-10
+        u = ((h.float() + 1.0) * 2.3283064e-10).clamp(max=1 - 2.0**-24)
         x = logits.double() / temps[:, None].double()
         score = x - torch.log(-torch.log(u.double()))
         for r in range(n):
@@ -856,7 +856,7 @@ class TestSampling:
         for mul, shift in ((0x2C1B3C6D, 12), (0x297A2D39, 15)):
             h = ((h ^ (h >> 15)) * mul & M) if shift == 12 else h * mul & M
             h = h ^ (h >> shift)
-        u = (h.float() + 1.0) * 2.3283064e-10
+        u = ((h.float() + 1.0) * 2.3283064e-10).clamp(max=1 - 2.0**-24)
         x = logits.double() / temps[:, None].double()
         score = x - torch.log(-torch.log(u.double()))
         for r in range(n):
@@ -876,6 +876,52 @@ class TestSampling:
             # fast fp32 logarithms and the fp32 score itself: a few ulp of it
             near = 1e-4 + 4 * 2.0 ** -24 * float(x[r][got].abs())
             assert s.max() <= score[r][got] + near, (r, got, int(s.argmax()))
+
+    @pytest.mark.parametrize("vocab", [9, 32000, 128256])
+    @pytest.mark.parametrize("limit", ["none", "gumbel", "cut"])
+    def test_last_hashes(self, dev, vocab, limit):
+        """u = (hash + 1) / 2^32 rounds to 1 for the last 128 hashes. An element of
+        e^-60 of the row's mass with such a hash does not win."""
+        import kserve_amd_C
+
+        M = 1 << 32
+
+        def seed_of(h, idx):  # the kernel's hash, backwards
+            h ^= h >> 15 ^ h >> 30
+            h = h * pow(0x297A2D39, -1, M) % M
+            h ^= h >> 12 ^ h >> 24
+            h = h * pow(0x2C1B3C6D, -1, M) % M
+            h ^= h >> 15 ^ h >> 30
+            h -= idx * 0x85EBCA77 + 0x165667B1
+            return h * pow(0x9E3779B1, -1, M) % M
+
+        picks = [0, vocab // 2, vocab - 1]
+        rows = [(i, M - 1 - r) for i in picks for r in (0, 1, 64, 127)]
+        logits = torch.zeros(len(rows), vocab)
+        for row, (i, _) in enumerate(rows):
+            logits[row, i] = -60.0
+            logits[row, i - 1] = -80.0  # what "cut" cuts
+        seeds = torch.tensor([seed_of(h, i) for i, h in rows])
+        # the hash forwards, as the tests of the limits have it
+        h = (seeds * 0x9E3779B1 + torch.tensor([i for i, _ in rows]) * 0x85EBCA77 + 0x165667B1) % M
+        for mul, shift in ((0x2C1B3C6D, 12), (0x297A2D39, 15)):
+            h = (h ^ (h >> 15)) * mul % M if shift == 12 else h * mul % M
+            h = h ^ (h >> shift)
+        assert h.tolist() == [b for _, b in rows]
+
+        n = len(rows)
+        args = [
+            torch.empty(n, dtype=torch.int64, device=dev),
+            logits.to(dev, torch.bfloat16), torch.ones(n, device=dev),
+        ]
+        top_k = torch.full((n,), vocab - 1 if limit == "cut" else 0, dtype=torch.int32)
+        if limit != "gumbel":
+            kserve_amd_C.topk_topp_sample(
+                *args, torch.ones(n, device=dev), top_k.to(dev), seeds.to(dev)
+            )
+        else:
+            kserve_amd_C.gumbel_sample(*args, top_k.to(dev), seeds.to(dev))
+        assert all(int(got) != i for got, (i, _) in zip(args[0], rows))
 
     @pytest.mark.parametrize("vocab", [5, 32000, 70001])
     def test_topk1_ties_are_greedy(self, dev, vocab):
