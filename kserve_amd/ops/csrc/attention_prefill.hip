@@ -44,7 +44,9 @@ namespace {
 using namespace mfma_attn;
 
 // adds the parts of prefill_attention_kernel's keys: 32 lanes per (token, head),
-// 4 of 128 columns each. Parts without a visible key wrote no sums (weight 0).
+// 4 of 128 columns each. Parts without a tile wrote no sums; the others count even
+// where their weights are NaN (by bits: a comparison of a NaN is the compiler's to
+// choose here), so that NaNs come out as from one part.
 __global__ __launch_bounds__(256) void prefill_attention_merge_kernel(
     short* __restrict__ out, const float* __restrict__ part_out,
     const float* __restrict__ part_ml, const int n_splits, const long rows) {
@@ -52,16 +54,19 @@ __global__ __launch_bounds__(256) void prefill_attention_merge_kernel(
   const long row = blockIdx.x * 8L + (threadIdx.x >> 5);
   if (row >= rows) return;
   const int d = (threadIdx.x & 31) * 4;
+  auto empty = [](float l) {
+    return __builtin_bit_cast(int, l) == __builtin_bit_cast(int, NO_KEYS);
+  };
   float top = -3.4e38f;
   for (int s = 0; s < n_splits; ++s) {
     const float2_t ml = *reinterpret_cast<const float2_t*>(part_ml + (s * rows + row) * 2);
-    if (ml[1] > 0.f) top = fmaxf(top, ml[0]);
+    if (!empty(ml[1])) top = fmaxf(top, ml[0]);
   }
   float sum = 0.f;
   f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
   for (int s = 0; s < n_splits; ++s) {
     const float2_t ml = *reinterpret_cast<const float2_t*>(part_ml + (s * rows + row) * 2);
-    if (ml[1] > 0.f) {
+    if (!empty(ml[1])) {
       const float f = __builtin_amdgcn_exp2f(ml[0] - top);
       sum += f * ml[1];
       acc += f * *reinterpret_cast<const f32x4_t*>(part_out + (s * rows + row) * D + d);

@@ -144,8 +144,9 @@ struct PrefillArgs {
   int n_splits;
   long rows;        // T * Hq
   float* part_out;  // [n_splits, T, Hq, D]
-  float* part_ml;   // [n_splits, T, Hq, 2]: exponent, sum of weights
+  float* part_ml;   // [n_splits, T, Hq, 2]: exponent, sum of weights or NO_KEYS
 };
+constexpr float NO_KEYS = -1.f;  // of a part without a tile, which writes no sums
 
 template <int D, int SRC, bool CAUSAL, bool WIN, int PARTS = 1>
 __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
@@ -499,8 +500,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
   const long tok = q_start + qrow;
   if (SPLITS && p.n_splits > 1) {
     const long row = split * p.rows + tok * p.Hq + head;
-    if (half == 0) *reinterpret_cast<float2_t*>(p.part_ml + row * 2) = float2_t{mc, l};
-    if (t_lo >= t_hi) return;
+    const bool none = t_lo >= t_hi;
+    if (half == 0)
+      *reinterpret_cast<float2_t*>(p.part_ml + row * 2) = float2_t{mc, none ? NO_KEYS : l};
+    if (none) return;
 #pragma unroll
     for (int b = 0; b < DB; ++b)
 #pragma unroll

@@ -589,6 +589,39 @@ class TestPrefillAttention:
         assert (got.double().cpu() - ref).norm() < 5e-4 * ref.norm()
 
     @pytest.mark.parametrize("fp8", [False, True])
+    @pytest.mark.parametrize("where", ["key", "late_key", "value", "query"])
+    def test_context_prefill_nan(self, dev, where, fp8):
+        """A NaN in a cached key, a value or a query reaches the outputs that it
+        reaches with the keys in one part, and no others."""
+        from kserve_amd import ops
+
+        H, Hkv, D, T, ctx = 4, 2, 128, 40, 1500  # few blocks, 24 tiles: many parts
+        torch.manual_seed(7)
+        q = torch.randn(T, H, D, device=dev).to(torch.bfloat16)
+        k, v = (torch.randn(ctx + 4, Hkv, D, device=dev).to(torch.bfloat16) for _ in "kv")
+        at = ctx - 20 if where == "late_key" else 700  # among the queries, or before
+        if where == "query":
+            q[9, 2, 5] = float("nan")
+        else:
+            (v if where == "value" else k)[at, 1, 3] = float("nan")
+        pages = [x.view(-1, 16, Hkv, D).transpose(1, 2).contiguous() for x in (k, v)]
+        if fp8:
+            pages = [x.to(torch.float8_e4m3fn) for x in pages]
+        i32 = dict(dtype=torch.int32, device=dev)
+        out = ops.context_attention_varlen(
+            q, *pages, torch.arange(pages[0].shape[0], **i32)[None],
+            torch.tensor([0, T], **i32), torch.tensor([ctx], **i32), T, D**-0.5,
+        )
+        want = torch.zeros(T, H, D, dtype=torch.bool)
+        if where == "query":
+            want[9, 2] = True
+        elif where == "value":
+            want[:, 2:, 3] = True
+        else:
+            want[max(0, at - (ctx - T)):, 2:] = True
+        assert (out.isnan().cpu() == want).all()
+
+    @pytest.mark.parametrize("fp8", [False, True])
     @pytest.mark.parametrize("window", [0, 50])
     @pytest.mark.parametrize("H,Hkv", [(4, 1), (6, 3), (2, 2), (8, 1)])
     def test_context_prefill_tile_edges(self, dev, H, Hkv, window, fp8):
