@@ -130,14 +130,19 @@ __device__ __forceinline__ float noise_of_hash(unsigned int h) {
 // most; the rest of the 0.15 and the term in |best| are for the fp32 sums of scores.
 struct GumbelBound {
   static constexpr float ONE = 8388608.f;  // 2^23: 1 in log2 as a pattern
-  float c1, c0 = 3e38f;                    // everything passes at first
+  float c1, c0 = __builtin_bit_cast(float, 0x7f800000);  // every number passes at first
 
   __device__ __forceinline__ explicit GumbelBound(float inv_t)
-      : c1(inv_t * 1.44269504f * ONE) {}
+      : c1(inv_t * 1.44269504f * ONE) {
+    asm("" : "+v"(c0));  // (infinite, which fast math would take for impossible)
+  }
   __device__ __forceinline__ bool passes(float x, unsigned int hash) const {
     const float r = (float)(~hash);
-    // at least the pattern of 4096, and within the range of an int
-    const float t = __builtin_amdgcn_fmed3f(x * c1 + c0, 1166016512.f, 2.1e9f);
+    // At least the pattern of 4096, and within the range of an int. The product of a
+    // low x is past the range of a float, as c0 is after such a best: in one rounding
+    // the sum is infinite for every number and NaN, which is taken for the lower
+    // limit, for an x of -inf.
+    const float t = __builtin_amdgcn_fmed3f(__builtin_fmaf(x, c1, c0), 1166016512.f, 2.1e9f);
     return __builtin_bit_cast(int, r) <= (int)t;
   }
   // by a whole wave

@@ -910,6 +910,29 @@ class TestSampling:
             near = 1e-4 + 4 * 2.0 ** -24 * float(x[r][got].abs())
             assert s.max() <= score[r][got] + near, (r, got, int(s.argmax()))
 
+    @pytest.mark.parametrize("low", [-3e33, -1.5e32])
+    @pytest.mark.parametrize("limit", [0, 70002, 70000])
+    def test_lowest_rows(self, dev, low, limit):
+        """Logits beside which any noise is nothing: the largest wins, wherever it
+        stands, -inf before it or not."""
+        import kserve_amd_C
+
+        vocab, n = 70003, 12
+        logits = torch.full((n, vocab), low * 2)
+        best = torch.randint(9, vocab - 9, (n,), generator=torch.Generator().manual_seed(3))
+        logits[torch.arange(n), best] = low
+        logits[::2, :8192] = logits[::2, :8192].masked_fill(
+            logits[::2, :8192] != low, float("-inf"))
+        logits[:, -1] = float("-inf")
+        out = torch.empty(n, dtype=torch.int64, device=dev)
+        kserve_amd_C.topk_topp_sample(
+            out, logits.to(dev, torch.bfloat16), torch.ones(n, device=dev),
+            torch.ones(n, device=dev),
+            torch.full((n,), limit, dtype=torch.int32, device=dev),
+            torch.arange(n, device=dev),
+        )
+        assert torch.equal(out.cpu(), best)
+
     @pytest.mark.parametrize("vocab", [9, 32000, 128256])
     @pytest.mark.parametrize("limit", ["none", "gumbel", "cut"])
     def test_last_hashes(self, dev, vocab, limit):
