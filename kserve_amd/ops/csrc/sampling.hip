@@ -341,9 +341,11 @@ __global__ __launch_bounds__(AM_NT) void argmax_f32_kernel(
 // between 2^-16 and 2^16 of either sign in 8193 bins (those closer to 0 share one)
 // and the first and last bin, by 16-bit packed operations while the row comes from
 // memory. The mass is formed from the counts, and the bins are scanned from the
-// row's largest, 1024 at a time, until both limits are found; one scan nearly always
-// does. Rows with NaNs or numbers past 2^16, and limits
-// among the numbers closer to 0 than 2^-16 go through the passes above.
+// row's largest, 1024 at a time, until the higher limit is found; one scan nearly
+// always does. Where fewer than k elements have a bin, the others being masked, all
+// of those survive. Where a limit, or mass that counts, lies at 0, a pass more tells
+// the zeros apart. Rows with NaNs or numbers above 2^16, and those where numbers
+// between 0 and 2^-16 of either sign decide, go through the passes above.
 //
 // The last pass queues a wave's survivors in LDS and evaluates them 64 at a time,
 // so a set of any density costs what it holds.
@@ -353,7 +355,9 @@ __global__ __launch_bounds__(AM_NT) void argmax_f32_kernel(
 // logits, one per compute unit (us, three passes / this): 256 x 128256 top-p 0.9 75
 // / 41, top-k 50 49 / 29, both 52 / 30; 15 x 128256 66 / 34, 40 / 20, 45 / 22; 256 x
 // 32000 33 / 20, 23 / 14, 29 / 16; limits below zero 131 / 68 (a histogram by the
-// keys' upper byte took 704 at 256 x 128256). Holding the row in registers over the
+// keys' upper byte took 704 at 256 x 128256). 256 x 128256, top-k 50 of 20 numbers, the
+// rest masked, 306 / 38; half of the row 0, top-p 0.99 212 / 111 (all of it 0: 137 /
+// 162, the counts of one bin one after the other). Holding the row in registers over the
 // passes was no faster.
 // ---------------------------------------------------------------------------
 constexpr int RT = 1024;
@@ -435,7 +439,7 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
     long* __restrict__ out,            // [S]
     const short* __restrict__ logits,  // [S, V] bf16
     const float* __restrict__ temperatures,
-    const float* __restrict__ top_p,  // [S] (>=1 disables)
+    const float* __restrict__ top_p,  // [S] (>=1 and <=0 disable)
     const int* __restrict__ top_k,    // [S] (<=0 disables)
     const long* __restrict__ seeds,   // [S]
     const int V) {
@@ -446,7 +450,7 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
   const int k = top_k[s];
   const unsigned int seed = (unsigned int)(seeds[s] & 0xFFFFFFFF);
   const bool use_k = (k > 0) && (k < V);
-  bool use_p = p < 1.0f;
+  bool use_p = p > 0.f && p < 1.f;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   constexpr int NWV = RT / 64;
@@ -541,14 +545,13 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
         for (int w = 0; w < NWV; ++w) zz += w_mass[w];
       }
       const double want = (double)p * zz;
-      bool find_k = use_k, find_p = use_p && want > 0;
       unsigned int over_k = 0;  // elements and mass of the bins before
       double over_p = 0;
-      for (int b0 = lo; b0 < FBINS && (find_k || find_p); b0 += RT) {
+      for (int b0 = lo; b0 < FBINS; b0 += RT) {
         __syncthreads();  // the sums of the round before are read
         const int bin = b0 + tid;
         const unsigned int n = bin < FBINS ? lds.win[bin] : 0u;
-        const double m = find_p && n ? n * weight_of_bin(bin) : 0.0;
+        const double m = use_p && n ? n * weight_of_bin(bin) : 0.0;
         unsigned int nk = n;
         double mp = m;
 #pragma unroll
@@ -576,23 +579,70 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
         }
         // the first bin at which the running sum reaches its target; in
         // floating point a thread's end need not be the next one's start
-        if (find_k && n && ck < (unsigned int)k && ck + n >= (unsigned int)k)
+        if (use_k && n && ck < (unsigned int)k && ck + n >= (unsigned int)k) {
           atomicMin(&sh_bin[0], bin);
-        if (find_p && n && cp < want && cp + m >= want) atomicMin(&sh_bin[1], bin);
+          if (bin == FSPAN) sh_above_k = ck;
+        }
+        if (use_p && n && cp < want && cp + m >= want) {
+          atomicMin(&sh_bin[1], bin);
+          if (bin == FSPAN) sh_above_p = cp;
+        }
         __syncthreads();
-        if (sh_bin[0] != NONE) find_k = false;
-        if (sh_bin[1] != NONE) find_p = false;
+        // the smaller bin is the higher limit, and what is not found yet lies below
+        if (min(sh_bin[0], sh_bin[1]) != NONE) break;
       }
-      // the smaller bin is the higher limit; a limit that was not found lies
-      // below one that was
       const int bin = min(sh_bin[0], sh_bin[1]);
-      // What the mass is not exact in has to be nothing beside it: numbers closer
-      // to 0 than 2^-16 (known to 2^-16 / T of theirs) and those below -2^16.
-      const double off =
-          lds.win[FSPAN] * weight_of_bin(FSPAN) * c2 * 1.6e-5 +
-          (hi < FBINS ? 0.0 : V * (double)__builtin_amdgcn_exp2f((-65536.f - most) * c2));
-      if (bin != NONE && bin != FSPAN && (!use_p || off <= 3e-8 * zz))
-        thr = (unsigned int)(bin_ordered(bin) + 32768);
+      // Numbers below -2^16 and -inf have no bin. Where the largest stands 40 / ln 2
+      // scaled logits above them, no noise (-3.1 to 16.7) brings one up, and their mass
+      // has to be nothing beside the row's.
+      const double below = V * (double)__builtin_amdgcn_exp2f((-65536.f - most) * c2);
+      const bool whole =
+          hi < FBINS || ((most + 65536.f) * c2 >= 40.f && below <= 3e-8);
+      // Numbers closer to 0 than 2^-16 share a bin. With a limit in it, or their mass
+      // (known to 2^-16 / T of it) not to be left uncertain, zeros are told apart.
+      const unsigned int near = lds.win[FSPAN];
+      const double weight0 = near ? weight_of_bin(FSPAN) : 0.0;
+      auto known = [&](unsigned int n) {
+        return !use_p || n * weight0 * c2 * 1.6e-5 <= 3e-8 * zz;
+      };
+      bool sure = known(near);
+      // positive numbers down to the last before 0, to the last +0, to the last -0
+      unsigned int to[3] = {0, 0, 0};
+      if (near && (bin == FSPAN || !sure)) {
+        row.each([&](short b, int) {
+          const unsigned int u = (unsigned short)b;
+          to[0] += u - 1 < (unsigned int)NEAR_HI ? 1u : 0u;
+          to[1] += u == 0u ? 1u : 0u;
+          to[2] += u == 0x8000u ? 1u : 0u;
+        });
+        unsigned int* const sums[3] = {w_cnt, s_key, s_bad};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+#pragma unroll
+          for (int off = 32; off > 0; off >>= 1)
+            to[i] += (unsigned int)__shfl_xor((int)to[i], off, 64);
+          if (lane == 0) sums[i][wave] = to[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          to[i] = i ? to[i - 1] : 0u;
+#pragma unroll
+          for (int w = 0; w < NWV; ++w) to[i] += sums[i][w];
+        }
+        sure = known(near - (to[2] - to[0]));
+      }
+      // (a limit of top-k above all that has no bin needs no mass)
+      if (sure && (whole || (bin != NONE && !use_p))) {
+        if (bin == FSPAN) {
+          const double k_left = sh_bin[0] == FSPAN ? (double)k - sh_above_k : 1e30;
+          const double p_left = sh_bin[1] == FSPAN ? want - sh_above_p : 1e30;
+          auto reached = [&](unsigned int n) { return k_left <= n || p_left <= n * weight0; };
+          if (!reached(to[0])) thr = reached(to[1]) ? 0x8000u : reached(to[2]) ? 0x7fffu : 0u;
+        } else {  // no limit among the bins: all that is in them
+          thr = (unsigned int)(bin_ordered(bin == NONE ? FBINS - 1 : bin) + 32768);
+        }
+      }
     }
     __syncthreads();
   }

@@ -847,13 +847,16 @@ class TestSampling:
             assert s[got] >= s.max() - 1e-4, (r, got, int(s.argmax()))
 
     @pytest.mark.parametrize(
-        "mode", ["near_zero", "huge", "lowest", "below_zero", "zeros", "warm"]
+        "mode",
+        ["near_zero", "huge", "lowest", "below_zero", "zeros", "warm", "few",
+         "few_lowest", "few_hot", "signed_zeros", "all_zeros", "deep", "no_mass"],
     )
     @pytest.mark.parametrize("vocab", [9, 1031, 8200, 40003])
     def test_limits_of_the_first_pass(self, dev, vocab, mode):
         """Rows at the edges of the bins from 2^-16 to 2^16: limits closer to 0,
         numbers past the bins on either side, limits among negative numbers,
-        survivors from a handful to nearly all. Every token is one that the
+        survivors from a handful to nearly all, rows with fewer numbers than top-k
+        (the rest masked), limits among zeros of either sign. Every token is one that the
         float64 limits leave, and the best of them by the kernel's noise."""
         import kserve_amd_C
 
@@ -876,6 +879,22 @@ class TestSampling:
             logits[:, ::2] = 0.0
         if mode == "warm":
             temps = temps * 40
+        if mode.startswith("few"):
+            masked = torch.rand(n, vocab, generator=g).argsort(1) >= min(12, vocab - 2)
+            masks = torch.finfo(torch.bfloat16).min, float("-inf")
+            logits = logits.masked_fill(masked, masks[mode != "few_lowest"])
+            if mode == "few_hot":  # masked by less than the noise reaches
+                logits = logits.masked_fill(logits < -1e9, -7e4)
+                temps = temps * 1e4
+        if "zeros" in mode and mode != "zeros":
+            signs = torch.randint(0, 2, (n, vocab), generator=g).float() * 2 - 1
+            some = torch.rand(n, vocab, generator=g) < 0.6
+            logits = torch.where(some | (mode == "all_zeros"), signs * 0.0, logits)
+            logits[:, 5] = 1e-6  # a positive number closer to 0 than the bins go
+        if mode == "deep":
+            logits = logits - 150.0
+        if mode == "no_mass":
+            top_p = torch.tensor([0.0, 0.0, -1.0, 1e-9] * 2)
         logits = logits.to(torch.bfloat16)
         seeds = torch.randint(0, 1 << 31, (n,), generator=g)
         out = torch.empty(n, dtype=torch.int64, device=dev)
@@ -891,13 +910,14 @@ class TestSampling:
             h = h ^ (h >> shift)
         u = ((h.float() + 1.0) * 2.3283064e-10).clamp(max=1 - 2.0**-24)
         x = logits.double() / temps[:, None].double()
+        x[(logits == 0) & logits.signbit()] = -1e-300  # limits put -0 below 0
         score = x - torch.log(-torch.log(u.double()))
         for r in range(n):
             vals, order = x[r].sort(descending=True)
             least = torch.tensor([float("-inf")], dtype=torch.float64)
             if 0 < top_k[r] < vocab:
                 least = vals[top_k[r] - 1 : top_k[r]]
-            if top_p[r] < 1:
+            if 0 < top_p[r] < 1:
                 c = torch.softmax(x[r], 0)[order].cumsum(0)
                 # either side of the limit where the sum meets it within its rounding
                 at = [int((c < float(top_p[r]) * f).sum()) for f in (1 - 1e-6, 1 + 1e-6)]
