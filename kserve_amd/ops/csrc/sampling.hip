@@ -868,18 +868,24 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
   block_argmax<RT>(best, best_idx, out + s);
 }
 
-// 1024 threads for rows past 64k elements (256 rows of 128256, greedy 24.7 ->
-// 12.3 us, with noise 36.5 -> 26.2); shorter rows are over before a block that
-// size has merged its waves (256 x 32000, greedy: 5.9 us with 256 threads, 7.0
-// with 1024; with noise 10.5 with 256 threads that evaluate every element, 11.9
-// with 512 and the bound)
-// Rows that fill 1024 threads a few times over take as many: a row's time is the
-// latency of its loads one after the other (1 / 96 rows of 32000 5.6 / 8.7 -> 4.7 / 5.8
-// us; noise for every element keeps 256 busy up to 65536).
+// 256 threads, or 1024: a row's time is the latency of its loads one after the
+// other, which more threads shorten, but a block of 1024 merges its waves for longer
+// and two fit a compute unit. Rows of more than 65536 take 1024 (256 x 128256, greedy
+// 24.7 -> 12.7 us, with noise 36.5 -> 25.8). Shorter ones with noise stay with 256, which
+// evaluate every element (256 x 32000 10.5 us, 11.9 with 512 and the bound). Greedy ones
+// take 1024 as long as the rows come to one or two a unit (us with 256 / 1024: 1, 256
+// rows of 18000 4.2 / 4.1, 4.7 / 4.8, of 32000 5.4 / 4.6, 6.1 / 5.3; 300, 512 rows of 28000
+// 5.8 / 6.2, 7.8 / 6.8, of 32000 8.6 / 6.9, 9.0 / 7.5; 1024 rows of 32000 12.2 / 14.1; 256 rows
+// of 14000 4.3 / 4.6).
+bool wide_argmax(bool noise, int num_seqs, int vocab) {
+  if (vocab > 65536) return true;
+  return !noise && num_seqs <= 512 && vocab > (num_seqs <= 256 ? 18000 : 30000);
+}
+
 template <bool GUMBEL>
 void launch_argmax(void* out, const void* logits, const void* temperatures,
                    const void* seeds, int num_seqs, int vocab, hipStream_t stream) {
-  if (vocab > (GUMBEL ? 65536 : 8192))
+  if (wide_argmax(GUMBEL, num_seqs, vocab))
     hipLaunchKernelGGL((argmax_kernel<GUMBEL, 1024>), dim3(num_seqs), dim3(1024), 0,
                        stream, (long*)out, (const short*)logits,
                        (const float*)temperatures, (const long*)seeds, vocab);

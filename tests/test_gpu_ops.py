@@ -666,6 +666,19 @@ class TestSampling:
         ref = logits.float().argmax(dim=-1).cpu()
         assert (got.cpu() == ref).all()
 
+    @pytest.mark.parametrize(
+        "rows,vocab", [(256, 18000), (256, 18001), (257, 18008), (257, 30001), (513, 30008)]
+    )
+    def test_greedy_by_either_block(self, dev, rows, vocab):
+        """Rows on both sides of the rule for the block's size; ties to the first."""
+        from kserve_amd import ops
+
+        g = torch.Generator().manual_seed(vocab)
+        logits = torch.randn(rows, vocab, generator=g).clamp(max=3.0).to(torch.bfloat16)
+        got = ops.greedy_sample(logits.to(dev)).cpu()
+        want = (logits == logits.max(1, keepdim=True).values).int().argmax(1)
+        assert torch.equal(got, want)
+
     def test_gumbel_distribution(self, dev):
         """Gumbel-max sampling matches softmax probabilities statistically."""
         import kserve_amd_C
