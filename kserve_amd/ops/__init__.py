@@ -285,15 +285,37 @@ def random_sample(
     )
 
 
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def _direct(x: torch.Tensor) -> bool:
+    """Whether a kernel may take a torch call's place: nothing records the calls
+    (fx, jit, compile), intercepts them (modes) or transforms them (functorch,
+    forward-mode gradients)."""
+    return (
+        type(x) in _TENSORS
+        and not torch.compiler.is_compiling()
+        and torch._C._get_tracing_state() is None
+        and torch._C._len_torch_dispatch_stack() == 0
+        and torch._C._len_torch_function_stack() == 0
+        and torch._C._functorch.peek_interpreter_stack() is None
+        and torch.autograd.forward_ad._current_level < 0
+    )
+
+
 def _skinny_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
     n = x.shape[0]
     # (above 64 rows: 32-bit offsets within a tile; the rules bound K)
-    return (n <= 64 or n <= 256 and x.stride(0) < 1 << 22) and _plain_operands(x, weight)
+    return (
+        (n <= 64 or n <= 256 and x.stride(0) < 1 << 22)
+        and _direct(x)
+        and _plain_operands(x, weight)
+    )
 
 
 def _plain_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """What the GEMM kernels read directly: plain bf16 matrices on one GPU with
-    16-byte aligned rows, outside autograd and its transforms."""
+    16-byte aligned rows, without gradients."""
     return (
         _C is not None
         and x.is_cuda
@@ -309,11 +331,7 @@ def _plain_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
         and x.stride(1) == 1
         and x.stride(0) % 8 == 0
         and weight.is_contiguous()
-        and type(x) in (torch.Tensor, torch.nn.Parameter)
-        and type(weight) in (torch.Tensor, torch.nn.Parameter)
-        and not torch._C._functorch.is_functorch_wrapped_tensor(x)
-        and not torch._C._functorch.is_functorch_wrapped_tensor(weight)
-        and torch.autograd.forward_ad._current_level < 0
+        and type(weight) in _TENSORS
         and not (
             torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad)
         )
@@ -409,18 +427,18 @@ def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
     m = weight.shape[0]
     if not (
         bias is not None
+        and _direct(x)
         and x.dim() == 2
         and _dense_rows(x.shape[0], x.shape[1], m, gelu)
         and _plain_operands(x, weight)
         and x.shape[0] < 1 << 30
         and x.shape[1] <= x.stride(0) < 1 << 22
-        and type(bias) in (torch.Tensor, torch.nn.Parameter)
+        and type(bias) in _TENSORS
         and bias.shape == (m,)
         and bias.dtype == torch.bfloat16
         and bias.device == x.device
         and bias.is_contiguous()
         and bias.data_ptr() % 16 == 0
-        and not torch._C._functorch.is_functorch_wrapped_tensor(bias)
         and not (torch.is_grad_enabled() and bias.requires_grad)
         and not torch.is_autocast_enabled("cuda")
     ):
@@ -441,6 +459,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     # sizes first: most calls that are not for the kernel end there
     if (
         bias is None
+        and type(x) in _TENSORS
         and x.dim() == 2
         and _skinny_rows(x.shape[0], x.shape[1], weight.shape[0])
         and _skinny_operands(x, weight)

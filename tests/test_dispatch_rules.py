@@ -113,3 +113,53 @@ def test_encoder_product_on_cpu_is_the_librarys():
     assert x3.grad is not None
     z = torch.vmap(lambda v: ops.linear(v, w, b))(torch.randn(3, 5, 64))
     assert z.shape == (3, 5, 16)
+
+
+def _recorded(how, f, x):
+    """(calls that the recording holds, its replay on x)"""
+    if how == "fx":
+        g = torch.fx.symbolic_trace(f)
+    elif how == "make_fx":
+        g = torch.fx.experimental.proxy_tensor.make_fx(f)(x)
+    elif how == "jit":
+        g = torch.jit.trace(f, x, check_trace=False)
+        return [n.kind() for n in g.graph.nodes()], g(x)
+    elif how == "compile":
+        seen = []
+
+        def backend(gm, _):
+            seen.append(gm)
+            return gm
+
+        y = torch.compile(f, backend=backend, fullgraph=True)(x)
+        return [str(n.target) for n in seen[0].graph.nodes], y
+    elif how == "function_mode":
+        names = []
+
+        class Mode(torch.overrides.TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                names.append(func.__name__)
+                return func(*args, **(kwargs or {}))
+
+        with Mode():
+            y = f(x)
+        return names, y
+    return [str(n.target) for n in g.graph.nodes], g(x)
+
+
+@pytest.mark.parametrize("how", ["fx", "make_fx", "jit", "compile", "function_mode"])
+@pytest.mark.parametrize(
+    "dev,dtype",
+    [("cpu", torch.float32), pytest.param("cuda", torch.bfloat16, marks=pytest.mark.gpu)],
+)
+def test_products_are_recorded(how, dev, dtype):
+    """A recorded or intercepted call of `linear` is torch's, also at sizes that a
+    kernel would take."""
+    torch.manual_seed(0)
+    x, w = torch.randn(5, 64, dtype=dtype, device=dev), torch.randn(16, 64, dtype=dtype, device=dev)
+    b = torch.randn(16, dtype=dtype, device=dev)
+    y = torch.nn.functional.linear(x, w)
+    for bias, want in ((b, torch.nn.functional.linear(x, w, b)), (None, y)):
+        names, got = _recorded(how, lambda v: ops.linear(v, w, bias), x)
+        assert any(k in n for n in names for k in ("linear", "mm")), names
+        assert torch.equal(got, want)
