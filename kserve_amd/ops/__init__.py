@@ -401,24 +401,37 @@ def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
 
 def _dense_rows(n: int, k: int, m: int, gelu: bool) -> bool:
     """Whether the encoder kernel beats the library at [n, k] x [m, k]^T + bias
-    (MI355X, us, kernel / library). Up to k 768 with gelu always (m 3072 at 200 / 4500 /
-    7864 / 30000 rows 6.8 / 11.3, 36 / 38, 50 / 69, 211 / 230). Without, on small
-    products (m 768 at 100 / 2000 / 7000 rows 4.8 / 5.1, 7.6 / 9.9, 12.9 / 15.4; m 2304 at
-    1200 / 3200 rows 10.5 / 10.9, 16.9 / 17.8) and again where the library's choice of
-    tile turns (m 2304 at 3700 / 7000 rows 20.8 / 19.7, 31 / 26, but at 7864 / 10000 /
-    12000 33 / 63, 40 / 54, 51 / 61). At k 1024 while the rows leave the library short
-    of tiles (m 1024 at 1000 / 3500 rows 6.7 / 9.4, 11.6 / 12.8, with gelu m 4096 at 2500
-    30 / 35; m 1024 at 16384 rows 43 / 30). Up to k 3072 where one round of the smallest
-    tiles holds the product (m 768 at 350 / 1200 rows 12.4 / 12.5, 12.9 / 15.1; at 100
-    rows 11.7 / 8.4, which the shorter call's 14 us of host time outweigh); past that
-    the library's larger tiles win (m 768 at 2000 / 3200 rows 19.8 / 18.6, 29 / 25)."""
+    (MI355X, us, kernel / library).
+
+    Where one round of the smallest tiles holds the product it does to k 2048, from
+    one row on (weights not in cache; k 768, m 2304 at 1 / 16 / 64 / 256 rows 4.4 / 7.0,
+    4.6 / 5.2, 5.0 / 7.2, 5.5 / 7.5; k 1024, m 4096 6.8 / 9.3, 7.0 / 7.6, 7.7 / 11.7, 8.3 /
+    12.1; k 2048, m 2560 10.5 / 13.1, 10.8 / 11.4, 12.2 / 12.1, 12.3 / 13.3; m 128 the worst,
+    k 1536 at 16 / 64 rows 6.1 / 5.5, 6.6 / 5.8). Beyond, the library's splits of K win
+    (k 3072, m 768 at 1 / 64 / 128 / 512 rows 13.5 / 13.5, 16.5 / 11.8, 16.0 / 9.8, 17.0 / 15.3),
+    but its call takes 10 us more of the host: `_dense` lets it have these in
+    captured graphs only.
+
+    Past one round, with gelu, up to k 768 always (m 3072 at 200 / 4500 / 7864 / 30000
+    rows 6.8 / 11.3, 36 / 38, 50 / 69, 211 / 230). Without, the library's choice of tile
+    turns from one size to the next, so that the line is where it is not ahead for
+    long (m 512 to 3072, n to 30000): on small products (m 768 at 2048 / 7000 rows 7.6 /
+    9.3, 11.7 / 14.2, m 2304 at 3200 16.9 / 17.8, m 2048 at 2048 / 3072 10.2 / 11.3, 16.0 / 13.9)
+    and on some that give this kernel a few full rounds (m 2304 at 7864 / 10000 rows 33 /
+    63, 38 / 51, but at 7000 29 / 24, at 12288 47 / 42, at 20000 78 / 69; m 3072 at 7000 38 / 37;
+    k 512 throughout, m 2304 at 7000 / 12288 / 30000 22 / 22, 35 / 62, 86 / 109). Not on wide
+    ones (m 4096 at 1536 / 8192 rows 24 / 14, 63 / 44, at k 512 17 / 13, 45 / 39). At k 1024
+    while the rows leave the library short of tiles (m 1024 at 1000 / 3500 rows 6.7 / 9.4,
+    11.6 / 12.8, with gelu m 4096 at 2500 30 / 35; m 1024 at 16384 rows 43 / 30)."""
     if m % 8 or not 8 <= m <= 4096 or k > 3072:
         return False
     if -(-n // 64) * -(-m // 64) <= 256:
         return True
     work = n * m * k  # multiply-adds
     if k <= 768:
-        return gelu or work <= 5.8e9 or work >= 13.1e9
+        return gelu or m <= 3072 and (
+            work <= 5.8e9 or work >= 13.1e9 and (k <= 512 or work <= 20e9)
+        )
     return k <= 1024 and n <= 3584 and (gelu or work <= 5.8e9)
 
 
@@ -441,6 +454,8 @@ def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
         and bias.data_ptr() % 16 == 0
         and not (torch.is_grad_enabled() and bias.requires_grad)
         and not torch.is_autocast_enabled("cuda")
+        # (host time is nothing there, and the library's kernel the faster one)
+        and (x.shape[1] <= 2048 or not torch.cuda.is_current_stream_capturing())
     ):
         return None
     out = torch.empty((x.shape[0], m), dtype=x.dtype, device=x.device)

@@ -95,6 +95,9 @@ def test_scan_apart(lens, heads, P, apart):
         (16384, 1024, 1024, False, False),                                 # 43 / 30
         (1344, 3072, 768, False, True), (1345, 3072, 768, False, False),
         (64, 3136, 768, False, False), (64, 768, 30522, False, False),
+        (1, 2048, 2560, False, True), (1536, 768, 4096, False, False),     # 24 / 14
+        (8192, 768, 4096, False, False), (8192, 768, 4096, True, True),    # 63 / 44
+        (12288, 768, 2304, False, False), (12288, 512, 2304, False, True),
         (64, 768, 4, False, False), (64, 768, 4104, False, False),
     ],
 )

@@ -1208,6 +1208,34 @@ class TestDenseGemm:
         xg = x.clone().requires_grad_()
         assert ops.linear(xg, w, b).requires_grad
 
+    @pytest.mark.parametrize("K,own", [(2048, True), (2560, False)])
+    def test_captured_products(self, dev, K, own):
+        """A captured graph keeps the long K of few rows with the library, whose
+        kernel is the faster one there; eager calls, where host time counts, do not."""
+        from kserve_amd import ops
+        import kserve_amd_C
+
+        torch.manual_seed(K)
+        x = torch.randn(64, K, device=dev, dtype=torch.bfloat16)
+        w = (torch.randn(768, K, device=dev) * K**-0.5).to(torch.bfloat16)
+        b = torch.randn(768, device=dev, dtype=torch.bfloat16)
+        eager, kernel = ops.linear(x, w, b), torch.empty(64, 768, device=dev, dtype=torch.bfloat16)
+        kernel_gelu, library = torch.empty_like(kernel), torch.nn.functional.linear(x, w, b)
+        kserve_amd_C.dense_gemm(kernel, x, w, b, False)
+        kserve_amd_C.dense_gemm(kernel_gelu, x, w, b, True)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            got, got_gelu = ops.linear(x, w, b), ops.linear_gelu(x, w, b)
+        for _ in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(eager, kernel)
+            assert torch.equal(got, kernel if own else library)
+            assert torch.equal(got_gelu, kernel_gelu if own else ops.gelu(library))
+            got.zero_()
+            got_gelu.zero_()
+
     def test_gelu_tails(self, dev):
         """gelu alone: the product passes x through one column of ones."""
         import kserve_amd_C
