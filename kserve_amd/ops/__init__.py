@@ -881,22 +881,39 @@ def _scan_in_chunks(
     return max(rounds * chunk * (1 + 0.75 * (chunks - 1)), last) < walk
 
 
-def _scan_chunks_apart(tokens: int, seqs: int, longest: int, heads: int, P: int) -> bool:
+def _scan_chunks_apart(
+    tokens: int, seqs: int, longest: int, heads: int, P: int, N: int = 128
+) -> bool:
     """Whether the scan in chunks forms what needs no state in a launch of its own.
-    Both times are estimated, in us, for 64 heads of 64 columns and 128 states: one
-    launch pays every chunk its chain of barriers, a block a compute unit; two pay the
-    launch and run two blocks a unit, or smaller ones on units that would be idle.
-    (One / two launches: 1 x 64 tokens 12.7 / 15.1, 1 x 100 21.8 / 18.0, 2 x 100 22.4
-    / 23.4, 4 x 200 46.0 / 46.2, 8 x 128 52.9 / 50.3, 6 x 130 64.7 / 53.1, 32 x 64 104 /
-    97, 32 x 100 180 / 149, 40 + 300 49.2 / 36.7.)"""
+    Both times are estimated, in us, fitted over 8 to 128 heads, P 32 to 128, N 16 to
+    128 and 1 to 104 portions of 1 to 4000 tokens (off by 8 % at the mean): one launch
+    pays every chunk its chain of barriers, a block a compute unit; two pay the launch,
+    what it writes for every chunk and head, and a chain that is shorter, more so the
+    more states there are, two blocks a unit or smaller ones on units that would be
+    idle. (One / two launches, 64 heads of 64 columns, 128 states: 1 x 64 tokens 12.7 /
+    15.1, 1 x 100 21.8 / 18.0, 2 x 100 25.3 / 26.6, 4 x 200 46.0 / 46.2, 6 x 130 64.7 / 53.1,
+    32 x 100 180 / 149, 40 + 300 49.2 / 36.7; 16 states: 1 x 100 14.7 / 16.5, 16 x 100 51.8 /
+    58.2, 4 x 500 50.6 / 55.6; 24 heads of 128 columns, 32 states, 4 x 130 20.8 / 29.3.)"""
     if seqs == 0:
         return False
-    blocks = -(-P // 64) * heads * seqs
     most = -(-max(longest, -(-tokens // seqs)) // 64)  # chunks
     average = min(most, tokens / seqs / 64 + 0.5)
-    one = 4 + 0.0133 * blocks + 9.3 * max(most, average * -(-blocks // 256))
-    a_chunk = max(1.5 + 0.0245 * blocks, 0.031 * blocks)
-    return 14 + 0.012 * blocks + max(3.1 * most, average * a_chunk) < one
+    blocks = -(-P // 64) * heads * seqs
+    a_chunk = 4.8 if N <= 32 else 6.5 if N <= 64 else 9.6
+    one = 4.6 + 0.011 * blocks + a_chunk * max(most, average * -(-blocks // 256))
+
+    # blocks of 32 columns or of 16, as the launcher has them
+    narrow = P <= 16 or -(-P // 32) * heads * seqs <= 192
+    blocks = -(-P // (16 if narrow else 32)) * heads * seqs
+    if N <= 64:
+        alone, shared, writes = (1.6 if narrow else 3.0), 3.7, 0.0041
+    else:
+        alone, shared, writes = (2.8 if narrow else 4.6), 6.6, 0.0070
+    chain = alone * most
+    if blocks > 256:  # `shared`: a chunk of two wide blocks on one unit
+        chain = max(chain, average * shared * (0.5 if narrow else 1) * blocks / 512)
+    two = 12.7 + 0.0057 * blocks + writes * average * seqs * heads + chain
+    return two < 0.98 * one
 
 
 def ssd_scan(
@@ -915,7 +932,10 @@ def ssd_scan(
             0 if not _scan_in_chunks(
                 xbc.shape[0], slots.numel(), longest, heads, P, state.shape[3]
             )
-            else 1 + _scan_chunks_apart(xbc.shape[0], slots.numel(), longest, heads, P),
+            else 1
+            + _scan_chunks_apart(
+                xbc.shape[0], slots.numel(), longest, heads, P, state.shape[3]
+            ),
         )
         return y
     return torch_ref.ssd_scan(

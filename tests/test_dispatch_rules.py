@@ -85,6 +85,20 @@ def test_scan_apart(lens, heads, P, apart):
 
 
 @pytest.mark.parametrize(
+    "lens,heads,P,N,apart",
+    [
+        ([100], 64, 64, 16, False), ([100] * 16, 64, 64, 16, False),  # 14.7 / 16.5, 51.8 / 58.2 us
+        ([500] * 4, 64, 64, 16, False), ([1000], 64, 64, 16, True),
+        ([130] * 4, 24, 128, 32, False), ([300] * 8, 24, 64, 32, False),
+        ([200] * 4, 128, 64, 32, False), ([64] * 32, 128, 64, 128, True),
+        ([4000], 8, 32, 16, True),
+    ],
+)
+def test_scan_apart_of_other_heads(lens, heads, P, N, apart):
+    assert ops._scan_chunks_apart(sum(lens), len(lens), max(lens), heads, P, N) is apart
+
+
+@pytest.mark.parametrize(
     "n,k,m,gelu,own",
     [
         (1, 768, 768, False, True), (30000, 768, 3072, True, True),
