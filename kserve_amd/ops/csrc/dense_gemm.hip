@@ -340,6 +340,7 @@ extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
 static bool mid_narrow(int M, int K) { return M <= 4096 && K <= 8192; }
 
 extern "C" int ks_mid_takes(int M, int K, int N) {
+  if (K >= 1 << 22) return 0;  // (offsets within a tile of 32 bits)
   return N > 128 || (N > (M < 4096 ? 64 : 96) && mid_narrow(M, K));
 }
 

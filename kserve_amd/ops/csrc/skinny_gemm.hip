@@ -1,7 +1,8 @@
 // Products of few rows with a weight matrix: out[N][M] = x[N][K] w[M][K]^T for
 // N <= 256 tokens (decode batches, short prompts), where reading the weights
-// is what bounds them. The kernel here takes up to 64, and up to 128 of wide
-// weights; the rest goes to the tiles of dense_gemm.hip.
+// is what bounds them. The kernel here takes up to 64 rows, up to 128 of wide
+// weights, gate|up products of any number, and rows or K of 2^22 elements and more;
+// the rest goes to the tiles of dense_gemm.hip.
 //
 // A block takes 64 F features (16 F per wave) and all tokens over a range of
 // K, in steps of 64: each step's weight and token rows come by LDS-direct
@@ -228,7 +229,9 @@ __global__ __launch_bounds__(256) void reduce_splits_kernel(
   else if ((N) <= 48) GO(3, 1, 5)       \
   else if ((N) <= 64) GO(4, 1, 5)       \
   else if ((N) <= 96) GO(6, 2, 5)       \
-  else GO(8, 2, 5)
+  else if ((N) <= 128) GO(8, 2, 5)      \
+  else if ((N) <= 192) GO(12, 2, 4)     \
+  else GO(16, 2, 3)
 
 int feature_tile(int N) { return N <= 64 ? 64 : 128; }
 
@@ -292,7 +295,8 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
   const bool sums = splits > 1 || !out;
   const GemmArgs p{sums ? partial : out, (const short*)x, (const short*)w, M,
                    K, N, xs};
-  if (!glu && ks_mid_takes(M, K, N)) {
+  // (their offsets within a tile are 32 bits wide: longer rows stay here)
+  if (!glu && ks_mid_takes(M, K, N) && xs < 1 << 22) {
     const hipError_t e = ks_mid_gemm(p.out, x, w, M, K, N, xs, splits, sums, stream);
     if (e != hipSuccess) return e;
   } else {
@@ -310,14 +314,7 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
       hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, BF16_OUT>), grid,       \
                          dim3(256), 0, stream, p);                             \
   }
-    if (N <= 128) {
-      FOR_TILE(N, GO)
-    } else if (glu) {
-      if (N <= 192)
-        hipLaunchKernelGGL((skinny_gemm_kernel<12, 2, 4, GLU>), grid, dim3(256), 0, stream, p);
-      else
-        hipLaunchKernelGGL((skinny_gemm_kernel<16, 2, 3, GLU>), grid, dim3(256), 0, stream, p);
-    }
+    FOR_TILE(N, GO)
 #undef GO
     HIP_CHECK_KERNEL();
   }

@@ -1095,6 +1095,26 @@ class TestSkinnyGemmEdges:
         assert ((out.double() - ref).abs() <= off + ref.abs() * 2.0 ** -8).all()
 
     @pytest.mark.parametrize(
+        "N,K,M,stride",
+        [(65, 192, 68, 1 << 22), (129, 192, 68, (1 << 22) + 8), (200, 1 << 22, 4, 0), (70, 1 << 22, 8, 0)],
+    )
+    def test_long_rows(self, dev, N, K, M, stride):
+        """Strides and K past the 32-bit offsets of the tiles for many rows. Whole
+        numbers: the sums are exact, and the output rounds them to bf16."""
+        import kserve_amd_C
+
+        torch.manual_seed(N)
+        stride = stride or K
+        x = torch.empty((N - 1) * stride + K, device=dev, dtype=torch.bfloat16)
+        x = x.as_strided((N, K), (stride, 1))
+        x.copy_(torch.randint(-1, 2, (N, K), device=dev))
+        w = torch.randint(-1, 2, (M, K), device=dev).to(torch.bfloat16)
+        out = torch.full((N, M), float("nan"), device=dev, dtype=torch.bfloat16)
+        kserve_amd_C.skinny_gemm(out, x, w)
+        ref = sum(a.double() @ b.double().t() for a, b in zip(x.split(1 << 18, 1), w.split(1 << 18, 1)))
+        assert ((out.double() - ref).abs() <= ref.abs() * 2.0**-8).all()
+
+    @pytest.mark.parametrize(
         "N,K,M", [(33, 8192, 4096), (48, 8192, 10240), (17, 3584, 18944),
                   (72, 8192, 8192), (5, 28672, 2048), (64, 2112, 768)]
     )
