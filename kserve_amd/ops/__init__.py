@@ -286,6 +286,13 @@ def random_sample(
 
 
 _TENSORS = (torch.Tensor, torch.nn.Parameter)
+# (names of their own: the chains of attributes took a third of the check's 0.9 us)
+_is_compiling = torch.compiler.is_compiling
+_tracing_state = torch._C._get_tracing_state
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_modes = torch._C._len_torch_function_stack
+_transforms = torch._C._functorch.peek_interpreter_stack
+_forward_ad = torch.autograd.forward_ad
 
 
 def _direct(x: torch.Tensor) -> bool:
@@ -294,12 +301,12 @@ def _direct(x: torch.Tensor) -> bool:
     forward-mode gradients)."""
     return (
         type(x) in _TENSORS
-        and not torch.compiler.is_compiling()
-        and torch._C._get_tracing_state() is None
-        and torch._C._len_torch_dispatch_stack() == 0
-        and torch._C._len_torch_function_stack() == 0
-        and torch._C._functorch.peek_interpreter_stack() is None
-        and torch.autograd.forward_ad._current_level < 0
+        and not _is_compiling()
+        and _tracing_state() is None
+        and not _dispatch_modes()
+        and not _function_modes()
+        and _transforms() is None
+        and _forward_ad._current_level < 0
     )
 
 
