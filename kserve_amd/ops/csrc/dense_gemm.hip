@@ -15,9 +15,9 @@
 // 41 us for 34, their 64-byte rows come at two thirds of the rate. The rows of a
 // fragment never share a bank (0 conflicts).
 //
-// us, this / the library (and gelu's kernel): 7864 x 768 to 2304 33 / 63, to 768
-// 13.5 / 15.1, to 3072 with gelu 50 / 68; 1500 rows to 768 7.2 / 8.7, to 3072 with
-// gelu 15.8 / 20.9; 200 rows to 2304 5.8 / 7.9.
+// us, this / the library (and gelu's kernel): 7864 x 768 to 2304 32 / 63, to 768
+// 12.6 / 15.1, to 3072 with gelu 47 / 68; 1500 rows to 768 7.0 / 8.7, to 3072 with
+// gelu 15.2 / 20.9; 200 rows to 2304 5.4 / 7.9.
 #include "common.h"
 #include "mfma_layouts.h"
 
@@ -113,6 +113,20 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
              step * BK * 2);
   };
 
+  const int wn = wave % WN, wm = wave / WN;
+  // This lane's bias, ahead of the ring's loads: in the epilogue each would be waited
+  // for, and with it the stores of the features before, since loads and stores count as
+  // one (us, 7864 rows: 768 to 2304 32.3 -> 31.6, to 3072 with gelu 49.2 -> 47.2, to 768
+  // 13.0 -> 12.6; 200 rows to 2304 5.5 -> 5.4).
+  short8_t bias[FM / 2];
+#pragma unroll
+  for (int f = 0; f < FM; f += 2) {
+    const int feat = m0 + wm * FM * 16 + f * 16 + g * 8;
+    bias[f / 2] = short8_t{};
+    if (EPI != PARTIAL && p.bias && feat < p.M)
+      bias[f / 2] = *reinterpret_cast<const short8_t*>(p.bias + feat);
+  }
+
   f32x4_t acc[FM][FN];
 #pragma unroll
   for (int f = 0; f < FM; ++f)
@@ -121,7 +135,6 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
 
   // fragment rows: tokens in order; features so that a lane's rows of two
   // fragments are 8 consecutive ones, 16 bytes of the output
-  const int wn = wave % WN, wm = wave / WN;
   const int xrow = wn * FN * 16 + col, xkey = (col >> 1) & 7;
   const int frow = TN + wm * FM * 16 + (col >> 2) * 8 + (col & 3);
   const int fkey = ((col >> 1) & 1) | ((col >> 2) << 1);
@@ -207,6 +220,10 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
     slot = slot + 1 == S ? 0 : slot + 1;
     multiply(a1, b1, a0, b0, slot, 0, 0, 0, 0, 0);
   }
+  if constexpr (EPI != PARTIAL) {  // (left to itself the compiler loads it at its use)
+#pragma unroll
+    for (int f = 0; f < FM / 2; ++f) asm volatile("" : "+v"(bias[f]));
+  }
   multiply(a0, b0, a1, b1, slot, 1, 0, 0, 0, 0);
 #pragma unroll
   for (int t = 0; t < FN; ++t)
@@ -228,12 +245,9 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
         if (feat + 4 < p.M) o[1] = acc[f + 1][t];
       }
     } else {
-      float b[8] = {};
-      if (p.bias) {
-        const short8_t bv = *reinterpret_cast<const short8_t*>(p.bias + feat);
+      float b[8];
 #pragma unroll
-        for (int r = 0; r < 8; ++r) b[r] = bf16_bits_to_float(bv[r]);
-      }
+      for (int r = 0; r < 8; ++r) b[r] = bf16_bits_to_float(bias[f / 2][r]);
 #pragma unroll
       for (int t = 0; t < FN; ++t) {
         const int tok = n0 + wn * FN * 16 + t * 16 + col;
