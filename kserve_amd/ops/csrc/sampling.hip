@@ -17,13 +17,18 @@ constexpr unsigned int HASH_STEP = 0x85EBCA77u;
 __device__ __forceinline__ unsigned int hash_start(unsigned int seed) {
   return seed * 0x9E3779B1u + 0x165667B1u;
 }
-__device__ __forceinline__ unsigned int hash_end(unsigned int h) {
+// all but the last step, which leaves the upper 15 bits as they are
+constexpr unsigned int HASH_LOW = 0x1ffffu;
+__device__ __forceinline__ unsigned int hash_upper(unsigned int h) {
   h ^= h >> 15;
   h *= 0x2C1B3C6Du;
   h ^= h >> 12;
   h *= 0x297A2D39u;
-  h ^= h >> 15;
   return h;
+}
+__device__ __forceinline__ unsigned int hash_end(unsigned int h) {
+  h = hash_upper(h);
+  return h ^ (h >> 15);
 }
 
 // One row of bf16 logits walked by a block of NT threads. The row starts at
@@ -87,9 +92,10 @@ struct Bf16Row {
   }
 };
 
-// the block's largest value and its index (ties: the lower index) to out
-template <int NT>
-__device__ __forceinline__ void block_argmax(float best, int best_idx, long* out) {
+// the block's largest value and its index (ties: the lower index), to all threads or
+// the first
+template <int NT, bool ALL>
+__device__ __forceinline__ void block_best(float& best, int& best_idx) {
   __shared__ float s_val[NT / 64];
   __shared__ int s_idx[NT / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -107,10 +113,14 @@ __device__ __forceinline__ void block_argmax(float best, int best_idx, long* out
     s_idx[wave] = best_idx;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < NT / 64; ++w) merge(s_val[w], s_idx[w]);
-    *out = best_idx;
+  if (ALL || threadIdx.x == 0) {
+    for (int w = ALL ? 0 : 1; w < NT / 64; ++w) merge(s_val[w], s_idx[w]);
   }
+}
+template <int NT>
+__device__ __forceinline__ void block_argmax(float best, int best_idx, long* out) {
+  block_best<NT, false>(best, best_idx);
+  if (threadIdx.x == 0) *out = best_idx;
 }
 
 __device__ __forceinline__ float noise_of_hash(unsigned int h) {
@@ -348,12 +358,13 @@ __global__ __launch_bounds__(AM_NT) void argmax_f32_kernel(
 // between 0 and 2^-16 of either sign decide, go through the passes above.
 //
 // The last pass queues a wave's survivors in LDS and evaluates them 64 at a time,
-// so a set of any density costs what it holds.
+// so a set of any density costs what it holds. Of a large one it forms every hash and
+// queues the few whose noise can exceed what some of them nearly surely reach.
 //
 // What bounds it: the first pass runs at memory speed (8 operations an element
 // hide under it), the last at the vector units' and the queue's. Rows of N(0, 2.5)
 // logits, one per compute unit (us, three passes / this): 256 x 128256 top-p 0.9 75
-// / 41, top-k 50 49 / 29, both 52 / 30; 15 x 128256 66 / 34, 40 / 20, 45 / 22; 256 x
+// / 37, top-k 50 49 / 29, both 52 / 30; 15 x 128256 66 / 31, 40 / 20, 45 / 22; 256 x
 // 32000 33 / 20, 23 / 14, 29 / 16; limits below zero 131 / 68 (a histogram by the
 // keys' upper byte took 704 at 256 x 128256). 256 x 128256, top-k 50 of 20 numbers, the
 // rest masked, 306 / 38; half of the row 0, top-p 0.99 212 / 111 (all of it 0: 137 /
@@ -435,6 +446,60 @@ __device__ __forceinline__ void find_bin(F value, T target, T* wave_sum, int* bi
   __syncthreads();
 }
 
+// Elements whose scores can reach the cut (in log2), queued by a whole wave as its
+// vectors pass by. With 1 - u = r / 2^32 the noise is at most ln(2^32 / r), so an
+// element whose r is above 2^32 exp(x / T - cut) cannot. The upper 15 bits of r decide,
+// against the largest x of a lane's eight, and r below 2^17 always passes: beside the
+// hash that is half an operation an element, where GumbelBound takes eight.
+// Margin: u's rounding and the two hardware logarithms are off by 0.031 in log2 at most
+// from r 4096 on; the rest, and the term in the cut, are for the fp32 scores.
+struct CandidateQueue {
+  uint2* queue;
+  int most;  // entries
+  float c2, c0;
+  unsigned int h0;
+  int queued = 0;
+
+  __device__ __forceinline__ CandidateQueue(uint2* q, int n, float c2_, float cut, unsigned int h)
+      : queue(q), most(n), c2(c2_), c0(32.25f + 4e-6f * fabsf(cut) - cut), h0(h) {}
+  __device__ __forceinline__ bool full() const { return queued > most; }
+  __device__ __forceinline__ void add8(const short8_t& v, int i0) {
+    short2_v m = {-32768, -32768};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      m = __builtin_elementwise_max(m, ordered(short2_v{v[2 * q], v[2 * q + 1]}));
+    const float x = ordered_value(max(m.x, m.y));
+    const float t = __builtin_amdgcn_fmed3f(
+        __builtin_amdgcn_exp2f(__builtin_fmaf(x, c2, c0)), 131072.f, 4294967040.f);
+    const unsigned int least = ~((unsigned int)t | HASH_LOW);
+    const unsigned int hi = h0 + (unsigned int)i0 * HASH_STEP;
+    unsigned int h[8], last = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      h[j] = hash_upper(hi + j * HASH_STEP);
+      last = max(last, h[j]);
+    }
+    if (!__ballot(last >= least)) return;
+    unsigned int in = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) in |= (h[j] >= least ? 1u : 0u) << j;
+    for (;;) {  // one of each lane's at a time
+      const unsigned long long set = __ballot(in != 0);
+      if (!set) break;
+      const int j = __builtin_ctz(in | 0x100);
+      short b = v[0];
+#pragma unroll
+      for (int q = 1; q < 8; ++q) b = j == q ? v[q] : b;
+      const int at = __builtin_amdgcn_mbcnt_hi(
+          (unsigned int)(set >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)set, queued));
+      if (in && at < most)
+        queue[at] = uint2{(unsigned int)(i0 + j), (unsigned int)(unsigned short)b << 16};
+      queued += __builtin_popcountll(set);
+      in &= in - 1;
+    }
+  }
+};
+
 __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
     long* __restrict__ out,            // [S]
     const short* __restrict__ logits,  // [S, V] bf16
@@ -473,12 +538,15 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
   __shared__ unsigned int w_cnt[NWV];
   __shared__ u64 w_fix[NWV];
   __shared__ int sh_bin[4];
-  __shared__ unsigned int sh_above_k;
+  __shared__ unsigned int sh_above_k, sh_live;
   __shared__ double sh_above_p;
   __shared__ u64 sh_above_f;
 
   const Bf16Row<RT> row(logits + (long)s * V, V);
   unsigned int thr = 0;
+  // where many survive: how many, and log2 of a score that some of them exceed
+  unsigned int live = 0;
+  float cut = 0.f;
   if (use_k || use_p) {
     // ---- first pass: counts per bin, extremes, mass ----
     for (int i = tid; i < FBINS; i += RT) lds.win[i] = 0;
@@ -589,7 +657,11 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
         }
         __syncthreads();
         // the smaller bin is the higher limit, and what is not found yet lies below
-        if (min(sh_bin[0], sh_bin[1]) != NONE) break;
+        const int found = min(sh_bin[0], sh_bin[1]);
+        if (found != NONE) {
+          if (bin == found) sh_live = ck + n;
+          break;
+        }
       }
       const int bin = min(sh_bin[0], sh_bin[1]);
       // Numbers below -2^16 and -inf have no bin. Where the largest stands 40 / ln 2
@@ -641,6 +713,12 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
           if (!reached(to[0])) thr = reached(to[1]) ? 0x8000u : reached(to[2]) ? 0x7fffu : 0u;
         } else {  // no limit among the bins: all that is in them
           thr = (unsigned int)(bin_ordered(bin == NONE ? FBINS - 1 : bin) + 32768);
+          // with the mass known, elements above its logarithm less 2.5 are Poisson with
+          // a mean of 12
+          if (use_p && bin == sh_bin[1]) {
+            live = sh_live;
+            cut = most * c2 + __builtin_amdgcn_logf((float)want) - 2.5f * 1.44269504f;
+          }
         }
       }
     }
@@ -805,6 +883,40 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
         take(bf16_bits_to_float(b), hash_end(h0 + (unsigned int)i * HASH_STEP), i);
     };
     __syncthreads();  // the counts are read
+    // Where many survive, each element's hash is formed and the few that can exceed the
+    // cut are evaluated; where few do, queueing the survivors costs less (us, queue /
+    // this, 256 rows: 128256 logits, a fifth surviving 41.5 / 37.0, a third 44.1 / 36.9,
+    // 7 % 37.6 / 37.8; 32000 logits 20.6 / 20.0, 21.6 / 19.9, 18.9 / 20.4; 16 x 128256
+    // 35.7 / 31.3, 38.3 / 31.2).
+    if (live > (unsigned int)V / 10) {
+      CandidateQueue could(lds.queue[wave], QUEUE, inv_t * 1.44269504f, cut, h0);
+      row.groups(
+          [&](const short8_t* v, auto count, int i0) {
+            if (could.full()) return;
+#pragma unroll
+            for (int u = 0; u < decltype(count)::value; ++u)
+              could.add8(v[u], i0 + u * RT * 8);
+          },
+          [&](const short8_t& v, int i0) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) take_one(v[j], i0 + j);
+          },
+          take_one);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      for (int at = lane; at < min(could.queued, QUEUE); at += 64) {
+        const uint2 e = lds.queue[wave][at];
+        take_one((short)(e.y >> 16), (int)e.x);
+      }
+      float most = could.full() ? 3e38f : best;
+      int most_idx = best_idx;
+      block_best<RT, true>(most, most_idx);
+      // (not so if a queue ran over or, by chance, nothing exceeds the cut)
+      if (most < 1e38f && most * 1.44269504f >= cut) {
+        if (tid == 0) out[s] = most_idx;
+        return;
+      }
+      __syncthreads();  // block_best is called again
+    }
     uint2* queue = lds.queue[wave];
     int queued = 0;
     auto drain = [&](int from) {  // 64 of the queue, by a whole wave

@@ -943,6 +943,58 @@ class TestSampling:
             near = 1e-4 + 4 * 2.0 ** -24 * float(x[r][got].abs())
             assert s.max() <= score[r][got] + near, (r, got, int(s.argmax()))
 
+    @pytest.mark.parametrize("shape", ["narrow", "equal", "clumps", "half"])
+    @pytest.mark.parametrize("vocab", [528, 8703, 40003, 131080])
+    def test_many_survivors(self, dev, vocab, shape):
+        """Rows of which a tenth and more survives: a score that some of them exceed
+        picks who is evaluated. The first four rows of 528 equal logits draw no
+        noise above it (seeds searched for; one row in 200000) and are walked again."""
+        import kserve_amd_C
+
+        n = 16
+        g = torch.Generator().manual_seed(vocab)
+        logits = torch.randn(n, vocab, generator=g) * 0.3
+        top_p = torch.tensor([0.999, 0.97] * (n // 2))
+        temps = torch.rand(n, generator=g) + 0.5
+        if shape == "equal":
+            logits, top_p, temps = logits * 0 + 1, top_p * 0 + 0.999, temps * 0 + 1
+        if shape == "clumps":  # one large of eight, and none in whole vectors
+            logits[:, ::8] += 6
+            logits[:, 1024:4096] = -30.0
+        if shape == "half":
+            logits[:, vocab // 2:] = float("-inf")
+        logits = logits.to(torch.bfloat16)
+        seeds = torch.randint(0, 1 << 31, (n,), generator=g)
+        seeds[:4] = torch.tensor([64610, 157832, 195058, 774214])
+        out = torch.empty(n, dtype=torch.int64, device=dev)
+        kserve_amd_C.topk_topp_sample(
+            out, logits.to(dev), temps.to(dev), top_p.to(dev),
+            torch.zeros(n, dtype=torch.int32, device=dev), seeds.to(dev),
+        )
+        M = 0xFFFFFFFF
+        h = ((seeds[:, None] * 0x9E3779B1) & M) + ((torch.arange(vocab) * 0x85EBCA77) & M)
+        h = (h + 0x165667B1) & M
+        for mul, shift in ((0x2C1B3C6D, 12), (0x297A2D39, 15)):
+            h = ((h ^ (h >> 15)) * mul & M) if shift == 12 else h * mul & M
+            h = h ^ (h >> shift)
+        u = ((h.float() + 1.0) * 2.3283064e-10).clamp(max=1 - 2.0**-24)
+        x = logits.double() / temps[:, None].double()
+        score = x - torch.log(-torch.log(u.double()))
+        for r in range(n):
+            vals, order = x[r].sort(descending=True)
+            c = torch.softmax(x[r], 0)[order].cumsum(0)
+            # either side of the limit where the sum meets it within its rounding
+            at = [int((c < float(top_p[r]) * f).sum()) for f in (1 - 1e-6, 1 + 1e-6)]
+            hi, lo = (float(vals[min(a, vocab - 1)]) for a in at)
+            if shape != "clumps":
+                assert (x[r] >= hi).sum() > vocab / 10
+            if vocab == 528 and shape == "equal" and r < 4:
+                assert score[r].max() < 1 + math.log(0.999 * vocab) - 2.5
+            got = int(out[r])
+            # (fast fp32 logarithms: 2e-6 of values up to 20)
+            assert x[r][got] >= lo, (r, got)
+            assert score[r][got] >= score[r][x[r] >= hi].max() - 1e-4, (r, got)
+
     @pytest.mark.parametrize("low", [-3e33, -1.5e32])
     @pytest.mark.parametrize("limit", [0, 70002, 70000])
     def test_lowest_rows(self, dev, low, limit):
