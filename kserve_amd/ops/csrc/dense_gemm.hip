@@ -16,8 +16,8 @@
 // fragment never share a bank (0 conflicts).
 //
 // us, this / the library (and gelu's kernel): 7864 x 768 to 2304 32 / 63, to 768
-// 12.6 / 15.1, to 3072 with gelu 47 / 68; 1500 rows to 768 7.0 / 8.7, to 3072 with
-// gelu 15.2 / 20.9; 200 rows to 2304 5.4 / 7.9.
+// 12.6 / 15.1, to 3072 with gelu 44 / 68; 1500 rows to 768 7.0 / 8.7, to 3072 with
+// gelu 14.6 / 20.9; 200 rows to 2304 5.4 / 7.9.
 #include "common.h"
 #include "mfma_layouts.h"
 
@@ -261,7 +261,13 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
         }
         short* to = reinterpret_cast<short*>(p.out) + (long)tok * p.M + feat;
         if (p.M % 8 == 0) {
-          *reinterpret_cast<bf16x8_t*>(to) = o;
+          // (as wide as these are, they are no longer in the L2 when the next product
+          // reads them, and leave it to this one's operands: us, 7864 rows 768 to 3072
+          // 47.2 -> 43.7; without gelu attention and norms lose what this gains)
+          if constexpr (EPI == BIAS_GELU)
+            __builtin_nontemporal_store(o, reinterpret_cast<bf16x8_t*>(to));
+          else
+            *reinterpret_cast<bf16x8_t*>(to) = o;
         } else {  // (M a multiple of 4)
           typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
           *reinterpret_cast<bf16x4_t*>(to) = bf16x4_t{o[0], o[1], o[2], o[3]};
