@@ -183,55 +183,88 @@ __global__ void clamped_swiglu_kernel(T* __restrict__ out,
 }
 
 // 8 bf16 per lane when rows are 8-element aligned
-__global__ void clamped_swiglu_bf16x8_kernel(short* __restrict__ out,
-                                             const short* __restrict__ input,
-                                             const long rows, const int d,
-                                             const float alpha,
-                                             const float limit) {
-  const int nvec = d >> 3;
-  const short8_t* in_vec = reinterpret_cast<const short8_t*>(input);
-  short8_t* out_vec = reinterpret_cast<short8_t*>(out);
-  const long total = rows * nvec;
-  for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total;
-       idx += (long)gridDim.x * blockDim.x) {
-    const long row = idx / nvec;
-    const long col = idx % nvec;
-    const short8_t g8 = in_vec[row * (2 * nvec) + col];
-    const short8_t u8 = in_vec[row * (2 * nvec) + nvec + col];
-    short8_t o;
+// [gate | up] rows of bf16 to f(gate, up), eight at a time. Bound by memory: a block
+// does 256 vectors of a row and ends, so that loads are under way everywhere (blocks
+// that stride over the rows waited for each one's: us, 7931 x 14336 silu 129.5 -> 118.0
+// = 5.8 TB/s, 8000 x 8192 75.0 -> 67.3), and what no cache holds passes them by in both
+// directions (NT; 106.2 = 6.4 TB/s, 62.1. 2000 x 14336 32.4 -> 28.4 by itself, but the
+// next product then reads the result from memory: two prompts of 1000, 4 layers, 4690
+// -> 4709).
+struct SiluMul {
+  __device__ __forceinline__ float operator()(float g, float u) const {
+    return g / (1.f + __expf(-g)) * u;
+  }
+};
+// (the hardware's exponential and reciprocal: 2e-6 of the result, a thousandth of its
+// rounding to bf16; with the library's the vector units bound this, 8000 x 8192 80 us)
+struct ClampedSwiglu {
+  float slope, limit;  // slope: -alpha log2(e)
+  __device__ __forceinline__ float operator()(float g, float u) const {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(slope * g)) * (u + 1.0f);
+  }
+};
+
+template <bool NT, typename F>
+__device__ __forceinline__ void glu8(short8_t* out, const short8_t* gate,
+                                     const short8_t* up, F f) {
+  const short8_t g = NT ? __builtin_nontemporal_load(gate) : *gate;
+  const short8_t u = NT ? __builtin_nontemporal_load(up) : *up;
+  short8_t o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float g = fminf(bf16_bits_to_float(g8[j]), limit);
-      const float u = fminf(fmaxf(bf16_bits_to_float(u8[j]), -limit), limit);
-      o[j] = float_to_bf16_bits(g / (1.0f + expf(-alpha * g)) * (u + 1.0f));
+  for (int j = 0; j < 8; ++j)
+    o[j] = float_to_bf16_bits(f(bf16_bits_to_float(g[j]), bf16_bits_to_float(u[j])));
+  if constexpr (NT) __builtin_nontemporal_store(o, out);
+  else *out = o;
+}
+
+// ROWS: blocks have `per` parts of a row each; else 256 vectors wherever they fall
+template <bool ROWS, bool NT, typename F>
+__global__ __launch_bounds__(256) void glu_bf16x8_kernel(short* __restrict__ out,
+                                                         const short* __restrict__ input,
+                                                         const long rows, const int d,
+                                                         const int per, const F f) {
+  const int nvec = d >> 3;
+  const short8_t* in = reinterpret_cast<const short8_t*>(input);
+  short8_t* to = reinterpret_cast<short8_t*>(out);
+  if constexpr (ROWS) {
+    for (long w = blockIdx.x; w < rows * per; w += gridDim.x) {
+      const long row = w / per;
+      const int c = (int)(w - row * per) * 256 + threadIdx.x;
+      if (c < nvec) {
+        const short8_t* gate = in + row * 2 * nvec + c;
+        glu8<NT>(to + row * nvec + c, gate, gate + nvec, f);
+      }
     }
-    out_vec[idx] = o;
+  } else {
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < rows * nvec; i += gridDim.x * 256L) {
+      const long row = i / nvec;
+      const short8_t* gate = in + row * nvec + i;
+      glu8<NT>(to + i, gate, gate + nvec, f);
+    }
   }
 }
 
-__global__ void silu_and_mul_kernel(short* __restrict__ out,
-                                    const short* __restrict__ input,
-                                    const int rows, const int d) {
-  const int nvec = d >> 3;
-  const short8_t* in_vec = reinterpret_cast<const short8_t*>(input);
-  short8_t* out_vec = reinterpret_cast<short8_t*>(out);
-  const long total = (long)rows * nvec;
-  for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total;
-       idx += (long)gridDim.x * blockDim.x) {
-    const long row = idx / nvec;
-    const long col = idx % nvec;
-    short8_t g = in_vec[row * (2 * nvec) + col];
-    short8_t u = in_vec[row * (2 * nvec) + nvec + col];
-    short8_t o;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float gf = bf16_bits_to_float(g[j]);
-      float uf = bf16_bits_to_float(u[j]);
-      float s = gf / (1.f + __expf(-gf));
-      o[j] = float_to_bf16_bits(s * uf);
-    }
-    out_vec[idx] = o;
-  }
+template <typename F>
+hipError_t launch_glu_bf16x8(void* out, const void* input, long rows, int d, F f,
+                             hipStream_t stream) {
+  const int nvec = d / 8, per = (nvec + 255) / 256;
+  const bool by_rows = nvec >= 1024 || nvec % 256 == 0;  // (few idle lanes)
+  // (what the 256 MB memory-side cache holds of one product is read there by the next)
+  const bool nt = rows * d * 6 > 256L << 20;
+  const long blocks = by_rows ? rows * per : (rows * nvec + 255) / 256;
+  const dim3 grid((unsigned)(blocks < 1 << 30 ? blocks : 1 << 30));
+#define GO(R, N)                                                                       \
+  hipLaunchKernelGGL((glu_bf16x8_kernel<R, N, F>), grid, dim3(256), 0, stream, (short*)out, \
+                     (const short*)input, rows, d, per, f)
+  if (by_rows && nt) GO(true, true);
+  else if (by_rows) GO(true, false);
+  else if (nt) GO(false, true);
+  else GO(false, false);
+#undef GO
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
 }
 
 }  // namespace
@@ -239,14 +272,8 @@ __global__ void silu_and_mul_kernel(short* __restrict__ out,
 extern "C" hipError_t ks_silu_and_mul(void* out, const void* input, int rows,
                                       int d, hipStream_t stream) {
   if (d % 8 != 0) return hipErrorInvalidValue;
-  long total = (long)rows * (d >> 3);
-  if (total == 0) return hipSuccess;
-  int grid = (int)((total + 255) / 256);
-  if (grid > 2048) grid = 2048;  // grid-stride (G11)
-  hipLaunchKernelGGL(silu_and_mul_kernel, dim3(grid), dim3(256), 0, stream,
-                     (short*)out, (const short*)input, rows, d);
-  HIP_CHECK_KERNEL();
-  return hipSuccess;
+  if (rows == 0 || d == 0) return hipSuccess;
+  return launch_glu_bf16x8(out, input, rows, d, SiluMul{}, stream);
 }
 
 extern "C" hipError_t ks_clamped_swiglu(void* out, const void* input, int rows,
@@ -261,14 +288,10 @@ extern "C" hipError_t ks_clamped_swiglu(void* out, const void* input, int rows,
                        stream, (float*)out, (const float*)input, (long)rows, d,
                        alpha, limit);
   else if (d % 8 == 0 && ((uintptr_t)input % 16) == 0 &&
-           ((uintptr_t)out % 16) == 0) {
-    long tv = (long)rows * (d >> 3);
-    int gv = (int)((tv + 255) / 256);
-    if (gv > 8192) gv = 8192;
-    hipLaunchKernelGGL(clamped_swiglu_bf16x8_kernel, dim3(gv), dim3(256), 0,
-                       stream, (short*)out, (const short*)input, (long)rows, d,
-                       alpha, limit);
-  } else
+           ((uintptr_t)out % 16) == 0)
+    return launch_glu_bf16x8(out, input, rows, d, ClampedSwiglu{alpha * -1.44269504f, limit},
+                              stream);
+  else
     hipLaunchKernelGGL(clamped_swiglu_kernel<short>, dim3(grid), dim3(256), 0,
                        stream, (short*)out, (const short*)input, (long)rows, d,
                        alpha, limit);

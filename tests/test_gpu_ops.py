@@ -79,6 +79,30 @@ class TestActivation:
         ref = torch_ref.silu_and_mul(x.float().cpu())
         bf16_close(got, ref)
 
+    @pytest.mark.parametrize("clamped", [False, True])
+    @pytest.mark.parametrize(
+        "rows,d",
+        # vectors anywhere, by rows with a part row, full parts; past the caches each way
+        [(1, 8), (3, 2056), (5, 10248), (7, 8192), (5700, 8000), (3301, 14344)],
+    )
+    def test_glu_parts(self, dev, rows, d, clamped):
+        """Each value within a rounding to bf16 (2^-8) and the fp32 terms (2^-17 at
+        most) of what float64 gives."""
+        from kserve_amd import ops
+
+        g = torch.Generator(device=dev).manual_seed(d)
+        x = torch.randn(rows, 2 * d, device=dev, generator=g).mul_(3).to(torch.bfloat16)
+        got = ops.clamped_swiglu(x, 1.702, 4.0) if clamped else ops.silu_and_mul(x)
+        for r0 in range(0, rows, 1000):
+            gate, up = x[r0 : r0 + 1000].double().chunk(2, 1)
+            if clamped:
+                gate, up = gate.clamp(max=4.0), up.clamp(-4.0, 4.0)
+                ref = gate * torch.sigmoid(1.702 * gate) * (up + 1)
+            else:
+                ref = gate * torch.sigmoid(gate) * up
+            off = (got[r0 : r0 + 1000].double() - ref).abs()
+            assert (off <= ref.abs() * (2**-8 + 2**-17) + 1e-37).all()
+
 
 class TestRope:
     def test_rotary_embedding(self, dev):
