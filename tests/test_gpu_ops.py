@@ -104,6 +104,49 @@ class TestActivation:
             assert (off <= ref.abs() * (2**-8 + 2**-17) + 1e-37).all()
 
 
+class TestNormedQueries:
+    @pytest.mark.parametrize(
+        "heads,kv_heads,d,dv,pad",
+        # one, two and four chunks a thread, part chunks; rows off 16 bytes
+        [(16, 4, 128, 128, 0), (3, 1, 40, 24, 8), (33, 2, 128, 64, 0),
+         (64, 16, 128, 128, 16), (4, 2, 32, 32, 4)],
+    )
+    def test_norm_temp_cache(self, dev, heads, kv_heads, d, dv, pad):
+        """Queries in fp32 and cached rows within a rounding to bf16 of float64; a
+        token without a slot leaves the pages alone."""
+        from kserve_amd import ops
+
+        g = torch.Generator().manual_seed(heads * d)
+        T, a, b = 37, heads * d, heads * d + kv_heads * d
+        rows = torch.randn(T, b + kv_heads * dv + pad, generator=g).to(torch.bfloat16)
+        qw, kw = torch.rand(a, generator=g) + 0.5, torch.rand(b - a, generator=g) + 0.5
+        pos = torch.randint(0, 9000, (T,), generator=g)
+        slots = torch.randperm(64, generator=g)[:T].to(torch.int32)
+        slots[5] = -1
+        kc = torch.zeros(4, kv_heads, 16, d, dtype=torch.bfloat16, device=dev)
+        vc = torch.zeros(4, kv_heads, 16, dv, dtype=torch.bfloat16, device=dev)
+        x = rows.to(dev)
+        q = ops.qk_norm_temp_cache(
+            x[:, :a], x[:, a:b], x[:, b : b + kv_heads * dv], qw.to(dev), kw.to(dev),
+            pos.to(dev), slots.to(dev), kc, vc, 1e-5, 0.1, 1024, heads,
+        )
+        x = rows.double()
+
+        def normed(y, w):
+            return y * torch.rsqrt(y.square().mean(1, keepdim=True) + 1e-5) * w.double()
+
+        want = normed(x[:, :a], qw) * (1 + 0.1 * torch.log((pos + 1) // 1024 + 1.0)[:, None].double())
+        assert ((q.cpu().double() - want).abs() <= 2e-6 * want.abs() + 1e-12).all()
+        k = normed(x[:, a:b], kw).view(T, kv_heads, d)
+        v = x[:, b : b + kv_heads * dv].view(T, kv_heads, dv)
+        wk, wv = torch.zeros(64, kv_heads, d).double(), torch.zeros(64, kv_heads, dv).double()
+        held = slots >= 0
+        wk[slots[held].long()], wv[slots[held].long()] = k[held], v[held]
+        got = kc.cpu().double().transpose(1, 2).reshape(64, kv_heads, d)
+        assert ((got - wk).abs() <= 2**-8 * wk.abs() * 1.001).all()
+        assert torch.equal(vc.cpu().double().transpose(1, 2).reshape(64, kv_heads, dv), wv)
+
+
 class TestRope:
     def test_rotary_embedding(self, dev):
         from kserve_amd import ops
