@@ -135,6 +135,29 @@ __device__ __forceinline__ void st4<short>(short* p, const float* v) {
   *reinterpret_cast<short4_t*>(p) = o;
 }
 
+// embed_scale_sinpos by fours: an angle's sine and cosine are neighbours, and with one element a
+// lane both were formed for each (us, width 2048: 8000 tokens 32.7 -> 18.5, without angles
+// 19.4 -> 15.7, 128 tokens 5.2 -> 2.4, 3.0 -> 2.2).
+template <typename T>
+__global__ __launch_bounds__(NT) void embed_scale_sinpos_vec4_kernel(
+    float* __restrict__ out, const T* __restrict__ table, const long* __restrict__ tokens,
+    const long* __restrict__ positions, const float* __restrict__ inv_freq, float scale,
+    int width) {
+  const long t = blockIdx.x;
+  const int i = (blockIdx.y * NT + threadIdx.x) * 4;
+  if (i >= width) return;
+  float x[4], pe[4] = {0.f, 0.f, 0.f, 0.f};
+  ld4<T>(table + tokens[t] * width + i, x);
+  if (inv_freq) {
+    const float pos = (float)positions[t];
+    sincosf(pos * inv_freq[i >> 1], &pe[0], &pe[1]);
+    sincosf(pos * inv_freq[(i >> 1) + 1], &pe[2], &pe[3]);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = x[j] * scale + pe[j];
+  st4<float>(out + t * width + i, x);
+}
+
 template <typename TD, typename TO>
 __global__ void add_rms_norm_f32res_vec4_kernel(
     float* __restrict__ residual, const TD* __restrict__ d0, long d0_stride,
@@ -817,7 +840,18 @@ extern "C" hipError_t ks_embed_scale_sinpos(void* out, const void* table,
                                             int rows, int width, int is_f32,
                                             hipStream_t stream) {
   if (rows == 0) return hipSuccess;
-  if (is_f32)
+  const bool vec = width % 4 == 0 && ((uintptr_t)out % 16) == 0 &&
+                   ((uintptr_t)table % (is_f32 ? 16 : 8)) == 0;
+  const dim3 grid(rows, cdiv(width, NT * 4));
+  if (vec && is_f32)
+    hipLaunchKernelGGL(embed_scale_sinpos_vec4_kernel<float>, grid, dim3(NT), 0, stream,
+                       (float*)out, (const float*)table, (const long*)tokens,
+                       (const long*)positions, (const float*)inv_freq, scale, width);
+  else if (vec)
+    hipLaunchKernelGGL(embed_scale_sinpos_vec4_kernel<short>, grid, dim3(NT), 0, stream,
+                       (float*)out, (const short*)table, (const long*)tokens,
+                       (const long*)positions, (const float*)inv_freq, scale, width);
+  else if (is_f32)
     hipLaunchKernelGGL(embed_scale_sinpos_kernel<float>, dim3(rows), dim3(NT),
                        0, stream, (float*)out, (const float*)table,
                        (const long*)tokens, (const long*)positions,

@@ -146,6 +146,26 @@ class TestNormedQueries:
         assert ((got - wk).abs() <= 2**-8 * wk.abs() * 1.001).all()
         assert torch.equal(vc.cpu().double().transpose(1, 2).reshape(64, kv_heads, dv), wv)
 
+    @pytest.mark.parametrize("width", [4, 1028, 2048, 2050])
+    @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+    def test_embedding_by_fours(self, dev, width, dtype):
+        """By fours and, off a multiple of four, one by one: angles are fp32 products,
+        so sines carry the rounding of positions up to 8191 (2^-12)."""
+        from kserve_amd import ops
+
+        g = torch.Generator().manual_seed(width)
+        table = torch.randn(50, width, generator=g).to(dtype)
+        tok, pos = torch.randint(0, 50, (70,), generator=g), torch.randint(0, 8192, (70,), generator=g)
+        inv = torch.rand(width // 2, generator=g)
+        for freq in (inv, None):
+            got = ops.embed_scale_sinpos(
+                table.to(dev), tok.to(dev), pos.to(dev), None if freq is None else freq.to(dev), 2.5)
+            want = table[tok].double() * 2.5
+            if freq is not None:
+                ang = pos[:, None].double() * freq.double()
+                want = want + torch.stack([ang.sin(), ang.cos()], 2).flatten(1)
+            assert ((got.cpu().double() - want).abs() <= 2e-6 + (5e-4 if freq is not None else 0)).all()
+
 
 class TestRope:
     def test_rotary_embedding(self, dev):
