@@ -107,8 +107,9 @@ __device__ __forceinline__ void load4<float>(const float* p, float* v) {
 // cache up to there, while the loads of a walk are one after the other and short
 // portions start it anew (with the state update, us, 4 / 16 tokens, 6144
 // channels: 500 tokens 11 / 16, 6000 48 / 48, 8000 75 / 70; 127 sequences of 1
-// and one of 385 23 / 39; 10240 channels, 6000 tokens 103 / 85). Bound by memory:
-// 8000 tokens of 6144 channels 61 us = 4.8 TB/s without the update.
+// and one of 385 23 / 39; 10240 channels, 6000 tokens 103 / 85). Bound by memory and
+// the exact exponential: 8000 tokens of 6144 channels 55 us = 5.3 TB/s without the
+// update (59.5 with one load under way at a time).
 constexpr int CONV_TT = 4, CONV_TT_LONG = 16;
 constexpr long CONV_LONG = 42L << 20;  // tokens x channels
 
@@ -134,38 +135,50 @@ __global__ __launch_bounds__(256) void causal_conv_silu_vec4_kernel(
   const int t_end = min(tokens, t0 + TT);
   float win[TAPS][4];  // inputs of tokens t - hist .. t
   int end = 0;         // first token after the sequence that t is in
-  for (int t = t0; t < t_end; ++t) {
-    if (t == t0 || t >= end) {  // the inputs before t, from the rows or the state
-      const int s = seq_of_token[t];
-      const int first = cu_seqlens[s];
-      end = cu_seqlens[s + 1];
-      const long pos = positions[t];
-      const long slot = slots[s];
+  float ahead[4][4];   // four tokens' loads are under way at a time
+#pragma unroll 1
+  for (int t4 = t0; t4 < t_end; t4 += 4) {
 #pragma unroll
-      for (int back = hist; back > 0; --back) {
-        float* v = win[hist - back];
-        if (pos - back < 0)
-          v[0] = v[1] = v[2] = v[3] = 0.f;
-        else if (t - back >= first)
-          load4<T>(in + (long)(t - back) * in_stride + c, v);
-        else
-          load4<T>(conv_state + (slot * hist + (hist - back + (t - first))) * channels + c, v);
+    for (int u = 0; u < 4; ++u)
+      load4<T>(in + (long)min(t4 + u, t_end - 1) * in_stride + c, ahead[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int t = t4 + u;
+      if (t >= t_end) break;
+      if (t == t0 || t >= end) {  // the inputs before t, from the rows or the state
+        const int s = seq_of_token[t];
+        const int first = cu_seqlens[s];
+        end = cu_seqlens[s + 1];
+        const long pos = positions[t];
+        const long slot = slots[s];
+#pragma unroll
+        for (int back = hist; back > 0; --back) {
+          float* v = win[hist - back];
+          if (pos - back < 0)
+            v[0] = v[1] = v[2] = v[3] = 0.f;
+          else if (t - back >= first)
+            load4<T>(in + (long)(t - back) * in_stride + c, v);
+          else
+            load4<T>(conv_state + (slot * hist + (hist - back + (t - first))) * channels + c,
+                     v);
+        }
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) win[hist][i] = ahead[u][i];
+      float acc[4] = {b4[0], b4[1], b4[2], b4[3]};
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] += wt[i][j] * win[j][i];
+      float4_t o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] = silu ? silu_f(acc[i]) : acc[i];
+      *reinterpret_cast<float4_t*>(out + (long)t * channels + c) = o;
+#pragma unroll
+      for (int j = 0; j < hist; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) win[j][i] = win[j + 1][i];
     }
-    load4<T>(in + (long)t * in_stride + c, win[hist]);
-    float acc[4] = {b4[0], b4[1], b4[2], b4[3]};
-#pragma unroll
-    for (int j = 0; j < TAPS; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] += wt[i][j] * win[j][i];
-    float4_t o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = silu ? silu_f(acc[i]) : acc[i];
-    *reinterpret_cast<float4_t*>(out + (long)t * channels + c) = o;
-#pragma unroll
-    for (int j = 0; j < hist; ++j)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) win[j][i] = win[j + 1][i];
   }
 }
 
