@@ -362,7 +362,10 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     sums do not depend on the rows beside it, and small weights stay here for
     that. The widest stay to 112 rows (k 4096, m 32000 at 64 / 80 / 96 / 112 rows 50 / 51,
     48 / 63, 49 / 53, 55 / 73, m 16384 at 80 / 112 33 / 36, 36 / 38, k 2048, m 32000 at 96
-    rows 27 / 35; but m 16384 22 / 19).
+    rows 27 / 35; but m 16384 22 / 19), and at k 2048 to 128 where their tiles of 128
+    features fill seven eighths of the units' last round (at 128 rows m 32000 30 / 32, in
+    a captured step 41 / 50, m 65536 60 / 71, m 128256 127 / 133; but m 24576 29 / 28, m
+    50304 57 / 54).
     Otherwise it gains above where the
     library does not split K over the chip: k 14336, m 4096 at 128 / 256 rows 34 / 74,
     46 / 62, k 8192, m 2048 at 77 / 256 rows 15 / 21, 21 / 27, k 4096, m 4096 at 128
@@ -374,8 +377,11 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
         return False
     if n <= 48 or (n <= 64 and m <= 8192):
         return True
-    if m >= 16384 and n <= 112:
-        return k % 2048 == 0 and (n <= 64 or k * m >= 60 << 20)
+    if m >= 16384 and n <= 128:
+        if k % 2048 or n > 64 and k * m < 60 << 20:
+            return False
+        tiles = -(-m // 128)
+        return n <= 112 or k <= 2048 and tiles * 8 >= -(-tiles // 256) * 256 * 7
     if 2048 <= m < 4096:
         return 8192 <= k < 1 << 22
     return (

@@ -21,6 +21,8 @@ from kserve_amd import ops
         (64, 4096, 32000, True), (112, 4096, 32000, True), (113, 4096, 32000, False),
         (64, 2048, 16384, True), (65, 2048, 16384, False),   # 22 us, library 19
         (64, 5120, 27648, False),                            # 68 / 55
+        (128, 2048, 32000, True), (128, 2048, 128256, True),  # 30 / 32, 127 / 133
+        (129, 2048, 32000, False), (128, 2048, 24576, False),  # 29 / 28
     ],
 )
 def test_few_row_product(n, k, m, own):
