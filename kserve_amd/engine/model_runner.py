@@ -364,7 +364,7 @@ class ModelRunner:
         return input_ids, pos, meta, sel
 
     def _ensure_decode_buffers(self, n: int, max_blocks: int):
-        """Pinned staging rows for a decode batch (one async H2D per step) as
+        """Pinned staging rows for a decode batch (read by one kernel) as
         (pin, views): the rows' fields as numpy arrays, their page tables just
         wide enough for this batch."""
         rows = max(n, self.config.scheduler.max_num_seqs)
@@ -465,20 +465,20 @@ class ModelRunner:
             block_tables=torch.empty((n, nb), dtype=torch.int32, device=dev),
             context_lens=vector(torch.int32),
         )
-        ops.unpack_decode_rows(
-            self._staged_rows(n), nb, input_ids, pos, meta.context_lens,
-            state_slots, meta.slot_mapping, meta.block_tables,
+        self._unpack_staged(
+            n, nb, input_ids, pos, meta.context_lens, state_slots,
+            meta.slot_mapping, meta.block_tables,
         )
         if self._layout is not None:
             self._decode_layout_meta(meta, n, state_slots)
         return input_ids, pos, meta
 
-    def _staged_rows(self, rows: int) -> torch.Tensor:
-        """The first pinned rows on the device, in one copy."""
-        rows_pin = self._pin[: rows * self._pin_stride]
-        staged = rows_pin.to(self.device, non_blocking=True)
+    def _unpack_staged(self, rows: int, width: int, *buffers) -> None:
+        """The first pinned rows spread over the step's buffers by one kernel,
+        which reads them where they are."""
+        staged = self._pin[: rows * self._pin_stride].view(rows, self._pin_stride)
+        ops.unpack_decode_rows(staged, width, *buffers)
         self._mark_staging()
-        return staged.view(rows, self._pin_stride)
 
     def _decode_layout_meta(self, meta, n: int, state_slots) -> None:
         """Decode is the flat-batch layout with one token per sequence."""
@@ -747,7 +747,7 @@ class ModelRunner:
         return self._graph_buffers["logits"][bucket][:n]
 
     def _stage_graph_inputs(self, bucket: int, batch, block_manager) -> int:
-        """The batch in the graph buffers: one H2D copy, one kernel."""
+        """The batch in the graph buffers: one kernel."""
         n, nb = self._fill_pinned(batch, block_manager)
         if n < bucket:
             # padded rows: write scratch KV to block 0 (reserved), ctx len 1
@@ -755,10 +755,9 @@ class ModelRunner:
             pad.zero_()
             self._pin_np["context_lens"][n:bucket] = 1
         buf = self._graph_buffers
-        ops.unpack_decode_rows(
-            self._staged_rows(bucket), nb, buf["input_ids"], buf["positions"],
-            buf["context_lens"], buf["state_slots"], buf["slots"],
-            buf["block_tables"],
+        self._unpack_staged(
+            bucket, nb, buf["input_ids"], buf["positions"], buf["context_lens"],
+            buf["state_slots"], buf["slots"], buf["block_tables"],
         )
         return n
 

@@ -99,11 +99,14 @@ void unpack_decode_rows(at::Tensor& staged, int64_t width, at::Tensor& ids,
                         at::Tensor& positions, at::Tensor& context_lens,
                         at::Tensor& state_slots, at::Tensor& slots,
                         at::Tensor& tables) {
-  TORCH_CHECK(staged.is_cuda() && staged.scalar_type() == at::kInt &&
-                  staged.dim() == 2 && staged.is_contiguous(),
-              "staged: int32 rows");
-  const c10::Device dev = staged.device();
+  TORCH_CHECK(ids.is_cuda(), "ids: a GPU tensor expected");
+  const c10::Device dev = ids.device();
   const c10::DeviceGuard guard(dev);
+  // rows in pinned host memory are read by the kernel itself
+  TORCH_CHECK((staged.device() == dev || staged.is_pinned()) &&
+                  staged.scalar_type() == at::kInt && staged.dim() == 2 &&
+                  staged.is_contiguous(),
+              "staged: int32 rows");
   const int64_t rows = staged.size(0);
   CHECK_STEP(ids, at::kLong, rows);
   CHECK_STEP(positions, at::kLong, rows);

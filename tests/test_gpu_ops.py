@@ -1607,6 +1607,32 @@ class TestDecodeStep:
             assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
 
 
+    @pytest.mark.parametrize("rows,width", [(1, 1), (5, 255), (256, 129), (3, 2049)])
+    def test_unpack_from_pinned(self, dev, rows, width):
+        """Rows that the kernel reads in pinned host memory, and again after the
+        host has changed them; rows in other host memory are refused."""
+        from kserve_amd import ops
+
+        torch.manual_seed(rows)
+        stride = ops.DECODE_ROW_HEAD + width + width % 2
+        staged = torch.empty(rows, stride, dtype=torch.int32, pin_memory=True)
+
+        def buffers(where):
+            v = lambda dt: torch.zeros(rows, dtype=dt, device=where)  # noqa: E731
+            return [v(torch.int64), v(torch.int64), v(torch.int32), v(torch.int32),
+                    v(torch.int32), torch.zeros(rows, width, dtype=torch.int32, device=where)]
+
+        got, want = buffers(dev), buffers("cpu")
+        for _ in range(3):
+            staged.copy_(torch.randint(0, 1 << 20, (rows, stride), dtype=torch.int32))
+            ops.unpack_decode_rows(staged, width, *got)
+            torch.cuda.synchronize()
+            ops.unpack_decode_rows(staged, width, *want)
+            assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
+        with pytest.raises(RuntimeError):
+            ops.unpack_decode_rows(staged.clone(), width, *got)
+
+
 class TestLayerNormEdges:
     """Rows at the edges of what a wave holds, against fp64: fp32 sums of
     ``hidden`` terms, then one rounding to bf16."""
