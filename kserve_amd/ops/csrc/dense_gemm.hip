@@ -114,19 +114,6 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
   };
 
   const int wn = wave % WN, wm = wave / WN;
-  // This lane's bias, ahead of the ring's loads: in the epilogue each would be waited
-  // for, and with it the stores of the features before, since loads and stores count as
-  // one (us, 7864 rows: 768 to 2304 32.3 -> 31.6, to 3072 with gelu 49.2 -> 47.2, to 768
-  // 13.0 -> 12.6; 200 rows to 2304 5.5 -> 5.4).
-  short8_t bias[FM / 2];
-#pragma unroll
-  for (int f = 0; f < FM; f += 2) {
-    const int feat = m0 + wm * FM * 16 + f * 16 + g * 8;
-    bias[f / 2] = short8_t{};
-    if (EPI != PARTIAL && p.bias && feat < p.M)
-      bias[f / 2] = *reinterpret_cast<const short8_t*>(p.bias + feat);
-  }
-
   f32x4_t acc[FM][FN];
 #pragma unroll
   for (int f = 0; f < FM; ++f)
@@ -220,15 +207,29 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
     slot = slot + 1 == S ? 0 : slot + 1;
     multiply(a1, b1, a0, b0, slot, 0, 0, 0, 0, 0);
   }
-  if constexpr (EPI != PARTIAL) {  // (left to itself the compiler loads it at its use)
+  // This lane's bias, under the last step's products: in the epilogue each would be
+  // waited for, and with it the stores of the features before, since loads and stores
+  // count as one (us, 7864 rows: 768 to 2304 32.4 -> 31.8, to 3072 with gelu 51 -> 46, to
+  // 768 12.8 -> 12.4; 1500 rows with gelu 15.5 -> 14.3). No earlier: the ring's waits
+  // count loads.
+  short8_t bias[FM / 2];
 #pragma unroll
-    for (int f = 0; f < FM / 2; ++f) asm volatile("" : "+v"(bias[f]));
+  for (int f = 0; f < FM; f += 2) {
+    const int feat = m0 + wm * FM * 16 + f * 16 + g * 8;
+    bias[f / 2] = short8_t{};
+    if (EPI != PARTIAL && p.bias && feat < p.M)
+      bias[f / 2] = *reinterpret_cast<const short8_t*>(p.bias + feat);
   }
+  __builtin_amdgcn_sched_barrier(0);
   multiply(a0, b0, a1, b1, slot, 1, 0, 0, 0, 0);
 #pragma unroll
   for (int t = 0; t < FN; ++t)
 #pragma unroll
     for (int f = 0; f < FM; ++f) acc[f][t] = mfma16x16x32(a1[f], b1[t], acc[f][t]);
+  if constexpr (EPI != PARTIAL) {  // (left to itself the compiler loads it at its use)
+#pragma unroll
+    for (int f = 0; f < FM / 2; ++f) asm volatile("" : "+v"(bias[f]));
+  }
 
 #pragma unroll
   for (int f = 0; f < FM; f += 2) {
