@@ -453,9 +453,17 @@ class LlamaForCausalLM(nn.Module):
         meta: AttentionMetadata,
     ) -> torch.Tensor:
         st = comm.get_state()
+        # the first norm comes with the embedding
+        normed = self.is_first_stage and len(self.layers) > 0
         if self.is_first_stage:
-            hidden = self.embed_tokens(input_ids)
             residual = None
+            if normed:
+                first = self.layers[0]
+                residual, hidden = self.embed_tokens(
+                    input_ids, norm=(first.input_layernorm, first.eps)
+                )
+            else:
+                hidden = self.embed_tokens(input_ids)
         else:
             # synchronous pipeline: activations + residual arrive from the
             # previous stage over RCCL p2p (xGMI)
@@ -469,7 +477,7 @@ class LlamaForCausalLM(nn.Module):
         for i, layer in enumerate(self.layers):
             hidden, residual = layer(
                 hidden, residual, positions, self.cos_sin_cache, kv_caches[i], meta,
-                normed=i > 0, next_norm=norms[i],
+                normed=normed or i > 0, next_norm=norms[i],
             )
         if not self.is_last_stage:
             comm.pp_send(hidden)

@@ -66,6 +66,43 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     return torch_ref.rms_norm(x, weight, eps)
 
 
+def embed_rms_norm(
+    ids: torch.Tensor, table: torch.Tensor, weight: torch.Tensor, eps: float
+) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(table[ids], its RMSNorm) for a vector of ids. In one kernel where it may take
+    the place of torch's lookup; there an id outside the table gives rows of NaN."""
+    hidden = table.shape[-1]
+    if (
+        _C is not None
+        and table.is_cuda
+        and ids.dim() == 1
+        and ids.dtype == torch.int64
+        and ids.is_contiguous()
+        and table.dtype == weight.dtype == torch.bfloat16
+        and table.is_contiguous()
+        and weight.is_contiguous()
+        and ids.device == weight.device == table.device
+        and table.shape[0] > 0
+        and hidden % 8 == 0
+        and 8 <= hidden <= 16384  # a row in registers
+        and weight.numel() == hidden
+        and (table.data_ptr() | weight.data_ptr()) % 16 == 0
+        and type(table) in _TENSORS
+        and _direct(ids)
+        and not (
+            torch.is_grad_enabled() and (table.requires_grad or weight.requires_grad)
+        )
+    ):
+        residual = torch.empty(
+            (ids.shape[0], hidden), dtype=table.dtype, device=table.device
+        )
+        out = torch.empty_like(residual)
+        _C.embed_rms_norm(residual, out, table, ids, weight, eps)
+        return residual, out
+    residual = torch.nn.functional.embedding(ids, table)
+    return residual, rms_norm(residual, weight, eps)
+
+
 def fused_add_rms_norm(
     x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, eps: float
 ) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -6,6 +6,8 @@
 extern "C" {
 hipError_t ks_rms_norm(void*, const void*, const void*, float, int, int,
                        hipStream_t);
+hipError_t ks_embed_rms_norm(void*, void*, const void*, const void*, const void*, float,
+                             int, int, long, hipStream_t);
 hipError_t ks_fused_add_rms_norm(void*, void*, const void*, float, int, int,
                                  hipStream_t);
 hipError_t ks_silu_and_mul(void*, const void*, int, int, hipStream_t);
@@ -85,6 +87,30 @@ void rms_norm(at::Tensor& out, at::Tensor& input, at::Tensor& weight,
   check_hip(ks_rms_norm(out.data_ptr(), input.data_ptr(), weight.data_ptr(),
                         (float)eps, rows, hidden, current_stream()),
             "rms_norm");
+}
+
+void embed_rms_norm(at::Tensor& residual, at::Tensor& out, at::Tensor& table,
+                    at::Tensor& ids, at::Tensor& weight, double eps) {
+  CHECK_BF16_CONTIG(residual);
+  CHECK_BF16_CONTIG(out);
+  CHECK_BF16_CONTIG(table);
+  CHECK_BF16_CONTIG(weight);
+  TORCH_CHECK(ids.is_cuda() && ids.scalar_type() == at::kLong && ids.is_contiguous(),
+              "ids int64");
+  TORCH_CHECK(table.dim() == 2 && weight.numel() == table.size(1) && out.dim() == 2 &&
+                  out.size(0) == ids.numel() && out.size(1) == table.size(1) &&
+                  residual.sizes() == out.sizes(),
+              "embed_rms_norm: shape mismatch");
+  const c10::Device dev = table.device();
+  TORCH_CHECK(residual.device() == dev && out.device() == dev && ids.device() == dev &&
+                  weight.device() == dev,
+              "operands on different devices");
+  const c10::DeviceGuard guard(dev);
+  check_hip(ks_embed_rms_norm(residual.data_ptr(), out.data_ptr(), table.data_ptr(),
+                              ids.data_ptr(), weight.data_ptr(), (float)eps,
+                              (int)out.size(0), (int)out.size(1), table.size(0),
+                              current_stream()),
+            "embed_rms_norm");
 }
 
 void fused_add_rms_norm(at::Tensor& x, at::Tensor& residual, at::Tensor& weight,
@@ -545,6 +571,7 @@ void mfma_probe(at::Tensor& c, at::Tensor& a, at::Tensor& b) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rms_norm", &rms_norm, "RMSNorm (bf16, CDNA4)");
+  m.def("embed_rms_norm", &embed_rms_norm, "embedding rows and their RMSNorm");
   m.def("fused_add_rms_norm", &fused_add_rms_norm,
         "fused residual-add + RMSNorm, in-place");
   m.def("silu_and_mul", &silu_and_mul, "SwiGLU activation");

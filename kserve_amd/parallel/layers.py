@@ -309,7 +309,13 @@ class VocabParallelEmbedding(nn.Module):
             requires_grad=False,
         )
 
-    def forward(self, ids: torch.Tensor) -> torch.Tensor:
+    def forward(self, ids: torch.Tensor, norm=None):
+        """The tokens' rows; with ``norm`` (weight, eps) their RMSNorm too."""
+        if norm is not None:
+            if self.tp_size == 1:
+                return ops.embed_rms_norm(ids, self.weight, *norm)
+            rows = self.forward(ids)
+            return rows, ops.rms_norm(rows, *norm)
         if self.tp_size == 1:
             return F.embedding(ids, self.weight)
         local = ids - self.vocab_start

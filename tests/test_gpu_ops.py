@@ -1633,6 +1633,36 @@ class TestDecodeStep:
             ops.unpack_decode_rows(staged.clone(), width, *got)
 
 
+class TestEmbeddedNorm:
+    """Embedding rows with their norm in one kernel: the rows as they are and the
+    norm of the kernel that takes them from memory, bit for bit."""
+
+    @pytest.mark.parametrize("hidden", [8, 2040, 2048, 2056, 4096, 4104, 8200, 16384])
+    @pytest.mark.parametrize("rows", [0, 1, 77, 2051])
+    def test_rows(self, dev, hidden, rows):
+        from kserve_amd import ops
+
+        torch.manual_seed(hidden)
+        table = torch.randn(301, hidden, dtype=torch.bfloat16, device=dev)
+        w = torch.randn(hidden, dtype=torch.bfloat16, device=dev)
+        ids = torch.randint(0, 301, (rows,), device=dev)
+        if rows > 1:
+            ids[0], ids[-1] = 300, 0
+        kept, normed = ops.embed_rms_norm(ids, table, w, 1e-5)
+        want = table[ids]
+        assert torch.equal(kept, want)
+        assert torch.equal(normed, ops.rms_norm(want, w, 1e-5) if rows else want)
+
+    def test_outside_the_table(self, dev):
+        from kserve_amd import ops
+
+        table = torch.randn(5, 64, dtype=torch.bfloat16, device=dev)
+        ids = torch.tensor([4, 5, -1, 1 << 40, 0], device=dev)
+        kept, normed = ops.embed_rms_norm(ids, table, table[0].clone(), 1e-5)
+        for got in (kept, normed):
+            assert got[1:4].isnan().all() and not got[[0, 4]].isnan().any()
+
+
 class TestLayerNormEdges:
     """Rows at the edges of what a wave holds, against fp64: fp32 sums of
     ``hidden`` terms, then one rounding to bf16."""
