@@ -656,9 +656,8 @@ class ModelRunner:
                 # greedy sample in-graph; it, its position and its page slot
                 # are the next replay's input, so multi-step windows advance
                 # with zero host involvement
-                sampled = _ops.greedy_sample(logits)
-                _ops.advance_decode(
-                    sampled, buf["input_ids"], buf["positions"],
+                sampled = _ops.greedy_advance(
+                    logits, buf["input_ids"], buf["positions"],
                     buf["context_lens"], buf["slots"], bt, bsz,
                 )
                 return logits, sampled

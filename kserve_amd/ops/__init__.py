@@ -279,6 +279,21 @@ def advance_decode(
     )
 
 
+def greedy_advance(
+    logits: torch.Tensor, ids, positions, context_lens, slots, tables, block: int
+) -> torch.Tensor:
+    """``greedy_sample`` and ``advance_decode`` with its tokens, in one launch."""
+    if logits.is_cuda:
+        out = torch.empty(logits.shape[0], dtype=torch.int64, device=logits.device)
+        _native_sampling("greedy_advance").greedy_advance(
+            out, logits, ids, positions, context_lens, slots, tables, int(block)
+        )
+        return out
+    greedy = greedy_sample(logits)
+    advance_decode(greedy, ids, positions, context_lens, slots, tables, block)
+    return greedy
+
+
 def random_sample(
     logits: torch.Tensor,
     temperatures: torch.Tensor,

@@ -11,6 +11,8 @@
 
 extern "C" {
 hipError_t ks_greedy_sample(void*, const void*, int, int, int, hipStream_t);
+hipError_t ks_greedy_advance(void*, const void*, int, int, int, void*, void*, void*, void*,
+                             const void*, long, int, int, hipStream_t);
 hipError_t ks_gumbel_sample(void*, const void*, const void*, const void*,
                             const void*, int, int, hipStream_t);
 hipError_t ks_topk_topp_sample(void*, const void*, const void*, const void*,
@@ -157,9 +159,34 @@ void advance_decode(at::Tensor& greedy, const c10::optional<at::Tensor>& random,
             "advance_decode");
 }
 
+void greedy_advance(at::Tensor& out, at::Tensor& logits, at::Tensor& ids,
+                    at::Tensor& positions, at::Tensor& context_lens, at::Tensor& slots,
+                    at::Tensor& tables, int64_t block) {
+  const bool f32 = logits.scalar_type() == at::kFloat;
+  TORCH_CHECK((f32 || logits.scalar_type() == at::kBFloat16) && logits.is_cuda() &&
+                  logits.dim() == 2 && logits.is_contiguous() && logits.size(1) > 0,
+              "logits bf16 or fp32 [S, V] on GPU");
+  const c10::Device dev = logits.device();
+  const c10::DeviceGuard guard(dev);
+  const int64_t rows = logits.size(0);
+  CHECK_STEP(out, at::kLong, rows);
+  CHECK_STEP(ids, at::kLong, rows);
+  CHECK_STEP(positions, at::kLong, rows);
+  CHECK_STEP(context_lens, at::kInt, rows);
+  CHECK_STEP(slots, at::kInt, rows);
+  CHECK_TABLES(tables, rows);
+  check_hip(ks_greedy_advance(out.data_ptr(), logits.data_ptr(), rows, logits.size(1),
+                              f32 ? 1 : 0, ids.data_ptr(), positions.data_ptr(),
+                              context_lens.data_ptr(), slots.data_ptr(),
+                              tables.data_ptr(), tables.stride(0), (int)tables.size(1),
+                              (int)block, current_stream()),
+            "greedy_advance");
+}
+
 void def_sampling(pybind11::module_& m) {
   m.def("unpack_decode_rows", &unpack_decode_rows, "staged decode inputs to buffers");
   m.def("advance_decode", &advance_decode, "the next decode step's inputs");
+  m.def("greedy_advance", &greedy_advance, "argmax and the next decode step's inputs");
   m.def("greedy_sample", &greedy_sample, "argmax sampling");
   m.def("gumbel_sample", &gumbel_sample, "Gumbel-max temperature sampling");
   m.def("topk_topp_sample", &topk_topp_sample,

@@ -7,6 +7,7 @@
 // took up to 16 us of a step (us, copied / read in place: 1 row 449.3 / 449.0, 24
 // rows 532.8 / 530.6, 96 1031 / 1015, 256 2312 / 2297).
 #include "common.h"
+#include "decode_step.h"
 
 namespace {
 
@@ -37,21 +38,13 @@ __global__ __launch_bounds__(256) void unpack_decode_rows_kernel(
 __global__ __launch_bounds__(256) void advance_decode_kernel(
     const long* __restrict__ greedy, const long* __restrict__ random,
     const unsigned char* __restrict__ greedy_mask, long* __restrict__ sampled,
-    long* __restrict__ ids, long* __restrict__ positions,
-    int* __restrict__ context_lens, int* __restrict__ slots,
-    long* __restrict__ seeds, const long seed_step, const int* __restrict__ tables,
-    const long table_stride, const int width, const int block, const int rows) {
+    const NextStep next, long* __restrict__ seeds, const long seed_step, const int rows) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= rows) return;
   const long token = random && !greedy_mask[i] ? random[i] : greedy[i];
   if (sampled) sampled[i] = token;
-  ids[i] = token;
-  const long pos = positions[i] + 1;
-  positions[i] = pos;
-  context_lens[i] += 1;
-  // past the table's end (after a window's last step) the slot is not used
-  const long page = min(max(pos / block, 0L), (long)width - 1);
-  slots[i] = tables[i * table_stride + page] * block + (int)(pos % block);
+  const long pos = next.positions[i] + 1;
+  write_next(next, i, token, pos, next_slot(next, i, pos));
   if (seeds) seeds[i] += seed_step;
 }
 
@@ -84,11 +77,12 @@ extern "C" hipError_t ks_advance_decode(const void* greedy, const void* random,
   if (rows < 0 || width < 1 || block < 1 || (random && !greedy_mask))
     return hipErrorInvalidValue;
   if (rows == 0) return hipSuccess;
+  const NextStep next{(long*)ids,         (long*)positions,   (int*)context_lens,
+                      (int*)slots,        (const int*)tables, table_stride, width, block};
   hipLaunchKernelGGL(advance_decode_kernel, dim3((rows + 255) / 256), dim3(256), 0,
                      stream, (const long*)greedy, (const long*)random,
-                     (const unsigned char*)greedy_mask, (long*)sampled, (long*)ids,
-                     (long*)positions, (int*)context_lens, (int*)slots, (long*)seeds,
-                     seed_step, (const int*)tables, table_stride, width, block, rows);
+                     (const unsigned char*)greedy_mask, (long*)sampled, next, (long*)seeds,
+                     seed_step, rows);
   HIP_CHECK_KERNEL();
   return hipSuccess;
 }

@@ -1633,6 +1633,27 @@ class TestDecodeStep:
             ops.unpack_decode_rows(staged.clone(), width, *got)
 
 
+    @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+    @pytest.mark.parametrize("rows,vocab,width", [(1, 32000, 7), (5, 1003, 1), (257, 9000, 130), (0, 64, 2)])
+    def test_greedy_advance(self, dev, dtype, rows, vocab, width):
+        """The token and what it leaves for the next step, against the CPU forms;
+        the last rows stand at their tables' ends."""
+        from kserve_amd import ops
+
+        torch.manual_seed(vocab)
+        logits = torch.randn(rows, vocab).to(dtype)
+        pos = torch.randint(0, width * 16, (rows + 2,))
+        pos[-3:] = width * 16 - 1
+        tables = torch.randint(0, 1 << 20, (rows + 2, width + 3), dtype=torch.int32)[:, :width]
+        outs = []
+        for where in (dev, "cpu"):
+            bufs = [torch.zeros(rows + 2, dtype=torch.int64, device=where), pos.to(where, copy=True)]
+            bufs += [torch.ones(rows + 2, dtype=torch.int32, device=where) for _ in "cs"]
+            got = ops.greedy_advance(logits.to(where), *bufs, tables.to(where), 16)
+            outs.append([got, *bufs])
+        assert all(torch.equal(a.cpu(), b) for a, b in zip(*outs))
+
+
 class TestEmbeddedNorm:
     """Embedding rows with their norm in one kernel: the rows as they are and the
     norm of the kernel that takes them from memory, bit for bit."""
