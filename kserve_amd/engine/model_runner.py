@@ -24,6 +24,8 @@ from kserve_amd.models.llama import AttentionMetadata, LlamaForCausalLM
 
 _DEFAULT_GRAPH_BATCH_SIZES = [1, 2, 4, 8, 16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512, 768, 1024, 1280, 1536, 2048]
 
+_TORCH_INTS = {4: torch.int32, 8: torch.int64}
+
 
 class ModelRunner:
     # event after the last async copies out of the pinned staging buffers
@@ -320,21 +322,15 @@ class ModelRunner:
             cu.append(cu[-1] + n)
             max_seqlen = max(max_seqlen, n)
             last_token_idx.append(cu[-1] - 1)
-        dev = self.device
-        meta = AttentionMetadata(
-            is_prefill=True,
-            slot_mapping=torch.from_numpy(slots).to(dev, non_blocking=True),
-            cu_seqlens=torch.tensor(cu, dtype=torch.int32, device=dev),
-            max_seqlen=max_seqlen,
-        )
+        arrays = [
+            tokens, positions, np.asarray(last_token_idx, dtype=np.int64),
+            slots, np.asarray(cu, dtype=np.int32),
+        ]
         if self._layout is not None:
             counts = np.asarray(batch.num_scheduled_tokens, dtype=np.int64)
-            meta.seq_of_token = torch.from_numpy(
-                np.repeat(np.arange(len(counts), dtype=np.int32), counts)
-            ).to(dev, non_blocking=True)
-            meta.state_slots = torch.tensor(
-                [r.state_slot for r in batch.requests],
-                dtype=torch.int32, device=dev,
+            arrays.append(np.repeat(np.arange(len(counts), dtype=np.int32), counts))
+            arrays.append(
+                np.asarray([r.state_slot for r in batch.requests], dtype=np.int32)
             )
         # chunked-prefill resume: any request with context already in pages
         # must attend to it — switch to the paged-context attention path
@@ -356,12 +352,39 @@ class ModelRunner:
                 t = block_manager.get_block_table(req)
                 btab[i, : nb_per[i]] = t[: nb_per[i]]
                 ctx[i] = req.num_computed_tokens + n
-            meta.block_tables = torch.from_numpy(btab).to(dev, non_blocking=True)
-            meta.context_lens = torch.from_numpy(ctx).to(dev, non_blocking=True)
-        input_ids = torch.from_numpy(tokens).to(dev, non_blocking=True)
-        pos = torch.from_numpy(positions).to(dev, non_blocking=True)
-        sel = torch.tensor(last_token_idx, dtype=torch.int64, device=dev)
+            arrays += [btab, ctx]
+        input_ids, pos, sel, slot_mapping, cu_seqlens, *rest = self._to_device(arrays)
+        meta = AttentionMetadata(
+            is_prefill=True, slot_mapping=slot_mapping, cu_seqlens=cu_seqlens,
+            max_seqlen=max_seqlen,
+        )
+        if self._layout is not None:
+            meta.seq_of_token, meta.state_slots, *rest = rest
+        if rest:
+            meta.block_tables, meta.context_lens = rest
         return input_ids, pos, meta, sel
+
+    def _to_device(self, arrays) -> List[torch.Tensor]:
+        """The arrays on the device. A GPU gets them in one copy out of pinned
+        memory, which nothing waits for: with copies of lists among them the host
+        waited for the step before, and the device for the host (a prompt of 77
+        tokens 627 -> 542 us, as a pageable copy each 554)."""
+        if not self.is_cuda:
+            return [torch.from_numpy(a) for a in arrays]
+        # each where an allocation of its own could be
+        starts, size = [], 0
+        for a in arrays:
+            starts.append(size)
+            size += -(-a.nbytes // 256) * 256
+        staged = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+        rows = staged.numpy()
+        for a, at in zip(arrays, starts):
+            rows[at : at + a.nbytes] = a.reshape(-1).view("uint8")
+        block = staged.to(self.device, non_blocking=True)
+        return [
+            block[at : at + a.nbytes].view(_TORCH_INTS[a.dtype.itemsize]).view(a.shape)
+            for a, at in zip(arrays, starts)
+        ]
 
     def _ensure_decode_buffers(self, n: int, max_blocks: int):
         """Pinned staging rows for a decode batch (read by one kernel) as
@@ -517,14 +540,18 @@ class ModelRunner:
         """Logits of each request's last scheduled token, or of the flat
         token rows in ``logit_rows`` when given."""
         input_ids, positions, meta, sel = self.prepare_prefill(batch, block_manager)
-        if logit_rows is not None:
-            sel = torch.tensor(logit_rows, dtype=torch.int64, device=self.device)
         if self.lora_manager is not None and any(
             r.lora_id for r in batch.requests
         ):
             meta.lora = self._lora_meta(batch, per_request_rows=False)
         hidden = self.model(input_ids, positions, self.kv_caches, meta)
-        return self.model.compute_logits(hidden[sel])
+        if logit_rows is None:
+            rows = hidden.index_select(0, sel)
+        else:
+            rows = hidden[
+                torch.tensor(logit_rows, dtype=torch.int64, device=self.device)
+            ]
+        return self.model.compute_logits(rows)
 
     @torch.no_grad()
     def execute_decode(self, batch, block_manager) -> torch.Tensor:

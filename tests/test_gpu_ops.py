@@ -1684,6 +1684,30 @@ class TestEmbeddedNorm:
             assert got[1:4].isnan().all() and not got[[0, 4]].isnan().any()
 
 
+class TestStagedArrays:
+    @pytest.mark.parametrize("sizes", [[1], [77, 1, 64, 65], [8191, 3, 0, 2]])
+    def test_to_device(self, dev, sizes):
+        """Arrays of both widths in one copy, and again while the first may still
+        be under way."""
+        from types import SimpleNamespace
+
+        import numpy as np
+
+        from kserve_amd.engine.model_runner import ModelRunner
+
+        own = SimpleNamespace(is_cuda=True, device=torch.device(dev))
+        rng = np.random.default_rng(sizes[0])
+        sets = []
+        for _ in range(3):
+            arrays = [rng.integers(-(2 ** 40), 2 ** 40, n) for n in sizes]
+            arrays += [rng.integers(0, 1 << 30, (n, 3)).astype(np.int32) for n in sizes]
+            sets.append((arrays, ModelRunner._to_device(own, arrays)))
+        for arrays, got in sets:
+            for a, t in zip(arrays, got):
+                assert t.is_contiguous() and t.data_ptr() % 256 == 0
+                assert t.cpu().numpy().dtype == a.dtype and (t.cpu().numpy() == a).all()
+
+
 class TestLayerNormEdges:
     """Rows at the edges of what a wave holds, against fp64: fp32 sums of
     ``hidden`` terms, then one rounding to bf16."""
