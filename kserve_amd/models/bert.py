@@ -89,9 +89,16 @@ class BertLayer(nn.Module):
         self.scale = 1.0 / math.sqrt(c.head_dim)
         self.eps = c.layer_norm_eps
 
-    def forward(self, hidden: torch.Tensor, cu_seqlens: torch.Tensor, max_seqlen: int):
+    def project(self, hidden: torch.Tensor) -> torch.Tensor:
+        return ops.linear(hidden, self.qkv_w, self.qkv_b)
+
+    def forward(
+        self, hidden: torch.Tensor, cu_seqlens: torch.Tensor, max_seqlen: int, qkv=None
+    ):
+        """``qkv``: ``project(hidden)``, where it is there already."""
         T = hidden.shape[0]
-        qkv = ops.linear(hidden, self.qkv_w, self.qkv_b)
+        if qkv is None:
+            qkv = self.project(hidden)
         q, k, v = qkv.split(hidden.shape[-1], dim=-1)
         q = q.view(T, self.num_heads, self.head_dim)
         k = k.view(T, self.num_heads, self.head_dim)
@@ -137,14 +144,30 @@ class BertModel(nn.Module):
         cu_seqlens: torch.Tensor,     # [num_seqs + 1] int32
         token_type_ids: Optional[torch.Tensor] = None,
     ) -> torch.Tensor:
-        lens = cu_seqlens[1:] - cu_seqlens[:-1]
         # one transfer for what the host needs to know, behind the embedding
-        stats = torch.stack([lens.max(), lens.min(), lens.sum()])
+        measured = ops.measures_lengths(self.word_embeddings, cu_seqlens)
+        if measured:
+            stats = torch.empty(3, dtype=torch.int64, device=cu_seqlens.device)
+        else:
+            lens = cu_seqlens[1:] - cu_seqlens[:-1]
+            stats = torch.stack([lens.max(), lens.min(), lens.sum()])
         hidden = ops.embed_layer_norm(
             self.word_embeddings, self.position_embeddings,
             self.token_type_embeddings, input_ids, cu_seqlens, token_type_ids,
             self.emb_ln_w, self.emb_ln_b, self.config.layer_norm_eps,
+            stats=stats if measured else None,
         )
+        qkv = None
+        if measured:
+            # the device has the first product to do while the host waits
+            host = torch.empty(3, dtype=torch.int64, pin_memory=True)
+            host.copy_(stats, non_blocking=True)
+            there = torch.cuda.Event()
+            there.record(torch.cuda.current_stream(stats.device))
+            if len(self.layers):
+                qkv = self.layers[0].project(hidden)
+            there.synchronize()
+            stats = host
         max_seqlen, shortest, tokens = stats.tolist()
         if shortest < 0 or tokens != input_ids.shape[0]:
             raise ValueError(
@@ -156,7 +179,8 @@ class BertModel(nn.Module):
                 f"{self.position_embeddings.shape[0]} positions"
             )
         for layer in self.layers:
-            hidden = layer(hidden, cu_seqlens, max_seqlen)
+            hidden = layer(hidden, cu_seqlens, max_seqlen, qkv)
+            qkv = None
         return hidden
 
     def pool(self, hidden: torch.Tensor, cu_seqlens: torch.Tensor) -> torch.Tensor:

@@ -722,11 +722,13 @@ def linear_rope_and_cache(
 
 
 def embed_layer_norm(
-    word, pos_table, type_table, ids, cu_seqlens, types, weight, bias, eps: float
+    word, pos_table, type_table, ids, cu_seqlens, types, weight, bias, eps: float,
+    stats=None,
 ):
     """LayerNorm of word[id] + pos_table[place in its sequence] +
     type_table[type] (``types`` None: type 0) for flat varlen tokens. On the
-    GPU an index outside its table gives a row of NaN."""
+    GPU an index outside its table gives a row of NaN. ``stats`` (int64 [3], where
+    ``measures_lengths``): the longest, the shortest and the sum of the lengths."""
     if word.is_cuda and word.shape[1] <= 2048:  # the kernel's row in registers
         out = torch.empty(
             (ids.numel(), word.shape[1]), dtype=word.dtype, device=word.device
@@ -734,11 +736,23 @@ def embed_layer_norm(
         _native("embed_layer_norm").embed_layer_norm(
             out, word, pos_table, type_table, ids.to(torch.int64).contiguous(),
             None if types is None else types.to(torch.int64).contiguous(),
-            cu_seqlens.to(torch.int32).contiguous(), weight, bias, eps,
+            cu_seqlens.to(torch.int32).contiguous(), weight, bias, eps, stats,
         )
         return out
     return torch_ref.embed_layer_norm(
         word, pos_table, type_table, ids, cu_seqlens, types, weight, bias, eps
+    )
+
+
+def measures_lengths(word, cu_seqlens) -> bool:
+    """Whether ``embed_layer_norm`` can say what the lengths of the sequences are."""
+    return (
+        word.is_cuda
+        and word.shape[1] <= 2048
+        and cu_seqlens.device == word.device
+        and cu_seqlens.dtype == torch.int32
+        and cu_seqlens.dim() == 1
+        and cu_seqlens.shape[0] >= 2
     )
 
 

@@ -38,7 +38,7 @@ hipError_t ks_reshape_and_cache_fp8(const void*, const void*, void*, void*,
 hipError_t ks_embed_layer_norm(void*, const void*, const void*, const void*,
                                const void*, const void*, const void*,
                                const void*, const void*, float, int, int, int,
-                               int, int, int, hipStream_t);
+                               int, int, int, void*, hipStream_t);
 hipError_t ks_layer_norm(void*, const void*, const void*, const void*, float,
                          int, int, hipStream_t);
 hipError_t ks_fused_add_layer_norm(void*, const void*, const void*,
@@ -294,7 +294,8 @@ void embed_layer_norm(at::Tensor& out, at::Tensor& word, at::Tensor& pos_table,
                       at::Tensor& type_table, at::Tensor& ids,
                       const c10::optional<at::Tensor>& types,
                       at::Tensor& cu_seqlens, at::Tensor& weight,
-                      at::Tensor& bias, double eps) {
+                      at::Tensor& bias, double eps,
+                      const c10::optional<at::Tensor>& stats) {
   CHECK_BF16_CONTIG(out);
   CHECK_BF16_CONTIG(word);
   CHECK_BF16_CONTIG(pos_table);
@@ -317,6 +318,10 @@ void embed_layer_norm(at::Tensor& out, at::Tensor& word, at::Tensor& pos_table,
                   weight.numel() == hidden && bias.numel() == hidden,
               "embed_layer_norm: shape mismatch");
   const c10::Device dev = word.device();
+  if (stats)
+    TORCH_CHECK(stats->device() == dev && stats->scalar_type() == at::kLong &&
+                    stats->is_contiguous() && stats->numel() == 3,
+                "stats int64 [3]");
   TORCH_CHECK(out.device() == dev && pos_table.device() == dev &&
                   type_table.device() == dev && ids.device() == dev &&
                   cu_seqlens.device() == dev && weight.device() == dev &&
@@ -330,7 +335,8 @@ void embed_layer_norm(at::Tensor& out, at::Tensor& word, at::Tensor& pos_table,
                 cu_seqlens.data_ptr(), weight.data_ptr(), bias.data_ptr(),
                 (float)eps, (int)tokens, (int)cu_seqlens.numel() - 1, (int)hidden,
                 (int)word.size(0), (int)pos_table.size(0),
-                (int)type_table.size(0), current_stream()),
+                (int)type_table.size(0), stats ? stats->data_ptr() : nullptr,
+                current_stream()),
             "embed_layer_norm");
 }
 
@@ -587,8 +593,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         pybind11::arg("causal") = true, pybind11::arg("window") = 0);
   m.def("context_prefill_varlen", &context_prefill_varlen,
         "MFMA prefill attention against the paged KV cache (chunked prefill)");
+  namespace py = pybind11;
   m.def("embed_layer_norm", &embed_layer_norm,
-        "word + position + type embedding rows and their LayerNorm (bf16)");
+        "token + position + type embeddings and their LayerNorm", py::arg("out"),
+        py::arg("word"), py::arg("pos_table"), py::arg("type_table"), py::arg("ids"),
+        py::arg("types"), py::arg("cu_seqlens"), py::arg("weight"), py::arg("bias"),
+        py::arg("eps"), py::arg("stats") = py::none());
   m.def("layer_norm", &layer_norm, "LayerNorm (bf16)");
   m.def("fused_add_layer_norm", &fused_add_layer_norm,
         "residual-add + LayerNorm");

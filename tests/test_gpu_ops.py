@@ -1708,6 +1708,41 @@ class TestStagedArrays:
                 assert t.cpu().numpy().dtype == a.dtype and (t.cpu().numpy() == a).all()
 
 
+class TestMeasuredLengths:
+    @pytest.mark.parametrize("seqs,tokens", [(1, 0), (1, 5), (63, 200), (64, 200), (65, 200), (1000, 1)])
+    def test_stats(self, dev, seqs, tokens):
+        """What the host is told of the lengths, of sequences in any order."""
+        from kserve_amd import ops
+
+        torch.manual_seed(seqs)
+        cu = torch.randint(-50, 500, (seqs + 1,), dtype=torch.int32)
+        word, vec = [torch.randn(n, 64, dtype=torch.bfloat16, device=dev) for n in (9, 1)]
+        ids = torch.randint(0, 9, (tokens,), device=dev)
+        args = [word, word, word, ids, cu.to(dev), None, vec[0], vec[0], 1e-12]
+        assert ops.measures_lengths(word, args[4])
+        stats = torch.empty(3, dtype=torch.int64, device=dev)
+        got = ops.embed_layer_norm(*args, stats=stats)
+        lens = (cu[1:] - cu[:-1]).long()
+        assert stats.tolist() == [lens.max(), lens.min(), lens.sum()]
+        assert torch.equal(got.nan_to_num(7), ops.embed_layer_norm(*args).nan_to_num(7))
+
+    def test_wrong_lengths_are_refused(self, dev):
+        from kserve_amd.models.bert import BertConfig, BertModel
+
+        c = BertConfig.tiny()
+        model = BertModel(c, dtype=torch.bfloat16, device=dev)
+        for p in model.parameters():
+            p.data.normal_(0, 0.02)
+        ids = torch.randint(0, c.vocab_size, (20,), device=dev)
+        for cu in ([0, 8, 19], [0, 21, 20], [0, 8, 21]):
+            with pytest.raises(ValueError):
+                model(ids, torch.tensor(cu, dtype=torch.int32, device=dev))
+        cu = torch.tensor([0, 8, 20], dtype=torch.int32, device=dev)
+        assert model(ids, cu).isfinite().all()
+        with pytest.raises(RuntimeError):  # (of another type, as ever)
+            model(ids, cu.long())
+
+
 class TestLayerNormEdges:
     """Rows at the edges of what a wave holds, against fp64: fp32 sums of
     ``hidden`` terms, then one rounding to bf16."""
