@@ -444,6 +444,19 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     )
 
 
+def _one_part_rows(n: int, k: int, m: int) -> bool:
+    """Whether 65 to 128 rows go to the few-row product's tiles of 64 features, K in
+    one part, which beat the library and its other tiles where they fill one round of
+    the chip (times at ``mid_wide`` in dense_gemm.hip)."""
+    tiles = -(-m // 64)
+    return (
+        64 < n <= 128
+        and m % 4 == 0
+        and tiles <= 256
+        and (tiles > 128 if 512 <= k <= 2048 else k == 4096 and tiles >= 192)
+    )
+
+
 def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     """The same for the gate|up product with silu(gate) * up on its sums,
     against the library's product and the activation kernel (k 4096, m 14336:
@@ -542,7 +555,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         bias is None
         and type(x) in _TENSORS
         and x.dim() == 2
-        and _skinny_rows(x.shape[0], x.shape[1], weight.shape[0])
+        and (
+            _skinny_rows(x.shape[0], x.shape[1], weight.shape[0])
+            or _one_part_rows(x.shape[0], x.shape[1], weight.shape[0])
+        )
         and _skinny_operands(x, weight)
     ):
         out = torch.empty(

@@ -108,7 +108,16 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
         i < NX ? min(r, p.N - 1 - n0) * p.xs : min(r, p.M - 1 - m0) * p.K;
     at[i] = (row + ((lane & 7) ^ key) * 8) * 2;
   }
+  // Wide products of few rows start their blocks' steps apart, as the few-row kernel
+  // does: rows of W a multiple of 4 KB apart would keep all blocks on the same memory
+  // channels (us at 128 rows of K 2048, M 16384 19.1 -> 18.3, of K 4096 34.7 -> 32.5)
+  constexpr bool APART = TN == 128 && TM == 64 && EPI == BIAS;
+  const int rot = APART ? (int)(blockIdx.x >> 1) % steps : 0;
   auto issue = [&](int step, int slot, int i) {
+    if constexpr (APART) {
+      step += rot;
+      step -= step >= steps ? steps : 0;
+    }
     load_lds(i < NX ? xb : wb, &ring[slot * STAGE + (i * NW + wave) * 8 * BK], at[i],
              step * BK * 2);
   };
@@ -360,12 +369,30 @@ extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
 // long K (K 14336, M 4096 at 77 rows 29.7, 128 x 128 here 34.1).
 static bool mid_narrow(int M, int K) { return M <= 4096 && K <= 8192; }
 
+// Wide products of 65 to 128 rows and K to 4096 in one round of blocks of 64 features
+// and all rows, 8 waves, K in one part. Bound by the reads of W and, per unit, as many
+// of x. us, here / the few-row kernel / the library at 65 and 128 rows, weights not in
+// a cache: K 512, M 10240 6.8 / 11.5 / 10.0, 7.5 / 15.7 / 10.6; K 1024, M 16384 9.7 /
+// 14.3 / 13.8, 11.2 / 18.7 / 14.5; K 2048, M 10304 15.1 / 16.4 / 21.2, 17.7 / 20.8 / 18.1;
+// K 2048, M 16384 16.3 / 19.9 / 18.4, 18.4 / 24.7 / 20.2; K 4096, M 14336 26.8 / 28.4 / 30.0,
+// 31.5 / 35.3 / 33.0. Not at 128 tiles or fewer (K 2048, M 8192 14.2 / 14.5 / 14.0, 16.9 /
+// 18.8 / 15.7), nor where K is long and a quarter of the units idle (K 4096, M 10304
+// 25.6 / 22.9 / 38.4), nor at K between (K 3072, M 16384 at 128 rows 28.6 / 30.8 / 27.0) or
+// longer (K 5120, M 14336 43.6 / 43.1 / 41.7); past 256 tiles a second round is nearly
+// empty (K 2048, M 17408 26.4 / 23.3 / 27.5).
+static bool mid_wide(int M, int K, int N) {
+  const int tiles = (M + 63) / 64;
+  return N > 64 && N <= 128 && tiles <= UNITS &&
+         (K >= 512 && K <= 2048 ? tiles > 128 : K == 4096 && tiles >= 192);
+}
+
 extern "C" int ks_mid_takes(int M, int K, int N) {
   if (K >= 1 << 22) return 0;  // (offsets within a tile of 32 bits)
-  return N > 128 || (N > (M < 4096 ? 64 : 96) && mid_narrow(M, K));
+  return N > 128 || (N > (M < 4096 ? 64 : 96) && mid_narrow(M, K)) || mid_wide(M, K, N);
 }
 
 extern "C" int ks_mid_splits(int M, int K, int N) {
+  if (mid_wide(M, K, N)) return 1;
   const int tm = mid_narrow(M, K) ? 64 : 128;
   const int tiles = (M + tm - 1) / tm * (tm == 64 && N > 128 ? 2 : 1);
   int s = UNITS / (tiles > 0 ? tiles : 1);
@@ -389,9 +416,9 @@ extern "C" hipError_t ks_mid_gemm(void* out, const void* x, const void* w, int M
     hipLaunchKernelGGL((dense_gemm_kernel<tn, tm, wn, wm, s, epi>),                   \
                        dim3(p.tiles, splits), dim3(wn * wm * 64), 0, stream, p);      \
   }
-  if (mid_narrow(M, K)) {
+  if (mid_narrow(M, K) || mid_wide(M, K, N)) {
     if (sums) GO(128, 64, 2, 2, 3, PARTIAL)
-    else GO(128, 64, 2, 2, 3, BIAS)
+    else GO(128, 64, 4, 2, 4, BIAS)
   } else {
     if (sums) GO(256, 128, 4, 2, 3, PARTIAL)
     else GO(256, 128, 4, 2, 3, BIAS)

@@ -32,6 +32,21 @@ def test_few_row_product(n, k, m, own):
 @pytest.mark.parametrize(
     "n,k,m,own",
     [
+        (65, 2048, 16384, True), (128, 2048, 10304, True), (64, 2048, 16384, False),
+        (129, 2048, 16384, False), (65, 512, 8196, True), (65, 448, 10240, False),
+        (65, 2048, 8192, False), (65, 2048, 16388, False),   # 23.3 / 26.4
+        (128, 4096, 12288, True), (128, 4096, 12284, True),  # 192 tiles
+        (128, 4096, 12224, False),                           # 28.6 / 30.3 at 10304
+        (128, 3072, 16384, False), (80, 2048, 10302, False),
+    ],
+)
+def test_one_part_product(n, k, m, own):
+    assert ops._one_part_rows(n, k, m) is own
+
+
+@pytest.mark.parametrize(
+    "n,k,m,own",
+    [
         (1, 4096, 14336, True), (64, 4096, 14336, True), (96, 4096, 14336, True),
         (1, 8192, 14336, True), (1, 8192, 7168, False),  # 56 us, library 50
         (64, 2560, 9728, False), (64, 5120, 13824, False),  # 71 / 62

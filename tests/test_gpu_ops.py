@@ -1525,6 +1525,27 @@ class TestFusedProjections:
         torch.testing.assert_close(out.double(), norm, rtol=2.0 ** -6, atol=2.0 ** -6)
 
 
+class TestOnePartProducts:
+    @pytest.mark.parametrize("K,M", [(512, 8196), (576, 10304), (2048, 8260), (2048, 16384), (4096, 12284)])
+    @pytest.mark.parametrize("N", [65, 97, 128])
+    def test_linear(self, dev, N, K, M):
+        """The first and last widths of the rule, rows of another stride, features and
+        rows that end within a tile; against fp64: fp32 sums of K terms, one rounding."""
+        from kserve_amd import ops
+
+        torch.manual_seed(N + M)
+        assert ops._one_part_rows(N, K, M)
+        x = torch.randn(N, K + 64, device=dev, dtype=torch.bfloat16)[:, :K]
+        w = (torch.randn(M, K, device=dev) * K ** -0.5).to(torch.bfloat16)
+        got = ops.linear(x, w)
+        want = x.double() @ w.double().t()
+        off = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+        assert ((got.double() - want).abs() <= off + 2.0 ** -8 * want.abs()).all()
+        sums = ops._C.skinny_sums(x, w)
+        assert sums.shape == (1, N, M)
+        assert ((sums[0].double() - want).abs() <= off).all()
+
+
 class TestOperandDevices:
     """The entry points that took over from guarded torch calls."""
 
