@@ -290,8 +290,8 @@ class ClampedGLU(nn.Module):
         self.down.copy_(get(prefix + "down").to(dt))
 
     def forward(self, h, parts: bool = False):
-        act = ops.clamped_swiglu(
-            ops.linear(h, self.gate_up), self.ALPHA, self.spec.limit
+        act = ops.linear_clamped_swiglu(
+            h, self.gate_up, self.ALPHA, self.spec.limit
         )
         return (ops.linear_parts if parts else ops.linear)(act, self.down)
 

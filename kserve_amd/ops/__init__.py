@@ -616,6 +616,26 @@ def linear_silu_and_mul(
     return silu_and_mul(linear(x, weight, bias))
 
 
+def linear_clamped_swiglu(
+    x: torch.Tensor, weight: torch.Tensor, alpha: float, limit: float
+) -> torch.Tensor:
+    """``clamped_swiglu`` of [gate | up] = x @ weight^T. Up to 64 rows, where the product
+    of both is the few-row kernel's either way, on its sums in 32 bits."""
+    m = weight.shape[0] // 2
+    if (
+        x.dim() == 2
+        and x.shape[0] <= 64
+        and weight.shape[0] % 2 == 0
+        and _skinny_glu_rows(x.shape[0], x.shape[1], m)
+        and _skinny_rows(x.shape[0], x.shape[1], 2 * m)
+        and _skinny_operands(x, weight)
+    ):
+        out = torch.empty((x.shape[0], m), dtype=x.dtype, device=x.device)
+        _C.skinny_clamped_glu(out, x, weight, float(alpha), float(limit))
+        return out
+    return clamped_swiglu(linear(x, weight), alpha, limit)
+
+
 def linear_add_rms_norm(
     x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor,
     norm_weight: torch.Tensor, eps: float,

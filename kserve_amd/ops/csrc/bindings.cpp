@@ -56,6 +56,8 @@ hipError_t ks_dense_gemm(void*, const void*, const void*, const void*, int, int,
                          long, int, int, hipStream_t);
 hipError_t ks_skinny_gemm(void*, void*, const void*, const void*, int, int,
                           int, long, int, int, hipStream_t);
+hipError_t ks_skinny_clamped_glu(void*, const void*, const void*, int, int, int, long,
+                                 float, float, hipStream_t);
 hipError_t ks_gemm8(void*, const void*, const void*, int, int, int, int,
                     hipStream_t);
 }
@@ -433,6 +435,21 @@ void skinny_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
   skinny_product(out, x, w, true);
 }
 
+void skinny_clamped_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w, double alpha,
+                        double limit) {
+  // out [N, M] = clamped gate and up of x @ w^T, bf16, N <= 256
+  CHECK_BF16_CONTIG(out);
+  const SkinnyShape z = skinny_shape(x, w, 2);
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == z.N && out.size(1) == z.M &&
+                  out.device() == x.device(),
+              "output shape mismatch");
+  const c10::DeviceGuard guard(x.device());
+  check_hip(ks_skinny_clamped_glu(out.data_ptr(), x.data_ptr(), w.data_ptr(), z.M, z.K,
+                                  z.N, z.stride, (float)alpha, (float)limit,
+                                  current_stream()),
+            "skinny_clamped_glu");
+}
+
 void dense_gemm(at::Tensor& out, at::Tensor& x, at::Tensor& w,
                 const c10::optional<at::Tensor>& bias, bool gelu, int64_t tile) {
   // out [N, M] = act(x [N, K] @ w [M, K]^T + bias), bf16
@@ -613,6 +630,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_rope_cache", &skinny_rope_cache,
         "few-row qkv GEMM, rotary embedding and K/V scatter");
   m.def("skinny_glu", &skinny_glu, "gate|up GEMM (N<=256) with silu(gate) * up");
+  m.def("skinny_clamped_glu", &skinny_clamped_glu,
+        "gate|up GEMM (N<=256) with the clamped gate");
   m.def("dense_gemm", &dense_gemm, "GEMM with bias and, if asked for, erf GELU",
         pybind11::arg("out"), pybind11::arg("x"), pybind11::arg("w"),
         pybind11::arg("bias"), pybind11::arg("gelu"), pybind11::arg("tile") = -1);

@@ -34,14 +34,18 @@ constexpr int BK = 64;  // K per step
 constexpr int NWAVES = 4;
 constexpr int NT_AUX = 2;  // cache policy of a non-temporal load
 
-enum Epilogue { BF16_OUT, PARTIAL, GLU };
+enum Epilogue { BF16_OUT, PARTIAL, GLU, CLAMPED };
+// gate and up rows: silu(gate) * up or, CLAMPED, gate sigmoid(alpha gate) (up + 1) of
+// gate up to a limit and up within it
+constexpr bool has_halves(int epi) { return epi == GLU || epi == CLAMPED; }
 
 struct GemmArgs {
   void* out;       // [N][M] bf16; PARTIAL: [splits][N][M] fp32
   const short* x;  // [N][K], row stride xs
-  const short* w;  // [M][K]; GLU: [2 M][K], gate rows first
+  const short* w;  // [M][K]; with halves [2 M][K], gate rows first
   int M, K, N;
   long xs;
+  float alpha, limit;  // CLAMPED
 };
 
 // s_waitcnt with vmcnt <= n (bits 3:0 and 15:14), lgkmcnt 0, expcnt free
@@ -73,10 +77,10 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
   // at one step (K 14336, M 4096 at 96 / 128 rows 28.1 / 30.0, 29.3 / 34.5 with it).
   const int rot = NT > 4 && gridDim.y > 3 ? 0 : (int)(blockIdx.x / 2) % n;
 
-  // first feature of the block's W rows (GLU: of gate and up rows)
-  const int f0 = blockIdx.x * (EPI == GLU ? BM / 2 : BM);
+  // first feature of the block's W rows (with halves: of gate and up rows)
+  const int f0 = blockIdx.x * (has_halves(EPI) ? BM / 2 : BM);
   auto w_row = [&](int r) {  // row of w for row r of the tile, clamped
-    if constexpr (EPI == GLU) {
+    if constexpr (has_halves(EPI)) {
       const int f = min(f0 + (r < BM / 2 ? r : r - BM / 2), p.M - 1);
       return r < BM / 2 ? f : p.M + f;
     } else {
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
     }
   }
 
-  if constexpr (EPI == GLU) {
+  if constexpr (has_halves(EPI)) {
     // up waves hand their sums to the gate waves through LDS
     __syncthreads();
     f32x4_t* up = reinterpret_cast<f32x4_t*>(ring);  // [2][F][NT][64]
@@ -179,8 +183,14 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
         const f32x4_t u = up[((wave * F + f) * NT + t) * 64 + lane];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float x = acc[f][t][r];
-          acc[f][t][r] = x / (1.f + __expf(-x)) * u[r];
+          if constexpr (EPI == GLU) {
+            const float x = acc[f][t][r];
+            acc[f][t][r] = x / (1.f + __expf(-x)) * u[r];
+          } else {
+            const float x = fminf(acc[f][t][r], p.limit);
+            const float v = fminf(fmaxf(u[r], -p.limit), p.limit);
+            acc[f][t][r] = x / (1.f + __expf(-p.alpha * x)) * (v + 1.f);
+          }
         }
       }
   }
@@ -294,7 +304,7 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
     return hipErrorInvalidValue;
   const bool sums = splits > 1 || !out;
   const GemmArgs p{sums ? partial : out, (const short*)x, (const short*)w, M,
-                   K, N, xs};
+                   K, N, xs, 0.f, 0.f};
   // (their offsets within a tile are 32 bits wide: longer rows stay here)
   if (!glu && ks_mid_takes(M, K, N) && xs < 1 << 22) {
     const hipError_t e = ks_mid_gemm(p.out, x, w, M, K, N, xs, splits, sums, stream);
@@ -325,5 +335,26 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
                        splits);
     HIP_CHECK_KERNEL();
   }
+  return hipSuccess;
+}
+
+// silu-like gate within limits (CLAMPED above), gate and up of w [2 M][K]. The
+// activation kernel and its launch take 3.5 us of a decode layer, and the sums reach
+// it in 32 bits (hybrid step of 4 layers at 1 / 8 / 24 / 64 sequences 345 -> 342, 380 ->
+// 375, 446 -> 435, 652 -> 642 us).
+extern "C" hipError_t ks_skinny_clamped_glu(void* out, const void* x, const void* w, int M,
+                                            int K, int N, long xs, float alpha,
+                                            float limit, hipStream_t stream) {
+  if (N < 1 || N > 256 || M < 1 || M % 4 != 0 || K < BK || K % BK != 0 || xs % 8 != 0 ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
+    return hipErrorInvalidValue;
+  const GemmArgs p{out, (const short*)x, (const short*)w, M, K, N, xs, alpha, limit};
+  const int bm = feature_tile(N) / 2;
+  const dim3 grid((M + bm - 1) / bm, 1);
+#define GO(nt, f, s)                                                                     \
+  hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, CLAMPED>), grid, dim3(256), 0, stream, p);
+  FOR_TILE(N, GO)
+#undef GO
+  HIP_CHECK_KERNEL();
   return hipSuccess;
 }

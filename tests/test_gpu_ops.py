@@ -1546,6 +1546,32 @@ class TestOnePartProducts:
         assert ((sums[0].double() - want).abs() <= off).all()
 
 
+class TestClampedProducts:
+    @pytest.mark.parametrize("K,M", [(2048, 8192), (64, 4612), (1088, 5000)])
+    @pytest.mark.parametrize("N", [1, 16, 33, 64, 100])
+    def test_linear_clamped_swiglu(self, dev, N, K, M):
+        """Against fp64, gates and ups past their limits among them: fp32 sums of K terms
+        with the slopes of the function (at most 1.1 in the gate and the limit in up),
+        exp and one rounding to bf16."""
+        from kserve_amd import ops
+
+        torch.manual_seed(N + M)
+        alpha, limit = 1.702, 2.5
+        x = torch.randn(N, K + 8, device=dev, dtype=torch.bfloat16)[:, :K]
+        w = (torch.randn(2 * M, K, device=dev) * 2 * K ** -0.5).to(torch.bfloat16)
+        got = torch.empty(N, M, device=dev, dtype=torch.bfloat16)
+        ops._C.skinny_clamped_glu(got, x, w, alpha, limit)
+        if N <= 48:
+            assert torch.equal(got, ops.linear_clamped_swiglu(x, w, alpha, limit))
+        y = x.double() @ w.double().t()
+        g, u = y[:, :M].clamp(max=limit), y[:, M:].clamp(-limit, limit)
+        want = g * torch.sigmoid(alpha * g) * (u + 1)
+        off = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+        lim = 1.2 * off[:, :M] * (u + 1).abs() + limit * off[:, M:] + 2.0 ** -20 * (g * (u + 1)).abs()
+        assert ((got.double() - want).abs() <= lim + 2.0 ** -8 * want.abs()).all()
+        assert y[:, :M].max() > limit and y[:, M:].min() < -limit
+
+
 class TestOperandDevices:
     """The entry points that took over from guarded torch calls."""
 
