@@ -457,6 +457,24 @@ def _one_part_rows(n: int, k: int, m: int) -> bool:
     )
 
 
+def _biased_rows(n: int, k: int, m: int) -> bool:
+    """Whether a wide product with a bias goes to the few-row kernel, which adds it to
+    its sums (MI355X, us, kernel / library; at one row the library's addition is a copy
+    into the output before the product): k 2048, m 13376 at 1 / 24 / 64 / 96 / 128 rows
+    11.3 / 17.5, 11.7 / 15.3, 15.9 / 16.7, 17.0 / 17.7, 18.3 / 19.6; k 512, m 16384 at 1 / 128
+    rows 6.0 / 13.6, 7.7 / 11.1; k 4096, m 10304 at 1 / 24 rows 18.9 / 26.5, 18.9 / 20.7; k
+    8192, m 32000 at 24 rows 80 / 129. Past 8 rows only where the tiles fill the units'
+    rounds (k 4096, m 24576 at 1 / 24 rows 42 / 45, 47 / 45), past 32 not on long K (k
+    2560, m 13376 at 64 rows 20.8 / 18.7, k 4096 at 48 26.0 / 24.9). Narrower ones are the encoder's."""
+    if m <= 8192 or m % 8:
+        return False
+    if n > 64:
+        return _one_part_rows(n, k, m)
+    tiles = -(-m // 64)
+    even = tiles <= 256 or tiles * 8 >= -(-tiles // 256) * 256 * 7
+    return n <= 8 or even and (n <= 32 or k <= 2048)
+
+
 def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     """The same for the gate|up product with silu(gate) * up on its sums,
     against the library's product and the activation kernel (k 4096, m 14336:
@@ -514,6 +532,19 @@ def _dense_rows(n: int, k: int, m: int, gelu: bool) -> bool:
     return k <= 1024 and n <= 3584 and (gelu or work <= 5.8e9)
 
 
+def _plain_bias(bias: torch.Tensor, m: int, x: torch.Tensor) -> bool:
+    return (
+        type(bias) in _TENSORS
+        and bias.shape == (m,)
+        and bias.dtype == torch.bfloat16
+        and bias.device == x.device
+        and bias.is_contiguous()
+        and bias.data_ptr() % 16 == 0
+        and not (torch.is_grad_enabled() and bias.requires_grad)
+        and not torch.is_autocast_enabled("cuda")
+    )
+
+
 def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
     """The encoder kernel's product, or None for operands that it does not take."""
     m = weight.shape[0]
@@ -525,14 +556,7 @@ def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
         and _plain_operands(x, weight)
         and x.shape[0] < 1 << 30
         and x.shape[1] <= x.stride(0) < 1 << 22
-        and type(bias) in _TENSORS
-        and bias.shape == (m,)
-        and bias.dtype == torch.bfloat16
-        and bias.device == x.device
-        and bias.is_contiguous()
-        and bias.data_ptr() % 16 == 0
-        and not (torch.is_grad_enabled() and bias.requires_grad)
-        and not torch.is_autocast_enabled("cuda")
+        and _plain_bias(bias, m, x)
         # (host time is nothing there, and the library's kernel the faster one)
         and (x.shape[1] <= 2048 or not torch.cuda.is_current_stream_capturing())
     ):
@@ -551,20 +575,21 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         if out is not None:
             return out
     # sizes first: most calls that are not for the kernel end there
+    m = weight.shape[0]
     if (
-        bias is None
-        and type(x) in _TENSORS
+        type(x) in _TENSORS
         and x.dim() == 2
         and (
-            _skinny_rows(x.shape[0], x.shape[1], weight.shape[0])
-            or _one_part_rows(x.shape[0], x.shape[1], weight.shape[0])
+            _biased_rows(x.shape[0], x.shape[1], m)
+            if bias is not None
+            else _skinny_rows(x.shape[0], x.shape[1], m)
+            or _one_part_rows(x.shape[0], x.shape[1], m)
         )
         and _skinny_operands(x, weight)
+        and (bias is None or _plain_bias(bias, m, x))
     ):
-        out = torch.empty(
-            (x.shape[0], weight.shape[0]), dtype=x.dtype, device=x.device
-        )
-        _C.skinny_gemm(out, x, weight)
+        out = torch.empty((x.shape[0], m), dtype=x.dtype, device=x.device)
+        _C.skinny_gemm(out, x, weight, bias)
         return out
     return torch.nn.functional.linear(x, weight, bias)
 

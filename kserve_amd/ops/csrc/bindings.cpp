@@ -54,7 +54,7 @@ hipError_t ks_add_splits_rms_norm(void*, void*, const void*, const void*, float,
 int ks_skinny_splits(int, int, int, int);
 hipError_t ks_dense_gemm(void*, const void*, const void*, const void*, int, int, int,
                          long, int, int, hipStream_t);
-hipError_t ks_skinny_gemm(void*, void*, const void*, const void*, int, int,
+hipError_t ks_skinny_gemm(void*, void*, const void*, const void*, const void*, int, int,
                           int, long, int, int, hipStream_t);
 hipError_t ks_skinny_clamped_glu(void*, const void*, const void*, int, int, int, long,
                                  float, float, hipStream_t);
@@ -401,38 +401,44 @@ static at::Tensor skinny_sums(const at::Tensor& x, const at::Tensor& w) {
   const c10::DeviceGuard guard(x.device());
   const int splits = ks_skinny_splits(z.M, z.K, z.N, 0);
   at::Tensor part = at::empty({splits, z.N, z.M}, x.options().dtype(at::kFloat));
-  check_hip(ks_skinny_gemm(nullptr, part.data_ptr(), x.data_ptr(), w.data_ptr(), z.M,
-                           z.K, z.N, z.stride, splits, 0, current_stream()),
+  check_hip(ks_skinny_gemm(nullptr, part.data_ptr(), x.data_ptr(), w.data_ptr(), nullptr,
+                           z.M, z.K, z.N, z.stride, splits, 0, current_stream()),
             "skinny_gemm");
   return part;
 }
 
 static void skinny_product(at::Tensor& out, at::Tensor& x, at::Tensor& w,
-                           bool glu) {
+                           const c10::optional<at::Tensor>& bias, bool glu) {
   CHECK_BF16_CONTIG(out);
   const SkinnyShape z = skinny_shape(x, w, glu ? 2 : 1);
   TORCH_CHECK(out.dim() == 2 && out.size(0) == z.N && out.size(1) == z.M &&
                   out.device() == x.device(),
               "output shape mismatch");
+  if (bias)
+    TORCH_CHECK(bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() &&
+                    bias->dim() == 1 && bias->size(0) == z.M &&
+                    bias->device() == x.device(),
+                "bias [M] bf16");
   const c10::DeviceGuard guard(x.device());
   const int splits = ks_skinny_splits(z.M, z.K, z.N, glu);
   at::Tensor part;  // fp32 sums of the K splits
   if (splits > 1)
     part = at::empty({(long)splits * z.N * z.M}, x.options().dtype(at::kFloat));
   check_hip(ks_skinny_gemm(out.data_ptr(), splits > 1 ? part.data_ptr() : nullptr,
-                           x.data_ptr(), w.data_ptr(), z.M, z.K, z.N, z.stride,
-                           splits, glu, current_stream()),
+                           x.data_ptr(), w.data_ptr(), bias ? bias->data_ptr() : nullptr,
+                           z.M, z.K, z.N, z.stride, splits, glu, current_stream()),
             "skinny_gemm");
 }
 
-void skinny_gemm(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
-  // out [N, M] = x [N, K] @ w [M, K]^T, bf16, N <= 256
-  skinny_product(out, x, w, false);
+void skinny_gemm(at::Tensor& out, at::Tensor& x, at::Tensor& w,
+                 const c10::optional<at::Tensor>& bias) {
+  // out [N, M] = x [N, K] @ w [M, K]^T + bias, bf16, N <= 256 (bias: M % 8 == 0)
+  skinny_product(out, x, w, bias, false);
 }
 
 void skinny_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
   // out [N, M] = silu(x @ w[:M]^T) * (x @ w[M:]^T), bf16, N <= 256
-  skinny_product(out, x, w, true);
+  skinny_product(out, x, w, c10::nullopt, true);
 }
 
 void skinny_clamped_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w, double alpha,
@@ -621,7 +627,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual-add + LayerNorm");
   m.def("gelu", &gelu, "erf GELU");
   def_sampling(m);
-  m.def("skinny_gemm", &skinny_gemm, "decode GEMM (N<=256, MFMA streaming)");
+  m.def("skinny_gemm", &skinny_gemm, "decode GEMM (N<=256, MFMA streaming)",
+        pybind11::arg("out"), pybind11::arg("x"), pybind11::arg("w"),
+        pybind11::arg("bias") = pybind11::none());
   m.def("skinny_sums", &skinny_sums, "few-row GEMM as fp32 sums of parts of K");
   m.def("skinny_add_rms_norm", &skinny_add_rms_norm,
         "few-row GEMM into a residual and its RMS norm");

@@ -400,15 +400,17 @@ extern "C" int ks_mid_splits(int M, int K, int N) {
   return s < 1 ? 1 : s > 16 ? 16 : s;
 }
 
-// out: fp32 sums of the parts (sums) or bf16
-extern "C" hipError_t ks_mid_gemm(void* out, const void* x, const void* w, int M, int K,
-                                  int N, long xs, int splits, int sums,
-                                  hipStream_t stream) {
-  if (N < 1 || N > 256 || M < 4 || M % 4 != 0 || K < BK || K % BK != 0 ||
+// out: fp32 sums of the parts (sums) or bf16 with the bias, if there is one
+extern "C" hipError_t ks_mid_gemm(void* out, const void* x, const void* w,
+                                  const void* bias, int M, int K, int N, long xs,
+                                  int splits, int sums, hipStream_t stream) {
+  if ((bias && (sums || M % 8 != 0)) || N < 1 || N > 256 || M < 4 || M % 4 != 0 || K < BK || K % BK != 0 ||
       K >= 1 << 22 || xs % 8 != 0 || xs >= 1 << 22 || splits < 1 || splits > K / BK ||
-      (splits > 1 && !sums) || (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
+      (splits > 1 && !sums) ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)bias) & 15) != 0)
     return hipErrorInvalidValue;
-  DenseArgs p{out, (const short*)x, (const short*)w, nullptr, M, K, N, (int)xs, 0, 0};
+  DenseArgs p{out, (const short*)x, (const short*)w, (const short*)bias, M, K, N, (int)xs,
+              0, 0};
 #define GO(tn, tm, wn, wm, s, epi)                                                    \
   {                                                                                   \
     p.ftiles = (M + tm - 1) / tm;                                                     \

@@ -47,6 +47,19 @@ def test_one_part_product(n, k, m, own):
 @pytest.mark.parametrize(
     "n,k,m,own",
     [
+        (1, 2048, 13376, True), (64, 2048, 13376, True), (128, 2048, 13376, True),
+        (1, 2048, 8192, False), (1, 2048, 13380, False), (8, 4096, 24576, True),
+        (24, 4096, 24576, False), (32, 4096, 13376, True), (33, 4096, 13376, False),
+        (24, 8192, 32000, True), (129, 2048, 13376, False), (96, 5120, 13376, False),
+    ],
+)
+def test_biased_product(n, k, m, own):
+    assert ops._biased_rows(n, k, m) is own
+
+
+@pytest.mark.parametrize(
+    "n,k,m,own",
+    [
         (1, 4096, 14336, True), (64, 4096, 14336, True), (96, 4096, 14336, True),
         (1, 8192, 14336, True), (1, 8192, 7168, False),  # 56 us, library 50
         (64, 2560, 9728, False), (64, 5120, 13824, False),  # 71 / 62

@@ -1546,6 +1546,27 @@ class TestOnePartProducts:
         assert ((sums[0].double() - want).abs() <= off).all()
 
 
+class TestBiasedProducts:
+    @pytest.mark.parametrize("N,K,M", [
+        (1, 64, 8200), (1, 2048, 13376), (17, 4096, 8264), (64, 2048, 13376), (8, 8192, 10248),
+        (65, 512, 8200), (128, 2048, 13376), (100, 4096, 12296),
+    ])
+    def test_linear(self, dev, N, K, M):
+        """One part of K and several, last tiles with features past the end, rows of
+        another stride; against fp64: fp32 sums of K terms and the bias, one rounding."""
+        from kserve_amd import ops
+
+        torch.manual_seed(N + M)
+        assert ops._biased_rows(N, K, M)
+        x = torch.randn(N, K + 64, device=dev, dtype=torch.bfloat16)[:, :K]
+        w = (torch.randn(M, K, device=dev) * K ** -0.5).to(torch.bfloat16)
+        b = torch.randn(M, device=dev, dtype=torch.bfloat16) * 4
+        got = ops.linear(x, w, b)
+        want = x.double() @ w.double().t() + b.double()
+        off = (K + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+        assert ((got.double() - want).abs() <= off + 2.0 ** -8 * want.abs()).all()
+
+
 class TestClampedProducts:
     @pytest.mark.parametrize("K,M", [(2048, 8192), (64, 4612), (1088, 5000)])
     @pytest.mark.parametrize("N", [1, 16, 33, 64, 100])
