@@ -180,14 +180,17 @@ class MerulornForCausalLM(nn.Module):
 
     # -- forward --------------------------------------------------------------
     def forward(self, input_ids, positions, caches, meta):
-        x = ops.embed_scale_sinpos(
+        # (the first norm comes with the embedding)
+        first = self.layers[0].norm1 if len(self.layers) else self.final_norm
+        x, h = ops.embed_scale_norm(
             self.embed, input_ids, positions, self.inv_freq,
-            self.config.embedding_scale,
+            self.config.embedding_scale, first, self.eps, 1.0, self.dtype,
         )
-        pending = (None, 1.0, None, 1.0)
+        pending = None
         dbg = self.debug_residuals
         for layer, cache in zip(self.layers, caches):
-            h = self._add_norm(x, layer.norm1, pending)
+            if pending is not None:
+                h = self._add_norm(x, layer.norm1, pending)
             pending = layer.mixer(h, positions, cache, meta)
             if layer.mlp is not None:
                 h = self._add_norm(x, layer.norm2, pending)
@@ -198,7 +201,7 @@ class MerulornForCausalLM(nn.Module):
                     if d is not None:
                         r += s * (d.sum(0) if d.dim() == 3 else d.float())
                 dbg.append(r)
-        return self._add_norm(x, self.final_norm, pending)
+        return h if pending is None else self._add_norm(x, self.final_norm, pending)
 
     def _add_norm(self, x, weight, pending):
         d0, s0, d1, s1 = pending

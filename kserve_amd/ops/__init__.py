@@ -894,6 +894,37 @@ def embed_scale_sinpos(table, tokens, positions, inv_freq, scale: float):
     return torch_ref.embed_scale_sinpos(table, tokens, positions, inv_freq, scale)
 
 
+def embed_scale_norm(
+    table, tokens, positions, inv_freq, scale: float, weight, eps: float,
+    w_offset: float, out_dtype,
+):
+    """(``embed_scale_sinpos``, its RMS norm with weight (w_offset + w) in
+    ``out_dtype``). In one kernel for bf16 rows that its registers hold; there a token
+    outside the table gives rows of NaN."""
+    width = table.shape[1]
+    if (
+        table.is_cuda
+        and table.dtype == out_dtype == torch.bfloat16
+        and table.shape[0] > 0
+        and 4 <= width <= 8192
+        and width % 4 == 0
+        and table.is_contiguous()
+        and weight.dtype == torch.float32
+        and weight.is_contiguous()
+        and weight.data_ptr() % 16 == 0
+        and table.data_ptr() % 8 == 0
+    ):
+        residual = _f32_like(tokens.shape[0], width, table)
+        out = torch.empty(residual.shape, dtype=out_dtype, device=table.device)
+        _native_seq("embed_scale_norm").embed_scale_norm(
+            residual, out, table, tokens, positions, inv_freq, float(scale), weight,
+            float(w_offset), float(eps),
+        )
+        return residual, out
+    residual = embed_scale_sinpos(table, tokens, positions, inv_freq, scale)
+    return residual, add_rms_norm_f32res(residual, weight, eps, w_offset, out_dtype)
+
+
 def add_rms_norm_f32res(
     residual, weight, eps: float, w_offset: float, out_dtype,
     d0=None, s0: float = 1.0, d1=None, s1: float = 1.0, c0=None, c1=None,

@@ -8,6 +8,9 @@ extern "C" {
 hipError_t ks_embed_scale_sinpos(void*, const void*, const void*, const void*,
                                  const void*, float, int, int, int,
                                  hipStream_t);
+hipError_t ks_embed_scale_norm(void*, void*, const void*, const void*, const void*,
+                               const void*, float, const void*, float, float, int, int,
+                               long, hipStream_t);
 hipError_t ks_add_parts_rms_norm_f32res(void*, const void*, long, int, float, const void*,
                                         long, int, float, const void*, float, float,
                                         void*, int, int, hipStream_t);
@@ -173,6 +176,39 @@ void embed_scale_sinpos(at::Tensor& out, at::Tensor& table, at::Tensor& tokens,
                                   width, act_is_f32(table, "table"),
                                   current_stream()),
             "embed_scale_sinpos");
+}
+
+void embed_scale_norm(at::Tensor& residual, at::Tensor& out, at::Tensor& table,
+                      at::Tensor& tokens, at::Tensor& positions,
+                      const c10::optional<at::Tensor>& inv_freq, double scale,
+                      at::Tensor& weight, double w_offset, double eps) {
+  CHECK_F32(residual);
+  CHECK_F32(weight);
+  CHECK_I64(tokens);
+  CHECK_I64(positions);
+  if (inv_freq.has_value()) CHECK_F32(*inv_freq);
+  TORCH_CHECK(table.is_cuda() && table.scalar_type() == at::kBFloat16 &&
+                  table.is_contiguous() && table.dim() == 2 && out.is_cuda() &&
+                  out.scalar_type() == at::kBFloat16 && out.is_contiguous(),
+              "table and rows bf16");
+  const int64_t width = table.size(1), rows = tokens.numel();
+  TORCH_CHECK(residual.numel() == rows * width && out.numel() == rows * width &&
+                  positions.numel() == rows && weight.numel() == width &&
+                  (!inv_freq.has_value() || inv_freq->numel() * 2 >= width),
+              "embed_scale_norm: shape mismatch");
+  const c10::Device dev = table.device();
+  TORCH_CHECK(residual.device() == dev && out.device() == dev && tokens.device() == dev &&
+                  positions.device() == dev && weight.device() == dev &&
+                  (!inv_freq.has_value() || inv_freq->device() == dev),
+              "operands on different devices");
+  const c10::DeviceGuard guard(dev);
+  check_hip(ks_embed_scale_norm(residual.data_ptr(), out.data_ptr(), table.data_ptr(),
+                                tokens.data_ptr(), positions.data_ptr(),
+                                inv_freq.has_value() ? inv_freq->data_ptr() : nullptr,
+                                (float)scale, weight.data_ptr(), (float)w_offset,
+                                (float)eps, (int)rows, (int)width, table.size(0),
+                                current_stream()),
+            "embed_scale_norm");
 }
 
 void add_rms_norm_f32res(at::Tensor& residual,
@@ -1380,6 +1416,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "scaled embedding + interleaved sinusoidal positions (fp32 out)");
   m.def("add_parts_rms_norm_f32res", &add_parts_rms_norm_f32res,
         "add_rms_norm_f32res of deltas that may be in parts");
+  m.def("embed_scale_norm", &embed_scale_norm, "scaled embedding rows and their RMSNorm");
   m.def("add_rms_norm_f32res", &add_rms_norm_f32res,
         "fp32 residual += scaled deltas, then offset-weight RMS norm");
   m.def("gated_group_rms_norm", &gated_group_rms_norm,

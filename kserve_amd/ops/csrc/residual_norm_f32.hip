@@ -228,6 +228,64 @@ __global__ void add_rms_norm_f32res_vec4_kernel(
   }
 }
 
+// The start of a stream: embed_scale_sinpos by fours and the norm of the row, which is
+// kept in registers, in the order of sums of the kernel above. A token outside the
+// table gets rows of NaN. us, two launches / this, width 2048, with angles: 1 token 4.5 /
+// 3.4, 128 5.1 / 3.9, 8000 35.9 / 24.4, without 33.2 / 20.7.
+template <int STEPS>
+__global__ __launch_bounds__(NT) void embed_scale_norm_kernel(
+    float* __restrict__ residual, short* __restrict__ out, const short* __restrict__ table,
+    const long* __restrict__ tokens, const long* __restrict__ positions,
+    const float* __restrict__ inv_freq, float scale, const float* __restrict__ weight,
+    float w_offset, float eps, int width, long vocab) {
+  __shared__ float scratch[NW];
+  const long row = blockIdx.x;
+  const long id = tokens[row];
+  const bool known = id >= 0 && id < vocab;
+  const short* src = table + (known ? id : 0) * width;
+  const float pos = inv_freq ? (float)positions[row] : 0.f;
+  const float nan = __builtin_bit_cast(float, 0x7fc00000);
+  float x[STEPS][4], w[STEPS][4];
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) {
+    const int i = (threadIdx.x + NT * k) * 4;
+    if (i < width) {
+      ld4<short>(src + i, x[k]);
+      ld4<float>(weight + i, w[k]);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) {
+    const int i = (threadIdx.x + NT * k) * 4;
+    if (i < width) {
+      float pe[4] = {0.f, 0.f, 0.f, 0.f};
+      if (inv_freq) {
+        sincosf(pos * inv_freq[i >> 1], &pe[0], &pe[1]);
+        sincosf(pos * inv_freq[(i >> 1) + 1], &pe[2], &pe[3]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[k][j] = known ? x[k][j] * scale + pe[j] : nan;
+        ss += x[k][j] * x[k][j];
+      }
+      st4<float>(residual + row * width + i, x[k]);
+    }
+  }
+  ss = block_sum_sync<NW>(ss, scratch);
+  const float inv = 1.0f / sqrtf(ss / (float)width + eps);
+#pragma unroll
+  for (int k = 0; k < STEPS; ++k) {
+    const int i = (threadIdx.x + NT * k) * 4;
+    if (i < width) {
+      float o[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[j] = x[k][j] * inv * (w_offset + w[k][j]);
+      st4<short>(out + row * width + i, o);
+    }
+  }
+}
+
 // The same for deltas that may still be in parts, as the few-row products
 // leave them: [parts][rows][width] fp32 sums, added here in order, which saves a
 // decode layer a launch and a pass over the rows for each such product (hybrid step of
@@ -861,6 +919,31 @@ extern "C" hipError_t ks_embed_scale_sinpos(void* out, const void* table,
                        0, stream, (float*)out, (const short*)table,
                        (const long*)tokens, (const long*)positions,
                        (const float*)inv_freq, scale, width);
+  HIP_CHECK_KERNEL();
+  return hipSuccess;
+}
+
+extern "C" hipError_t ks_embed_scale_norm(void* residual, void* out, const void* table,
+                                          const void* tokens, const void* positions,
+                                          const void* inv_freq, float scale,
+                                          const void* weight, float w_offset, float eps,
+                                          int rows, int width, long vocab,
+                                          hipStream_t stream) {
+  if (rows < 0 || vocab < 1 || width < 4 || width % 4 != 0 || width > NT * 4 * VEC_STEPS ||
+      (((uintptr_t)residual | (uintptr_t)weight) & 15) != 0 ||
+      (((uintptr_t)out | (uintptr_t)table) & 7) != 0)
+    return hipErrorInvalidValue;
+  if (rows == 0) return hipSuccess;
+#define GO(STEPS)                                                                         \
+  hipLaunchKernelGGL((embed_scale_norm_kernel<STEPS>), dim3(rows), dim3(NT), 0, stream,   \
+                     (float*)residual, (short*)out, (const short*)table,                  \
+                     (const long*)tokens, (const long*)positions, (const float*)inv_freq, \
+                     scale, (const float*)weight, w_offset, eps, width, vocab)
+  if (width <= NT * 4) GO(1);
+  else if (width <= NT * 8) GO(2);
+  else if (width <= NT * 16) GO(4);
+  else GO(VEC_STEPS);
+#undef GO
   HIP_CHECK_KERNEL();
   return hipSuccess;
 }

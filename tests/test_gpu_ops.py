@@ -1567,6 +1567,28 @@ class TestBiasedProducts:
         assert ((got.double() - want).abs() <= off + 2.0 ** -8 * want.abs()).all()
 
 
+class TestEmbeddedStream:
+    @pytest.mark.parametrize("width", [4, 1020, 1028, 2048, 2052, 4100, 8192])
+    @pytest.mark.parametrize("rows", [0, 1, 70])
+    def test_embed_scale_norm(self, dev, width, rows):
+        """The two kernels' rows, bit for bit; a token outside the table is NaN."""
+        from kserve_amd import ops
+
+        torch.manual_seed(width)
+        table = torch.randn(50, width, device=dev).to(torch.bfloat16)
+        tok, pos = (torch.randint(0, n, (rows,), device=dev) for n in (50, 8192))
+        w, inv = torch.randn(width, device=dev), torch.rand(width // 2, device=dev)
+        for freq in (inv, None):
+            x, h = ops.embed_scale_norm(table, tok, pos, freq, 2.5, w, 1e-5, 1.0, torch.bfloat16)
+            want = ops.embed_scale_sinpos(table, tok, pos, freq, 2.5)
+            assert torch.equal(x, want)
+            assert torch.equal(h, ops.add_rms_norm_f32res(want, w, 1e-5, 1.0, torch.bfloat16))
+        if rows:
+            tok[0], tok[-1] = 50, -1
+            x, h = ops.embed_scale_norm(table, tok, pos, inv, 2.5, w, 1e-5, 1.0, torch.bfloat16)
+            assert all(t[[0, -1]].isnan().all() and not t[1:-1].isnan().any() for t in (x, h))
+
+
 class TestClampedProducts:
     @pytest.mark.parametrize("K,M", [(2048, 8192), (64, 4612), (1088, 5000)])
     @pytest.mark.parametrize("N", [1, 16, 33, 64, 100])
