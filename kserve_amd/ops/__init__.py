@@ -600,14 +600,15 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     dtype otherwise. Without a launch of its own for the sums it also gains on the
     narrow weights that `linear` leaves to the library above 64 rows (k 4096, m 2048
     at 128 / 200 rows 9.0 / 11.5 us and the reading of 8 / 4 parts, library 12.4 /
-    14.3)."""
+    14.3; 2048 x 2048 7.1 / 8.3, library 11.0 / 11.9: a hybrid step of 72 / 96 / 128
+    sequences 705 -> 695, 807 -> 798, 1000 -> 992)."""
     n, k, m = x.shape[0], x.shape[-1], weight.shape[0]
     if (
         x.dim() == 2
         and m <= 8192
         and (
             _skinny_rows(n, k, m)
-            or n <= 256 and m % 4 == 0 and 2048 <= m < 4096 and 4096 <= k < 1 << 22
+            or n <= 256 and m % 4 == 0 and 2048 <= m < 4096 and 2048 <= k < 1 << 22
         )
         and _skinny_operands(x, weight)
     ):
