@@ -42,11 +42,13 @@ typedef __attribute__((address_space(3))) void lds_t;
 
 // 16 bytes per lane from a uniform address (lane and step offsets below 2^32)
 // straight to 1 KB of LDS
+constexpr int NT_AUX = 2;  // cache policy of a non-temporal load
+template <int AUX = 0>
 __device__ __forceinline__ void load_lds(const short* from, short* to, unsigned int lane_at,
                                          int step_at) {
   const __amdgpu_buffer_rsrc_t rows =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<short*>(from), 0, -1, 0x00027000);
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_t*)to, 16, lane_at, step_at, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_t*)to, 16, lane_at, step_at, 0, AUX);
 }
 
 // s_waitcnt with vmcnt <= n (bits 3:0 and 15:14), lgkmcnt 0, expcnt free
@@ -118,8 +120,13 @@ __global__ __launch_bounds__(WN * WM * 64, 2) void dense_gemm_kernel(const Dense
       step += rot;
       step -= step >= steps ? steps : 0;
     }
-    load_lds(i < NX ? xb : wb, &ring[slot * STAGE + (i * NW + wave) * 8 * BK], at[i],
-             step * BK * 2);
+    short* const to = &ring[slot * STAGE + (i * NW + wave) * 8 * BK];
+    // Weights that one block alone reads pass the caches by: they leave no room there
+    // otherwise to what the next kernels read and to what the last ones wrote (steps in
+    // us: hybrid 72 / 128 sequences 695 -> 683, 992 -> 981, llama 256 2268 -> 2260, 192
+    // level). Not the narrow products' in parts (72 / 128 sequences 8 and 6 us slower).
+    if ((APART || TN == 256) && i >= NX) load_lds<NT_AUX>(wb, to, at[i], step * BK * 2);
+    else load_lds(i < NX ? xb : wb, to, at[i], step * BK * 2);
   };
 
   const int wn = wave % WN, wm = wave / WN;

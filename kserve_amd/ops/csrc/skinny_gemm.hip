@@ -16,7 +16,7 @@
 // parentheses): K 4096, M 14336 GLU at 1 row 40 = 5.9 TB/s (67 with the
 // activation kernel), at 24 rows 41; K 4096, M 32000 at 1 row 42 (61); K
 // 14336, M 4096 at 1 / 24 rows 23 / 24 (27 / 32). Up to 48 rows the loads bound it
-// (non-temporal ones took 5 to 10 % off; no gain above); above, LDS reads and the
+// (non-temporal ones took 5 to 10 % off); above, LDS reads and the
 // matrix cores of the few blocks that fit, so M of a few thousand or off a multiple of
 // 4 KB a row goes back to the library. The kernel before kept a barrier per step behind
 // one load in flight and rounded the splits to bf16.
@@ -110,7 +110,10 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
         if (wave + i * NWAVES < BN / 8)  // token rows: every block reads them
           __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
         else
-          __builtin_amdgcn_global_load_lds(from, to, 16, 0, NT <= 3 ? NT_AUX : 0);
+          // past the caches, which hold what the kernels around write and read (us, with
+          // / without: prompt of 77 tokens 537 / 558, llama steps of 64 / 96 E4M3
+          // sequences 633 / 645, 998 / 997, hybrid ones of 56 / 72 597 / 611, 672 / 683)
+          __builtin_amdgcn_global_load_lds(from, to, 16, 0, NT_AUX);
         src[i] += BK * 2;
       }
     }
