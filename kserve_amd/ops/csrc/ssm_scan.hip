@@ -523,9 +523,12 @@ __global__ void __launch_bounds__(256) ssd_step_kernel(
     if (nl % 4 == 0)
       y[(long)t * inner + h * P + p0 + RP * i + pl] = sum + Dh * xr[RP * i + pl];
   }
+  // Past the caches like the loads: written back by and by, the states took the memory
+  // from the products that follow (hybrid step of 1 / 72 / 128 sequences 328 -> 318, 677
+  // -> 651, 975 -> 931 us).
 #pragma unroll
   for (int i = 0; i < NP; ++i)
-    *reinterpret_cast<float4_t*>(sp + RP * i * N + at) = S[i];
+    __builtin_nontemporal_store(S[i], reinterpret_cast<float4_t*>(sp + RP * i * N + at));
 }
 
 // ---------------------------------------------------------------------------
