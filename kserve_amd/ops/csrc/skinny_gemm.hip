@@ -111,9 +111,11 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const GemmArgs p) {
           __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
         else
           // past the caches, which hold what the kernels around write and read (us, with
-          // / without: prompt of 77 tokens 537 / 558, llama steps of 64 / 96 E4M3
-          // sequences 633 / 645, 998 / 997, hybrid ones of 56 / 72 597 / 611, 672 / 683)
-          __builtin_amdgcn_global_load_lds(from, to, 16, 0, NT_AUX);
+          // / without: llama steps of 64 sequences 632 / 645, hybrid ones of 56 561 /
+          // 574); not above 64 rows in parts, whose sums then come back slower (96 E4M3
+          // sequences 1006 / 997, 96 of 500 706 / 698, a prompt of 77 tokens 546 / 541)
+          __builtin_amdgcn_global_load_lds(from, to, 16, 0,
+                                           NT <= 4 || EPI != PARTIAL ? NT_AUX : 0);
         src[i] += BK * 2;
       }
     }
