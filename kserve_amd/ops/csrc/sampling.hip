@@ -567,11 +567,13 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
   unsigned int thr = 0;
   // where many survive: how many, and log2 of a score that some of them exceed
   unsigned int live = 0;
+  bool by_mass = false;
   float cut = 0.f;
   if (use_k || use_p) {
     // ---- first pass: counts per bin, extremes, mass ----
     for (int i = tid; i < FBINS; i += RT) lds.win[i] = 0;
     if (tid < 4) sh_bin[tid] = NONE;
+    if (tid == 0) sh_live = 0;
     __syncthreads();
     const float c2 = inv_t * 1.44269504f;
     ushort2_v lo2 = {65535, 65535}, hi2 = {0, 0};  // first and last bin
@@ -737,13 +739,14 @@ __global__ __launch_bounds__(RT) void topk_topp_sample_kernel(
           // with the mass known, elements above its logarithm less 2.5 are Poisson with
           // a mean of 12
           if (use_p && bin == sh_bin[1]) {
-            live = sh_live;
+            by_mass = true;
             cut = most * c2 + __builtin_amdgcn_logf((float)want) - 2.5f * 1.44269504f;
           }
         }
       }
     }
     __syncthreads();
+    if (by_mass) live = sh_live;  // (written after the scan's last barrier)
   }
   if ((use_k || use_p) && thr == 0) {
     // ---- largest number (exp stability), and whether a mass can be formed ----
