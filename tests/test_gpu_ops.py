@@ -1082,6 +1082,66 @@ class TestSampling:
             assert x[r][got] >= lo, (r, got)
             assert score[r][got] >= score[r][x[r] >= hi].max() - 1e-4, (r, got)
 
+    @pytest.mark.parametrize("shape", ["k below p", "k with p", "k above p", "ties", "tenth"])
+    @pytest.mark.parametrize("vocab", [530, 2051, 40010])
+    def test_sets_by_both_limits(self, dev, vocab, shape):
+        """Rows of a few levels, so that each limit's place is known: top-k's below, at
+        and above top-p's where a tenth and more survives, top-k of one among as many
+        largest (no noise: the first of them), and sets of a tenth and one more. More
+        rows than compute units; the survivors are exact, and among them the score is
+        the largest to the fast fp32 logarithms (2e-6 of values up to 20)."""
+        import kserve_amd_C
+
+        n, tenth = 300, vocab // 10
+        g = torch.Generator().manual_seed(vocab)
+        top, mid = tenth - 2, 2 * tenth
+        counts = {"ties": (tenth + 3, 0), "tenth": (tenth, tenth)}.get(shape, (top, mid))
+        logits = torch.full((n, vocab), 1.0)
+        place = torch.rand(n, vocab, generator=g).argsort(1)
+        more = torch.arange(n) % 2 if shape == "tenth" else torch.zeros(n, dtype=torch.int64)
+        for r in range(n):
+            a = counts[0] + int(more[r])
+            logits[r, place[r, :a]] = 3.0
+            logits[r, place[r, a : a + counts[1]]] = 2.0
+        mass = torch.softmax(logits.double(), 1)
+        first, second = ((mass * (logits >= x)).sum(1) for x in (3.0, 2.0))
+        k = torch.zeros(n, dtype=torch.int32)
+        least = torch.full((n,), 2.0)
+        p = (first + second) / 2  # among the twos
+        if shape == "k below p":
+            k[:] = top + mid + 5
+        if shape == "k with p":
+            k[:] = top + mid // 2
+        if shape == "k above p":
+            k[:], least[:] = top, 3.0
+        if shape == "ties":
+            k[:], least[:] = 1, 3.0
+            p = first * torch.tensor([1e-5, 3.0 / tenth, 0.5])[torch.arange(n) % 3]
+        if shape == "tenth":
+            p, least[:] = first / 2, 3.0
+        seeds = torch.randint(0, 1 << 31, (n,), generator=g)
+        out = torch.empty(n, dtype=torch.int64, device=dev)
+        kserve_amd_C.topk_topp_sample(
+            out, logits.to(dev, torch.bfloat16), torch.ones(n, device=dev),
+            p.float().to(dev), k.to(dev), seeds.to(dev),
+        )
+        M = 0xFFFFFFFF
+        h = ((seeds[:, None] * 0x9E3779B1) & M) + ((torch.arange(vocab) * 0x85EBCA77) & M)
+        h = (h + 0x165667B1) & M
+        h = (h ^ (h >> 15)) * 0x2C1B3C6D & M
+        h = (h ^ (h >> 12)) * 0x297A2D39 & M
+        h = h ^ (h >> 15)
+        u = ((h.float() + 1.0) * 2.3283064e-10).clamp(max=1 - 2.0**-24)
+        score = logits.double() - torch.log(-torch.log(u.double()))
+        got = out.cpu()[:, None]
+        held = logits >= least[:, None]
+        if shape == "ties":
+            assert torch.equal(got[:, 0], held.int().argmax(1))
+            return
+        assert held.gather(1, got).all()
+        best = score.masked_fill(~held, float("-inf")).max(1).values
+        assert (score.gather(1, got)[:, 0] >= best - 1e-4).all()
+
     @pytest.mark.parametrize("low", [-3e33, -1.5e32])
     @pytest.mark.parametrize("limit", [0, 70002, 70000])
     def test_lowest_rows(self, dev, low, limit):
