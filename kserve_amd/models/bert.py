@@ -18,6 +18,7 @@ import torch
 import torch.nn as nn
 
 from kserve_amd import ops
+from kserve_amd.models.hooks import unhooked
 
 
 @dataclass
@@ -164,7 +165,7 @@ class BertModel(nn.Module):
             host.copy_(stats, non_blocking=True)
             there = torch.cuda.Event()
             there.record(torch.cuda.current_stream(stats.device))
-            if len(self.layers):
+            if len(self.layers) and unhooked(self.layers[0], BertLayer):
                 qkv = self.layers[0].project(hidden)
             there.synchronize()
             stats = host
@@ -179,8 +180,10 @@ class BertModel(nn.Module):
                 f"{self.position_embeddings.shape[0]} positions"
             )
         for layer in self.layers:
-            hidden = layer(hidden, cu_seqlens, max_seqlen, qkv)
-            qkv = None
+            if qkv is None:
+                hidden = layer(hidden, cu_seqlens, max_seqlen)
+            else:
+                hidden, qkv = layer(hidden, cu_seqlens, max_seqlen, qkv), None
         return hidden
 
     def pool(self, hidden: torch.Tensor, cu_seqlens: torch.Tensor) -> torch.Tensor:

@@ -1876,6 +1876,54 @@ class TestMeasuredLengths:
         assert stats.tolist() == [lens.max(), lens.min(), lens.sum()]
         assert torch.equal(got.nan_to_num(7), ops.embed_layer_norm(*args).nan_to_num(7))
 
+    @pytest.mark.parametrize("at", ["layer", "all", "wrapped", "subclass"])
+    def test_hooked_first_layer(self, dev, at):
+        """What changes the first layer's rows reaches its projection: the embedding's
+        rows doubled there give what doubled norm weights give."""
+        from kserve_amd.models import bert
+
+        class Doubled(bert.BertLayer):
+            def forward(self, hidden, cu_seqlens, max_seqlen):
+                return super().forward(hidden * 2, cu_seqlens, max_seqlen)
+
+        c = bert.BertConfig.tiny()
+        model = bert.BertModel(c, dtype=torch.bfloat16, device=dev)
+        torch.manual_seed(5)
+        for p in model.parameters():
+            p.data.normal_(0, 0.2)
+        ids = torch.randint(0, c.vocab_size, (20,), device=dev)
+        cu = torch.tensor([0, 8, 20], dtype=torch.int32, device=dev)
+        plain = model(ids, cu)
+        model.emb_ln_w.data.mul_(2), model.emb_ln_b.data.mul_(2)
+        want = model(ids, cu)
+        model.emb_ln_w.data.div_(2), model.emb_ln_b.data.div_(2)
+        first, undo = model.layers[0], None
+
+        def double(module, args):
+            assert len(args) == 3
+            if module is first:
+                return (args[0] * 2, *args[1:])
+
+        if at == "layer":
+            undo = first.register_forward_pre_hook(double)
+        elif at == "all":
+            from torch.nn.modules.module import register_module_forward_pre_hook
+
+            undo = register_module_forward_pre_hook(
+                lambda m, args: double(m, args) if m is first else None
+            )
+        elif at == "wrapped":
+            inner = first.forward
+            first.forward = lambda hidden, *rest: inner(hidden * 2, *rest)
+        else:
+            first.__class__ = Doubled
+        try:
+            got = model(ids, cu)
+        finally:
+            if undo is not None:
+                undo.remove()
+        assert torch.equal(got, want) and not torch.equal(got, plain)
+
     def test_wrong_lengths_are_refused(self, dev):
         from kserve_amd.models.bert import BertConfig, BertModel
 
