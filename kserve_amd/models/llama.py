@@ -20,6 +20,7 @@ import torch.nn as nn
 
 from kserve_amd import ops
 from kserve_amd.engine.config import ModelConfig
+from kserve_amd.models.hooks import unhooked
 from kserve_amd.ops.torch_ref import make_cos_sin_cache
 from kserve_amd.parallel import comm
 from kserve_amd.parallel.layers import (
@@ -453,12 +454,15 @@ class LlamaForCausalLM(nn.Module):
         meta: AttentionMetadata,
     ) -> torch.Tensor:
         st = comm.get_state()
-        # the first norm comes with the embedding
-        normed = self.is_first_stage and len(self.layers) > 0
+        normed = False
         if self.is_first_stage:
             residual = None
+            # the first norm comes with the embedding, if nothing stands between
+            first = self.layers[0] if len(self.layers) else None
+            normed = unhooked(first, LlamaDecoderLayer) and unhooked(
+                self.embed_tokens, VocabParallelEmbedding
+            )
             if normed:
-                first = self.layers[0]
                 residual, hidden = self.embed_tokens(
                     input_ids, norm=(first.input_layernorm, first.eps)
                 )

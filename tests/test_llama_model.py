@@ -39,6 +39,55 @@ def full_forward_logits(model, token_ids):
     return model.compute_logits(hidden)
 
 
+class TestHookedEmbedding:
+    @pytest.mark.parametrize(
+        "at", ["embedding", "all", "wrapped", "subclass", "layer", "wrapped layer"]
+    )
+    def test_rows_reach_the_first_norm(self, at):
+        """Rows doubled by a hook of the embedding or of the first layer, or by what
+        stands in their place, give what a doubled table gives."""
+        from torch.nn.modules.module import register_module_forward_hook
+
+        from kserve_amd.parallel.layers import VocabParallelEmbedding
+
+        class Doubled(VocabParallelEmbedding):
+            def forward(self, ids):
+                return super().forward(ids) * 2
+
+        model, ids = build_model(tiny_config()), [5, 9, 2, 77]
+        plain = full_forward_logits(model, ids)
+        embed, first = model.embed_tokens, model.layers[0]
+        embed.weight.data.mul_(2)
+        want = full_forward_logits(model, ids)
+        embed.weight.data.div_(2)
+        undo = None
+        if at == "embedding":
+            undo = embed.register_forward_hook(lambda m, args, out: out * 2)
+        elif at == "all":
+            undo = register_module_forward_hook(
+                lambda m, args, out: out * 2 if m is embed else None
+            )
+        elif at == "wrapped":
+            inner = embed.forward
+            embed.forward = lambda ids: inner(ids) * 2
+        elif at == "subclass":
+            embed.__class__ = Doubled
+        elif at == "layer":
+            undo = first.register_forward_pre_hook(
+                lambda m, args: (args[0] * 2, *args[1:])
+            )
+        else:
+            call = first.forward
+            first.forward = lambda hidden, *rest, **kw: call(hidden * 2, *rest, **kw)
+        try:
+            got = full_forward_logits(model, ids)
+        finally:
+            if undo is not None:
+                undo.remove()
+        assert torch.equal(got, want) and not torch.equal(got, plain)
+        assert torch.equal(full_forward_logits(build_model(tiny_config()), ids), plain)
+
+
 class TestVsTransformers:
     def test_logits_match_hf(self):
         transformers = pytest.importorskip("transformers")
