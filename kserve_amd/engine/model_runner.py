@@ -292,7 +292,7 @@ class ModelRunner:
 
     # -- input prep -----------------------------------------------------------
     def prepare_prefill(
-        self, batch: ScheduledBatch, block_manager: BlockManager
+        self, batch: ScheduledBatch, block_manager: BlockManager, logit_rows=None
     ):
         import numpy as np
 
@@ -322,10 +322,11 @@ class ModelRunner:
             cu.append(cu[-1] + n)
             max_seqlen = max(max_seqlen, n)
             last_token_idx.append(cu[-1] - 1)
-        arrays = [
-            tokens, positions, np.asarray(last_token_idx, dtype=np.int64),
-            slots, np.asarray(cu, dtype=np.int32),
-        ]
+        if logit_rows is None:
+            sel = np.asarray(last_token_idx, dtype=np.int64)
+        else:
+            sel = torch.tensor(logit_rows, dtype=torch.int64, device="cpu").numpy()
+        arrays = [tokens, positions, sel, slots, np.asarray(cu, dtype=np.int32)]
         if self._layout is not None:
             counts = np.asarray(batch.num_scheduled_tokens, dtype=np.int64)
             arrays.append(np.repeat(np.arange(len(counts), dtype=np.int32), counts))
@@ -539,18 +540,16 @@ class ModelRunner:
     def execute_prefill(self, batch, block_manager, logit_rows=None) -> torch.Tensor:
         """Logits of each request's last scheduled token, or of the flat
         token rows in ``logit_rows`` when given."""
-        input_ids, positions, meta, sel = self.prepare_prefill(batch, block_manager)
+        input_ids, positions, meta, sel = self.prepare_prefill(
+            batch, block_manager, logit_rows
+        )
         if self.lora_manager is not None and any(
             r.lora_id for r in batch.requests
         ):
             meta.lora = self._lora_meta(batch, per_request_rows=False)
         hidden = self.model(input_ids, positions, self.kv_caches, meta)
-        if logit_rows is None:
-            rows = hidden.index_select(0, sel)
-        else:
-            rows = hidden[
-                torch.tensor(logit_rows, dtype=torch.int64, device=self.device)
-            ]
+        # (given rows may count from the end)
+        rows = hidden.index_select(0, sel) if logit_rows is None else hidden[sel]
         return self.model.compute_logits(rows)
 
     @torch.no_grad()

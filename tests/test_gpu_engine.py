@@ -616,3 +616,31 @@ def test_draft_model_speculation_on_gpu():
     assert [t[0] for t in toks1] == [t[0] for t in ref]
     # perfect draft at k=3: ~20/4 spec rounds + prefill per wave
     assert steps1 <= 12, f"expected compressed steps, got {steps1}"
+
+
+@pytest.mark.parametrize("rows", [None, [3, 0, -1, 6], []])
+def test_prefill_waits_for_nothing(rows):
+    """Nothing between a prompt's tokens and its logits waits for the device, the rows
+    asked for included; these come out as from all rows."""
+    from kserve_amd.engine.engine import LLMEngine
+    from kserve_amd.engine.request import Request
+    from kserve_amd.engine.sampling_params import SamplingParams
+    from kserve_amd.engine.scheduler import ScheduledBatch
+
+    engine = LLMEngine(_cfg(enforce_eager=True))
+    bm = engine.scheduler.block_manager
+    reqs = [Request(f"r{n}", list(range(1, n + 1)), SamplingParams()) for n in (5, 3)]
+    for r in reqs:
+        bm.allocate(r)
+    batch = ScheduledBatch(True, reqs, [5, 3])
+    every = engine.runner.execute_prefill(batch, bm, logit_rows=list(range(8)))
+    torch.cuda.synchronize()
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        got = engine.runner.execute_prefill(batch, bm, logit_rows=rows)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    want = every[[4, 7] if rows is None else rows]
+    assert got.shape == want.shape
+    # (a row's product with the vocabulary may be another kernel's beside fewer rows)
+    torch.testing.assert_close(got, want, rtol=2.0 ** -7, atol=2.0 ** -7)
