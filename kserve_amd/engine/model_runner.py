@@ -321,7 +321,8 @@ class ModelRunner:
             off += n
             cu.append(cu[-1] + n)
             max_seqlen = max(max_seqlen, n)
-            last_token_idx.append(cu[-1] - 1)
+            # (nothing scheduled so far: a row all the same, the batch's last)
+            last_token_idx.append((cu[-1] or total) - 1)
         if logit_rows is None:
             sel = np.asarray(last_token_idx, dtype=np.int64)
         else:

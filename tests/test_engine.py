@@ -405,3 +405,27 @@ def test_mixed_batches_same_tokens_as_separate_steps():
     mixed, n1 = run(True)
     assert n0 == 0 and n1 > 0
     assert plain == mixed
+
+
+def test_requests_without_tokens_in_a_prefill():
+    """A request of which nothing is scheduled gets a row of logits all the same, also
+    ahead of those that have tokens; theirs are as without it."""
+    from kserve_amd.engine.request import Request
+    from kserve_amd.engine.scheduler import ScheduledBatch
+
+    torch.manual_seed(0)
+    eng = LLMEngine(EngineConfig(
+        model=ModelConfig.tiny(vocab_size=128),
+        cache=CacheConfig(block_size=4, num_gpu_blocks=128),
+        scheduler=SchedulerConfig(max_num_seqs=8, max_num_batched_tokens=64, max_model_len=128),
+        device="cpu", eos_token_id=-1,
+    ))
+    bm = eng.scheduler.block_manager
+    reqs = [Request(f"r{n}", list(range(1, n + 1)), SamplingParams()) for n in (5, 3, 4)]
+    for r in reqs:
+        bm.allocate(r)
+    whole = eng.runner.execute_prefill(ScheduledBatch(True, reqs, [5, 3, 4]), bm)
+    for counts, kept in (([0, 3, 4], [1, 2]), ([0, 0, 4], [2]), ([5, 0, 4], [0, 2])):
+        got = eng.runner.execute_prefill(ScheduledBatch(True, reqs, counts), bm)
+        assert got.shape == whole.shape
+        assert torch.equal(got[kept], whole[kept])
