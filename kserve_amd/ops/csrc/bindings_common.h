@@ -5,6 +5,8 @@
 
 #include <torch/extension.h>
 
+#include <ATen/core/CachingHostAllocator.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
 
 #include <hip/hip_runtime.h>
@@ -123,6 +125,14 @@ void unpack_decode_rows(at::Tensor& staged, int64_t width, at::Tensor& ids,
                 state_slots.data_ptr(), slots.data_ptr(), tables.data_ptr(),
                 std::max<int64_t>(tables.stride(0), tables.size(1)), current_stream()),
             "unpack_decode_rows");
+  // pinned rows that are let go of now stay out of use until the kernel has read them,
+  // as those of a copy do
+  if (!staged.is_cuda()) {
+    const at::DataPtr& block = staged.storage().data_ptr();
+    at::getHostAllocator(at::kCUDA)->record_event(
+        block.get(), block.get_context(),
+        c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
+  }
 }
 
 void advance_decode(at::Tensor& greedy, const c10::optional<at::Tensor>& random,

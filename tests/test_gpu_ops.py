@@ -1783,6 +1783,30 @@ class TestDecodeStep:
             ops.unpack_decode_rows(staged.clone(), width, *got)
 
 
+    def test_pinned_rows_that_are_let_go(self, dev):
+        """Rows that nobody holds any more are not handed out again before the kernel,
+        held up by the work ahead of it, has read them."""
+        from kserve_amd import ops
+
+        rows, width = 100, 1016
+        want = torch.randint(0, 1 << 20, (rows, 8 + width), dtype=torch.int32)
+        v = lambda dt: torch.zeros(rows, dtype=dt, device=dev)  # noqa: E731
+        got = [v(torch.int64), v(torch.int64), v(torch.int32), v(torch.int32), v(torch.int32),
+               torch.zeros(rows, width, dtype=torch.int32, device=dev)]
+        staged = torch.empty(rows, 8 + width, dtype=torch.int32, pin_memory=True)
+        staged.copy_(want)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(200_000_000)
+        ops.unpack_decode_rows(staged, width, *got)
+        del staged
+        later = [torch.empty(rows, 8 + width, dtype=torch.int32, pin_memory=True).fill_(-1)
+                 for _ in range(4)]
+        torch.cuda.synchronize()
+        assert len(later) == 4
+        assert torch.equal(got[5].cpu(), want[:, 8:])
+        assert torch.equal(got[2].cpu(), want[:, 4])
+
+
     @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
     @pytest.mark.parametrize("rows,vocab,width", [(1, 32000, 7), (5, 1003, 1), (257, 9000, 130), (0, 64, 2)])
     def test_greedy_advance(self, dev, dtype, rows, vocab, width):
