@@ -246,9 +246,10 @@ def unpack_decode_rows(
     slots, tables,
 ) -> None:
     """Spreads staged decode rows (int32 [rows, DECODE_ROW_HEAD + width or
-    more]; on the GPU or in pinned host memory, which the caller leaves as it is
-    until the kernel has read it) over the buffers that a decode step reads."""
-    if ids.is_cuda:
+    more]) over the buffers that a decode step reads. One kernel does where the rows
+    are on the GPU or in pinned host memory, which the caller leaves as it is until
+    the kernel has read it; other host memory is copied field by field."""
+    if staged.is_cuda or ids.is_cuda and staged.is_pinned():
         _native_sampling("unpack_decode_rows").unpack_decode_rows(
             staged, int(width), ids, positions, context_lens, state_slots, slots,
             tables,

@@ -1760,7 +1760,7 @@ class TestDecodeStep:
     @pytest.mark.parametrize("rows,width", [(1, 1), (5, 255), (256, 129), (3, 2049)])
     def test_unpack_from_pinned(self, dev, rows, width):
         """Rows that the kernel reads in pinned host memory, and again after the
-        host has changed them; rows in other host memory are refused."""
+        host has changed them; rows in other host memory reach the buffers too."""
         from kserve_amd import ops
 
         torch.manual_seed(rows)
@@ -1779,8 +1779,12 @@ class TestDecodeStep:
             torch.cuda.synchronize()
             ops.unpack_decode_rows(staged, width, *want)
             assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
-        with pytest.raises(RuntimeError):
-            ops.unpack_decode_rows(staged.clone(), width, *got)
+        plain = torch.randint(0, 1 << 20, (rows, stride), dtype=torch.int32)
+        for to in (got, want):
+            ops.unpack_decode_rows(plain, width, *to)
+        assert all(torch.equal(a.cpu(), b) for a, b in zip(got, want))
+        with pytest.raises(RuntimeError):  # rows on the GPU, buffers not
+            ops.unpack_decode_rows(staged.to(dev), width, *want)
 
 
     def test_pinned_rows_that_are_let_go(self, dev):
