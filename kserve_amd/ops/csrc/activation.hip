@@ -246,15 +246,23 @@ __global__ __launch_bounds__(256) void glu_bf16x8_kernel(short* __restrict__ out
   }
 }
 
+// Whether blocks go by rows (few idle lanes then), and how many there are: HIP takes
+// fewer than 2^32 threads in a dimension, and the blocks stride over what is left.
+bool glu_by_rows(int d) { return d / 8 >= 1024 || d / 8 % 256 == 0; }
+int glu_blocks(long rows, int d) {
+  const long nvec = d / 8, per = (nvec + 255) / 256;
+  const long blocks = glu_by_rows(d) ? rows * per : (rows * nvec + 255) / 256;
+  return (int)(blocks < (1 << 24) - 1 ? blocks : (1 << 24) - 1);
+}
+
 template <typename F>
 hipError_t launch_glu_bf16x8(void* out, const void* input, long rows, int d, F f,
                              hipStream_t stream) {
-  const int nvec = d / 8, per = (nvec + 255) / 256;
-  const bool by_rows = nvec >= 1024 || nvec % 256 == 0;  // (few idle lanes)
+  const int per = (d / 8 + 255) / 256;
+  const bool by_rows = glu_by_rows(d);
   // (what the 256 MB memory-side cache holds of one product is read there by the next)
   const bool nt = rows * d * 6 > 256L << 20;
-  const long blocks = by_rows ? rows * per : (rows * nvec + 255) / 256;
-  const dim3 grid((unsigned)(blocks < 1 << 30 ? blocks : 1 << 30));
+  const dim3 grid(glu_blocks(rows, d));
 #define GO(R, N)                                                                       \
   hipLaunchKernelGGL((glu_bf16x8_kernel<R, N, F>), grid, dim3(256), 0, stream, (short*)out, \
                      (const short*)input, rows, d, per, f)
@@ -268,6 +276,8 @@ hipError_t launch_glu_bf16x8(void* out, const void* input, long rows, int d, F f
 }
 
 }  // namespace
+
+extern "C" int ks_glu_blocks(long rows, int d) { return glu_blocks(rows, d); }
 
 extern "C" hipError_t ks_silu_and_mul(void* out, const void* input, int rows,
                                       int d, hipStream_t stream) {

@@ -1,10 +1,17 @@
 """Dispatch rules of the products at sizes on both sides of their lines, where the
 times of both kernels are known (no GPU needed: the rules take sizes only)."""
 
+import ctypes
+
 import pytest
 import torch
 
 from kserve_amd import ops
+
+
+@pytest.fixture(scope="module")
+def native():
+    return ctypes.CDLL(pytest.importorskip("kserve_amd_C").__file__)
 
 
 @pytest.mark.parametrize(
@@ -210,3 +217,16 @@ def test_products_are_recorded(how, dev, dtype):
         names, got = _recorded(how, lambda v: ops.linear(v, w, bias), x)
         assert any(k in n for n in names for k in ("linear", "mm")), names
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("d", [8, 2056, 8192, 14344, 1 << 20])
+def test_blocks_of_gated_activations(native, d):
+    """A block per 256 vectors (of a row, where rows are long), and never as many as
+    come to 2^32 threads, which HIP refuses: the blocks stride over the rest."""
+    blocks = native.ks_glu_blocks
+    blocks.argtypes = [ctypes.c_long, ctypes.c_int]
+    by_rows = d >= 8192 or d % 2048 == 0
+    for rows in (1, 7, 8000, (1 << 24) - 1, 1 << 24, 1 << 28, (1 << 31) - 1):
+        got = blocks(rows, d)
+        want = rows * -(-d // 2048) if by_rows else -(-rows * (d // 8) // 256)
+        assert got == min(want, (1 << 24) - 1) and got * 256 < 1 << 32
