@@ -195,8 +195,11 @@ struct SiluMul {
     return g / (1.f + __expf(-g)) * u;
   }
 };
-// (the hardware's exponential and reciprocal: 2e-6 of the result, a thousandth of its
-// rounding to bf16; with the library's the vector units bound this, 8000 x 8192 80 us)
+// (the hardware's exponential and reciprocal; with the library's the vector units bound
+// this, 8000 x 8192 80 us. Of 16 million results from gates of N(0, s), s 0.1 / 1 / 3 / 10,
+// 7 / 3 / 6 / 16 in a million are not float64's rounded, with the library's 5 / 4 / 26 / 346:
+// what rounds off alpha * gate counts most, and a correction for it turned as many. A
+// reciprocal below 2^-126 is 0.)
 struct ClampedSwiglu {
   float slope, limit;  // slope: -alpha log2(e)
   __device__ __forceinline__ float operator()(float g, float u) const {
