@@ -448,13 +448,13 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
 def _one_part_rows(n: int, k: int, m: int) -> bool:
     """Whether 65 to 128 rows go to the few-row product's tiles of 64 features, K in
     one part, which beat the library and its other tiles where they fill one round of
-    the chip (times at ``mid_wide`` in dense_gemm.hip)."""
+    the chip (``mid_wide`` in dense_gemm.hip, the same rule, has the times)."""
     tiles = -(-m // 64)
     return (
         64 < n <= 128
         and m % 4 == 0
-        and tiles <= 256
-        and (tiles > 128 if 512 <= k <= 2048 else k == 4096 and tiles >= 192)
+        and 512 <= k <= 4608
+        and (129 if k <= 2048 else 192) <= tiles <= 256
     )
 
 

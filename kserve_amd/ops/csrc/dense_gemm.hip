@@ -376,22 +376,25 @@ extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
 // long K (K 14336, M 4096 at 77 rows 29.7, 128 x 128 here 34.1).
 static bool mid_narrow(int M, int K) { return M <= 4096 && K <= 8192; }
 
-// Wide products of 65 to 128 rows and K to 4096 in one round of blocks of 64 features
-// and all rows, 8 waves, K in one part. Bound by the reads of W and, per unit, as many
-// of x. us, here / the few-row kernel / the library at 65 and 128 rows, weights not in
-// a cache: K 512, M 10240 6.8 / 11.5 / 10.0, 7.5 / 15.7 / 10.6; K 1024, M 16384 9.7 /
-// 14.3 / 13.8, 11.2 / 18.7 / 14.5; K 2048, M 10304 15.1 / 16.4 / 21.2, 17.7 / 20.8 / 18.1;
-// K 2048, M 16384 16.3 / 19.9 / 18.4, 18.4 / 24.7 / 20.2; K 4096, M 14336 26.8 / 28.4 / 30.0,
-// 31.5 / 35.3 / 33.0. Not at 128 tiles or fewer (K 2048, M 8192 14.2 / 14.5 / 14.0, 16.9 /
-// 18.8 / 15.7), nor where K is long and a quarter of the units idle (K 4096, M 10304
-// 25.6 / 22.9 / 38.4), nor at K between (K 3072, M 16384 at 128 rows 28.6 / 30.8 / 27.0) or
-// longer (K 5120, M 14336 43.6 / 43.1 / 41.7); past 256 tiles a second round is nearly
-// empty (K 2048, M 17408 26.4 / 23.3 / 27.5).
+// Wide products of 65 to 128 rows in one round of blocks of 64 features and all rows, 8
+// waves, K in one part. Bound by the reads of W and, per unit, as many of x. us, here /
+// the few-row kernel / the library at 65 and 128 rows, weights not in a cache: K 512, M
+// 10304 5.6 / 11.3 / 10.0, 6.1 / 15.8 / 10.5; K 1088, M 16384 9.5 / 15.2 / 14.6, 11.2 / 19.5
+// / 14.8; K 1984, M 10304 13.1 / 15.9 / 21.0, 16.0 / 20.4 / 21.7; K 2304, M 12288 15.4 / 19.2 /
+// 17.6, 18.9 / 24.6 / 20.5; K 3072, M 16384 21.3 / 25.0 / 24.0, 26.6 / 30.8 / 27.2; K 4096, M
+// 14336 25.3 / 28.0 / 30.5, 29.9 / 35.2 / 33.0; K 4608, M 16384 29.9 / 33.6 / 32.7, 36.6 / 40.2 /
+// 36.8. Not at 128 tiles or fewer (K 1792, M 6144 11.1 / 14.1 / 12.2, 12.8 / 17.9 / 14.0, but
+// K 2048, M 8192 at 128 rows 16.9 / 18.8 / 15.7), nor where K is long and a quarter of the
+// units idle (K 4096, M 10304 23.9 / 22.9 / 38.3, 28.3 / 28.6 / 30.8), nor past K 4608, where
+// it turns (K 5120, M 12288 at 65 / 112 rows 32.3 / 34.2 / 33.6, 37.5 / 41.1 / 35.7, M 16384 at
+// 128 43.7 / 44.9 / 41.6); past 256 tiles a second round is nearly empty (K 2048, M 17408
+// 26.4 / 23.3 / 27.5).
 static bool mid_wide(int M, int K, int N) {
   const int tiles = (M + 63) / 64;
-  return N > 64 && N <= 128 && tiles <= UNITS &&
-         (K >= 512 && K <= 2048 ? tiles > 128 : K == 4096 && tiles >= 192);
+  return N > 64 && N <= 128 && tiles <= UNITS && K >= 512 && K <= 4608 &&
+         (K <= 2048 ? tiles > 128 : tiles >= 192);
 }
+extern "C" int ks_mid_wide(int M, int K, int N) { return mid_wide(M, K, N); }
 
 extern "C" int ks_mid_takes(int M, int K, int N) {
   if (K >= 1 << 22) return 0;  // (offsets within a tile of 32 bits)

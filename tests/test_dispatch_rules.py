@@ -44,11 +44,27 @@ def test_few_row_product(n, k, m, own):
         (65, 2048, 8192, False), (65, 2048, 16388, False),   # 23.3 / 26.4
         (128, 4096, 12288, True), (128, 4096, 12284, True),  # 192 tiles
         (128, 4096, 12224, False),                           # 28.6 / 30.3 at 10304
-        (128, 3072, 16384, False), (80, 2048, 10302, False),
+        (128, 3072, 16384, True),                            # 27.3, library 27.1
+        (80, 2048, 10302, False),
+        (65, 2304, 12288, True), (128, 2304, 12284, True), (128, 2304, 12224, False),
+        (112, 3584, 16384, True), (128, 4032, 14336, True),  # 28 / 31, 32 / 41
+        (65, 4608, 16384, True), (128, 4672, 16384, False),  # 30 / 33, 44 / 42 at 5120
     ],
 )
 def test_one_part_product(n, k, m, own):
     assert ops._one_part_rows(n, k, m) is own
+
+
+def test_one_part_product_is_one_rule(native):
+    """The wrapper's rule and the library's, which picks the kernel and the parts."""
+    ks = [64, 448, 512, 576, 1984, 2048, 2112, 3072, 4032, 4096, 4160, 4608, 4672, 8192]
+    ms = [64 * t + d for t in (1, 128, 129, 191, 192, 255, 256) for d in (-4, 0, 4)]
+    for n in (1, 64, 65, 97, 128, 129, 256):
+        for k in ks:
+            for m in ms:
+                own = ops._one_part_rows(n, k, m)
+                assert bool(native.ks_mid_wide(m, k, n)) is own, (n, k, m)
+                assert not own or native.ks_skinny_splits(m, k, n, 0) == 1
 
 
 @pytest.mark.parametrize(

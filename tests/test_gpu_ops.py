@@ -1586,7 +1586,10 @@ class TestFusedProjections:
 
 
 class TestOnePartProducts:
-    @pytest.mark.parametrize("K,M", [(512, 8196), (576, 10304), (2048, 8260), (2048, 16384), (4096, 12284)])
+    @pytest.mark.parametrize("K,M", [
+        (512, 8196), (576, 10304), (2048, 8260), (2048, 16384), (2112, 12228), (3072, 14340),
+        (4096, 12284), (4608, 16384),
+    ])
     @pytest.mark.parametrize("N", [65, 97, 128])
     def test_linear(self, dev, N, K, M):
         """The first and last widths of the rule, rows of another stride, features and
@@ -1609,7 +1612,7 @@ class TestOnePartProducts:
 class TestBiasedProducts:
     @pytest.mark.parametrize("N,K,M", [
         (1, 64, 8200), (1, 2048, 13376), (17, 4096, 8264), (64, 2048, 13376), (8, 8192, 10248),
-        (65, 512, 8200), (128, 2048, 13376), (100, 4096, 12296),
+        (65, 512, 8200), (128, 2048, 13376), (100, 4096, 12296), (77, 4544, 16376),
     ])
     def test_linear(self, dev, N, K, M):
         """One part of K and several, last tiles with features past the end, rows of
