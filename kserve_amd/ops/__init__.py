@@ -414,12 +414,15 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     75), up to 64 rows but for wide ones with rows off a multiple of 4 KB (k 5120, m
     27648 68 / 55). So far a row's
     sums do not depend on the rows beside it, and small weights stay here for
-    that. The widest stay to 112 rows (k 4096, m 32000 at 64 / 80 / 96 / 112 rows 50 / 51,
-    48 / 63, 49 / 53, 55 / 73, m 16384 at 80 / 112 33 / 36, 36 / 38, k 2048, m 32000 at 96
-    rows 27 / 35; but m 16384 22 / 19), and at k 2048 to 128 where their tiles of 128
-    features fill seven eighths of the units' last round (at 128 rows m 32000 30 / 32, in
-    a captured step 41 / 50, m 65536 60 / 71, m 128256 127 / 133; but m 24576 29 / 28, m
-    50304 57 / 54).
+    that. The widest with rows a multiple of 4 KB apart, which keep the library's blocks on
+    the same memory channels and not the kernel's, stay to 112 rows (k 4096, m 32000 at 65 /
+    80 / 96 / 112 rows 44 / 61, 45 / 67, 45 / 61, 54 / 75, m 16384 at 65 / 96 30 / 33, 32 / 34,
+    k 2048, m 32000 at 96 26 / 34; but m 16384 22 / 19), and at k 2048 to 128 where their
+    tiles of 128 features fill seven eighths of the units' last round (at 128 rows m 32000
+    31 / 35, captured steps of 128 sequences with it 824 / 837, m 65536 64 / 71, 98304 99 / 108,
+    128256 129 / 127; but m 24576 30 / 28, 50304 59 / 52). Not so at longer k: k 4096, m 32000
+    54 / 61 by itself, but captured steps 759 / 753, m 128256 236 / 231, k 6144, m 62464 162 /
+    159, k 8192, m 65536 226 / 198.
     Otherwise it gains above where the
     library does not split K over the chip: k 14336, m 4096 at 128 / 256 rows 34 / 74,
     46 / 62, k 8192, m 2048 at 77 / 256 rows 15 / 21, 21 / 27, k 4096, m 4096 at 128
