@@ -443,7 +443,7 @@ void skinny_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
 
 void skinny_clamped_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w, double alpha,
                         double limit) {
-  // out [N, M] = clamped gate and up of x @ w^T, bf16, N <= 256
+  // out [N, M] = clamped gate and up of x @ w^T, bf16, N <= 64
   CHECK_BF16_CONTIG(out);
   const SkinnyShape z = skinny_shape(x, w, 2);
   TORCH_CHECK(out.dim() == 2 && out.size(0) == z.N && out.size(1) == z.M &&
@@ -639,7 +639,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "few-row qkv GEMM, rotary embedding and K/V scatter");
   m.def("skinny_glu", &skinny_glu, "gate|up GEMM (N<=256) with silu(gate) * up");
   m.def("skinny_clamped_glu", &skinny_clamped_glu,
-        "gate|up GEMM (N<=256) with the clamped gate");
+        "gate|up GEMM (N<=64) with the clamped gate");
   m.def("dense_gemm", &dense_gemm, "GEMM with bias and, if asked for, erf GELU",
         pybind11::arg("out"), pybind11::arg("x"), pybind11::arg("w"),
         pybind11::arg("bias"), pybind11::arg("gelu"), pybind11::arg("tile") = -1);

@@ -251,11 +251,13 @@ __global__ __launch_bounds__(256) void reduce_splits_kernel(
 
 // token tiles, feature groups per wave and ring slots: two blocks per compute
 // unit up to 64 tokens, one with twice the features above
-#define FOR_TILE(N, GO)                 \
+#define FOR_FEW(N, GO)                  \
   if ((N) <= 16) GO(1, 1, 8)            \
   else if ((N) <= 32) GO(2, 1, 6)       \
   else if ((N) <= 48) GO(3, 1, 5)       \
-  else if ((N) <= 64) GO(4, 1, 5)       \
+  else if ((N) <= 64) GO(4, 1, 5)
+#define FOR_TILE(N, GO)                 \
+  FOR_FEW(N, GO)                        \
   else if ((N) <= 96) GO(6, 2, 5)       \
   else if ((N) <= 128) GO(8, 2, 5)      \
   else if ((N) <= 192) GO(12, 2, 4)     \
@@ -365,11 +367,11 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
 // silu-like gate within limits (CLAMPED above), gate and up of w [2 M][K]. The
 // activation kernel and its launch take 3.5 us of a decode layer, and the sums reach
 // it in 32 bits (hybrid step of 4 layers at 1 / 8 / 24 / 64 sequences 345 -> 342, 380 ->
-// 375, 446 -> 435, 652 -> 642 us).
+// 375, 446 -> 435, 652 -> 642 us). Up to 64 rows: above, the library has the product.
 extern "C" hipError_t ks_skinny_clamped_glu(void* out, const void* x, const void* w, int M,
                                             int K, int N, long xs, float alpha,
                                             float limit, hipStream_t stream) {
-  if (N < 1 || N > 256 || M < 1 || M % 4 != 0 || K < BK || K % BK != 0 || xs % 8 != 0 ||
+  if (N < 1 || N > 64 || M < 1 || M % 4 != 0 || K < BK || K % BK != 0 || xs % 8 != 0 ||
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
     return hipErrorInvalidValue;
   const GemmArgs p{out, (const short*)x, (const short*)w, M, K, N, xs, alpha, limit, nullptr};
@@ -377,7 +379,7 @@ extern "C" hipError_t ks_skinny_clamped_glu(void* out, const void* x, const void
   const dim3 grid((M + bm - 1) / bm, 1);
 #define GO(nt, f, s)                                                                     \
   hipLaunchKernelGGL((skinny_gemm_kernel<nt, f, s, CLAMPED>), grid, dim3(256), 0, stream, p);
-  FOR_TILE(N, GO)
+  FOR_FEW(N, GO)
 #undef GO
   HIP_CHECK_KERNEL();
   return hipSuccess;
