@@ -112,7 +112,7 @@ __global__ void qk_norm_temp_cache_kernel(
 // elements a thread, and one exchange gives both sums. Element by element, with the two
 // sums and the three rows one after the other, the loads' latency bound it (us, 16 / 4
 // heads of 128: 8000 tokens 39.7 -> 22.4 = 5.8 TB/s, 500 6.6 -> 4.5, 128 5.7 -> 3.6).
-template <int VQ, int VK>  // chunks a thread has of q; of k and of v
+template <int VQ>  // chunks of q a thread has; one of k and of v
 __global__ __launch_bounds__(NT) void qk_norm_temp_cache_vec8_kernel(
     float* __restrict__ q_out, const short* __restrict__ q, const short* __restrict__ k,
     const short* __restrict__ v, long row_stride, const float* __restrict__ qw,
@@ -124,18 +124,14 @@ __global__ __launch_bounds__(NT) void qk_norm_temp_cache_vec8_kernel(
   const long t = blockIdx.x;
   const int k_width = kv_heads * D, v_width = kv_heads * DV;
   const short8_t zero = short8_t{};
-  short8_t xq[VQ], xk[VK], xv[VK];
+  short8_t xq[VQ];
   auto load = [&](const short* row, int u, int width) {
     const int i = (threadIdx.x + u * NT) * 8;
     return i < width ? *reinterpret_cast<const short8_t*>(row + t * row_stride + i) : zero;
   };
 #pragma unroll
   for (int u = 0; u < VQ; ++u) xq[u] = load(q, u, q_width);
-#pragma unroll
-  for (int u = 0; u < VK; ++u) {
-    xk[u] = load(k, u, k_width);
-    xv[u] = load(v, u, v_width);
-  }
+  const short8_t xk = load(k, 0, k_width), xv = load(v, 0, v_width);
   const long pos = positions[t], slot = slot_mapping[t];
   float sq = 0.f, sk = 0.f;
 #pragma unroll
@@ -145,11 +141,8 @@ __global__ __launch_bounds__(NT) void qk_norm_temp_cache_vec8_kernel(
       const float x = bf16_bits_to_float(xq[u][j]);
       sq += x * x;
     }
-#pragma unroll
-    for (int u = 0; u < VK; ++u) {
-      const float x = bf16_bits_to_float(xk[u][j]);
-      sk += x * x;
-    }
+    const float x = bf16_bits_to_float(xk[j]);
+    sk += x * x;
   }
   sq = wave_reduce_sum(sq);
   sk = wave_reduce_sum(sk);
@@ -186,21 +179,18 @@ __global__ __launch_bounds__(NT) void qk_norm_temp_cache_vec8_kernel(
   auto row_of = [&](int head, int dim) {
     return ((blk * kv_heads + head) * block_size + off) * dim;
   };
+  const int i = threadIdx.x * 8;
+  if (i < k_width) {
+    const int g = i / D;
+    short8_t o;
 #pragma unroll
-  for (int u = 0; u < VK; ++u) {
-    const int i = (threadIdx.x + u * NT) * 8;
-    if (i < k_width) {
-      const int g = i / D;
-      short8_t o;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        o[j] = float_to_bf16_bits(bf16_bits_to_float(xk[u][j]) * kw[i + j] * kinv);
-      *reinterpret_cast<short8_t*>(k_cache + row_of(g, D) + i - g * D) = o;
-    }
-    if (i < v_width) {
-      const int g = i / DV;
-      *reinterpret_cast<short8_t*>(v_cache + row_of(g, DV) + i - g * DV) = xv[u];
-    }
+    for (int j = 0; j < 8; ++j)
+      o[j] = float_to_bf16_bits(bf16_bits_to_float(xk[j]) * kw[i + j] * kinv);
+    *reinterpret_cast<short8_t*>(k_cache + row_of(g, D) + i - g * D) = o;
+  }
+  if (i < v_width) {
+    const int g = i / DV;
+    *reinterpret_cast<short8_t*>(v_cache + row_of(g, DV) + i - g * DV) = xv;
   }
 }
 
@@ -906,7 +896,7 @@ extern "C" hipError_t ks_qk_norm_temp_cache(
            (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)qw |
              (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16) == 0) {
 #define GO(VQ)                                                                         \
-  hipLaunchKernelGGL((qk_norm_temp_cache_vec8_kernel<VQ, 1>), dim3(tokens), dim3(NT),  \
+  hipLaunchKernelGGL((qk_norm_temp_cache_vec8_kernel<VQ>), dim3(tokens), dim3(NT),  \
                      0, stream, (float*)q_out, (const short*)q, (const short*)k,       \
                      (const short*)v, row_stride, (const float*)qw, (const float*)kw,  \
                      (const long*)positions, (const int*)slot_mapping,                 \
