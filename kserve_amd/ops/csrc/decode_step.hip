@@ -5,7 +5,9 @@
 // in place of 15 launches of 4.4 us. The rows may lie in pinned host memory, where
 // the kernel reads them itself. The copy ahead of it, and the wait between the two,
 // took up to 16 us of a step (us, copied / read in place: 1 row 449.3 / 449.0, 24
-// rows 532.8 / 530.6, 96 1031 / 1015, 256 2312 / 2297).
+// rows 532.8 / 530.6, 96 1031 / 1015, 256 2312 / 2297). Wide tables are bound by the bus
+// either way (alone, 96 rows of 4096 pages 47 / 32, 256 of 4096 93 / 80, 2048 of 4096, 33
+// MB, 623 / 608), so that no size goes back to the copy.
 #include "common.h"
 #include "decode_step.h"
 
