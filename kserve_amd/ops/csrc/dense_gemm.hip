@@ -383,12 +383,13 @@ static bool mid_narrow(int M, int K) { return M <= 4096 && K <= 8192; }
 // / 14.8; K 1984, M 10304 13.1 / 15.9 / 21.0, 16.0 / 20.4 / 21.7; K 2304, M 12288 15.4 / 19.2 /
 // 17.6, 18.9 / 24.6 / 20.5; K 3072, M 16384 21.3 / 25.0 / 24.0, 26.6 / 30.8 / 27.2; K 4096, M
 // 14336 25.3 / 28.0 / 30.5, 29.9 / 35.2 / 33.0; K 4608, M 16384 29.9 / 33.6 / 32.7, 36.6 / 40.2 /
-// 36.8. Not at 128 tiles or fewer (K 1792, M 6144 11.1 / 14.1 / 12.2, 12.8 / 17.9 / 14.0, but
-// K 2048, M 8192 at 128 rows 16.9 / 18.8 / 15.7), nor where K is long and a quarter of the
-// units idle (K 4096, M 10304 23.9 / 22.9 / 38.3, 28.3 / 28.6 / 30.8), nor past K 4608, where
-// it turns (K 5120, M 12288 at 65 / 112 rows 32.3 / 34.2 / 33.6, 37.5 / 41.1 / 35.7, M 16384 at
-// 128 43.7 / 44.9 / 41.6); past 256 tiles a second round is nearly empty (K 2048, M 17408
-// 26.4 / 23.3 / 27.5).
+// 36.8. Not past K 4608, where it turns (K 5120, M 12288 at 65 / 112 rows 32.1 / 33.9 / 33.3,
+// 37.5 / 39.9 / 36.0, M 16384 at 128 43.9 / 44.9 / 41.5), nor where K is long and a quarter of
+// the units idle (K 4096, M 10304 23.8 / 22.4 / 38.7, 28.2 / 28.4 / 30.6); past 256 tiles a
+// second round is nearly empty (K 2048, M 17408 26.4 / 23.3 / 27.5). The line at 129 tiles is
+// from weights that came through the caches (K 2048, M 8192 at 128 rows 16.9 / 18.8 / 15.7);
+// as they are loaded now these are ahead at 128 too (14.8 / 18.2 / 15.8, K 512 6.5 / 14.3 /
+// 9.9), and it could be lower.
 static bool mid_wide(int M, int K, int N) {
   const int tiles = (M + 63) / 64;
   return N > 64 && N <= 128 && tiles <= UNITS && K >= 512 && K <= 4608 &&
