@@ -63,7 +63,7 @@ MODULES = {
 }
 
 HEADERS = ["common.h", "mfma_layouts.h", "dtype_io.h", "cache_chunk.h",
-           "mfma_attention.h", "decode_step.h"]
+           "mfma_attention.h", "decode_step.h", "gemm_tile.h"]
 # hipcc makes packed-fp32 instructions on its own from plain float code; keep
 # them off for every kernel of this package
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

@@ -500,6 +500,47 @@ def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     return m >= 4608 and (n <= 48 or m <= 8192 or m >= 10240)
 
 
+def _streamed_rows(n: int, k: int, m: int) -> bool:
+    """Wide products of 49 to 256 rows that the rules above leave to the library and the
+    few-row kernel's tiles of all rows take sooner, with a bias or without (MI355X, us,
+    kernel / library): k 1024, m 12288 at 65 / 256 rows 8.6 / 14.4, 15.2 / 16.8, k 2048, m
+    10304 at 64 / 129 / 256 13.2 / 15.5, 18.0 / 17.6, 25.3 / 27.0, m 16384 at 129 / 256 20.3 /
+    25.8, 26.7 / 28.8, m 32000 at 128 / 192 28.8 / 33.7, 32.8 / 39.2, k 4096, m 12288 at 65 /
+    256 26.5 / 29.6, 42.5 / 48.6, m 32000 at 128 / 256 53.8 / 63.6, 70.0 / 79.6, k 8192, m
+    16384 54 / 66, 85 / 102, m 28672 82 / 115, 128 / 146. Past 16384 features where they come
+    to five eighths of the units at least, and where rows lie a multiple of 4 KB apart or
+    are short (k 5120, m 28672 at 96 / 128 rows 66 / 65, 73 / 71; k 14336, m 20480 at 128 169 /
+    157). Up to 64 rows on short k or full rounds only (k 4096, m 12288 at 33 rows 26.7 /
+    25.2)."""
+    if m % 4 or not 48 < n <= 256 or k < 1024:
+        return False
+    if n <= 64:
+        return 8192 < m <= 16384 and (k <= 2048 or m > 12288 and k <= 5120)
+    if m <= 16384:
+        return m > 8192
+    return 20352 < m <= 32768 and k <= 8192 and (k <= 4096 or k % 4096 == 0)
+
+
+def _streamed_glu_rows(n: int, k: int, m: int) -> bool:
+    """The same for gate|up products, whose activation comes with them (without the
+    library's 3 to 6 us for it): k 4096, m 14336 at 64 / 128 / 192 / 256 rows 42.8 / 53.3,
+    51.1 / 57.3, 60.6 / 68.9, 67.9 / 74.4, k 2048, m 4096 at 33 / 96 / 256 11.0 / 13.4, 14.6 /
+    14.4, 24.1 / 24.6, m 8192 at 128 / 256 18.5 / 20.9, 27.1 / 29.3, k 4096, m 5504 at 65 / 256
+    24.0 / 28.2, 44.8 / 48.4, k 5120, m 13824 at 64 / 128 / 256 56.5 / 59.1, 71 / 70, 85 / 92, k
+    8192, m 7168 at 33 / 128 / 256 41.6 / 49.7, 62 / 68, 89 / 95, m 14336 at 49 / 128 / 256 78 /
+    103, 98 / 112, 128 / 141. Level or behind below 4096 features (k 4096, m 3584 at 128 rows
+    28.1 / 25.9) and past 16384, where they take two rounds (k 3584, m 18944 at 128 83 /
+    74)."""
+    return m % 4 == 0 and 32 < n <= 256 and k >= 1024 and 4096 <= m <= 16384
+
+
+def _streamed_parts(n: int, k: int, m: int) -> bool:
+    """The same where the sums over parts of k stay in 32 bits for the next kernel to add
+    (us, their writing, library): k 2048, m 4096 at 65 / 128 / 256 rows 6.7 / 12.3, 8.3 / 14.6,
+    11.8 / 13.3, m 8192 at 129 / 256 13.4 / 15.2, 18.1 / 24.4, k 4096, m 4096 at 256 17.9 / 22.4."""
+    return m % 4 == 0 and 64 < n <= 256 and k >= 2048 and 4096 <= m <= 8192
+
+
 def _dense_rows(n: int, k: int, m: int, gelu: bool) -> bool:
     """Whether the encoder kernel beats the library at [n, k] x [m, k]^T + bias
     (MI355X, us, kernel / library).
@@ -584,10 +625,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         type(x) in _TENSORS
         and x.dim() == 2
         and (
-            _biased_rows(x.shape[0], x.shape[1], m)
-            if bias is not None
-            else _skinny_rows(x.shape[0], x.shape[1], m)
-            or _one_part_rows(x.shape[0], x.shape[1], m)
+            (
+                _biased_rows(x.shape[0], x.shape[1], m)
+                if bias is not None
+                else _skinny_rows(x.shape[0], x.shape[1], m)
+                or _one_part_rows(x.shape[0], x.shape[1], m)
+            )
+            or _streamed_rows(x.shape[0], x.shape[1], m)
+            and (bias is None or m % 8 == 0)
         )
         and _skinny_operands(x, weight)
         and (bias is None or _plain_bias(bias, m, x))
@@ -613,6 +658,7 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         and (
             _skinny_rows(n, k, m)
             or n <= 256 and m % 4 == 0 and 2048 <= m < 4096 and 2048 <= k < 1 << 22
+            or _streamed_parts(n, k, m)
         )
         and _skinny_operands(x, weight)
     ):
@@ -635,7 +681,10 @@ def linear_silu_and_mul(
         bias is None
         and x.dim() == 2
         and weight.shape[0] % 2 == 0
-        and _skinny_glu_rows(x.shape[0], x.shape[1], weight.shape[0] // 2)
+        and (
+            _skinny_glu_rows(x.shape[0], x.shape[1], weight.shape[0] // 2)
+            or _streamed_glu_rows(x.shape[0], x.shape[1], weight.shape[0] // 2)
+        )
         and _skinny_operands(x, weight)
     ):
         out = torch.empty(
@@ -649,19 +698,22 @@ def linear_silu_and_mul(
 def linear_clamped_swiglu(
     x: torch.Tensor, weight: torch.Tensor, alpha: float, limit: float
 ) -> torch.Tensor:
-    """``clamped_swiglu`` of [gate | up] = x @ weight^T. Up to 64 rows, where the product
-    of both is the few-row kernel's either way, on its sums in 32 bits."""
+    """``clamped_swiglu`` of [gate | up] = x @ weight^T, on the sums in 32 bits where the
+    few-row kernel takes the product."""
     m = weight.shape[0] // 2
     if (
         x.dim() == 2
-        and x.shape[0] <= 64
         and weight.shape[0] % 2 == 0
-        and _skinny_glu_rows(x.shape[0], x.shape[1], m)
-        and _skinny_rows(x.shape[0], x.shape[1], 2 * m)
+        and (
+            x.shape[0] <= 64
+            and _skinny_glu_rows(x.shape[0], x.shape[1], m)
+            and _skinny_rows(x.shape[0], x.shape[1], 2 * m)
+            or _streamed_glu_rows(x.shape[0], x.shape[1], m)
+        )
         and _skinny_operands(x, weight)
     ):
         out = torch.empty((x.shape[0], m), dtype=x.dtype, device=x.device)
-        _C.skinny_clamped_glu(out, x, weight, float(alpha), float(limit))
+        _C.streamed_clamped_glu(out, x, weight, float(alpha), float(limit))
         return out
     return clamped_swiglu(linear(x, weight), alpha, limit)
 
@@ -676,7 +728,10 @@ def linear_add_rms_norm(
     if (
         m <= 16384
         and x.dim() == 2
-        and _skinny_rows(x.shape[0], x.shape[1], m)
+        and (
+            _skinny_rows(x.shape[0], x.shape[1], m)
+            or _streamed_parts(x.shape[0], x.shape[1], m)
+        )
         and _skinny_operands(x, weight)
         and residual.shape == (x.shape[0], m)
         and norm_weight.shape == (m,)

@@ -95,6 +95,46 @@ def test_few_row_gate_up(n, k, m, own):
 
 
 @pytest.mark.parametrize(
+    "n,k,m,own",
+    [
+        (48, 2048, 10304, False), (49, 2048, 10304, True), (64, 4096, 12288, False),
+        (64, 4096, 14336, True), (64, 5184, 14336, False), (65, 14336, 12288, True),
+        (65, 1024, 8192, False), (65, 1024, 8196, True), (256, 960, 16384, False),
+        (256, 2048, 16384, True), (257, 2048, 16384, False), (129, 2048, 16388, False),
+        (129, 2048, 20352, False), (256, 4096, 20356, True), (128, 5120, 28672, False),
+        (128, 8192, 32768, True), (128, 8192, 32772, False), (128, 12288, 28672, False),
+        (80, 2048, 10302, False),
+    ],
+)
+def test_streamed_product(n, k, m, own):
+    assert ops._streamed_rows(n, k, m) is own
+
+
+@pytest.mark.parametrize(
+    "n,k,m,own",
+    [
+        (32, 4096, 14336, False), (33, 4096, 14336, True), (256, 4096, 14336, True),
+        (257, 4096, 14336, False), (128, 4096, 4092, False), (128, 960, 8192, False),
+        (128, 2048, 4096, True), (128, 4096, 16384, True), (128, 4096, 16388, False),
+    ],
+)
+def test_streamed_gate_up(n, k, m, own):
+    assert ops._streamed_glu_rows(n, k, m) is own
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 96, 97, 128, 129, 192, 193, 256])
+def test_parts_of_streamed_products(native, n):
+    """Parts of K: at least four steps in each, one where the next kernel takes no sums,
+    and up to 64 rows as many for every row count."""
+    for k in (64, 128, 256, 1088, 4096, 14336, 1 << 22):
+        for m in (4, 68, 1024, 4096, 6144, 16384, 50304):
+            s = native.ks_skinny_splits(m, k, n, 0)
+            assert 1 <= s <= 16 and (s == 1 or s * 4 <= k // 64), (m, k, s)
+            assert native.ks_skinny_splits(m, k, n, 1) == 1
+            assert n > 64 or s == native.ks_skinny_splits(m, k, 1, 0)
+
+
+@pytest.mark.parametrize(
     "lens,heads,P,N,chunks",
     [
         ([15], 64, 64, 128, False), ([16] * 4, 64, 64, 128, True),

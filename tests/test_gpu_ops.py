@@ -1313,6 +1313,31 @@ class TestSkinnyGemmEdges:
         ref = sum(a.double() @ b.double().t() for a, b in zip(x.split(1 << 18, 1), w.split(1 << 18, 1)))
         assert ((out.double() - ref).abs() <= ref.abs() * 2.0**-8).all()
 
+    @pytest.mark.parametrize("N", [17, 33, 64, 65, 96, 97, 128, 129, 192, 193, 256])
+    @pytest.mark.parametrize("K,M,glu", [(128, 24580, False), (4096, 24580, False),
+                                         (14336, 2052, False), (128, 12292, True)])
+    def test_wide_tiles(self, dev, N, K, M, glu):
+        """The tiles of 128 features, in one part and in many."""
+        self.test_against_fp64(dev, N, K, M, glu)
+
+    @pytest.mark.parametrize("N,glu", [(3, False), (3, True), (64, True), (65, True)])
+    def test_long_rows_of_few(self, dev, N, glu):
+        import kserve_amd_C
+
+        torch.manual_seed(N)
+        K, M, stride = 192, 68, (1 << 22) + 64
+        x = torch.empty((N - 1) * stride + K, device=dev, dtype=torch.bfloat16)
+        x = x.as_strided((N, K), (stride, 1)).normal_()
+        w = torch.randn((2 if glu else 1) * M, K, device=dev).to(torch.bfloat16)
+        f = kserve_amd_C.skinny_glu if glu else kserve_amd_C.skinny_gemm
+        out, near = (torch.full((N, M), float("nan"), device=dev, dtype=torch.bfloat16)
+                     for _ in range(2))
+        f(out, x, w)
+        f(near, x.contiguous(), w)
+        # the same tiles up to 64 rows, another order of sums above
+        assert torch.equal(out, near) or N > 64
+        assert ((out.double() - near.double()).abs() <= near.double().abs() * 2.0**-7 + 1e-5).all()
+
     @pytest.mark.parametrize(
         "N,K,M", [(33, 8192, 4096), (48, 8192, 10240), (17, 3584, 18944),
                   (72, 8192, 8192), (5, 28672, 2048), (64, 2112, 768)]
@@ -1676,6 +1701,23 @@ class TestClampedProducts:
         lim = 1.2 * off[:, :M] * (u + 1).abs() + limit * off[:, M:] + 2.0 ** -20 * (g * (u + 1)).abs()
         assert ((got.double() - want).abs() <= lim + 2.0 ** -8 * want.abs()).all()
         assert y[:, :M].max() > limit and y[:, M:].min() < -limit
+
+    @pytest.mark.parametrize("K,M", [(2048, 8192), (1088, 5000)])
+    @pytest.mark.parametrize("N", [64, 65, 96, 128, 192, 256])
+    def test_more_rows(self, dev, N, K, M):
+        """Row by row what a few of them give, to the order of sums and its slopes (the
+        same bound as above, of two sums), and bit by bit up to 64 rows."""
+        from kserve_amd import ops
+
+        torch.manual_seed(N)
+        x = torch.randn(N, K, device=dev, dtype=torch.bfloat16)
+        w = (torch.randn(2 * M, K, device=dev) * K ** -0.5).to(torch.bfloat16)
+        got = ops.linear_clamped_swiglu(x, w, 1.702, 2.5)
+        few = torch.cat([ops.linear_clamped_swiglu(r, w, 1.702, 2.5) for r in x.split(32)])
+        assert torch.equal(got, few) or N > 64
+        off = K * 2.0 ** -23 * (x.double().abs() @ w.double().abs().t())
+        lim = 1.2 * 3.5 * off[:, :M] + 2.5 * off[:, M:] + 2.0 ** -19 * few.double().abs()
+        assert ((got.double() - few.double()).abs() <= lim + 2.0 ** -7 * few.double().abs()).all()
 
     @pytest.mark.parametrize("N", [6, 64])
     def test_values_past_all_limits(self, dev, N):

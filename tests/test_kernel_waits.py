@@ -149,6 +149,21 @@ def test_product_rings_count_their_loads(tmp_path):
 
 
 @pytest.mark.skipif(HIPCC is None, reason="needs hipcc")
+def test_few_row_rings_count_their_loads(tmp_path):
+    listed = compiled(os.path.join(build_hip.CSRC, "skinny_gemm.hip"), tmp_path, True)
+    listed = {n: x for n, x in listed.items() if "dense_gemm_kernel" in n}
+    # 12 tiles and 2 for long rows with four epilogues, but those of dense_gemm.hip
+    assert len(listed) == 54
+    for name, lines in listed.items():
+        tn, tm, wn, wm, slots, _ = map(int, re.findall(r"Li(\d+)E", name))
+        loads = (tn + tm) // 8 // (wn * wm)
+        lines = [re.sub(r"global_load_lds_dwordx4 (.*)", r"global_load_dwordx4 \1 lds", x)
+                 for x in lines]
+        assert sum(bool(re.search(r"\blds\b", x)) for x in lines) >= 2 * loads, name
+        assert not ring_faults(lines, loads, slots), name
+
+
+@pytest.mark.skipif(HIPCC is None, reason="needs hipcc")
 @pytest.mark.parametrize("fast_math", [False, True])
 def test_prefill_attention_waits_for_lds_loads(tmp_path, fast_math):
     src = tmp_path / "forms.hip"
