@@ -8,7 +8,8 @@
 // several splits of its context) and its waves take pairs of pages in turn,
 // each wave in LDS of its own, without a barrier: a pair's rows pass through
 // registers, and the next pair's loads are under way while one is multiplied.
-// E4M3 pages are widened (exactly) on the way. LDS-direct loads into a ring of
+// E4M3 rows stay bytes in LDS and are widened (exactly) between there and the product:
+// half the LDS, so blocks of four waves where contexts are long. LDS-direct loads into a ring of
 // two pairs were slower, the more so the shorter the contexts (500 sequences of
 // 100, 8 heads: 60 us, 39 here; 24 of 900 29 / 22; 256 of 2048 328 / 332): the
 // ring takes twice the LDS, so half the blocks were resident, and the compiler
@@ -30,7 +31,7 @@
 // wave per query head walked the pages with vector dot products): 256 sequences
 // of 2048 +- 60% tokens 741 -> 352 us (6.2 TB/s of pages), all of 2048 606 ->
 // 332 us (6.5); 512 of 576 341 -> 189 us; E4M3, 96 of 3000 268 -> 93 us, 3000 +-
-// 60% 390 -> 108 us; one of 560 12.5 -> 9.7 us, of 7000 66 -> 14.5 us; 64 / 8
+// 60% 390 -> 108 us (119 as it came to be measured, 112 now); one of 560 12.5 -> 9.7 us, of 7000 66 -> 14.5 us; 64 / 8
 // heads, 64 of 600 83 -> 29 us. Short contexts are bound by a block's fixed work
 // (about 5 us) and not by the pages: 500 of 100 tokens, 8 heads 98 -> 42 us, E4M3
 // 50 -> 31; one or two pages under one query head each are the only ones slower

@@ -64,6 +64,17 @@ struct Split3 {
   }
 };
 
+// two numbers as bf16
+struct Rounded2 {
+  unsigned int bits;
+  __device__ __forceinline__ Rounded2(float x, float y) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    bits = __builtin_bit_cast(unsigned int, __builtin_convertvector((float2_t{x, y}), bf16x2_t));
+  }
+  __device__ __forceinline__ float first() const { return __uint_as_float(bits << 16); }
+  __device__ __forceinline__ float second() const { return __uint_as_float(bits & 0xffff0000u); }
+};
+
 // what the fp32 form adds to plain attention
 struct Extra {
   const short* gate;  // [T, H] bf16 (row stride gate_stride): output * sigmoid
@@ -606,6 +617,10 @@ __device__ __forceinline__ uint4 load16_nt(const char* from) {
       uint4, __builtin_nontemporal_load(reinterpret_cast<const u4*>(from)));
 }
 
+// Waves of a block that share a context, and page pairs of a split from which on the
+// launches with four use all of them.
+constexpr int WAVES = 2, DEEP_PAIRS = 16;
+
 struct DecodeArgs {
   void* out;                // [S, H, D]
   const void* q;            // [S, H, D] bf16 (PARTS 1) or fp32, row stride sq
@@ -649,16 +664,17 @@ __device__ __forceinline__ float final_factor(const DecodeArgs& p, long tok, int
   }
 }
 
-// E4M3 pages: two waves per SIMD at least, or the compiler keeps the output in
-// accumulation registers and copies it out and back for every rescale (96 x
-// 3000 +- 60%: 114 us, 108 so; bf16 pages 353 and 360 the other way round)
+// E4M3 pages: four waves per SIMD at least, or the compiler keeps the output in
+// accumulation registers and copies it out and back for every rescale.
 template <int D, int NW, int SRC, bool WIDE, int PARTS = 1>  // WIDE: groups of 6 to 8
-__global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_attention_kernel(
+__global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 4 : 1) void paged_attention_kernel(
     const DecodeArgs p) {
   constexpr int KC = D / 32;           // contraction chunks of K Q^T
   constexpr int DB = D / 16;           // 16-column blocks of the output
   constexpr int ROWS = 2 * PAGE;       // rows of a stage (a pair of pages)
-  constexpr int STAGE = 2 * ROWS * D;  // K rows, then V rows
+  constexpr int ES = SRC == PAGES_FP8 ? 1 : 2;
+  constexpr int STAGE = ROWS * D * ES;  // shorts: K rows, then V rows
+  static_assert(SRC != PAGES_FP8 || D == 128, "E4M3 rows are 8 chunks");
   // elements per lane and load, loads per stage and tensor
   constexpr int EPL = SRC == PAGES_FP8 ? 16 : 8;
   constexpr int LPR = D / EPL;  // lanes per row
@@ -667,15 +683,18 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
 
   const int kvh = blockIdx.x, s = blockIdx.y, split = blockIdx.z;
   const int ctx = p.ctx_lens[s];
-  const Range rg = page_range(ctx, p.window, p.x.chunk, p.n_splits, NW);
+  const Range rg = page_range(ctx, p.window, p.x.chunk, p.n_splits, min(NW, WAVES));
   const int tok = token_of(p, s);
-  if (split >= rg.splits || tok < 0) return;
-  const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // waves with work: the others end here (and are not waited for at the barrier)
+  const int nw = NW > WAVES && rg.per < DEEP_PAIRS ? WAVES : NW;
+  if (split >= rg.splits || tok < 0 || wave >= nw) return;
+  const int lane = threadIdx.x & 63;
   const int col = lane & 15, g = lane >> 4;
   const int G = p.group;
   const int part = col / G;  // of the weights: high, middle, low
   const bool used = part < (WIDE ? 2 : 3);
+  const float past_hi = part > 0 ? 1.f : 0.f, past_mid = part > 1 ? 1.f : 0.f;
 
   __shared__ __attribute__((aligned(16))) short lds[NW][STAGE];
   static_assert(STAGE * 2 >= 8 * (D + 4) * 4 + 64, "merge area");
@@ -723,7 +742,6 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
   // where this lane's bytes of load i come from; rows past the context repeat
   // its last one (their weights are 0, their values finite)
   auto src = [&](const void* cache, long stride, int n, Pages pg, int i, int chunk) {
-    constexpr int ES = SRC == PAGES_FP8 ? 1 : 2;
     const bool second = i >= NI / 2;
     const int number = min(rg.first + 2 * n + (second ? 1 : 0), rg.last);
     const int row = min((i % (NI / 2)) * RPI + lrow, ctx - 1 - number * PAGE);
@@ -747,40 +765,41 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
       const int r = i * RPI + lrow;
 #pragma unroll
       for (int kv = 0; kv < 2; ++kv) {
-        short* row = &lds[wave][kv * ROWS * D + r * D];
-        const int sw = kv ? v_swz<D>(r) : k_swz<D>(r);
-        const uint4 x = raw[2 * i + kv];
-        if constexpr (SRC == PAGES_REG) {
-          *reinterpret_cast<uint4*>(row + (lchunk ^ sw) * 8) = x;
-        } else {
-          const unsigned int w[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            uint4 o;
-            o.x = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h], 1.0f, false));
-            o.y = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h], 1.0f, true));
-            o.z = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h + 1], 1.0f, false));
-            o.w = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w[2 * h + 1], 1.0f, true));
-            *reinterpret_cast<uint4*>(row + ((2 * lchunk + h) ^ sw) * 8) = o;
-          }
-        }
+        char* row = reinterpret_cast<char*>(lds[wave]) + (kv * ROWS + r) * D * ES;
+        const int sw = SRC == PAGES_FP8 ? (r >> 1) & 7 : kv ? v_swz<D>(r) : k_swz<D>(r);
+        *reinterpret_cast<uint4*>(row + (lchunk ^ sw) * 16) = raw[2 * i + kv];
       }
     }
   };
 
-  // operand addresses inside a stage (elements)
+  // Operand addresses inside a stage (bytes). E4M3 rows stay one byte an element and are
+  // widened on the way to the product.
   int kaddr[KC];
 #pragma unroll
   for (int c = 0; c < KC; ++c)
-    kaddr[c] = col * D + ((4 * c + g) ^ k_swz<D>(col)) * 8;
-  // transposing load: lane i of 16 brings key i/4, columns 4 (i%4) .. + 3 and
-  // receives column i of its four keys
-  const int vrow = g * 4 + (col >> 2);
+    kaddr[c] = SRC == PAGES_FP8
+                   ? col * D + ((2 * c + (g >> 1)) ^ (col >> 1)) * 16 + (g & 1) * 8
+                   : (col * D + ((4 * c + g) ^ k_swz<D>(col)) * 8) * 2;
+  // Transposing load: lane i of 16 brings key i/4, columns 4 (i%4) .. + 3 and
+  // receives column i of its four keys; of E4M3 key i/2, columns 8 (i%2) .. + 7 and
+  // column i of eight keys, the fragment's of both pages.
+  const int vrow = SRC == PAGES_FP8 ? (col >> 3) * PAGE + g * 4 + ((col >> 1) & 3)
+                                    : g * 4 + (col >> 2);
   int vaddr[DB];
 #pragma unroll
   for (int b = 0; b < DB; ++b)
-    vaddr[b] = ROWS * D + vrow * D +
-               ((2 * b + ((col & 3) >> 1)) ^ v_swz<D>(vrow)) * 8 + (col & 1) * 4;
+    vaddr[b] = SRC == PAGES_FP8
+                   ? (ROWS + vrow) * D + (b ^ ((vrow >> 1) & 7)) * 16 + (col & 1) * 8
+                   : (ROWS * D + vrow * D + ((2 * b + ((col & 3) >> 1)) ^ v_swz<D>(vrow)) * 8 +
+                      (col & 1) * 4) * 2;
+  auto widen = [](uint2 x) {  // eight E4M3 bytes, exactly
+    uint4 o;
+    o.x = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x.x, 1.0f, false));
+    o.y = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x.x, 1.0f, true));
+    o.z = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x.y, 1.0f, false));
+    o.w = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(x.y, 1.0f, true));
+    return __builtin_bit_cast(bf16x8_t, o);
+  };
 
   float c2 = p.scale * LOG2E;
   const bool flip = c2 < 0.f;
@@ -791,7 +810,7 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
 #pragma unroll
   for (int b = 0; b < DB; ++b) o[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  auto compute = [&](int n, const short* st) {
+  auto compute = [&](int n, const char* st) {
     f32x4_t sc[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -799,8 +818,10 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
       f32x4_t rest = sc[h];  // the products with the query's lower parts
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
-        const bf16x8_t a =
-            *reinterpret_cast<const bf16x8_t*>(st + h * PAGE * D + kaddr[c]);
+        const char* from = st + h * PAGE * D * ES + kaddr[c];
+        bf16x8_t a;
+        if constexpr (SRC == PAGES_FP8) a = widen(*reinterpret_cast<const uint2*>(from));
+        else a = *reinterpret_cast<const bf16x8_t*>(from);
         if constexpr (PARTS == 3) {
           rest = mfma16x16x32(a, qf[PARTS - 1][c], rest);
           rest = mfma16x16x32(a, qf[PARTS - 2][c], rest);
@@ -836,30 +857,57 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
     }
     const float mc = m * c2;
     bf16x8_t pf, pl;
+    if constexpr (WIDE || SRC == PAGES_FP8) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float w = __builtin_amdgcn_exp2f(sc[h][r] * c2 - mc);
-        l += w;
-        const Split3 w3(w);
-        if constexpr (WIDE) {
-          pf[h * 4 + r] = part == 0 ? w3.hi : w3.mid;
-          pl[h * 4 + r] = part == 0 ? w3.lo : (__bf16)0.f;
-        } else {
-          pf[h * 4 + r] = part == 0 ? w3.hi : part == 1 ? w3.mid : w3.lo;
+        for (int r = 0; r < 4; ++r) {
+          const float w = __builtin_amdgcn_exp2f(sc[h][r] * c2 - mc);
+          l += w;
+          const Split3 w3(w);
+          if constexpr (WIDE) {
+            pf[h * 4 + r] = part == 0 ? w3.hi : w3.mid;
+            pl[h * 4 + r] = part == 0 ? w3.lo : (__bf16)0.f;
+          } else {
+            pf[h * 4 + r] = part == 0 ? w3.hi : part == 1 ? w3.mid : w3.lo;
+          }
         }
+    } else {
+      // a lane's part by two factors of its own, two weights to a conversion: half of
+      // what forming all three and choosing takes (weights are 0 to 1 or NaN; for E4M3
+      // the factors' registers are spilled, and scratch costs 1.3 us a launch)
+      unsigned int u[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float x = __builtin_amdgcn_exp2f(sc[i >> 1][(i & 1) * 2] * c2 - mc);
+        const float y = __builtin_amdgcn_exp2f(sc[i >> 1][(i & 1) * 2 + 1] * c2 - mc);
+        l += x;
+        l += y;
+        const Rounded2 hi(x, y);
+        const float x1 = __builtin_fmaf(-past_hi, hi.first(), x);
+        const float y1 = __builtin_fmaf(-past_hi, hi.second(), y);
+        const Rounded2 mid(x1, y1);
+        u[i] = Rounded2(__builtin_fmaf(-past_mid, mid.first(), x1),
+                        __builtin_fmaf(-past_mid, mid.second(), y1)).bits;
       }
+      pf = __builtin_bit_cast(bf16x8_t, uint4{u[0], u[1], u[2], u[3]});
+    }
 #pragma unroll
     for (int b = 0; b < DB; ++b) {
-      typedef __attribute__((address_space(3))) s16x4_t lds4_t;
-      const short* a0 = st + vaddr[b];
       union {
         s16x4_t h[2];
         bf16x8_t v;
       } a;
-      a.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)a0);
-      a.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)(a0 + PAGE * D));
+      const char* a0 = st + vaddr[b];
+      if constexpr (SRC == PAGES_FP8) {
+        typedef int i2_t __attribute__((ext_vector_type(2)));
+        typedef __attribute__((address_space(3))) i2_t lds2_t;
+        a.v = widen(__builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds2_t*)a0)));
+      } else {
+        typedef __attribute__((address_space(3))) s16x4_t lds4_t;
+        a.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)a0);
+        a.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4_t*)(a0 + PAGE * D * 2));
+      }
       o[b] = mfma16x16x32(a.v, pf, o[b]);
       if constexpr (WIDE) o[b] = mfma16x16x32(a.v, pl, o[b]);
     }
@@ -869,10 +917,10 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
   const int n_hi = min((split + 1) * rg.per, rg.pairs);
   if (n_lo < n_hi) load(n_lo);
   // the next pair's loads are under way while this one is multiplied
-  for (int n = n_lo; n < n_hi; n += NW) {
+  for (int n = n_lo; n < n_hi; n += nw) {
     commit();
-    if (n + NW < n_hi) load(n + NW);
-    compute(n, lds[wave]);
+    if (n + nw < n_hi) load(n + nw);
+    compute(n, reinterpret_cast<const char*>(lds[wave]));
   }
 
   // ---- merge: the parts of the weights, then the waves ----
@@ -897,15 +945,17 @@ __global__ __launch_bounds__(NW * 64, SRC == PAGES_FP8 ? 2 : 1) void paged_atten
   __syncthreads();
   constexpr int WF = STAGE / 2;  // floats between the waves' areas
   const float* all = reinterpret_cast<const float*>(lds);
-  for (int i = threadIdx.x; i < G * (D / 4); i += NW * 64) {
+  for (int i = threadIdx.x; i < G * (D / 4); i += nw * 64) {
     const int h = i / (D / 4), d = i % (D / 4) * 4;
     float top = NO_MAX;
 #pragma unroll
-    for (int w = 0; w < NW; ++w) top = fmaxf(top, all[w * WF + 8 * (D + 4) + h]);
+    for (int w = 0; w < NW; ++w)
+      if (w < nw) top = fmaxf(top, all[w * WF + 8 * (D + 4) + h]);
     float sum = 0.f;
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
+      if (w >= nw) continue;
       const float* a = all + w * WF;
       const float f = __builtin_amdgcn_exp2f((a[8 * (D + 4) + h] - top) * c2);
       sum += f * a[8 * (D + 4) + 8 + h];
@@ -937,7 +987,7 @@ __global__ __launch_bounds__(256) void paged_attention_reduce_kernel(
   const int lane = threadIdx.x & 63;
   if (sh >= total) return;
   const int s = sh / p.H;
-  const Range rg = page_range(p.ctx_lens[s], p.window, p.x.chunk, p.n_splits, NW);
+  const Range rg = page_range(p.ctx_lens[s], p.window, p.x.chunk, p.n_splits, min(NW, WAVES));
   const int tok = token_of(p, s);
   if (rg.splits == 1 || tok < 0) return;
   const float* ml = p.part_ml + sh * p.n_splits * 2;
@@ -977,7 +1027,6 @@ __global__ __launch_bounds__(256) void paged_attention_reduce_kernel(
 // 16 heads 58 / 52; 256 of 16, 32 / 8 heads 16 / 12; level at 1024 blocks). Above,
 // the longest sequence's block takes its time (400 +- 60% of 4096 blocks 4% to
 // 10% slower).
-constexpr int WAVES = 2;
 constexpr long ONE_WAVE_BLOCKS = 2048;
 
 template <int D, int SRC, int PARTS, int NW>
@@ -991,13 +1040,30 @@ void launch_decode_waves(const DecodeArgs& p, int num_seqs, hipStream_t stream) 
                        dim3(NW * 64), 0, stream, p);
 }
 
+// E4M3 pages: four waves, two of which end at once where a split has few pairs. Its
+// stages are half as large, so that four take the LDS of two, and long contexts among
+// short ones end sooner (us, 2 / 4 waves: 96 of 3000 +- 60% 114.2 / 109.3, 192 of 1500
+// 101.8 / 95.4, 250 of 1000 +- 60% 102.6 / 97.5, of 150 20.3 / 22.0; before, with stages
+// widened in LDS, 119, 113, 104 and 22.3). Not past 4096 blocks (1000 of 16 tokens 23.5 /
+// 35.2) nor in many splits, which are short (one of 2000 8.6 / 8.9).
+constexpr long MOST_DEEP_BLOCKS = 4096;
+
 template <int D, int SRC, int PARTS = 1>
 hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) {
   const bool few = p.max_blocks <= (SRC == PAGES_FP8 ? 8 : 4);
-  if (few && p.n_splits == 1 && (long)num_seqs * p.Hkv >= ONE_WAVE_BLOCKS)
+  const long blocks = (long)num_seqs * p.Hkv;
+  if (few && p.n_splits == 1 && blocks >= ONE_WAVE_BLOCKS) {
     launch_decode_waves<D, SRC, PARTS, 1>(p, num_seqs, stream);
-  else
-    launch_decode_waves<D, SRC, PARTS, WAVES>(p, num_seqs, stream);
+  } else {
+    if constexpr (SRC == PAGES_FP8) {
+      if (p.n_splits <= 2 && blocks < MOST_DEEP_BLOCKS)
+        launch_decode_waves<D, SRC, PARTS, 2 * WAVES>(p, num_seqs, stream);
+      else
+        launch_decode_waves<D, SRC, PARTS, WAVES>(p, num_seqs, stream);
+    } else {
+      launch_decode_waves<D, SRC, PARTS, WAVES>(p, num_seqs, stream);
+    }
+  }
   HIP_CHECK_KERNEL();
   if (p.n_splits > 1) {
     const long sh = (long)num_seqs * p.H;

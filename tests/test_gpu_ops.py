@@ -295,6 +295,11 @@ class TestDecodeAttention:
             assert (err <= 2 ** -8 * ref.abs() + 1e-5).all(), float(err.max())
             assert err.norm() < 2 ** -9 * ref.norm()
 
+    @pytest.mark.parametrize("H,window", [(4, 0), (3, 50)])
+    def test_e4m3_of_many_blocks(self, dev, H, window):
+        """Past 4096 blocks E4M3 pages go back to blocks of two waves."""
+        self.test_paged_decode_edges(dev, H, 1, 128, window, 0, True, 400)
+
     @pytest.mark.parametrize("window", [0, 20])
     @pytest.mark.parametrize(
         "H,Hkv,D,fp8", [(4, 4, 128, False), (8, 1, 128, False), (6, 3, 64, False),
