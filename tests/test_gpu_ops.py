@@ -300,6 +300,49 @@ class TestDecodeAttention:
         """Past 4096 blocks E4M3 pages go back to blocks of two waves."""
         self.test_paged_decode_edges(dev, H, 1, 128, window, 0, True, 400)
 
+    @pytest.mark.parametrize("H,Hkv,window", [(4, 1, 0), (8, 1, 0), (6, 2, 768), (6, 2, 767)])
+    def test_four_waves_per_block(self, dev, H, Hkv, window):
+        """bf16 pages in blocks of four waves, two of which end at once where a context
+        has fewer than four page pairs, in both precisions of the scores; a window that
+        is a token shorter than fp32 queries take four from."""
+        from kserve_amd import ops
+
+        D, ctx = 128, [1, 32, 96, 97, 112, 113, 128, 129, 160, 161, 767, 780, 1553]
+        torch.manual_seed(H)
+        width = -(-max(ctx) // 16)
+        NB = len(ctx) * width
+        kc, vc = (torch.randn(NB, Hkv, 16, D, device=dev).to(torch.bfloat16) for _ in "kv")
+        bt = torch.randperm(NB).view(len(ctx), width).to(torch.int32)
+        for row, c in zip(bt.long(), ctx):
+            for x in (kc, vc):  # rows that no sequence owns
+                x[row[-(-c // 16) :]] = float("nan")
+                if c % 16:
+                    x[row[c // 16], :, c % 16 :] = float("nan")
+        ctx_t = torch.tensor(ctx, dtype=torch.int32)
+        q = (torch.randn(len(ctx), H, D, device=dev) * 1.5).to(torch.bfloat16)
+        ref = torch_ref.paged_attention_decode(
+            q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt, ctx_t,
+            D ** -0.5, window=window,
+        )
+        n = -(-512 // (len(ctx) * Hkv))
+        many = [x.to(dev) for x in (bt.repeat(n, 1), ctx_t.repeat(n))]
+        got = ops.paged_attention_decode(
+            q.repeat(n, 1, 1), kc, vc, *many, D ** -0.5, window=window
+        )
+        for part in got.float().cpu().split(len(ctx)):
+            # fp32 weights and sums, the output rounded to bf16
+            err = (part - ref).abs()
+            assert (err <= 2 ** -8 * ref.abs() + 1e-5).all(), float(err.max())
+        cu = torch.arange(n * len(ctx) + 1, dtype=torch.int32, device=dev)
+        got = ops.ctx_attention_f32(
+            q.float().reshape(len(ctx), -1).repeat(n, 1), kc, vc, many[0], cu, many[1],
+            D ** -0.5, 1, H, window=window,
+        )
+        for part in got.cpu().split(len(ctx)):
+            # fp32 sums of 1553 terms on both sides: sqrt(1553) roundings of 2^-24
+            err = (part - ref.reshape(len(ctx), -1)).norm() / ref.norm()
+            assert err < 2.4e-6, float(err)
+
     @pytest.mark.parametrize("window", [0, 20])
     @pytest.mark.parametrize(
         "H,Hkv,D,fp8", [(4, 4, 128, False), (8, 1, 128, False), (6, 3, 64, False),
