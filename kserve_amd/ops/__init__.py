@@ -577,6 +577,31 @@ def _dense_rows(n: int, k: int, m: int, gelu: bool) -> bool:
     return k <= 1024 and n <= 3584 and (gelu or work <= 5.8e9)
 
 
+def _dense_round(n: int, k: int, m: int) -> bool:
+    """Whether one round of the encoder kernel's largest tiles holds the product and the
+    kernel beats the library (MI355X, device us, kernel / library; without a bias too).
+
+    By a tenth to a third as a rule (k 512, m 2304 at 2600 / 3500 rows 10.9 / 14.0, 12.8 /
+    16.2; k 1024, m 1024 at 8000 18.2 / 20.2; k 1536, m 1536 at 3000 18.0 / 22.9; k 2048, m
+    2048 at 800 / 2000 / 4000 13.9 / 15.6, 17.9 / 21.7, 30.4 / 33.2, m 256 at 8192 14.1 / 20.9,
+    at 32000 41.4 / 41.1; k 3072, m 768 at 2000 / 4600 / 7000 / 9800 17.9 / 19.3, 23.4 / 28.5,
+    31.4 / 36.8, 40.6 / 45.7, with the rows not in a cache at 7864 40 / 43; k 4096, m 1024 at
+    1400 / 8000 22.3 / 22.9, 54.6 / 58.7, m 2048 at 2600 43 / 50). Few rows of a long k leave
+    units idle where the library splits it (k 4096, m 256 at 768 13.4 / 10.5; m 128 at 2000
+    11.1 / 9.2). On wider ones the library's times turn from one size to the next (k 2048, m
+    3072 at 768 / 1280 / 2048 16.4 / 19.3, 24.4 / 21.1, 28.7 / 27.7; k 768, m 4096 at 1400 / 1872
+    14.0 / 18.5, 19.3 / 17.4; k 4096, m 4096 at 1400 50 / 50), on longer k too (k 8192, m 2048
+    at 768 / 2600 45 / 39, 81 / 93), and past one round its tiles are ahead (k 2048, m 768 at
+    10900 rows 37 / 33, k 3072 58 / 52)."""
+    return (
+        m % 8 == 0
+        and 256 <= m <= 2304
+        and 512 <= k <= 4096
+        and n >= (1024 if k > 2048 else 1)
+        and -(-n // 256) * -(-m // 128) <= 256
+    )
+
+
 def _plain_bias(bias: torch.Tensor, m: int, x: torch.Tensor) -> bool:
     return (
         type(bias) in _TENSORS
@@ -594,16 +619,23 @@ def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
     """The encoder kernel's product, or None for operands that it does not take."""
     m = weight.shape[0]
     if not (
-        bias is not None
-        and _direct(x)
+        _direct(x)
         and x.dim() == 2
-        and _dense_rows(x.shape[0], x.shape[1], m, gelu)
+        and (
+            _dense_round(x.shape[0], x.shape[1], m)
+            or bias is not None
+            and _dense_rows(x.shape[0], x.shape[1], m, gelu)
+            # (host time is nothing there, and the library's kernel the faster one)
+            and not (
+                x.shape[1] > 2048
+                and x.is_cuda
+                and torch.cuda.is_current_stream_capturing()
+            )
+        )
         and _plain_operands(x, weight)
         and x.shape[0] < 1 << 30
         and x.shape[1] <= x.stride(0) < 1 << 22
-        and _plain_bias(bias, m, x)
-        # (host time is nothing there, and the library's kernel the faster one)
-        and (x.shape[1] <= 2048 or not torch.cuda.is_current_stream_capturing())
+        and (bias is None or _plain_bias(bias, m, x))
     ):
         return None
     out = torch.empty((x.shape[0], m), dtype=x.dtype, device=x.device)
@@ -615,12 +647,17 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     """x @ weight^T (+ bias): kernels of our own for the few rows of a decode
     batch and for the encoder's short K where they are the faster ones, the
     library otherwise."""
-    if bias is not None:
+    # sizes first: most calls that are not for the kernel end there
+    m = weight.shape[0]
+    if bias is not None or (
+        type(x) in _TENSORS
+        and x.dim() == 2
+        and x.shape[0] > 256
+        and _dense_round(x.shape[0], x.shape[1], m)
+    ):
         out = _dense(x, weight, bias, False)
         if out is not None:
             return out
-    # sizes first: most calls that are not for the kernel end there
-    m = weight.shape[0]
     if (
         type(x) in _TENSORS
         and x.dim() == 2

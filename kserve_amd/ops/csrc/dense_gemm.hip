@@ -16,8 +16,8 @@
 // fragment never share a bank (0 conflicts).
 //
 // us, this / the library (and gelu's kernel): 7864 x 768 to 2304 32 / 63, to 768
-// 12.6 / 15.1, to 3072 with gelu 44 / 68; 1500 rows to 768 7.0 / 8.7, to 3072 with
-// gelu 14.6 / 20.9; 200 rows to 2304 5.4 / 7.9.
+// 12.6 / 15.1, to 3072 with gelu 44 / 68; 7864 x 3072 to 768 32 / 40; 1500 rows to 768 7.0
+// / 8.7, to 3072 with gelu 14.6 / 20.9; 200 rows to 2304 5.4 / 7.9.
 #include "gemm_tile.h"
 
 namespace {
@@ -27,17 +27,21 @@ namespace {
 // and b are us at K 768 without gelu, fitted over 768 to 3072 features and 1200 to
 // 12000 rows; all grow with K and gelu alike, so the order holds. Where a unit has a
 // single tile, one block of eight waves with a deeper ring beats one of four (7864 x
-// 768 to 768 13.5 / 15.0, 1200 to 2304 10.5 / 12.8).
+// 768 to 768 13.5 / 15.0, 1200 to 2304 10.5 / 12.8). The largest tile is for what it
+// alone brings into one round (us, without / with it: 9000 x 768 to 768 15.7 / 14.7, 2048
+// to 768 28.5 / 26.5, 3072 to 768 43.0 / 38.3, 5400 x 3072 to 1024 46 / 31.8, 8000 57 / 42, 8000
+// x 4096 to 1024 63 / 55).
 struct Tile {
   int tn, tm;
   float a, b;
   bool pairs;
 };
-constexpr int NTILES = 6;
+constexpr int NTILES = 7;
 constexpr Tile TILES[NTILES] = {
     {128, 192, 12.6f, 0.5f, false}, {128, 192, 9.8f, 2.f, true},
     {128, 128, 9.5f, 0.f, false},   {128, 128, 7.2f, 2.2f, true},
-    {64, 128, 4.4f, 2.6f, false},   {64, 64, 2.9f, 2.5f, false}};
+    {64, 128, 4.4f, 2.6f, false},   {64, 64, 2.9f, 2.5f, false},
+    {256, 128, 14.1f, 0.5f, false}};
 
 }  // namespace
 
@@ -85,7 +89,8 @@ extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
     case 2: GO(128, 128, 4, 2, 4) break;
     case 3: GO(128, 128, 2, 2, 2) break;
     case 4: GO(64, 128, 2, 2, 3) break;
-    default: GO(64, 64, 2, 2, 4) break;
+    case 5: GO(64, 64, 2, 2, 4) break;
+    default: GO(256, 128, 4, 2, 3) break;
   }
 #undef GO
   HIP_CHECK_KERNEL();

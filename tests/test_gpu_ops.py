@@ -1461,7 +1461,7 @@ class TestDenseGemm:
         tol = 2.0**-8 * y.abs() + 1e-5 * x.shape[1] ** 0.5
         assert ((out.double().cpu() - y).abs() <= tol).all()
 
-    @pytest.mark.parametrize("tile", range(6))
+    @pytest.mark.parametrize("tile", range(7))
     @pytest.mark.parametrize(
         "N,K,M",
         [(1, 64, 8), (63, 128, 200), (129, 192, 72), (130, 256, 392), (257, 320, 1160)],
@@ -1499,6 +1499,30 @@ class TestDenseGemm:
         assert ops.linear(x.view(1, N, 768), w, b).shape == (1, N, 768)
         xg = x.clone().requires_grad_()
         assert ops.linear(xg, w, b).requires_grad
+
+    @pytest.mark.parametrize(
+        "N,K,M", [(8192, 512, 768), (1024, 4096, 256), (3583, 2112, 2304), (300, 512, 264)]
+    )
+    def test_one_round(self, dev, N, K, M):
+        """Products that one round of the largest tiles holds, without a bias too, at the
+        ends of the rule; weights of rows of rows and with gradients as before."""
+        from kserve_amd import ops
+        import kserve_amd_C
+
+        torch.manual_seed(N)
+        x = torch.randn(N, K, device=dev, dtype=torch.bfloat16)
+        w = (torch.randn(M, K, device=dev) * K**-0.5).to(torch.bfloat16)
+        b = torch.randn(M, device=dev, dtype=torch.bfloat16)
+        want = torch.empty(N, M, device=dev, dtype=torch.bfloat16)
+        kserve_amd_C.dense_gemm(want, x, w, b, False)
+        assert torch.equal(ops.linear(x, w, b), want)
+        kserve_amd_C.dense_gemm(want, x, w, None, False)
+        assert torch.equal(ops.linear(x, w), want)
+        rows = torch.randperm(N)[:300]
+        self._check(want[rows], x[rows], w, torch.zeros_like(b), False)
+        assert ops.linear(x.view(1, N, K), w).shape == (1, N, M)
+        assert ops.linear(x, w.clone().requires_grad_()).requires_grad
+        assert ops.linear(x.float(), w.float()).dtype == torch.float32
 
     @pytest.mark.parametrize("K,own", [(2048, True), (2560, False)])
     def test_captured_products(self, dev, K, own):
