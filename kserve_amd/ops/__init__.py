@@ -584,21 +584,21 @@ def _dense_round(n: int, k: int, m: int) -> bool:
     By a tenth to a third as a rule (k 512, m 2304 at 2600 / 3500 rows 10.9 / 14.0, 12.8 /
     16.2; k 1024, m 1024 at 8000 18.2 / 20.2; k 1536, m 1536 at 3000 18.0 / 22.9; k 2048, m
     2048 at 800 / 2000 / 4000 13.9 / 15.6, 17.9 / 21.7, 30.4 / 33.2, m 256 at 8192 14.1 / 20.9,
-    at 32000 41.4 / 41.1; k 3072, m 768 at 2000 / 4600 / 7000 / 9800 17.9 / 19.3, 23.4 / 28.5,
-    31.4 / 36.8, 40.6 / 45.7, with the rows not in a cache at 7864 40 / 43; k 4096, m 1024 at
-    1400 / 8000 22.3 / 22.9, 54.6 / 58.7, m 2048 at 2600 43 / 50). Few rows of a long k leave
-    units idle where the library splits it (k 4096, m 256 at 768 13.4 / 10.5; m 128 at 2000
-    11.1 / 9.2). On wider ones the library's times turn from one size to the next (k 2048, m
-    3072 at 768 / 1280 / 2048 16.4 / 19.3, 24.4 / 21.1, 28.7 / 27.7; k 768, m 4096 at 1400 / 1872
-    14.0 / 18.5, 19.3 / 17.4; k 4096, m 4096 at 1400 50 / 50), on longer k too (k 8192, m 2048
-    at 768 / 2600 45 / 39, 81 / 93), and past one round its tiles are ahead (k 2048, m 768 at
-    10900 rows 37 / 33, k 3072 58 / 52)."""
+    at 32000 41.4 / 41.1). On longer k by less, since operands that are in no cache cost this
+    kernel more (a layer's time against the library's in a chain of an encoder's twelve: k
+    3072, m 768 at 5500 / 7000 / 7864 rows -1.4, -3.0, -3.8, k 4096, m 1024 at 3600 / 7000 -7.5,
+    -3.9), and only where its tiles of 128 x 128 fill three quarters of the units: the
+    library splits k (k 3072, m 768 at 1500 / 3600 / 4200 +3.1, +5.3, -0.5, k 4096, m 1024 at
+    1100 / 2600 / 3100 +5.2, -0.3, -2.4). On wider ones the library's times turn from one size
+    to the next (k 2048, m 3072 at 768 / 1280 / 2048 16.4 / 19.3, 24.4 / 21.1, 28.7 / 27.7; k 768,
+    m 4096 at 1400 / 1872 14.0 / 18.5, 19.3 / 17.4; k 4096, m 4096 at 1400 50 / 50), and past one
+    round its tiles are ahead (k 2048, m 768 at 10900 rows 37 / 33, k 3072 58 / 52)."""
     return (
         m % 8 == 0
         and 256 <= m <= 2304
         and 512 <= k <= 4096
-        and n >= (1024 if k > 2048 else 1)
         and -(-n // 256) * -(-m // 128) <= 256
+        and (k <= 2048 or -(-n // 128) * -(-m // 128) >= 192)
     )
 
 

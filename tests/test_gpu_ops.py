@@ -1501,7 +1501,7 @@ class TestDenseGemm:
         assert ops.linear(xg, w, b).requires_grad
 
     @pytest.mark.parametrize(
-        "N,K,M", [(8192, 512, 768), (1024, 4096, 256), (3583, 2112, 2304), (300, 512, 264)]
+        "N,K,M", [(8192, 512, 768), (12200, 4096, 256), (3583, 2112, 2304), (300, 512, 264)]
     )
     def test_one_round(self, dev, N, K, M):
         """Products that one round of the largest tiles holds, without a bias too, at the
