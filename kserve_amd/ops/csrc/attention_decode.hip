@@ -46,8 +46,8 @@
 using namespace mfma_attn;
 
 extern "C" int ks_paged_decode_splits(int num_seqs, int num_kv_heads,
-                                      int max_blocks) {
-  return decode_splits(num_seqs, num_kv_heads, max_blocks);
+                                      int max_blocks, int head_dim, int fp8) {
+  return decode_splits(num_seqs, num_kv_heads, max_blocks, fp8 || head_dim <= 64);
 }
 
 extern "C" hipError_t ks_paged_attention_decode(

@@ -1117,8 +1117,8 @@ extern "C" int ks_ctx_attention_mfma(const void* out, const void* q,
 
 // key splits of a decode launch on that path
 extern "C" int ks_ctx_attention_mfma_splits(int num_seqs, int kv_heads,
-                                            int max_blocks) {
-  return mfma_attn::decode_splits(num_seqs, kv_heads, max_blocks);
+                                            int max_blocks, int head_dim) {
+  return mfma_attn::decode_splits(num_seqs, kv_heads, max_blocks, head_dim <= 64);
 }
 
 static hipError_t ctx_attention_mfma(const CtxArgs& a) {

@@ -21,7 +21,7 @@ hipError_t ks_paged_attention_decode(void*, const void*, const void*,
                                      float, int, int, int, int, int, int,
                                      long, int, void*, void*, int, int,
                                      hipStream_t);
-int ks_paged_decode_splits(int, int, int);
+int ks_paged_decode_splits(int, int, int, int, int);
 hipError_t ks_flash_prefill_varlen(void*, const void*, const void*,
                                    const void*, const void*, int, int, int,
                                    int, int, float, long, long, long, int,
@@ -204,7 +204,7 @@ void paged_attention_decode(at::Tensor& out, at::Tensor& q,
   int Hkv = k_cache.size(1);
   int block_size = k_cache.size(2);
   int max_blocks = block_tables.size(1);
-  const int n_splits = ks_paged_decode_splits(S, Hkv, max_blocks);
+  const int n_splits = ks_paged_decode_splits(S, Hkv, max_blocks, D, fp8);
   at::Tensor part_out, part_ml;
   void *po = nullptr, *pml = nullptr;
   if (n_splits > 1) {

@@ -46,7 +46,7 @@ int ks_ctx_attention_decode_splits(int, int, int, int, int, int);
 int ks_ctx_attention_mfma(const void*, const void*, const void*, const void*, int,
                           int, int, int, int, int, int, const void*, long, int,
                           float, int);
-int ks_ctx_attention_mfma_splits(int, int, int);
+int ks_ctx_attention_mfma_splits(int, int, int, int);
 hipError_t ks_qk_headnorm_rope_cache(void*, const void*, const void*,
                                      const void*, long, const void*,
                                      const void*, const void*, const void*,
@@ -561,7 +561,7 @@ void ctx_attention_f32(at::Tensor& out, at::Tensor& q, at::Tensor& k_cache,
         (int)heads, G, D, DV, bs, f32, fp, (long)vrs, (int)maps, (float)softcap,
         (int)keep_first);
     nsplit = mfma ? ks_ctx_attention_mfma_splits(num_seqs, G,
-                                                 (int)block_tables.size(1))
+                                                 (int)block_tables.size(1), D)
                   : ks_ctx_attention_decode_splits(num_seqs, (int)heads, G,
                                                    (int)window, (int)keep_first,
                                                    fp != nullptr);

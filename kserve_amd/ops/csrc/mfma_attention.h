@@ -1064,11 +1064,16 @@ bool deep_blocks(const DecodeArgs& p) {
   return D == 128 && p.n_splits == 1 && tokens >= (PARTS == 1 ? 24 : 48) * PAGE;
 }
 
+// Blocks from which on short contexts have no splits, and none.
+constexpr long UNSPLIT_BLOCKS = 192, FULL_BLOCKS = 512;
+
 template <int D, int SRC, int PARTS = 1>
 hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) {
   const bool few = p.max_blocks <= (SRC == PAGES_FP8 ? 8 : 4);
   const long blocks = (long)num_seqs * p.Hkv;
-  if (few && p.n_splits == 1 && blocks >= ONE_WAVE_BLOCKS) {
+  if (p.n_splits == 1 && blocks >= UNSPLIT_BLOCKS && blocks < FULL_BLOCKS) {
+    launch_decode_waves<D, SRC, PARTS, 2 * WAVES>(p, num_seqs, stream);
+  } else if (few && p.n_splits == 1 && blocks >= ONE_WAVE_BLOCKS) {
     launch_decode_waves<D, SRC, PARTS, 1>(p, num_seqs, stream);
   } else {
     if constexpr (SRC == PAGES_FP8) {
@@ -1092,18 +1097,37 @@ hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) 
   return hipSuccess;
 }
 
-// Context splits for a launch over num_seqs x num_kv_heads: none from 512
-// blocks on (8 KV heads, us: 64 sequences of 1500 61.5 unsplit, 65 with 2 splits,
-// 69 with 4), about 640 blocks below that. Splits cost even contexts up to a
-// tenth there (48 of 900: 32 unsplit, 35 with 2; 24 of 900: 21 and 22 with 4) and
-// keep one long context from being what the launch waits for (40 of 500 and one
-// of 7000: 118 unsplit, 71 with 2; 24 of 1000 to 4000: 63, 45 with 4). At most 32
-// (one of 7000: 14 us with 32, 16 with 16). A sequence uses as many of them as it
-// has page pairs for every wave.
-inline int decode_splits(int num_seqs, int num_kv_heads, int max_blocks) {
+// Context splits for a launch over num_seqs x num_kv_heads; `light`: pages of 2 KB (E4M3,
+// heads of 64), whose blocks take half the LDS. None from FULL_BLOCKS blocks on (8 KV
+// heads, us: 64 sequences of 1500 61.5 unsplit, 65 with 2 splits, 69 with 4).
+//
+// Below, 512 to 960 blocks (light: 640 to 1024), as even a number on each unit as that
+// allows (us, about 640 blocks / so: 8 of 1500 16.9 / 15.0, of 4000 29.8 / 25.9, 16 of 900
+// 19.0 / 16.9, 32 of 3000 77.9 / 76.9, 40 of 2500 83.5 / 78.1, E4M3 49.2 / 44.8). At most 32
+// (one of 7000: 14 us with 32, 16 with 16). A sequence uses as many of them as it has
+// page pairs for every wave.
+//
+// Short contexts have none from UNSPLIT_BLOCKS on: blocks of four waves spare the launch
+// that merges (us, split / not: 24 of 100 9.2 / 6.9, of 400 14.2 / 11.8, of 900 21.1 / 21.0,
+// 32 of 1300 38.4 / 37.2, 63 of 1000 53.2 / 50.4, E4M3 33.1 / 28.4; fp32 queries, 4 KV heads,
+// 64 of 200 14.2 / 11.2, of 1000 33.7 / 30.0). Long ones do, so that one of them is not what
+// the launch waits for (waves of two, 40 of 500 and one of 7000: 118 unsplit, 71 with 2),
+// and between 257 and 383 blocks, one on some units and two on the others (40 of 1200 41
+// / 42), and light pages up to there (24 of 900 E4M3 15.6 / 17.3, heads of 64 12.4 / 13.2).
+inline int decode_splits(int num_seqs, int num_kv_heads, int max_blocks, bool light) {
   const long base = (long)num_seqs * num_kv_heads;
-  if (base <= 0 || base >= 512) return 1;
-  long n = (640 + base - 1) / base;
+  if (base <= 0 || base >= FULL_BLOCKS) return 1;
+  const int short_pages = base >= 384 ? 128
+                          : light     ? 16
+                          : base > 256 ? 40
+                                       : 128;
+  if (base >= UNSPLIT_BLOCKS && max_blocks <= short_pages) return 1;
+  const long least = light ? 640 : 512, target = light ? 1024 : 960;
+  long n = (least + base - 1) / base;
+  // blocks of the busiest unit, each with 1 / t of the context
+  auto rounds = [&](long t) { return (base * t + 255) / 256; };
+  for (long t = n + 1; t * base <= target; ++t)
+    if (rounds(t) * n < rounds(n) * t) n = t;
   const long most = ((long)max_blocks + 2 * WAVES - 1) / (2 * WAVES);
   if (n > most) n = most;
   if (n > 32) n = 32;

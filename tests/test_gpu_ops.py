@@ -300,14 +300,25 @@ class TestDecodeAttention:
         """Past 4096 blocks E4M3 pages go back to blocks of two waves."""
         self.test_paged_decode_edges(dev, H, 1, 128, window, 0, True, 400)
 
-    @pytest.mark.parametrize("H,Hkv,window", [(4, 1, 0), (8, 1, 0), (6, 2, 768), (6, 2, 767)])
-    def test_four_waves_per_block(self, dev, H, Hkv, window):
-        """bf16 pages in blocks of four waves, two of which end at once where a context
-        has fewer than four page pairs, in both precisions of the scores; a window that
-        is a token shorter than fp32 queries take four from."""
+    @pytest.mark.parametrize(
+        "H,Hkv,D,fp8,window,blocks",
+        [
+            (4, 1, 128, False, 0, 512), (8, 1, 128, False, 0, 512),
+            (6, 2, 128, False, 768, 512), (6, 2, 128, False, 767, 512),
+            (4, 1, 128, False, 0, 192), (4, 2, 128, False, 50, 192),   # no splits
+            (4, 1, 64, False, 0, 192), (4, 1, 128, True, 0, 192),
+            (3, 1, 64, False, 33, 384), (3, 1, 128, True, 0, 384),
+        ],
+    )
+    def test_four_waves_per_block(self, dev, H, Hkv, D, fp8, window, blocks):
+        """Blocks of four waves, two of which end at once where a context has few page
+        pairs, in both precisions of the scores; a window that is a token shorter than
+        fp32 queries take four from at 512 blocks."""
         from kserve_amd import ops
 
-        D, ctx = 128, [1, 32, 96, 97, 112, 113, 128, 129, 160, 161, 767, 780, 1553]
+        ctx = [1, 32, 96, 97, 112, 113, 128, 129, 160, 161, 225, 256]
+        if blocks > 192 or D == 128 and not fp8:
+            ctx += [481, 512, 767, 780, 1553]
         torch.manual_seed(H)
         width = -(-max(ctx) // 16)
         NB = len(ctx) * width
@@ -318,13 +329,15 @@ class TestDecodeAttention:
                 x[row[-(-c // 16) :]] = float("nan")
                 if c % 16:
                     x[row[c // 16], :, c % 16 :] = float("nan")
+        if fp8:
+            kc, vc = kc.to(torch.float8_e4m3fn), vc.to(torch.float8_e4m3fn)
         ctx_t = torch.tensor(ctx, dtype=torch.int32)
         q = (torch.randn(len(ctx), H, D, device=dev) * 1.5).to(torch.bfloat16)
         ref = torch_ref.paged_attention_decode(
             q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt, ctx_t,
             D ** -0.5, window=window,
         )
-        n = -(-512 // (len(ctx) * Hkv))
+        n = -(-blocks // (len(ctx) * Hkv))
         many = [x.to(dev) for x in (bt.repeat(n, 1), ctx_t.repeat(n))]
         got = ops.paged_attention_decode(
             q.repeat(n, 1, 1), kc, vc, *many, D ** -0.5, window=window
@@ -333,6 +346,8 @@ class TestDecodeAttention:
             # fp32 weights and sums, the output rounded to bf16
             err = (part - ref).abs()
             assert (err <= 2 ** -8 * ref.abs() + 1e-5).all(), float(err.max())
+        if fp8:
+            return
         cu = torch.arange(n * len(ctx) + 1, dtype=torch.int32, device=dev)
         got = ops.ctx_attention_f32(
             q.float().reshape(len(ctx), -1).repeat(n, 1), kc, vc, many[0], cu, many[1],
