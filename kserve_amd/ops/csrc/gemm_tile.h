@@ -145,10 +145,6 @@ void dense_gemm_kernel(const DenseArgs p) {
       step -= step >= steps ? steps : 0;
     }
     short* const to = &ring[slot * STAGE + (i * NW + wave) * 8 * BK];
-    // Weights that one block alone reads pass the caches by: they leave no room there
-    // otherwise to what the next kernels read and to what the last ones wrote (steps in
-    // us: hybrid 72 / 128 sequences 695 -> 683, 992 -> 981, llama 256 2268 -> 2260, 192
-    // level). Not the narrow products' in parts (72 / 128 sequences 8 and 6 us slower).
     const short* from = i < NX ? xb : wb;
     if (HALVES && i >= NX && ((i - NX) * NW + wave) * 8 / HR % 2)
       from += (long)p.M * p.K;  // up rows
