@@ -29,9 +29,10 @@
 // that is followed in steps of 2^8, tile addresses from scalars, and keys read six
 // products ahead took 700 vector cycles and most waits off a tile. Measured (32 query
 // and 8 KV heads of 128, causal; the 16x16x32 kernel with one head per block before,
-// then before and with those): 1 x 8191 tokens 2497 / 621 / 557 us (990 TFLOP/s), 8 x
-// 2048 1280 / 373 / 329 us, 16 x 500 77 / 72 us; 2 x 1000 queries over 13000 paged
-// keys 2441 / 484 / 438 us (E4M3 pages 2596 / 567 / 500); 8 x 500, 12 heads of 64,
+// then before and with those; waves with products ahead of waves with vector
+// instructions take another 1 to 4 % off): 1 x 8191 tokens 2497 / 621 / 557 us (990
+// TFLOP/s), 8 x 2048 1280 / 373 / 329 us, 16 x 500 77 / 72 us; 2 x 1000 queries over 13000
+// paged keys 2441 / 484 / 438 us (E4M3 pages 2596 / 567 / 500); 8 x 500, 12 heads of 64,
 // bidirectional 20 / 17 us, 64 x 123 level at 13; fp32 scores, 4 x 2000, 16 / 4 heads
 // 239 / 223 us.
 //

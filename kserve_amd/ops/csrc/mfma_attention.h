@@ -159,6 +159,18 @@ struct PrefillArgs {
 };
 constexpr float NO_KEYS = -1.f;  // of a part without a tile, which writes no sums
 
+// While a wave has products to issue it goes ahead of the other on its SIMD: that one's
+// exponentials fill the cycles between, where by age a wave among its vector
+// instructions keeps the products waiting (us: 1 x 8191 tokens 542 -> 533, 2 x 1000 queries
+// over 13000 keys 366 -> 348, fp32 scores 4 x 2000 204 -> 198; only around the second
+// product 550 and 362, the second above the first 541 and 357, the other way about 557 and
+// 360, the vector part ahead 576 and 367). Not heads of 64, whose units have four waves a
+// SIMD (64 texts of 123 tokens 19.0 / 19.2).
+template <int D, int FIRST>
+__device__ __forceinline__ void go_first() {
+  if constexpr (D == 128) __builtin_amdgcn_s_setprio(FIRST);
+}
+
 template <int D, int SRC, bool CAUSAL, bool WIN, int PARTS = 1>
 __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
     const PrefillArgs p) {
@@ -398,6 +410,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
 #pragma unroll
           for (int r = 0; r < 16; ++r) s[kb][r] = 0.f;
         // both key blocks' chains side by side, keys read ahead of the products
+        go_first<D, 1>();
 #pragma unroll
         for (int c = 0; c < KC; ++c)
 #pragma unroll
@@ -412,6 +425,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+        go_first<D, 0>();
       } else {
 #pragma unroll
       for (int kb = 0; kb < NKB; ++kb) {
@@ -480,6 +494,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
           }
         }
       l += sum;
+      go_first<D, 1>();
 #pragma unroll
       for (int kc = 0; kc < NKB * 2; ++kc)
 #pragma unroll
@@ -499,6 +514,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(
           for (int part = PARTS - 1; part >= 0; --part)
             o[b] = mfma32(a.v, pf[part][kc], o[b]);
         }
+      go_first<D, 0>();
       }
     }
     if (t + 1 < t_hi) commit(buf ^ 1);
