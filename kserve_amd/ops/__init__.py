@@ -617,28 +617,30 @@ def _plain_bias(bias: torch.Tensor, m: int, x: torch.Tensor) -> bool:
 
 def _dense(x, weight, bias, gelu: bool) -> Optional[torch.Tensor]:
     """The encoder kernel's product, or None for operands that it does not take."""
+    if not _direct(x) or x.dim() != 2:
+        return None
+    n, k = x.shape
     m = weight.shape[0]
     if not (
-        _direct(x)
-        and x.dim() == 2
-        and (
-            _dense_round(x.shape[0], x.shape[1], m)
-            or bias is not None
-            and _dense_rows(x.shape[0], x.shape[1], m, gelu)
-            # (host time is nothing there, and the library's kernel the faster one)
-            and not (
-                x.shape[1] > 2048
-                and x.is_cuda
-                and torch.cuda.is_current_stream_capturing()
-            )
-        )
-        and _plain_operands(x, weight)
-        and x.shape[0] < 1 << 30
-        and x.shape[1] <= x.stride(0) < 1 << 22
-        and (bias is None or _plain_bias(bias, m, x))
+        bias is not None
+        and _dense_rows(n, k, m, gelu)
+        # (host time is nothing there, and the library's kernel the faster one)
+        and not (k > 2048 and x.is_cuda and torch.cuda.is_current_stream_capturing())
+        or _dense_round(n, k, m)
     ):
         return None
-    out = torch.empty((x.shape[0], m), dtype=x.dtype, device=x.device)
+    if not (
+        _plain_operands(x, weight)
+        and n < 1 << 30
+        and k <= x.stride(0) < 1 << 22
+        and (
+            not torch.is_autocast_enabled("cuda")
+            if bias is None
+            else _plain_bias(bias, m, x)
+        )
+    ):
+        return None
+    out = torch.empty((n, m), dtype=x.dtype, device=x.device)
     _C.dense_gemm(out, x, weight, bias, gelu)
     return out
 
@@ -647,15 +649,20 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
     """x @ weight^T (+ bias): kernels of our own for the few rows of a decode
     batch and for the encoder's short K where they are the faster ones, the
     library otherwise."""
+    if bias is not None:
+        out = _dense(x, weight, bias, False)
+        if out is not None:
+            return out
     # sizes first: most calls that are not for the kernel end there
     m = weight.shape[0]
-    if bias is not None or (
-        type(x) in _TENSORS
+    if (
+        bias is None
+        and type(x) in _TENSORS
         and x.dim() == 2
         and x.shape[0] > 256
         and _dense_round(x.shape[0], x.shape[1], m)
     ):
-        out = _dense(x, weight, bias, False)
+        out = _dense(x, weight, None, False)
         if out is not None:
             return out
     if (

@@ -1538,6 +1538,8 @@ class TestDenseGemm:
         assert ops.linear(x.view(1, N, K), w).shape == (1, N, M)
         assert ops.linear(x, w.clone().requires_grad_()).requires_grad
         assert ops.linear(x.float(), w.float()).dtype == torch.float32
+        with torch.autocast("cuda", torch.float16):
+            assert ops.linear(x, w).dtype == ops.linear(x, w, b).dtype == torch.float16
 
     @pytest.mark.parametrize("K,own", [(2048, True), (2560, False)])
     def test_captured_products(self, dev, K, own):
