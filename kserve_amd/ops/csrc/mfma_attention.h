@@ -635,7 +635,7 @@ __device__ __forceinline__ uint4 load16_nt(const char* from) {
 
 // Waves of a block that share a context, and page pairs of a split from which on the
 // launches with four use all of them: bf16 pages a pair for each (the LDS of the other
-// two is taken in any case: 256 sequences of 200, 8 heads 40.6 us with 16, 38.6 so).
+// two is taken in any case).
 constexpr int WAVES = 2;
 constexpr int deep_pairs(int src) { return src == PAGES_FP8 ? 16 : 2 * WAVES; }
 
@@ -1033,7 +1033,8 @@ __global__ __launch_bounds__(256) void paged_attention_reduce_kernel(
 }
 
 // Two waves per block: 32 KB of LDS, four blocks per compute unit, so one
-// block's first loads run under the others' last ones. Four where contexts are long.
+// block's first loads run under the others' last ones. Four from UNSPLIT_BLOCKS to
+// FULL_BLOCKS blocks without splits, and of E4M3 pages.
 //
 // One wave where a table holds a page pair or two per wave (four of E4M3) and
 // the blocks are more than the chip takes at once: the second wave has little or
@@ -1063,22 +1064,12 @@ void launch_decode_waves(const DecodeArgs& p, int num_seqs, hipStream_t stream) 
 // 35.2) nor in many splits, which are short (one of 2000 8.6 / 8.9).
 constexpr long MOST_DEEP_BLOCKS = 4096;
 
-// bf16 pages: four waves where splits leave none (from 512 blocks on) and a sequence can
-// be long. The longest contexts of a ragged batch end sooner, and two blocks of four
-// waves a unit read fewer pages at a time than four of two, which memory takes better
-// (us, 2 / 4 waves, 8 KV heads: 256 of 2048 +- 60% 350 / 339, all of 2048 330 / 322, of
-// 450 80 / 77, 200 of 1200 171 / 160, 128 of 900 86 / 84, 1000 of 500 328 / 322, 64 level;
-// 256 of 300 55 / 53, of 200 37.5 / 38.6, of 100 22.6 / 27.4; fp32 queries, 4 KV heads:
-// 128 of 1500 79 / 76, 500 of 600 108 / 105, 200 of 700 58 / 56, 128 of 400 24.3 / 24.9, 256
-// of 300 32.5 / 34.5). Half the LDS, values over the keys once these are read, lets more
-// blocks in, and all of it was slower (64 of 1000 50 -> 57, 256 of 2048 350 -> 355).
-template <int D, int PARTS>
-bool deep_blocks(const DecodeArgs& p) {
-  int tokens = p.max_blocks * PAGE;
-  if (p.window > 0 && p.window < tokens) tokens = p.window;
-  if (p.x.chunk > 0 && p.x.chunk < tokens) tokens = p.x.chunk;
-  return D == 128 && p.n_splits == 1 && tokens >= (PARTS == 1 ? 24 : 48) * PAGE;
-}
+// bf16 pages stay with two where splits leave none: four are ahead on long contexts, but
+// two of them have nothing to do on short ones, and their LDS keeps other blocks out. Which
+// it is only the device knows in a captured step, whose tables are as wide as the longest
+// allowed (us, 2 / 4 waves, 8 KV heads: 256 of 2048 +- 60% 350 / 339, of 400 74 / 71, of 200
+// 40 / 41, of 100 23 / 28, of 30 13 / 19). Half the LDS, values over the keys once these are
+// read, lets more blocks in than memory takes well (64 of 1000 50 -> 57).
 
 // Blocks from which on short contexts have no splits, and none.
 constexpr long UNSPLIT_BLOCKS = 192, FULL_BLOCKS = 512;
@@ -1097,8 +1088,6 @@ hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) 
         launch_decode_waves<D, SRC, PARTS, 2 * WAVES>(p, num_seqs, stream);
       else
         launch_decode_waves<D, SRC, PARTS, WAVES>(p, num_seqs, stream);
-    } else if (deep_blocks<D, PARTS>(p)) {
-      if constexpr (D == 128) launch_decode_waves<D, SRC, PARTS, 2 * WAVES>(p, num_seqs, stream);
     } else {
       launch_decode_waves<D, SRC, PARTS, WAVES>(p, num_seqs, stream);
     }

@@ -303,17 +303,16 @@ class TestDecodeAttention:
     @pytest.mark.parametrize(
         "H,Hkv,D,fp8,window,blocks",
         [
-            (4, 1, 128, False, 0, 512), (8, 1, 128, False, 0, 512),
-            (6, 2, 128, False, 768, 512), (6, 2, 128, False, 767, 512),
+            (4, 1, 128, False, 0, 512), (8, 1, 128, False, 0, 256),
+            (6, 2, 128, False, 768, 192), (6, 2, 128, False, 767, 384),
             (4, 1, 128, False, 0, 192), (4, 2, 128, False, 50, 192),   # no splits
             (4, 1, 64, False, 0, 192), (4, 1, 128, True, 0, 192),
             (3, 1, 64, False, 33, 384), (3, 1, 128, True, 0, 384),
         ],
     )
     def test_four_waves_per_block(self, dev, H, Hkv, D, fp8, window, blocks):
-        """Blocks of four waves, two of which end at once where a context has few page
-        pairs, in both precisions of the scores; a window that is a token shorter than
-        fp32 queries take four from at 512 blocks."""
+        """Blocks of four waves without splits, two of which end at once where a context
+        has few page pairs, in both precisions of the scores; from 512 blocks on two."""
         from kserve_amd import ops
 
         ctx = [1, 32, 96, 97, 112, 113, 128, 129, 160, 161, 225, 256]
