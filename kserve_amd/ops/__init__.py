@@ -364,9 +364,19 @@ def _direct(x: torch.Tensor) -> bool:
     )
 
 
+def _keeps_dtype(x: torch.Tensor) -> bool:
+    """Whether the library's product would have x's type, under autocast too. The calls
+    of `_skinny_rows` and of few rows beside it are the kernel's whatever autocast asks
+    for; the wider rules leave those that would change their type to the library."""
+    return (
+        not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == x.dtype
+    )
+
+
 def _skinny_operands(x: torch.Tensor, weight: torch.Tensor) -> bool:
     n = x.shape[0]
-    # (above 64 rows: 32-bit offsets within a tile; the rules bound K)
+    # (above 64 rows x stays within 32-bit offsets of a tile; a longer K is the kernel's
+    # 64-bit form's)
     return (
         (n <= 64 or n <= 256 and x.stride(0) < 1 << 22)
         and _direct(x)
@@ -677,6 +687,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
             )
             or _streamed_rows(x.shape[0], x.shape[1], m)
             and (bias is None or m % 8 == 0)
+            and _keeps_dtype(x)
         )
         and _skinny_operands(x, weight)
         and (bias is None or _plain_bias(bias, m, x))
@@ -703,6 +714,7 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
             _skinny_rows(n, k, m)
             or n <= 256 and m % 4 == 0 and 2048 <= m < 4096 and 2048 <= k < 1 << 22
             or _streamed_parts(n, k, m)
+            and _keeps_dtype(x)
         )
         and _skinny_operands(x, weight)
     ):
@@ -728,6 +740,7 @@ def linear_silu_and_mul(
         and (
             _skinny_glu_rows(x.shape[0], x.shape[1], weight.shape[0] // 2)
             or _streamed_glu_rows(x.shape[0], x.shape[1], weight.shape[0] // 2)
+            and _keeps_dtype(x)
         )
         and _skinny_operands(x, weight)
     ):
@@ -753,6 +766,7 @@ def linear_clamped_swiglu(
             and _skinny_glu_rows(x.shape[0], x.shape[1], m)
             and _skinny_rows(x.shape[0], x.shape[1], 2 * m)
             or _streamed_glu_rows(x.shape[0], x.shape[1], m)
+            and _keeps_dtype(x)
         )
         and _skinny_operands(x, weight)
     ):
@@ -775,6 +789,7 @@ def linear_add_rms_norm(
         and (
             _skinny_rows(x.shape[0], x.shape[1], m)
             or _streamed_parts(x.shape[0], x.shape[1], m)
+            and _keeps_dtype(x)
         )
         and _skinny_operands(x, weight)
         and residual.shape == (x.shape[0], m)

@@ -1765,6 +1765,52 @@ class TestEmbeddedStream:
             assert all(t[[0, -1]].isnan().all() and not t[1:-1].isnan().any() for t in (x, h))
 
 
+class TestAutocast:
+    @staticmethod
+    def _outcome(f):
+        try:
+            y = f()
+        except RuntimeError:
+            return "refused"
+        return [(t.dtype, t.shape) for t in (y if isinstance(y, tuple) else (y,))]
+
+    @pytest.mark.parametrize("autocast", [torch.float16, torch.bfloat16])
+    def test_products_of_many_rows(self, dev, autocast):
+        """Products that the library had until the streaming tiles took them: to another
+        type they are the library's, and so is what follows; to bf16 nothing changes."""
+        from kserve_amd import ops
+
+        def rnd(*shape):
+            return torch.randn(*shape, device=dev, dtype=torch.bfloat16)
+
+        linear = torch.nn.functional.linear
+        x, w, b = rnd(200, 4096), rnd(12288, 4096) / 64, rnd(12288)
+        few, res, nw = w[:4096], rnd(200, 4096), rnd(4096)
+        assert ops._streamed_rows(200, 4096, 12288) and not ops._skinny_rows(200, 4096, 12288)
+        assert ops._streamed_parts(200, 4096, 4096) and not ops._skinny_rows(200, 4096, 4096)
+        assert ops._streamed_glu_rows(200, 4096, 6144) and not ops._skinny_glu_rows(200, 4096, 6144)
+        pairs = [
+            (lambda: ops.linear(x, w), lambda: linear(x, w)),
+            (lambda: ops.linear(x, w, b), lambda: linear(x, w, b)),
+            (lambda: ops.linear_silu_and_mul(x, w), lambda: ops.silu_and_mul(linear(x, w))),
+            (lambda: ops.linear_clamped_swiglu(x, w, 1.7, 7.0),
+             lambda: ops.clamped_swiglu(linear(x, w), 1.7, 7.0)),
+            (lambda: ops.linear_add_rms_norm(x, few, res.clone(), nw, 1e-5),
+             lambda: ops.fused_add_rms_norm(linear(x, few), res.clone(), nw, 1e-5)),
+        ]
+        plain = [self._outcome(f) for f, _ in pairs]
+        with torch.autocast("cuda", autocast):
+            for (f, want), bf16 in zip(pairs, plain):
+                assert self._outcome(f) == self._outcome(want)
+                assert autocast != torch.bfloat16 or self._outcome(f) == bf16
+            assert ops.linear(x, w).dtype == ops.linear(x, w, b).dtype == autocast
+            parts = ops.linear_parts(x, few)
+            if autocast == torch.bfloat16:
+                assert parts.dim() == 3 and parts.dtype == torch.float32
+            else:
+                assert parts.dim() == 2 and parts.dtype == autocast
+
+
 class TestClampedProducts:
     @pytest.mark.parametrize("K,M", [(2048, 8192), (64, 4612), (1088, 5000)])
     @pytest.mark.parametrize("N", [1, 16, 33, 64])
