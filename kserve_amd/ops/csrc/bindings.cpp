@@ -56,10 +56,8 @@ hipError_t ks_dense_gemm(void*, const void*, const void*, const void*, int, int,
                          long, int, int, hipStream_t);
 hipError_t ks_skinny_gemm(void*, void*, const void*, const void*, const void*, int, int,
                           int, long, int, int, hipStream_t);
-hipError_t ks_skinny_clamped_glu(void*, const void*, const void*, int, int, int, long,
-                                 float, float, hipStream_t);
 hipError_t ks_streamed_clamped_glu(void*, const void*, const void*, int, int, int, long,
-                                 float, float, hipStream_t);
+                                   float, float, hipStream_t);
 hipError_t ks_gemm8(void*, const void*, const void*, int, int, int, int,
                     hipStream_t);
 }
@@ -443,30 +441,19 @@ void skinny_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w) {
   skinny_product(out, x, w, c10::nullopt, true);
 }
 
-template <typename Kernel>
-static void clamped_product(at::Tensor& out, at::Tensor& x, at::Tensor& w, double alpha,
-                            double limit, Kernel kernel) {
+void streamed_clamped_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w, double alpha,
+                          double limit) {
+  // out [N, M] = clamped gate and up of x @ w^T, bf16, N <= 256
   CHECK_BF16_CONTIG(out);
   const SkinnyShape z = skinny_shape(x, w, 2);
   TORCH_CHECK(out.dim() == 2 && out.size(0) == z.N && out.size(1) == z.M &&
                   out.device() == x.device(),
               "output shape mismatch");
   const c10::DeviceGuard guard(x.device());
-  check_hip(kernel(out.data_ptr(), x.data_ptr(), w.data_ptr(), z.M, z.K, z.N, z.stride,
-                   (float)alpha, (float)limit, current_stream()),
-            "clamped_glu");
-}
-
-void skinny_clamped_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w, double alpha,
-                        double limit) {
-  // out [N, M] = clamped gate and up of x @ w^T, bf16, N <= 64
-  clamped_product(out, x, w, alpha, limit, ks_skinny_clamped_glu);
-}
-
-void streamed_clamped_glu(at::Tensor& out, at::Tensor& x, at::Tensor& w, double alpha,
-                          double limit) {
-  // the same, N <= 256
-  clamped_product(out, x, w, alpha, limit, ks_streamed_clamped_glu);
+  check_hip(ks_streamed_clamped_glu(out.data_ptr(), x.data_ptr(), w.data_ptr(), z.M, z.K,
+                                    z.N, z.stride, (float)alpha, (float)limit,
+                                    current_stream()),
+            "streamed_clamped_glu");
 }
 
 void dense_gemm(at::Tensor& out, at::Tensor& x, at::Tensor& w,
@@ -651,9 +638,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_rope_cache", &skinny_rope_cache,
         "few-row qkv GEMM, rotary embedding and K/V scatter");
   m.def("skinny_glu", &skinny_glu, "gate|up GEMM (N<=256) with silu(gate) * up");
-  m.def("skinny_clamped_glu", &skinny_clamped_glu,
-        "gate|up GEMM (N<=64) with the clamped gate");
-  m.def("streamed_clamped_glu", &streamed_clamped_glu, "the same for up to 256 rows");
+  m.def("streamed_clamped_glu", &streamed_clamped_glu,
+        "gate|up GEMM (N<=256) with the clamped gate");
   m.def("dense_gemm", &dense_gemm, "GEMM with bias and, if asked for, erf GELU",
         pybind11::arg("out"), pybind11::arg("x"), pybind11::arg("w"),
         pybind11::arg("bias"), pybind11::arg("gelu"), pybind11::arg("tile") = -1);

@@ -247,26 +247,13 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
 // activation kernel and its launch take 3.5 us of a decode layer, and the sums reach
 // it in 32 bits (hybrid step of 4 layers at 1 / 8 / 24 / 64 sequences 345 -> 342, 380 ->
 // 375, 446 -> 435, 652 -> 642 us).
-static hipError_t clamped_glu(void* out, const void* x, const void* w, int M, int K, int N,
-                              long xs, float alpha, float limit, int most,
-                              hipStream_t stream) {
-  if (N < 1 || N > most || M < 1 || M % 4 != 0 || K < BK || K % BK != 0 || xs % 8 != 0 ||
+extern "C" hipError_t ks_streamed_clamped_glu(void* out, const void* x, const void* w,
+                                              int M, int K, int N, long xs, float alpha,
+                                              float limit, hipStream_t stream) {
+  if (N < 1 || N > 256 || M < 1 || M % 4 != 0 || K < BK || K % BK != 0 || xs % 8 != 0 ||
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
     return hipErrorInvalidValue;
   return run({out, (const short*)x, (const short*)w, nullptr, M, K, N, (int)xs, 0, 0, 1,
               alpha, limit, xs},
              plan(M, K, N, true).tm, CLAMPED, stream);
-}
-
-extern "C" hipError_t ks_skinny_clamped_glu(void* out, const void* x, const void* w, int M,
-                                            int K, int N, long xs, float alpha,
-                                            float limit, hipStream_t stream) {
-  return clamped_glu(out, x, w, M, K, N, xs, alpha, limit, 64, stream);
-}
-
-// up to 256 rows
-extern "C" hipError_t ks_streamed_clamped_glu(void* out, const void* x, const void* w,
-                                              int M, int K, int N, long xs, float alpha,
-                                              float limit, hipStream_t stream) {
-  return clamped_glu(out, x, w, M, K, N, xs, alpha, limit, 256, stream);
 }

@@ -1813,11 +1813,11 @@ class TestAutocast:
 
 class TestClampedProducts:
     @pytest.mark.parametrize("K,M", [(2048, 8192), (64, 4612), (1088, 5000)])
-    @pytest.mark.parametrize("N", [1, 16, 33, 64])
+    @pytest.mark.parametrize("N", [1, 16, 33, 64, 65, 97, 129, 193, 256])
     def test_linear_clamped_swiglu(self, dev, N, K, M):
         """Against fp64, gates and ups past their limits among them: fp32 sums of K terms
         with the slopes of the function (at most 1.1 in the gate and the limit in up),
-        exp and one rounding to bf16."""
+        exp and one rounding to bf16. Odd M and short K by the kernel's entry."""
         from kserve_amd import ops
 
         torch.manual_seed(N + M)
@@ -1825,8 +1825,8 @@ class TestClampedProducts:
         x = torch.randn(N, K + 8, device=dev, dtype=torch.bfloat16)[:, :K]
         w = (torch.randn(2 * M, K, device=dev) * 2 * K ** -0.5).to(torch.bfloat16)
         got = torch.empty(N, M, device=dev, dtype=torch.bfloat16)
-        ops._C.skinny_clamped_glu(got, x, w, alpha, limit)
-        if N <= 48 or (K, M) == (2048, 8192):  # what comes here
+        ops._C.streamed_clamped_glu(got, x, w, alpha, limit)
+        if N <= 48 or K > 64:  # what comes here
             assert torch.equal(got, ops.linear_clamped_swiglu(x, w, alpha, limit))
         y = x.double() @ w.double().t()
         g, u = y[:, :M].clamp(max=limit), y[:, M:].clamp(-limit, limit)
@@ -1853,7 +1853,7 @@ class TestClampedProducts:
         lim = 1.2 * 3.5 * off[:, :M] + 2.5 * off[:, M:] + 2.0 ** -19 * few.double().abs()
         assert ((got.double() - few.double()).abs() <= lim + 2.0 ** -7 * few.double().abs()).all()
 
-    @pytest.mark.parametrize("N", [6, 64])
+    @pytest.mark.parametrize("N", [6, 64, 65, 129, 256])
     def test_values_past_all_limits(self, dev, N):
         """NaNs and infinities come out as from the product and the activation."""
         from kserve_amd import ops
@@ -1864,7 +1864,7 @@ class TestClampedProducts:
         w = (torch.randn(2 * M, K, device=dev) * K ** -0.5).to(torch.bfloat16)
         x[0], x[1, 5], x[2, 7], x[3] = float("nan"), float("inf"), float("-inf"), 1e30
         w[5, 9], w[M + 6, 9], w[7, 9] = float("inf"), float("nan"), float("-inf")
-        assert ops._skinny_glu_rows(N, K, M) and ops._skinny_rows(N, K, 2 * M)
+        assert ops._skinny_glu_rows(N, K, M) or ops._streamed_glu_rows(N, K, M)
         got = ops.linear_clamped_swiglu(x, w, 1.702, 7.0)
         want = ops.clamped_swiglu(torch.nn.functional.linear(x, w), 1.702, 7.0)
         assert torch.equal(got.isnan(), want.isnan()) and want[:4].isnan().any()
@@ -1874,10 +1874,10 @@ class TestClampedProducts:
     def test_more_rows_are_refused(self, dev):
         from kserve_amd import ops
 
-        x, w = (torch.zeros(n, 64, device=dev, dtype=torch.bfloat16) for n in (65, 9224))
-        out = torch.empty(65, 4612, device=dev, dtype=torch.bfloat16)
+        x, w = (torch.zeros(n, 64, device=dev, dtype=torch.bfloat16) for n in (257, 9224))
+        out = torch.empty(257, 4612, device=dev, dtype=torch.bfloat16)
         with pytest.raises(RuntimeError):
-            ops._C.skinny_clamped_glu(out, x, w, 1.702, 7.0)
+            ops._C.streamed_clamped_glu(out, x, w, 1.702, 7.0)
 
 
 class TestOperandDevices:
