@@ -532,16 +532,35 @@ def _streamed_rows(n: int, k: int, m: int) -> bool:
 
 
 def _streamed_glu_rows(n: int, k: int, m: int) -> bool:
-    """The same for gate|up products, whose activation comes with them (without the
-    library's 3 to 6 us for it): k 4096, m 14336 at 64 / 128 / 192 / 256 rows 42.8 / 53.3,
-    51.1 / 57.3, 60.6 / 68.9, 67.9 / 74.4, k 2048, m 4096 at 33 / 96 / 256 11.0 / 13.4, 14.6 /
-    14.4, 24.1 / 24.6, m 8192 at 128 / 256 18.5 / 20.9, 27.1 / 29.3, k 4096, m 5504 at 65 / 256
-    24.0 / 28.2, 44.8 / 48.4, k 5120, m 13824 at 64 / 128 / 256 56.5 / 59.1, 71 / 70, 85 / 92, k
-    8192, m 7168 at 33 / 128 / 256 41.6 / 49.7, 62 / 68, 89 / 95, m 14336 at 49 / 128 / 256 78 /
-    103, 98 / 112, 128 / 141. Level or behind below 4096 features (k 4096, m 3584 at 128 rows
-    28.1 / 25.9) and past 16384, where they take two rounds (k 3584, m 18944 at 128 83 /
-    74)."""
-    return m % 4 == 0 and 32 < n <= 256 and k >= 1024 and 4096 <= m <= 16384
+    """The same for gate|up products, whose activation comes with them (without its own
+    kernel's 3 to 6 us), against the product by the rules above or the library's and the
+    activation kernel: k 4096, m 14336 at 64 / 128 / 192 / 256 rows 42.8 / 53.3, 51.1 /
+    57.3, 60.6 / 68.9, 67.9 / 74.4, k 2048, m 4096 at 33 / 96 / 256 11.0 / 13.4, 14.6 / 14.4,
+    24.1 / 24.6, m 8192 at 128 / 256 18.5 / 20.9, 27.1 / 29.3, k 4096, m 5504 at 65 / 256 24.0 /
+    28.2, 44.8 / 48.4, k 8192, m 7168 at 33 / 128 41.6 / 49.7, 62 / 68, m 14336 at 49 / 128 /
+    256 78 / 103, 98 / 112, 128 / 141. Level or behind below 4096 features (k 4096, m 3584 at
+    128 rows 28.1 / 25.9) and past 16384, where they take two rounds (k 3584, m 18944 at 128
+    83 / 74).
+
+    K is never split here, so on long K only where the tiles fill the chip: half of it is
+    idle at 4096 features (k 14336 at 256 rows 147 / 71, k 5120 at 64 / 192 30.8 / 24.5, 52 /
+    38.9, k 4096 at 256 44.5 / 36.2), a third up to 5504 (m 5120, k 4096 at 128 / 256 31.0 /
+    33.4, 44.9 / 41.3, k 6144 at 192 61 / 44). Up to 8192 one round of 64 rows of weights is
+    behind two parts of 128 where sums are many (m 7168, k 6144 at 128 / 192 50.3 / 52.5, 66 /
+    59; k 14336 at 64 / 65 / 256 76 / 92, 84 / 81, 158 / 118), and between there and 12288
+    blocks come out uneven (k 5120, m 9728 at 64 / 96 / 128 62 / 53, 59 / 60, 60 / 57, k
+    3072 at 64 36.5 / 34.8, k 4096 42.3 / 45.0)."""
+    if m % 4 or not 32 < n <= 256 or k < 1024 or not 4096 <= m <= 16384:
+        return False
+    if k <= 2048 or m >= 12288:
+        return True
+    if m > 8192:
+        if n <= 64:
+            return k == 4096
+        return k <= 4096 or n <= 96 or n > 128
+    if m >= 5504:
+        return n <= 64 or k <= 4096 or n <= 128 and k <= 8192
+    return m >= 4608 and k <= 4096 and n * k <= 600 << 10
 
 
 def _streamed_parts(n: int, k: int, m: int) -> bool:

@@ -116,6 +116,14 @@ def test_streamed_product(n, k, m, own):
         (32, 4096, 14336, False), (33, 4096, 14336, True), (256, 4096, 14336, True),
         (257, 4096, 14336, False), (128, 4096, 4092, False), (128, 960, 8192, False),
         (128, 2048, 4096, True), (128, 4096, 16384, True), (128, 4096, 16388, False),
+        # long K that half the chip or an uneven round would sum in one part
+        (256, 14336, 4096, False), (64, 5120, 4096, False), (256, 4096, 4096, False),
+        (128, 4096, 5120, True), (192, 4096, 5120, False), (64, 6144, 5120, False),
+        (192, 3072, 4608, True), (193, 3264, 4608, False), (256, 4096, 5504, True),
+        (128, 8192, 7168, True), (129, 6144, 7168, False), (64, 14336, 8192, True),
+        (65, 14336, 8192, False), (64, 5120, 9728, False), (64, 4096, 9728, True),
+        (64, 3072, 9728, False), (96, 5120, 9728, True), (128, 5120, 9728, False),
+        (129, 5120, 9728, True), (256, 14336, 12288, True), (256, 2048, 4100, True),
     ],
 )
 def test_streamed_gate_up(n, k, m, own):
