@@ -133,12 +133,17 @@ void dense_gemm_kernel(const DenseArgs p) {
   // and wrap around (us, in step / apart: K 2048, M 16384 at 128 rows 19.1 / 18.3, K
   // 4096, M 28672 at 77 57.5 / 43.7, K 14336, M 4096 in 8 parts at 77 26.2 / 25.2). Up to
   // 64 rows a step for 128 features, so that a row's sums do not depend on how many
-  // rows there are, nor on the tile; above, in runs, the XCDs apart too.
+  // rows there are, nor on the tile; above, in runs, the XCDs apart too, with halves two
+  // steps a block, since each reads rows in two places that can lie a power of two apart
+  // (a step / two, us: K 4096, M 16384 at 65 / 96 / 128 rows 51.7 / 43.1, 53.2 / 44.5, 56.5 /
+  // 48.2, M 14336 at 96 42.4 / 42.6, K 8192, M 16384 at 96 86 / 83, M 13824 at 112 82 / 85;
+  // two steps of fewer than 32 leave blocks together: K 1024, M 14336 at 65 13.4 / 14.8).
   constexpr bool APART = STREAM || (TN == 128 && TM == 64 && EPI == BIAS);
   const int rot = !APART ? 0
                   : !STREAM ? (int)(blockIdx.x >> 1) % steps
-                  : TN <= 64 || TM == 64 ? tile / (128 / TM) % steps
-                                         : (nth + 4 * xcd) % steps;
+                  : TN <= 64 || TM == 64   ? tile / (128 / TM) % steps
+                  : HALVES && steps >= 32 ? (2 * nth + 8 * xcd) % steps
+                                          : (nth + 4 * xcd) % steps;
   auto issue = [&](int step, int slot, int i) {
     if constexpr (APART) {
       step += rot;

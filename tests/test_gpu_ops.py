@@ -1377,7 +1377,8 @@ class TestSkinnyGemmEdges:
 
     @pytest.mark.parametrize("N", [17, 33, 64, 65, 96, 97, 128, 129, 192, 193, 256])
     @pytest.mark.parametrize("K,M,glu", [(128, 24580, False), (4096, 24580, False),
-                                         (14336, 2052, False), (128, 12292, True)])
+                                         (14336, 2052, False), (128, 12292, True),
+                                         (1984, 12292, True), (2112, 12292, True)])
     def test_wide_tiles(self, dev, N, K, M, glu):
         """The tiles of 128 features, in one part and in many."""
         self.test_against_fp64(dev, N, K, M, glu)
