@@ -143,6 +143,19 @@ def test_parts_of_streamed_products(native, n):
 
 
 @pytest.mark.parametrize(
+    "n,k,m,parts",
+    [
+        (256, 8192, 2048, 4), (193, 8192, 2048, 4), (192, 8192, 2048, 8), (256, 8256, 2048, 8),
+        (224, 2048, 4096, 2), (193, 3072, 4096, 2), (192, 3072, 4096, 4), (224, 3136, 4096, 4),
+        (224, 4096, 3072, 5),
+    ],
+)
+def test_parts_of_small_weights(native, n, k, m, parts):
+    """Above 192 rows tiles of 128 rows and 64 features, which leave half as many sums."""
+    assert native.ks_skinny_splits(m, k, n, 0) == parts
+
+
+@pytest.mark.parametrize(
     "lens,heads,P,N,chunks",
     [
         ([15], 64, 64, 128, False), ([16] * 4, 64, 64, 128, True),
