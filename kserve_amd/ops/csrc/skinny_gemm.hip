@@ -133,7 +133,10 @@ int few_parts(int M, int K) {
 // in a cache): a launch, the steps of the busiest unit and the sums that are written,
 // off by 5 % in the mean (K 14336, M 4096 at 96 / 256 rows 27.6 / 25.6, 53.6 / 38.6; K
 // 4096, M 4096 10.4 / 11.8, 18.3 / 21.4, M 6144 15.9 / 14.4, 27.0 / 23.7; K 2048, M 16384
-// 16.5 / 23.9, 26.7 / 35.6).
+// 16.5 / 23.9, 26.7 / 35.6); no caller's K is shorter there. Past 8192 features a pass of its own adds the sums, to 10240
+// features the norm's kernel for some callers: those cost less (one part of 64 features /
+// three of 128, with the norm: K 3072, M 10240 at 65 / 160 / 192 rows 26.9 / 23.8, 37.0 /
+// 29.8, 39.8 / 31.1, without at 192 32.8 / 29.5; K 2048 at 65 / 129 19.3 / 21.7, 23.8 / 27.5).
 Plan plan(int M, int K, int N, bool halves) {
   const long rows = halves ? 2L * M : M;
   const int tiles = cdiv(rows, 128), steps = K / BK;
@@ -170,7 +173,7 @@ Plan plan(int M, int K, int N, bool halves) {
     const float us = cost.launch[i] +
                      cost.step[i] * (cdiv(steps, s) * (float)cdiv((long)n * s, UNITS)) +
                      (s > 1 ? cost.sums * 4e-6f * s * N * M : 0.f) +
-                     (s > 1 && M > 8192 ? 6.f : 0.f);  // (a pass of their own adds them)
+                     (s > 1 && M > 8192 ? M > 10240 ? 6.f : 2.5f : 0.f);
     if (i == 0 || us < least) {
       least = us;
       best = {STREAMED, tm, s};

@@ -156,6 +156,18 @@ def test_parts_of_small_weights(native, n, k, m, parts):
 
 
 @pytest.mark.parametrize(
+    "n,k,m,parts",
+    [
+        (65, 3072, 10240, 3), (128, 3072, 10240, 3), (192, 3072, 10240, 3), (160, 3072, 9216, 3),
+        (65, 2048, 10240, 1), (129, 2048, 10240, 1), (192, 3072, 10304, 1), (160, 3072, 8256, 3),
+    ],
+)
+def test_parts_past_8192_features(native, n, k, m, parts):
+    """Sums that the norm's kernel adds for some callers, and those of a pass of their own."""
+    assert native.ks_skinny_splits(m, k, n, 0) == parts
+
+
+@pytest.mark.parametrize(
     "lens,heads,P,N,chunks",
     [
         ([15], 64, 64, 128, False), ([16] * 4, 64, 64, 128, True),
