@@ -25,7 +25,7 @@
 
 extern "C" int ks_mid_wide(int, int, int);
 extern "C" hipError_t ks_mid_gemm(void*, const void*, const void*, const void*, int, int,
-                                  int, long, int, int, int, hipStream_t);
+                                  int, long, int, int, int, int, hipStream_t);
 
 namespace {
 
@@ -182,6 +182,14 @@ Plan plan(int M, int K, int N, bool halves) {
   return best;
 }
 
+// Whether an XCD takes all parts of its features (gemm_tile.h): where 2.5 MB of token
+// rows and its share of the sums fit its L2 of 4 MB (us with the sums added, else / so: K
+// 8192, M 8192 at 129 / 256 rows 39.4 / 36.4, 47.1 / 52.0, K 14336, M 5120 at 192 44.5 /
+// 58.6; K 8192, M 9216 at 160 43.1 / 45.6). Up to 128 rows the sums are few.
+int parts_first(int M, int K, int N) {
+  return N > 128 && M <= 8192 && (long)N * K <= 5 << 18;
+}
+
 hipError_t run(DenseArgs p, int tm, int epi, hipStream_t stream) {
   const bool far = is_long(p.K, p.long_xs);
   if (far) tm = 64;
@@ -203,7 +211,7 @@ hipError_t run(DenseArgs p, int tm, int epi, hipStream_t stream) {
                       : go<256, 64, 4, 2, 4>(p, epi, stream);
   if (N > 192 && !has_halves(epi))
     return ks_mid_gemm(p.out, p.x, p.w, p.bias, p.M, p.K, N, p.long_xs, p.splits, epi == PARTIAL, 128,
-                       stream);
+                       p.parts_first, stream);
   return N <= 32    ? go<32, 128, 2, 2, 7>(p, epi, stream)
          : N <= 64  ? go<64, 128, 2, 2, 6>(p, epi, stream)
          : N <= 96  ? go<96, 128, 2, 2, 5>(p, epi, stream)
@@ -234,11 +242,11 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
   const bool sums = splits > 1 || !out;
   const DenseArgs p{sums ? partial : out, (const short*)x, (const short*)w,
                     (const short*)(sums ? nullptr : bias), M, K, N, (int)xs, 0, 0, splits,
-                    0.f, 0.f, xs};
+                    parts_first(M, K, N), 0.f, 0.f, xs};
   const Plan how = plan(M, K, N, glu);
   const hipError_t err =
       how.form != STREAMED && !is_long(K, xs)
-          ? ks_mid_gemm(p.out, x, w, p.bias, M, K, N, xs, splits, sums, 64, stream)
+          ? ks_mid_gemm(p.out, x, w, p.bias, M, K, N, xs, splits, sums, 64, 0, stream)
           : run(p, how.tm, glu ? GLU : sums ? PARTIAL : BIAS, stream);
   if (err != hipSuccess) return err;
   if (sums && out) {
@@ -262,6 +270,6 @@ extern "C" hipError_t ks_streamed_clamped_glu(void* out, const void* x, const vo
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
     return hipErrorInvalidValue;
   return run({out, (const short*)x, (const short*)w, nullptr, M, K, N, (int)xs, 0, 0, 1,
-              alpha, limit, xs},
+              0, alpha, limit, xs},
              plan(M, K, N, true).tm, CLAMPED, stream);
 }
