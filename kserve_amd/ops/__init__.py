@@ -612,22 +612,33 @@ def _dense_round(n: int, k: int, m: int) -> bool:
 
     By a tenth to a third as a rule (k 512, m 2304 at 2600 / 3500 rows 10.9 / 14.0, 12.8 /
     16.2; k 1024, m 1024 at 8000 18.2 / 20.2; k 1536, m 1536 at 3000 18.0 / 22.9; k 2048, m
-    2048 at 800 / 2000 / 4000 13.9 / 15.6, 17.9 / 21.7, 30.4 / 33.2, m 256 at 8192 14.1 / 20.9,
+    2048 at 2000 / 4000 17.9 / 21.7, 30.4 / 33.2, m 256 at 8192 14.1 / 20.9,
     at 32000 41.4 / 41.1). On longer k by less, since operands that are in no cache cost this
     kernel more (a layer's time against the library's in a chain of an encoder's twelve: k
     3072, m 768 at 5500 / 7000 / 7864 rows -1.4, -3.0, -3.8, k 4096, m 1024 at 3600 / 7000 -7.5,
-    -3.9), and only where its tiles of 128 x 128 fill three quarters of the units: the
-    library splits k (k 3072, m 768 at 1500 / 3600 / 4200 +3.1, +5.3, -0.5, k 4096, m 1024 at
-    1100 / 2600 / 3100 +5.2, -0.3, -2.4). On wider ones the library's times turn from one size
-    to the next (k 2048, m 3072 at 768 / 1280 / 2048 16.4 / 19.3, 24.4 / 21.1, 28.7 / 27.7; k 768,
-    m 4096 at 1400 / 1872 14.0 / 18.5, 19.3 / 17.4; k 4096, m 4096 at 1400 50 / 50), and past one
-    round its tiles are ahead (k 2048, m 768 at 10900 rows 37 / 33, k 3072 58 / 52)."""
+    -3.9), and only where its tiles of 128 x 128 fill more than three quarters of the units:
+    the library splits k (k 3072, m 768 at 1500 / 3600 / 4200 +3.1, +5.3, -0.5, k 4096, m 1024
+    at 1100 / 2600 / 3100 +5.2, -0.3, -2.4; at three quarters k 3072, m 2048 at 1500 31.6 / 27.4,
+    k 4096, m 1536 at 2000 35.8 / 33.0). Of the widest that holds to k 1536 already, while
+    more than 48 tiles are there and too few for the units (k 2048, m 2304 at 257 / 350 / 512 /
+    800 / 900 10.3 / 10.9, 11.6 / 11.3, 17.6 / 14.1, 18.2 / 16.9, 18.6 / 23.8, m 2048 at 300 / 512
+    / 700 / 1150 9.3 / 11.0, 12.4 / 11.3, 15.6 / 13.7, 21.7 / 23.5, k 1536, m 2048 at 512 / 600
+    10.6 / 9.5, 11.9 / 13.2). Its times turn from one size to the next (k 2560, m 2304 at 1700 /
+    2000 / 2600 27 / 30, 37 / 33, 36 / 37), on wider ones more than that (k 2048, m 3072 at 768 /
+    1280 / 2048 16.4 / 19.3, 24.4 / 21.1, 28.7 / 27.7; k 768, m 4096 at 1400 / 1872 14.0 / 18.5,
+    19.3 / 17.4; k 4096, m 4096 at 1400 50 / 50), and past one round its tiles are ahead (k
+    2048, m 768 at 10900 rows 37 / 33, k 3072 58 / 52)."""
+    tiles = -(-n // 128) * -(-m // 128)
     return (
         m % 8 == 0
         and 256 <= m <= 2304
         and 512 <= k <= 4096
         and -(-n // 256) * -(-m // 128) <= 256
-        and (k <= 2048 or -(-n // 128) * -(-m // 128) >= 192)
+        and (
+            tiles > 192
+            if k > 2048
+            else k <= 1024 or m <= 1792 or tiles <= 48 or tiles * 8 > k - 960
+        )
     )
 
 

@@ -249,10 +249,16 @@ def test_encoder_product(n, k, m, gelu, own):
     "n,k,m,own",
     [
         (7864, 3072, 768, True), (10752, 3072, 768, True), (10753, 3072, 768, False),
-        (1409, 4096, 2048, True), (1408, 4096, 2048, False), (4096, 4096, 2048, True),
+        (1537, 4096, 2048, True), (1536, 4096, 2048, False), (4096, 4096, 2048, True),
         (4097, 4096, 2048, False), (2000, 4160, 2048, False), (32768, 2048, 256, True),
         (2000, 2048, 248, False), (1, 512, 256, True), (300, 448, 2304, False),
         (300, 768, 2300, False), (300, 768, 2312, False), (1280, 2048, 3072, False),
+        # too few tiles for the units, too many for one another: the library splits k
+        (1500, 3072, 2048, False), (2000, 4096, 1536, False), (3000, 2560, 1024, False),
+        (1700, 3072, 2048, True), (512, 2048, 2048, False), (1024, 2048, 2048, False),
+        (1025, 2048, 2048, True), (384, 2048, 2048, True), (385, 2048, 2048, False),
+        (512, 1536, 2048, False), (513, 1536, 2048, True), (512, 1024, 2304, True),
+        (512, 2048, 1792, True), (300, 2048, 2304, False), (257, 2048, 2304, False),
     ],
 )
 def test_one_round_of_the_encoders_tiles(n, k, m, own):
