@@ -303,21 +303,30 @@ class TestDecodeAttention:
     @pytest.mark.parametrize(
         "H,Hkv,D,fp8,window,blocks",
         [
-            (4, 1, 128, False, 0, 512), (8, 1, 128, False, 0, 256),
-            (6, 2, 128, False, 768, 192), (6, 2, 128, False, 767, 384),
-            (4, 1, 128, False, 0, 192), (4, 2, 128, False, 50, 192),   # no splits
-            (4, 1, 64, False, 0, 192), (4, 1, 128, True, 0, 192),
+            (4, 1, 128, False, 0, 512), (8, 1, 128, False, 0, 192),   # groups past 5
+            (8, 1, 128, False, 0, 384), (6, 1, 128, False, 50, 256), (8, 1, 64, False, 0, 192),
+            (6, 2, 128, False, 768, 384), (6, 2, 128, False, 767, 384),
+            (4, 1, 128, False, 0, 192), (4, 2, 128, False, 50, 192),
+            (4, 1, 64, False, 0, 192), (4, 1, 128, True, 0, 192), (4, 1, 128, False, 0, 256),
             (3, 1, 64, False, 33, 384), (3, 1, 128, True, 0, 384),
         ],
     )
     def test_four_waves_per_block(self, dev, H, Hkv, D, fp8, window, blocks):
         """Blocks of four waves without splits, two of which end at once where a context
         has few page pairs, in both precisions of the scores; from 512 blocks on two."""
+        import ctypes
+
         from kserve_amd import ops
 
         ctx = [1, 32, 96, 97, 112, 113, 128, 129, 160, 161, 225, 256]
-        if blocks > 192 or D == 128 and not fp8:
-            ctx += [481, 512, 767, 780, 1553]
+        if blocks > 192:
+            ctx += [481, 512, 767, 1553]
+        elif D == 128 and not fp8:
+            ctx += [481, 512, 639, 640]
+        n = -(-blocks // (len(ctx) * Hkv))
+        splits = ctypes.CDLL(ops._C.__file__).ks_paged_decode_splits
+        assert splits(n * len(ctx), Hkv, -(-max(ctx) // 16), D, int(fp8)) == 1
+        assert blocks == 512 or 192 <= n * len(ctx) * Hkv < 512
         torch.manual_seed(H)
         width = -(-max(ctx) // 16)
         NB = len(ctx) * width
@@ -336,7 +345,6 @@ class TestDecodeAttention:
             q.float().cpu(), kc.float().cpu(), vc.float().cpu(), bt, ctx_t,
             D ** -0.5, window=window,
         )
-        n = -(-blocks // (len(ctx) * Hkv))
         many = [x.to(dev) for x in (bt.repeat(n, 1), ctx_t.repeat(n))]
         got = ops.paged_attention_decode(
             q.repeat(n, 1, 1), kc, vc, *many, D ** -0.5, window=window
