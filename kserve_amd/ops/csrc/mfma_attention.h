@@ -1108,31 +1108,38 @@ hipError_t launch_decode(const DecodeArgs& p, int num_seqs, hipStream_t stream) 
 //
 // Below, 512 to 960 blocks (light: 640 to 1024), as even a number on each unit as that
 // allows (us, about 640 blocks / so: 8 of 1500 16.9 / 15.0, of 4000 29.8 / 25.9, 16 of 900
-// 19.0 / 16.9, 32 of 3000 77.9 / 76.9, 40 of 2500 83.5 / 78.1, E4M3 49.2 / 44.8). At most 32
-// (one of 7000: 14 us with 32, 16 with 16). A sequence uses as many of them as it has
-// page pairs for every wave.
+// 19.0 / 16.9, 40 of 2500 83.5 / 78.1, E4M3 49.2 / 44.8); of counts as even as each other the
+// larger up to 640 blocks, since a long context among short ones is what the launch waits
+// for (32 of 3000 76.9 / 77.9, but 24 of 100 and one of 7000, 25 in all, 44.6 / 36.2). At most
+// 32 (one of 7000: 14 us with 32, 16 with 16). A sequence uses as many of them as it has page
+// pairs for every wave.
 //
-// Short contexts have none from UNSPLIT_BLOCKS on: blocks of four waves spare the launch
-// that merges (us, split / not: 24 of 100 9.2 / 6.9, of 400 14.2 / 11.8, of 900 21.1 / 21.0,
-// 32 of 1300 38.4 / 37.2, 63 of 1000 53.2 / 50.4, E4M3 33.1 / 28.4; fp32 queries, 4 KV heads,
-// 64 of 200 14.2 / 11.2, of 1000 33.7 / 30.0). Long ones do, so that one of them is not what
-// the launch waits for (waves of two, 40 of 500 and one of 7000: 118 unsplit, 71 with 2),
-// and between 257 and 383 blocks, one on some units and two on the others (40 of 1200 41
-// / 42), and light pages up to there (24 of 900 E4M3 15.6 / 17.3, heads of 64 12.4 / 13.2).
+// Tables of few pages have none from UNSPLIT_BLOCKS on: blocks of four waves spare the launch
+// that merges (us, split / not: 24 of 100 9.2 / 6.9, of 400 14.2 / 11.8, 32 of 1300 38.4 /
+// 37.2, 63 of 1000 53.2 / 50.4, E4M3 33.1 / 28.4; fp32 queries, 4 KV heads, 64 of 200 14.2 /
+// 11.2, of 1000 33.7 / 30.0). How few is what one long context among short ones allows: 40
+// pages up to 255 blocks (others of 100: 24 with one of 640 11.3 / 11.1, of 1500 14.4 / 18.6,
+// of 2000 16.3 / 22.8), 128 at one block a unit and from 384 on (32 with one of 1500 22.9 /
+// 18.9, 48 22.1 / 19.3), 40 again between, one on some units and two on the others (40
+// of 1200 41 / 42); light pages 16 up to there (24 of 900 E4M3 15.6 / 17.3, heads of 64 12.4 /
+// 13.2). The width of the table stands for the longest context: a captured step's is the
+// longest that the model allows, so the models of more than 2048 tokens keep their splits
+// there (24 of 400 15.0 with 512 pages a row, 12.4 with as many as it needs).
 inline int decode_splits(int num_seqs, int num_kv_heads, int max_blocks, bool light) {
   const long base = (long)num_seqs * num_kv_heads;
   if (base <= 0 || base >= FULL_BLOCKS) return 1;
   const int short_pages = base >= 384 ? 128
                           : light     ? 16
-                          : base > 256 ? 40
-                                       : 128;
+                          : base == 256 ? 128
+                                        : 40;
   if (base >= UNSPLIT_BLOCKS && max_blocks <= short_pages) return 1;
   const long least = light ? 640 : 512, target = light ? 1024 : 960;
   long n = (least + base - 1) / base;
   // blocks of the busiest unit, each with 1 / t of the context
   auto rounds = [&](long t) { return (base * t + 255) / 256; };
+  const long even = (640 + base - 1) / base;  // up to here the larger of two that tie
   for (long t = n + 1; t * base <= target; ++t)
-    if (rounds(t) * n < rounds(n) * t) n = t;
+    if (rounds(t) * n < rounds(n) * t + (t <= even)) n = t;
   const long most = ((long)max_blocks + 2 * WAVES - 1) / (2 * WAVES);
   if (n > most) n = most;
   if (n > 32) n = 32;

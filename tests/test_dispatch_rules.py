@@ -168,6 +168,31 @@ def test_parts_past_8192_features(native, n, k, m, parts):
 
 
 @pytest.mark.parametrize(
+    "seqs,pages,dim,fp8,splits",
+    [
+        (24, 40, 128, 0, 1), (24, 41, 128, 0, 4), (24, 125, 128, 0, 4), (31, 128, 128, 0, 3),
+        (32, 128, 128, 0, 1), (32, 129, 128, 0, 3), (33, 40, 128, 0, 1), (33, 41, 128, 0, 3),
+        (48, 128, 128, 0, 1), (48, 129, 128, 0, 2), (64, 512, 128, 0, 1), (23, 10, 128, 0, 3),
+        (24, 16, 128, 1, 1), (24, 17, 128, 1, 4), (24, 17, 64, 0, 4), (48, 128, 128, 1, 1),
+        (16, 512, 128, 0, 4), (25, 512, 128, 0, 4), (1, 512, 128, 0, 32), (0, 512, 128, 0, 1),
+    ],
+)
+def test_decode_splits(native, seqs, pages, dim, fp8, splits):
+    """8 KV heads: none for tables too short for one long context to hold up the launch;
+    of counts that fill the units alike the larger."""
+    assert native.ks_paged_decode_splits(seqs, 8, pages, dim, fp8) == splits
+
+
+def test_decode_splits_are_no_fewer(native):
+    """Where contexts can be long there are as many blocks as one and a quarter a unit
+    take, or fewer only where that leaves the units more even."""
+    for base in range(1, 512):
+        n, least = native.ks_paged_decode_splits(base, 1, 4096, 128, 0), min(-(-640 // base), 32)
+        rounds = lambda t: -(-base * t // 256) / t  # of blocks on the busiest unit, in contexts
+        assert n >= least or rounds(n) < rounds(least), base
+
+
+@pytest.mark.parametrize(
     "lens,heads,P,N,chunks",
     [
         ([15], 64, 64, 128, False), ([16] * 4, 64, 64, 128, True),
