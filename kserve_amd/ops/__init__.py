@@ -521,8 +521,14 @@ def _streamed_rows(n: int, k: int, m: int) -> bool:
     to five eighths of the units at least, and where rows lie a multiple of 4 KB apart or
     are short (k 5120, m 28672 at 96 / 128 rows 66 / 65, 73 / 71; k 14336, m 20480 at 128 169 /
     157). Up to 64 rows on short k or full rounds only (k 4096, m 12288 at 33 rows 26.7 /
-    25.2)."""
+    25.2). Not where the library's blocks come to two thirds of the units and the streamed ones
+    to half (k 2560, m 9216 at 129 / 176 / 192 rows 24.5 / 22.1, 28.1 / 23.5, 28.8 / 31.9, m
+    8704 at 96 / 112 21.7 / 21.5, 23.4 / 21.5; k 3072, m 10752 at 176 31.9 / 26.6). Captured
+    steps of 128 sequences are level with the library's product to the vocabulary (k 4096, m
+    32000; contexts of 500 / 2000 tokens 768 / 764, 1292 / 1298), of 256 ahead (1101 / 1118)."""
     if m % 4 or not 48 < n <= 256 or k < 1024:
+        return False
+    if m < 11264 and 2048 < k < 4096 and (96 if 2304 < k < 3072 else 128) < n < 192:
         return False
     if n <= 64:
         return 8192 < m <= 16384 and (k <= 2048 or m > 12288 and k <= 5120)

@@ -104,6 +104,10 @@ def test_few_row_gate_up(n, k, m, own):
         (129, 2048, 20352, False), (256, 4096, 20356, True), (128, 5120, 28672, False),
         (128, 8192, 32768, True), (128, 8192, 32772, False), (128, 12288, 28672, False),
         (80, 2048, 10302, False),
+        (129, 2560, 9216, False), (191, 3072, 11260, False), (192, 2560, 9216, True),
+        (144, 2048, 9216, True), (144, 4096, 9216, True), (144, 2560, 11264, True),
+        (96, 2560, 8704, True), (97, 2560, 8704, False), (128, 2304, 8704, True),
+        (128, 3072, 10752, True), (129, 2304, 8704, False),
     ],
 )
 def test_streamed_product(n, k, m, own):
