@@ -430,8 +430,8 @@ def _skinny_rows(n: int, k: int, m: int) -> bool:
     k 2048, m 32000 at 96 26 / 34; but m 16384 22 / 19), and at k 2048 to 128 where their
     tiles of 128 features fill seven eighths of the units' last round (at 128 rows m 32000
     31 / 35, captured steps of 128 sequences with it 824 / 837, m 65536 64 / 71, 98304 99 / 108,
-    128256 129 / 127; but m 24576 30 / 28, 50304 59 / 52). Not so at longer k: k 4096, m 32000
-    54 / 61 by itself, but captured steps 759 / 753, m 128256 236 / 231, k 6144, m 62464 162 /
+    128256 129 / 127; but m 24576 30 / 28, 50304 59 / 52). Not so at longer k (see `_streamed_rows`
+    for m to 32768): m 128256 236 / 231, k 6144, m 62464 162 /
     159, k 8192, m 65536 226 / 198.
     Otherwise it gains above where the
     library does not split K over the chip: k 14336, m 4096 at 128 / 256 rows 34 / 74,
@@ -632,7 +632,9 @@ def _dense_round(n: int, k: int, m: int) -> bool:
     10.6 / 9.5, 11.9 / 13.2). Its times turn from one size to the next (k 2560, m 2304 at 1700 /
     2000 / 2600 27 / 30, 37 / 33, 36 / 37), on wider ones more than that (k 2048, m 3072 at 768 /
     1280 / 2048 16.4 / 19.3, 24.4 / 21.1, 28.7 / 27.7; k 768, m 4096 at 1400 / 1872 14.0 / 18.5,
-    19.3 / 17.4; k 4096, m 4096 at 1400 50 / 50), and past one round its tiles are ahead (k
+    19.3 / 17.4; k 4096, m 4096 at 1400 50 / 50; without a bias m 2560 to
+    3072 would mostly gain a tenth to a third to k 1536, and at some sizes k 2048 lose as much),
+    and past one round its tiles are ahead (k
     2048, m 768 at 10900 rows 37 / 33, k 3072 58 / 52)."""
     tiles = -(-n // 128) * -(-m // 128)
     return (

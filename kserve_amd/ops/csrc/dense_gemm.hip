@@ -97,20 +97,19 @@ extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
   return hipSuccess;
 }
 
-// Wide products of 65 to 128 rows in one round of blocks of 64 features and all rows, 8
-// waves, K in one part. Bound by the reads of W and, per unit, as many of x. us, here /
-// the few-row kernel / the library at 65 and 128 rows, weights not in a cache: K 512, M
-// 10304 5.6 / 11.3 / 10.0, 6.1 / 15.8 / 10.5; K 1088, M 16384 9.5 / 15.2 / 14.6, 11.2 / 19.5
-// / 14.8; K 1984, M 10304 13.1 / 15.9 / 21.0, 16.0 / 20.4 / 21.7; K 2304, M 12288 15.4 / 19.2 /
-// 17.6, 18.9 / 24.6 / 20.5; K 3072, M 16384 21.3 / 25.0 / 24.0, 26.6 / 30.8 / 27.2; K 4096, M
-// 14336 25.3 / 28.0 / 30.5, 29.9 / 35.2 / 33.0; K 4608, M 16384 29.9 / 33.6 / 32.7, 36.6 / 40.2 /
-// 36.8. Not past K 4608, where it turns (K 5120, M 12288 at 65 / 112 rows 32.1 / 33.9 / 33.3,
-// 37.5 / 39.9 / 36.0, M 16384 at 128 43.9 / 44.9 / 41.5), nor where K is long and a quarter of
-// the units idle (K 4096, M 10304 23.8 / 22.4 / 38.7, 28.2 / 28.4 / 30.6); past 256 tiles a
-// second round is nearly empty (K 2048, M 17408 26.4 / 23.3 / 27.5). The line at 129 tiles is
-// from weights that came through the caches (K 2048, M 8192 at 128 rows 16.9 / 18.8 / 15.7);
-// as they are loaded now these are ahead at 128 too (14.8 / 18.2 / 15.8, K 512 6.5 / 14.3 /
-// 9.9), and it could be lower.
+// Wide products of 65 to 128 rows in one round of blocks of 64 features and all rows, K in
+// one part: from 97 rows on 8 waves here, below on the streaming tiles of 96 rows
+// (skinny_gemm.hip). Bound by the reads of W and, per unit, as many of x. us, so / the
+// library at 65, 96 and 128 rows, weights not in a cache: K 1024, M 10304 8.5 / 13.1, 9.3 /
+// 13.5, 10.4 / 14.1; K 2048, M 10304 13.7 / 21.4, 15.1 / 17.7, 17.0 / 18.9, M 16384 15.0 /
+// 19.2, 16.4 / 19.9, 18.0 / 21.0; K 3072, M 16384 21.4 / 25.7, 23.4 / 27.8, 27.7 / 29.6; K
+// 4096, M 14336 24.6 / 31.6, 27.2 / 33.3, 30.9 / 35.0. The lines are from a kernel before, of
+// which these were ahead by a tenth to a half: not past K 4608, where that turned (K 5120, M
+// 12288 at 65 / 112 rows 32.1 / 33.9, 37.5 / 39.9, M 16384 at 128 43.9 / 44.9), nor where K is
+// long and a quarter of the units idle (K 4096, M 10304 23.8 / 22.4, 28.2 / 28.4); past 256
+// tiles a second round is nearly empty (K 2048, M 17408 26.4 / 23.3); the line at 129 tiles is
+// from weights that came through the caches (K 2048, M 8192 at 128 rows 16.9, library 15.7,
+// as they are loaded now 14.8), and it could be lower.
 static bool mid_wide(int M, int K, int N) {
   const int tiles = (M + 63) / 64;
   return N > 64 && N <= 128 && tiles <= UNITS && K >= 512 && K <= 4608 &&

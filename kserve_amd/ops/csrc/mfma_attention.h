@@ -1060,8 +1060,11 @@ void launch_decode_waves(const DecodeArgs& p, int num_seqs, hipStream_t stream) 
 // stages are half as large, so that four take the LDS of two, and long contexts among
 // short ones end sooner (us, 2 / 4 waves: 96 of 3000 +- 60% 114.2 / 109.3, 192 of 1500
 // 101.8 / 95.4, 250 of 1000 +- 60% 102.6 / 97.5, of 150 20.3 / 22.0; before, with stages
-// widened in LDS, 119, 113, 104 and 22.3). Not past 4096 blocks (1000 of 16 tokens 23.5 /
-// 35.2) nor in many splits, which are short (one of 2000 8.6 / 8.9).
+// widened in LDS, 119, 113, 104 and 22.3). Behind where contexts are about as long as
+// those from which on all four work (before / now 96 / 128 of 400 +- 60 % 21.3 / 23.3, 24.8
+// / 28.3; a higher line moves that to longer ones and gives up 96 of 100 with one of 640,
+// 16.9 / 12.6). Not past 4096 blocks (1000 of 16 tokens 23.5 / 35.2) nor in many splits,
+// which are short (one of 2000 8.6 / 8.9).
 constexpr long MOST_DEEP_BLOCKS = 4096;
 
 // bf16 pages stay with two where splits leave none: four are ahead on long contexts, but

@@ -4,7 +4,7 @@
 //
 // A block takes 64 or 128 features and all tokens over a range of K, on the tiles of
 // gemm_tile.h: 4 waves (8 above 128 rows), the ring as deep as LDS lets it be (64
-// features: two blocks a unit up to 128 rows). K is split over blocks until the chip is
+// features: two blocks a unit up to 96 rows). K is split over blocks until the chip is
 // full; the parts leave fp32 sums that the consumer's kernel or a second one adds in
 // order (no atomics). With halves a block's rows are as many gate as up features and
 // the activation leaves it directly.
