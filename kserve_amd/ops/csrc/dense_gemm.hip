@@ -25,7 +25,14 @@ namespace {
 // Which tile: the least a n + b, for n tiles on the busiest unit (a quarter more for
 // an odd one where two blocks share a unit: alone it hides less of its latency). a
 // and b are us at K 768 without gelu, fitted over 768 to 3072 features and 1200 to
-// 12000 rows; all grow with K and gelu alike, so the order holds. Where a unit has a
+// 12000 rows; all grow with K and gelu alike, so the order holds but for the largest tile,
+// whose one round has nothing to hide its first loads and its output behind: on short K
+// it is not taken (us, tiles of 128 x 128 / so, at K 128, 256, 384, 512, 640, 768, 1024, 1536:
+// 8086 x K to 1896 11.2 / 12.9, 15.4 / 15.9, 18.2 / 20.9, 21.6 / 23.9, 26.1 / 26.5, 29.3 / 29.5,
+// 34.6 / 35.3, 49.2 / 46.7; 2886 to 2312 7.4 / 8.4, 8.9 / 9.7, 10.9 / 11.2, 12.6 / 12.9, 14.5 /
+// 14.0, 16.1 / 16.2, 19.6 / 18.4, 26.7 / 23.9; with gelu 4800 to 3072 15.9 / 17.7, 19.1 / 21.2,
+// 22.5 / 24.4, 25.7 / 26.9, 29.3 / 30.6, 33.2 / 33.7, 39.6 / 39.0, 54.8 / 50.5; than tiles of 64 x 128 it is better from K
+// 512 on, 5429 to 1024 12.0 / 11.1, 3034 to 2048 13.1 / 12.5). Where a unit has a
 // single tile, one block of eight waves with a deeper ring beats one of four (7864 x
 // 768 to 768 13.5 / 15.0, 1200 to 2304 10.5 / 12.8). The largest tile is for what it
 // alone brings into one round (us, without / with it: 9000 x 768 to 768 15.7 / 14.7, 2048
@@ -36,7 +43,7 @@ struct Tile {
   float a, b;
   bool pairs;
 };
-constexpr int NTILES = 7;
+constexpr int NTILES = 7, LARGEST = 6;
 constexpr Tile TILES[NTILES] = {
     {128, 192, 12.6f, 0.5f, false}, {128, 192, 9.8f, 2.f, true},
     {128, 128, 9.5f, 0.f, false},   {128, 128, 7.2f, 2.2f, true},
@@ -45,10 +52,11 @@ constexpr Tile TILES[NTILES] = {
 
 }  // namespace
 
-extern "C" int ks_dense_tile(int M, int N) {
+extern "C" int ks_dense_tile(int M, int N, int K) {
   int best = 0;
   float least = 0.f;
   for (int i = 0; i < NTILES; ++i) {
+    if (i == LARGEST && K < (TILES[best].pairs ? 704 : 512)) continue;
     const Tile& t = TILES[i];
     const long tiles = (long)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
     const long n = (tiles + UNITS - 1) / UNITS;
@@ -70,7 +78,7 @@ extern "C" hipError_t ks_dense_gemm(void* out, const void* x, const void* w,
       xs % 8 != 0 || xs < K || xs >= 1 << 22 || tile >= NTILES ||
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)bias) & 15) != 0)
     return hipErrorInvalidValue;
-  if (tile < 0) tile = ks_dense_tile(M, N);
+  if (tile < 0) tile = ks_dense_tile(M, N, K);
   const Tile& t = TILES[tile];
   const long ftiles = (M + t.tm - 1) / t.tm, tiles = ftiles * ((N + t.tn - 1) / t.tn);
   if (tiles > 0x7fffffff) return hipErrorInvalidValue;

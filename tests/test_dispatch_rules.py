@@ -172,6 +172,19 @@ def test_parts_past_8192_features(native, n, k, m, parts):
 
 
 @pytest.mark.parametrize(
+    "m,n,k,tile",
+    [
+        (1896, 8086, 64, 3), (1896, 8086, 640, 3), (1896, 8086, 704, 6), (2312, 2886, 256, 3),
+        (3072, 4800, 512, 3), (3072, 4800, 1024, 6), (1024, 5429, 448, 4), (1024, 5429, 512, 6),
+        (2048, 3034, 320, 4), (2608, 13970, 384, 1), (2608, 13970, 768, 6), (768, 7864, 3072, 0),
+    ],
+)
+def test_tile_of_many_rows(native, m, n, k, tile):
+    """The largest tile's one round of blocks is behind on short K."""
+    assert native.ks_dense_tile(m, n, k) == tile
+
+
+@pytest.mark.parametrize(
     "seqs,pages,dim,fp8,splits",
     [
         (24, 40, 128, 0, 1), (24, 41, 128, 0, 4), (24, 125, 128, 0, 4), (31, 128, 128, 0, 3),
