@@ -137,6 +137,14 @@ int few_parts(int M, int K) {
 // features the norm's kernel for some callers: those cost less (one part of 64 features /
 // three of 128, with the norm: K 3072, M 10240 at 65 / 160 / 192 rows 26.9 / 23.8, 37.0 /
 // 29.8, 39.8 / 31.1, without at 192 32.8 / 29.5; K 2048 at 65 / 129 19.3 / 21.7, 23.8 / 27.5).
+//
+// At 129 to 192 rows blocks of 64 features fall behind where K is long: in parts from token
+// rows of 1.4 MB on, in one part from K 3840 on, but where the other's two parts lie a
+// multiple of 4 KB apart (us, 64 features / 128, with the sums added: M 13824, K 3584 at 160 /
+// 176 rows 34.2 / 35.7, 36.3 / 37.7, K 4608 43.3 / 41.8, 46.4 / 43.3, K 5120 52.9 / 45.7, 53.9 /
+// 46.7, but M 16384, K 4096 at 176 38.5 / 40.9; M 4352, K 4096 at 160 / 176 21.4 / 22.8, 22.4 /
+// 23.3, K 5120 26.0 / 23.8, 27.8 / 24.7; M 5120, K 6144 29.9 / 26.5, 30.1 / 27.6). Over K 2112 to
+// 8192 and M 4352 to 16384 this takes the better one to 0.1 % in the mean, to 4 % without.
 Plan plan(int M, int K, int N, bool halves) {
   const long rows = halves ? 2L * M : M;
   const int tiles = cdiv(rows, 128), steps = K / BK;
@@ -166,6 +174,7 @@ Plan plan(int M, int K, int N, bool halves) {
                {{0.f, 2.f}, {0.58f, 0.79f}, 0.4f},
                {{0.f, 0.5f}, {0.8f, 0.92f}, 0.5f}};
   const auto& cost = COST[N <= 96 ? 0 : N <= 128 ? 1 : N <= 192 ? 2 : 3];
+  const bool long_k = !halves && N > 128 && N <= 192 && M > 4096;
   Plan best{STREAMED, 64, 1};
   float least = 0.f;
   for (int i = 0; i < 2; ++i) {
@@ -173,7 +182,10 @@ Plan plan(int M, int K, int N, bool halves) {
     const float us = cost.launch[i] +
                      cost.step[i] * (cdiv(steps, s) * (float)cdiv((long)n * s, UNITS)) +
                      (s > 1 ? cost.sums * 4e-6f * s * N * M : 0.f) +
-                     (s > 1 && M > 8192 ? M > 10240 ? 6.f : 2.5f : 0.f);
+                     (s > 1 && M > 8192 ? M > 10240 ? 6.f : 2.5f : 0.f) +
+                     (i == 0 && long_k && (s > 1 ? (long)N * K > 725000 : K >= 3840 && K % 4096 != 0)
+                          ? 8.f
+                          : 0.f);
     if (i == 0 || us < least) {
       least = us;
       best = {STREAMED, tm, s};

@@ -152,6 +152,7 @@ def test_parts_of_streamed_products(native, n):
         (256, 8192, 2048, 4), (193, 8192, 2048, 4), (192, 8192, 2048, 8), (256, 8256, 2048, 8),
         (224, 2048, 4096, 2), (193, 3072, 4096, 2), (192, 3072, 4096, 4), (224, 3136, 4096, 4),
         (224, 4096, 3072, 5),
+        (176, 4096, 4352, 3), (160, 5120, 4352, 7), (177, 4096, 4352, 3), (192, 4096, 4352, 7),
     ],
 )
 def test_parts_of_small_weights(native, n, k, m, parts):
@@ -164,6 +165,9 @@ def test_parts_of_small_weights(native, n, k, m, parts):
     [
         (65, 3072, 10240, 3), (128, 3072, 10240, 3), (192, 3072, 10240, 3), (160, 3072, 9216, 3),
         (65, 2048, 10240, 1), (129, 2048, 10240, 1), (192, 3072, 10304, 1), (160, 3072, 8256, 3),
+        # long K: tiles of 128 features in two parts rather than of 64 in one
+        (176, 5120, 13824, 2), (192, 6144, 16384, 2), (145, 3840, 13824, 2),
+        (176, 3776, 13824, 1), (192, 4096, 13824, 1), (128, 5120, 16640, 1),
     ],
 )
 def test_parts_past_8192_features(native, n, k, m, parts):

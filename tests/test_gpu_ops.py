@@ -1422,7 +1422,8 @@ class TestSkinnyGemmEdges:
         "N,K,M", [(65, 8192, 2048), (129, 8192, 2052), (256, 2112, 772),
                   (128, 4096, 4096), (129, 14336, 4100), (200, 4096, 6144),
                   (193, 8192, 2044), (225, 3072, 4092), (161, 3072, 10236),
-                  (129, 4096, 8188), (193, 4096, 5116), (129, 3072, 8180), (256, 5120, 7172)]
+                  (129, 4096, 8188), (193, 4096, 5116), (129, 3072, 8180), (256, 5120, 7172),
+                  (145, 3904, 13828), (177, 5120, 4356)]
     )
     def test_parts_of_many_rows(self, dev, N, K, M):
         """Narrow and wide weights above 64 and 128 rows, in parts of K."""
