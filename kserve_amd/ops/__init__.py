@@ -523,12 +523,17 @@ def _streamed_rows(n: int, k: int, m: int) -> bool:
     157). Up to 64 rows on short k or full rounds only (k 4096, m 12288 at 33 rows 26.7 /
     25.2). Not where the library's blocks come to two thirds of the units and the streamed ones
     to half (k 2560, m 9216 at 129 / 176 / 192 rows 24.5 / 22.1, 28.1 / 23.5, 28.8 / 31.9, m
-    8704 at 96 / 112 21.7 / 21.5, 23.4 / 21.5; k 3072, m 10752 at 176 31.9 / 26.6). Captured
+    8704 at 96 / 112 21.7 / 21.5, 23.4 / 21.5; k 3072, m 10752 at 176 31.9 / 26.6), nor past 13568
+    features, where from 161 to 191 rows its blocks fill the units, on whole steps of 128 of k
+    (k 2560, m 13824 at 176 29.3 / 27.8, k 3072 at 176 / 191 32.8 / 30.0, 33.8 / 30.5, k 4608 42.1 /
+    40.9; but m 13568 32.7 / 32.3, k 3904 37.8 / 42.1, k 2304 and 4096 a tenth ahead). Captured
     steps of 128 sequences are level with the library's product to the vocabulary (k 4096, m
     32000; contexts of 500 / 2000 tokens 768 / 764, 1292 / 1298), of 256 ahead (1101 / 1118)."""
     if m % 4 or not 48 < n <= 256 or k < 1024:
         return False
     if m < 11264 and 2048 < k < 4096 and (96 if 2304 < k < 3072 else 128) < n < 192:
+        return False
+    if 13568 < m <= 16384 and 160 < n < 192 and 2304 < k < 4736 and k % 128 == 0 and k != 4096:
         return False
     if n <= 64:
         return 8192 < m <= 16384 and (k <= 2048 or m > 12288 and k <= 5120)

@@ -106,6 +106,10 @@ def test_few_row_gate_up(n, k, m, own):
         (80, 2048, 10302, False),
         (129, 2560, 9216, False), (191, 3072, 11260, False), (192, 2560, 9216, True),
         (144, 2048, 9216, True), (144, 4096, 9216, True), (144, 2560, 11264, True),
+        (176, 3072, 13824, False), (161, 2560, 16384, False), (191, 4608, 13572, False),
+        (176, 3072, 13568, True), (160, 3072, 13824, True), (192, 3072, 13824, True),
+        (176, 2304, 13824, True), (176, 4096, 13824, True), (176, 3904, 13824, True),
+        (176, 4736, 13824, True),
         (96, 2560, 8704, True), (97, 2560, 8704, False), (128, 2304, 8704, True),
         (128, 3072, 10752, True), (129, 2304, 8704, False),
     ],
