@@ -131,7 +131,7 @@ extern "C" int ks_mid_wide(int M, int K, int N) { return mid_wide(M, K, N); }
 // is one
 extern "C" hipError_t ks_mid_gemm(void* out, const void* x, const void* w,
                                   const void* bias, int M, int K, int N, long xs,
-                                  int splits, int sums, int tm, int parts_first,
+                                  int splits, int sums, int tm, int order,
                                   hipStream_t stream) {
   if ((bias && (sums || M % 8 != 0)) || N < 1 || N > 256 || M < 4 || M % 4 != 0 || K < BK || K % BK != 0 ||
       K >= 1 << 22 || xs % 8 != 0 || xs >= 1 << 22 || splits < 1 || splits > K / BK ||
@@ -139,7 +139,7 @@ extern "C" hipError_t ks_mid_gemm(void* out, const void* x, const void* w,
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)bias) & 15) != 0)
     return hipErrorInvalidValue;
   DenseArgs p{out, (const short*)x, (const short*)w, (const short*)bias, M, K, N, (int)xs,
-              0, 0, splits, parts_first, 0.f, 0.f, xs};
+              0, 0, splits, order, 0.f, 0.f, xs};
 #define GO(tn, tm, wn, wm, s, epi, stream_)                                           \
   {                                                                                   \
     p.ftiles = (M + tm - 1) / tm;                                                     \

@@ -23,6 +23,10 @@ constexpr int BK = 64;  // K per step
 enum Epilogue { BIAS, BIAS_GELU, PARTIAL, GLU, CLAMPED };
 constexpr bool has_halves(int epi) { return epi == GLU || epi == CLAMPED; }
 
+// Blocks of an XCD: runs of tiles, part of K by part of K; runs with all parts of their
+// features; every eighth block.
+enum Order { RUNS, PARTS_FIRST, IN_TURN };
+
 struct DenseArgs {
   void* out;          // [N][M] bf16; PARTIAL: [splits][N][M] fp32
   const short* x;     // [N][K], row stride xs
@@ -31,7 +35,7 @@ struct DenseArgs {
   int M, K, N, xs;
   int ftiles, tiles;   // tiles along M, in all
   int splits;          // STREAM: parts of K
-  int parts_first;     // STREAM, PARTIAL: which runs an XCD takes
+  int order;           // STREAM, PARTIAL: which blocks an XCD takes
   float alpha, limit;  // CLAMPED
   long long_xs;        // LONG: the row stride
 };
@@ -94,15 +98,20 @@ void dense_gemm_kernel(const DenseArgs p) {
 
   // Blocks go to the 8 XCDs in turn. Each takes a run of tiles, features first (STREAM:
   // part of K by part of K), which share their token rows in its L2; the narrow
-  // streaming tiles go in turn themselves. `parts_first`: a run has all parts of its
+  // streaming tiles go in turn themselves. PARTS_FIRST: a run has all parts of its
   // features, whose sums are then mostly in the L2 that the blocks which add them read
   // through (us with the sums added in a pass / by the norm, else -> so: K 4096, M 8192 at
   // 129 / 193 rows 30.3 -> 25.5, 32.7 -> 31.0 / 31.6 -> 29.7, 33.7 -> 32.1; K 8192, M 8192 at
   // 129 39.4 -> 36.4 / 44.0 -> 39.5; K 5120, M 5120 at 224 30.1 -> 29.1 / 31.7 -> 31.6; the
-  // product alone 2 % slower), while the token rows still fit beside them.
+  // product alone 2 % slower), while the token rows still fit beside them. IN_TURN: an XCD has
+  // features from all over, which come out even for what adds them (us with the sums added
+  // in a pass, runs / in turn, 256 rows of 128 features: K 6144, M 4352 at 224 / 256 30.5 / 29.6,
+  // 31.7 / 30.5, K 3072, M 8704 31.5 / 30.1, 33.0 / 31.3, K 4096 34.2 / 32.8, 35.7 / 34.7, K 6144 42.7 /
+  // 41.5, 44.4 / 43.8).
   constexpr bool HALVES = has_halves(EPI);
-  const bool parts_first = STREAM && EPI == PARTIAL && TN > 128 && p.parts_first;
-  const bool runs = !STREAM || TM == 128 || parts_first;
+  const bool parts_first = STREAM && EPI == PARTIAL && TN > 128 && p.order == PARTS_FIRST;
+  const bool in_turn = STREAM && EPI == PARTIAL && TN == 256 && p.order == IN_TURN;
+  const bool runs = !STREAM || (TM == 128 && !in_turn) || parts_first;
   const int xcd = blockIdx.x & 7, nth = blockIdx.x >> 3;
   const int count = STREAM ? p.tiles * p.splits : p.tiles;
   const int at_tile = runs ? xcd * (count >> 3) + min(xcd, count & 7) + nth : blockIdx.x;

@@ -138,12 +138,13 @@ int few_parts(int M, int K) {
 // three of 128, with the norm: K 3072, M 10240 at 65 / 160 / 192 rows 26.9 / 23.8, 37.0 /
 // 29.8, 39.8 / 31.1, without at 192 32.8 / 29.5; K 2048 at 65 / 129 19.3 / 21.7, 23.8 / 27.5).
 //
-// At 129 to 192 rows blocks of 64 features fall behind where K is long: in parts from token
-// rows of 1.4 MB on, in one part from K 3840 on, but where the other's two parts lie a
+// At 129 to 192 rows blocks of 64 features fall behind where K is long: in more than two
+// parts from token rows of 1.6 MB on, in two of 1.4, in one part from K 3840 on, but where the other's two parts lie a
 // multiple of 4 KB apart (us, 64 features / 128, with the sums added: M 13824, K 3584 at 160 /
 // 176 rows 34.2 / 35.7, 36.3 / 37.7, K 4608 43.3 / 41.8, 46.4 / 43.3, K 5120 52.9 / 45.7, 53.9 /
-// 46.7, but M 16384, K 4096 at 176 38.5 / 40.9; M 4352, K 4096 at 160 / 176 21.4 / 22.8, 22.4 /
-// 23.3, K 5120 26.0 / 23.8, 27.8 / 24.7; M 5120, K 6144 29.9 / 26.5, 30.1 / 27.6). Over K 2112 to
+// 46.7, but M 16384, K 4096 at 176 38.5 / 40.9; M 4352, K 4096 at 160 / 192 21.4 / 22.8, 23.7 /
+// 24.1, K 5120 at 160 / 176 26.0 / 23.8, 27.8 / 24.7; M 7168, K 4096 at 176 / 192 28.1 / 25.9, 29.6 /
+// 26.7; M 5120, K 6144 29.9 / 26.5, 30.1 / 27.6). Over K 2112 to
 // 8192 and M 4352 to 16384 this takes the better one to 0.1 % in the mean, to 4 % without.
 Plan plan(int M, int K, int N, bool halves) {
   const long rows = halves ? 2L * M : M;
@@ -183,7 +184,9 @@ Plan plan(int M, int K, int N, bool halves) {
                      cost.step[i] * (cdiv(steps, s) * (float)cdiv((long)n * s, UNITS)) +
                      (s > 1 ? cost.sums * 4e-6f * s * N * M : 0.f) +
                      (s > 1 && M > 8192 ? M > 10240 ? 6.f : 2.5f : 0.f) +
-                     (i == 0 && long_k && (s > 1 ? (long)N * K > 725000 : K >= 3840 && K % 4096 != 0)
+                     (i == 0 && long_k &&
+                              (s > 1 ? (long)N * K > (s > 2 ? 800000 : 700000)
+                                     : K >= 3840 && K % 4096 != 0)
                           ? 8.f
                           : 0.f);
     if (i == 0 || us < least) {
@@ -197,9 +200,12 @@ Plan plan(int M, int K, int N, bool halves) {
 // Whether an XCD takes all parts of its features (gemm_tile.h): where 2.5 MB of token
 // rows and its share of the sums fit its L2 of 4 MB (us with the sums added, else / so: K
 // 8192, M 8192 at 129 / 256 rows 39.4 / 36.4, 47.1 / 52.0, K 14336, M 5120 at 192 44.5 /
-// 58.6; K 8192, M 9216 at 160 43.1 / 45.6). Up to 128 rows the sums are few.
-int parts_first(int M, int K, int N) {
-  return N > 128 && M <= 8192 && (long)N * K <= 5 << 18;
+// 58.6; K 8192, M 9216 at 160 43.1 / 45.6). Up to 128 rows the sums are few. Every eighth
+// block above 192 rows to K 6144, past which runs' token rows count for more (K 8192 at 193
+// rows, runs / in turn, M 4352 32.7 / 34.8, M 9728 50.0 / 50.5; K 14336 level).
+Order order(int M, int K, int N) {
+  if (N > 128 && M <= 8192 && (long)N * K <= 5 << 18) return PARTS_FIRST;
+  return N > 192 && K <= 6144 ? IN_TURN : RUNS;
 }
 
 hipError_t run(DenseArgs p, int tm, int epi, hipStream_t stream) {
@@ -223,7 +229,7 @@ hipError_t run(DenseArgs p, int tm, int epi, hipStream_t stream) {
                       : go<256, 64, 4, 2, 4>(p, epi, stream);
   if (N > 192 && !has_halves(epi))
     return ks_mid_gemm(p.out, p.x, p.w, p.bias, p.M, p.K, N, p.long_xs, p.splits, epi == PARTIAL, 128,
-                       p.parts_first, stream);
+                       p.order, stream);
   return N <= 32    ? go<32, 128, 2, 2, 7>(p, epi, stream)
          : N <= 64  ? go<64, 128, 2, 2, 6>(p, epi, stream)
          : N <= 96  ? go<96, 128, 2, 2, 5>(p, epi, stream)
@@ -254,11 +260,11 @@ extern "C" hipError_t ks_skinny_gemm(void* out, void* partial, const void* x,
   const bool sums = splits > 1 || !out;
   const DenseArgs p{sums ? partial : out, (const short*)x, (const short*)w,
                     (const short*)(sums ? nullptr : bias), M, K, N, (int)xs, 0, 0, splits,
-                    parts_first(M, K, N), 0.f, 0.f, xs};
+                    order(M, K, N), 0.f, 0.f, xs};
   const Plan how = plan(M, K, N, glu);
   const hipError_t err =
       how.form != STREAMED && !is_long(K, xs)
-          ? ks_mid_gemm(p.out, x, w, p.bias, M, K, N, xs, splits, sums, 64, 0, stream)
+          ? ks_mid_gemm(p.out, x, w, p.bias, M, K, N, xs, splits, sums, 64, RUNS, stream)
           : run(p, how.tm, glu ? GLU : sums ? PARTIAL : BIAS, stream);
   if (err != hipSuccess) return err;
   if (sums && out) {
@@ -282,6 +288,6 @@ extern "C" hipError_t ks_streamed_clamped_glu(void* out, const void* x, const vo
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) != 0)
     return hipErrorInvalidValue;
   return run({out, (const short*)x, (const short*)w, nullptr, M, K, N, (int)xs, 0, 0, 1,
-              0, alpha, limit, xs},
+              RUNS, alpha, limit, xs},
              plan(M, K, N, true).tm, CLAMPED, stream);
 }
