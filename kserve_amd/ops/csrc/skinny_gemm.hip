@@ -129,23 +129,26 @@ int few_parts(int M, int K) {
 // rows 38.6 / 38.8, 40.0 / 39.1, 44.8 / 40.3, 48.5 / 41.5, M 50304 at 64 89.9 / 82.3;
 // but K 2048, M 32000 at 24 / 48 / 64 22.7 / 24.1, 24.8 / 24.6, 26.3 / 25.0).
 //
-// Above by an estimate from the times of K 1024 to 14336, M 1024 to 50304 (weights not
-// in a cache): a launch, the steps of the busiest unit and the sums that are written,
-// off by 5 % in the mean (K 14336, M 4096 at 96 / 256 rows 27.6 / 25.6, 53.6 / 38.6; K
-// 4096, M 4096 10.4 / 11.8, 18.3 / 21.4, M 6144 15.9 / 14.4, 27.0 / 23.7; K 2048, M 16384
-// 16.5 / 23.9, 26.7 / 35.6); no caller's K is shorter there. Past 8192 features a pass of its own adds the sums, to 10240
-// features the norm's kernel for some callers: those cost less (one part of 64 features /
-// three of 128, with the norm: K 3072, M 10240 at 65 / 160 / 192 rows 26.9 / 23.8, 37.0 /
-// 29.8, 39.8 / 31.1, without at 192 32.8 / 29.5; K 2048 at 65 / 129 19.3 / 21.7, 23.8 / 27.5).
+// Above by an estimate from the times of K 1024 to 14336, M 1024 to 50304 (weights not in a
+// cache): a launch, the steps of the busiest unit and the sums that are written, off by 5 %
+// in the mean (K 14336, M 4096 at 96 / 256 rows 27.6 / 25.6, 53.6 / 38.6; K 4096, M 4096 10.4
+// / 11.8, 18.3 / 21.4, M 6144 15.9 / 14.4, 27.0 / 23.7; K 2048, M 16384 16.5 / 23.9, 26.7 /
+// 35.6); in parts no caller's K is shorter (gate|up to 112 rows: M 12288 to 16384, K 64 to
+// 960 15 % ahead of the kernel before in the mean, 2 % behind at most). Past 8192 features a
+// pass of its own adds the sums, to 10240 features the norm's kernel for some callers: those
+// cost less (one part of 64 features / three of 128, with the norm: K 3072, M 10240 at 65 /
+// 160 / 192 rows 26.9 / 23.8, 37.0 / 29.8, 39.8 / 31.1, without at 192 32.8 / 29.5; K 2048 at
+// 65 / 129 19.3 / 21.7, 23.8 / 27.5).
 //
-// At 129 to 192 rows blocks of 64 features fall behind where K is long: in more than two
-// parts from token rows of 1.6 MB on, in two of 1.4, in one part from K 3840 on, but where the other's two parts lie a
-// multiple of 4 KB apart (us, 64 features / 128, with the sums added: M 13824, K 3584 at 160 /
-// 176 rows 34.2 / 35.7, 36.3 / 37.7, K 4608 43.3 / 41.8, 46.4 / 43.3, K 5120 52.9 / 45.7, 53.9 /
-// 46.7, but M 16384, K 4096 at 176 38.5 / 40.9; M 4352, K 4096 at 160 / 192 21.4 / 22.8, 23.7 /
-// 24.1, K 5120 at 160 / 176 26.0 / 23.8, 27.8 / 24.7; M 7168, K 4096 at 176 / 192 28.1 / 25.9, 29.6 /
-// 26.7; M 5120, K 6144 29.9 / 26.5, 30.1 / 27.6). Over K 2112 to
-// 8192 and M 4352 to 16384 this takes the better one to 0.1 % in the mean, to 4 % without.
+// At 129 to 192 rows blocks of 64 features fall behind where K is long: in more than two parts
+// from token rows of 1.6 MB on, in two of 1.4, in one part from K 3840 on, but where the
+// other's two parts lie a multiple of 4 KB apart (us, 64 features / 128, with the sums added:
+// M 13824, K 3584 at 160 / 176 rows 34.2 / 35.7, 36.3 / 37.7, K 4608 43.3 / 41.8, 46.4 /
+// 43.3, K 5120 52.9 / 45.7, 53.9 / 46.7, but M 16384, K 4096 at 176 38.5 / 40.9; M 4352, K
+// 4096 at 160 / 192 21.4 / 22.8, 23.7 / 24.1, K 5120 at 160 / 176 26.0 / 23.8, 27.8 / 24.7; M
+// 7168, K 4096 at 176 / 192 28.1 / 25.9, 29.6 / 26.7; M 5120, K 6144 29.9 / 26.5, 30.1 /
+// 27.6). Over K 2112 to 8192 and M 4352 to 16384 this takes the better one to 0.1 % in the
+// mean, to 4 % without.
 Plan plan(int M, int K, int N, bool halves) {
   const long rows = halves ? 2L * M : M;
   const int tiles = cdiv(rows, 128), steps = K / BK;
@@ -197,15 +200,16 @@ Plan plan(int M, int K, int N, bool halves) {
   return best;
 }
 
-// Whether an XCD takes all parts of its features (gemm_tile.h): where 2.5 MB of token
-// rows and its share of the sums fit its L2 of 4 MB (us with the sums added, else / so: K
-// 8192, M 8192 at 129 / 256 rows 39.4 / 36.4, 47.1 / 52.0, K 14336, M 5120 at 192 44.5 /
-// 58.6; K 8192, M 9216 at 160 43.1 / 45.6). Up to 128 rows the sums are few. Every eighth
-// block above 192 rows to K 6144, past which runs' token rows count for more (K 8192 at 193
-// rows, runs / in turn, M 4352 32.7 / 34.8, M 9728 50.0 / 50.5; K 14336 level).
+// Whether an XCD takes all parts of its features (gemm_tile.h): where 2.5 MB of token rows and
+// its share of the sums fit its L2 of 4 MB (us with the sums added, else / so: K 8192, M 8192
+// at 129 / 256 rows 39.4 / 36.4, 47.1 / 52.0, K 14336, M 5120 at 192 44.5 / 58.6; K 8192, M
+// 9216 at 160 43.1 / 45.6). Up to 128 rows the sums are few. Every eighth block above 192
+// rows to K 10240, past which it is level, but where parts lie powers of two apart (at 193
+// rows, runs / in turn, K 7168, M 5120 32.9 / 30.5, K 8064 34.2 / 31.9, K 10240 39.3 / 37.3,
+// K 8192, M 4352 32.7 / 34.8, M 9728 50.0 / 50.5).
 Order order(int M, int K, int N) {
   if (N > 128 && M <= 8192 && (long)N * K <= 5 << 18) return PARTS_FIRST;
-  return N > 192 && K <= 6144 ? IN_TURN : RUNS;
+  return N > 192 && K <= 10240 && K != 8192 ? IN_TURN : RUNS;
 }
 
 hipError_t run(DenseArgs p, int tm, int epi, hipStream_t stream) {
