@@ -159,14 +159,17 @@ Plan plan(int M, int K, int N, bool halves) {
   }
   if (!halves && ks_mid_wide(M, K, N)) return {N > 96 ? ONE_PART : STREAMED, 64, 1};
   // Small weights: their rows twice rather than all token rows in a block (us, K 2048, M
-  // 2048 at 129 / 192 / 256 rows 7.4 / 8.8 / 10.1 streamed, 7.7 / 7.8 / 7.8 so, M 4096 9.4 /
-  // 10.9 / 12.9, 11.3 / 11.4 / 11.8), and above 192 rows some larger ones, which leave half
-  // as many sums to add (with those, K 8192, M 2048 at 193 / 224 / 256 21.5 / 23.4 / 25.3
+  // 2048 at 129 / 192 / 256 rows 7.4 / 8.8 / 10.1 streamed, 7.7 / 7.8 / 7.8 so, M 4096 9.4 / 10.9
+  // / 12.9, 11.3 / 11.4 / 11.8), and above 192 rows some larger ones, which leave half as
+  // many sums to add (with those, K 8192, M 2048 at 193 / 224 / 256 21.5 / 23.4 / 25.3
   // streamed, 20.6 / 20.7 / 21.1 so, added by the norm K 2048, M 4096 at 193 / 224 18.7 /
-  // 19.9, 15.6 / 15.9, K 3072 at 224 22.4, 20.0; but K 4096, M 3072 without at 224 15.8, 18.1).
+  // 19.9, 15.6 / 15.9, K 3072 at 224 22.4, 20.0; K 8192, M 2560 at 224, sums, added by a
+  // pass, by the norm 18.9, 28.5, 28.8 streamed, 21.1, 24.2, 25.1 so, M 2112 17.7, 22.0, 23.2
+  // and 21.0, 23.6, 25.0 at 193; but K 4096, M 3072 without at 224 15.8, 18.1).
   if (!halves && N > 128 && M <= 4096 &&
       ((long)K * M <= 3000000 + (N - 128) * 50000L ||
-       (N > 192 && (M <= 2048 ? K <= 8192 : M > 3584 && K <= 3072)))) {
+       (N > 192 && (M <= 2048 || (M > 2240 && M <= 2560 && K > 7168) ? K <= 8192
+                                                                       : M > 3584 && K <= 3072)))) {
     const int n = 2 * cdiv(M, 64);
     return {ROW_TILES, 64, parts(n, K)};
   }

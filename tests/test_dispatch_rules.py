@@ -155,7 +155,7 @@ def test_parts_of_streamed_products(native, n):
     [
         (256, 8192, 2048, 4), (193, 8192, 2048, 4), (192, 8192, 2048, 8), (256, 8256, 2048, 8),
         (224, 2048, 4096, 2), (193, 3072, 4096, 2), (192, 3072, 4096, 4), (224, 3136, 4096, 4),
-        (224, 4096, 3072, 5),
+        (224, 4096, 3072, 5), (224, 8192, 2560, 3), (224, 8192, 2240, 7), (224, 7168, 2560, 6),
         (192, 4096, 4352, 3), (160, 5120, 4352, 7), (173, 4608, 4352, 3), (174, 4608, 4352, 7),
         (176, 4096, 7168, 4), (192, 4096, 8192, 4),
     ],
