@@ -510,6 +510,33 @@ def _skinny_glu_rows(n: int, k: int, m: int) -> bool:
     return m >= 4608 and (n <= 48 or m <= 8192 or m >= 10240)
 
 
+def _library_fills(n: int, k: int, m: int) -> bool:
+    """Wide products where the library's blocks fill the units better than one part of K or
+    two of the streaming tiles, which it does not at whole 32 rows, nor where k is no whole
+    128 (us, kernel / library: k 3072, m 11264 at 193 / 224 / 239 rows 35.2 / 31.3, 31 / 34, 36.3 /
+    32.1, k 3904, m 13824 at 176 37.8 / 42.1). 129 to 191 rows: k 2048, m 8320 to 10304 4 to 23 %
+    behind, but m 11200 at 150 19.2 / 26.2; 161 on, k 2560, m 13824 at 176 29.3 / 27.8, k 3072 at
+    176 / 191 32.8 / 30.0, 33.8 / 30.5, k 4608 42.1 / 40.9, but m 13568 32.7 / 32.3, k 2304 and 4096 a
+    tenth ahead. Above, to 13311 features: k 2560 at 239 rows, m 9216 / 10304 / 12288 5, 28, 8 %
+    behind, but m 12800 at 219 31 / 32, k 3584, m 10304 / 11264 10, 7 %, k 4096, m 10304 / 11264 7, 1 %;
+    further on k 2816, m 13312 to 16384 5 to 8 %, from 225 rows on k 3072 to 3840 4 to 7 %, but k
+    2560 and 4096 level. 113 to 127: k 3072, m 10304 5 to 8 %, k 5120, m 11264 / 12288 6 to 12, 6
+    to 8 %, but m 10880 34 / 36, at 97 rows 3, 2 %, k 4096 level."""
+    if n < 128:
+        return n > 112 and m <= 12288 and (
+            2816 < k < 4096 and 10240 < m < 12288
+            or 4096 < k <= 6144 and 11264 <= m and (k > 4608 or m < 12288)
+        )
+    if n < 192:
+        return (
+            1920 < k <= 2048 and m < 10496
+            or 13568 < m <= 16384 and n > 160 and 2304 < k < 4736 and k != 4096
+        )
+    if m < 13312:
+        return 2304 < k <= 4096 and 8704 <= m < (10752 if k == 4096 else 12544 if k < 2816 else 13312)
+    return 2816 <= k < 4096 and m <= 16384 and (k < 3072 or n > 224)
+
+
 def _streamed_rows(n: int, k: int, m: int) -> bool:
     """Wide products of 49 to 256 rows that the rules above leave to the library and the
     few-row kernel's tiles of all rows take sooner, with a bias or without (MI355X, us,
@@ -523,17 +550,15 @@ def _streamed_rows(n: int, k: int, m: int) -> bool:
     157). Up to 64 rows on short k or full rounds only (k 4096, m 12288 at 33 rows 26.7 /
     25.2). Not where the library's blocks come to two thirds of the units and the streamed ones
     to half (k 2560, m 9216 at 129 / 176 / 192 rows 24.5 / 22.1, 28.1 / 23.5, 28.8 / 31.9, m
-    8704 at 96 / 112 21.7 / 21.5, 23.4 / 21.5; k 3072, m 10752 at 176 31.9 / 26.6), nor past 13568
-    features, where from 161 to 191 rows its blocks fill the units, on whole steps of 128 of k
-    (k 2560, m 13824 at 176 29.3 / 27.8, k 3072 at 176 / 191 32.8 / 30.0, 33.8 / 30.5, k 4608 42.1 /
-    40.9; but m 13568 32.7 / 32.3, k 3904 37.8 / 42.1, k 2304 and 4096 a tenth ahead). Captured
-    steps of 128 sequences are level with the library's product to the vocabulary (k 4096, m
-    32000; contexts of 500 / 2000 tokens 768 / 764, 1292 / 1298), of 256 ahead (1101 / 1118)."""
+    8704 at 96 / 112 21.7 / 21.5, 23.4 / 21.5; k 3072, m 10752 at 176 31.9 / 26.6), nor where
+    `_library_fills`. Captured steps of 128 sequences are level with the library's product to
+    the vocabulary (k 4096, m 32000; contexts of 500 / 2000 tokens 768 / 764, 1292 / 1298), of
+    256 ahead (1101 / 1118)."""
     if m % 4 or not 48 < n <= 256 or k < 1024:
         return False
     if m < 11264 and 2048 < k < 4096 and (96 if 2304 < k < 3072 else 128) < n < 192:
         return False
-    if 13568 < m <= 16384 and 160 < n < 192 and 2304 < k < 4736 and k % 128 == 0 and k != 4096:
+    if n % 32 and k % 128 == 0 and _library_fills(n, k, m):
         return False
     if n <= 64:
         return 8192 < m <= 16384 and (k <= 2048 or m > 12288 and k <= 5120)

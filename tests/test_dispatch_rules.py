@@ -105,11 +105,17 @@ def test_few_row_gate_up(n, k, m, own):
         (128, 8192, 32768, True), (128, 8192, 32772, False), (128, 12288, 28672, False),
         (80, 2048, 10302, False),
         (129, 2560, 9216, False), (191, 3072, 11260, False), (192, 2560, 9216, True),
-        (144, 2048, 9216, True), (144, 4096, 9216, True), (144, 2560, 11264, True),
+        (160, 2048, 9216, True), (150, 2048, 9216, False), (144, 4096, 9216, True), (144, 2560, 11264, True),
         (176, 3072, 13824, False), (161, 2560, 16384, False), (191, 4608, 13572, False),
         (176, 3072, 13568, True), (160, 3072, 13824, True), (192, 3072, 13824, True),
         (176, 2304, 13824, True), (176, 4096, 13824, True), (176, 3904, 13824, True),
-        (176, 4736, 13824, True),
+        (176, 4736, 13824, True), (239, 2560, 10304, False), (224, 2560, 10304, True),
+        (193, 3072, 13308, False), (193, 3072, 13312, True), (225, 3072, 13312, False),
+        (239, 2304, 10304, True), (239, 3904, 11264, True),
+        (120, 5120, 12288, False), (112, 5120, 12288, True), (120, 3072, 12288, True),
+        (120, 3072, 11264, False), (120, 4096, 11264, True), (128, 5120, 11264, True),
+        (120, 5120, 10880, True), (150, 2048, 11200, True), (239, 4096, 10748, False),
+        (239, 2560, 12544, True), (197, 2816, 13824, False),
         (96, 2560, 8704, True), (97, 2560, 8704, False), (128, 2304, 8704, True),
         (128, 3072, 10752, True), (129, 2304, 8704, False),
     ],
