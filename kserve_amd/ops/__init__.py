@@ -585,8 +585,15 @@ def _streamed_glu_rows(n: int, k: int, m: int) -> bool:
     behind two parts of 128 where sums are many (m 7168, k 6144 at 128 / 192 50.3 / 52.5, 66 /
     59; k 14336 at 64 / 65 / 256 76 / 92, 84 / 81, 158 / 118), and between there and 12288
     blocks come out uneven (k 5120, m 9728 at 64 / 96 / 128 62 / 53, 59 / 60, 60 / 57, k
-    3072 at 64 36.5 / 34.8, k 4096 42.3 / 45.0)."""
+    3072 at 64 36.5 / 34.8, k 4096 42.3 / 45.0). Nor where the library is ahead but at whole 32
+    rows (at 170 / 193 / 250 rows k 2048, m 4096 5, 12, 14 % behind, at 192 25.7 / 21.0, m 4352 at
+    197 28.0 / 22.5; at 210 / 250 k 3072, m 5504 3, 6 %, at 256 40.7 / 37.0)."""
     if m % 4 or not 32 < n <= 256 or k < 1024 or not 4096 <= m <= 16384:
+        return False
+    if n % 32 and (
+        n > 160 and m < 4224 and (1728 if n < 192 else 1920) < k <= 2048
+        or n > 208 and 5504 <= m < 7168 and 3072 <= k <= 4096
+    ):
         return False
     if k <= 2048 or m >= 12288:
         return True
@@ -596,7 +603,7 @@ def _streamed_glu_rows(n: int, k: int, m: int) -> bool:
         return k <= 4096 or n <= 96 or n > 128
     if m >= 5504:
         return n <= 64 or k <= 4096 or n <= 128 and k <= 8192
-    return m >= 4608 and k <= 4096 and n * k <= 600 << 10
+    return m >= 4608 and k <= 4096 and n * k <= 576 << 10
 
 
 def _streamed_parts(n: int, k: int, m: int) -> bool:

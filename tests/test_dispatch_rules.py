@@ -138,6 +138,8 @@ def test_streamed_product(n, k, m, own):
         (65, 14336, 8192, False), (64, 5120, 9728, False), (64, 4096, 9728, True),
         (64, 3072, 9728, False), (96, 5120, 9728, True), (128, 5120, 9728, False),
         (129, 5120, 9728, True), (256, 14336, 12288, True), (256, 2048, 4100, True),
+        (161, 2048, 4096, False), (192, 2048, 4096, True), (193, 1536, 4096, True), (193, 2048, 4352, True),
+        (209, 3072, 5504, False), (224, 4096, 5504, True), (209, 4096, 7168, True),
     ],
 )
 def test_streamed_gate_up(n, k, m, own):
