@@ -609,7 +609,17 @@ def _streamed_glu_rows(n: int, k: int, m: int) -> bool:
 def _streamed_parts(n: int, k: int, m: int) -> bool:
     """The same where the sums over parts of k stay in 32 bits for the next kernel to add
     (us, their writing, library): k 2048, m 4096 at 65 / 128 / 256 rows 6.7 / 12.3, 8.3 / 14.6,
-    11.8 / 13.3, m 8192 at 129 / 256 13.4 / 15.2, 18.1 / 24.4, k 4096, m 4096 at 256 17.9 / 22.4."""
+    11.8 / 13.3, m 8192 at 129 / 256 13.4 / 15.2, 18.1 / 24.4, k 4096, m 4096 at 256 17.9 / 22.4. On
+    short k the library is ahead above 192 rows but for whole 32 of them (with the norm, k
+    2048 at 193 / 224 / 239 rows, m 6144 22.2 / 20.9, 24.0 / 28.4, 24.5 / 21.8, m 8192 24.0 / 23.3, 25.6 /
+    29.9, 26.1 / 23.9, k 2560, m 6144 at 193 / 240 25.5 / 23.9, 27.9 / 25.2, m 7168 level, k 3072, m 6144 at 208 28.4 /
+    26.6; m 4608 from 225 on, k 2560 at 240 25.1 / 22.4)."""
+    if n > 192 and n % 32 and (
+        k < 2560 and 4352 <= m <= 8192
+        or k < 3072 and 4352 <= m <= 6144
+        or k == 3072 and 5120 < m <= 6144
+    ) and (m >= 5120 or n > 224):
+        return False
     return m % 4 == 0 and 64 < n <= 256 and k >= 2048 and 4096 <= m <= 8192
 
 

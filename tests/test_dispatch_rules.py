@@ -146,6 +146,19 @@ def test_streamed_gate_up(n, k, m, own):
     assert ops._streamed_glu_rows(n, k, m) is own
 
 
+@pytest.mark.parametrize(
+    "n,k,m,own",
+    [
+        (193, 2048, 5120, False), (192, 2048, 5120, True), (224, 2048, 6144, True),
+        (240, 2560, 6144, False), (240, 2560, 6152, True), (240, 2304, 8192, False),
+        (240, 3072, 6144, False), (240, 3072, 5120, True), (240, 2560, 4608, False),
+        (208, 2560, 4608, True), (240, 2048, 4096, True), (240, 4096, 4096, True),
+    ],
+)
+def test_streamed_parts(n, k, m, own):
+    assert ops._streamed_parts(n, k, m) == own
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 96, 97, 128, 129, 192, 193, 256])
 def test_parts_of_streamed_products(native, n):
     """Parts of K: at least four steps in each, one where the next kernel takes no sums,
