@@ -140,6 +140,14 @@ int few_parts(int M, int K) {
 // 160 / 192 rows 26.9 / 23.8, 37.0 / 29.8, 39.8 / 31.1, without at 192 32.8 / 29.5; K 2048 at
 // 65 / 129 19.3 / 21.7, 23.8 / 27.5).
 //
+// To 128 rows, 8192 features and K 8192 parts of 128 features cost 2.25 us more, since they
+// leave twice as many sums to add (us, 128 features / 64, with the norm that adds them: M
+// 6144, K 3776 at 70 / 96 / 127 rows 20.8 / 18.9, 22.8 / 20.3, 25.9 / 23.2, K 4608 22.3 /
+// 21.1, 24.4 / 23.2, 27.4 / 26.2; M 4776, K 7168 24.9 / 22.7, 26.4 / 24.2 at 84, 29.9 / 27.6;
+// M 5120, K 8192 at 128 31.8 / 28.8; not K 6144, M 7168 at 127 32.9 / 35.0): over K 2048 to
+// 8192, M 2112 to 8192 0.1 % off the better one, 1.4 % without. On longer K it is the other
+// way in a model (a 77-token prompt of 4 layers 504, with K 14336 so too 516).
+//
 // At 129 to 192 rows blocks of 64 features fall behind where K is long: in more than two parts
 // from token rows of 1.6 MB on, in two of 1.4, in one part from K 3840 on, but where the
 // other's two parts lie a multiple of 4 KB apart (us, 64 features / 128, with the sums added:
@@ -190,6 +198,7 @@ Plan plan(int M, int K, int N, bool halves) {
                      cost.step[i] * (cdiv(steps, s) * (float)cdiv((long)n * s, UNITS)) +
                      (s > 1 ? cost.sums * 4e-6f * s * N * M : 0.f) +
                      (s > 1 && M > 8192 ? M > 10240 ? 6.f : 2.5f : 0.f) +
+                     (i == 1 && s > 1 && N <= 128 && M <= 8192 && K <= 8192 ? 2.25f : 0.f) +
                      (i == 0 && long_k &&
                               (s > 1 ? (long)N * K > (s > 2 ? 800000 : 700000)
                                      : K >= 3840 && K % 4096 != 0)

@@ -173,6 +173,16 @@ def test_parts_of_streamed_products(native, n):
 
 @pytest.mark.parametrize(
     "n,k,m,parts",
+    [(128, 4096, 6144, 2), (70, 4608, 6144, 2), (128, 8192, 5120, 3), (77, 14336, 4096, 8),
+     (96, 3072, 10240, 3), (129, 4096, 6144, 5), (64, 4096, 6144, 5)],
+)
+def test_parts_to_128_rows(native, n, k, m, parts):
+    """Tiles of 64 features, which leave half as many sums."""
+    assert native.ks_skinny_splits(m, k, n, 0) == parts
+
+
+@pytest.mark.parametrize(
+    "n,k,m,parts",
     [
         (256, 8192, 2048, 4), (193, 8192, 2048, 4), (192, 8192, 2048, 8), (256, 8256, 2048, 8),
         (224, 2048, 4096, 2), (193, 3072, 4096, 2), (192, 3072, 4096, 4), (224, 3136, 4096, 4),
