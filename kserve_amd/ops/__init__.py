@@ -672,17 +672,20 @@ def _dense_round(n: int, k: int, m: int) -> bool:
     -3.9), and only where its tiles of 128 x 128 fill more than three quarters of the units:
     the library splits k (k 3072, m 768 at 1500 / 3600 / 4200 +3.1, +5.3, -0.5, k 4096, m 1024
     at 1100 / 2600 / 3100 +5.2, -0.3, -2.4; at three quarters k 3072, m 2048 at 1500 31.6 / 27.4,
-    k 4096, m 1536 at 2000 35.8 / 33.0). Of the widest that holds to k 1536 already, while
-    more than 48 tiles are there and too few for the units (k 2048, m 2304 at 257 / 350 / 512 /
-    800 / 900 10.3 / 10.9, 11.6 / 11.3, 17.6 / 14.1, 18.2 / 16.9, 18.6 / 23.8, m 2048 at 300 / 512
-    / 700 / 1150 9.3 / 11.0, 12.4 / 11.3, 15.6 / 13.7, 21.7 / 23.5, k 1536, m 2048 at 512 / 600
-    10.6 / 9.5, 11.9 / 13.2). Its times turn from one size to the next (k 2560, m 2304 at 1700 /
-    2000 / 2600 27 / 30, 37 / 33, 36 / 37), on wider ones more than that (k 2048, m 3072 at 768 /
-    1280 / 2048 16.4 / 19.3, 24.4 / 21.1, 28.7 / 27.7; k 768, m 4096 at 1400 / 1872 14.0 / 18.5,
-    19.3 / 17.4; k 4096, m 4096 at 1400 50 / 50; without a bias m 2560 to
-    3072 would mostly gain a tenth to a third to k 1536, and at some sizes k 2048 lose as much),
-    and past one round its tiles are ahead (k
-    2048, m 768 at 10900 rows 37 / 33, k 3072 58 / 52)."""
+    k 4096, m 1536 at 2000 35.8 / 33.0).
+    So it does from k 1664 on with 65 to 99 of them, to 120 at k 2048, past m 256 (m 512, k 1792
+    / 2048 with 60 / 80 / 100 / 124 tiles 0.87 / 1.13 / 0.80 / 0.82, 0.87 / 1.16 / 1.04 /
+    0.99 of the library's time, m 1536, k 1920 with 60 / 84 / 108 0.90 / 1.20 / 0.84). Of
+    the widest that holds to k 1536 already, while more than 48 tiles are there and too few
+    for the units (k 2048, m 2304 at 257 / 350 / 512 / 800 / 900 10.3 / 10.9, 11.6 / 11.3,
+    17.6 / 14.1, 18.2 / 16.9, 18.6 / 23.8, m 2048 at 300 / 512 / 700 / 1150 9.3 / 11.0, 12.4
+    / 11.3, 15.6 / 13.7, 21.7 / 23.5, k 1536, m 2048 at 512 / 600 10.6 / 9.5, 11.9 / 13.2).
+    Its times turn from one size to the next (k 2560, m 2304 at 1700 / 2000 / 2600 27 / 30,
+    37 / 33, 36 / 37), on wider ones more than that (k 2048, m 3072 at 768 / 1280 / 2048
+    16.4 / 19.3, 24.4 / 21.1, 28.7 / 27.7; k 768, m 4096 at 1400 / 1872 14.0 / 18.5, 19.3 /
+    17.4; k 4096, m 4096 at 1400 50 / 50; without a bias m 2560 to 3072 would mostly gain a
+    tenth to a third to k 1536, and at some sizes k 2048 lose as much), and past one round
+    its tiles are ahead (k 2048, m 768 at 10900 rows 37 / 33, k 3072 58 / 52)."""
     tiles = -(-n // 128) * -(-m // 128)
     return (
         m % 8 == 0
@@ -692,7 +695,14 @@ def _dense_round(n: int, k: int, m: int) -> bool:
         and (
             tiles > 192
             if k > 2048
-            else k <= 1024 or m <= 1792 or tiles <= 48 or tiles * 8 > k - 960
+            else k <= 1024
+            or m <= 256
+            or tiles <= (64 if m <= 1792 else 48)
+            or (
+                k <= 1536 or tiles > (120 if k > 1920 else 99)
+                if m <= 1792
+                else tiles * 8 > k - 960
+            )
         )
     )
 

@@ -340,6 +340,10 @@ def test_encoder_product(n, k, m, gelu, own):
         (1700, 3072, 2048, True), (512, 2048, 2048, False), (1024, 2048, 2048, False),
         (1025, 2048, 2048, True), (384, 2048, 2048, True), (385, 2048, 2048, False),
         (512, 1536, 2048, False), (513, 1536, 2048, True), (512, 1024, 2304, True),
+        (2316, 2048, 512, False), (838, 1920, 1672, False), (838, 1536, 1672, True),
+        (1900, 1920, 768, False), (2100, 1920, 256, True), (2048, 1792, 512, True),
+        (2049, 1792, 512, False), (3201, 1792, 512, True), (3840, 2048, 512, False),
+        (3841, 2048, 512, True),
         (512, 2048, 1792, True), (300, 2048, 2304, False), (257, 2048, 2304, False),
     ],
 )
