@@ -587,7 +587,8 @@ def _streamed_glu_rows(n: int, k: int, m: int) -> bool:
     blocks come out uneven (k 5120, m 9728 at 64 / 96 / 128 62 / 53, 59 / 60, 60 / 57, k
     3072 at 64 36.5 / 34.8, k 4096 42.3 / 45.0). Nor where the library is ahead but at whole 32
     rows (at 170 / 193 / 250 rows k 2048, m 4096 5, 12, 14 % behind, at 192 25.7 / 21.0, m 4352 at
-    197 28.0 / 22.5; at 210 / 250 k 3072, m 5504 3, 6 %, at 256 40.7 / 37.0)."""
+    197 28.0 / 22.5; at 139 / 170 / 185 k 2560, m 4608 7, 9, 11, m 5120 3, 7, 8 %, from 200 on ahead; at
+    210 / 250 k 3072, m 5504 3, 6 %, at 256 40.7 / 37.0)."""
     if m % 4 or not 32 < n <= 256 or k < 1024 or not 4096 <= m <= 16384:
         return False
     if n % 32 and (

@@ -139,6 +139,8 @@ def test_streamed_product(n, k, m, own):
         (64, 3072, 9728, False), (96, 5120, 9728, True), (128, 5120, 9728, False),
         (129, 5120, 9728, True), (256, 14336, 12288, True), (256, 2048, 4100, True),
         (161, 2048, 4096, False), (192, 2048, 4096, True), (193, 1536, 4096, True), (193, 2048, 4352, True),
+        (139, 2560, 5120, False), (160, 2560, 5120, True), (193, 2560, 5120, True), (139, 2432, 5120, True),
+        (139, 2560, 5504, True), (128, 2560, 4608, True),
         (209, 3072, 5504, False), (224, 4096, 5504, True), (209, 4096, 7168, True),
     ],
 )
