@@ -593,6 +593,7 @@ def _streamed_glu_rows(n: int, k: int, m: int) -> bool:
         return False
     if n % 32 and (
         n > 160 and m < 4224 and (1728 if n < 192 else 1920) < k <= 2048
+        or 128 < n < 192 and 4608 <= m < 5504 and 2432 < k < 3072
         or n > 208 and 5504 <= m < 7168 and 3072 <= k <= 4096
     ):
         return False
